@@ -105,7 +105,7 @@ __global__ void __launch_bounds__(NW * 64) attn_prefill_kernel(AttnPrefillDesc a
   // K rows as bf16 (the twin of the rotated keys), V as bf16 V^T [b, kv, d, T]: both were narrowed
   // once, not once per query block
   const uint16_t *K = a.k16 + (int64_t)b * a.k_sb + (int64_t)kvh * a.k_skv + (int64_t)rp * a.k_srep;
-  const uint16_t *VT = a.vt16 + ((int64_t)b * (a.heads / a.rep) + kvh) * D * (int64_t)a.t;
+  const uint16_t *VT = a.vt16 + ((int64_t)b * (a.heads / a.rep) + kvh) * D * (int64_t)a.vt_st;
   const float *V = a.v + (int64_t)b * a.v_sb + (int64_t)kvh * a.v_skv + (int64_t)rp * a.v_srep;
   const float *M = a.mask ? a.mask + (int64_t)b * a.m_sb + (int64_t)h * a.m_sh + (int64_t)qc * a.m_ss : nullptr;
 
@@ -149,14 +149,14 @@ __global__ void __launch_bounds__(NW * 64) attn_prefill_kernel(AttnPrefillDesc a
 #pragma unroll
     for (int c = 0; c < KCH; ++c) {
       const int ch = tid + c * NT, dim = ch / (BN / 8), k8 = (ch % (BN / 8)) * 8;
-      vreg[c] = *(const uint4 *)(VT + (int64_t)dim * a.t + min(t0 + k8, a.t - 8));
+      vreg[c] = *(const uint4 *)(VT + (int64_t)dim * a.vt_st + min(t0 + k8, a.vt_st - 8));
     }
-    if (step_mask(t0)) {  // mask rows allow 16-byte loads and T % 8 == 0 (checked by the host)
+    if (step_mask(t0)) {  // mask rows allow 16-byte loads (checked by the host)
 #pragma unroll
       for (int kt = 0; kt < KT; ++kt)
 #pragma unroll
         for (int j = 0; j < 4; ++j)
-          mreg[kt][j] = *(const float4 *)(M + min(t0 + kt * 32 + j * 8 + half * 4, a.t - 4));
+          mreg[kt][j] = *(const float4 *)(M + min(t0 + kt * 32 + j * 8 + half * 4, a.m_len - 4));
     }
   };
   uint32_t t0 = next_step(0);
@@ -350,7 +350,7 @@ attn_prefill_keysplit_kernel(AttnPrefillDesc a) {
   const bool q_ok = query < a.s;
   const uint32_t qc = q_ok ? query : a.s - 1;
   const uint16_t *K = a.k16 + (int64_t)b * a.k_sb + (int64_t)kvh * a.k_skv + (int64_t)rp * a.k_srep;
-  const uint16_t *VT = a.vt16 + ((int64_t)b * (a.heads / a.rep) + kvh) * D * (int64_t)a.t;
+  const uint16_t *VT = a.vt16 + ((int64_t)b * (a.heads / a.rep) + kvh) * D * (int64_t)a.vt_st;
   const float *V = a.v + (int64_t)b * a.v_sb + (int64_t)kvh * a.v_skv + (int64_t)rp * a.v_srep;
   const float *M = a.mask ? a.mask + (int64_t)b * a.m_sb + (int64_t)h * a.m_sh + (int64_t)qc * a.m_ss : nullptr;
 
@@ -370,7 +370,7 @@ attn_prefill_keysplit_kernel(AttnPrefillDesc a) {
 #pragma unroll
     for (int c = 0; c < KCH; ++c) {
       const int ch = lane + c * 64, dim = ch / (BN / 8), k8 = (ch % (BN / 8)) * 8;
-      vreg[c] = *(const uint4 *)(VT + (int64_t)dim * a.t + min(t0 + k8, a.t - 8));
+      vreg[c] = *(const uint4 *)(VT + (int64_t)dim * a.vt_st + min(t0 + k8, a.vt_st - 8));
     }
   };
   uint32_t t0 = skip_steps(tiles.next_step(0), wave);
@@ -426,7 +426,7 @@ attn_prefill_keysplit_kernel(AttnPrefillDesc a) {
       for (int kt = 0; kt < KT; ++kt)
 #pragma unroll
         for (int j = 0; j < 4; ++j)
-          mcur[kt][j] = *(const float4 *)(M + min(t_cur + kt * 32 + j * 8 + half * 4, a.t - 4));
+          mcur[kt][j] = *(const float4 *)(M + min(t_cur + kt * 32 + j * 8 + half * 4, a.m_len - 4));
     }
     // registers -> this wave's LDS region.  Its LDS instructions run in program order, so the fragment
     // reads of the previous step are behind these writes and the reads below are ahead of them; the
@@ -664,7 +664,7 @@ __global__ void __launch_bounds__(NW * 64) attn_prefill_f32_kernel(AttnPrefillDe
       for (int kt = 0; kt < KT; ++kt)
 #pragma unroll
         for (int j = 0; j < 4; ++j)
-          mreg[kt][j] = *(const float4 *)(M + min(t0 + kt * 32 + j * 8 + half * 4, a.t - 4));
+          mreg[kt][j] = *(const float4 *)(M + min(t0 + kt * 32 + j * 8 + half * 4, a.m_len - 4));
     }
   };
   uint32_t t0 = next_step(0);
@@ -867,6 +867,21 @@ __global__ void __launch_bounds__(256) mask_tiles_kernel(const float *mask, int6
   if (threadIdx.x == 0) out[(size_t)blockIdx.y * gridDim.x + blockIdx.x] = !(flags & 1u) ? 0 : (flags & 2u) ? 1 : 2;
 }
 
+// A mask whose rows do not allow 16-byte loads (an odd number of keys), copied once to rows of `pitch` floats; past the
+// last key every value is f32::MIN.
+__global__ void __launch_bounds__(256) mask_pad_kernel(const float *mask, int64_t m_ss, uint32_t t, uint32_t pitch, float *out) {
+  const float *row = mask + (int64_t)blockIdx.y * m_ss;
+  const uint32_t c = blockIdx.x * 256 + threadIdx.x;
+  if (c < pitch) out[(size_t)blockIdx.y * pitch + c] = c < t ? row[c] : -3.40282347e+38f;
+}
+
+hipError_t launch_mask_pad(const LaunchCtx &lc, const float *mask, int64_t m_ss, uint32_t s, uint32_t t, uint32_t pitch, float *out) {
+  if (!s || !t) return hipSuccess;
+  if (pitch < t || s > 65535) return hipErrorInvalidValue;
+  CG_LAUNCH(lc, mask_pad_kernel, dim3((pitch + 255) / 256, s), 256, mask, m_ss, t, pitch, out);
+  return hipGetLastError();
+}
+
 hipError_t launch_mask_tiles(const LaunchCtx &lc, const float *mask, int64_t m_ss, uint32_t s, uint32_t t, uint32_t q_rows,
                              uint32_t keys, uint8_t *out) {
   if (!s || !t) return hipSuccess;
@@ -876,7 +891,8 @@ hipError_t launch_mask_tiles(const LaunchCtx &lc, const float *mask, int64_t m_s
 
 hipError_t launch_attn_prefill(const LaunchCtx &lc, const AttnPrefillDesc &d) {
   if (!d.b || !d.heads || !d.s) return hipSuccess;
-  if (d.f32 ? !d.k : (!d.k16 || !d.vt16)) return hipErrorInvalidValue;
+  if (d.f32 ? !d.k : (!d.k16 || !d.vt16 || d.vt_st < d.t || d.vt_st % 8)) return hipErrorInvalidValue;
+  if (d.mask && (d.m_len < d.t || d.m_len % 4)) return hipErrorInvalidValue;
   if (attn_prefill_keysplit(lc, d)) {
     dim3 g32((d.s + 31) / 32, d.heads, d.b);
     CG_LAUNCH(lc, (attn_prefill_keysplit_kernel<64, 64, 4>), g32, 256, d);

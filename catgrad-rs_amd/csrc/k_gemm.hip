@@ -804,6 +804,7 @@ __global__ void __launch_bounds__(WR *WC * 64) gemm_bf16_dma_kernel(GemmDesc g) 
       return;
     }
     if (role == 2) {  // the values: also as bf16 [sequence][head][hd][position], four consecutive positions per store
+      const uint32_t Sp = (S + 7) & ~7u;  // (rows of positions end on a 16-byte boundary, zeros past the last)
 #pragma unroll
       for (int i = 0; i < TM; ++i)
 #pragma unroll
@@ -812,11 +813,26 @@ __global__ void __launch_bounds__(WR *WC * 64) gemm_bf16_dma_kernel(GemmDesc g) 
           const float bv = Bias ? Bias[min(col, Nl - 1)] : 0.f;
 #pragma unroll
           for (int q = 0; q < 4; ++q) {
-            const uint32_t r0 = m0 + wm * WM + i * 32 + q * 8 + (lane >> 5) * 4;  // S % 4 == 0: the four share a sequence
-            if (r0 < g.M && col < Nl) {
-              const uint32_t sq = r0 / S, pos = r0 - sq * S;
-              *(uint2 *)(g.rope_out16[grp] + ((uint64_t)sq * Nl + col) * S + pos) =
-                  bf16_pack4(make_float4(acc[i][j][q * 4] + bv, acc[i][j][q * 4 + 1] + bv, acc[i][j][q * 4 + 2] + bv, acc[i][j][q * 4 + 3] + bv));
+            const uint32_t r0 = m0 + wm * WM + i * 32 + q * 8 + (lane >> 5) * 4;
+            if (r0 >= g.M || col >= Nl) continue;
+            const uint32_t sq = r0 / S, pos = r0 - sq * S;
+            const uint2 v = bf16_pack4(make_float4(acc[i][j][q * 4] + bv, acc[i][j][q * 4 + 1] + bv, acc[i][j][q * 4 + 2] + bv, acc[i][j][q * 4 + 3] + bv));
+            uint16_t *row = g.rope_out16[grp] + ((uint64_t)sq * Nl + col) * Sp;
+            if (S % 4 == 0) {  // (uniform) the four positions share a sequence
+              *(uint2 *)(row + pos) = v;
+              if (pos + 4 == S && Sp > S) *(uint2 *)(row + S) = make_uint2(0u, 0u);
+            } else {
+              const uint32_t w[2] = {v.x, v.y};
+#pragma unroll
+              for (int e = 0; e < 4; ++e) {
+                const uint32_t r = r0 + e;
+                if (r >= g.M) break;
+                const uint32_t s_e = r / S, p_e = r - s_e * S;
+                uint16_t *dst = g.rope_out16[grp] + ((uint64_t)s_e * Nl + col) * Sp + p_e;
+                *dst = (uint16_t)(w[e >> 1] >> ((e & 1) * 16));
+                if (p_e + 1 == S)
+                  for (uint32_t z = 1; z <= Sp - S; ++z) dst[z] = 0;
+              }
             }
           }
         }
@@ -903,13 +919,13 @@ __global__ void __launch_bounds__(256) cast_bf16_kernel(const float *in, uint16_
 // B[k, n] with unit stride along n (f32 or bf16)  ->  bf16 [batch][n][k], k-contiguous: the layout
 // the direct-to-LDS GEMM wants.  64 x 64 tiles through LDS: reads run along n, writes along k.
 template <typename TB, bool VEC>
-__global__ void __launch_bounds__(256) transpose_cast_bf16_kernel(const TB *b, uint16_t *out, uint32_t K,
+__global__ void __launch_bounds__(256) transpose_cast_bf16_kernel(const TB *b, uint16_t *out, uint32_t K, uint32_t Kp,
                                                                   uint32_t N, int64_t sbk, uint32_t nb1,
                                                                   int64_t sb_b0, int64_t sb_b1) {
   __shared__ __attribute__((aligned(8))) uint16_t tile[64][68];  // pitch 136 bytes keeps 8-byte alignment
   const uint32_t bz = blockIdx.z, b0 = bz / nb1, b1 = bz - b0 * nb1;
   const TB *src = b + b0 * sb_b0 + b1 * sb_b1;
-  uint16_t *dst = out + (uint64_t)bz * N * K;
+  uint16_t *dst = out + (uint64_t)bz * N * Kp;
   const uint32_t n0 = blockIdx.x * 64, k0 = blockIdx.y * 64;
   const int r = threadIdx.x >> 4, c4 = (threadIdx.x & 15) * 4;
 #pragma unroll
@@ -944,29 +960,30 @@ __global__ void __launch_bounds__(256) transpose_cast_bf16_kernel(const TB *b, u
     const uint32_t n = n0 + r + i * 16, k = k0 + c4;
     const uint16_t *t = &tile[r + i * 16][c4];
     if (VEC) {
-      if (n < N && k < K) *(uint2 *)(dst + (uint64_t)n * K + k) = *(const uint2 *)t;
+      if (n < N && k < Kp) *(uint2 *)(dst + (uint64_t)n * Kp + k) = *(const uint2 *)t;
     } else {
 #pragma unroll
       for (int j = 0; j < 4; ++j)
-        if (n < N && k + j < K) dst[(uint64_t)n * K + k + j] = t[j];
+        if (n < N && k + j < Kp) dst[(uint64_t)n * Kp + k + j] = t[j];
     }
   }
 }
 
-hipError_t launch_transpose_cast_bf16(const LaunchCtx &lc, const void *b, int b_stype, void *out, uint32_t K,
+hipError_t launch_transpose_cast_bf16(const LaunchCtx &lc, const void *b, int b_stype, void *out, uint32_t K, uint32_t Kp,
                                       uint32_t N, int64_t sbk, uint32_t nb0, uint32_t nb1, int64_t sb_b0,
                                       int64_t sb_b1) {
   if (!K || !N || !nb0 || !nb1) return hipSuccess;
-  dim3 grid((N + 63) / 64, (K + 63) / 64, nb0 * nb1);
+  if (Kp < K) return hipErrorInvalidValue;
+  dim3 grid((N + 63) / 64, (Kp + 63) / 64, nb0 * nb1);
   const int es = b_stype == ST_BF16 ? 2 : 4;
-  const bool vec = N % 4 == 0 && K % 4 == 0 && sbk % 4 == 0 && sb_b0 % 4 == 0 && sb_b1 % 4 == 0 &&
+  const bool vec = N % 4 == 0 && Kp % 4 == 0 && sbk % 4 == 0 && sb_b0 % 4 == 0 && sb_b1 % 4 == 0 &&
                    ((uintptr_t)b % (4 * es)) == 0 && ((uintptr_t)out % 8) == 0;
   if (b_stype == ST_BF16) {
-    if (vec) CG_LAUNCH(lc, (transpose_cast_bf16_kernel<uint16_t, true>), grid, 256, (const uint16_t *)b, (uint16_t *)out, K, N, sbk, nb1, sb_b0, sb_b1);
-    else CG_LAUNCH(lc, (transpose_cast_bf16_kernel<uint16_t, false>), grid, 256, (const uint16_t *)b, (uint16_t *)out, K, N, sbk, nb1, sb_b0, sb_b1);
+    if (vec) CG_LAUNCH(lc, (transpose_cast_bf16_kernel<uint16_t, true>), grid, 256, (const uint16_t *)b, (uint16_t *)out, K, Kp, N, sbk, nb1, sb_b0, sb_b1);
+    else CG_LAUNCH(lc, (transpose_cast_bf16_kernel<uint16_t, false>), grid, 256, (const uint16_t *)b, (uint16_t *)out, K, Kp, N, sbk, nb1, sb_b0, sb_b1);
   } else {
-    if (vec) CG_LAUNCH(lc, (transpose_cast_bf16_kernel<float, true>), grid, 256, (const float *)b, (uint16_t *)out, K, N, sbk, nb1, sb_b0, sb_b1);
-    else CG_LAUNCH(lc, (transpose_cast_bf16_kernel<float, false>), grid, 256, (const float *)b, (uint16_t *)out, K, N, sbk, nb1, sb_b0, sb_b1);
+    if (vec) CG_LAUNCH(lc, (transpose_cast_bf16_kernel<float, true>), grid, 256, (const float *)b, (uint16_t *)out, K, Kp, N, sbk, nb1, sb_b0, sb_b1);
+    else CG_LAUNCH(lc, (transpose_cast_bf16_kernel<float, false>), grid, 256, (const float *)b, (uint16_t *)out, K, Kp, N, sbk, nb1, sb_b0, sb_b1);
   }
   return hipGetLastError();
 }
@@ -2573,7 +2590,7 @@ bool gemm_epilogue_ok(const GemmDesc &g) {
 bool gemm_rope_epilogue_ok(const LaunchCtx &lc, const GemmDesc &g) {
   if (!g.rope_s || !g.n_group || !gemm_epilogue_ok(g)) return false;
   if (g.rope_hd != 64 && g.rope_hd != 128) return false;
-  if (g.nb0 * g.nb1 != 1 || g.glu_gate || g.c16 || g.dual_b || g.M % g.rope_s || g.rope_s % 4 || g.M < 64) return false;
+  if (g.nb0 * g.nb1 != 1 || g.glu_gate || g.c16 || g.dual_b || g.M % g.rope_s || g.M < 64) return false;
   bool grp256 = true;
   for (uint32_t p = 0; p < g.n_group; ++p) {
     if (g.grp_n[p] % 128) return false;

@@ -227,7 +227,7 @@ hipError_t launch_attn_decode(const LaunchCtx &lc, const AttnDecodeDesc &d);
 //   out[b, h, i, :] = softmax_j(q[b,h,i,:] . k[b,h,j,:] / scale + mask[b,h,i,j]) . v[b,h,j,:]
 // q, v: f32 with unit stride along d (v through the kv-head strides as in AttnDecodeDesc; only read for
 // rows whose every key is masked); k16: the keys as bf16 through the same kind of strides; vt16: the
-// values as bf16, transposed, contiguous [b, kv heads, d, t]; t % 8 == 0;
+// values as bf16, transposed, [b, kv heads, d] rows of vt_st values (vt_st % 8 == 0, zeros from t on);
 // mask: additive f32 through its strides (0 = broadcast) or a constant; out [b, heads, s, d] through its strides.
 struct AttnPrefillDesc {
   const float *q, *v, *mask;
@@ -242,6 +242,8 @@ struct AttnPrefillDesc {
   int64_t v_sb, v_skv, v_srep, v_st;
   int64_t m_sb, m_sh, m_ss, m_st;
   uint32_t b, heads, rep, s, t, d;
+  uint32_t vt_st;                      // row pitch of vt16
+  uint32_t m_len;                      // readable floats of a mask row (>= t, a multiple of 4; f32::MIN from t on)
   int32_t has_scale, has_mask_const, m_vec;  // m_vec: mask rows allow 16-byte loads
   float scale, mask_const;
   // optional, for a mask shared by every batch and head (m_sb == m_sh == 0): the class of every
@@ -256,6 +258,8 @@ hipError_t launch_attn_prefill(const LaunchCtx &lc, const AttnPrefillDesc &d);
 void attn_prefill_tiling(const LaunchCtx &lc, const AttnPrefillDesc &d, uint32_t *q_rows, uint32_t *keys);
 // out[qt * ceil(t / keys) + kt] = class of mask[qt * q_rows .., kt * keys ..] (values <= -3e38 count as masked);
 // mask is [s, t] with unit stride along t and row stride m_ss
+// mask [s, t] copied to rows of `pitch` >= t floats, f32::MIN from t on
+hipError_t launch_mask_pad(const LaunchCtx &lc, const float *mask, int64_t m_ss, uint32_t s, uint32_t t, uint32_t pitch, float *out);
 hipError_t launch_mask_tiles(const LaunchCtx &lc, const float *mask, int64_t m_ss, uint32_t s, uint32_t t, uint32_t q_rows,
                              uint32_t keys, uint8_t *out);
 
@@ -310,7 +314,8 @@ struct GemmDesc {
   // (64 or 128) columns.  A group with rope_role 1 leaves the kernel rotated (apply_rope_embedding, cos / sin
   // rows of rope_hd floats at rope_cs_ss apart, indexed by position) as [sequence][head][position][rope_hd] at
   // rope_out (f32) and rope_out16 (bf16, optional) instead of grp_c; a group with rope_role 2 is stored as usual
-  // and also transposed, as bf16 [sequence][head][rope_hd][position], at rope_out16.
+  // and also transposed, as bf16 [sequence][head][rope_hd][position], at rope_out16 (rows of positions padded with
+  // zeros to a multiple of 8).
   uint32_t rope_s, rope_hd;
   uint32_t rope_role[3];
   float *rope_out[3];
@@ -332,8 +337,8 @@ hipError_t launch_matmul(const LaunchCtx &lc, const GemmDesc &g, const char **ke
 // contiguous f32 -> bf16 (RNE); n % 8 == 0, 16-byte aligned
 hipError_t launch_cast_bf16(const LaunchCtx &lc, const float *in, void *out, uint64_t n);
 // B[k, n] (unit stride along n, row stride sbk, f32 or bf16, nb0 x nb1 batches through sb_b0 / sb_b1)
-// -> contiguous bf16 [nb0 * nb1][N][K]
-hipError_t launch_transpose_cast_bf16(const LaunchCtx &lc, const void *b, int b_stype, void *out, uint32_t K,
+// -> bf16 [nb0 * nb1][N] rows of Kp >= K values, zeros from K on
+hipError_t launch_transpose_cast_bf16(const LaunchCtx &lc, const void *b, int b_stype, void *out, uint32_t K, uint32_t Kp,
                                       uint32_t N, int64_t sbk, uint32_t nb0, uint32_t nb1, int64_t sb_b0,
                                       int64_t sb_b1);
 // Several GEMVs y_p = x . B_p^T that share x (M == 1, B_p k-contiguous, 16-byte aligned rows):

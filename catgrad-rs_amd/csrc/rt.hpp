@@ -44,6 +44,10 @@ struct Storage {
   // layer that reads the mask; tiles_key = {element offset of the mask, rows, keys, query rows per tile, keys per tile}
   Storage *tiles = nullptr;
   int64_t tiles_key[5] = {-1, 0, 0, 0, 0};
+  // the same mask with rows padded for 16-byte loads (launch_mask_pad), kept like the table above;
+  // padded_key = {element offset of the mask, rows, keys, row stride}
+  Storage *padded = nullptr;
+  int64_t padded_key[4] = {-1, 0, 0, 0};
 };
 
 enum NodeOp : uint8_t {

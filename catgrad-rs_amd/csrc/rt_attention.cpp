@@ -22,13 +22,12 @@ int try_attn_prefill(cg_backend *be, cg_tensor *n, bool *done) {
   cg_tensor *S = m.src;
   if (S->op != N_MATMUL || S->rank != 4 || refs(S) != (S == m.x ? 2 : 1)) return CG_OK;
   const int64_t Sq = S->shape[2], T = S->shape[3], d = n->shape[3], heads = n->shape[1], nb = n->shape[0];
-  if (Sq < 16 || T < 1 || (d != 64 && d != 128 && d != 256) || n->in[1]->shape[2] != T || S->in[0]->shape[3] != d)
+  if (Sq < 2 || T < 1 || (d != 64 && d != 128 && d != 256) || n->in[1]->shape[2] != T || S->in[0]->shape[3] != d)
     return CG_OK;
-  // Below this the three-launch path (GEMM, softmax, GEMM) is as fast and the scores are small;
-  // above it the scores of one layer run to hundreds of MB.  CG_FLAG_ATTN_ONE_PASS lifts the threshold.
-  // (bf16 mode from 256 keys on: 4 x 16 heads x 256 x 256, d = 128 - two batched GEMMs, a softmax, the copy
-  // of the transposed result and two casts, 44 us - take 21 us in one pass)
-  if (T < (f32 ? 512 : 256) && !(be->flags & CG_FLAG_ATTN_ONE_PASS)) return CG_OK;
+  // f32 products of a middling number of keys: the pass walks them one tile after the other with too few workgroups to
+  // cover for it (1 x 32 heads x 200 x 200: 37 us), GEMM + softmax + GEMM take 31; at 50 keys it is 13 us against 21,
+  // at 700 95 against 155.  bf16: one pass at every length (37 keys: 10 us against 45; 2900: 202 against 1130).
+  if (f32 && T > 128 && T < 512 && !(be->flags & CG_FLAG_ATTN_ONE_PASS)) return CG_OK;
   if (nb > 65535 || heads > 65535) return CG_OK;
   cg_tensor *q = S->in[0];
   // queries and keys both still to be rotated: one launch for the two (each alone otherwise, below)
@@ -38,7 +37,9 @@ int try_attn_prefill(cg_backend *be, cg_tensor *n, bool *done) {
     ~Held() { storage_release(s); }
   } vt_made;
   const Storage *vt_of = nullptr;
-  if (cg_tensor *kr = node_under_repeat_kv(S->in[1])) {
+  // (few keys and narrow heads: nothing but launch latency, the rotations keep the launches of their own)
+  const bool few_keys = T < (f32 ? 512 : 256) && !(be->flags & CG_FLAG_ATTN_ONE_PASS);
+  if (cg_tensor *kr = few_keys && heads * d < 512 ? nullptr : node_under_repeat_kv(S->in[1])) {
     bool paired = false;
     // ... or none at all: the projections still deferred rotate q and k in their epilogue
     if (!f32 && (d == 64 || d == 128)) TRY(try_qkv_rope_gemm(be, q, kr, node_under_repeat_kv(n->in[1]), &vt_made.s, &vt_of, &paired));
@@ -92,14 +93,37 @@ int try_attn_prefill(cg_backend *be, cg_tensor *n, bool *done) {
     a.m_st = mask->shape[3] == 1 ? 0 : mask->strides[3];
     a.m_vec = a.m_st == 1 && (uintptr_t)a.mask % 16 == 0 && a.m_sb % 4 == 0 && a.m_sh % 4 == 0 && a.m_ss % 4 == 0;
   }
-  // the kernel reads mask rows and value columns 16 bytes at a time, and (bf16) the keys from their bf16 twin
+  // The kernel reads mask rows and value columns 16 bytes at a time, and (bf16) the keys from their bf16 twin.  A mask
+  // shared by every batch and head whose rows do not allow that (a number of keys that is no multiple of four) is
+  // copied once to rows that do.
   Storage *ksh = nullptr;
   const bool twin_ok = f32 || (Kop.t->st->grow_dim < 0 && Kop.t->st->bytes % 32 == 0);
-  if ((mask && !a.m_vec) || T % 8 || !twin_ok) {
+  const bool shared_mask = mask && a.m_sb == 0 && a.m_sh == 0 && a.m_ss > 0 && a.m_st == 1 && mask->st->grow_dim < 0 && Sq <= 65535;
+  const bool pad_mask = mask && (!a.m_vec || T % 4);
+  a.m_len = (uint32_t)T;
+  if ((pad_mask && !shared_mask) || !twin_ok) {
     storage_release(n->st);
     n->st = nullptr;
     return CG_OK;
   }
+  if (pad_mask) {
+    Storage *ms = mask->st;
+    const int64_t key[4] = {mask->offset, Sq, T, a.m_ss}, pitch = (T + 63) / 64 * 64;
+    if (!ms->padded || !std::equal(key, key + 4, ms->padded_key)) {
+      storage_release(ms->padded);
+      ms->padded = nullptr;
+      TRY(dev_alloc(be, (size_t)Sq * pitch * 4, &ms->padded));
+      std::copy(key, key + 4, ms->padded_key);
+      KernelScope ks(be, "attn_mask_pad", (double)Sq * (T + pitch) * 4, 0);
+      HIPCHK(be, launch_mask_pad(be->lc(), a.mask, a.m_ss, (uint32_t)Sq, (uint32_t)T, (uint32_t)pitch, (float *)ms->padded->ptr));
+    }
+    a.mask = (const float *)ms->padded->ptr;
+    a.m_ss = pitch;
+    a.m_len = (uint32_t)pitch;
+    a.m_vec = 1;
+  }
+  const int64_t Tp = (T + 7) / 8 * 8;  // row pitch of the transposed values
+  a.vt_st = (uint32_t)Tp;
   Storage *vt = nullptr;
   bool vt_ready = false;
   const int64_t kvh = Kop.shape[1];
@@ -111,17 +135,17 @@ int try_attn_prefill(cg_backend *be, cg_tensor *n, bool *done) {
     a.k16 = (const uint16_t *)ksh->ptr + Kop.t->offset;
     // the values as the projections left them, [T, kv heads * d] read as [kv heads][T][d]: their transposed copy is there
     if (vt_made.s && vt_of == Vop.t->st && Vop.t->offset == 0 && Vop.strides[1] == d && Vop.strides[3] == kvh * d &&
-        Vop.strides[4] == 1 && (nb == 1 || Vop.strides[0] == T * kvh * d) && (size_t)nb * kvh * d * T * 2 <= vt_made.s->bytes) {
+        Vop.strides[4] == 1 && (nb == 1 || Vop.strides[0] == T * kvh * d) && (size_t)nb * kvh * d * Tp * 2 <= vt_made.s->bytes) {
       vt = vt_made.s;
       vt_made.s = nullptr;
       vt_ready = true;
     } else {
-      TRY(dev_alloc(be, (size_t)nb * kvh * d * T * 2, &vt));
+      TRY(dev_alloc(be, (size_t)nb * kvh * d * Tp * 2, &vt));
     }
   }
   if (!f32 && !vt_ready) {
     KernelScope ks(be, "transpose_cast_bf16", (double)nb * kvh * d * T * 6, 0);
-    hipError_t te = launch_transpose_cast_bf16(be->lc(), data_ptr(Vop.t), ST_F32, vt->ptr, (uint32_t)T, (uint32_t)d,
+    hipError_t te = launch_transpose_cast_bf16(be->lc(), data_ptr(Vop.t), ST_F32, vt->ptr, (uint32_t)T, (uint32_t)Tp, (uint32_t)d,
                                                Vop.strides[3], (uint32_t)nb, (uint32_t)kvh, Vop.strides[0], Vop.strides[1]);
     if (te != hipSuccess) {
       storage_release(vt);
@@ -169,7 +193,8 @@ int try_attn_prefill(cg_backend *be, cg_tensor *n, bool *done) {
   }
   {
     const double qo = 2.0 * nb * heads * Sq * d * 4, kvb = 2.0 * nb * Kop.shape[1] * T * d * 4;
-    KernelScope ks(be, "attn_prefill", qo + kvb + (mask ? (double)Sq * T * 4 : 0.0), 4.0 * nb * heads * Sq * T * d);
+    // (the records tell the plain launches from those of few keys and of mask rows copied for alignment)
+    KernelScope ks(be, T % 8 ? "attn_ragged" : few_keys ? "attn_short" : "attn_prefill", qo + kvb + (mask ? (double)Sq * T * 4 : 0.0), 4.0 * nb * heads * Sq * T * d);
     hipError_t ae = launch_attn_prefill(be->lc(), a);
     storage_release(vt);
     HIPCHK(be, ae);

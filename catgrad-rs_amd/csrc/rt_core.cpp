@@ -98,6 +98,7 @@ void storage_release(Storage *s) {
   if (!s || s->rc.fetch_sub(1) != 1) return;
   storage_release(s->shadow);
   storage_release(s->tiles);
+  storage_release(s->padded);
   cg_backend *be = s->be;
   // Safe to recycle at once: every consumer was enqueued on the backend's only stream.
   be->pool[s->bytes].push_back(s->ptr);

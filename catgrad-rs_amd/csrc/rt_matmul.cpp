@@ -622,7 +622,7 @@ int realize_matmul(cg_backend *be, cg_tensor *n, cg_tensor *addend, bool *added,
     TRY(try_attn_decode(be, n, &done));
     if (done) return CG_OK;
   }
-  if (!addend && n->dtype == CG_F32 && n->rank == 4 && n->shape[2] >= 16 && !(be->flags & CG_FLAG_NO_PATTERNS)) {
+  if (!addend && n->dtype == CG_F32 && n->rank == 4 && n->shape[2] >= 2 && !(be->flags & CG_FLAG_NO_PATTERNS)) {
     bool done = false;
     TRY(try_attn_prefill(be, n, &done));
     if (done) return CG_OK;
@@ -775,7 +775,7 @@ int realize_matmul(cg_backend *be, cg_tensor *n, cg_tensor *addend, bool *added,
       hipError_t te;
       {
         KernelScope ks(be, "transpose_cast_bf16", (double)tb0 * tb1 * N * K * (esize(g.b_stype) + 2), 0);
-        te = launch_transpose_cast_bf16(be->lc(), g.b, g.b_stype, bt->ptr, K, N, g.sbk, tb0, tb1, g.sb_b0, g.sb_b1);
+        te = launch_transpose_cast_bf16(be->lc(), g.b, g.b_stype, bt->ptr, K, K, N, g.sbk, tb0, tb1, g.sb_b0, g.sb_b1);
       }
       if (te != hipSuccess) {
         storage_release(bt);

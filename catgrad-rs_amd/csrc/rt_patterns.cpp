@@ -778,7 +778,7 @@ int try_qkv_rope_gemm(cg_backend *be, cg_tensor *rq, cg_tensor *rk, cg_tensor *v
   if (!pq || !pk || !pv || pq == pk || pq == pv || pk == pv) return CG_OK;
   const int64_t positions = rq->shape[2], seqs = rq->shape[0];
   if (rk->shape[2] != positions || rk->shape[0] != seqs || v->shape[2] != positions || v->shape[0] != seqs ||
-      pk->shape[2] != pv->shape[2] || positions % 4)
+      pk->shape[2] != pv->shape[2])
     return CG_OK;
   bool tq = false, tk = false;
   TRY(rope_tables(be, mq, &tq));
@@ -799,7 +799,7 @@ int try_qkv_rope_gemm(cg_backend *be, cg_tensor *rq, cg_tensor *rk, cg_tensor *v
     }
   }
   Storage *t = nullptr;
-  if (!st) st = dev_alloc(be, (size_t)pv->shape[1] * pv->shape[2] * 2, &t);
+  if (!st) st = dev_alloc(be, (size_t)seqs * ((positions + 7) / 8 * 8) * pv->shape[2] * 2, &t);
   if (!st) {
     req.out16[2] = (uint16_t *)t->ptr;
     req.mm[0] = pq;
