@@ -77,6 +77,13 @@ hipError_t launch_topk(const LaunchCtx &lc, const float *x, float *values, uint3
 // *flag |= 1 if any element differs (u32: bit compare, f32: IEEE ==, so NaN differs)
 hipError_t launch_compare(const LaunchCtx &lc, const void *a, const void *b, uint64_t n,
                           int is_f32, uint32_t *flag);
+// n 32-bit words of src (device) to dst (pinned host memory), both 16-byte aligned, at most TO_HOST_MAX_PIECES pieces of
+// TO_HOST_PIECE words.  Behind each piece (one at least, also when n is 0) err[0], err[1] and 1 go to the first three words
+// of its tail (pinned host memory, TO_HOST_TAIL words a piece).  done: a device word per piece, zero between launches.
+enum : uint32_t { TO_HOST_PIECE = 32768, TO_HOST_MAX_PIECES = 16, TO_HOST_TAIL = 16 };
+hipError_t launch_to_host(const LaunchCtx &lc, const void *src, void *dst, uint64_t n, const uint32_t *err, uint32_t *tail, uint32_t *done);
+// n words of src (pinned host memory) to dst (device); then 1 to *flag (pinned host memory)
+hipError_t launch_from_host(const LaunchCtx &lc, const void *src, void *dst, uint32_t n, uint32_t *flag);
 hipError_t launch_fill_u32(const LaunchCtx &lc, uint32_t *dst, uint32_t value, uint64_t n);
 // Contiguous copy of a strided view whose unit-stride axis is not the last one (a materialised
 // transpose): 64 x 64 tiles through LDS, reads along the input's unit-stride axis `j`, writes

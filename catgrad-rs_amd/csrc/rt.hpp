@@ -123,10 +123,9 @@ struct cg_tensor {
   // shared: cse_key is this node's entry in cg_backend::shared_nodes while it is still deferred
   bool const_like = false;
   std::string *cse_key = nullptr;
-  // cg_tensor_prefetch: a pinned host copy in flight (data, then the backend's error words) and the
-  // event recorded behind the copy
+  // cg_tensor_prefetch: a pinned host copy in flight: data, and in the last words of the buffer the backend's
+  // error words and the flag that says the copy has landed
   void *host_copy = nullptr;
-  hipEvent_t host_ev = nullptr;
 
   int64_t size() const {
     int64_t n = 1;
@@ -142,8 +141,12 @@ struct cg_backend {
   hipStream_t stream = nullptr;
   int n_cus = 256;
   std::string err;
-  uint32_t *d_words = nullptr;  // [0] kernel error flags, [1] compare flag
-  uint32_t *h_words = nullptr;  // pinned mirror
+  uint32_t *d_words = nullptr;  // [0] kernel error flags, [1] compare flag, [2], [3] unused, [4 ..] workgroups of a launch_to_host that are done, by piece
+  uint32_t *h_words = nullptr;  // pinned mirror of [0], [1]; [2]: the flag that says they have landed
+  // pinned buffers values pass through on their way to and from the host, made when first needed
+  char *h_out = nullptr;        // two halves, each TO_HOST_MAX_PIECES pieces and their tails
+  char *h_in = nullptr;         // HOST_IN_SLOTS slots of HOST_IN_BYTES, each ending in its flag
+  uint32_t h_in_next = 0;
   // caching allocator
   std::map<size_t, std::vector<void *>> pool;
   uint64_t pool_bytes = 0, device_bytes = 0, launches = 0;
@@ -196,9 +199,9 @@ struct cg_backend {
   // set by try_gemv_add around realize_matmul when the addend it passes is a bias vector (one row added
   // to every row of the product) instead of a tensor shaped like the product
   bool addend_is_row = false;
-  // recycled pinned buffers (PREFETCH_BYTES each) and events of cg_tensor_prefetch
-  std::vector<void *> pinned_pool;
-  std::vector<hipEvent_t> event_pool;
+  // pinned buffers (PREFETCH_BYTES each) of cg_tensor_prefetch no tensor holds any more; the copy into the
+  // last ones given back may still be in flight (its flag says)
+  std::deque<void *> pinned_pool;
   // scratch of the decode attention that divides the keys over several workgroups: partial results
   // and one counter per (batch, head); the counters are zero whenever no launch is running
   float *attn_part = nullptr;

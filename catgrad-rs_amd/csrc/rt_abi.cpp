@@ -101,34 +101,25 @@ int cg_tensor_prefetch(cg_backend *be, cg_tensor *t) {
   HIPCHK(be, hipSetDevice(be->device));
   TRY(realize(be, t));
   const size_t bytes = (size_t)t->size() * 4;
-  if (t->host_copy || bytes == 0 || bytes > PREFETCH_BYTES - 8 || esize(t->stype) != 4 || !is_contiguous(t))
+  if (t->host_copy || bytes == 0 || bytes > PREFETCH_BYTES - PREFETCH_TAIL || esize(t->stype) != 4 || !is_contiguous(t) ||
+      (uintptr_t)data_ptr(t) % 16)
     return CG_OK;  // the read will take the synchronising path
+  auto flag_of = [](void *b) { return (uint32_t *)((char *)b + PREFETCH_BYTES - PREFETCH_TAIL) + 2; };
   void *buf = nullptr;
-  hipEvent_t ev = nullptr;
-  if (!be->pinned_pool.empty()) {
-    buf = be->pinned_pool.back();
-    be->pinned_pool.pop_back();
+  if (!be->pinned_pool.empty() && __atomic_load_n(flag_of(be->pinned_pool.front()), __ATOMIC_ACQUIRE)) {
+    buf = be->pinned_pool.front();
+    be->pinned_pool.pop_front();
   } else {
     HIPCHK(be, hipHostMalloc(&buf, PREFETCH_BYTES, hipHostMallocDefault));
   }
-  if (!be->event_pool.empty()) {
-    ev = be->event_pool.back();
-    be->event_pool.pop_back();
-  } else if (hipEventCreateWithFlags(&ev, hipEventDisableTiming) != hipSuccess) {
-    be->pinned_pool.push_back(buf);
-    return fail(be, CG_ERR_DEVICE, "hipEventCreate failed");
-  }
-  hipError_t e = hipMemcpyAsync(buf, data_ptr(t), bytes, hipMemcpyDeviceToHost, be->ordered_stream());
-  if (e == hipSuccess)
-    e = hipMemcpyAsync((char *)buf + PREFETCH_BYTES - 8, be->d_words, 8, hipMemcpyDeviceToHost, be->ordered_stream());
-  if (e == hipSuccess) e = hipEventRecord(ev, be->ordered_stream());
+  *flag_of(buf) = 0;
+  const hipError_t e = launch_to_host(be->lc(), data_ptr(t), buf, bytes / 4, be->d_words, flag_of(buf) - 2, be->d_words + 4);
   if (e != hipSuccess) {
+    *flag_of(buf) = 1;
     be->pinned_pool.push_back(buf);
-    be->event_pool.push_back(ev);
     return fail(be, CG_ERR_DEVICE, hipGetErrorString(e));
   }
   t->host_copy = buf;
-  t->host_ev = ev;
   return CG_OK;
 }
 

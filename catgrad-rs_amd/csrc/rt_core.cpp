@@ -117,11 +117,12 @@ void backend_release(cg_backend *be) {
   }
   trim_pool(be);
   for (void *p : be->pinned_pool) (void)hipHostFree(p);
-  for (hipEvent_t ev : be->event_pool) (void)hipEventDestroy(ev);
   if (be->d_words) (void)hipFree(be->d_words);
   if (be->attn_part) (void)hipFree(be->attn_part);
   if (be->attn_count) (void)hipFree(be->attn_count);
   if (be->h_words) (void)hipHostFree(be->h_words);
+  if (be->h_out) (void)hipHostFree(be->h_out);
+  if (be->h_in) (void)hipHostFree(be->h_in);
   delete be->queue;  // drains and joins its thread
   be->queue = nullptr;
   noalloc_release_slot(be->device, be->noalloc_slot);
@@ -184,12 +185,7 @@ void node_release(cg_tensor *t) {
     if (n->in[1]) stack.push_back(n->in[1]);
     storage_release(n->st);
     cg_backend *be = n->be;
-    if (n->host_copy) {
-      // the copy may still be in flight: the buffer is only reused after its event has completed
-      (void)hipEventSynchronize(n->host_ev);
-      be->pinned_pool.push_back(n->host_copy);
-      be->event_pool.push_back(n->host_ev);
-    }
+    if (n->host_copy) be->pinned_pool.push_back(n->host_copy);  // (used again once its copy has landed)
     delete n;
     backend_release(be);
   }

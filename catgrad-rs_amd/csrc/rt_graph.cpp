@@ -235,13 +235,40 @@ int realize(cg_backend *be, cg_tensor *n) {
 }
 
 
+// Waits for the flag a launch_to_host sets in pinned memory: every kernel enqueued before it has ended.  Polled, which
+// sees it ~10 us sooner than a wait on the stream; should the flag not come for a long time (work of seconds is
+// queued, or the launch could not be made), the stream is waited for and asked.
+int wait_host_flag(cg_backend *be, const uint32_t *flag) {
+  for (int round = 0; round < 20000; ++round) {  // a second or so
+    for (int i = 0; i < 1000; ++i) {
+      if (__atomic_load_n(flag, __ATOMIC_ACQUIRE)) {
+        if (be->queue) HIPCHK(be, be->queue->take_error());  // a launch the queue's thread could not make
+        return CG_OK;
+      }
+#if defined(__x86_64__)
+      __builtin_ia32_pause();
+#endif
+    }
+  }
+  HIPCHK(be, hipStreamSynchronize(be->ordered_stream()));
+  if (be->queue) HIPCHK(be, be->queue->take_error());
+  return __atomic_load_n(flag, __ATOMIC_ACQUIRE) ? CG_OK : fail(be, CG_ERR_DEVICE, "a copy to the host was not made");
+}
+
+
 // wait for the stream and surface device-side error flags
 int sync_and_check(cg_backend *be) {
-  HIPCHK(be, hipMemcpyAsync(be->h_words, be->d_words, 8, hipMemcpyDeviceToHost, be->ordered_stream()));
-  if (be->queue) HIPCHK(be, be->queue->take_error());  // a launch the queue's thread could not make
-  HIPCHK(be, hipStreamSynchronize(be->ordered_stream()));
+  be->h_words[2] = 0;
+  HIPCHK(be, launch_to_host(be->lc(), nullptr, nullptr, 0, be->d_words, be->h_words, be->d_words + 4));
+  TRY(wait_host_flag(be, be->h_words + 2));
+  return check_error_words(be, be->h_words);
+}
+
+
+// what the device's error words say (words: their copy on the host, the stream idle)
+int check_error_words(cg_backend *be, const uint32_t *words) {
   cap_pool(be);
-  const uint32_t e = be->h_words[0];
+  const uint32_t e = words[0];
   if (e) {
     HIPCHK(be, launch_fill_u32(be->lc(), be->d_words, 0u, 1));
     if (e & ERRF_DIV_ZERO) return fail(be, CG_ERR_ARITH, "attempt to divide by zero");
@@ -538,7 +565,28 @@ int upload(cg_backend *be, const void *data, size_t n, const int64_t *shape, int
     return CG_OK;
   }
   hipError_t e = hipSuccess;
-  if (!narrow) {
+  if (!narrow && n * 4 <= HOST_IN_BYTES - 64 && be->queue) {
+    // a prompt's token ids, a small vector: through a slot of pinned memory, without a wait
+    const size_t tail = HOST_IN_BYTES - 64;
+    if (!be->h_in) {
+      e = hipHostMalloc((void **)&be->h_in, HOST_IN_BYTES * HOST_IN_SLOTS, hipHostMallocDefault);
+      for (size_t i = 0; i < HOST_IN_SLOTS && e == hipSuccess; ++i) *(uint32_t *)(be->h_in + i * HOST_IN_BYTES + tail) = 1;
+    }
+    if (e == hipSuccess) {
+      char *slot = be->h_in + be->h_in_next * HOST_IN_BYTES;
+      uint32_t *flag = (uint32_t *)(slot + tail);
+      st = wait_host_flag(be, flag);  // (HOST_IN_SLOTS uploads ago)
+      if (st) {
+        node_release(t);
+        return st;
+      }
+      std::memcpy(slot, data, n * 4);
+      *flag = 0;
+      e = launch_from_host(be->lc(), slot, t->st->ptr, (uint32_t)n, flag);
+      if (e != hipSuccess) *flag = 1;
+      else be->h_in_next = (be->h_in_next + 1) % HOST_IN_SLOTS;
+    }
+  } else if (!narrow) {
     e = hipMemcpyAsync(t->st->ptr, data, n * 4, hipMemcpyHostToDevice, be->ordered_stream());
     if (e == hipSuccess) e = hipStreamSynchronize(be->ordered_stream());
   } else {
@@ -586,14 +634,39 @@ int upload(cg_backend *be, const void *data, size_t n, const int64_t *shape, int
 }
 
 
+// Through pinned memory: launches of up to TO_HOST_MAX_PIECES pieces fill its two halves in turn, and each piece is
+// copied on to its destination while the device stores the next ones.
+static int download_pieces(cg_backend *be, const char *src, char *dst, size_t bytes) {
+  const size_t piece = (size_t)TO_HOST_PIECE * 4, half = piece * TO_HOST_MAX_PIECES, tails = (size_t)TO_HOST_TAIL * 4 * TO_HOST_MAX_PIECES;
+  if (!be->h_out) HIPCHK(be, hipHostMalloc((void **)&be->h_out, 2 * (half + tails), hipHostMallocDefault));
+  const size_t pieces = (bytes + piece - 1) / piece;
+  auto data = [&](size_t i) { return be->h_out + i / TO_HOST_MAX_PIECES % 2 * half + i % TO_HOST_MAX_PIECES * piece; };
+  auto words = [&](size_t i) { return (uint32_t *)(be->h_out + 2 * half) + i % (2 * TO_HOST_MAX_PIECES) * TO_HOST_TAIL; };
+  auto ask = [&](size_t first) -> int {  // for the pieces from `first` that fill one half
+    for (size_t i = first; i < std::min(pieces, first + TO_HOST_MAX_PIECES); ++i) words(i)[2] = 0;
+    const size_t len = std::min(half, bytes - first * piece);
+    HIPCHK(be, launch_to_host(be->lc(), src + first * piece, data(first), len / 4, be->d_words, words(first), be->d_words + 4));
+    return CG_OK;
+  };
+  for (size_t i = 0; i < 2 * TO_HOST_MAX_PIECES && i < pieces; i += TO_HOST_MAX_PIECES) TRY(ask(i));
+  for (size_t i = 0; i < pieces; ++i) {
+    TRY(wait_host_flag(be, words(i) + 2));
+    std::memcpy(dst + i * piece, data(i), std::min(piece, bytes - i * piece));
+    // a half that has been copied on takes the pieces two halves later
+    if ((i + 1) % TO_HOST_MAX_PIECES == 0 && i + 1 + TO_HOST_MAX_PIECES < pieces) TRY(ask(i + 1 + TO_HOST_MAX_PIECES));
+  }
+  return check_error_words(be, words(pieces - 1));
+}
+
+
 int download(cg_backend *be, cg_tensor *x, void *dst, size_t n, cg_dtype want) {
   if (!be || !x || (!dst && n)) return fail(be, CG_ERR_ARG, "null argument");
   if (x->dtype != want) return fail(be, CG_ERR_DTYPE, "to_vec: wrong dtype for this accessor");
   if ((int64_t)n != x->size()) return fail(be, CG_ERR_SHAPE, "to_vec: size mismatch");
   HIPCHK(be, hipSetDevice(be->device));
   if (x->host_copy) {  // prefetched: wait for that copy only, not for work queued behind it
-    HIPCHK(be, hipEventSynchronize(x->host_ev));
-    const uint32_t *words = (const uint32_t *)((const char *)x->host_copy + PREFETCH_BYTES - 8);
+    const uint32_t *words = (const uint32_t *)((const char *)x->host_copy + PREFETCH_BYTES - PREFETCH_TAIL);
+    TRY(wait_host_flag(be, words + 2));
     if (words[0] == 0) {
       std::memcpy(dst, x->host_copy, n * 4);
       return CG_OK;
@@ -603,11 +676,15 @@ int download(cg_backend *be, cg_tensor *x, void *dst, size_t n, cg_dtype want) {
   cg_tensor *c = nullptr;
   TRY(contiguous(be, x, &c));
   int st = CG_OK;
-  if (n) {
-    hipError_t e = hipMemcpyAsync(dst, data_ptr(c), n * 4, hipMemcpyDeviceToHost, be->ordered_stream());
-    if (e != hipSuccess) st = fail(be, CG_ERR_DEVICE, hipGetErrorString(e));
+  if (n && (uintptr_t)data_ptr(c) % 16 == 0) {
+    st = download_pieces(be, (const char *)data_ptr(c), (char *)dst, n * 4);
+  } else {
+    if (n) {
+      hipError_t e = hipMemcpyAsync(dst, data_ptr(c), n * 4, hipMemcpyDeviceToHost, be->ordered_stream());
+      if (e != hipSuccess) st = fail(be, CG_ERR_DEVICE, hipGetErrorString(e));
+    }
+    if (!st) st = sync_and_check(be);
   }
-  if (!st) st = sync_and_check(be);
   node_release(c);
   return st;
 }

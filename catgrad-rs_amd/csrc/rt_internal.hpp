@@ -38,7 +38,8 @@ using namespace cgk;
   } while (0)
 
 
-enum { PREFETCH_BYTES = 4096 };  // pinned buffer of a prefetched tensor: data + 8 bytes of error words
+enum { PREFETCH_BYTES = 4096, PREFETCH_TAIL = 16 };  // pinned buffer of a prefetched tensor: data, error words and flag
+enum : size_t { HOST_IN_BYTES = 16 << 10, HOST_IN_SLOTS = 8 };
 enum : uint32_t { F_ONE = 0x3F800000u, F_HALF = 0x3F000000u, F_E = 0x402DF854u, F_TWO = 0x40000000u };
 
 struct KernelScope;
@@ -178,6 +179,8 @@ int realize_index(cg_backend *be, cg_tensor *n);
 int realize_arange(cg_backend *be, cg_tensor *n);
 int realize(cg_backend *be, cg_tensor *n);
 int sync_and_check(cg_backend *be);
+int wait_host_flag(cg_backend *be, const uint32_t *flag);
+int check_error_words(cg_backend *be, const uint32_t *words);
 bool share_node(cg_backend *be, cg_tensor *n, cg_tensor **out);
 int finish(cg_backend *be, cg_tensor *n, cg_tensor **out);
 int run_pending_flush(cg_backend *be);

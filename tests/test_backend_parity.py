@@ -596,3 +596,20 @@ def test_one_row_matmuls_sharing_x_go_out_together(oracle, hip, hip_bf16):
         assert rep[name]["launches"] == 1, rep
         for ref, got, w in zip(r, d, ws):
             assert_close(ref, got, tol, scale=np.abs(x) @ np.abs(w.T) + 1e-6)
+
+
+# to_vec goes through pinned memory in pieces of 128 KB, sixteen to a launch: no element, the tail of a piece, whole
+# pieces, one launch and a bit, more than both halves of the buffer; small uploads share eight slots
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [1, 3, 1023, 1025, 32767, 32768, 32769, 16 * 32768, 16 * 32768 + 5, 33 * 32768 + 1021, 64 * 32768])
+def test_values_to_and_from_the_host(hip, n):
+    g = np.random.default_rng(n)
+    a = g.integers(0, 2 ** 32, n, dtype=np.uint32)
+    t = hip.ndarray_from_vec_u32(a, [n])
+    assert np.array_equal(hip.to_vec(t), a)
+    if n > 1:   # a view that starts off a 16-byte boundary
+        assert np.array_equal(hip.to_vec(hip.slice(t, 0, 1, n - 1)), a[1:])
+    many = [g.integers(0, 2 ** 32, min(n, 4000), dtype=np.uint32) for _ in range(20)]
+    kept = [hip.prefetch(hip.ndarray_from_vec_u32(m, [m.size])) for m in many]
+    for m, t in zip(many, kept):
+        assert np.array_equal(hip.to_vec(t), m)
