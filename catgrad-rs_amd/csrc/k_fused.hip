@@ -293,6 +293,175 @@ hipError_t launch_softmax(const LaunchCtx &lc, const SoftmaxDesc &d) {
   return hipGetLastError();
 }
 
+// ---- the largest softmax value of a row (and its column) ----------------------------------------------------
+// max(softmax(x)), what a classifier reports as the confidence of its choice, without the probabilities ever being
+// stored: exp(max - max) / sum exp(x - max) in one pass over x with a running maximum; the same pass finds the column of
+// the largest x when argmax(x) is asked for as well.  Bound by reading x once: 4096 x 4096 f32 197 us in four launches
+// (the exponentials written and read twice) -> 18.  Rows of any length and alignment: 16-byte loads that need no
+// alignment, a scalar tail.  A wave to a row of up to 1024 values, a workgroup to a longer one, several workgroups
+// when there are fewer rows than CUs.
+struct RowBest {  // what is known of a part of a row
+  float xm = -INFINITY, s = 0.f;       // largest value (NaN ignored), sum of exp(x - max(xm, f32::MIN))
+  uint32_t key = 0, col = 0;           // f32::total_cmp order of the largest value as an unsigned word, its (last) column
+  __device__ __forceinline__ void merge(const RowBest &o) {
+    const float m = fmaxf(xm, -3.40282347e+38f), mo = fmaxf(o.xm, -3.40282347e+38f), mn = fmaxf(m, mo);
+    s = s * expf(m - mn) + o.s * expf(mo - mn);
+    xm = fmaxf(xm, o.xm);
+    if (o.key > key || (o.key == key && o.col > col)) { key = o.key; col = o.col; }
+  }
+  // what the 64 lanes of a wave know together: one rescaling of each lane's sum, the rest maxima and a sum through DPP
+  __device__ __forceinline__ void merge_wave() {
+    const int32_t k = wave_max_i32(total_key_f(xm));  // (xm is no NaN)
+    const float all = __int_as_float(k ^ (int32_t)((uint32_t)(k >> 31) >> 1));
+    s = wave_sum(s * expf(fmaxf(xm, -3.40282347e+38f) - fmaxf(all, -3.40282347e+38f)));
+    xm = all;
+    const uint32_t best_key = (uint32_t)wave_max_i32((int32_t)(key ^ 0x80000000u)) ^ 0x80000000u;
+    col = (uint32_t)wave_max_i32(key == best_key ? (int32_t)col : 0);
+    key = best_key;
+  }
+  __device__ __forceinline__ void store(float *p) const {
+    p[0] = xm; p[1] = s; p[2] = __uint_as_float(key); p[3] = __uint_as_float(col);
+  }
+  __device__ __forceinline__ void load(const float *p) {
+    xm = p[0]; s = p[1]; key = __float_as_uint(p[2]); col = __float_as_uint(p[3]);
+  }
+  // fold(f32::MIN, f32::max) over exp(x - m) / s: no value of x above -inf leaves 0 / s, a NaN anywhere f32::MIN
+  __device__ __forceinline__ float best() const {
+    const float r = (xm >= -3.40282347e+38f ? 1.0f : 0.0f) / s;
+    return r == r ? r : -3.40282347e+38f;
+  }
+};
+
+template <typename T, int TPR>
+__global__ void __launch_bounds__(256) softmax_best_kernel(SoftmaxBestDesc d) {
+  constexpr int W = sizeof(T) == 4 ? 4 : 8, U = sizeof(T) == 4 ? 4 : 2, RPB = 256 / TPR;
+  __shared__ float part[4][4];
+  const uint32_t rc = blockIdx.x * RPB + (RPB > 1 ? threadIdx.x / TPR : 0), t = threadIdx.x % TPR;
+  const uint32_t row = rc / d.chunks, chunk = rc - row * d.chunks;
+  RowBest b;
+  if (row < d.rows) {
+    const T *x = (const T *)d.x + (int64_t)row * d.x_row_stride;
+    const uint32_t c_begin = chunk * d.chunk_len, c_end = min(d.n, c_begin + d.chunk_len);
+    float m = -3.40282347e+38f;
+    for (uint32_t c0 = c_begin + t * W; c0 < c_end; c0 += TPR * W * U) {
+      float v[U][W];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const uint32_t c = c0 + u * TPR * W;
+        if (c + W <= c_end) {
+          uint4 q;
+          __builtin_memcpy(&q, __builtin_assume_aligned(x + c, sizeof(T)), 16);
+          const uint32_t h[4] = {q.x, q.y, q.z, q.w};
+          if constexpr (sizeof(T) == 4) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) v[u][j] = __uint_as_float(h[j]);
+          } else {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+              v[u][2 * j] = __uint_as_float(h[j] << 16);
+              v[u][2 * j + 1] = __uint_as_float(h[j] & 0xFFFF0000u);
+            }
+          }
+        } else {
+#pragma unroll
+          for (int j = 0; j < W; ++j) {
+            v[u][j] = -INFINITY;
+            if (c + j < c_end) {
+              if constexpr (sizeof(T) == 4) v[u][j] = x[c + j];
+              else v[u][j] = __uint_as_float((uint32_t)x[c + j] << 16);
+            }
+          }
+        }
+      }
+      float gm = -INFINITY;
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int j = 0; j < W; ++j) gm = fmaxf(gm, v[u][j]);
+      b.xm = fmaxf(b.xm, gm);
+      const float mn = fmaxf(m, gm);
+      b.s *= expf(m - mn);
+      m = mn;
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int j = 0; j < W; ++j) {
+          b.s += expf(v[u][j] - m);
+          if (d.arg) {  // a thread meets its columns in increasing order: "not smaller" replaces
+            const uint32_t w = __float_as_uint(v[u][j]), o = w ^ ((uint32_t)((int32_t)w >> 31) | 0x80000000u);
+            const uint32_t c = c0 + u * TPR * W + j;
+            const bool take = o >= b.key && c < c_end;
+            b.key = take ? o : b.key;
+            b.col = take ? c : b.col;
+          }
+        }
+    }
+  }
+  b.merge_wave();
+  if constexpr (RPB == 1) {
+    if ((threadIdx.x & 63) == 0) b.store(part[threadIdx.x >> 6]);
+    __syncthreads();
+    if (threadIdx.x == 0)
+      for (int w = 1; w < 4; ++w) {
+        RowBest o;
+        o.load(part[w]);
+        b.merge(o);
+      }
+  }
+  if (t == 0 && row < d.rows) {
+    if (d.chunks > 1) {
+      b.store(d.part + (size_t)rc * 4);
+    } else {
+      d.best[row] = b.best();
+      if (d.arg) d.arg[row] = b.col;
+    }
+  }
+}
+
+// one wave per row: the records of its chunks
+__global__ void __launch_bounds__(64) softmax_best_merge_kernel(SoftmaxBestDesc d) {
+  RowBest b;
+  for (uint32_t c = threadIdx.x; c < d.chunks; c += 64) {
+    RowBest o;
+    o.load(d.part + ((size_t)blockIdx.x * d.chunks + c) * 4);
+    b.merge(o);
+  }
+  b.merge_wave();
+  if (threadIdx.x == 0) {
+    d.best[blockIdx.x] = b.best();
+    if (d.arg) d.arg[blockIdx.x] = b.col;
+  }
+}
+
+// fewer rows than CUs and long rows: every row is cut so that about two workgroups come to a CU, 2048 values each at least
+uint32_t softmax_best_chunks(const LaunchCtx &lc, uint32_t rows, uint32_t n) {
+  if (!rows || rows >= (uint32_t)lc.n_cus || n < 8192) return 1;
+  const uint32_t chunks = (uint32_t)lc.n_cus * 2 / rows;
+  return chunks < n / 2048 ? chunks : n / 2048;
+}
+
+hipError_t launch_softmax_best(const LaunchCtx &lc, const SoftmaxBestDesc &in) {
+  if (!in.rows || !in.n) return hipSuccess;
+  SoftmaxBestDesc d = in;
+  if (!d.chunks || !d.best || (d.chunks > 1 && !d.part)) return hipErrorInvalidValue;
+  d.chunk_len = ((d.n + d.chunks - 1) / d.chunks + 15) / 16 * 16;
+  const bool wave = d.chunks == 1 && d.n <= 1024;
+  const unsigned grid = wave ? (d.rows + 3) / 4 : d.rows * d.chunks;
+  if (d.x_bf16) {
+    if (wave) CG_LAUNCH(lc, (softmax_best_kernel<uint16_t, 64>), grid, 256, d);
+    else CG_LAUNCH(lc, (softmax_best_kernel<uint16_t, 256>), grid, 256, d);
+  } else {
+    if (wave) CG_LAUNCH(lc, (softmax_best_kernel<float, 64>), grid, 256, d);
+    else CG_LAUNCH(lc, (softmax_best_kernel<float, 256>), grid, 256, d);
+  }
+  if (d.chunks > 1) {
+    LaunchCtx untimed = lc;  // the events stay with the pass over x
+    untimed.ev_start = untimed.ev_stop = nullptr;
+    CG_LAUNCH(untimed, softmax_best_merge_kernel, d.rows, 64, d);
+  }
+  return hipGetLastError();
+}
+
 // ---- one-query attention ----------------------------------------------------------------------------------
 // The decode step of models/llama.rs:77-112: scores = q . K^T, / sqrt(d), + mask, softmax, . V, for one
 // query row per head.  One workgroup per (batch, head); LPK lanes share a key/value row (16 bytes

@@ -148,6 +148,21 @@ struct SoftmaxDesc {
 };
 hipError_t launch_softmax(const LaunchCtx &lc, const SoftmaxDesc &d);
 
+// best[r] = max_j softmax(x[r, :])[j], and arg[r] = argmax(x[r, :]) when arg is not null; rows of n unit-stride values
+// (f32, or bf16 when x_bf16), row r at x + r * x_row_stride, any alignment.  chunks (softmax_best_chunks) > 1: part holds
+// rows * chunks * 4 floats of scratch, 16-byte aligned.
+struct SoftmaxBestDesc {
+  const void *x;
+  int64_t x_row_stride;
+  float *best;
+  uint32_t *arg;
+  float *part;
+  uint32_t rows, n, chunks, chunk_len;  // chunk_len: set by the launcher
+  int32_t x_bf16;
+};
+uint32_t softmax_best_chunks(const LaunchCtx &lc, uint32_t rows, uint32_t n);
+hipError_t launch_softmax_best(const LaunchCtx &lc, const SoftmaxBestDesc &d);
+
 struct RopeDesc {
   const float *x, *cos, *sin;
   float *out;            // [b, h, s, dim] through o_sb / o_sh / o_ss (e.g. a slot of the KV cache)

@@ -111,6 +111,7 @@ struct cg_tensor {
   uint32_t cbits = 0;
   bool gemv_candidate = false;  // listed in cg_backend::gemv_candidates (a weak reference)
   bool gemm_candidate = false;  // listed in cg_backend::gemm_candidates (a weak reference)
+  bool argmax_candidate = false;  // listed in cg_backend::argmax_candidates (a weak reference)
   // `linear(x) + bias`: on a deferred few-row product, the add that reads it next to a broadcast bias
   // vector (a weak reference, cleared when that add lets go of its inputs); on the add, the product
   cg_tensor *bias_user = nullptr, *bias_of = nullptr;
@@ -166,6 +167,8 @@ struct cg_backend {
   std::vector<cg_tensor *> gemv_candidates;
   // the same for many-row products in bf16 mode (q/k/v of a prefill as one grouped GEMM)
   std::vector<cg_tensor *> gemm_candidates;
+  // deferred argmax nodes (weak references): the pass that finds the largest softmax value of the same rows takes one along
+  std::vector<cg_tensor *> argmax_candidates;
   hipEvent_t cur_start = nullptr, cur_stop = nullptr;  // set while a traced launch is issued
   // arange(n) is immutable and models ask for the same few n over and over (masks, RoPE tables of
   // every layer): one node per n, realised once

@@ -453,6 +453,11 @@ static int reduce(cg_backend *be, cg_tensor *x, cg_tensor **out, int f_kind, int
   n->op = N_REDUCE;
   n->p0 = x->dtype == CG_F32 ? f_kind : u_kind;
   n->in[0] = retain(x);
+  if (n->p0 == R_ARGMAX_F && !(be->flags & (CG_FLAG_EAGER | CG_FLAG_NO_PATTERNS))) {
+    if (be->argmax_candidates.size() >= 64) forget_argmax_candidate(be->argmax_candidates.front());
+    be->argmax_candidates.push_back(n);
+    n->argmax_candidate = true;
+  }
   return finish(be, n, out);
 }
 // ndarray.rs:455-467, 522-529, 469-493

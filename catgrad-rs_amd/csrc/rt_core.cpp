@@ -168,6 +168,18 @@ void forget_gemm_candidate(cg_tensor *n) {
 }
 
 
+void forget_argmax_candidate(cg_tensor *n) {
+  auto &v = n->be->argmax_candidates;
+  for (size_t i = 0; i < v.size(); ++i)
+    if (v[i] == n) {
+      v[i] = v.back();
+      v.pop_back();
+      break;
+    }
+  n->argmax_candidate = false;
+}
+
+
 void node_release(cg_tensor *t) {
   if (!t || t->rc.fetch_sub(1) != 1) return;  // the common case takes no allocation
   std::vector<cg_tensor *> stack{t};
@@ -177,6 +189,7 @@ void node_release(cg_tensor *t) {
     if (n != t && n->rc.fetch_sub(1) != 1) continue;
     if (n->gemv_candidate) forget_gemv_candidate(n);
     if (n->gemm_candidate) forget_gemm_candidate(n);
+    if (n->argmax_candidate) forget_argmax_candidate(n);
     forget_shared(n);
     if (n->bias_of && n->bias_of->bias_user == n) n->bias_of->bias_user = nullptr;  // its inputs are still alive here
     if (n->glu_of && n->glu_of->glu_user == n) n->glu_of->glu_user = nullptr;

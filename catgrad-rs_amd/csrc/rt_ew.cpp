@@ -383,9 +383,63 @@ bool rows_layout(const cg_tensor *t, int64_t *row_stride) {
 }
 
 
+// max(softmax(x)) where nobody else reads the probabilities: one pass over x, which also answers an argmax(x) that is
+// still deferred (launch_softmax_best)
+static int try_softmax_best(cg_backend *be, cg_tensor *n, bool *done) {
+  cg_tensor *p = n->in[0];
+  SoftmaxMatch m;
+  if (p->op == N_REAL || refs(p) != 1 || !match_softmax(p, &m, (int64_t)1 << 31) || m.src != m.x) return CG_OK;
+  cg_tensor *x = m.x;
+  TRY(realize(be, x));
+  int64_t rs = 0;
+  if ((x->stype != ST_F32 && x->stype != ST_BF16) || !rows_layout(x, &rs)) return CG_OK;
+  const int64_t cols = x->shape[x->rank - 1], rows = x->size() / cols;
+  if (rows < 1 || rows > 0x7FFFFFFF / 1024) return CG_OK;
+  cg_tensor *arg = nullptr;
+  for (cg_tensor *c : be->argmax_candidates)
+    if (c->op == N_REDUCE && c->in[0] == x) arg = c;
+  SoftmaxBestDesc d;
+  std::memset(&d, 0, sizeof(d));
+  d.x = data_ptr(x);
+  d.x_bf16 = x->stype == ST_BF16;
+  d.x_row_stride = rs;
+  d.rows = (uint32_t)rows;
+  d.n = (uint32_t)cols;
+  d.chunks = softmax_best_chunks(be->lc(), d.rows, d.n);
+  Storage *part = nullptr;
+  if (d.chunks > 1) TRY(dev_alloc(be, (size_t)rows * d.chunks * 16, &part));
+  int st = alloc_result(be, n, ST_F32);
+  if (!st && arg) st = alloc_result(be, arg, ST_U32);
+  if (!st) {
+    d.best = (float *)n->st->ptr;
+    d.arg = arg ? (uint32_t *)arg->st->ptr : nullptr;
+    d.part = part ? (float *)part->ptr : nullptr;
+    KernelScope ks(be, "softmax_best", (double)x->size() * esize(x->stype) + (double)rows * (arg ? 8 : 4), 0);
+    const hipError_t e = launch_softmax_best(be->lc(), d);
+    if (e != hipSuccess) st = fail(be, CG_ERR_DEVICE, hipGetErrorString(e));
+  }
+  storage_release(part);
+  if (st) return st;
+  for (cg_tensor *t : {arg, n}) {  // (n last: it holds the graph above x)
+    if (!t) continue;
+    if (t->argmax_candidate) forget_argmax_candidate(t);
+    t->op = N_REAL;
+    drop_inputs(t);
+  }
+  *done = true;
+  return CG_OK;
+}
+
+
 int realize_reduce(cg_backend *be, cg_tensor *n) {
   cg_tensor *x = n->in[0];
   const int kind = (int)n->p0;
+  if (n->argmax_candidate) forget_argmax_candidate(n);
+  if (kind == R_MAX_F && !(be->flags & CG_FLAG_NO_PATTERNS)) {
+    bool done = false;
+    TRY(try_softmax_best(be, n, &done));
+    if (done) return CG_OK;
+  }
   // Greedy decoding (llm/utils.rs: argmax of the last position's logits): the row is a one-row product that is
   // still deferred.  Its launch keeps, per wave, the largest value it stores; the argmax merges those records
   // instead of reading 128 K logits back with two launches of its own.

@@ -109,7 +109,8 @@ int gemm_readers(cg_backend *be, const cg_tensor *n, bool *all);
 int as_rows(cg_backend *be, cg_tensor *t, cg_tensor **out, int64_t *row_stride);
 void finish_fused(cg_tensor *n);
 int twin_for_result(cg_backend *be, cg_tensor *n, uint16_t **out);
-bool match_softmax(cg_tensor *root, SoftmaxMatch *m);
+bool match_softmax(cg_tensor *root, SoftmaxMatch *m, int64_t max_n = 16384);
+void forget_argmax_candidate(cg_tensor *n);
 int try_softmax(cg_backend *be, cg_tensor *root, bool *done);
 bool match_rmsnorm(cg_tensor *root, RmsNormMatch *m);
 int gamma_row_vector(cg_backend *be, cg_tensor *gb, bool *ok);

@@ -151,7 +151,7 @@ int twin_for_result(cg_backend *be, cg_tensor *n, uint16_t **out) {
 }
 
 
-bool match_softmax(cg_tensor *root, SoftmaxMatch *m) {
+bool match_softmax(cg_tensor *root, SoftmaxMatch *m, int64_t max_n) {
   if (root->dtype != CG_F32 || root->rank == 0 || !is_bin(root, E_DIV_F)) return false;
   cg_tensor *ex = root->in[0], *bs = root->in[1];
   if (!is_bin(ex, E_POW_F) || refs(ex) != 2 || !is_constf(ex->in[0], F_E)) return false;
@@ -165,7 +165,7 @@ bool match_softmax(cg_tensor *root, SoftmaxMatch *m) {
   cg_tensor *mx = bm->in[0];
   if (mx->op != N_REDUCE || mx->p0 != R_MAX_F || refs(mx) != 1 || mx->in[0] != x) return false;
   const int64_t n = root->shape[root->rank - 1];
-  if (n == 0 || n > 16384 || root->size() >= ((int64_t)1 << 31)) return false;
+  if (n == 0 || n > max_n || root->size() >= ((int64_t)1 << 31)) return false;
   m->src = x;
   m->x = x;
   if (x->op != N_REAL && refs(x) == 2) {

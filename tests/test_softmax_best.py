@@ -1,0 +1,51 @@
+"""max(softmax(x)) and argmax(x) of the same rows in one pass (nn/mod.rs:162-171, ndarray.rs:455-480): rows of every length
+and alignment, a wave / a workgroup / several workgroups to a row, and the values the folds treat specially."""
+import numpy as np
+import pytest
+
+import vectors
+
+lang, nn = vectors.cg.lang, vectors.cg.nn
+
+
+def best(b, x):
+    return lang.max(b, nn.softmax(b, x)), lang.argmax(b, x)
+
+
+def run(be, x):
+    if be.name.startswith("hip"):
+        be.launch_counts(reset=True)
+    out = vectors.run(be, best, 2, x)
+    return out, (be.launch_counts(reset=True) if be.name.startswith("hip") else {})
+
+
+# a few values; both sides of a wave's 1024; a piece of 8 or 16 and a bit; rows that start off a 16-byte boundary; few long
+# rows (chunks) with a last chunk that is short
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", [(1, 1), (3, 2), (5, 63), (7, 1024), (6, 1025), (300, 513), (2, 3, 4099), (257, 2049), (1, 8191),
+                                   (1, 8192), (3, 20001), (1, 128256), (100, 8195)])
+def test_best_of_rows(oracle, hip, hip_bf16, shape):
+    g = np.random.default_rng(shape[-1])
+    x = vectors.bf16_round((g.standard_normal(shape) * 3).astype(np.float32))     # (bf16 values: ties at the top are common)
+    (p, a), _ = run(oracle, x)
+    for be in (hip, hip_bf16):
+        (gp, ga), counts = run(be, x)
+        assert counts.get("softmax_best") == 1 and not any(n.startswith(("reduce", "row_fused")) for n in counts), counts
+        # one f32 exponential and a sum of n of them on both sides: 1e-5
+        assert np.allclose(gp, p, rtol=1e-5, atol=0) and np.array_equal(ga, a)
+
+
+@pytest.mark.gpu
+def test_best_of_rows_with_special_values(oracle, hip):
+    x = np.random.default_rng(3).standard_normal((9, 70)).astype(np.float32)
+    x[0, 5] = np.inf
+    x[1, 69] = np.nan
+    x[2] = -np.inf
+    x[3, :69] = -np.inf
+    x[4] = np.nan
+    x[5] = 2.5
+    x[6, 3], x[6, 66] = 90.0, -3e38
+    x[7] = np.finfo(np.float32).min
+    (p, a), _ = run(oracle, x)
+    (gp, ga), _ = run(hip, x)
+    assert np.allclose(gp, p, rtol=1e-5, atol=0, equal_nan=True) and np.array_equal(ga, a), (p, gp, a, ga)
