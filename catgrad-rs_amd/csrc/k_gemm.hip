@@ -514,23 +514,29 @@ template <int N> __device__ __forceinline__ void wait_vmcnt() {
 // different banks), and the MFMA operand - eight consecutive k of one column per lane - comes out of LDS through
 // the transposing read (ds_read_b64_tr_b16: the 16 lanes of a group hand in four rows of 16 columns, lane c
 // receives column c of the four rows), two reads per fragment.
-template <int BM_, int BN_, int WR, int WC, bool EPI, int NS, bool DUAL = false, bool BKM = false, bool ROPE = false>
-__global__ void __launch_bounds__(WR *WC * 64) gemm_bf16_dma_kernel(GemmDesc g) {
-  constexpr int NW = WR * WC, BK = 64;
-  static_assert(!ROPE || (BN_ % 64 == 0 && !EPI && !DUAL && !BKM && (BM_ * BN_ / 4) % (WR * WC * 64) == 0),
+// KG: the wavefronts form KG groups of WR x WC, each with the whole tile and every KG-th part of a k-step; the groups'
+// sums meet in LDS at the end.  For tiles of a few rows against weights nobody has touched (a prompt of 17 to 128
+// tokens), which are bound by the stream of weights: narrow tiles put a workgroup on every CU, and more wavefronts than
+// such a tile has MFMA columns for share the issue of its loads (a global_load_lds costs its wave 55 - 120 cycles).
+template <int BM_, int BN_, int WR, int WC, bool EPI, int NS, bool DUAL = false, bool BKM = false, bool ROPE = false, int KG = 1>
+__global__ void __launch_bounds__(WR *WC *KG * 64) gemm_bf16_dma_kernel(GemmDesc g) {
+  constexpr int NW = WR * WC * KG, BK = 64;
+  static_assert(!ROPE || (BN_ % 64 == 0 && !EPI && !DUAL && !BKM && (BM_ * BN_ / 4) % (NW * 64) == 0),
                 "rotated heads: whole heads of 64 columns per tile");
+  static_assert(KG == 1 || (!BKM && 4 % KG == 0 && (KG - 1) * BM_ * BN_ * 4 <= NS * (BM_ + BN_) * 128), "k-groups");
   static_assert(!BKM || (!EPI && !DUAL && (BM_ / 8) % ((BM_ + BN_) / 8 / (WR * WC)) == 0), "k-major B: the plain product");
   constexpr int WM = BM_ / WR, WN = BN_ / WC, TM = WM / 32, TN = WN / 32;
   constexpr int BNO = DUAL ? BN_ / 2 : BN_;    // output columns of a tile
   constexpr int OC = BNO / WC, TNH = OC / 32;  // DUAL: output columns per wave, fragments per product
-  static_assert(!DUAL || (EPI && BN_ == 256 && TN == 2 * TNH), "stacked gate / up tile");
+  static_assert(!DUAL || (EPI && OC % 32 == 0 && TN == 2 * TNH), "stacked gate / up tile");
   constexpr int LPW = (BM_ + BN_) / 8 / NW;   // 1 KB loads per wave per stage
   constexpr int STAGE = (BM_ + BN_) * BK * 2;  // bytes
   extern __shared__ __attribute__((aligned(16))) uint16_t dma_smem[];
   warm_kernel_arguments<sizeof(GemmDesc)>();
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = wave / WC, wn = wave % WC;
+  const int kgrp = KG > 1 ? wave / (WR * WC) : 0, wt = KG > 1 ? wave % (WR * WC) : wave;
+  const int wm = wt / WC, wn = wt % WC;
   const uint32_t tiles_m = (g.M + BM_ - 1) / BM_, tiles_n = (g.N + BNO - 1) / BNO;
   const uint32_t per_batch = tiles_m * tiles_n, batch = g.nb0 * g.nb1;
   // Workgroups are dealt round-robin to the 8 XCDs (one L2 each): give every XCD a contiguous
@@ -633,12 +639,14 @@ __global__ void __launch_bounds__(WR *WC * 64) gemm_bf16_dma_kernel(GemmDesc g) 
         }
       }
     };
-    frags(0, 0);
+    constexpr int KS = BK / 16 / KG;  // k-slices of this wave's group
+    const int k_first = KG > 1 ? kgrp * KS : 0;
+    frags(k_first, 0);
     // the wave that is in its MFMA phase goes first when both waves of a SIMD have something to issue
     __builtin_amdgcn_s_setprio(1);
 #pragma unroll
-    for (int ks = 0; ks < BK / 16; ++ks) {
-      if (ks + 1 < BK / 16) frags(ks + 1, (ks + 1) & 1);
+    for (int ks = 0; ks < KS; ++ks) {
+      if (ks + 1 < KS) frags(k_first + ks + 1, (ks + 1) & 1);
 #pragma unroll
       for (int i = 0; i < TM; ++i)
 #pragma unroll
@@ -650,7 +658,7 @@ __global__ void __launch_bounds__(WR *WC * 64) gemm_bf16_dma_kernel(GemmDesc g) 
       // Issue order within the slice: one LDS read behind each of the first MFMAs, so that the reads of
       // the next slice go out while the matrix pipe is busy instead of in a block during which it drains
       // (measured on 4096^3: 0.93 -> 1.06 PFLOP/s).
-      if (ks + 1 < BK / 16) {
+      if (ks + 1 < KS) {
         constexpr int READS = TM + TN < TM * TN ? TM + TN : TM * TN;
 #pragma unroll
         for (int q = 0; q < READS; ++q) {
@@ -686,6 +694,31 @@ __global__ void __launch_bounds__(WR *WC * 64) gemm_bf16_dma_kernel(GemmDesc g) 
   if (g.clock_ticks && tid == 0) {
     atomicAdd(g.clock_ticks, __builtin_amdgcn_s_memtime() - tick0);
     atomicAdd(g.clock_ticks + 1, __builtin_amdgcn_s_memrealtime() - real0);
+  }
+  if constexpr (KG > 1) {
+    float *sums = (float *)dma_smem;
+    __syncthreads();  // every wave is done with the last stage
+    if (kgrp) {
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+          for (int e = 0; e < 16; ++e) sums[((((kgrp - 1) * WR * WC + wt) * TM + i) * TN + j) * 1024 + e * 64 + lane] = acc[i][j][e];
+    }
+    __syncthreads();
+    if (kgrp == 0) {
+#pragma unroll
+      for (int k = 1; k < KG; ++k)
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+          for (int j = 0; j < TN; ++j)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) acc[i][j][e] += sums[((((k - 1) * WR * WC + wt) * TM + i) * TN + j) * 1024 + e * 64 + lane];
+    } else if (!ROPE) {
+      return;
+    }
   }
   if constexpr (EPI) {
     // acc[i][j][e] = C[m0 + wm * WM + i * 32 + (lane & 31)][n0 + (this fragment's columns) + (e >> 2) * 8 + half * 4 + (e & 3)]:
@@ -764,6 +797,7 @@ __global__ void __launch_bounds__(WR *WC * 64) gemm_bf16_dma_kernel(GemmDesc g) 
       }
       float *tile = (float *)dma_smem;
       __syncthreads();  // every wave is done with the last stage
+      if (kgrp == 0)
 #pragma unroll
       for (int i = 0; i < TM; ++i)
 #pragma unroll
@@ -803,6 +837,7 @@ __global__ void __launch_bounds__(WR *WC * 64) gemm_bf16_dma_kernel(GemmDesc g) 
       }
       return;
     }
+    if (KG > 1 && kgrp) return;
     if (role == 2) {  // the values: also as bf16 [sequence][head][hd][position], four consecutive positions per store
       const uint32_t Sp = (S + 7) & ~7u;  // (rows of positions end on a 16-byte boundary, zeros past the last)
 #pragma unroll
@@ -860,18 +895,18 @@ __global__ void __launch_bounds__(WR *WC * 64) gemm_bf16_dma_kernel(GemmDesc g) 
     }
 }
 
-template <int BM_, int BN_, int WR, int WC, bool EPI = false, int NS = 2, bool DUAL = false, bool BKM = false, bool ROPE = false>
+template <int BM_, int BN_, int WR, int WC, bool EPI = false, int NS = 2, bool DUAL = false, bool BKM = false, bool ROPE = false, int KG = 1>
 static hipError_t launch_gemm_dma(const LaunchCtx &lc, const GemmDesc &g, uint32_t grid) {
   // (ROPE: the f32 tile is exchanged through LDS at the end, BN_ + 8 floats per row)
   constexpr int stages = NS * (BM_ + BN_) * 64 * 2, smem = ROPE && BM_ * (BN_ + 8) * 4 > stages ? BM_ * (BN_ + 8) * 4 : stages;
   static bool configured = false;  // one attribute call per kernel and process
   if (!configured) {
-    hipError_t e = hipFuncSetAttribute((const void *)gemm_bf16_dma_kernel<BM_, BN_, WR, WC, EPI, NS, DUAL, BKM, ROPE>,
+    hipError_t e = hipFuncSetAttribute((const void *)gemm_bf16_dma_kernel<BM_, BN_, WR, WC, EPI, NS, DUAL, BKM, ROPE, KG>,
                                        hipFuncAttributeMaxDynamicSharedMemorySize, smem);
     if (e != hipSuccess) return e;
     configured = true;
   }
-  cg_launch(lc, gemm_bf16_dma_kernel<BM_, BN_, WR, WC, EPI, NS, DUAL, BKM, ROPE>, dim3(grid), dim3(WR * WC * 64), smem, g);
+  cg_launch(lc, gemm_bf16_dma_kernel<BM_, BN_, WR, WC, EPI, NS, DUAL, BKM, ROPE, KG>, dim3(grid), dim3(WR * WC * KG * 64), smem, g);
   return hipGetLastError();
 }
 
@@ -2564,7 +2599,7 @@ static void launch_rowdot(const LaunchCtx &lc, const GemmDesc &g, int bv, int av
 
 // the direct-to-LDS kernel: both operands unit-stride along k, K (and each split) a multiple of 64
 static bool gemm_dma_ok(const GemmDesc &g) {
-  return g.sak == 1 && g.sbk == 1 && g.K % 64 == 0 && g.K >= 64 && g.M >= 64 && g.N >= 64;
+  return g.sak == 1 && g.sbk == 1 && g.K % 64 == 0 && g.K >= 64 && g.M > GEMV_PRO_MAX_ROWS && g.N >= 64;
 }
 
 // B [K, N] with unit stride along n, used as it lies by the k-major form of the direct-to-LDS kernel
@@ -2590,7 +2625,7 @@ bool gemm_epilogue_ok(const GemmDesc &g) {
 bool gemm_rope_epilogue_ok(const LaunchCtx &lc, const GemmDesc &g) {
   if (!g.rope_s || !g.n_group || !gemm_epilogue_ok(g)) return false;
   if (g.rope_hd != 64 && g.rope_hd != 128) return false;
-  if (g.nb0 * g.nb1 != 1 || g.glu_gate || g.c16 || g.dual_b || g.M % g.rope_s || g.M < 64) return false;
+  if (g.nb0 * g.nb1 != 1 || g.glu_gate || g.c16 || g.dual_b || g.M % g.rope_s || g.M <= GEMV_PRO_MAX_ROWS) return false;
   bool grp256 = true;
   for (uint32_t p = 0; p < g.n_group; ++p) {
     if (g.grp_n[p] % 128) return false;
@@ -2603,7 +2638,7 @@ bool gemm_rope_epilogue_ok(const LaunchCtx &lc, const GemmDesc &g) {
       return false;
     }
   }
-  // launch_matmul's tiles of 128 rows have this epilogue (128 columns, or 64 - for heads of 64 - where those are
+  // launch_matmul's tiles of 64 and 128 rows have this epilogue (128 columns, or 64 - for heads of 64 - where those are
   // too few for the CUs); the 256 x 256 tile of the largest problems has not
   const uint64_t t256 = (uint64_t)((g.M + 255) / 256) * ((g.N + 255) / 256);
   if (t256 >= (uint64_t)lc.n_cus && grp256) return false;
@@ -2659,6 +2694,11 @@ uint32_t gemm_split_k(const LaunchCtx &lc, const GemmDesc &g) {
     if (g.M <= 8 || g.b_index || !g.K) return 1;
     while (tiles * splits * 2 <= (uint64_t)lc.n_cus && g.K / (splits * 2) >= 256 && splits < 16) splits *= 2;
     return splits;
+  }
+  if (gemm_dma_ok(g) && g.M <= 64) {  // tiles of 64 x 64: a workgroup to every CU, four k-steps at least to each
+    const uint64_t t64 = (uint64_t)((g.N + 63) / 64) * batch;
+    while (t64 * splits * 2 <= (uint64_t)lc.n_cus && g.K / (splits * 2) >= 256 && splits < 8) splits *= 2;
+    return g.N <= 64 && ((uint64_t)batch * g.M * g.N) % 4 ? 1 : splits;
   }
   // (a narrow product - the router of a MoE prefill, 1024 x 60 x 2048: 16 tiles of 64 x 64 walking all of k, 27 us -
   // is split like any other when its slices stay 16-byte aligned for the summing pass)
@@ -2778,11 +2818,33 @@ hipError_t launch_matmul(const LaunchCtx &lc_in, const GemmDesc &g, const char *
       if (g.n_group && (batch != 1 || splits != 1 || g.glu_gate || g.c16)) return hipErrorInvalidValue;
       const uint64_t t128 = (uint64_t)((g.M + 127) / 128) * ((g.N + 127) / 128) * batch * splits;
       const bool deep = t128 < 2 * (uint64_t)lc.n_cus;  // at most one workgroup per CU at a time: four stages
-      if (g.dual_b) {  // gate and up stacked: 128 output columns per tile, 256 rows when that still fills the CUs
+      if (g.M <= 64) {
+        // A few rows: bound by the stream of weights, so narrow tiles, one workgroup to a CU with as much in flight
+        // as its LDS holds (the 128-row tiles put 64 workgroups on the chip for a 16384 x 2048 gate and up).
+        const uint64_t t64 = (uint64_t)((g.N + 63) / 64) * batch * splits;
+        if (g.n_group > 0 && splits != 1) return hipErrorInvalidValue;
+        if (g.dual_b) {
+          if (g.n_group || g.glu_gate || splits != 1) return hipErrorInvalidValue;
+          e = launch_gemm_dma<64, 64, 2, 1, true, 8, true, false, false, 2>(lc, gg, (uint32_t)((g.N + 31) / 32 * batch));
+        } else if (g.glu_gate || g.c16) {
+          e = launch_gemm_dma<64, 64, 2, 2, true, 8, false, false, false, 2>(lc, gg, (uint32_t)t64);
+        } else if (g.rope_s && g.rope_hd > 64) {
+          e = launch_gemm_dma<64, 128, 2, 2, false, 5, false, false, true, 2>(lc, gg, (uint32_t)((g.N + 127) / 128));
+        } else if (g.rope_s) {
+          e = launch_gemm_dma<64, 64, 2, 2, false, 8, false, false, true, 2>(lc, gg, (uint32_t)t64);
+        } else {
+          e = launch_gemm_dma<64, 64, 2, 2, false, 8, false, false, false, 2>(lc, gg, (uint32_t)t64);
+        }
+      } else if (g.dual_b) {  // gate and up stacked: 128 output columns per tile, 256 rows when that still fills the CUs
         if (g.n_group || g.glu_gate || splits != 1) return hipErrorInvalidValue;
         const uint64_t d256 = (uint64_t)((g.M + 255) / 256) * ((g.N + 127) / 128) * batch;
         const uint64_t d128 = (uint64_t)((g.M + 127) / 128) * ((g.N + 127) / 128) * batch;
+        // (fewer tiles of 128 than half the CUs: 64 or 32 output columns per tile)
         if (d256 >= (uint64_t)lc.n_cus) e = launch_gemm_dma<256, 256, 2, 4, true, 2, true>(lc, gg, (uint32_t)d256);
+        else if (d128 * 4 <= (uint64_t)lc.n_cus)
+          e = launch_gemm_dma<128, 64, 4, 1, true, 5, true, false, false, 2>(lc, gg, (uint32_t)((uint64_t)((g.M + 127) / 128) * ((g.N + 31) / 32) * batch));
+        else if (d128 * 2 <= (uint64_t)lc.n_cus)
+          e = launch_gemm_dma<128, 128, 4, 2, true, 4, true>(lc, gg, (uint32_t)((uint64_t)((g.M + 127) / 128) * ((g.N + 63) / 64) * batch));
         else e = launch_gemm_dma<128, 256, 2, 4, true, 3, true>(lc, gg, (uint32_t)d128);
       } else if (g.glu_gate || g.c16) {  // the epilogue variant stages a 128 x 128 tile
         if (deep) e = launch_gemm_dma<128, 128, 2, 4, true, 4>(lc, gg, (uint32_t)t128);

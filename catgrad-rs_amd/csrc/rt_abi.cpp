@@ -347,7 +347,7 @@ int cg_matmul(cg_backend *be, cg_tensor *a, cg_tensor *b, cg_tensor **out) {
     be->gemv_candidates.push_back(n);
     n->gemv_candidate = true;
   }
-  if (a->dtype == CG_F32 && a->rank == 3 && shape[0] == 1 && shape[1] >= 64 && (be->flags & CG_FLAG_BF16) &&
+  if (a->dtype == CG_F32 && a->rank == 3 && shape[0] == 1 && shape[1] > GEMV_PRO_MAX_ROWS && (be->flags & CG_FLAG_BF16) &&
       !(be->flags & (CG_FLAG_EAGER | CG_FLAG_NO_PATTERNS))) {
     if (be->gemm_candidates.size() >= 1024) forget_gemm_candidate(be->gemm_candidates.front());
     be->gemm_candidates.push_back(n);
