@@ -792,12 +792,251 @@ __global__ void __launch_bounds__(256) attn_decode_split_kernel(AttnDecodeDesc a
   if (tid == 0) __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// The split form for grouped queries: a workgroup takes its keys for all `rep` query heads of a kv head, so that a cache
+// row is read once instead of rep times by workgroups of as many XCDs (32 / 8 heads of 64 over 4000 keys: 66 MB asked of
+// the memory-side cache for 16 MB of rows: 20.7 us -> 11.4), and both products run on the matrix cores (v_mfma_f32_16x16x4_f32: all f32):
+// on the vector ALUs four heads to a row cost more than the reads they save (a dot product over 16 lanes is four
+// multiply-adds and as many exchanges).  Everything is computed transposed, a lane column is a query head:
+//   S^T[key, head]  = K[key, :] . Q[head, :]     A: lane (key, kb) holds dims kb * D/4 .. of its row; step s takes dim kb * D/4 + s
+//   O^T[dim, head] += V^T[dim, key] . P^T[key, head]   the scores' registers are P^T's operand as they are (step i: keys
+//                     4 kb + i); A: lane (m, kb) holds V[4 kb + i][64 u + 4 m ..], component t belongs to dim 64 u + 4 m + t
+// A wave takes tiles of 16 keys, U at a time with the next U in flight, with running maximum and sum per head; the waves
+// meet in LDS, the workgroups as in attn_decode_split_kernel.
+template <int D, int NWV>
+__global__ void __launch_bounds__(NWV * 64) attn_decode_group_kernel(AttnDecodeDesc a) {
+  typedef __attribute__((ext_vector_type(4))) float f32x4;
+  constexpr int U = D == 64 ? 2 : 1, KD = D / 4, K4 = D / 16, H = D / 64;  // K4: 16-byte pieces of a lane's part of a row
+  constexpr float FMIN = -3.40282347e+38f;
+  __shared__ float red[NWV][16][D + 4];
+  __shared__ float red_m[NWV][16], red_l[NWV][16];
+  __shared__ uint32_t last_flag;
+  const uint32_t kv = blockIdx.x, b = blockIdx.y, c = blockIdx.z, rep = a.rep, h0 = kv * rep;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, m = lane & 15, kb = lane >> 4;
+  const float *K = a.k + (int64_t)b * a.k_sb + (int64_t)kv * a.k_skv;
+  const float *V = a.v + (int64_t)b * a.v_sb + (int64_t)kv * a.v_skv;
+  const uint32_t t_begin = c * a.chunk, t_end = min(a.t, t_begin + a.chunk);
+  f32x4 kn[U][K4], vn[U][4][H];
+  auto fetch = [&](uint32_t t0) {  // tiles t0, t0 + NWV * 16, ..; rows past the end repeat the last (their weight is zero)
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const uint32_t tt = t0 + u * NWV * 16;
+      const float *kr = K + (int64_t)min(tt + m, t_end - 1) * a.k_st + kb * KD;
+#pragma unroll
+      for (int q = 0; q < K4; ++q) kn[u][q] = *(const f32x4 *)(kr + q * 4);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float *vr = V + (int64_t)min(tt + kb * 4 + i, t_end - 1) * a.v_st + m * 4;
+#pragma unroll
+        for (int w = 0; w < H; ++w) vn[u][i][w] = *(const f32x4 *)(vr + w * 64);
+      }
+    }
+  };
+  const uint32_t t_wave = t_begin + wave * 16;
+  if (t_wave < t_end) fetch(t_wave);
+  // a row of D floats, this lane's part of it, rotated (apply_rope_embedding, the arithmetic of rope_kernel)
+  auto rotated = [&](const float *row, const float *cos, const float *sin, f32x4 (&x)[K4]) {
+    const float *pr = row + (kb < 2 ? kb + 2 : kb - 2) * KD;
+#pragma unroll
+    for (int q = 0; q < K4; ++q) {
+      x[q] = *(const f32x4 *)(row + kb * KD + q * 4);
+      if (cos) {
+        f32x4 p = *(const f32x4 *)(pr + q * 4);
+        if (kb < 2) p = -p;
+        const f32x4 cs = *(const f32x4 *)(cos + kb * KD + q * 4), sn = *(const f32x4 *)(sin + kb * KD + q * 4);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) x[q][e] = cs[e] * x[q][e] + sn[e] * p[e];
+      }
+    }
+  };
+  f32x4 qv[K4];
+  rotated(a.q + (int64_t)b * a.q_sb + (int64_t)(h0 + min((uint32_t)m, rep - 1)) * a.q_sh, a.q_cos, a.q_sin, qv);
+  if ((uint32_t)m >= rep) {  // (columns without a head)
+#pragma unroll
+    for (int q = 0; q < K4; ++q) qv[q] = (f32x4){0.f, 0.f, 0.f, 0.f};
+  }
+  // this step's own key / value row comes from the projections; its tile's lanes also store it into the cache
+  const bool has_new = a.k_new != nullptr && a.t_new >= t_begin && a.t_new < t_end;
+  const uint32_t t_new = has_new ? a.t_new : 0xFFFFFFFFu;
+  const float inv_scale = a.has_scale ? 1.0f / a.scale : 1.0f;
+  float m_run = FMIN, l_run = 0.f;
+  f32x4 o[H][4];
+#pragma unroll
+  for (int w = 0; w < H; ++w)
+#pragma unroll
+    for (int t = 0; t < 4; ++t) o[w][t] = (f32x4){0.f, 0.f, 0.f, 0.f};
+  for (uint32_t t0 = t_wave; t0 < t_end; t0 += U * NWV * 16) {
+    f32x4 kr[U][K4], vr[U][4][H];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const uint32_t tt = t0 + u * NWV * 16;
+#pragma unroll
+      for (int q = 0; q < K4; ++q) kr[u][q] = kn[u][q];
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int w = 0; w < H; ++w) vr[u][i][w] = vn[u][i][w];
+      if (t_new - tt < 16u) {  // (uniform over the wave)
+        if (tt + m == t_new) {
+          rotated(a.k_new + (int64_t)b * a.kn_sb + (int64_t)kv * a.kn_skv, a.kn_cos, a.kn_sin, kr[u]);
+#pragma unroll
+          for (int q = 0; q < K4; ++q) *(f32x4 *)(const_cast<float *>(K) + (int64_t)t_new * a.k_st + kb * KD + q * 4) = kr[u][q];
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          if (tt + kb * 4 + i == t_new) {
+#pragma unroll
+            for (int w = 0; w < H; ++w) {
+              vr[u][i][w] = *(const f32x4 *)(a.v_new + (int64_t)b * a.vn_sb + (int64_t)kv * a.vn_skv + w * 64 + m * 4);
+              *(f32x4 *)(const_cast<float *>(V) + (int64_t)t_new * a.v_st + w * 64 + m * 4) = vr[u][i][w];
+            }
+          }
+      }
+    }
+    if (t0 + U * NWV * 16 < t_end) fetch(t0 + U * NWV * 16);  // in flight during the arithmetic below
+    f32x4 s[U];
+    float mx = FMIN;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const uint32_t tt = t0 + u * NWV * 16;
+      s[u] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int q = 0; q < K4; ++q)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) s[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(kr[u][q][e], qv[q][e], s[u], 0, 0, 0);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        float x = s[u][i];
+        if (a.has_scale) x = x * inv_scale;
+        if (a.has_mask_const) x = x + a.mask_const;
+        s[u][i] = tt + kb * 4 + i < t_end ? x : FMIN;
+        mx = fmaxf(mx, s[u][i]);
+      }
+    }
+    mx = fmaxf(mx, __shfl_xor(mx, 16));
+    mx = fmaxf(mx, __shfl_xor(mx, 32));
+    const float m_new = fmaxf(m_run, mx), alpha = __expf(m_run - m_new);
+    l_run *= alpha;
+#pragma unroll
+    for (int w = 0; w < H; ++w)
+#pragma unroll
+      for (int t = 0; t < 4; ++t) o[w][t] *= alpha;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const uint32_t tt = t0 + u * NWV * 16;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float p = tt + kb * 4 + i < t_end ? __expf(s[u][i] - m_new) : 0.f;
+        l_run += p;
+#pragma unroll
+        for (int w = 0; w < H; ++w)
+#pragma unroll
+          for (int t = 0; t < 4; ++t) o[w][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(vr[u][i][w][t], p, o[w][t], 0, 0, 0);
+      }
+    }
+    m_run = m_new;
+  }
+  // a lane's sum covers its own keys: the four lanes of a head add up theirs
+  l_run += __shfl_xor(l_run, 16);
+  l_run += __shfl_xor(l_run, 32);
+  if ((uint32_t)m < rep) {
+    // o[w][t][e]: dim 64 w + 4 (4 kb + e) + t of head m
+#pragma unroll
+    for (int w = 0; w < H; ++w)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        *(f32x4 *)(&red[wave][m][w * 64 + (kb * 4 + e) * 4]) = (f32x4){o[w][0][e], o[w][1][e], o[w][2][e], o[w][3][e]};
+    if (kb == 0) { red_m[wave][m] = m_run; red_l[wave][m] = l_run; }
+  }
+  __syncthreads();
+  const uint32_t pw = D + 2;  // floats per partial: max, sum, D values
+  for (uint32_t i = tid; i < rep * D; i += NWV * 64) {
+    const uint32_t r = i / D, dim = i - r * D;
+    const uint64_t rec = ((uint64_t)b * a.heads + h0 + r) * a.splits + c;
+    float M = FMIN;
+#pragma unroll
+    for (int g = 0; g < NWV; ++g) M = fmaxf(M, red_m[g][r]);
+    float L = 0.f, v = 0.f;
+#pragma unroll
+    for (int g = 0; g < NWV; ++g) {
+      const float w = __expf(red_m[g][r] - M);
+      L += w * red_l[g][r];
+      v += w * red[g][r][dim];
+    }
+    if (a.splits == 1) {
+      a.out[((uint64_t)b * a.heads + h0 + r) * D + dim] = v / L;
+    } else if (a.merge_later) {
+      float *p = a.part + rec * (D + 4);
+      p[dim] = v;
+      if (dim == 0) { p[D] = M; p[D + 1] = L; }
+    } else {  // agent-scope stores, acknowledged before the counter moves (the hand-over of attn_decode_split_kernel)
+      float *p = a.part + rec * pw;
+      __hip_atomic_store(p + 2 + dim, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (dim == 0) {
+        __hip_atomic_store(p, M, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(p + 1, L, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+    }
+  }
+  if (a.splits == 1 || a.merge_later) return;
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  uint32_t *counter = a.count + (uint64_t)b * (a.heads / rep) + kv;
+  if (tid == 0)
+    last_flag = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == a.splits - 1 ? 1u : 0u;
+  __syncthreads();
+  if (!last_flag) return;
+  for (uint32_t i = tid; i < rep * D; i += NWV * 64) {
+    const uint32_t r = i / D, dim = i - r * D;
+    const float *base = a.part + ((uint64_t)b * a.heads + h0 + r) * a.splits * pw;
+    float M = FMIN, L = 0.f, v = 0.f;
+    constexpr int B = 16;  // partials asked for at once
+    for (uint32_t s0 = 0; s0 < a.splits; s0 += B) {
+      float pm[B], pl[B], pv[B];
+#pragma unroll
+      for (int u = 0; u < B; ++u) {
+        const uint32_t sp = min(s0 + u, a.splits - 1);
+        pm[u] = __hip_atomic_load(base + sp * pw, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        pl[u] = __hip_atomic_load(base + sp * pw + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        pv[u] = __hip_atomic_load(base + sp * pw + 2 + dim, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+      float mx = M;
+#pragma unroll
+      for (int u = 0; u < B; ++u)
+        if (s0 + u < a.splits) mx = fmaxf(mx, pm[u]);
+      const float keep = __expf(M - mx);
+      L *= keep;
+      v *= keep;
+      M = mx;
+#pragma unroll
+      for (int u = 0; u < B; ++u)
+        if (s0 + u < a.splits) {
+          const float w = __expf(pm[u] - M);
+          L += w * pl[u];
+          v += w * pv[u];
+        }
+    }
+    a.out[((uint64_t)b * a.heads + h0 + r) * D + dim] = v / L;
+  }
+  if (tid == 0) __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+bool attn_decode_group_ok(const AttnDecodeDesc &d) {
+  return d.rep >= 1 && d.rep <= 16 && d.k_srep == 0 && d.v_srep == 0 && (d.d == 64 || d.d == 128);
+}
+
 uint32_t attn_decode_rows_per_pass(uint32_t d) { return d <= 64 ? 128 : d <= 128 ? 64 : 32; }
 
 hipError_t launch_attn_decode(const LaunchCtx &lc, const AttnDecodeDesc &d) {
   if (!d.b || !d.heads || !d.d) return hipSuccess;
   if (d.splits) {
     if (!d.part || !d.count || !d.chunk || (uint64_t)d.chunk * d.splits < d.t || d.splits > 64) return hipErrorInvalidValue;
+    if (d.group) {
+      if (!attn_decode_group_ok(d)) return hipErrorInvalidValue;
+      dim3 gg(d.heads / d.rep, d.b, d.splits);
+      if (d.d == 64) CG_LAUNCH(lc, (attn_decode_group_kernel<64, 4>), gg, 256, d);
+      else CG_LAUNCH(lc, (attn_decode_group_kernel<128, 4>), gg, 256, d);
+      return hipGetLastError();
+    }
     dim3 grid(d.heads, d.b, d.splits);
     if (d.d <= 64) CG_LAUNCH(lc, (attn_decode_split_kernel<16>), grid, 256, d);
     else if (d.d <= 128) CG_LAUNCH(lc, (attn_decode_split_kernel<32>), grid, 256, d);

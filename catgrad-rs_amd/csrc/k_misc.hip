@@ -286,13 +286,17 @@ hipError_t launch_to_host(const LaunchCtx &lc, const void *src, void *dst, uint6
 
 // n words of pinned host memory into device memory, then the flag: the host may use the words again (one workgroup)
 __global__ void __launch_bounds__(1024) from_host_kernel(const uint32_t *src, uint32_t *dst, uint32_t n, uint32_t *flag) {
-  for (uint32_t i = threadIdx.x; i < n; i += 1024) dst[i] = __hip_atomic_load(src + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  // (16 bytes a request: each is a trip across the bus, and there is one workgroup to make them; a fresh slot was not
+  // read before, so ordinary loads find the host's values)
+  const uint32_t n4 = n / 4;
+  for (uint32_t i = threadIdx.x; i < n4; i += 1024) ((uint4 *)dst)[i] = ((const uint4 *)src)[i];
+  if (threadIdx.x < n - n4 * 4) dst[n4 * 4 + threadIdx.x] = src[n4 * 4 + threadIdx.x];
   __syncthreads();
   if (threadIdx.x == 0) __hip_atomic_store(flag, 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 hipError_t launch_from_host(const LaunchCtx &lc, const void *src, void *dst, uint32_t n, uint32_t *flag) {
-  if (!n) return hipErrorInvalidValue;
+  if (!n || (uintptr_t)src % 16 || (uintptr_t)dst % 16) return hipErrorInvalidValue;
   CG_LAUNCH(lc, from_host_kernel, 1, 1024, (const uint32_t *)src, (uint32_t *)dst, n, flag);
   return hipGetLastError();
 }

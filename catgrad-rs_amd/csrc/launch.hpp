@@ -238,7 +238,10 @@ struct AttnDecodeDesc {
   // maximum, the sum and two unused floats (stride d + 4: every record 16-byte aligned); out and count
   // are not touched.
   int32_t merge_later;
+  // splits != 0 only: a workgroup takes its keys for all `rep` heads of a kv head (attn_decode_group_ok)
+  int32_t group;
 };
+bool attn_decode_group_ok(const AttnDecodeDesc &d);
 enum { ATTN_DECODE_MAX_T = 8192, ATTN_DECODE_MAX_D = 256 };
 // keys one workgroup of the split form visits per pass over its chunk
 uint32_t attn_decode_rows_per_pass(uint32_t d);

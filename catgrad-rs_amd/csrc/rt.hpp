@@ -148,6 +148,7 @@ struct cg_backend {
   char *h_out = nullptr;        // two halves, each TO_HOST_MAX_PIECES pieces and their tails
   char *h_in = nullptr;         // HOST_IN_SLOTS slots of HOST_IN_BYTES, each ending in its flag
   uint32_t h_in_next = 0;
+  uint32_t host_waits = 0;
   // caching allocator
   std::map<size_t, std::vector<void *>> pool;
   uint64_t pool_bytes = 0, device_bytes = 0, launches = 0;

@@ -487,12 +487,26 @@ int try_attn_decode(cg_backend *be, cg_tensor *n, bool *done, AttnMergeLater *la
     // whole decode loop: T ~ 540: 4 ranges 1367, 5 1392, 6 1382, 8 1372 tokens/s; T ~ 200: 2 1415, 3 1421,
     // 4 1421, 8 1397.
     if (later && nb == 1 && ns <= ATTN_MERGE_MAX_SPLITS) ns = std::max<int64_t>((T + 109) / 110, std::min<int64_t>(3, (T + 31) / 32));
+    // Longer caches go to the matrix-core form, 64 KB of keys to a workgroup (fewer: the hand-over of more partials costs
+    // what the shorter chains save; more: a workgroup's chain of passes is what the launch waits for): 32 / 8 heads of 64
+    // over 1500 keys 10.1 -> 9.1 us, 4000 20.7 -> 11.4, 7000 25 -> 13.9; 3 x 16 heads of 128 over 900 16.9 -> 13.4.
+    // Where the reader merges, up to as many ranges as it can take (16 heads of 128, 500 keys: 10.3 -> 6.4 us).  Below,
+    // the vector kernel has the shorter chain (32 / 8 heads of 64 over 520 keys: 5.7 us against 6.8).
+    bool reader_merges = later && nb == 1;
+    if (attn_decode_group_ok(a) && (d == 128 ? T > 128 : a.rep >= 2 && T > 880)) {
+      a.group = 1;
+      const int64_t rows = d == 64 && T < 2048 ? 128 : 16384 / d;
+      ns = (T + rows - 1) / rows;
+      reader_merges = reader_merges && d == 128;  // (32 heads of 64, 1500 keys: 9.1 + 4.3 us merged here, 8.4 + 5.0 by the reader)
+      if (reader_merges && ns <= ATTN_MERGE_MAX_SPLITS) ns = std::min<int64_t>(ATTN_MERGE_MAX_SPLITS, (T + 63) / 64);
+      ns = std::min<int64_t>(ns, 64);
+    }
     if (ns >= 2 || T > ATTN_DECODE_MAX_T) {
       const int64_t chunk = (T + ns - 1) / ns;
       a.chunk = (uint32_t)chunk;
       a.splits = (uint32_t)((T + chunk - 1) / chunk);
       // the reader of the result merges the partials when it can (one row, few splits)
-      if (later && nb == 1 && a.splits >= 2 && a.splits <= ATTN_MERGE_MAX_SPLITS && heads * a.splits <= 256 &&
+      if (reader_merges && a.splits >= 2 && a.splits <= ATTN_MERGE_MAX_SPLITS && heads * a.splits <= 256 &&
           heads * d <= 2048 && d % 4 == 0)
         a.merge_later = 1;
       TRY(attn_decode_scratch(be, (size_t)bh * a.splits * (d + 4), (size_t)bh));

@@ -267,6 +267,8 @@ int sync_and_check(cg_backend *be) {
 
 // what the device's error words say (words: their copy on the host, the stream idle)
 int check_error_words(cg_backend *be, const uint32_t *words) {
+  // (the runtime lets go of finished launches when it is waited for)
+  if (++be->host_waits % 32 == 0) HIPCHK(be, hipStreamSynchronize(be->ordered_stream()));
   cap_pool(be);
   const uint32_t e = words[0];
   if (e) {

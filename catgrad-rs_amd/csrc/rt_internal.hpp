@@ -39,7 +39,7 @@ using namespace cgk;
 
 
 enum { PREFETCH_BYTES = 4096, PREFETCH_TAIL = 16 };  // pinned buffer of a prefetched tensor: data, error words and flag
-enum : size_t { HOST_IN_BYTES = 16 << 10, HOST_IN_SLOTS = 8 };
+enum : size_t { HOST_IN_BYTES = (64 << 10) + 64, HOST_IN_SLOTS = 8 };
 enum : uint32_t { F_ONE = 0x3F800000u, F_HALF = 0x3F000000u, F_E = 0x402DF854u, F_TWO = 0x40000000u };
 
 struct KernelScope;

@@ -62,3 +62,30 @@ def test_rotation_in_the_projections_launch_at_odd_lengths(oracle, hip_bf16, tok
 def test_rotation_of_several_odd_sequences(oracle, hip_bf16, batch, tokens, heads, kv_heads, head_dim):
     """Four rows of a tile may belong to two sequences: the transposed values are stored one by one there."""
     moe_tests.test_qwen_prefill_biases_and_rotation_in_the_projections_launch(oracle, hip_bf16, batch, tokens, heads, kv_heads, head_dim)
+
+
+# One query over long caches (the matrix-core form): kv heads shared by 2 to 8 query heads or none, last ranges that are short,
+# more ranges than the reader merges, several sequences; the step's own rows go into the cache through the same launch.
+@pytest.mark.gpu
+@pytest.mark.parametrize("H,KV,d,T,steps", [(4, 1, 64, 881, 2), (8, 8, 128, 129, 3), (4, 2, 128, 515, 2), (16, 2, 64, 2049, 2),
+                                            (2, 1, 128, 4100, 1), (4, 2, 64, 1300, 2)])
+def test_decode_over_a_long_cache(oracle, hip, H, KV, d, T, steps):
+    cfg = llm.Config(hidden_size=H * d, intermediate_size=64, num_hidden_layers=1, num_attention_heads=H, num_key_value_heads=KV,
+                     vocab_size=97, rms_norm_eps=1e-5, rope_theta=10000.0)
+    arrays = llm.random_init.llama_params(cfg, seed=T, std=0.08)
+    g = np.random.default_rng(T)
+    kv = [g.standard_normal((1, KV, T, d)).astype(np.float32) for _ in range(2)]
+    runners = []
+    for be in (oracle, hip):
+        r = llm.CachedRunner(be, cfg, arrays, T + 8)
+        # (rotations at small positions: an angle of hundreds of radians in f32 is itself off by T * 2^-24, which is the
+        # tables' error on both sides and not this launch's)
+        r.batch, r.pos, r.kv = 1, 3, [be.tensor(a) for a in kv]
+        runners.append(r)
+    for token in (5, 11, 90)[:steps + 1]:     # (the first step copies the cache, the following ones append)
+        hip.launch_counts(reset=True)
+        out = [r.step(token)[1] for r in runners]
+        parity.assert_f32(oracle.to_vec(out[0]), hip.to_vec(out[1]), f"token {token}")
+        assert hip.launch_counts(reset=True).get("attn_decode") == 1
+    for a, b in zip(runners[0].kv, runners[1].kv):
+        parity.assert_f32(oracle.to_vec(a), hip.to_vec(b), "cache")
