@@ -2288,13 +2288,16 @@ __global__ void __launch_bounds__(256) moe_gemm_dma_kernel(MoeGemmDesc g) {
       for (int h = 0; h < MT; ++h)
 #pragma unroll
         for (int i = 0; i < 16; ++i) acc[p][h][i] = 0.f;
-    const uint16_t *gp[LPW];  // per-lane source of each of this wave's loads; advances by BK per stage
+    // Load i of a wave: i < MT: its eight rows of the i-th 32-row tile of token rows (not made when no pair is in
+    // that tile: an expert of a few pairs moves its weights and 32 rows, not 128), then its share of the weight rows.
+    const uint16_t *gp[LPW];  // per-lane source; advances by BK per stage
+    auto block_of = [&](int i) { return i < MT ? i * 4 + wave : BM_ / 8 + wave * (LPW - MT) + i - MT; };  // 8-row block of the stacked tile
 #pragma unroll
     for (int i = 0; i < LPW; ++i) {
-      const int q = wave * LPW + i;  // 8-row block of the stacked tile
+      const int q = block_of(i);
       const int R = q * 8 + (lane >> 3);
       const int c = (lane & 7) ^ ((R >> 1) & 7);
-      if (q * 8 < BM_) {
+      if (i < MT) {
         // rows past the expert's last pair repeat it: loaded, multiplied, never stored
         const uint32_t ent = list[min(m0 + (uint32_t)R, cnt - 1)], sl = ent >> 16, tok = ent & 0xFFFFu;
         const uint16_t *rows = g.slot[0].a16;
@@ -2314,8 +2317,8 @@ __global__ void __launch_bounds__(256) moe_gemm_dma_kernel(MoeGemmDesc g) {
     auto issue = [&](int buf) {
 #pragma unroll
       for (int i = 0; i < LPW; ++i) {
-        if ((wave * LPW + i) * 8 < BM_) lds_dma16(gp[i], lds0 + buf * STAGE + (wave * LPW + i) * 1024);
-        else lds_dma16_stream(gp[i], lds0 + buf * STAGE + (wave * LPW + i) * 1024);
+        if (i >= MT) lds_dma16_stream(gp[i], lds0 + buf * STAGE + block_of(i) * 1024);
+        else if (i < live_tiles) lds_dma16(gp[i], lds0 + buf * STAGE + block_of(i) * 1024);
         gp[i] += BK;
       }
     };
@@ -2348,8 +2351,12 @@ __global__ void __launch_bounds__(256) moe_gemm_dma_kernel(MoeGemmDesc g) {
     for (int s0 = 0; s0 < NS - 1; ++s0)
       if (s0 < n_steps) issue(s0);
     for (int step = 0; step < n_steps; ++step) {
-      if (step + NS - 1 <= n_steps) wait_vmcnt<(NS - 2) * LPW>();
-      else wait_vmcnt<0>();
+      // (a stage is as many loads as there are weight pieces and live row tiles)
+      if (step + NS - 1 > n_steps || NS == 2) wait_vmcnt<0>();
+      else if (live_tiles == 1) wait_vmcnt<(NS - 2) * (LPW - MT + 1)>();
+      else if (live_tiles == 2) wait_vmcnt<(NS - 2) * (LPW - MT + 2)>();
+      else if (live_tiles == 3) wait_vmcnt<(NS - 2) * (LPW - MT + 3)>();
+      else wait_vmcnt<(NS - 2) * LPW>();
       __syncthreads();
       if (step + NS - 1 < n_steps) issue((step + NS - 1) % NS);
       compute(step % NS);
@@ -2599,7 +2606,7 @@ static void launch_rowdot(const LaunchCtx &lc, const GemmDesc &g, int bv, int av
 
 // the direct-to-LDS kernel: both operands unit-stride along k, K (and each split) a multiple of 64
 static bool gemm_dma_ok(const GemmDesc &g) {
-  return g.sak == 1 && g.sbk == 1 && g.K % 64 == 0 && g.K >= 64 && g.M > GEMV_PRO_MAX_ROWS && g.N >= 64;
+  return g.sak == 1 && g.sbk == 1 && g.K % 64 == 0 && g.K >= 64 && gemm_rows(g.M, g.K) && g.N >= 64;
 }
 
 // B [K, N] with unit stride along n, used as it lies by the k-major form of the direct-to-LDS kernel
@@ -2611,7 +2618,7 @@ bool gemm_dma_bkm_ok(const GemmDesc &g) {
 }
 
 static bool gemm_fast_path(const GemmDesc &g, int av, int bv) {
-  return g.bf16_math && g.M > 8 && g.a_stype == ST_BF16 && g.b_stype == ST_BF16 && g.sak == 1 &&
+  return g.bf16_math && (g.M > 8 || gemm_rows(g.M, g.K)) && g.a_stype == ST_BF16 && g.b_stype == ST_BF16 && g.sak == 1 &&
          (g.sbk == 1 || g.sbn == 1) && g.K % 8 == 0 && (g.sbk == 1 || g.N % 8 == 0) && av && bv;
 }
 
@@ -2625,7 +2632,7 @@ bool gemm_epilogue_ok(const GemmDesc &g) {
 bool gemm_rope_epilogue_ok(const LaunchCtx &lc, const GemmDesc &g) {
   if (!g.rope_s || !g.n_group || !gemm_epilogue_ok(g)) return false;
   if (g.rope_hd != 64 && g.rope_hd != 128) return false;
-  if (g.nb0 * g.nb1 != 1 || g.glu_gate || g.c16 || g.dual_b || g.M % g.rope_s || g.M <= GEMV_PRO_MAX_ROWS) return false;
+  if (g.nb0 * g.nb1 != 1 || g.glu_gate || g.c16 || g.dual_b || g.M % g.rope_s || !gemm_rows(g.M, g.K)) return false;
   bool grp256 = true;
   for (uint32_t p = 0; p < g.n_group; ++p) {
     if (g.grp_n[p] % 128) return false;

@@ -499,6 +499,19 @@ int binary(cg_backend *be, cg_tensor *a, cg_tensor *b, cg_tensor **out, EwOp f_o
       block_end = dense;
     }
   }
+  // A block that ends in `residual + norm(linear(...))` (gemma3.rs:198-240) is one kernel with the norm that follows and
+  // cannot be cut there; its closing product can: nothing but that norm reads it, and all its reads are recorded.  A prompt
+  // of 100 tokens through 26 such layers: 1.2 ms of recording in front of 2.7 ms of kernels, 4.2 -> 2.9 ms.
+  cg_tensor *closing = nullptr;
+  if (n->ew == E_ADD_F && n->rank == 3 && !block_end && be->queue && !(be->flags & (CG_FLAG_EAGER | CG_FLAG_NO_PATTERNS))) {
+    for (int side = 0; side < 2 && !closing; ++side) {
+      cg_tensor *t = n->in[side];
+      if (!is_bin(t, E_MUL_F) || !is_bin(t->in[0], E_DIV_F)) continue;
+      cg_tensor *y = t->in[0]->in[0];
+      const cg_tensor *mm = y->op == N_RESHAPE ? y->in[0] : y;
+      if (mm->op == N_MATMUL && mm->rank == 3) closing = y;
+    }
+  }
   // `linear(x) + bias`: the product's launch can add the bias itself (a few rows: try_gemv_prologue; many rows
   // in bf16 mode: the grouped q / k / v launch of realize_matmul)
   if (n->ew == E_ADD_F && !(be->flags & (CG_FLAG_EAGER | CG_FLAG_NO_PATTERNS))) {
@@ -523,7 +536,7 @@ int binary(cg_backend *be, cg_tensor *a, cg_tensor *b, cg_tensor **out, EwOp f_o
   }
   TRY(finish(be, n, out));
   if (*out != n) return CG_OK;  // folded or shared: n is gone
-  if (block_end && !be->flush_node) be->flush_node = retain(n);
+  if (!be->flush_node && (block_end || closing)) be->flush_node = retain(block_end ? n : closing);
   return CG_OK;
 }
 

@@ -728,7 +728,7 @@ int realize_matmul(cg_backend *be, cg_tensor *n, cg_tensor *addend, bool *added,
     g.b_stype = B.t->stype;
     // MFMA path in bf16 mode: f32 operands with a unit k stride are read from the bf16 twin of
     // their storage (narrowed once, shared by every GEMM on the same activations)
-    if ((be->flags & CG_FLAG_BF16) && M > GEMV_PRO_MAX_ROWS && K % 8 == 0) {
+    if ((be->flags & CG_FLAG_BF16) && gemm_rows(M, K) && K % 8 == 0) {
       auto twin = [&](MatOperand &o, bool unit_k, const void **ptr, int32_t *stype) -> int {
         Storage *st = o.t->st;
         if (o.t->stype != ST_F32 || !unit_k || st->grow_dim >= 0 || st->bytes % 32) return CG_OK;

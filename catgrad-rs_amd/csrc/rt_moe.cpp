@@ -22,7 +22,7 @@ bool match_expert_operand(const cg_tensor *t, int64_t S, ExpertOperand *o) {
 // stacked weights joins, with its own indices, input rows and output (launch_moe_gemm).
 int try_moe_gemm(cg_backend *be, cg_tensor *n, bool *done) {
   const int64_t S = n->shape[0];
-  if (S < 64 || S > 65535 || !(be->flags & CG_FLAG_BF16)) return CG_OK;
+  if (S <= 8 || S > 65535 || !(be->flags & CG_FLAG_BF16)) return CG_OK;
   ExpertOperand eo;
   if (!match_expert_operand(n->in[1], S, &eo)) return CG_OK;
   const int64_t K = n->in[0]->shape[2];

@@ -482,7 +482,7 @@ int try_rmsnorm(cg_backend *be, cg_tensor *root, bool *done) {
   // In bf16 mode with many rows: the GEMMs that wait for this value read it as bf16.  If nothing
   // else holds it, it is written in that form only; if something else does, in both.
   bool to_gemms = false, only_gemms = false;
-  if (!residual && (be->flags & CG_FLAG_BF16) && root->rank >= 2 && n % 8 == 0 && root->size() / n > GEMV_PRO_MAX_ROWS)
+  if (!residual && (be->flags & CG_FLAG_BF16) && root->rank >= 2 && n % 8 == 0 && gemm_rows(root->size() / n, n))
     to_gemms = gemm_readers(be, root, &only_gemms) > 0;
   int st = alloc_result(be, root, only_gemms ? ST_BF16 : ST_F32);
   if (!st) {
@@ -951,7 +951,7 @@ int try_glu(cg_backend *be, cg_tensor *root, bool *done) {
     if (gm->op == N_MATMUL && um->op == N_MATMUL && gm != um && refs(gate) == (gelu ? 3 : 2) && refs(up) == 1 && refs(um) == 1 &&
         same_rows(gm->in[0], um->in[0]) && !gm->gemv_candidate && !um->gemv_candidate && gm->rank == r && r >= 2 &&
         std::equal(gm->shape, gm->shape + r, um->shape) && um->size() == um->shape[r - 2] * um->shape[r - 1] &&
-        um->shape[r - 2] > GEMV_PRO_MAX_ROWS && um->shape[r - 1] >= 64 && um->shape[r - 1] % 8 == 0 && um->in[0]->shape[r - 1] % 64 == 0) {
+        gemm_rows(um->shape[r - 2], um->in[0]->shape[r - 1]) && um->shape[r - 1] >= 64 && um->shape[r - 1] % 8 == 0 && um->in[0]->shape[r - 1] % 64 == 0) {
       cg_tensor *wg = gm->in[1], *wu = um->in[1];
       TRY(realize(be, wg));
       TRY(realize(be, wu));
