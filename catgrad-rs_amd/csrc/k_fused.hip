@@ -27,7 +27,7 @@ namespace cgk {
 // norm reads; it is written to y_mid and normed a second time (gamma2) from the registers it sits in.
 // RPW rows per workgroup: with many short rows (a prefill) a wave takes a whole row (BLOCK = 64) - no
 // barrier, no LDS - and four such waves share a workgroup.
-template <int BLOCK, int EPT, bool PAIR, int RPW = 1>  // BLOCK = threads per row, EPT = float4 chunks per thread
+template <int BLOCK, int EPT, bool PAIR, int RPW = 1, bool SLICES = false>  // BLOCK = threads per row, EPT = float4 chunks per thread
 __global__ void __launch_bounds__(BLOCK * RPW) rmsnorm_kernel(RmsNormDesc d) {
   static_assert(RPW == 1 || BLOCK == 64, "several rows per workgroup: one wave each");
   __shared__ float lds[BLOCK / 64];
@@ -45,28 +45,66 @@ __global__ void __launch_bounds__(BLOCK * RPW) rmsnorm_kernel(RmsNormDesc d) {
   float *y = d.y ? d.y + (int64_t)row * d.n : nullptr;
   float4 v[EPT];
   float ss = 0.f;
+  // Everything the row needs is asked for at once (a short row is one trip to memory long: with a trip per k-slice and
+  // one for gamma behind the reduction, 37 rows of 2048 as eight slices took 7.6 us, now 4.5).  Pieces past the end repeat
+  // the first.
+  constexpr bool EARLY = EPT <= 2 && RPW == 1;
+  float4 gm[EARLY ? EPT : 1];
+  if (EARLY && d.gamma) {
+#pragma unroll
+    for (int e = 0; e < EPT; ++e) {
+      const uint32_t c = (tid + e * BLOCK) * 4;
+      gm[EARLY ? e : 0] = *(const float4 *)(d.gamma + (c < d.n ? c : 0));
+    }
+  }
+  if constexpr (SLICES) {  // the row is still the k-slices of a split product: sum them, keep the sum
+    constexpr int SB = EPT <= 2 ? 8 : 2;  // slices asked for at once
+    float4 add[EPT];
+    const uint64_t at0 = (uint64_t)row * d.n;
+#pragma unroll
+    for (int e = 0; e < EPT; ++e) {
+      const uint32_t c = (tid + e * BLOCK) * 4;
+      v[e] = make_float4(0.f, 0.f, 0.f, 0.f);
+      if (d.x_add) add[e] = *(const float4 *)(d.x_add + at0 + (c < d.n ? c : 0));
+    }
+    for (uint32_t k0 = 0; k0 < d.x_n_slices; k0 += SB) {
+      float4 t[EPT][SB];
+#pragma unroll
+      for (int e = 0; e < EPT; ++e) {
+        const uint32_t c = (tid + e * BLOCK) * 4;
+#pragma unroll
+        for (int j = 0; j < SB; ++j) {
+          const uint32_t k = k0 + j < d.x_n_slices ? k0 + j : d.x_n_slices - 1;
+          t[e][j] = *(const float4 *)(d.x_slices + k * d.x_slice_stride + at0 + (c < d.n ? c : 0));
+        }
+      }
+#pragma unroll
+      for (int e = 0; e < EPT; ++e)
+#pragma unroll
+        for (int j = 0; j < SB; ++j)
+          if (k0 + j < d.x_n_slices) {
+            v[e].x += t[e][j].x; v[e].y += t[e][j].y; v[e].z += t[e][j].z; v[e].w += t[e][j].w;
+          }
+    }
+#pragma unroll
+    for (int e = 0; e < EPT; ++e) {
+      const uint32_t c = (tid + e * BLOCK) * 4;
+      if (d.x_add) {
+        v[e].x += add[e].x; v[e].y += add[e].y; v[e].z += add[e].z; v[e].w += add[e].w;
+      }
+      if (c < d.n) *(float4 *)(d.x_out + at0 + c) = v[e];
+    }
+  } else {
+#pragma unroll
+    for (int e = 0; e < EPT; ++e) {
+      const uint32_t c = (tid + e * BLOCK) * 4;
+      if (c < d.n) v[e] = *(const float4 *)(x + c);
+    }
+  }
 #pragma unroll
   for (int e = 0; e < EPT; ++e) {
     const uint32_t c = (tid + e * BLOCK) * 4;
-    if (c < d.n) {
-      if (d.x_slices) {  // the row is still the k-slices of a split product: sum them, keep the sum
-        const uint64_t at = (uint64_t)row * d.n + c;
-        float4 s = *(const float4 *)(d.x_slices + at);
-        for (uint32_t k = 1; k < d.x_n_slices; ++k) {
-          const float4 t = *(const float4 *)(d.x_slices + k * d.x_slice_stride + at);
-          s.x += t.x; s.y += t.y; s.z += t.z; s.w += t.w;
-        }
-        if (d.x_add) {
-          const float4 t = *(const float4 *)(d.x_add + at);
-          s.x += t.x; s.y += t.y; s.z += t.z; s.w += t.w;
-        }
-        *(float4 *)(d.x_out + at) = s;
-        v[e] = s;
-      } else {
-        v[e] = *(const float4 *)(x + c);
-      }
-      ss += v[e].x * v[e].x + v[e].y * v[e].y + v[e].z * v[e].z + v[e].w * v[e].w;
-    }
+    if (c < d.n) ss += v[e].x * v[e].x + v[e].y * v[e].y + v[e].z * v[e].z + v[e].w * v[e].w;
   }
   ss = block_reduce<BLOCK, false>(ss, lds);
   // the reference divides by sqrt (pow(.., 0.5)); keep a true division for the 1e-4 bar
@@ -79,7 +117,7 @@ __global__ void __launch_bounds__(BLOCK * RPW) rmsnorm_kernel(RmsNormDesc d) {
       float4 o;
       o.x = v[e].x / rms; o.y = v[e].y / rms; o.z = v[e].z / rms; o.w = v[e].w / rms;
       if (d.gamma) {
-        const float4 g = *(const float4 *)(d.gamma + c);
+        const float4 g = EARLY ? gm[EARLY ? e : 0] : *(const float4 *)(d.gamma + c);
         o.x *= d.gamma_offset + g.x; o.y *= d.gamma_offset + g.y;
         o.z *= d.gamma_offset + g.z; o.w *= d.gamma_offset + g.w;
       }
@@ -117,6 +155,14 @@ __global__ void __launch_bounds__(BLOCK * RPW) rmsnorm_kernel(RmsNormDesc d) {
 template <bool PAIR>
 static void launch_rmsnorm_as(const LaunchCtx &lc, const RmsNormDesc &d) {
   // n % 4 == 0 and n <= 16384 are checked by the caller
+  if (d.x_slices) {  // (a block end of a product too small to fill the CUs: a workgroup to a row)
+    if (d.n <= 256) CG_LAUNCH(lc, (rmsnorm_kernel<64, 1, PAIR, 1, true>), d.rows, 64, d);
+    else if (d.n <= 1024) CG_LAUNCH(lc, (rmsnorm_kernel<256, 1, PAIR, 1, true>), d.rows, 256, d);
+    else if (d.n <= 2048) CG_LAUNCH(lc, (rmsnorm_kernel<512, 1, PAIR, 1, true>), d.rows, 512, d);
+    else if (d.n <= 4096) CG_LAUNCH(lc, (rmsnorm_kernel<1024, 1, PAIR, 1, true>), d.rows, 1024, d);
+    else CG_LAUNCH(lc, (rmsnorm_kernel<1024, 4, PAIR, 1, true>), d.rows, 1024, d);
+    return;
+  }
   if (d.rows >= 2048 && d.n <= 2048) {  // a wave per row, four rows per workgroup
     const uint32_t wgs = (d.rows + 3) / 4;
     if (d.n <= 256) CG_LAUNCH(lc, (rmsnorm_kernel<64, 1, PAIR, 4>), wgs, 256, d);
@@ -128,8 +174,9 @@ static void launch_rmsnorm_as(const LaunchCtx &lc, const RmsNormDesc &d) {
   }
   if (d.n <= 256) CG_LAUNCH(lc, (rmsnorm_kernel<64, 1, PAIR>), d.rows, 64, d);
   else if (d.n <= 1024) CG_LAUNCH(lc, (rmsnorm_kernel<256, 1, PAIR>), d.rows, 256, d);
-  else if (d.n <= 2048) CG_LAUNCH(lc, (rmsnorm_kernel<256, 2, PAIR>), d.rows, 256, d);
-  else if (d.n <= 4096) CG_LAUNCH(lc, (rmsnorm_kernel<256, 4, PAIR>), d.rows, 256, d);
+  // (a float4 to a thread, as in the form above that sums slices: the two give the same bits)
+  else if (d.n <= 2048) CG_LAUNCH(lc, (rmsnorm_kernel<512, 1, PAIR>), d.rows, 512, d);
+  else if (d.n <= 4096) CG_LAUNCH(lc, (rmsnorm_kernel<1024, 1, PAIR>), d.rows, 1024, d);
   else CG_LAUNCH(lc, (rmsnorm_kernel<1024, 4, PAIR>), d.rows, 1024, d);
 }
 
