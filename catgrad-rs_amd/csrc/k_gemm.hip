@@ -246,6 +246,7 @@ __global__ void __launch_bounds__(256) gemm_kernel(GemmDesc g, int a_vec, int b_
 
   // 32x32 accumulator layout: element e of a lane sits at
   //   row = (e / 4) * 8 + (lane / 32) * 4 + e % 4,  col = lane % 32
+  const bool act = g.act_sigmoid && g.splits <= 1;
 #pragma unroll
   for (int i = 0; i < 2; ++i)
 #pragma unroll
@@ -254,7 +255,7 @@ __global__ void __launch_bounds__(256) gemm_kernel(GemmDesc g, int a_vec, int b_
 #pragma unroll
       for (int e = 0; e < 16; ++e) {
         const uint32_t row = m0 + wm * 64 + i * 32 + (e >> 2) * 8 + (lane >> 5) * 4 + (e & 3);
-        if (row < g.M && col < g.N) C[(uint64_t)row * g.N + col] = acc[i][j][e];
+        if (row < g.M && col < g.N) C[(uint64_t)row * g.N + col] = act ? sigmoid_ref(acc[i][j][e]) : acc[i][j][e];
       }
     }
 }
@@ -335,8 +336,10 @@ __global__ void __launch_bounds__(256) gemm_small_f32_kernel(GemmDesc g, int a_v
   for (int i = tid; i < 1024; i += 256) {
     const int e = i >> 6, l = i & 63;
     const uint32_t row = m0 + (e >> 2) * 8 + (l >> 5) * 4 + (e & 3), col = n0 + (l & 31);
-    if (row < g.M && col < g.N)
-      C[(uint64_t)row * g.N + col] = (part[0][i] + part[1][i]) + (part[2][i] + part[3][i]);
+    if (row < g.M && col < g.N) {
+      const float v = (part[0][i] + part[1][i]) + (part[2][i] + part[3][i]);
+      C[(uint64_t)row * g.N + col] = g.act_sigmoid && g.splits <= 1 ? sigmoid_ref(v) : v;
+    }
   }
 }
 
@@ -732,6 +735,17 @@ __global__ void __launch_bounds__(WR *WC *KG * 64) gemm_bf16_dma_kernel(GemmDesc
         float4 gt[4];
         uint64_t at[4];
         bool live[4];
+        if (!DUAL && g.c16_pitch) {  // sigmoid as the next product's operand: whole rows of c16_pitch values
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            const uint32_t col = n0 + wn * WN + j * 32 + q * 8 + half * 4;
+            if (row >= g.M || col >= g.c16_pitch) continue;
+            const float4 v = make_float4(col < Nl ? sigmoid_fast(acc[i][j][q * 4]) : 0.f, col + 1 < Nl ? sigmoid_fast(acc[i][j][q * 4 + 1]) : 0.f,
+                                         col + 2 < Nl ? sigmoid_fast(acc[i][j][q * 4 + 2]) : 0.f, col + 3 < Nl ? sigmoid_fast(acc[i][j][q * 4 + 3]) : 0.f);
+            *(uint2 *)(C16 + (uint64_t)row * g.c16_pitch + col) = bf16_pack4(v);
+          }
+          continue;
+        }
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
           const uint32_t col = n0 + (DUAL ? wn * OC : wn * WN) + j * 32 + q * 8 + half * 4;
@@ -760,6 +774,8 @@ __global__ void __launch_bounds__(WR *WC *KG * 64) gemm_bf16_dma_kernel(GemmDesc
               v.x *= gt[q].x * sigmoid_ref(gt[q].x); v.y *= gt[q].y * sigmoid_ref(gt[q].y);
               v.z *= gt[q].z * sigmoid_ref(gt[q].z); v.w *= gt[q].w * sigmoid_ref(gt[q].w);
             }
+          } else if (g.act_sigmoid) {
+            v = make_float4(sigmoid_ref(v.x), sigmoid_ref(v.y), sigmoid_ref(v.z), sigmoid_ref(v.w));
           }
           if (!DUAL || g.c) *(float4 *)(C + at[q]) = v;
           if (C16) *(uint2 *)(C16 + at[q]) = bf16_pack4(v);
@@ -913,7 +929,7 @@ static hipError_t launch_gemm_dma(const LaunchCtx &lc, const GemmDesc &g, uint32
 // C = sum over splits of workspace[split] (float4 per thread; sizes are multiples of 4 or the
 // tail is handled scalar)
 __global__ void __launch_bounds__(256) splitk_reduce_kernel(const float *ws, float *c, uint64_t n,
-                                                            uint32_t splits, const float *cadd) {
+                                                            uint32_t splits, const float *cadd, int act) {
   const uint64_t n4 = n / 4;
   for (uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x; i < n4;
        i += (uint64_t)gridDim.x * 256) {
@@ -926,13 +942,15 @@ __global__ void __launch_bounds__(256) splitk_reduce_kernel(const float *ws, flo
       const float4 v = ((const float4 *)cadd)[i];
       s.x += v.x; s.y += v.y; s.z += v.z; s.w += v.w;
     }
+    if (act) s = make_float4(sigmoid_ref(s.x), sigmoid_ref(s.y), sigmoid_ref(s.z), sigmoid_ref(s.w));
     ((float4 *)c)[i] = s;
   }
   if (blockIdx.x == 0 && threadIdx.x < (n & 3)) {
     const uint64_t i = n4 * 4 + threadIdx.x;
     float s = ws[i];
     for (uint32_t k = 1; k < splits; ++k) s += ws[(uint64_t)k * n + i];
-    c[i] = s + (cadd ? cadd[i] : 0.f);
+    s += cadd ? cadd[i] : 0.f;
+    c[i] = act ? sigmoid_ref(s) : s;
   }
 }
 
@@ -1019,6 +1037,54 @@ hipError_t launch_transpose_cast_bf16(const LaunchCtx &lc, const void *b, int b_
   } else {
     if (vec) CG_LAUNCH(lc, (transpose_cast_bf16_kernel<float, true>), grid, 256, (const float *)b, (uint16_t *)out, K, Kp, N, sbk, nb1, sb_b0, sb_b1);
     else CG_LAUNCH(lc, (transpose_cast_bf16_kernel<float, false>), grid, 256, (const float *)b, (uint16_t *)out, K, Kp, N, sbk, nb1, sb_b0, sb_b1);
+  }
+  return hipGetLastError();
+}
+
+// Rows with unit stride along k copied for the direct-to-LDS GEMM: bf16, a pitch of Kp (a multiple of 64), zeros past K.
+// Bound by the copy; a thread stores 16 bytes and reads them in 16-byte pieces where VEC says the rows are aligned.
+template <typename T, bool VEC>
+__global__ void __launch_bounds__(256) pack_rows_bf16_kernel(const T *src, uint16_t *out, uint32_t rows, uint32_t K, uint32_t Kp,
+                                                             int64_t stride, uint32_t nb1, int64_t s_b0, int64_t s_b1) {
+  const uint32_t b0 = blockIdx.y / nb1, b1 = blockIdx.y - b0 * nb1, per = Kp / 8;
+  src += b0 * s_b0 + b1 * s_b1;
+  out += (uint64_t)blockIdx.y * rows * Kp;
+  const uint64_t n = (uint64_t)rows * per;
+  for (uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (uint64_t)gridDim.x * 256) {
+    const uint32_t r = (uint32_t)(i / per), k = (uint32_t)(i - (uint64_t)r * per) * 8;
+    const T *p = src + (int64_t)r * stride + k;
+    uint4 q;
+    if (VEC && k + 8 <= K) {
+      if (sizeof(T) == 2) {
+        q = *(const uint4 *)p;
+      } else {
+        const uint2 lo = bf16_pack4(*(const float4 *)p), hi = bf16_pack4(*((const float4 *)p + 1));
+        q = make_uint4(lo.x, lo.y, hi.x, hi.y);
+      }
+    } else {
+      uint32_t v[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) v[j] = k + j < K ? (sizeof(T) == 2 ? (uint32_t)p[j] : bf16_bits((float)p[j])) : 0u;
+      q = make_uint4(v[0] | v[1] << 16, v[2] | v[3] << 16, v[4] | v[5] << 16, v[6] | v[7] << 16);
+    }
+    *(uint4 *)(out + (uint64_t)r * Kp + k) = q;
+  }
+}
+
+hipError_t launch_pack_rows_bf16(const LaunchCtx &lc, const void *src, int stype, void *out, uint32_t rows, uint32_t k, uint32_t kp,
+                                 int64_t stride, uint32_t nb0, uint32_t nb1, int64_t s_b0, int64_t s_b1) {
+  if (!rows || !k || !nb0 || !nb1) return hipSuccess;
+  if (kp < k || kp % 8 || (uint64_t)nb0 * nb1 > 65535) return hipErrorInvalidValue;
+  const uint64_t blocks = ((uint64_t)rows * (kp / 8) + 255) / 256, cap = (uint64_t)lc.n_cus * 32;
+  const dim3 grid((unsigned)(blocks < cap ? blocks : cap), nb0 * nb1);
+  const int al = stype == ST_BF16 ? 8 : 4;  // elements of 16 bytes
+  const bool vec = (uintptr_t)src % 16 == 0 && stride % al == 0 && s_b0 % al == 0 && s_b1 % al == 0;
+  if (stype == ST_BF16) {
+    if (vec) CG_LAUNCH(lc, (pack_rows_bf16_kernel<uint16_t, true>), grid, 256, (const uint16_t *)src, (uint16_t *)out, rows, k, kp, stride, nb1, s_b0, s_b1);
+    else CG_LAUNCH(lc, (pack_rows_bf16_kernel<uint16_t, false>), grid, 256, (const uint16_t *)src, (uint16_t *)out, rows, k, kp, stride, nb1, s_b0, s_b1);
+  } else {
+    if (vec) CG_LAUNCH(lc, (pack_rows_bf16_kernel<float, true>), grid, 256, (const float *)src, (uint16_t *)out, rows, k, kp, stride, nb1, s_b0, s_b1);
+    else CG_LAUNCH(lc, (pack_rows_bf16_kernel<float, false>), grid, 256, (const float *)src, (uint16_t *)out, rows, k, kp, stride, nb1, s_b0, s_b1);
   }
   return hipGetLastError();
 }
@@ -2626,7 +2692,44 @@ bool gemm_epilogue_ok(const GemmDesc &g) {
   const int asz = g.a_stype == ST_BF16 ? 2 : 4, bsz = g.b_stype == ST_BF16 ? 2 : 4;
   const int av = vec_ok(g.a, asz, g.sak == 1 ? g.sam : g.sak, g.sa_b0, g.sa_b1);
   const int bv = vec_ok(g.b, bsz, g.sbk == 1 ? g.sbn : g.sbk, g.sb_b0, g.sb_b1);
-  return gemm_fast_path(g, av, bv) && gemm_dma_ok(g) && g.splits <= 1 && !g.b_index && !g.c_add && g.N % 4 == 0;
+  return gemm_fast_path(g, av, bv) && gemm_dma_ok(g) && g.splits <= 1 && !g.b_index && !g.c_add &&
+         (g.N % 4 == 0 || g.c16_pitch);
+}
+
+bool gemv_rows_plain_ok(const LaunchCtx &lc, const GemmDesc &g);
+bool gemm_act_ok(const LaunchCtx &lc, const GemmDesc &g) {
+  if (g.b_index || g.c_add || g.n_group || g.dual_b || g.glu_gate || g.defer_reduce || !g.K || g.M <= 8) return false;
+  if (g.c16_pitch) return g.nb0 * g.nb1 == 1 && g.c16_pitch % 64 == 0 && g.c16_pitch >= g.N && gemm_epilogue_ok(g);
+  if (gemv_rows_plain_ok(lc, g)) return false;
+  if (g.splits > 1) return true;  // the pass that sums the slices applies it
+  const int asz = g.a_stype == ST_BF16 ? 2 : 4, bsz = g.b_stype == ST_BF16 ? 2 : 4;
+  const int av = vec_ok(g.a, asz, g.sak == 1 ? g.sam : g.sak, g.sa_b0, g.sa_b1);
+  const int bv = vec_ok(g.b, bsz, g.sbk == 1 ? g.sbn : g.sbk, g.sb_b0, g.sb_b1);
+  return !gemm_fast_path(g, av, bv) || gemm_epilogue_ok(g);
+}
+
+// Copies of the operands in rows of a multiple of 64 bf16 values put a product of ragged sizes (K % 64, or rows that do
+// not start on 16 bytes) on the direct-to-LDS kernel.  Up to two launches of 3 - 8 us, against a generic kernel that
+// widens and rounds every element on its way into LDS, eight at a time: sigmoid(x W1) W2 of 64 x 128 x 256 x 10 in
+// 57 us without, 34 with the copies; 300 x 500 x 1000 x 50 145, 54; 1000 x 1000 x 1000 x 10 105, 65; 6000 x 1000 x 4100
+// x 100 802, 230 (the product 420 us at 117 TFLOP/s -> 76 us at 650).  Below PACK_MIN_FLOPS nothing was measured; operands
+// that gemm_bf16_nt_kernel reads in 16-byte pieces are copied from PACK_ALIGNED_MIN_FLOPS on only.
+constexpr double PACK_MIN_FLOPS = 1e5, PACK_ALIGNED_MIN_FLOPS = 8e9;
+bool gemm_pack_wanted(const GemmDesc &g, bool epilogue) {
+  const uint32_t batch = g.nb0 * g.nb1;
+  if (!g.bf16_math || g.b_index || !gemm_rows(g.M, g.K) || g.K < 64 || g.N < 8 || batch > 65535) return false;
+  if ((g.sak != 1 && g.sam != 1) || (g.sbk != 1 && g.sbn != 1)) return false;
+  if (2.0 * batch * g.M * g.N * g.K < PACK_MIN_FLOPS) return false;
+  GemmDesc t = g;  // (as it would run: f32 operands with unit strides along k are read from their bf16 twins)
+  const int asz = g.a_stype == ST_BF16 ? 2 : 4, bsz = g.b_stype == ST_BF16 ? 2 : 4;
+  const int av = vec_ok(g.a, asz, g.sak == 1 ? g.sam : g.sak, g.sa_b0, g.sa_b1);
+  const int bv = vec_ok(g.b, bsz, g.sbk == 1 ? g.sbn : g.sbk, g.sb_b0, g.sb_b1);
+  t.a_stype = t.b_stype = ST_BF16;
+  const bool as_it_lies = g.K % 64 == 0 && av && bv && g.sak == 1;
+  if (as_it_lies && g.sbk == 1) return false;
+  if (gemm_dma_bkm_ok(t)) return epilogue;  // (the k-major form has no epilogue)
+  // (both operands in 16-byte pieces already: gemm_bf16_nt_kernel reads them where they lie)
+  return epilogue || !gemm_fast_path(t, av, bv) || 2.0 * batch * g.M * g.N * g.K >= PACK_ALIGNED_MIN_FLOPS;
 }
 
 bool gemm_rope_epilogue_ok(const LaunchCtx &lc, const GemmDesc &g) {
@@ -2676,7 +2779,7 @@ hipError_t launch_splitk_sum(const LaunchCtx &lc, const float *ws, float *c, uin
   if (!n || !splits) return hipSuccess;
   if ((uintptr_t)ws % 16 || (uintptr_t)c % 16 || (cadd && (uintptr_t)cadd % 16) || (splits > 1 && n % 4)) return hipErrorInvalidValue;
   uint64_t blocks = (n / 4 + 255) / 256, cap = (uint64_t)lc.n_cus * 16;
-  CG_LAUNCH(lc, (splitk_reduce_kernel), (unsigned)(blocks < cap ? (blocks ? blocks : 1) : cap), 256, ws, c, n, splits, cadd);
+  CG_LAUNCH(lc, (splitk_reduce_kernel), (unsigned)(blocks < cap ? (blocks ? blocks : 1) : cap), 256, ws, c, n, splits, cadd, 0);
   return hipGetLastError();
 }
 
@@ -2736,6 +2839,7 @@ hipError_t launch_matmul(const LaunchCtx &lc_in, const GemmDesc &g, const char *
   if (g.b_index && !one_row) return hipErrorInvalidValue;
   if (g.c_add && !one_row && g.splits <= 1) return hipErrorInvalidValue;
   if ((g.glu_gate || g.c16 || g.n_group || g.dual_b) && !gemm_epilogue_ok(g)) return hipErrorInvalidValue;
+  if (g.act_sigmoid && !gemm_act_ok(lc_in, g)) return hipErrorInvalidValue;
   if (g.rope_s && !gemm_rope_epilogue_ok(lc_in, g)) return hipErrorInvalidValue;
 
   if (gemv_rows_plain_ok(lc_in, g)) {
@@ -2833,7 +2937,7 @@ hipError_t launch_matmul(const LaunchCtx &lc_in, const GemmDesc &g, const char *
         if (g.dual_b) {
           if (g.n_group || g.glu_gate || splits != 1) return hipErrorInvalidValue;
           e = launch_gemm_dma<64, 64, 2, 1, true, 8, true, false, false, 2>(lc, gg, (uint32_t)((g.N + 31) / 32 * batch));
-        } else if (g.glu_gate || g.c16) {
+        } else if (g.glu_gate || g.c16 || (g.act_sigmoid && splits == 1)) {
           e = launch_gemm_dma<64, 64, 2, 2, true, 8, false, false, false, 2>(lc, gg, (uint32_t)t64);
         } else if (g.rope_s && g.rope_hd > 64) {
           e = launch_gemm_dma<64, 128, 2, 2, false, 5, false, false, true, 2>(lc, gg, (uint32_t)((g.N + 127) / 128));
@@ -2853,8 +2957,9 @@ hipError_t launch_matmul(const LaunchCtx &lc_in, const GemmDesc &g, const char *
         else if (d128 * 2 <= (uint64_t)lc.n_cus)
           e = launch_gemm_dma<128, 128, 4, 2, true, 4, true>(lc, gg, (uint32_t)((uint64_t)((g.M + 127) / 128) * ((g.N + 63) / 64) * batch));
         else e = launch_gemm_dma<128, 256, 2, 4, true, 3, true>(lc, gg, (uint32_t)d128);
-      } else if (g.glu_gate || g.c16) {  // the epilogue variant stages a 128 x 128 tile
-        if (deep) e = launch_gemm_dma<128, 128, 2, 4, true, 4>(lc, gg, (uint32_t)t128);
+      } else if (g.glu_gate || g.c16 || (g.act_sigmoid && splits == 1)) {
+        if (g.act_sigmoid && t256 >= (uint64_t)lc.n_cus) e = launch_gemm_dma<256, 256, 2, 4, true, 2>(lc, gg, (uint32_t)t256);
+        else if (deep) e = launch_gemm_dma<128, 128, 2, 4, true, 4>(lc, gg, (uint32_t)t128);
         else e = launch_gemm_dma<128, 128, 2, 2, true, 2>(lc, gg, (uint32_t)t128);
       } else if (t256 >= (uint64_t)lc.n_cus && grp256) {
         // 256 x 256 tiles run one to a CU, 128 x 128 two to a CU: when the big tiles leave the last round of
@@ -2927,7 +3032,7 @@ hipError_t launch_matmul(const LaunchCtx &lc_in, const GemmDesc &g, const char *
       const uint64_t n = (uint64_t)batch * g.M * g.N;
       uint64_t blocks = (n / 4 + 255) / 256, cap = (uint64_t)lc.n_cus * 16;
       CG_LAUNCH(tail, (splitk_reduce_kernel), (unsigned)(blocks < cap ? (blocks ? blocks : 1) : cap), 256,
-                (const float *)g.workspace, g.c, n, splits, g.c_add);
+                (const float *)g.workspace, g.c, n, splits, g.c_add, (int)g.act_sigmoid);
     }
     return hipGetLastError();
   }
@@ -2937,7 +3042,7 @@ hipError_t launch_matmul(const LaunchCtx &lc_in, const GemmDesc &g, const char *
       const uint64_t n = (uint64_t)batch * g.M * g.N;
       uint64_t blocks = (n / 4 + 255) / 256, cap = (uint64_t)lc.n_cus * 16;
       CG_LAUNCH(tail, (splitk_reduce_kernel), (unsigned)(blocks < cap ? (blocks ? blocks : 1) : cap), 256,
-                (const float *)g.workspace, g.c, n, gsplits, g.c_add);
+                (const float *)g.workspace, g.c, n, gsplits, g.c_add, (int)g.act_sigmoid);
     }
   };
   if (gemm_small_ok(lc, g)) {

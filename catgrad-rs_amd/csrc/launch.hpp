@@ -321,6 +321,11 @@ struct GemmDesc {
   const float *glu_gate;
   int32_t glu_kind;
   uint16_t *c16;
+  // optional (gemm_act_ok): C = sigmoid(A . B).  With c16_pitch the sigmoid leaves as bf16 only, in rows of c16_pitch
+  // (a multiple of 64, at least N) values at c16 with zeros past column N: the left operand of the next product as the
+  // direct-to-LDS kernel reads it (c is not written; gemm_epilogue_ok, one batch)
+  int32_t act_sigmoid;
+  uint32_t c16_pitch;
   // optional (same conditions): a second B matrix laid out like b (same strides, same N).  The kernel computes
   // both products and stores C = act(A . b) * (A . dual_b) - gate_proj, up_proj and the gated activation of an
   // MLP in one launch; c may be null when only the bf16 copy c16 is wanted
@@ -356,6 +361,14 @@ uint32_t gemm_split_k(const LaunchCtx &lc, const GemmDesc &g);
 // whether launch_matmul would run this problem (splits as given) on the kernel that honours
 // glu_gate / c16
 bool gemm_epilogue_ok(const GemmDesc &g);
+// whether launch_matmul's kernel for this problem (splits as given) honours act_sigmoid
+bool gemm_act_ok(const LaunchCtx &lc, const GemmDesc &g);
+// whether a bf16-mode product is worth copies of its operands in the direct-to-LDS kernel's layout (epilogue: it has one
+// to run, which that kernel's k-major form cannot)
+bool gemm_pack_wanted(const GemmDesc &g, bool epilogue);
+// rows[b][r][k] (f32 or bf16, unit stride along k, rows `stride` apart) -> bf16 rows of kp >= k values, zeros past k
+hipError_t launch_pack_rows_bf16(const LaunchCtx &lc, const void *src, int stype, void *out, uint32_t rows, uint32_t k, uint32_t kp,
+                                 int64_t stride, uint32_t nb0, uint32_t nb1, int64_t s_b0, int64_t s_b1);
 // whether launch_matmul would run this grouped problem on the tile whose epilogue honours rope_role
 bool gemm_rope_epilogue_ok(const LaunchCtx &lc, const GemmDesc &g);
 hipError_t launch_matmul(const LaunchCtx &lc, const GemmDesc &g, const char **kernel_name);

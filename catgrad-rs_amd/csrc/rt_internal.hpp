@@ -540,6 +540,9 @@ struct MatmulEpilogue {
   // kernel then computes both products and stores act(A . dual_w) * (A . B)
   cg_tensor *dual_w = nullptr;
   int gelu = 0;
+  // or: sigmoid(product); with packed as bf16 rows padded to a multiple of 64 values, the left operand of a product (the
+  // node then holds a strided bf16 value)
+  bool sigmoid = false, packed = false;
   bool applied = false;
 };
 

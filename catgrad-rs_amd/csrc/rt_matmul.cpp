@@ -656,6 +656,28 @@ int realize_matmul(cg_backend *be, cg_tensor *n, cg_tensor *addend, bool *added,
     TRY(peel_repeat_kv(be, n->in[1], &B, &pb));
     if (!pb) TRY(peel_repeat_kv(be, n->in[0], &A, &pa));
   }
+  // The left operand is sigmoid(product) that nobody else reads, in bf16 mode: that product's launch leaves the sigmoid as
+  // this one's operand (6000 x 4100 values: no f32 product, sigmoid pass and bf16 copy; 330 MB less to move).
+  bool a_packed = false;
+  if (!pa && !pb && !ex.w && (be->flags & CG_FLAG_BF16) && !(be->flags & CG_FLAG_NO_PATTERNS) && n->dtype == CG_F32 && n->rank >= 2) {
+    const cg_tensor *arg = nullptr;
+    cg_tensor *act = n->in[0];
+    if (is_sigmoid_of(act, &arg) && arg->op == N_MATMUL && refs(arg) == 1 && arg->dtype == CG_F32 && !arg->gemv_candidate &&
+        arg->rank == n->rank && arg->size() == arg->shape[arg->rank - 2] * arg->shape[arg->rank - 1]) {
+      cg_tensor *mm = retain(const_cast<cg_tensor *>(arg));
+      MatmulEpilogue sep;
+      sep.sigmoid = sep.packed = true;
+      const int st = realize_matmul(be, mm, nullptr, nullptr, &sep);
+      if (st || !sep.applied) {
+        node_release(mm);
+        if (st) return st;
+      } else {  // mm holds the activations: it takes the chain's place
+        n->in[0] = mm;
+        node_release(act);
+        a_packed = true;
+      }
+    }
+  }
   if (!pa) {
     TRY(realize(be, n->in[0]));
     A.set(retain(n->in[0]));
@@ -759,6 +781,54 @@ int realize_matmul(cg_backend *be, cg_tensor *n, cg_tensor *addend, bool *added,
     g.sb_b0 = sbo[0];
     g.sb_b1 = sbo[1];
     g.bf16_math = (be->flags & CG_FLAG_BF16) ? 1 : 0;
+    Storage *packs[2] = {nullptr, nullptr};  // copies of the operands for the direct-to-LDS kernel
+    {
+      if (!ex.w && n->dtype == CG_F32 && gemm_pack_wanted(g, ep && ep->sigmoid)) {
+        const uint32_t Kp = (K + 63) / 64 * 64;
+        const bool keep_a = g.a_stype == ST_BF16 && g.sak == 1 && (uintptr_t)g.a % 16 == 0 && g.sam % 8 == 0 && g.sa_b0 % 8 == 0 &&
+                            g.sa_b1 % 8 == 0 && (K == Kp || (a_packed && g.sam == (int64_t)Kp));
+        const bool keep_b = K == Kp && g.b_stype == ST_BF16 && g.sbk == 1 && (uintptr_t)g.b % 16 == 0 && g.sbn % 8 == 0 &&
+                            g.sb_b0 % 8 == 0 && g.sb_b1 % 8 == 0;
+        const uint32_t ab0 = g.sa_b0 ? g.nb0 : 1, ab1 = g.sa_b1 ? g.nb1 : 1, bb0 = g.sb_b0 ? g.nb0 : 1, bb1 = g.sb_b1 ? g.nb1 : 1;
+        // (no room for the copies: the general kernels read the operands as they are)
+        const bool room = (keep_a || dev_alloc(be, (size_t)ab0 * ab1 * M * Kp * 2, &packs[0]) == CG_OK) &&
+                          (keep_b || dev_alloc(be, (size_t)bb0 * bb1 * N * Kp * 2, &packs[1]) == CG_OK);
+        hipError_t pe = hipSuccess;
+        if (room) {
+          KernelScope ks(be, "pack_bf16", (double)(keep_a ? 0 : ab0 * ab1) * M * K * (esize(g.a_stype) + 2) +
+                                              (double)(keep_b ? 0 : bb0 * bb1) * N * K * (esize(g.b_stype) + 2), 0);
+          if (!keep_a)
+            pe = g.sak == 1 ? launch_pack_rows_bf16(be->lc(), g.a, g.a_stype, packs[0]->ptr, M, K, Kp, g.sam, ab0, ab1, g.sa_b0, g.sa_b1)
+                            : launch_transpose_cast_bf16(be->lc(), g.a, g.a_stype, packs[0]->ptr, K, Kp, M, g.sak, ab0, ab1, g.sa_b0, g.sa_b1);
+          if (!keep_b && pe == hipSuccess)
+            pe = g.sbk == 1 ? launch_pack_rows_bf16(be->lc(), g.b, g.b_stype, packs[1]->ptr, N, K, Kp, g.sbn, bb0, bb1, g.sb_b0, g.sb_b1)
+                            : launch_transpose_cast_bf16(be->lc(), g.b, g.b_stype, packs[1]->ptr, K, Kp, N, g.sbk, bb0, bb1, g.sb_b0, g.sb_b1);
+          if (!keep_a) {
+            g.a = packs[0]->ptr;
+            g.a_stype = ST_BF16;
+            g.sak = 1;
+            g.sam = Kp;
+            g.sa_b1 = g.sa_b1 ? (int64_t)M * Kp : 0;
+            g.sa_b0 = g.sa_b0 ? (int64_t)ab1 * M * Kp : 0;
+          }
+          if (!keep_b) {
+            g.b = packs[1]->ptr;
+            g.b_stype = ST_BF16;
+            g.sbk = 1;
+            g.sbn = Kp;
+            g.sb_b1 = g.sb_b1 ? (int64_t)N * Kp : 0;
+            g.sb_b0 = g.sb_b0 ? (int64_t)bb1 * N * Kp : 0;
+          }
+          g.K = Kp;
+        }
+        if (!room || pe != hipSuccess) {
+          storage_release(packs[0]);
+          storage_release(packs[1]);
+          packs[0] = packs[1] = nullptr;
+          HIPCHK(be, pe);
+        }
+      }
+    }
     // B with unit stride along n (bmm of row-major matrices, p . V): re-laid out once as bf16 [N, K]
     // so that the product takes the direct-to-LDS kernel (one pass over B against K/64 strided ones)
     Storage *bt = nullptr;
@@ -1034,11 +1104,37 @@ int realize_matmul(cg_backend *be, cg_tensor *n, cg_tensor *addend, bool *added,
     Storage *ws = nullptr;
     const bool dual = ep && ep->dual_w;  // twice the work per tile: no k-slices on top
     const uint32_t splits = group.empty() && !dual ? gemm_split_k(be->lc(), g) : 1;
+    if (ep && ep->sigmoid && group.empty()) {
+      GemmDesc t = g;
+      t.act_sigmoid = 1;
+      t.splits = splits;
+      if (ep->packed) {  // (a product split along k leaves the sigmoid of its sum as f32)
+        t.c16_pitch = (N + 63) / 64 * 64;
+        Storage *st = nullptr;
+        if (splits == 1 && batch == 1 && gemm_act_ok(be->lc(), t) && dev_alloc(be, (size_t)M * t.c16_pitch * 2, &st) == CG_OK) {
+          storage_release(n->st);
+          n->st = st;
+          n->stype = ST_BF16;
+          n->offset = 0;
+          for (int i = 0; i < r; ++i) n->strides[i] = i == r - 1 ? 1 : i == r - 2 ? t.c16_pitch : (int64_t)M * t.c16_pitch;
+          t.c = nullptr;
+          t.c16 = (uint16_t *)st->ptr;
+          t.splits = 0;
+          g = t;
+          ep->applied = true;
+        }
+        t.c16_pitch = 0;
+      }
+      if (!ep->applied && !g.c_add && gemm_act_ok(be->lc(), t)) {
+        g.act_sigmoid = 1;
+        ep->applied = true;
+      }
+    }
     if (splits > 1) {
       TRY(dev_alloc(be, (size_t)splits * n->size() * 4, &ws));
       g.workspace = (float *)ws->ptr;
       g.splits = splits;
-      g.k_per_split = ((K + splits - 1) / splits + 63) / 64 * 64;
+      g.k_per_split = ((g.K + splits - 1) / splits + 63) / 64 * 64;
       if (addend && !be->addend_is_row && !g.c_add && !g.b_index) {  // the pass that sums the k-slices adds the residual too
         g.c_add = (const float *)data_ptr(addend);
         *added = true;
@@ -1060,7 +1156,7 @@ int realize_matmul(cg_backend *be, cg_tensor *n, cg_tensor *addend, bool *added,
         g.c16 = (uint16_t *)n->st->ptr;
         ep->applied = true;
       }
-    } else if (ep && !g.c_add && gemm_epilogue_ok(g)) {
+    } else if (ep && !ep->sigmoid && !g.c_add && gemm_epilogue_ok(g)) {
       g.glu_gate = ep->gate;
       g.glu_kind = ep->gelu;
       (void)twin_for_result(be, n, &g.c16);  // the gated activations are down_proj's operand
@@ -1106,6 +1202,8 @@ int realize_matmul(cg_backend *be, cg_tensor *n, cg_tensor *addend, bool *added,
       storage_release(ws);
     }
     storage_release(bt);
+    storage_release(packs[0]);
+    storage_release(packs[1]);
     HIPCHK(be, e);
   }
   if (n->gemv_candidate) forget_gemv_candidate(n);

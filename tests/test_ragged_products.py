@@ -1,0 +1,71 @@
+"""Products of sizes that are no multiple of a tile or of 16 bytes in bf16 mode: operands copied to padded rows for the
+direct-to-LDS kernel, from every storage order; and sigmoid(product), stored by the product's launch as f32, as the next
+product's bf16 operand, or by the pass that sums the k-slices."""
+import numpy as np
+import pytest
+
+import parity
+import vectors
+
+lang, nn = vectors.cg.lang, vectors.cg.nn
+
+
+def mlp(b, x, w1, w2):
+    return [lang.matmul(b, nn.sigmoid(b, lang.matmul(b, x, w1)), w2)]
+
+
+def sigmoid_of_product(b, x, w1):
+    return [nn.sigmoid(b, lang.matmul(b, x, w1))]
+
+
+def transposed(b, x, w):   # x [.., k, m], w [.., n, k]
+    return [lang.matmul(b, lang.transpose(b, 1, 2, x), lang.transpose(b, 1, 2, w))]
+
+
+def plain(b, x, w):
+    return [lang.matmul(b, x, w)]
+
+
+def draw(g, shape, std):
+    return vectors.bf16_round((g.standard_normal(shape) * std).astype(np.float32))
+
+
+# below and above the size from which operands are copied; hidden sizes of one value past a tile, of a multiple of 64 and
+# with an odd tail; outputs of less than a tile; rows that end inside a tile
+SIZES = [(64, 128, 256, 10), (70, 100, 300, 17), (300, 200, 130, 64), (257, 999, 2050, 100), (513, 1000, 1027, 12),
+         (1000, 513, 1024, 99), (1030, 64, 8197, 65), (2100, 72, 4100, 10)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,inner,hidden,outer", SIZES)
+@pytest.mark.parametrize("bf16", [True, False])
+def test_hidden_layer(oracle, hip, hip_bf16, rows, inner, hidden, outer, bf16):
+    g = np.random.default_rng(rows)
+    x, w1, w2 = draw(g, (rows, inner), 1.0), draw(g, (inner, hidden), inner ** -0.5), draw(g, (hidden, outer), hidden ** -0.5)
+    (ref,) = vectors.run(oracle, mlp, 1, x, w1, w2)
+    (got,) = vectors.run(hip_bf16 if bf16 else hip, mlp, 1, x, w1, w2)
+    (parity.assert_bf16 if bf16 else parity.assert_f32)(ref, got, f"{rows}x{inner}x{hidden}x{outer}")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,inner,hidden", [(9, 40, 33), (64, 2048, 64), (100, 300, 77), (600, 256, 640), (777, 1001, 905)])
+@pytest.mark.parametrize("bf16", [True, False])
+def test_sigmoid_of_a_product(oracle, hip, hip_bf16, rows, inner, hidden, bf16):
+    g = np.random.default_rng(rows)
+    x, w = draw(g, (rows, inner), 1.0), draw(g, (inner, hidden), inner ** -0.5)
+    x[0, :] = 200.0 * np.sign(w[:, 0])      # a sum far into both tails
+    x[1, :] = -x[0, :]
+    (ref,) = vectors.run(oracle, sigmoid_of_product, 1, x, w)
+    (got,) = vectors.run(hip_bf16 if bf16 else hip, sigmoid_of_product, 1, x, w)
+    (parity.assert_bf16 if bf16 else parity.assert_f32)(ref, got, f"{rows}x{inner}x{hidden}")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("batch,m,n,k", [(1, 700, 900, 801), (3, 260, 516, 1002), (2, 1001, 300, 904), (1, 515, 1030, 1024)])
+@pytest.mark.parametrize("turned", [True, False])
+def test_ragged_operands_of_either_order(oracle, hip_bf16, batch, m, n, k, turned):
+    g = np.random.default_rng(m)
+    x, w = draw(g, (batch, k, m) if turned else (batch, m, k), 1.0), draw(g, (batch, n, k) if turned else (batch, k, n), k ** -0.5)
+    (ref,) = vectors.run(oracle, transposed if turned else plain, 1, x, w)
+    (got,) = vectors.run(hip_bf16, transposed if turned else plain, 1, x, w)
+    parity.assert_bf16(ref, got, f"{batch}x{m}x{n}x{k}")
