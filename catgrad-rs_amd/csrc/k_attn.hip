@@ -81,24 +81,111 @@ struct KeyTiles {
 
 constexpr float ATTN_MAX_SLACK = 8.0f;
 
-// BN keys per step; the K / V rows and the mask values of step i+1 are fetched into registers while
-// step i is being computed, so global latency is paid once per workgroup, not once per step.
+// One step of the online softmax: the scores S^T of KT x 32 keys (register e of tile kt is key t0 + kt*32 + (e>>2)*8 +
+// half*4 + (e&3)) become the B fragments of the second product, and the row's maximum and sum move on.  `l` sums this
+// lane's keys only: the two lanes of a query meet after the last step.  Returns the factor O has to be rescaled by.
+//
+// Most steps of a causal or sliding-window layer read no mask and have no key past the end: there a score costs a
+// maximum, one fma and an exp2 (the scale and log2 e in the factor; the scale is positive there), a sum and half a
+// conversion.  One path with the tail's and the mask's selects took 541 vector instructions for 32 scores a lane; this one
+// takes 110.  With it, one barrier a step and the long query tiles first: 2900 tokens of 32 heads of 64 212 -> 96 us a
+// layer, 8 x 2048 of 4 heads of 256 227 -> 168, 4 x 256 of 16 heads of 128 26.6 -> 22.7, 512 of 32 heads of 64 17.0 -> 14.9.
+template <int KT>
+__device__ __forceinline__ float attn_softmax_step(const AttnPrefillDesc &a, a_f32x16 (&st)[KT], const float4 (&mask)[KT][4],
+                                                   a_bf16x8 (&pf)[KT * 2], float &m_run, float &l_run, float inv_scale, bool plain,
+                                                   bool use_mask, uint32_t t0, int half) {
+  constexpr float LOG2E = 1.44269504f, LOWEST = -3.40282347e+38f;
+  float tmax = LOWEST, alpha, psum = 0.f;
+  if (plain) {
+#pragma unroll
+    for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) tmax = fmaxf(tmax, st[kt][e]);
+    tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64)) * inv_scale;
+    const float m_new = tmax > m_run + ATTN_MAX_SLACK ? tmax : m_run;
+    alpha = __expf(m_run - m_new);
+    m_run = m_new;
+    const float c = inv_scale * LOG2E, ref = fmaxf(m_new * LOG2E, LOWEST);
+#pragma unroll
+    for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+      for (int blk = 0; blk < 2; ++blk) {
+        float p[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          p[i] = __builtin_amdgcn_exp2f(__builtin_fmaf(st[kt][blk * 8 + i], c, -ref));
+          psum += p[i];
+        }
+        pf[kt * 2 + blk] = pack8(p);
+      }
+  } else {
+    const bool tail = t0 + KT * 32 > a.t;  // the only step with keys past the end (uniform)
+#pragma unroll
+    for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const uint32_t key = t0 + kt * 32 + j * 8 + half * 4;
+        float mv[4] = {0.f, 0.f, 0.f, 0.f};
+        if (use_mask) { mv[0] = mask[kt][j].x; mv[1] = mask[kt][j].y; mv[2] = mask[kt][j].z; mv[3] = mask[kt][j].w; }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          float v = st[kt][j * 4 + i];
+          if (a.has_scale) v = v * inv_scale;
+          if (use_mask) v = v + mv[i];
+          else if (!a.mask && a.has_mask_const) v = v + a.mask_const;
+          if (tail && key + i >= a.t) v = LOWEST;  // past the end: contributes exp(..) = 0
+          st[kt][j * 4 + i] = v;
+          tmax = fmaxf(tmax, v);
+        }
+      }
+    tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
+    const float m_new = tmax > m_run + ATTN_MAX_SLACK ? tmax : m_run;
+    alpha = __expf(m_run - m_new);
+    m_run = m_new;
+#pragma unroll
+    for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+      for (int blk = 0; blk < 2; ++blk) {
+        float p[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          const uint32_t key = t0 + kt * 32 + (blk * 2 + (i >> 2)) * 8 + half * 4 + (i & 3);
+          p[i] = __expf(st[kt][blk * 8 + i] - m_new);
+          if (tail && key >= a.t) p[i] = 0.f;
+          psum += p[i];
+        }
+        pf[kt * 2 + blk] = pack8(p);
+      }
+  }
+  l_run = l_run * alpha + psum;
+  return alpha;
+}
+
+// BN keys per step.  The K / V rows of step i + 1 are in registers, asked for a step ago, while step i is computed from
+// one LDS buffer, and go to the other buffer behind its first product: one barrier per step.
 // NW waves of 32 queries each per workgroup (4, or 2 when that is what it takes to occupy the CUs).
+// Workgroups: the query tiles with the most keys first (a causal mask gives the last tile all of them), and the heads of a
+// (batch, kv head) on one XCD, whose L2 then holds their keys and values.
+// (the register budget of two waves to a SIMD keeps the accumulators of heads of 64 and 128 out of the accumulation file,
+// 64 moves a step; three waves spill 20 bytes: 109 us where two take 96)
+#define ATTN_WAVES(D) __attribute__((amdgpu_waves_per_eu(D <= 128 ? 2 : 1, D <= 128 ? 2 : 1)))
 template <int D, int BN, int NW>
-__global__ void __launch_bounds__(NW * 64) attn_prefill_kernel(AttnPrefillDesc a) {
+__global__ void __launch_bounds__(NW * 64) ATTN_WAVES(D) attn_prefill_kernel(AttnPrefillDesc a) {
   constexpr int NT = NW * 64;
   constexpr int KP = D + 8;              // K tile row pitch (bf16 elements)
   constexpr int VP = BN + 8;             // V^T tile row pitch
   constexpr int DT = D / 32;             // 32-row tiles of O^T
   constexpr int KT = BN / 32;            // 32-key tiles of S^T
   constexpr int KCH = BN * D / 8 / NT;   // 16-byte chunks of the K tile / of the V^T tile per thread
-  __shared__ __attribute__((aligned(16))) uint16_t Ks[BN * KP];
-  __shared__ __attribute__((aligned(16))) uint16_t Vt[D * VP];
+  __shared__ __attribute__((aligned(16))) uint16_t tile[2][BN * KP + D * VP];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int col = lane & 31, half = lane >> 5;
-  const uint32_t h = blockIdx.y, b = blockIdx.z;
+  const uint32_t n_bh = a.heads * a.b, q_tiles = (a.s + NW * 32 - 1) / (NW * 32);
+  const uint32_t rank = blockIdx.x / n_bh, slot = blockIdx.x - rank * n_bh, q_tile = q_tiles - 1 - rank;
+  const uint32_t bh = n_bh % 8 == 0 ? (slot % 8) * (n_bh / 8) + slot / 8 : slot;
+  const uint32_t b = bh / a.heads, h = bh - b * a.heads;
   const uint32_t kvh = h / a.rep, rp = h % a.rep;
-  const uint32_t query = blockIdx.x * (NW * 32) + wave * 32 + col;
+  const uint32_t query = q_tile * (NW * 32) + wave * 32 + col;
   const bool q_ok = query < a.s;
   const uint32_t qc = q_ok ? query : a.s - 1;  // loads of lanes past the end go to a valid row
   const float *Q = a.q + (int64_t)b * a.q_sb + (int64_t)h * a.q_sh + (int64_t)qc * a.q_ss;
@@ -108,6 +195,40 @@ __global__ void __launch_bounds__(NW * 64) attn_prefill_kernel(AttnPrefillDesc a
   const uint16_t *VT = a.vt16 + ((int64_t)b * (a.heads / a.rep) + kvh) * D * (int64_t)a.vt_st;
   const float *V = a.v + (int64_t)b * a.v_sb + (int64_t)kvh * a.v_skv + (int64_t)rp * a.v_srep;
   const float *M = a.mask ? a.mask + (int64_t)b * a.m_sb + (int64_t)h * a.m_sh + (int64_t)qc * a.m_ss : nullptr;
+
+  typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+  u32x4 kreg[KCH], vreg[KCH];  // the step in flight
+  // All loads are unconditional (indices clamped into range) so that they are issued back to back;
+  // chunks past the end are zeroed when the registers are consumed.
+  // With a class table, dead key tiles are never visited and all-zero ones need no mask values.
+  const KeyTiles<BN> tiles(a, q_tile, lane);
+  auto fetch = [&](uint32_t t0) {
+#pragma unroll
+    for (int c = 0; c < KCH; ++c) {
+      const int ch = tid + c * NT, key = ch / (D / 8), d8 = (ch % (D / 8)) * 8;
+      kreg[c] = *(const u32x4 *)(K + (int64_t)min(t0 + key, a.t - 1) * a.k_st + d8);
+    }
+#pragma unroll
+    for (int c = 0; c < KCH; ++c) {
+      const int ch = tid + c * NT, dim = ch / (BN / 8), k8 = (ch % (BN / 8)) * 8;
+      vreg[c] = *(const u32x4 *)(VT + (int64_t)dim * a.vt_st + min(t0 + k8, a.vt_st - 8));
+    }
+  };
+  auto stash = [&](uint16_t *to, uint32_t t0) {  // registers -> LDS: K [BN, D] and V^T [D, BN]
+#pragma unroll
+    for (int c = 0; c < KCH; ++c) {
+      const int ch = tid + c * NT, key = ch / (D / 8), d8 = (ch % (D / 8)) * 8;
+      *(u32x4 *)(&to[key * KP + d8]) = kreg[c];  // (rows past the end repeat the last one: their scores are discarded)
+    }
+#pragma unroll
+    for (int c = 0; c < KCH; ++c) {
+      const int ch = tid + c * NT, dim = ch / (BN / 8), k8 = (ch % (BN / 8)) * 8;
+      const u32x4 none = {0u, 0u, 0u, 0u};
+      *(u32x4 *)(&to[BN * KP + dim * VP + k8]) = t0 + k8 < a.t ? vreg[c] : none;
+    }
+  };
+  uint32_t t0 = tiles.next_step(0), t_next = a.t;
+  if (t0 < a.t) fetch(t0);  // (uniform)
 
   // this lane's query row as B fragments: k-step ks covers dims 16 ks .. 16 ks + 15, half h takes 8
   a_bf16x8 qf[D / 16];
@@ -130,83 +251,30 @@ __global__ void __launch_bounds__(NW * 64) attn_prefill_kernel(AttnPrefillDesc a
     for (int e = 0; e < 16; ++e) o[t][e] = 0.f;
   float m_run = -3.40282347e+38f, l_run = 0.f;
   const float inv_scale = a.has_scale ? 1.0f / a.scale : 1.0f;  // bf16 mode: a product, not the reference's quotient
+  const bool can_be_plain = inv_scale > 0.f && (M || !a.has_mask_const);
 
-  // registers of the step in flight
-  uint4 kreg[KCH], vreg[KCH];
-  float4 mreg[KT][4];
-  // All loads are unconditional (indices clamped into range) so that they are issued back to back;
-  // chunks past the end are zeroed when the registers are consumed.
-  // With a class table, dead key tiles are never visited and all-zero ones need no mask values.
-  const KeyTiles<BN> tiles(a, blockIdx.x, lane);
-  auto next_step = [&](uint32_t t0) { return tiles.next_step(t0); };
-  auto step_mask = [&](uint32_t t0) { return M && tiles.reads_mask(t0); };
-  auto fetch = [&](uint32_t t0) {
-#pragma unroll
-    for (int c = 0; c < KCH; ++c) {
-      const int ch = tid + c * NT, key = ch / (D / 8), d8 = (ch % (D / 8)) * 8;
-      kreg[c] = *(const uint4 *)(K + (int64_t)min(t0 + key, a.t - 1) * a.k_st + d8);
-    }
-#pragma unroll
-    for (int c = 0; c < KCH; ++c) {
-      const int ch = tid + c * NT, dim = ch / (BN / 8), k8 = (ch % (BN / 8)) * 8;
-      vreg[c] = *(const uint4 *)(VT + (int64_t)dim * a.vt_st + min(t0 + k8, a.vt_st - 8));
-    }
-    if (step_mask(t0)) {  // mask rows allow 16-byte loads (checked by the host)
+  if (t0 < a.t) {
+    stash(tile[0], t0);
+    t_next = tiles.next_step(t0 + BN);
+    if (t_next < a.t) fetch(t_next);
+  }
+  __syncthreads();
+  for (int buf = 0; t0 < a.t; buf ^= 1) {
+    const uint16_t *Ks = tile[buf], *Vt = Ks + BN * KP;
+    const bool use_mask = M && tiles.reads_mask(t0);  // uniform
+    const bool plain = can_be_plain && !use_mask && t0 + BN <= a.t;
+    // The mask values of this step are asked for here and used after the score product; rows allow 16-byte loads
+    // (checked by the host).  A step whose every pair is masked - possible only without a class table - needs no
+    // special case: its weights exp(f32::MIN - m) are zero once any live key has been seen, and a row that never
+    // sees one is rebuilt at the end.
+    float4 mcur[KT][4];
+    if (use_mask) {
 #pragma unroll
       for (int kt = 0; kt < KT; ++kt)
 #pragma unroll
         for (int j = 0; j < 4; ++j)
-          mreg[kt][j] = *(const float4 *)(M + min(t0 + kt * 32 + j * 8 + half * 4, a.m_len - 4));
+          mcur[kt][j] = *(const float4 *)(M + min(t0 + kt * 32 + j * 8 + half * 4, a.m_len - 4));
     }
-  };
-  uint32_t t0 = next_step(0);
-  if (t0 < a.t) fetch(t0);
-  for (; t0 < a.t;) {
-    const uint32_t t_next = next_step(t0 + BN);
-    const bool use_mask = step_mask(t0);  // uniform
-    // ---- is any (query, key) pair of this step unmasked?  A causal or sliding-window mask kills
-    // most steps; a dead step only adds terms that the first live step rescales to zero.
-    const bool tail = t0 + BN > a.t;  // the only step with keys past the end (uniform)
-    bool live_pair = !use_mask;
-    float4 mcur[KT][4];
-    if (use_mask) {
-      float mmax = -3.40282347e+38f;
-#pragma unroll
-      for (int kt = 0; kt < KT; ++kt)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          mcur[kt][j] = mreg[kt][j];
-          float4 mk = mcur[kt][j];
-          if (tail) {
-            const uint32_t key = t0 + kt * 32 + j * 8 + half * 4;
-            if (key >= a.t) mk.x = -3.40282347e+38f;
-            if (key + 1 >= a.t) mk.y = -3.40282347e+38f;
-            if (key + 2 >= a.t) mk.z = -3.40282347e+38f;
-            if (key + 3 >= a.t) mk.w = -3.40282347e+38f;
-          }
-          mmax = fmaxf(mmax, fmaxf(fmaxf(mk.x, mk.y), fmaxf(mk.z, mk.w)));
-        }
-      live_pair = q_ok && mmax > -3.0e38f;
-    }
-    const bool live = __syncthreads_or(live_pair);  // also: the previous step's fragments have been read
-    if (live) {
-      // ---- registers -> LDS: K [BN, D] and V^T [D, BN]
-#pragma unroll
-      for (int c = 0; c < KCH; ++c) {
-        const int ch = tid + c * NT, key = ch / (D / 8), d8 = (ch % (D / 8)) * 8;
-        *(uint4 *)(&Ks[key * KP + d8]) = (t0 + key < a.t) ? kreg[c] : make_uint4(0u, 0u, 0u, 0u);
-      }
-#pragma unroll
-      for (int c = 0; c < KCH; ++c) {
-        const int ch = tid + c * NT, dim = ch / (BN / 8), k8 = (ch % (BN / 8)) * 8;
-        *(uint4 *)(&Vt[dim * VP + k8]) = (t0 + k8 < a.t) ? vreg[c] : make_uint4(0u, 0u, 0u, 0u);
-      }
-    }
-    __syncthreads();
-    if (t_next < a.t) fetch(t_next);  // in flight during the arithmetic below
-    const uint32_t t_cur = t0;
-    t0 = t_next;
-    if (!live) continue;
     // ---- S^T = K . Q^T
     a_f32x16 st[KT];
 #pragma unroll
@@ -219,51 +287,17 @@ __global__ void __launch_bounds__(NW * 64) attn_prefill_kernel(AttnPrefillDesc a
         st[kt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qf[ks], st[kt], 0, 0, 0);
       }
     }
-    // ---- scale, mask, running maximum.  Register e of tile kt is key t0 + kt*32 + (e>>2)*8 + half*4 + (e&3)
-    float tmax = -3.40282347e+38f;
-#pragma unroll
-    for (int kt = 0; kt < KT; ++kt)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const uint32_t key = t_cur + kt * 32 + j * 8 + half * 4;
-        float mv[4] = {0.f, 0.f, 0.f, 0.f};
-        if (use_mask) { mv[0] = mcur[kt][j].x; mv[1] = mcur[kt][j].y; mv[2] = mcur[kt][j].z; mv[3] = mcur[kt][j].w; }
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          float s = st[kt][j * 4 + i];
-          if (a.has_scale) s = s * inv_scale;
-          if (use_mask) s = s + mv[i];
-          else if (!M && a.has_mask_const) s = s + a.mask_const;
-          if (tail && key + i >= a.t) s = -3.40282347e+38f;  // past the end: contributes exp(..) = 0
-          st[kt][j * 4 + i] = s;
-          tmax = fmaxf(tmax, s);
-        }
-      }
-    tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
+    const uint32_t t_cur = t0, t_after = t_next < a.t ? tiles.next_step(t_next + BN) : a.t;
+    if (t_next < a.t) stash(tile[buf ^ 1], t_next);  // (everyone is past the barrier behind the last reads of that buffer)
+    if (t_after < a.t) fetch(t_after);
+    t0 = t_next;
+    t_next = t_after;
+    // ---- scale, mask, running maximum and sum; P^T as B fragments of the 16-key blocks.
     // The reference point of the exponentials only follows the maximum when that has moved by more than
     // ATTN_MAX_SLACK: the quotient O / l at the end does not depend on it, weights of up to e^slack are as
     // exact in f32 and bf16 as weights of up to 1, and O is rescaled on a few steps instead of on most.
-    const float m_new = tmax > m_run + ATTN_MAX_SLACK ? tmax : m_run;
-    const float alpha = __expf(m_run - m_new);
-    float psum = 0.f;
-    a_bf16x8 pf[KT * 2];  // P^T as B fragments of the 16-key blocks
-#pragma unroll
-    for (int kt = 0; kt < KT; ++kt)
-#pragma unroll
-      for (int blk = 0; blk < 2; ++blk) {
-        float p[8];
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          const uint32_t key = t_cur + kt * 32 + (blk * 2 + (i >> 2)) * 8 + half * 4 + (i & 3);
-          p[i] = __expf(st[kt][blk * 8 + i] - m_new);
-          if (tail && key >= a.t) p[i] = 0.f;
-          psum += p[i];
-        }
-        pf[kt * 2 + blk] = pack8(p);
-      }
-    psum += __shfl_xor(psum, 32, 64);
-    l_run = l_run * alpha + psum;
-    m_run = m_new;
+    a_bf16x8 pf[KT * 2];
+    const float alpha = attn_softmax_step<KT>(a, st, mcur, pf, m_run, l_run, inv_scale, plain, use_mask, t_cur, half);
     // ---- O^T = O^T * alpha + V^T . P^T
     if (__any(alpha != 1.0f)) {  // the running maximum moved for some query of this wave
 #pragma unroll
@@ -286,7 +320,9 @@ __global__ void __launch_bounds__(NW * 64) attn_prefill_kernel(AttnPrefillDesc a
         o[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf.hv, pf[blk], o[t], 0, 0, 0);
       }
     }
+    __syncthreads();
   }
+  l_run += __shfl_xor(l_run, 32, 64);
   // A row whose every key is masked has all scores equal to f32::MIN on the reference path:
   // uniform weights, i.e. the mean of V.  Dead steps were skipped above, so rebuild that here.
   if (M && q_ok && m_run <= -3.0e38f) {
@@ -410,6 +446,8 @@ attn_prefill_keysplit_kernel(AttnPrefillDesc a) {
   float m_run = -3.40282347e+38f, l_run = 0.f;
   const float inv_scale = a.has_scale ? 1.0f / a.scale : 1.0f;
 
+  const bool can_be_plain = inv_scale > 0.f && (M || !a.has_mask_const);
+
   while (t0 < a.t) {
     const uint32_t t_next = skip_steps(t0, NW);
     const bool use_mask = step_mask(t0);  // uniform over the wave
@@ -456,50 +494,8 @@ attn_prefill_keysplit_kernel(AttnPrefillDesc a) {
         st[kt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qf[ks], st[kt], 0, 0, 0);
       }
     }
-    float tmax = -3.40282347e+38f;
-#pragma unroll
-    for (int kt = 0; kt < KT; ++kt)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const uint32_t key = t_cur + kt * 32 + j * 8 + half * 4;
-        float mv[4] = {0.f, 0.f, 0.f, 0.f};
-        if (use_mask) { mv[0] = mcur[kt][j].x; mv[1] = mcur[kt][j].y; mv[2] = mcur[kt][j].z; mv[3] = mcur[kt][j].w; }
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          float s = st[kt][j * 4 + i];
-          if (a.has_scale) s = s * inv_scale;
-          if (use_mask) s = s + mv[i];
-          else if (!M && a.has_mask_const) s = s + a.mask_const;
-          if (tail && key + i >= a.t) s = -3.40282347e+38f;
-          st[kt][j * 4 + i] = s;
-          tmax = fmaxf(tmax, s);
-        }
-      }
-    tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
-    // The reference point of the exponentials only follows the maximum when that has moved by more than
-    // ATTN_MAX_SLACK: the quotient O / l at the end does not depend on it, weights of up to e^slack are as
-    // exact in f32 and bf16 as weights of up to 1, and O is rescaled on a few steps instead of on most.
-    const float m_new = tmax > m_run + ATTN_MAX_SLACK ? tmax : m_run;
-    const float alpha = __expf(m_run - m_new);
-    float psum = 0.f;
     a_bf16x8 pf[KT * 2];
-#pragma unroll
-    for (int kt = 0; kt < KT; ++kt)
-#pragma unroll
-      for (int blk = 0; blk < 2; ++blk) {
-        float p[8];
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          const uint32_t key = t_cur + kt * 32 + (blk * 2 + (i >> 2)) * 8 + half * 4 + (i & 3);
-          p[i] = __expf(st[kt][blk * 8 + i] - m_new);
-          if (tail && key >= a.t) p[i] = 0.f;
-          psum += p[i];
-        }
-        pf[kt * 2 + blk] = pack8(p);
-      }
-    psum += __shfl_xor(psum, 32, 64);
-    l_run = l_run * alpha + psum;
-    m_run = m_new;
+    const float alpha = attn_softmax_step<KT>(a, st, mcur, pf, m_run, l_run, inv_scale, can_be_plain && !use_mask && !tail, use_mask, t_cur, half);
     if (__any(alpha != 1.0f)) {
 #pragma unroll
       for (int t = 0; t < DT; ++t)
@@ -521,6 +517,7 @@ attn_prefill_keysplit_kernel(AttnPrefillDesc a) {
       }
     }
   }
+  l_run += __shfl_xor(l_run, 32, 64);
   // ---- the waves' partial results meet: [register][lane] floats in each wave's own region
   __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
   float *mine = (float *)(lds + wave * REGION);
@@ -898,9 +895,9 @@ hipError_t launch_attn_prefill(const LaunchCtx &lc, const AttnPrefillDesc &d) {
     CG_LAUNCH(lc, (attn_prefill_keysplit_kernel<64, 64, 4>), g32, 256, d);
     return hipGetLastError();
   }
-  dim3 grid((d.s + 127) / 128, d.heads, d.b);
   const bool small = attn_prefill_small_tiles(lc, d);
-  if (small) grid.x = (d.s + 63) / 64;
+  dim3 grid(small ? (d.s + 63) / 64 : (d.s + 127) / 128, d.heads, d.b);
+  if (!d.f32) grid = dim3(grid.x * d.heads * d.b);
 #define CG_ATTN_CASE(DD, ...)                                               \
   case DD:                                                                  \
     if (small) CG_LAUNCH(lc, (__VA_ARGS__, 2>), grid, 128, d);              \

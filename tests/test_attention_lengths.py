@@ -51,6 +51,27 @@ def test_attention_of_any_length(oracle, hip, hip_bf16, H, KV, S, d, window):
         check(ref, got, f"attention over {S} keys")
 
 
+# every pair visible: steps without mask values (a maximum over raw scores, the scale in the exponent) beside the ragged last
+# one; a scale that turns the order of the scores around, none at all, and scores that one key dominates
+@pytest.mark.gpu
+@pytest.mark.parametrize("H,KV,S,d", [(4, 2, 200, 64), (40, 8, 523, 64), (2, 1, 193, 128), (6, 3, 129, 256)])
+@pytest.mark.parametrize("scale,loud", [(8.0, 1.0), (-6.0, 1.0), (None, 0.2), (8.0, 60.0)])
+def test_attention_without_a_mask(oracle, hip_bf16, H, KV, S, d, scale, loud):
+    g = np.random.default_rng(S + d)
+    q, k, v = (vectors.bf16_round(g.standard_normal((1, h, S, d)).astype(np.float32)) for h in (H, KV, KV))
+    q = vectors.bf16_round(q * np.float32(loud))
+
+    def f(b, q, k, v):
+        q, k, v = q + q - q, k + k - k, v + v - v
+        attn = lang.matmul(b, q, lang.transpose(b, 2, 3, helpers.repeat_kv(b, H // KV, k)))
+        if scale is not None:
+            attn = attn / lang.constant(b, scale, lang.shape(b, attn))
+        return lang.matmul(b, nn.softmax(b, attn), helpers.repeat_kv(b, H // KV, v))
+    (ref,) = vectors.run(oracle, f, 1, q, k, v)
+    (got,) = vectors.run(hip_bf16, f, 1, q, k, v)
+    parity.assert_bf16(ref, got, f"{S} keys, scale {scale}")
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("tokens", [67, 259])
 def test_rotation_in_the_projections_launch_at_odd_lengths(oracle, hip_bf16, tokens):
