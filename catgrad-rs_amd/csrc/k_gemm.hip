@@ -343,11 +343,14 @@ __global__ void __launch_bounds__(256) gemm_small_f32_kernel(GemmDesc g, int a_v
   }
 }
 
-// few enough 32 x 32 tiles that the kernel above has the machine to itself
+// Few enough 32 x 32 tiles that the kernel above has the machine to itself, and each not too deep: a tile reads its 64 rows
+// of operands by itself, and 128 x 128 tiles split along k are ahead from tiles * K of about 400 000 on (500 x 1000 x 500
+// 18 us here, 30 there; 200 x 512 x 2048 21, 24; 400 x 512 x 2048 33, 27; 200 x 2048 x 2048 64, 36; 200 x 2048 x 8192 237,
+// 96) - unless most of such a tile's rows would be padding (16 x 2048 x 8192 34, 56; 40 x 8192 x 2048 59, 51).
 static bool gemm_small_ok(const LaunchCtx &lc, const GemmDesc &g) {
   if (g.bf16_math || g.a_stype != ST_F32 || g.b_stype != ST_F32 || g.M <= 8 || g.b_index || !g.K) return false;
   const uint64_t t32 = (uint64_t)((g.M + 31) / 32) * ((g.N + 31) / 32) * g.nb0 * g.nb1;
-  return t32 <= 2 * (uint64_t)lc.n_cus;
+  return t32 <= 2 * (uint64_t)lc.n_cus && (g.M <= 32 || t32 * g.K <= 400 * 1024);
 }
 
 // ---- bf16 x bf16 "NT" GEMM: the prefill fast path --------------------------------------------------
@@ -2802,7 +2805,10 @@ uint32_t gemm_split_k(const LaunchCtx &lc, const GemmDesc &g) {
   if (!gemm_fast_path(g, av, bv)) {
     // the generic kernel (f32 products): same idea, shorter k-steps, so thinner slices still pay
     if (g.M <= 8 || g.b_index || !g.K) return 1;
-    while (tiles * splits * 2 <= (uint64_t)lc.n_cus && g.K / (splits * 2) >= 256 && splits < 16) splits *= 2;
+    // (two workgroups to a CU, one's loads under the other's products: 700 x 2048 x 8192 357 -> 312 us, 400 x 2048 x 8192
+    // 185 -> 168; four k-steps at least to each: 1000 x 1000 x 1000 54 -> 36, 100 x 2048 x 2048 33 -> 27; four workgroups
+    // to a CU were slower throughout)
+    while (tiles * splits <= (uint64_t)lc.n_cus && g.K / (splits * 2) >= 128 && splits < 16) splits *= 2;
     return splits;
   }
   if (gemm_dma_ok(g) && g.M <= 64) {  // tiles of 64 x 64: a workgroup to every CU, four k-steps at least to each
