@@ -527,7 +527,7 @@ template <int N> __device__ __forceinline__ void wait_vmcnt() {
 template <int BM_, int BN_, int WR, int WC, bool EPI, int NS, bool DUAL = false, bool BKM = false, bool ROPE = false, int KG = 1>
 __global__ void __launch_bounds__(WR *WC *KG * 64) gemm_bf16_dma_kernel(GemmDesc g) {
   constexpr int NW = WR * WC * KG, BK = 64;
-  static_assert(!ROPE || (BN_ % 64 == 0 && !EPI && !DUAL && !BKM && (BM_ * BN_ / 4) % (NW * 64) == 0),
+  static_assert(!ROPE || ((BN_ % 64 == 0 || BN_ == 32) && !EPI && !DUAL && !BKM && (BM_ * BN_ / 4) % (NW * 64) == 0),
                 "rotated heads: whole heads of 64 columns per tile");
   static_assert(KG == 1 || (!BKM && 4 % KG == 0 && (KG - 1) * BM_ * BN_ * 4 <= NS * (BM_ + BN_) * 128), "k-groups");
   static_assert(!BKM || (!EPI && !DUAL && (BM_ / 8) % ((BM_ + BN_) / 8 / (WR * WC)) == 0), "k-major B: the plain product");
@@ -576,6 +576,10 @@ __global__ void __launch_bounds__(WR *WC *KG * 64) gemm_bf16_dma_kernel(GemmDesc
     Nl = g.grp_n[p];
     grp = p;
   }
+  // Columns of the tile.  (ROPE on 32 columns: 16 of a head's lower half and their partners in its upper half.)
+  constexpr bool PAIRS = ROPE && BN_ == 32;
+  const uint32_t pair_hd = PAIRS ? g.rope_hd : 64, pair_0 = PAIRS ? n0 / pair_hd * pair_hd + n0 % pair_hd / 2 : 0;
+  auto column = [&](uint32_t cl) { return PAIRS ? pair_0 + (cl & 15) + (cl >> 4) * (pair_hd / 2) : n0 + cl; };
   const float *Bias = g.n_group ? g.grp_bias[grp] : nullptr;
   const float *Gate = g.glu_gate ? g.glu_gate + (uint64_t)bz * g.M * g.N : nullptr;  // only without split-K
   uint16_t *C16 = g.c16 ? g.c16 + (uint64_t)bz * g.M * g.N : nullptr;
@@ -605,7 +609,7 @@ __global__ void __launch_bounds__(WR *WC *KG * 64) gemm_bf16_dma_kernel(GemmDesc
       const uint32_t n = n0 + (uint32_t)((pc ^ ((kr & 3) << 2)) * 8);
       gp[i] = B + (int64_t)(k_begin + kr) * g.sbk + min(n, Nl - 8);
     } else if (DUAL) gp[i] = (R - BM_ < BNO ? B : B2) + (int64_t)min(n0 + (uint32_t)((R - BM_) % BNO), Nl - 1) * g.sbn + k_begin + c * 8;
-    else gp[i] = B + (int64_t)min(n0 + (R - BM_), Nl - 1) * g.sbn + k_begin + c * 8;
+    else gp[i] = B + (int64_t)min(column(R - BM_), Nl - 1) * g.sbn + k_begin + c * 8;
   }
   // (k-major B: a wave's loads are all A's or all B's, and B's step down 64 rows per stage)
   const int64_t gp_step = BKM && wave * LPW * 8 >= BM_ ? (int64_t)BK * g.sbk : (int64_t)BK;
@@ -804,7 +808,7 @@ __global__ void __launch_bounds__(WR *WC *KG * 64) gemm_bf16_dma_kernel(GemmDesc
       const int64_t ss = g.rope_cs_ss[grp];
       auto table = [&](const float *tb, int it) {
         const int idx = it * NW * 64 + tid, r = idx / F4, c4 = (idx % F4) * 4;
-        return *(const float4 *)(tb + (int64_t)(min(m0 + r, g.M - 1) % S) * ss + (c4 & (hd - 1)));
+        return *(const float4 *)(tb + (int64_t)(min(m0 + r, g.M - 1) % S) * ss + (column(c4) & (hd - 1)));
       };
       // Table rows are requested a chunk of iterations ahead of their use (the first chunk before the tile is
       // exchanged): behind the stores of the iteration before, each would cost a trip to L2 of its own.
@@ -822,13 +826,13 @@ __global__ void __launch_bounds__(WR *WC *KG * 64) gemm_bf16_dma_kernel(GemmDesc
 #pragma unroll
         for (int j = 0; j < TN; ++j) {
           const int cl = wn * WN + j * 32 + (lane & 31);
-          const float bv = Bias ? Bias[min(n0 + cl, Nl - 1)] : 0.f;
+          const float bv = Bias ? Bias[min(column(cl), Nl - 1)] : 0.f;
 #pragma unroll
           for (int e = 0; e < 16; ++e)
             tile[(wm * WM + i * 32 + (e >> 2) * 8 + (lane >> 5) * 4 + (e & 3)) * P + cl] = acc[i][j][e] + bv;
         }
       __syncthreads();
-      const int half = (int)hd / 2;
+      const int half = PAIRS ? 16 : (int)hd / 2;  // tile columns between partners
 #pragma unroll
       for (int it = 0; it < ITERS; ++it) {
         if (it % CH == 0 && it + CH < ITERS) {
@@ -848,8 +852,8 @@ __global__ void __launch_bounds__(WR *WC *KG * 64) gemm_bf16_dma_kernel(GemmDesc
         o.x = c.x * xv.x + sn4.x * pv.x; o.y = c.y * xv.y + sn4.y * pv.y;
         o.z = c.z * xv.z + sn4.z * pv.z; o.w = c.w * xv.w + sn4.w * pv.w;
         if (row < g.M) {
-          const uint32_t sq = row / S, pos = row - sq * S, head = (n0 + c4) / hd;
-          const uint64_t at = (((uint64_t)sq * heads + head) * S + pos) * hd + (c4 & (hd - 1));
+          const uint32_t sq = row / S, pos = row - sq * S, head = column(c4) / hd;
+          const uint64_t at = (((uint64_t)sq * heads + head) * S + pos) * hd + (column(c4) & (hd - 1));
           *(float4 *)(g.rope_out[grp] + at) = o;
           if (g.rope_out16[grp]) *(uint2 *)(g.rope_out16[grp] + at) = bf16_pack4(o);
         }
@@ -863,7 +867,7 @@ __global__ void __launch_bounds__(WR *WC *KG * 64) gemm_bf16_dma_kernel(GemmDesc
       for (int i = 0; i < TM; ++i)
 #pragma unroll
         for (int j = 0; j < TN; ++j) {
-          const uint32_t col = n0 + wn * WN + j * 32 + (lane & 31);  // = head * hd + column of the head
+          const uint32_t col = column(wn * WN + j * 32 + (lane & 31));  // = head * hd + column of the head
           const float bv = Bias ? Bias[min(col, Nl - 1)] : 0.f;
 #pragma unroll
           for (int q = 0; q < 4; ++q) {
@@ -896,7 +900,7 @@ __global__ void __launch_bounds__(WR *WC *KG * 64) gemm_bf16_dma_kernel(GemmDesc
   for (int i = 0; i < TM; ++i)
 #pragma unroll
     for (int j = 0; j < TN; ++j) {
-      const uint32_t col = n0 + wn * WN + j * 32 + (lane & 31);
+      const uint32_t col = column(wn * WN + j * 32 + (lane & 31));
       if (Bias) {
         const float bv = Bias[min(col, Nl - 1)];
 #pragma unroll
@@ -2751,7 +2755,7 @@ bool gemm_rope_epilogue_ok(const LaunchCtx &lc, const GemmDesc &g) {
       return false;
     }
   }
-  // launch_matmul's tiles of 64 and 128 rows have this epilogue (128 columns, or 64 - for heads of 64 - where those are
+  // launch_matmul's tiles of 32 and 128 rows have this epilogue (128 columns, or 64 - for heads of 64 - where those are
   // too few for the CUs); the 256 x 256 tile of the largest problems has not
   const uint64_t t256 = (uint64_t)((g.M + 255) / 256) * ((g.N + 255) / 256);
   if (t256 >= (uint64_t)lc.n_cus && grp256) return false;
@@ -2935,7 +2939,16 @@ hipError_t launch_matmul(const LaunchCtx &lc_in, const GemmDesc &g, const char *
       if (g.n_group && (batch != 1 || splits != 1 || g.glu_gate || g.c16)) return hipErrorInvalidValue;
       const uint64_t t128 = (uint64_t)((g.M + 127) / 128) * ((g.N + 127) / 128) * batch * splits;
       const bool deep = t128 < 2 * (uint64_t)lc.n_cus;  // at most one workgroup per CU at a time: four stages
-      if (g.M <= 64) {
+      if (g.rope_s && g.M <= 128) {
+        // q / k / v of a few rows: a workgroup takes in its rows of both operands at about 42 GB/s however wide its tile is,
+        // and 64 x 64 or 128 x 64 tiles are 48 workgroups for 3072 columns.  32 x 32 tiles, of columns that rotate into
+        // each other: 37 rows 14.5 -> 12.1 us, 64 15.1 -> 10.5, 100 17.4 -> 12.4, 128 18.3 -> 14.6; with heads of 128 and
+        // 6144 columns 60 rows 24.3 -> 14.0, 120 27.2 -> 16.8 (from 200 rows on the two are even).  Eight stages while two
+        // workgroups to a CU hold every tile, else five and three workgroups (those 120 rows with eight: 22.8).
+        const uint64_t t32 = (uint64_t)((g.M + 31) / 32) * ((g.N + 31) / 32);
+        e = t32 <= 2 * (uint64_t)lc.n_cus ? launch_gemm_dma<32, 32, 1, 1, false, 8, false, false, true, 4>(lc, gg, (uint32_t)t32)
+                                          : launch_gemm_dma<32, 32, 1, 1, false, 5, false, false, true, 4>(lc, gg, (uint32_t)t32);
+      } else if (g.M <= 64) {
         // A few rows: bound by the stream of weights, so narrow tiles, one workgroup to a CU with as much in flight
         // as its LDS holds (the 128-row tiles put 64 workgroups on the chip for a 16384 x 2048 gate and up).
         const uint64_t t64 = (uint64_t)((g.N + 63) / 64) * batch * splits;
@@ -2945,10 +2958,6 @@ hipError_t launch_matmul(const LaunchCtx &lc_in, const GemmDesc &g, const char *
           e = launch_gemm_dma<64, 64, 2, 1, true, 8, true, false, false, 2>(lc, gg, (uint32_t)((g.N + 31) / 32 * batch));
         } else if (g.glu_gate || g.c16 || (g.act_sigmoid && splits == 1)) {
           e = launch_gemm_dma<64, 64, 2, 2, true, 8, false, false, false, 2>(lc, gg, (uint32_t)t64);
-        } else if (g.rope_s && g.rope_hd > 64) {
-          e = launch_gemm_dma<64, 128, 2, 2, false, 5, false, false, true, 2>(lc, gg, (uint32_t)((g.N + 127) / 128));
-        } else if (g.rope_s) {
-          e = launch_gemm_dma<64, 64, 2, 2, false, 8, false, false, true, 2>(lc, gg, (uint32_t)t64);
         } else {
           e = launch_gemm_dma<64, 64, 2, 2, false, 8, false, false, false, 2>(lc, gg, (uint32_t)t64);
         }

@@ -40,12 +40,12 @@ def test_gated_mlp_of_few_rows(oracle, hip_bf16, rows, K, F, N):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("tokens", [17, 40, 64])
+@pytest.mark.parametrize("tokens", [17, 40, 64, 99, 128])
 def test_rotation_in_the_projections_launch_of_few_rows(oracle, hip_bf16, tokens):
     llama_tests.test_llama_prefill_rotates_in_the_projections_launch(oracle, hip_bf16, tokens, 8, 2, 2)
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("batch,tokens", [(1, 40), (3, 20)])
-def test_rotation_of_wide_heads_of_few_rows(oracle, hip_bf16, batch, tokens):
-    moe_tests.test_qwen_prefill_biases_and_rotation_in_the_projections_launch(oracle, hip_bf16, batch, tokens, 4, 4, 128)
+@pytest.mark.parametrize("batch,tokens,heads", [(1, 40, 4), (3, 20, 4), (3, 41, 4), (1, 128, 4), (1, 101, 16)])
+def test_rotation_of_wide_heads_of_few_rows(oracle, hip_bf16, batch, tokens, heads):
+    moe_tests.test_qwen_prefill_biases_and_rotation_in_the_projections_launch(oracle, hip_bf16, batch, tokens, heads, heads, 128)
