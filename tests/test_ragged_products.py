@@ -69,3 +69,18 @@ def test_ragged_operands_of_either_order(oracle, hip_bf16, batch, m, n, k, turne
     (ref,) = vectors.run(oracle, transposed if turned else plain, 1, x, w)
     (got,) = vectors.run(hip_bf16, transposed if turned else plain, 1, x, w)
     parity.assert_bf16(ref, got, f"{batch}x{m}x{n}x{k}")
+
+
+# as many 128-row tiles as need a second round over the CUs, and few enough tiles of 192 rows for one; rows and columns that end
+# inside a tile, k of one step and of several
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,n,k", [(2300, 2048, 64), (2881, 1990, 192), (3071, 1920, 256), (193 * 16, 1536, 128)])
+def test_one_round_of_tall_tiles(oracle, hip_bf16, rows, n, k):
+    g = np.random.default_rng(rows)
+    x, w = draw(g, (1, rows, k), 1.0), draw(g, (1, n, k), k ** -0.5)
+
+    def f(b, x, w):
+        return [lang.matmul(b, x, lang.transpose(b, 1, 2, w))]
+    (ref,) = vectors.run(oracle, f, 1, x, w)
+    (got,) = vectors.run(hip_bf16, f, 1, x, w)
+    parity.assert_bf16(ref, got, f"{rows}x{n}x{k}")
