@@ -3001,7 +3001,8 @@ hipError_t launch_matmul(const LaunchCtx &lc_in, const GemmDesc &g, const char *
           return launch_matmul(second, rest, nullptr);
         }
         if (!g.n_group && fill(t128, 2 * (uint64_t)lc.n_cus) > 1.15 * fill(t256, (uint64_t)lc.n_cus))
-          e = launch_gemm_dma<128, 128, 2, 2>(lc, gg, (uint32_t)t128);
+          e = g.K < 2048 ? launch_gemm_dma<128, 128, 2, 4, false, 2>(lc, gg, (uint32_t)t128)  // (as below)
+                         : launch_gemm_dma<128, 128, 2, 2>(lc, gg, (uint32_t)t128);
         else
           e = launch_gemm_dma<256, 256, 2, 4>(lc, gg, (uint32_t)t256);
       } else if (splits == 1 && t128 * 2 <= (uint64_t)lc.n_cus && g.N >= 128) {
@@ -3025,7 +3026,11 @@ hipError_t launch_matmul(const LaunchCtx &lc_in, const GemmDesc &g, const char *
           e = launch_gemm_dma<192, 128, 2, 4, false, 3>(lc, gg, (uint32_t)t192);
         else e = launch_gemm_dma<128, 128, 2, 4, false, 4>(lc, gg, (uint32_t)t128);
       } else {
-        if (g.rope_s) e = launch_gemm_dma<128, 128, 2, 2, false, 2, false, false, true>(lc, gg, (uint32_t)t128);
+        // Eight waves share the tail of a tile - a rotation, or stores after few k-steps -, four are ahead in a long main loop:
+        // q / k / v rotated, 2900 rows of 3072 columns: four waves 79 us, eight 69; 1350 rows of 6144 with heads of 128 86, 77;
+        // plain, K = 1152, 16384 rows of 1536 62, 56; 4000 rows of 2048, K = 2048 and 8192 on average, 90, 93.
+        if (g.rope_s) e = launch_gemm_dma<128, 128, 2, 4, false, 2, false, false, true>(lc, gg, (uint32_t)t128);
+        else if (g.K < 2048) e = launch_gemm_dma<128, 128, 2, 4, false, 2>(lc, gg, (uint32_t)t128);
         else e = launch_gemm_dma<128, 128, 2, 2>(lc, gg, (uint32_t)t128);
       }
       if (e != hipSuccess) return e;
