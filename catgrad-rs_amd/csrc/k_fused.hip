@@ -863,7 +863,7 @@ __global__ void __launch_bounds__(NWV * 64) attn_decode_group_kernel(AttnDecodeD
   const float *V = a.v + (int64_t)b * a.v_sb + (int64_t)kv * a.v_skv;
   const uint32_t t_begin = c * a.chunk, t_end = min(a.t, t_begin + a.chunk);
   f32x4 kn[U][K4], vn[U][4][H];
-  auto fetch = [&](uint32_t t0) {  // tiles t0, t0 + NWV * 16, ..; rows past the end repeat the last (their weight is zero)
+  auto fetch = [&](uint32_t t0) {  // tiles t0, t0 + NWV * 16, ..; rows past the end repeat the last (never used: below)
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const uint32_t tt = t0 + u * NWV * 16;
@@ -970,6 +970,17 @@ __global__ void __launch_bounds__(NWV * 64) attn_decode_group_kernel(AttnDecodeD
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const uint32_t tt = t0 + u * NWV * 16;
+      // Value rows past the end are zeros, not whatever memory holds there: they meet a weight of zero inside the matrix
+      // instruction, where zero times a NaN or an infinity is a NaN, and in an appending step the last row of the range
+      // (which they repeat) is one that nobody has written yet.  (Keys need no such care: a score is selected away.)
+      if (tt + 16 > t_end) {  // (uniform over the wave: the last tiles of a range)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int w = 0; w < H; ++w)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) vr[u][i][w][e] = tt + kb * 4 + i < t_end ? vr[u][i][w][e] : 0.f;
+      }
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const float p = tt + kb * 4 + i < t_end ? __expf(s[u][i] - m_new) : 0.f;

@@ -110,3 +110,54 @@ def test_decode_over_a_long_cache(oracle, hip, H, KV, d, T, steps):
         assert hip.launch_counts(reset=True).get("attn_decode") == 1
     for a, b in zip(runners[0].kv, runners[1].kv):
         parity.assert_f32(oracle.to_vec(a), hip.to_vec(b), "cache")
+
+
+def leave_nan_in_memory(be, *sizes):
+    """Blocks of these many bytes, filled with NaN and given back: the next allocations of their size classes get them."""
+    be.sync()
+    held = [be.tensor(np.full(n // 4, np.nan, np.float32)) for n in sizes for _ in range(4)]
+    be.sync()
+    del held
+
+
+# What a cache's room to grow holds before it is written must not reach a result: an appending step of each decode kernel,
+# whose last range of keys ends inside a tile (one workgroup; split keys; the matrix-core form, with one and two tiles of a
+# pass past the end, merged by the launch itself and by the reader).
+@pytest.mark.gpu
+@pytest.mark.parametrize("mode", ["f32", "bf16"])
+@pytest.mark.parametrize("H,KV,d,T", [(4, 2, 64, 20), (4, 2, 64, 300), (4, 1, 64, 881), (16, 2, 64, 2049), (4, 2, 128, 129), (8, 4, 128, 516)])
+def test_unwritten_rows_of_a_cache_stay_out(oracle, hip, hip_bf16, mode, H, KV, d, T):
+    be, check = (hip, parity.assert_f32) if mode == "f32" else (hip_bf16, parity.assert_bf16)
+    cfg = llm.Config(hidden_size=H * d, intermediate_size=64, num_hidden_layers=1, num_attention_heads=H, num_key_value_heads=KV,
+                     vocab_size=97, rms_norm_eps=1e-5, rope_theta=10000.0)
+    arrays = llm.random_init.llama_params(cfg, seed=T, std=0.08)
+    rounded = {k: (vectors.bf16_round(a) if a.ndim >= 2 else a) for k, a in arrays.items()}
+    g = np.random.default_rng(T)
+    kv = [vectors.bf16_round(g.standard_normal((1, KV, T, d)).astype(np.float32)) for _ in range(2)]
+    room = 64
+    while room < 2 * (T + 1):
+        room *= 2
+    ref, got = (llm.CachedRunner(b, cfg, rounded, T + 8) for b in (oracle, be))
+    for r in (ref, got):
+        # (uploaded as vectors: a cache is f32 in both modes)
+        r.batch, r.pos, r.kv = 1, 3, [r.be.reshape(r.be.tensor(a.reshape(-1)), a.shape) for a in kv]
+    leave_nan_in_memory(be, KV * room * d * 4)
+    for token in (5, 11, 90):     # (the first step copies the cache, the following ones append)
+        want, have = (r.be.to_vec(r.step(token)[1]) for r in (ref, got))
+        assert np.isfinite(have).all(), f"token {token}"
+        check(want, have, f"token {token}")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("H,KV,S,d", [(4, 2, 7, 64), (2, 2, 33, 128), (2, 1, 130, 64), (4, 1, 67, 256), (64, 64, 523, 64)])
+def test_what_memory_held_stays_out_of_a_prompt(oracle, hip, hip_bf16, H, KV, S, d):
+    """The padding of mask rows and transposed values is written, and rows past the last key never count."""
+    g = np.random.default_rng(S + d)
+    q, k, v = (vectors.bf16_round(g.standard_normal((1, h, S, d)).astype(np.float32)) for h in (H, KV, KV))
+    f = attention(H, KV, S, d, 0)
+    (ref,) = vectors.run(oracle, f, 1, q, k, v)
+    for be, check in ((hip, parity.assert_f32), (hip_bf16, parity.assert_bf16)):
+        leave_nan_in_memory(be, *(256 << i for i in range(13)), 1 << 20, 2 << 20)
+        (got,) = vectors.run(be, f, 1, q, k, v)
+        assert np.isfinite(got).all()
+        check(ref, got, f"attention over {S} keys")
