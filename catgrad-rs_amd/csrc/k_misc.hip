@@ -286,11 +286,18 @@ hipError_t launch_to_host(const LaunchCtx &lc, const void *src, void *dst, uint6
 
 // n words of pinned host memory into device memory, then the flag: the host may use the words again (one workgroup)
 __global__ void __launch_bounds__(1024) from_host_kernel(const uint32_t *src, uint32_t *dst, uint32_t n, uint32_t *flag) {
-  // (16 bytes a request: each is a trip across the bus, and there is one workgroup to make them; a fresh slot was not
-  // read before, so ordinary loads find the host's values)
+  // The host has written these words since an earlier launch read the same addresses (the ring's slots are used again): no
+  // cache may answer, so the loads have system scope.  Sixteen bytes each - a request is a trip across the bus, and there
+  // is one workgroup to make them -, which an atomic load of eight is not (64 KB: 10.3 us each of a hundred, 7.4 so).
+  typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
   const uint32_t n4 = n / 4;
-  for (uint32_t i = threadIdx.x; i < n4; i += 1024) ((uint4 *)dst)[i] = ((const uint4 *)src)[i];
-  if (threadIdx.x < n - n4 * 4) dst[n4 * 4 + threadIdx.x] = src[n4 * 4 + threadIdx.x];
+  for (uint32_t i = threadIdx.x; i < n4; i += 1024) {
+    u32x4 v;
+    asm volatile("global_load_dwordx4 %0, %1, off sc0 sc1\n\ts_waitcnt vmcnt(0)" : "=&v"(v) : "v"(src + 4 * i) : "memory");
+    ((u32x4 *)dst)[i] = v;
+  }
+  if (threadIdx.x < n - n4 * 4)
+    dst[n4 * 4 + threadIdx.x] = __hip_atomic_load(src + n4 * 4 + threadIdx.x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
   __syncthreads();
   if (threadIdx.x == 0) __hip_atomic_store(flag, 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
