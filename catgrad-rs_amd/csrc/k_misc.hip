@@ -280,7 +280,9 @@ hipError_t launch_to_host(const LaunchCtx &lc, const void *src, void *dst, uint6
   if (n && ((uintptr_t)src % 16 || (uintptr_t)dst % 16)) return hipErrorInvalidValue;
   const uint64_t blocks = (n + 1023) / 1024;
   if (blocks > TO_HOST_GROUPS * TO_HOST_MAX_PIECES) return hipErrorInvalidValue;
-  CG_LAUNCH(lc, to_host_kernel, (unsigned)(blocks ? blocks : 1), 256, (const uint32_t *)src, (uint32_t *)dst, n, err, tail, done);
+  LaunchCtx own = lc;
+  own.failed = tail + 2;
+  CG_LAUNCH(own, to_host_kernel, (unsigned)(blocks ? blocks : 1), 256, (const uint32_t *)src, (uint32_t *)dst, n, err, tail, done);
   return hipGetLastError();
 }
 
@@ -304,7 +306,9 @@ __global__ void __launch_bounds__(1024) from_host_kernel(const uint32_t *src, ui
 
 hipError_t launch_from_host(const LaunchCtx &lc, const void *src, void *dst, uint32_t n, uint32_t *flag) {
   if (!n || (uintptr_t)src % 16 || (uintptr_t)dst % 16) return hipErrorInvalidValue;
-  CG_LAUNCH(lc, from_host_kernel, 1, 1024, (const uint32_t *)src, (uint32_t *)dst, n, flag);
+  LaunchCtx own = lc;
+  own.failed = flag;
+  CG_LAUNCH(own, from_host_kernel, 1, 1024, (const uint32_t *)src, (uint32_t *)dst, n, flag);
   return hipGetLastError();
 }
 

@@ -20,6 +20,8 @@ struct LaunchCtx {
   hipEvent_t ev_start, ev_stop;
   // when set, launches are handed to this queue's thread instead of being made by the caller
   LaunchQueue *queue;
+  // set by that thread to HOST_FLAG_FAILED when it cannot make the launch (optional)
+  uint32_t *failed = nullptr;
 };
 
 // Every kernel is launched through this: with null events it is an ordinary launch (made by the
@@ -28,7 +30,7 @@ struct LaunchCtx {
 template <typename... KArgs, typename... Args>
 inline void cg_launch(const LaunchCtx &lc, void (*kernel)(KArgs...), dim3 grid, dim3 block, size_t smem, Args &&...args) {
   if (lc.queue && !lc.ev_start && !lc.ev_stop) {
-    lc.queue->launch(kernel, grid, block, smem, lc.stream, std::forward<Args>(args)...);
+    lc.queue->launch(kernel, grid, block, smem, lc.stream, lc.failed, std::forward<Args>(args)...);
     return;
   }
   if (lc.queue) lc.queue->drain();
@@ -80,9 +82,10 @@ hipError_t launch_compare(const LaunchCtx &lc, const void *a, const void *b, uin
 // n 32-bit words of src (device) to dst (pinned host memory), both 16-byte aligned, at most TO_HOST_MAX_PIECES pieces of
 // TO_HOST_PIECE words.  Behind each piece (one at least, also when n is 0) err[0], err[1] and 1 go to the first three words
 // of its tail (pinned host memory, TO_HOST_TAIL words a piece).  done: a device word per piece, zero between launches.
+// A launch that the queue's thread cannot make sets the third word of the first tail to HOST_FLAG_FAILED.
 enum : uint32_t { TO_HOST_PIECE = 32768, TO_HOST_MAX_PIECES = 16, TO_HOST_TAIL = 16 };
 hipError_t launch_to_host(const LaunchCtx &lc, const void *src, void *dst, uint64_t n, const uint32_t *err, uint32_t *tail, uint32_t *done);
-// n words of src (pinned host memory) to dst (device); then 1 to *flag (pinned host memory)
+// n words of src (pinned host memory) to dst (device); then 1 to *flag (pinned host memory), or HOST_FLAG_FAILED as above
 hipError_t launch_from_host(const LaunchCtx &lc, const void *src, void *dst, uint32_t n, uint32_t *flag);
 hipError_t launch_fill_u32(const LaunchCtx &lc, uint32_t *dst, uint32_t value, uint64_t n);
 // Contiguous copy of a strided view whose unit-stride axis is not the last one (a materialised

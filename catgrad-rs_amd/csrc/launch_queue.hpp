@@ -25,6 +25,10 @@
 
 namespace cgk {
 
+// What a word of pinned memory that a copy kernel sets says to the host that polls it: not yet, done, or (set by the
+// queue's thread) that the launch could not be made and nothing will come.
+enum : uint32_t { HOST_FLAG_PENDING = 0, HOST_FLAG_DONE = 1, HOST_FLAG_FAILED = 2 };
+
 class LaunchQueue {
  public:
   enum : size_t { SLOTS = 256, SLOT_BYTES = 2048 };
@@ -42,9 +46,10 @@ class LaunchQueue {
   LaunchQueue(const LaunchQueue &) = delete;
   LaunchQueue &operator=(const LaunchQueue &) = delete;
 
-  // Copies a launch into the ring (waits while the ring is full).
+  // Copies a launch into the ring (waits while the ring is full).  failed (optional): becomes HOST_FLAG_FAILED when the
+  // launch cannot be made.
   template <typename... KArgs, typename... Args>
-  void launch(void (*kernel)(KArgs...), dim3 grid, dim3 block, size_t smem, hipStream_t stream, Args &&...args) {
+  void launch(void (*kernel)(KArgs...), dim3 grid, dim3 block, size_t smem, hipStream_t stream, uint32_t *failed, Args &&...args) {
     struct Payload {
       void (*kernel)(KArgs...);
       dim3 grid, block;
@@ -64,6 +69,7 @@ class LaunchQueue {
           [q](auto &...a) { hipExtLaunchKernelGGL(q->kernel, q->grid, q->block, q->smem, q->stream, nullptr, nullptr, 0, a...); },
           q->a);
     };
+    s.failed = failed;
     // sequentially consistent on both sides: either this thread sees the worker asleep, or the worker's
     // last look at the ring before it sleeps sees this slot
     head_.store(h + 1);
@@ -82,6 +88,7 @@ class LaunchQueue {
  private:
   struct Slot {
     void (*run)(void *);
+    uint32_t *failed;
     alignas(16) unsigned char buf[SLOT_BYTES];
   };
   static void pause() {
@@ -120,6 +127,7 @@ class LaunchQueue {
       if (e != hipSuccess) {
         int none = (int)hipSuccess;
         error_.compare_exchange_strong(none, (int)e, std::memory_order_acq_rel);
+        if (s.failed) __atomic_store_n(s.failed, HOST_FLAG_FAILED, __ATOMIC_RELEASE);
       }
       tail_.store(t + 1, std::memory_order_release);
     }

@@ -237,13 +237,15 @@ int realize(cg_backend *be, cg_tensor *n) {
 
 // Waits for the flag a launch_to_host sets in pinned memory: every kernel enqueued before it has ended.  Polled, which
 // sees it ~10 us sooner than a wait on the stream; should the flag not come for a long time (work of seconds is
-// queued, or the launch could not be made), the stream is waited for and asked.
-int wait_host_flag(cg_backend *be, const uint32_t *flag) {
+// queued), the stream is waited for and asked.  On an error the stream is idle: nothing is on its way to memory the caller
+// is about to use again.
+static int wait_host_flag_value(cg_backend *be, const uint32_t *flag) {
   for (int round = 0; round < 20000; ++round) {  // a second or so
     for (int i = 0; i < 1000; ++i) {
-      if (__atomic_load_n(flag, __ATOMIC_ACQUIRE)) {
+      const uint32_t f = __atomic_load_n(flag, __ATOMIC_ACQUIRE);
+      if (f != HOST_FLAG_PENDING) {
         if (be->queue) HIPCHK(be, be->queue->take_error());  // a launch the queue's thread could not make
-        return CG_OK;
+        return f == HOST_FLAG_DONE ? CG_OK : fail(be, CG_ERR_DEVICE, "a copy to or from the host could not be launched");
       }
 #if defined(__x86_64__)
       __builtin_ia32_pause();
@@ -252,13 +254,19 @@ int wait_host_flag(cg_backend *be, const uint32_t *flag) {
   }
   HIPCHK(be, hipStreamSynchronize(be->ordered_stream()));
   if (be->queue) HIPCHK(be, be->queue->take_error());
-  return __atomic_load_n(flag, __ATOMIC_ACQUIRE) ? CG_OK : fail(be, CG_ERR_DEVICE, "a copy to the host was not made");
+  return __atomic_load_n(flag, __ATOMIC_ACQUIRE) == HOST_FLAG_DONE ? CG_OK : fail(be, CG_ERR_DEVICE, "a copy to or from the host was not made");
+}
+
+int wait_host_flag(cg_backend *be, const uint32_t *flag) {
+  const int st = wait_host_flag_value(be, flag);
+  if (st) (void)hipStreamSynchronize(be->ordered_stream());
+  return st;
 }
 
 
 // wait for the stream and surface device-side error flags
 int sync_and_check(cg_backend *be) {
-  be->h_words[2] = 0;
+  be->h_words[2] = HOST_FLAG_PENDING;
   HIPCHK(be, launch_to_host(be->lc(), nullptr, nullptr, 0, be->d_words, be->h_words, be->d_words + 4));
   TRY(wait_host_flag(be, be->h_words + 2));
   return check_error_words(be, be->h_words);
@@ -585,20 +593,22 @@ int upload(cg_backend *be, const void *data, size_t n, const int64_t *shape, int
     const size_t tail = HOST_IN_BYTES - 64;
     if (!be->h_in) {
       e = hipHostMalloc((void **)&be->h_in, HOST_IN_BYTES * HOST_IN_SLOTS, hipHostMallocDefault);
-      for (size_t i = 0; i < HOST_IN_SLOTS && e == hipSuccess; ++i) *(uint32_t *)(be->h_in + i * HOST_IN_BYTES + tail) = 1;
+      for (size_t i = 0; i < HOST_IN_SLOTS && e == hipSuccess; ++i) *(uint32_t *)(be->h_in + i * HOST_IN_BYTES + tail) = HOST_FLAG_DONE;
     }
     if (e == hipSuccess) {
       char *slot = be->h_in + be->h_in_next * HOST_IN_BYTES;
       uint32_t *flag = (uint32_t *)(slot + tail);
-      st = wait_host_flag(be, flag);  // (HOST_IN_SLOTS uploads ago)
+      // (HOST_IN_SLOTS uploads ago.  One that was not made was reported where its error was taken; its slot is free.)
+      if (__atomic_load_n(flag, __ATOMIC_ACQUIRE) != HOST_FLAG_FAILED) st = wait_host_flag(be, flag);
       if (st) {
+        *flag = HOST_FLAG_DONE;  // (nothing is in flight)
         node_release(t);
         return st;
       }
       std::memcpy(slot, data, n * 4);
-      *flag = 0;
+      *flag = HOST_FLAG_PENDING;
       e = launch_from_host(be->lc(), slot, t->st->ptr, (uint32_t)n, flag);
-      if (e != hipSuccess) *flag = 1;
+      if (e != hipSuccess) *flag = HOST_FLAG_DONE;
       else be->h_in_next = (be->h_in_next + 1) % HOST_IN_SLOTS;
     }
   } else if (!narrow) {
@@ -651,14 +661,14 @@ int upload(cg_backend *be, const void *data, size_t n, const int64_t *shape, int
 
 // Through pinned memory: launches of up to TO_HOST_MAX_PIECES pieces fill its two halves in turn, and each piece is
 // copied on to its destination while the device stores the next ones.
-static int download_pieces(cg_backend *be, const char *src, char *dst, size_t bytes) {
+static int download_through_halves(cg_backend *be, const char *src, char *dst, size_t bytes) {
   const size_t piece = (size_t)TO_HOST_PIECE * 4, half = piece * TO_HOST_MAX_PIECES, tails = (size_t)TO_HOST_TAIL * 4 * TO_HOST_MAX_PIECES;
   if (!be->h_out) HIPCHK(be, hipHostMalloc((void **)&be->h_out, 2 * (half + tails), hipHostMallocDefault));
   const size_t pieces = (bytes + piece - 1) / piece;
   auto data = [&](size_t i) { return be->h_out + i / TO_HOST_MAX_PIECES % 2 * half + i % TO_HOST_MAX_PIECES * piece; };
   auto words = [&](size_t i) { return (uint32_t *)(be->h_out + 2 * half) + i % (2 * TO_HOST_MAX_PIECES) * TO_HOST_TAIL; };
   auto ask = [&](size_t first) -> int {  // for the pieces from `first` that fill one half
-    for (size_t i = first; i < std::min(pieces, first + TO_HOST_MAX_PIECES); ++i) words(i)[2] = 0;
+    for (size_t i = first; i < std::min(pieces, first + TO_HOST_MAX_PIECES); ++i) words(i)[2] = HOST_FLAG_PENDING;
     const size_t len = std::min(half, bytes - first * piece);
     HIPCHK(be, launch_to_host(be->lc(), src + first * piece, data(first), len / 4, be->d_words, words(first), be->d_words + 4));
     return CG_OK;
@@ -673,6 +683,13 @@ static int download_pieces(cg_backend *be, const char *src, char *dst, size_t by
   return check_error_words(be, words(pieces - 1));
 }
 
+static int download_pieces(cg_backend *be, const char *src, char *dst, size_t bytes) {
+  const int st = download_through_halves(be, src, dst, bytes);
+  // (the other half may still be on its way into the buffer that the next read uses)
+  if (st) (void)hipStreamSynchronize(be->ordered_stream());
+  return st;
+}
+
 
 int download(cg_backend *be, cg_tensor *x, void *dst, size_t n, cg_dtype want) {
   if (!be || !x || (!dst && n)) return fail(be, CG_ERR_ARG, "null argument");
@@ -681,7 +698,13 @@ int download(cg_backend *be, cg_tensor *x, void *dst, size_t n, cg_dtype want) {
   HIPCHK(be, hipSetDevice(be->device));
   if (x->host_copy) {  // prefetched: wait for that copy only, not for work queued behind it
     const uint32_t *words = (const uint32_t *)((const char *)x->host_copy + PREFETCH_BYTES - PREFETCH_TAIL);
-    TRY(wait_host_flag(be, words + 2));
+    const int st = wait_host_flag(be, words + 2);
+    if (st) {  // nothing came and nothing will: the next read takes the synchronising path
+      *(uint32_t *)(words + 2) = HOST_FLAG_DONE;
+      be->pinned_pool.push_back(x->host_copy);
+      x->host_copy = nullptr;
+      return st;
+    }
     if (words[0] == 0) {
       std::memcpy(dst, x->host_copy, n * 4);
       return CG_OK;

@@ -1,0 +1,95 @@
+// A HIP runtime without a GPU, for tests of what the host does: memory is host memory, a stream is always idle, the two
+// copy kernels are made on the spot and every other launch is none.  fake_hip_refuse(name, n): the n-th launch from now
+// of a kernel whose name holds `name` is refused, as the runtime refuses one that it cannot make.
+// Loaded with RTLD_GLOBAL before the library, whose references to the runtime it then answers.
+#include <hip/hip_runtime.h>
+#include <atomic>
+#include <cstdlib>
+#include <cstring>
+#include <map>
+#include <mutex>
+#include <string>
+
+namespace {
+std::map<const void *, std::string> &names() {
+  static std::map<const void *, std::string> m;
+  return m;
+}
+std::mutex lock;
+std::string refuse;
+std::atomic<int> countdown{0}, waits{0};
+thread_local hipError_t last = hipSuccess;
+
+// the argument lists of to_host_kernel and from_host_kernel (k_misc.hip)
+void to_host(void **a) {
+  const uint32_t *src = *(const uint32_t **)a[0], *err = *(const uint32_t **)a[3];
+  uint32_t *dst = *(uint32_t **)a[1], *tail = *(uint32_t **)a[4];
+  const uint64_t n = *(uint64_t *)a[2], piece = 32768, words = 16;
+  if (n) std::memcpy(dst, src, n * 4);
+  for (uint64_t p = 0; p == 0 || p * piece < n; ++p) {
+    tail[p * words] = err[0];
+    tail[p * words + 1] = err[1];
+    __atomic_store_n(tail + p * words + 2, 1u, __ATOMIC_RELEASE);
+  }
+}
+void from_host(void **a) {
+  std::memcpy(*(void **)a[1], *(void **)a[0], *(uint32_t *)a[2] * (size_t)4);
+  __atomic_store_n(*(uint32_t **)a[3], 1u, __ATOMIC_RELEASE);
+}
+hipError_t launch(const void *f, void **args) {
+  const std::string &name = names()[f];
+  {
+    std::lock_guard<std::mutex> lk(lock);
+    if (!refuse.empty() && name.find(refuse) != std::string::npos && countdown.fetch_sub(1) == 1) {
+      refuse.clear();
+      return last = hipErrorInvalidConfiguration;
+    }
+  }
+  if (name.find("to_host_kernel") != std::string::npos) to_host(args);
+  if (name.find("from_host_kernel") != std::string::npos) from_host(args);
+  return hipSuccess;
+}
+hipError_t memory(void **p, size_t n) { return (*p = aligned_alloc(4096, (n + 4095) / 4096 * 4096)) ? hipSuccess : hipErrorOutOfMemory; }
+}  // namespace
+
+extern "C" {
+void fake_hip_refuse(const char *name, int n) {
+  std::lock_guard<std::mutex> lk(lock);
+  refuse = name;
+  countdown = n;
+}
+int fake_hip_waits() { return waits; }  // on the stream
+
+void **__hipRegisterFatBinary(const void *) { static void *h[4]; return h; }
+void __hipUnregisterFatBinary(void **) {}
+void __hipRegisterVar(void **, void *, char *, char *, int, size_t, int, int) {}
+void __hipRegisterFunction(void **, const void *f, char *, const char *name, unsigned, uint3 *, uint3 *, dim3 *, dim3 *, int *) { names()[f] = name; }
+hipError_t __hipPopCallConfiguration(dim3 *, dim3 *, size_t *, hipStream_t *) { return hipSuccess; }
+hipError_t hipGetDeviceCount(int *n) { return *n = 1, hipSuccess; }
+hipError_t hipSetDevice(int) { return hipSuccess; }
+hipError_t hipGetDevicePropertiesR0600(hipDeviceProp_t *p, int) {
+  std::memset(p, 0, sizeof(*p));
+  p->multiProcessorCount = 256;
+  return hipSuccess;
+}
+hipError_t hipGetSymbolAddress(void **p, const void *) { static char room[1 << 18]; return *p = room, hipSuccess; }
+hipError_t hipGetLastError() { const hipError_t e = last; return last = hipSuccess, e; }
+const char *hipGetErrorString(hipError_t e) { return e == hipSuccess ? "no error" : "launch refused"; }
+hipError_t hipMalloc(void **p, size_t n) { return memory(p, n); }
+hipError_t hipHostMalloc(void **p, size_t n, unsigned) { return memory(p, n); }
+hipError_t hipFree(void *p) { return free(p), hipSuccess; }
+hipError_t hipHostFree(void *p) { return free(p), hipSuccess; }
+hipError_t hipMemcpy(void *d, const void *s, size_t n, hipMemcpyKind) { return std::memcpy(d, s, n), hipSuccess; }
+hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind, hipStream_t) { return std::memcpy(d, s, n), hipSuccess; }
+hipError_t hipMemsetAsync(void *d, int v, size_t n, hipStream_t) { return std::memset(d, v, n), hipSuccess; }
+hipError_t hipStreamCreate(hipStream_t *s) { return *s = nullptr, hipSuccess; }
+hipError_t hipStreamDestroy(hipStream_t) { return hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t) { return ++waits, hipSuccess; }
+hipError_t hipEventCreate(hipEvent_t *e) { return *e = nullptr, hipSuccess; }
+hipError_t hipEventDestroy(hipEvent_t) { return hipSuccess; }
+hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
+hipError_t hipEventElapsedTime(float *ms, hipEvent_t, hipEvent_t) { return *ms = 0.f, hipSuccess; }
+hipError_t hipFuncSetAttribute(const void *, hipFuncAttribute, int) { return hipSuccess; }
+hipError_t hipLaunchKernel(const void *f, dim3, dim3, void **args, size_t, hipStream_t) { return launch(f, args); }
+hipError_t hipExtLaunchKernel(const void *f, dim3, dim3, void **args, size_t, hipStream_t, hipEvent_t, hipEvent_t, int) { return launch(f, args); }
+}
