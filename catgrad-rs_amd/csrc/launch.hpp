@@ -470,11 +470,12 @@ uint32_t gemv_pro_multi_row_max_k(int b_stype);
 // most input rows any several-row form takes
 enum { GEMV_PRO_MAX_ROWS = 16 };
 // bf16 mode: whether a product of this many rows belongs on the tile kernels.  From 17 rows on; from 9 at depths whose rows
-// do not fit the few-row kernel's LDS (12 rows against a 2048 x 2048 matrix: 25.7 us on what was left, 6.5 on tiles); from
-// 5 where the few-row kernel does not go at all (8 x 8192 x 2048: 26 us on the vector ALUs, 19 with the narrowing of the
-// rows and the sum of the k-slices).
+// do not fit the few-row kernel's LDS (12 rows against a 2048 x 2048 matrix: 25.7 us on what was left, 6.5 on tiles).  Not
+// the 5 to 8 rows of a depth that the few-row kernel does not take: the vector ALUs multiply those as f32, and tiles would
+// round them to bf16 (8 x 8192 x 2048: 26 us, 19 on tiles with the narrowing of the rows and the sum of the k-slices; as
+// three products of bf16 parts that add up to the f32 value, on tiles, no faster at 8 rows and slower at 5).
 inline bool gemm_rows(uint64_t rows, uint64_t k) {
-  return rows > GEMV_PRO_MAX_ROWS || (rows > 8 && k >= 2048) || (rows > 4 && k >= 4096);
+  return rows > GEMV_PRO_MAX_ROWS || (rows > 8 && k >= 2048);
 }
 // whether launch_gemv_pro takes `rows` input rows of K values with prologue `pro` against weights of this
 // storage type: one row; up to 4 on the vector ALUs; up to 16 against bf16 weights on the matrix cores

@@ -1,0 +1,66 @@
+"""bf16 mode: which products keep f32 operands beside the bf16 weights.  Their results are held against 64-bit sums with the
+tolerance of f32 arithmetic, which an operand rounded to bf16 (2^-9 of each value) misses by two orders of magnitude."""
+import importlib
+
+import numpy as np
+import pytest
+
+import vectors
+
+lang, nn = vectors.cg.lang, vectors.cg.nn
+llm = importlib.import_module("catgrad-rs_amd.llm")
+helpers = llm.helpers
+
+
+def assert_f32_sums(exact, got, terms, what):
+    """A sum of n terms in f32: the rounding errors of its additions walk, sqrt(n) * 2^-24 of the terms' root mean square
+    sum at most a few times over; the norm of a row against the norm of its exact value."""
+    exact, got = (np.asarray(a, np.float64).reshape(-1, np.shape(exact)[-1]) for a in (exact, got))
+    err = np.linalg.norm(got - exact, axis=1) / np.linalg.norm(exact, axis=1)
+    assert err.max() <= 4 * np.sqrt(terms) * 2.0 ** -24, f"{what}: {err.max():.2e} off"
+
+
+# 5 to 8 rows at depths beyond the few-row kernel's
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows", [5, 8])
+@pytest.mark.parametrize("K,N", [(4096, 2048), (8192, 2048), (5632, 136), (4096, 65), (4160, 16500), (4100, 128)])
+def test_few_rows_of_a_deep_product(hip_bf16, rows, K, N):
+    g = np.random.default_rng(rows + K)
+    x = g.standard_normal(rows * K).astype(np.float32)
+    x[:K] *= np.float32(1e-25)
+    x[K:2 * K] *= np.float32(1e30)
+    w = vectors.bf16_round((g.standard_normal((N, K)) * K ** -0.5).astype(np.float32))
+
+    def f(b, x, w):
+        x = lang.reshape(b, lang.make_shape(b, 1, rows, K), x)     # (uploaded as a vector: f32)
+        return [lang.matmul(b, x, lang.reshape(b, lang.make_shape(b, 1, K, N), lang.transpose(b, 0, 1, w)))]
+    (got,) = vectors.run(hip_bf16, f, 1, x, w)
+    exact = x.reshape(rows, K).astype(np.float64) @ w.astype(np.float64).T
+    assert_f32_sums(exact, got, K, f"{rows} x {K} x {N}")
+
+
+@pytest.mark.gpu
+def test_few_rows_of_a_deep_product_with_a_residual_and_special_values(hip_bf16):
+    rows, K, N = 6, 4096, 256
+    g = np.random.default_rng(3)
+    x, res = (g.standard_normal((rows, n)).astype(np.float32) for n in (K, N))
+    w = vectors.bf16_round((g.standard_normal((N, K)) * K ** -0.5).astype(np.float32))
+    w[:, 9] = np.where(w[:, 9] == 0, 1, np.abs(w[:, 9]))
+    w[5, 9] = 0
+    x[0, 9] = np.inf
+    x[1, 9] = -np.inf
+    x[2].view(np.uint32)[9] = 0x7F800001      # a NaN that only its last bits tell from an infinity
+    x[3, 9] = np.finfo(np.float32).max
+    x[4] = 0
+
+    def f(b, x, res, w):
+        x, res = (lang.reshape(b, lang.make_shape(b, 1, rows, n), t) for t, n in ((x, K), (res, N)))
+        y = lang.matmul(b, x, lang.reshape(b, lang.make_shape(b, 1, K, N), lang.transpose(b, 0, 1, w)))
+        return [res + y]
+    (got,) = vectors.run(hip_bf16, f, 1, x.reshape(-1), res.reshape(-1), w)
+    with np.errstate(invalid="ignore"):
+        exact = x.astype(np.float64) @ w.astype(np.float64).T + res
+    got = got.reshape(rows, N)
+    for kind in (np.isposinf, np.isneginf, np.isnan):
+        assert np.array_equal(kind(exact), kind(got.astype(np.float64)))
+    assert_f32_sums(exact[3:], got[3:], K, "finite rows")
