@@ -13,6 +13,9 @@ namespace cgrt {
 // as one pass with online softmax (k_attn.hip); the [b, h, S, T] scores and probabilities are
 // never written.  With the bf16 flag the products run on bf16 MFMA (keys from their bf16 twin, values
 // from a bf16 V^T made once per call); without it every product is f32 and K / V are read as they lie.
+// Up to 8 queries in bf16 mode are not taken: the products of so few rows multiply f32 rows (as one query does), and their
+// sums over the lanes of a wave are closer to the exact ones than this pass's f32 form too (32 heads of 64, 8 queries, 64
+// keys: 2.7e-7 off in three launches of 18.6 us, 7.5e-7 in one of 13.5; with bf16 products 5.9e-3 and 11.4).
 int try_attn_prefill(cg_backend *be, cg_tensor *n, bool *done) {
   const bool f32 = !(be->flags & CG_FLAG_BF16);
   cg_tensor *P = n->in[0];
@@ -22,7 +25,7 @@ int try_attn_prefill(cg_backend *be, cg_tensor *n, bool *done) {
   cg_tensor *S = m.src;
   if (S->op != N_MATMUL || S->rank != 4 || refs(S) != (S == m.x ? 2 : 1)) return CG_OK;
   const int64_t Sq = S->shape[2], T = S->shape[3], d = n->shape[3], heads = n->shape[1], nb = n->shape[0];
-  if (Sq < 2 || T < 1 || (d != 64 && d != 128 && d != 256) || n->in[1]->shape[2] != T || S->in[0]->shape[3] != d)
+  if (Sq < (f32 ? 2 : 9) || T < 1 || (d != 64 && d != 128 && d != 256) || n->in[1]->shape[2] != T || S->in[0]->shape[3] != d)
     return CG_OK;
   // f32 products of a middling number of keys: the pass walks them one tile after the other with too few workgroups to
   // cover for it (1 x 32 heads x 200 x 200: 37 us), GEMM + softmax + GEMM take 31; at 50 keys it is 13 us against 21,

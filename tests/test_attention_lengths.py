@@ -1,6 +1,6 @@
 """One-pass attention (models/llama.rs:95-107, gemma3.rs:153-186) at numbers of queries and keys that are no multiple of
 anything: mask rows and transposed values are padded for the 16-byte loads of the kernel, and a prompt of a few tokens
-takes the same single launch."""
+takes the same single launch (in bf16 mode from 9 tokens on: test_f32_operands.py has the rest)."""
 import importlib
 
 import numpy as np
@@ -46,7 +46,7 @@ def test_attention_of_any_length(oracle, hip, hip_bf16, H, KV, S, d, window):
         be.launch_counts(reset=True)
         (got,) = vectors.run(be, f, 1, q, k, v)
         counts = be.launch_counts(reset=True)
-        three = be is hip and 128 < S < 512      # (f32: two products and a softmax at these lengths)
+        three = 128 < S < 512 if be is hip else S <= 8      # (two products and a softmax at these lengths)
         assert sum(counts.get(n, 0) for n in ("attn_prefill", "attn_short", "attn_ragged")) == (0 if three else 1), counts
         check(ref, got, f"attention over {S} keys")
 

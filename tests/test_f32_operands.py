@@ -64,3 +64,32 @@ def test_few_rows_of_a_deep_product_with_a_residual_and_special_values(hip_bf16)
     for kind in (np.isposinf, np.isneginf, np.isnan):
         assert np.array_equal(kind(exact), kind(got.astype(np.float64)))
     assert_f32_sums(exact[3:], got[3:], K, "finite rows")
+
+
+# A few queries: the scores, their exponentials and both products of the attention in f32
+@pytest.mark.gpu
+@pytest.mark.parametrize("S", [2, 3, 7, 8])
+@pytest.mark.parametrize("H,KV,d,T,causal", [(8, 2, 64, 0, True), (4, 4, 128, 0, True), (4, 1, 256, 0, True), (8, 2, 64, 61, False),
+                                             (8, 2, 64, 65, False), (2, 2, 128, 32, False), (2, 2, 128, 33, False), (4, 1, 64, 700, False)])
+def test_attention_of_a_few_queries(hip_bf16, S, H, KV, d, T, causal):
+    T = T or S
+    g = np.random.default_rng(S + T)
+    q, k, v = (g.standard_normal((h, n, d)).astype(np.float32) for h, n in ((H, S), (KV, T), (KV, T)))
+
+    def f(b, q, k, v):
+        q, k, v = (lang.reshape(b, lang.make_shape(b, 1, h, n, d), t) for t, h, n in ((q, H, S), (k, KV, T), (v, KV, T)))
+        q, k, v = q + q - q, k + k - k, v + v - v
+        a = lang.matmul(b, q, lang.transpose(b, 2, 3, helpers.repeat_kv(b, H // KV, k)))
+        sh = lang.shape(b, a)
+        a = a / lang.constant(b, float(np.sqrt(np.float32(d))), sh)
+        if causal:
+            a = a + lang.broadcast(b, helpers.causal_mask(b, lang.to_nat(b, S)), sh)
+        return [lang.matmul(b, nn.softmax(b, a), helpers.repeat_kv(b, H // KV, v))]
+    (got,) = vectors.run(hip_bf16, f, 1, q.reshape(-1), k.reshape(-1), v.reshape(-1))
+    q, k, v = q.astype(np.float64), *(np.repeat(t.astype(np.float64), H // KV, axis=0) for t in (k, v))
+    s = q @ k.transpose(0, 2, 1) / float(np.sqrt(np.float32(d)))
+    if causal:
+        s[:, np.triu(np.ones((S, S), bool), 1)] = -np.inf
+    p = np.exp(s - s.max(-1, keepdims=True))
+    exact = (p / p.sum(-1, keepdims=True)) @ v
+    assert_f32_sums(exact, got, d + T, f"{S} queries over {T} keys")
