@@ -961,6 +961,34 @@ __global__ void __launch_bounds__(256) splitk_reduce_kernel(const float *ws, flo
   }
 }
 
+// An f32 as the sum of three bf16 values, exactly (8 + 8 + 8 bits of its 24; below 2^-110 the last ones fall under the
+// smallest bf16): against bf16 weights the products of the parts add up to the product of the whole.  Cut, not rounded:
+// every part has the sign of the whole and the largest f32 stays finite.  Infinities and NaN are the first part alone.
+// (Beside an infinite weight a part that is zero makes a NaN of what was an infinity.)
+__device__ __forceinline__ void bf16_three(float x, uint32_t (&part)[3]) {
+  const uint32_t u = __float_as_uint(x);
+  part[0] = u >> 16;
+  part[1] = part[2] = 0;
+  if ((u & 0x7F800000u) == 0x7F800000u) {
+    if (u & 0x7FFFFFu) part[0] |= 0x40u;  // (a NaN whose bits are all in the part cut off)
+    return;
+  }
+  const float r1 = x - __uint_as_float(u & 0xFFFF0000u);
+  const uint32_t u1 = __float_as_uint(r1);
+  part[1] = u1 >> 16;
+  part[2] = __float_as_uint(r1 - __uint_as_float(u1 & 0xFFFF0000u)) >> 16;
+}
+// four values to the same place of three planes of bf16 that lie `plane` values apart
+__device__ __forceinline__ void bf16_planes4(float4 v, uint16_t *out, uint64_t plane) {
+  uint32_t a[3], b[3], c[3], d[3];
+  bf16_three(v.x, a);
+  bf16_three(v.y, b);
+  bf16_three(v.z, c);
+  bf16_three(v.w, d);
+#pragma unroll
+  for (int p = 0; p < 3; ++p) *(uint2 *)(out + p * plane) = make_uint2(a[p] | b[p] << 16, c[p] | d[p] << 16);
+}
+
 // f32 -> bf16 (round to nearest even, v_cvt_pk_bf16_f32), contiguous, 8 elements per thread
 __global__ void __launch_bounds__(256) cast_bf16_kernel(const float *in, uint16_t *out, uint64_t n8) {
   for (uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x; i < n8;
@@ -2238,13 +2266,24 @@ __global__ void __launch_bounds__(256) moe_gemm_kernel(MoeGemmDesc g) {
 // One workgroup of 1024 threads sorts the (slot, token) pairs by expert: a histogram in LDS, a scan,
 // and a scatter through per-expert cursors.  The order of an expert's pairs depends on the order
 // the atomics land in, which only decides the tile row a token occupies, never its result.
-// tiles (optional): tiles[0] = the number of 128-pair row tiles over all experts, tiles[1 + t] = expert << 16 |
+// tiles (optional): tiles[0] = the number of row tiles (moe_tile_pairs pairs each) over all experts, tiles[1 + t] = expert << 16 |
 // row tile within the expert, expert by expert - the work list of the GEMM, one workgroup per (row tile, column
 // tile), so that an expert most tokens chose is spread over the device instead of walked by one workgroup.
+// The workgroups behind the first, if any, split the S rows of slot 0's f32 input into the three planes at `planes`.
+__host__ __device__ constexpr uint32_t moe_tile_pairs(bool planes) { return planes ? 20 : 128; }
 __global__ void __launch_bounds__(1024) moe_route_kernel(MoeGemmDesc g, uint32_t *count, uint32_t *offset, uint32_t *list,
-                                                         uint32_t *tiles) {
+                                                         uint32_t *tiles, uint16_t *planes) {
   __shared__ uint32_t hist[MOE_ROUTE_MAX_EXPERTS], cursor[MOE_ROUTE_MAX_EXPERTS], scan[1024];
   const uint32_t tid = threadIdx.x, E = g.n_expert, S = g.S, pairs = S * g.n_slot;
+  if (blockIdx.x) {
+    const uint32_t per_row = g.K / 4, n = S * per_row;
+    for (uint32_t i = (blockIdx.x - 1) * 1024 + tid; i < n; i += (gridDim.x - 1) * 1024) {
+      const uint32_t r = i / per_row, k = (i - r * per_row) * 4;
+      const float *x = g.slot[0].a + (int64_t)r * g.slot[0].a_bs + k;
+      bf16_planes4(*(const float4 *)x, planes + (uint64_t)i * 4, (uint64_t)S * g.K);
+    }
+    return;
+  }
   for (uint32_t i = tid; i < E; i += 1024) hist[i] = 0;
   __syncthreads();
   for (uint32_t p = tid; p < pairs; p += 1024) {
@@ -2283,8 +2322,9 @@ __global__ void __launch_bounds__(1024) moe_route_kernel(MoeGemmDesc g, uint32_t
   }
   if (!tiles) return;
   // the same scan over row tiles per expert
+  const uint32_t tp = moe_tile_pairs(g.planes);
   uint32_t my_tiles = 0;
-  for (uint32_t i = first; i < min(E, first + per); ++i) my_tiles += (hist[i] + 127) / 128;
+  for (uint32_t i = first; i < min(E, first + per); ++i) my_tiles += (hist[i] + tp - 1) / tp;
   scan[tid] = my_tiles;
   __syncthreads();
   for (uint32_t d = 1; d < 1024; d <<= 1) {
@@ -2295,18 +2335,22 @@ __global__ void __launch_bounds__(1024) moe_route_kernel(MoeGemmDesc g, uint32_t
   }
   uint32_t tt = scan[tid] - my_tiles;
   for (uint32_t i = first; i < min(E, first + per); ++i)
-    for (uint32_t j = 0; j < (hist[i] + 127) / 128; ++j) tiles[1 + tt++] = i << 16 | j;
+    for (uint32_t j = 0; j < (hist[i] + tp - 1) / tp; ++j) tiles[1 + tt++] = i << 16 | j;
   if (tid == 1023) tiles[0] = scan[1023];
 }
 
 // most row tiles launch_moe_route can list for g: every expert may end in a partly filled one
-uint32_t moe_route_max_tiles(const MoeGemmDesc &g) { return (g.S * g.n_slot + 127) / 128 + g.n_expert; }
+uint32_t moe_route_max_tiles(const MoeGemmDesc &g) {
+  return (g.S * g.n_slot + moe_tile_pairs(g.planes) - 1) / moe_tile_pairs(g.planes) + g.n_expert;
+}
 
 hipError_t launch_moe_route(const LaunchCtx &lc, const MoeGemmDesc &g, uint32_t *count, uint32_t *offset, uint32_t *list,
-                            uint32_t *tiles) {
+                            uint32_t *tiles, uint16_t *planes) {
   if (!g.S || !g.n_slot || !g.n_expert) return hipSuccess;
   if (g.n_expert > MOE_ROUTE_MAX_EXPERTS || g.S > 65535 || g.n_slot > 8) return hipErrorInvalidValue;
-  CG_LAUNCH(lc, moe_route_kernel, 1, 1024, g, count, offset, list, tiles);
+  if (planes && (!g.slot[0].a || (uintptr_t)g.slot[0].a % 16 || g.slot[0].a_bs % 4 || g.K % 8 || (uintptr_t)planes % 16)) return hipErrorInvalidValue;
+  const uint32_t split = planes ? (g.S * (g.K / 4) + 1023) / 1024 : 0;
+  CG_LAUNCH(lc, moe_route_kernel, 1 + split, 1024, g, count, offset, list, tiles, planes);
   return hipGetLastError();
 }
 
@@ -2315,9 +2359,20 @@ hipError_t launch_moe_route(const LaunchCtx &lc, const MoeGemmDesc &g, uint32_t 
 // global_load_lds_dwordx4 exactly as in gemm_bf16_dma_kernel - same 1 KB wave loads, same XOR
 // swizzle, NS stages in flight - so a k-step no longer waits out a trip to memory.  Wavefront w
 // computes columns [32 w, 32 w + 32) of every 32-row tile that has a live row.
-template <int NP, int NS>
+//
+// PLANES: token rows that stay f32 (the 9 to 63 tokens of a short prompt), as three planes of bf16 parts (bf16_three).  A
+// 32-row tile holds ten pairs three times over - rows 0 to 9 their first parts, 10 to 19 the second, 20 to 29 the third -,
+// so that an expert of a few pairs still moves its weights and 32 rows; 20 pairs to a workgroup (where most tokens choose the
+// same experts, few column tiles have work: a 63-token prompt whose crowded experts took four turns of 20 in one workgroup
+// 7.4 ms, 5.1 so).  What a k-step adds
+// is summed apart and then added to the running sum: a chain of K / 64 roundings, like that of a lane of the one-row
+// kernels, instead of K / 16.  Bound by the stream of weights as without planes (60 experts of 2048 x 1408, 63 tokens: both
+// launches and the routing 193 us, 180 with rows rounded to bf16).
+template <int NP, int NS, bool PLANES = false>
 __global__ void __launch_bounds__(256) moe_gemm_dma_kernel(MoeGemmDesc g) {
-  constexpr int BM_ = 128, BN_ = 128, BK = 64, MT = BM_ / 32;
+  constexpr int BM_ = PLANES ? 64 : 128, BN_ = 128, BK = 64, MT = BM_ / 32;
+  constexpr int TPAIRS = PLANES ? 10 : 32, PAIRS = MT * TPAIRS;  // pairs of 32 rows, of a row tile
+  static_assert(PAIRS == moe_tile_pairs(PLANES), "the work list's row tiles");
   constexpr int ROWS = BM_ + NP * BN_;    // the stacked [A; B0; B1] tile of a stage
   constexpr int LPW = ROWS / 8 / 4;       // 1 KB loads per wave per stage
   constexpr int STAGE = ROWS * BK * 2;    // bytes
@@ -2336,8 +2391,8 @@ __global__ void __launch_bounds__(256) moe_gemm_dma_kernel(MoeGemmDesc g) {
     if (e >= g.route_tiles[0]) return;  // the grid is sized for the most tiles there can be
     const uint32_t ent = g.route_tiles[1 + e];
     e = ent >> 16;
-    m_first = (ent & 0xFFFFu) * BM_;
-    m_last = m_first + BM_;
+    m_first = (ent & 0xFFFFu) * PAIRS;
+    m_last = m_first + PAIRS;
   }
   if (e >= g.n_expert) return;  // the grid is sized for the wider problem
   const uint32_t cnt = min(g.route_count[e], m_last);
@@ -2352,15 +2407,19 @@ __global__ void __launch_bounds__(256) moe_gemm_dma_kernel(MoeGemmDesc g) {
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint16_t *)dma_smem;
   const int sw = (lane >> 1) & 7, half = lane >> 5;
   const int n_steps = (int)(K / BK);
-  for (uint32_t m0 = m_first; m0 < cnt; m0 += BM_) {
-    const int live_tiles = (int)min((uint32_t)MT, (cnt - m0 + 31) / 32);  // wave-uniform
-    f32x16 acc[NP][MT];
+  const int64_t plane = PLANES ? (int64_t)g.S * K : 0;
+  for (uint32_t m0 = m_first; m0 < cnt; m0 += PAIRS) {
+    const int live_tiles = (int)min((uint32_t)MT, (cnt - m0 + TPAIRS - 1) / TPAIRS);  // wave-uniform
+    f32x16 acc[NP][MT], run[PLANES ? NP : 1][PLANES ? MT : 1];  // run: the sum over the k-steps so far
 #pragma unroll
     for (int p = 0; p < NP; ++p)
 #pragma unroll
       for (int h = 0; h < MT; ++h)
 #pragma unroll
-        for (int i = 0; i < 16; ++i) acc[p][h][i] = 0.f;
+        for (int i = 0; i < 16; ++i) {
+          acc[p][h][i] = 0.f;
+          if constexpr (PLANES) run[p][h][i] = 0.f;
+        }
     // Load i of a wave: i < MT: its eight rows of the i-th 32-row tile of token rows (not made when no pair is in
     // that tile: an expert of a few pairs moves its weights and 32 rows, not 128), then its share of the weight rows.
     const uint16_t *gp[LPW];  // per-lane source; advances by BK per stage
@@ -2372,7 +2431,8 @@ __global__ void __launch_bounds__(256) moe_gemm_dma_kernel(MoeGemmDesc g) {
       const int c = (lane & 7) ^ ((R >> 1) & 7);
       if (i < MT) {
         // rows past the expert's last pair repeat it: loaded, multiplied, never stored
-        const uint32_t ent = list[min(m0 + (uint32_t)R, cnt - 1)], sl = ent >> 16, tok = ent & 0xFFFFu;
+        const int part = PLANES ? min((R & 31) / TPAIRS, 2) : 0, pair = PLANES ? (R >> 5) * TPAIRS + (R & 31) % TPAIRS : R;
+        const uint32_t ent = list[min(m0 + (uint32_t)pair, cnt - 1)], sl = ent >> 16, tok = ent & 0xFFFFu;
         const uint16_t *rows = g.slot[0].a16;
         int64_t bs = g.slot[0].a_bs;
 #pragma unroll
@@ -2381,7 +2441,7 @@ __global__ void __launch_bounds__(256) moe_gemm_dma_kernel(MoeGemmDesc g) {
             rows = g.slot[s].a16;
             bs = g.slot[s].a_bs;
           }
-        gp[i] = rows + (int64_t)tok * bs + c * 8;
+        gp[i] = rows + part * plane + (int64_t)tok * bs + c * 8;
       } else {
         const int rb = R - BM_, p = rb / BN_, col = rb - p * BN_;
         gp[i] = W[p < NP ? p : 0] + (int64_t)min(n0 + (uint32_t)col, N - 1) * sbn[p < NP ? p : 0] + c * 8;
@@ -2419,6 +2479,17 @@ __global__ void __launch_bounds__(256) moe_gemm_dma_kernel(MoeGemmDesc g) {
               acc[p][h] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[ks & 1][h], bfr[ks & 1][p], acc[p][h], 0, 0, 0);
         __builtin_amdgcn_sched_barrier(0);
       }
+      if constexpr (PLANES) {
+#pragma unroll
+        for (int p = 0; p < NP; ++p)
+#pragma unroll
+          for (int h = 0; h < MT; ++h)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+              run[p][h][i] += acc[p][h][i];
+              acc[p][h][i] = 0.f;
+            }
+      }
     };
 #pragma unroll
     for (int s0 = 0; s0 < NS - 1; ++s0)
@@ -2439,6 +2510,50 @@ __global__ void __launch_bounds__(256) moe_gemm_dma_kernel(MoeGemmDesc g) {
     // (the operand stages are free now) so that a row leaves as 16-byte pieces: f32 for a plain
     // product, bf16 act(gate) * up for the fused pair.
     __syncthreads();  // every wave is done reading the last stage
+    if constexpr (PLANES) {
+      constexpr int P = BN_ + 4;
+      float *T = (float *)dma_smem;
+#pragma unroll
+      for (int p = 0; p < NP; ++p)
+#pragma unroll
+        for (int h = 0; h < MT; ++h)
+#pragma unroll
+          for (int i = 0; i < 16; ++i)
+            T[(p * BM_ + h * 32 + (i >> 2) * 8 + (lane >> 5) * 4 + (i & 3)) * P + wave * 32 + (lane & 31)] = run[p][h][i];
+      __syncthreads();
+      const uint32_t pairs_here = min((uint32_t)PAIRS, cnt - m0);
+      for (uint32_t idx = tid; idx < pairs_here * (BN_ / 4); idx += 256) {
+        const uint32_t j = idx / (BN_ / 4), c = (idx - j * (BN_ / 4)) * 4;
+        if (n0 + c >= N) continue;
+        const uint32_t ent = list[m0 + j], sl = ent >> 16;
+        const uint64_t at = (uint64_t)(ent & 0xFFFFu) * N + n0 + c;
+        float4 v[NP];
+#pragma unroll
+        for (int p = 0; p < NP; ++p) {  // the parts' products, the smallest first
+          const float *t = T + (p * BM_ + j / TPAIRS * 32 + j % TPAIRS) * P + c;
+          const float4 hi = *(const float4 *)t, mid = *(const float4 *)(t + TPAIRS * P), lo = *(const float4 *)(t + 2 * TPAIRS * P);
+          v[p] = make_float4((lo.x + mid.x) + hi.x, (lo.y + mid.y) + hi.y, (lo.z + mid.z) + hi.z, (lo.w + mid.w) + hi.w);
+        }
+        if constexpr (NP == 2) {
+          auto act = [&](float x) { return g.fuse_glu == PRO_GEGLU ? gelu_ref(x) : x * sigmoid_ref(x); };
+          uint16_t *out = g.slot[0].h16;
+#pragma unroll
+          for (int s2 = 1; s2 < 8; ++s2)
+            if (sl == (uint32_t)s2) out = g.slot[s2].h16;
+          bf16_planes4(make_float4(act(v[0].x) * v[1].x, act(v[0].y) * v[1].y, act(v[0].z) * v[1].z, act(v[0].w) * v[1].w), out + at,
+                       (uint64_t)g.S * N);
+        } else {
+          float *out = g.slot[0].c[prob];
+#pragma unroll
+          for (int s2 = 1; s2 < 8; ++s2)
+            if (sl == (uint32_t)s2) out = g.slot[s2].c[prob];
+          *(float4 *)(out + at) = v[0];
+        }
+      }
+      wait_vmcnt<0>();
+      __syncthreads();
+      continue;
+    }
     constexpr int TP = NP == 2 ? BN_ + 8 : BN_ + 4;  // row pitch in elements (keeps 16-byte alignment)
     if (NP == 2) {
       uint16_t *T = dma_smem;
@@ -2502,18 +2617,19 @@ bool moe_gemm_pipelined_ok(const MoeGemmDesc &g) {
   return true;
 }
 
-template <int NP, int NS>
+template <int NP, int NS, bool PLANES = false>
 static hipError_t launch_moe_gemm_dma(const LaunchCtx &lc, const MoeGemmDesc &g, dim3 grid) {
   // the operand stages, or the staged output tile (f32 rows of 128 + 4, or bf16 rows of 128 + 8) if that is larger
-  constexpr int stages = NS * (128 + NP * 128) * 64 * 2, tile = NP == 2 ? 128 * (128 + 8) * 2 : 128 * (128 + 4) * 4;
+  constexpr int stages = NS * ((PLANES ? 64 : 128) + NP * 128) * 64 * 2;
+  constexpr int tile = PLANES ? NP * 64 * (128 + 4) * 4 : NP == 2 ? 128 * (128 + 8) * 2 : 128 * (128 + 4) * 4;
   constexpr int smem = stages > tile ? stages : tile;
   static bool configured = false;  // one attribute call per kernel and process
   if (!configured) {
-    hipError_t e = hipFuncSetAttribute((const void *)moe_gemm_dma_kernel<NP, NS>, hipFuncAttributeMaxDynamicSharedMemorySize, smem);
+    hipError_t e = hipFuncSetAttribute((const void *)moe_gemm_dma_kernel<NP, NS, PLANES>, hipFuncAttributeMaxDynamicSharedMemorySize, smem);
     if (e != hipSuccess) return e;
     configured = true;
   }
-  cg_launch(lc, moe_gemm_dma_kernel<NP, NS>, grid, dim3(256), smem, g);
+  cg_launch(lc, moe_gemm_dma_kernel<NP, NS, PLANES>, grid, dim3(256), smem, g);
   return hipGetLastError();
 }
 
@@ -2524,6 +2640,13 @@ hipError_t launch_moe_gemm(const LaunchCtx &lc, const MoeGemmDesc &g) {
   uint32_t max_n = 0;
   for (uint32_t i = 0; i < g.n_prob; ++i) max_n = g.prob[i].N > max_n ? g.prob[i].N : max_n;
   if (!max_n) return hipSuccess;
+  if (g.planes) {  // (dense planes of S rows of K)
+    if (!moe_gemm_pipelined_ok(g) || (g.fuse_glu ? g.n_prob != 2 || g.prob[0].N != g.prob[1].N : g.n_prob != 1)) return hipErrorInvalidValue;
+    for (uint32_t s = 0; s < g.n_slot; ++s)
+      if (g.slot[s].a_bs != (int64_t)g.K) return hipErrorInvalidValue;
+    const dim3 grid((max_n + 127) / 128 * (g.route_tiles ? moe_route_max_tiles(g) : g.n_expert), 1, 1);
+    return g.fuse_glu ? launch_moe_gemm_dma<2, 3, true>(lc, g, grid) : launch_moe_gemm_dma<1, 3, true>(lc, g, grid);
+  }
   if (g.fuse_glu) {
     if (g.n_prob != 2 || g.prob[0].N != g.prob[1].N || g.pro != PRO_NONE) return hipErrorInvalidValue;
     if (moe_gemm_pipelined_ok(g))

@@ -505,10 +505,10 @@ struct MoeGemmDesc {
     const uint32_t *idx;                    // idx[t * idx_stride] = expert of token t in this slot
     int64_t idx_stride;
     const float *a, *aux;                   // f32 input rows: a + t * a_bs (aux + t * aux_bs), unit stride along k
-    const uint16_t *a16;                    // or bf16 input rows (a16 + t * a_bs), taken as they are
+    const uint16_t *a16;                    // or bf16 input rows (a16 + t * a_bs), taken as they are (or planes, below)
     int64_t a_bs, aux_bs;
     float *c[2];                            // outputs per problem, contiguous [S, N]
-    uint16_t *h16;                          // fuse_glu: gated activations, contiguous bf16 [S, N]
+    uint16_t *h16;                          // fuse_glu: gated activations, contiguous bf16 [S, N] (or three planes of that)
   } slot[8];
   struct {
     const void *w;                          // [E, N, K], unit stride along k, row stride sbn
@@ -516,6 +516,9 @@ struct MoeGemmDesc {
     uint32_t N;
   } prob[2];
   uint32_t *err;                            // ERRF_INDEX_OOB for an index >= n_expert (served by the last expert)
+  // a16 and h16 are three planes [3][S][K], [3][S][N] of bf16 parts that add up to f32 values, and the products are those
+  // of the f32 values (moe_gemm_pipelined_ok; n_prob 1, or 2 with fuse_glu)
+  int32_t planes;
   // optional: the (slot, token) pairs already sorted by expert (launch_moe_route): pairs
   // route_list[route_offset[e] .. + route_count[e]) = slot << 16 | token chose expert e
   const uint32_t *route_count, *route_offset, *route_list;
@@ -528,11 +531,12 @@ hipError_t launch_moe_gemm(const LaunchCtx &lc, const MoeGemmDesc &g);
 // (slot[].a16 for every slot) and K % 64 == 0, launch_moe_gemm streams the weights through a
 // multi-stage direct-to-LDS pipeline.
 enum { MOE_ROUTE_MAX_EXPERTS = 4096 };
-// tiles (optional, 1 + moe_route_max_tiles(g) words): the number of 128-pair row tiles over all experts, then
+// tiles (optional, 1 + moe_route_max_tiles(g) words): the number of row tiles (128 pairs, 20 of planes) over all experts, then
 // expert << 16 | row tile for each; with it in g.route_tiles a workgroup of launch_moe_gemm owns one row tile
 // of one expert, so the launch stays balanced when most tokens choose the same few experts.
+// planes (optional): the S rows of K f32 values at slot[0].a, as the planes that launch_moe_gemm takes
 hipError_t launch_moe_route(const LaunchCtx &lc, const MoeGemmDesc &g, uint32_t *count, uint32_t *offset, uint32_t *list,
-                            uint32_t *tiles);
+                            uint32_t *tiles, uint16_t *planes);
 uint32_t moe_route_max_tiles(const MoeGemmDesc &g);
 bool moe_gemm_pipelined_ok(const MoeGemmDesc &g);
 // wrapping u32 matmul (ndarray's generic dot); all operands contiguous

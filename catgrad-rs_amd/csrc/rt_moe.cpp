@@ -20,9 +20,13 @@ bool match_expert_operand(const cg_tensor *t, int64_t S, ExpertOperand *o) {
 // The same products over many tokens (a prefill, bf16 mode): expert by expert instead of token by
 // token, and all k slots of the layer in one launch - every deferred expert product on the same
 // stacked weights joins, with its own indices, input rows and output (launch_moe_gemm).
+// From 64 tokens on the rows are rounded to bf16, like those of every product of many rows.  Fewer stay f32: token by token
+// (try_moe_gemv) below 12, as planes of bf16 parts from there on.  60 experts of 2048 x 1408, 4 to a token, both launches
+// and the routing, token by token and in planes: 9 tokens 97 us (105 on tiles of rounded rows); 12 128, 115; 16 152, 134; 24
+// 250, 174; 32 285, 180; 63 588, 193 (rounded 180).  Off the 64-bit result by 2.1e-7 to 2.2e-7 either way (rounded 2.9e-3).
 int try_moe_gemm(cg_backend *be, cg_tensor *n, bool *done) {
   const int64_t S = n->shape[0];
-  if (S <= 8 || S > 65535 || !(be->flags & CG_FLAG_BF16)) return CG_OK;
+  if (S < 12 || S > 65535 || !(be->flags & CG_FLAG_BF16)) return CG_OK;
   ExpertOperand eo;
   if (!match_expert_operand(n->in[1], S, &eo)) return CG_OK;
   const int64_t K = n->in[0]->shape[2];
@@ -163,16 +167,19 @@ int try_moe_gemm(cg_backend *be, cg_tensor *n, bool *done) {
         return w->rank == 3 && w->stype == ST_BF16 && w->shape[0] == d.n_expert && w->shape[1] == n_rows && w->shape[2] == k &&
                w->strides[2] == 1 && (uintptr_t)data_ptr(w) % 16 == 0 && w->strides[1] % 8 == 0 && w->strides[0] % 8 == 0;
       };
+      const bool planes = S < 64;
+      if (planes && (H % 64 || F % 64 || d.n_expert > MOE_ROUTE_MAX_EXPERTS)) return CG_OK;  // token by token
       if (H % 8 == 0 && x->stype == ST_F32 && x->strides[2] == 1 && x->strides[0] % 8 == 0 && x->offset % 8 == 0 &&
           x->st->bytes % 32 == 0 && x->st->grow_dim < 0 && w_ok(wg, F, H) && w_ok(wu, F, H) && wg->strides[0] == wu->strides[0]) {
-        Storage *xsh = nullptr;
-        TRY(bf16_shadow(be, x->st, &xsh));
+        Storage *xsh = nullptr, *xplanes = nullptr;
+        if (!planes) TRY(bf16_shadow(be, x->st, &xsh));
         std::vector<Storage *> hbuf(slot_a.size(), nullptr);
         auto drop_h = [&]() {
           for (Storage *h : hbuf) storage_release(h);
+          storage_release(xplanes);
         };
-        int st = CG_OK;
-        for (size_t sl = 0; sl < hbuf.size() && !st; ++sl) st = dev_alloc(be, (size_t)S * F * 2, &hbuf[sl]);
+        int st = planes ? dev_alloc(be, (size_t)S * H * 6, &xplanes) : CG_OK;
+        for (size_t sl = 0; sl < hbuf.size() && !st; ++sl) st = dev_alloc(be, (size_t)S * F * (planes ? 6 : 2), &hbuf[sl]);
         for (const Member &m : members)
           if (!st) st = alloc_result(be, m.c, ST_F32);
         if (st) {
@@ -188,13 +195,14 @@ int try_moe_gemm(cg_backend *be, cg_tensor *n, bool *done) {
         f.prob[0].w = data_ptr(wg); f.prob[0].sbn = wg->strides[1]; f.prob[0].N = (uint32_t)F;
         f.prob[1].w = data_ptr(wu); f.prob[1].sbn = wu->strides[1]; f.prob[1].N = (uint32_t)F;
         for (size_t sl = 0; sl < hbuf.size(); ++sl) {
-          f.slot[sl].a16 = (const uint16_t *)xsh->ptr + x->offset;
-          f.slot[sl].a_bs = x->strides[0];
+          f.slot[sl].a16 = planes ? (const uint16_t *)xplanes->ptr : (const uint16_t *)xsh->ptr + x->offset;
+          f.slot[sl].a_bs = planes ? H : x->strides[0];
           f.slot[sl].h16 = (uint16_t *)hbuf[sl]->ptr;
           d.slot[sl].a16 = (const uint16_t *)hbuf[sl]->ptr;
           d.slot[sl].a_bs = F;
         }
         d.pro = PRO_NONE;
+        f.planes = d.planes = planes;
         for (const Member &m : members) d.slot[m.slot].c[0] = (float *)m.c->st->ptr;
         hipError_t e = hipSuccess;
         // the pairs sorted by expert once, for both launches: count, offset (one word per expert), list
@@ -208,8 +216,11 @@ int try_moe_gemm(cg_backend *be, cg_tensor *n, bool *done) {
           }
           uint32_t *rc = (uint32_t *)route->ptr, *ro = rc + d.n_expert, *rl = ro + d.n_expert, *rt = rl + (size_t)S * d.n_slot;
           {
-            KernelScope ks(be, "experts_route", (double)S * d.n_slot * 8, 0);
-            e = launch_moe_route(be->lc(), d, rc, ro, rl, rt);
+            KernelScope ks(be, "experts_route", (double)S * d.n_slot * 8 + (planes ? (double)S * H * 10 : 0), 0);
+            MoeGemmDesc rd = f;
+            rd.slot[0].a = (const float *)data_ptr(x);
+            rd.slot[0].a_bs = x->strides[0];
+            e = launch_moe_route(be->lc(), rd, rc, ro, rl, rt, planes ? (uint16_t *)xplanes->ptr : nullptr);
           }
           f.route_tiles = d.route_tiles = rt;
           f.route_count = d.route_count = rc;
@@ -242,6 +253,7 @@ int try_moe_gemm(cg_backend *be, cg_tensor *n, bool *done) {
       }
     }
   }
+  if (S < 64) return CG_OK;  // token by token
   // input rows
   std::vector<cg_tensor *> held;
   auto drop_held = [&]() {

@@ -93,3 +93,39 @@ def test_attention_of_a_few_queries(hip_bf16, S, H, KV, d, T, causal):
     p = np.exp(s - s.max(-1, keepdims=True))
     exact = (p / p.sum(-1, keepdims=True)) @ v
     assert_f32_sums(exact, got, d + T, f"{S} queries over {T} keys")
+
+
+# The routed experts of 9 to 63 tokens: rows and gated values in f32 beside the bf16 matrices, an expert with no pair, with
+# few, with more than a tile of 20 holds; sizes that the tile kernel takes and (fewer than 12 tokens,
+# F = 96 or 136) those that it does not
+@pytest.mark.gpu
+@pytest.mark.parametrize("S,k,E,H,F", [(9, 2, 5, 256, 192), (11, 4, 7, 128, 64), (12, 4, 60, 128, 64), (30, 3, 4, 320, 256), (63, 4, 7, 64, 136), (63, 1, 3, 1024, 448),
+                                       (40, 8, 9, 128, 64), (21, 2, 6, 128, 96)])
+def test_experts_of_a_short_prompt(hip_bf16, S, k, E, H, F):
+    g = np.random.default_rng(S * 10 + k)
+    x = g.standard_normal((S, H)).astype(np.float32)
+    x[1] *= np.float32(1e-8)
+    x[2] *= np.float32(1e8)
+    wg, wu = (vectors.bf16_round((g.standard_normal((E, F, H)) * H ** -0.5).astype(np.float32)) for _ in range(2))
+    wd = vectors.bf16_round((g.standard_normal((E, H, F)) * F ** -0.5).astype(np.float32))
+    idx = g.choice(E - 1, (S, k), p=np.r_[0.7, np.full(E - 2, 0.3 / (E - 2))]).astype(np.uint32)    # the last expert has none
+
+    def f(b, x, idx, wg, wu, wd):
+        x = lang.reshape(b, lang.make_shape(b, S, 1, H), x)
+        x = x + x - x
+        out = []
+        for i in range(k):
+            slot = lang.get(b, 1, i, idx)
+            sel = lambda w: lang.transpose(b, 1, 2, lang.index(b, 0, slot, w))      # noqa: B023
+            out.append(lang.matmul(b, nn.silu(b, lang.matmul(b, x, sel(wg))) * lang.matmul(b, x, sel(wu)), sel(wd)))
+        return out
+    hip_bf16.launch_counts(reset=True)
+    got = vectors.run(hip_bf16, f, k, x.reshape(-1), idx, wg, wu, wd)
+    counts = hip_bf16.launch_counts(reset=True)
+    assert (counts.get("gemm_experts_bf16", 0), counts.get("experts_route", 0)) == ((2, 1) if S >= 12 and H % 64 == F % 64 == 0 else (0, 0)), counts
+    wg, wu, wd, x = (a.astype(np.float64) for a in (wg, wu, wd, x))
+    for i in range(k):
+        e = idx[:, i]
+        gate, up = (np.einsum("sh,sfh->sf", x, w[e]) for w in (wg, wu))
+        exact = np.einsum("sf,shf->sh", gate / (1 + np.exp(-np.maximum(gate, -700))) * up, wd[e])
+        assert_f32_sums(exact, got[i], H + F, f"slot {i}")
