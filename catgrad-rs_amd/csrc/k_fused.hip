@@ -1022,10 +1022,6 @@ __global__ void __launch_bounds__(NWV * 64) attn_decode_group_kernel(AttnDecodeD
     }
     if (a.splits == 1) {
       a.out[((uint64_t)b * a.heads + h0 + r) * D + dim] = v / L;
-    } else if (a.merge_later) {
-      float *p = a.part + rec * (D + 4);
-      p[dim] = v;
-      if (dim == 0) { p[D] = M; p[D + 1] = L; }
     } else {  // agent-scope stores, acknowledged before the counter moves (the hand-over of attn_decode_split_kernel)
       float *p = a.part + rec * pw;
       __hip_atomic_store(p + 2 + dim, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -1035,7 +1031,7 @@ __global__ void __launch_bounds__(NWV * 64) attn_decode_group_kernel(AttnDecodeD
       }
     }
   }
-  if (a.splits == 1 || a.merge_later) return;
+  if (a.splits == 1) return;
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
   uint32_t *counter = a.count + (uint64_t)b * (a.heads / rep) + kv;
@@ -1079,7 +1075,7 @@ __global__ void __launch_bounds__(NWV * 64) attn_decode_group_kernel(AttnDecodeD
 }
 
 bool attn_decode_group_ok(const AttnDecodeDesc &d) {
-  return d.rep >= 1 && d.rep <= 16 && d.k_srep == 0 && d.v_srep == 0 && (d.d == 64 || d.d == 128);
+  return d.rep >= 2 && d.rep <= 16 && d.k_srep == 0 && d.v_srep == 0 && !d.merge_later && (d.d == 64 || d.d == 128);
 }
 
 uint32_t attn_decode_rows_per_pass(uint32_t d) { return d <= 64 ? 128 : d <= 128 ? 64 : 32; }

@@ -490,26 +490,28 @@ int try_attn_decode(cg_backend *be, cg_tensor *n, bool *done, AttnMergeLater *la
     // whole decode loop: T ~ 540: 4 ranges 1367, 5 1392, 6 1382, 8 1372 tokens/s; T ~ 200: 2 1415, 3 1421,
     // 4 1421, 8 1397.
     if (later && nb == 1 && ns <= ATTN_MERGE_MAX_SPLITS) ns = std::max<int64_t>((T + 109) / 110, std::min<int64_t>(3, (T + 31) / 32));
-    // Longer caches go to the matrix-core form, 64 KB of keys to a workgroup (fewer: the hand-over of more partials costs
-    // what the shorter chains save; more: a workgroup's chain of passes is what the launch waits for): 32 / 8 heads of 64
-    // over 1500 keys 10.1 -> 9.1 us, 4000 20.7 -> 11.4, 7000 25 -> 13.9; 3 x 16 heads of 128 over 900 16.9 -> 13.4.
-    // Where the reader merges, up to as many ranges as it can take (16 heads of 128, 500 keys: 10.3 -> 6.4 us).  Below,
-    // the vector kernel has the shorter chain (32 / 8 heads of 64 over 520 keys: 5.7 us against 6.8).
-    bool reader_merges = later && nb == 1;
-    if (attn_decode_group_ok(a) && (d == 128 ? T > 128 : a.rep >= 2 && T > 880)) {
+    // Grouped queries over longer caches go to the matrix-core form, 64 KB of keys to a workgroup (fewer: the hand-over of
+    // more partials costs what the shorter chains save; more: a workgroup's chain of passes is what the launch waits for),
+    // merged by the launch (32 heads of 64, 1500 keys: 9.1 + 4.3 us with the reader, 8.4 + 5.0 merged there).
+    // Heads of 64 from 881 keys on, whatever the heads and sequences: 32 / 8 heads 881 keys 8.0 us on the vector kernel, 7.7
+    // so, 1600 9.4, 8.3, 4000 17.5, 11.6; 8 x 881 23.9, 12.5; 8 / 2 8.8, 7.2; 14 / 2 9.5, 8.4.  (520 keys 5.7, 6.8.)
+    // Heads of 128 ask twice the registers, one wave to a SIMD, and pay where the vector kernel reads each cache row for
+    // many heads and sequences, from about 40 000 keys over all of them: 32 / 8 heads 900 keys 10.4, 11.4, 1200 13.7, 12.4;
+    // 4 x 300 11.8, 11.3, 4 x 900 27.0, 14.0, 4 x 150 7.9, 10.5; 16 / 8 1200 11.1, 11.3, 4000 23.5, 15.1; 12 / 2 2400 14.0,
+    // 15.6, 4000 19.6, 16.1.  A query head to each kv head (rep 1) has no row to share: 16 heads of 128, 500 keys 8.9, 10.4;
+    // 4 x 4000 58.6, 82.5; a MoE decode step of 8 sequences at 300 keys 4.46 ms, 4.60.
+    const bool group = attn_decode_group_ok(a) && (d == 64 ? T > 880 : nb * heads * T >= 40960);
+    if (group) {
       a.group = 1;
       const int64_t rows = d == 64 && T < 2048 ? 128 : 16384 / d;
-      ns = (T + rows - 1) / rows;
-      reader_merges = reader_merges && d == 128;  // (32 heads of 64, 1500 keys: 9.1 + 4.3 us merged here, 8.4 + 5.0 by the reader)
-      if (reader_merges && ns <= ATTN_MERGE_MAX_SPLITS) ns = std::min<int64_t>(ATTN_MERGE_MAX_SPLITS, (T + 63) / 64);
-      ns = std::min<int64_t>(ns, 64);
+      ns = std::min<int64_t>((T + rows - 1) / rows, 64);
     }
     if (ns >= 2 || T > ATTN_DECODE_MAX_T) {
       const int64_t chunk = (T + ns - 1) / ns;
       a.chunk = (uint32_t)chunk;
       a.splits = (uint32_t)((T + chunk - 1) / chunk);
       // the reader of the result merges the partials when it can (one row, few splits)
-      if (reader_merges && a.splits >= 2 && a.splits <= ATTN_MERGE_MAX_SPLITS && heads * a.splits <= 256 &&
+      if (later && nb == 1 && !group && a.splits >= 2 && a.splits <= ATTN_MERGE_MAX_SPLITS && heads * a.splits <= 256 &&
           heads * d <= 2048 && d % 4 == 0)
         a.merge_later = 1;
       TRY(attn_decode_scratch(be, (size_t)bh * a.splits * (d + 4), (size_t)bh));
@@ -525,6 +527,12 @@ int try_attn_decode(cg_backend *be, cg_tensor *n, bool *done, AttnMergeLater *la
     }
     const double kv_bytes = 2.0 * nb * Kop.shape[1] * T * d * 4;
     KernelScope ks(be, "attn_decode", kv_bytes + 2.0 * nb * heads * d * 4, 4.0 * nb * heads * T * d);
+    if (be->trace_shapes) {
+      char buf[96];
+      snprintf(buf, sizeof buf, "attn_decode[%s,b%lld,%lld/%lldx%lld,T%lld,s%u]", a.group ? "group" : a.splits ? "split" : "one", (long long)nb,
+               (long long)heads, (long long)Kop.shape[1], (long long)d, (long long)T, a.splits);
+      ks.rename(buf);
+    }
     HIPCHK(be, launch_attn_decode(be->lc(), a));
   }
   if (n->gemv_candidate) forget_gemv_candidate(n);

@@ -85,11 +85,12 @@ def test_rotation_of_several_odd_sequences(oracle, hip_bf16, batch, tokens, head
     moe_tests.test_qwen_prefill_biases_and_rotation_in_the_projections_launch(oracle, hip_bf16, batch, tokens, heads, kv_heads, head_dim)
 
 
-# One query over long caches (the matrix-core form): kv heads shared by 2 to 8 query heads or none, last ranges that are short,
-# more ranges than the reader merges, several sequences; the step's own rows go into the cache through the same launch.
+# One query over long caches: kv heads shared by 2 to 8 query heads (the matrix-core form, from 881 keys or, heads of 128, from
+# 40960 keys over all heads on) or none (the vector form at every length), last ranges that are short; the step's own rows go
+# into the cache through the same launch.
 @pytest.mark.gpu
 @pytest.mark.parametrize("H,KV,d,T,steps", [(4, 1, 64, 881, 2), (8, 8, 128, 129, 3), (4, 2, 128, 515, 2), (16, 2, 64, 2049, 2),
-                                            (2, 1, 128, 4100, 1), (4, 2, 64, 1300, 2)])
+                                            (2, 1, 128, 4100, 1), (4, 2, 64, 1300, 2), (16, 2, 128, 2559, 1), (2, 2, 64, 1000, 1)])
 def test_decode_over_a_long_cache(oracle, hip, H, KV, d, T, steps):
     cfg = llm.Config(hidden_size=H * d, intermediate_size=64, num_hidden_layers=1, num_attention_heads=H, num_key_value_heads=KV,
                      vocab_size=97, rms_norm_eps=1e-5, rope_theta=10000.0)
@@ -103,11 +104,18 @@ def test_decode_over_a_long_cache(oracle, hip, H, KV, d, T, steps):
         # tables' error on both sides and not this launch's)
         r.batch, r.pos, r.kv = 1, 3, [be.tensor(a) for a in kv]
         runners.append(r)
-    for token in (5, 11, 90)[:steps + 1]:     # (the first step copies the cache, the following ones append)
+    hip.trace(2)
+    for i, token in enumerate((5, 11, 90)[:steps + 1]):     # (the first step copies the cache, the following ones append)
+        hip.trace_reset()
         hip.launch_counts(reset=True)
         out = [r.step(token)[1] for r in runners]
         parity.assert_f32(oracle.to_vec(out[0]), hip.to_vec(out[1]), f"token {token}")
         assert hip.launch_counts(reset=True).get("attn_decode") == 1
+        keys = T + i + 1
+        group = H > KV and (keys > 880 if d == 64 else H * keys >= 40960)
+        names = [n for n in hip.trace_report() if n.startswith("attn_decode[")]
+        assert len(names) == 1 and names[0].startswith("attn_decode[group," if group else "attn_decode[split,"), names
+    hip.trace(0)
     for a, b in zip(runners[0].kv, runners[1].kv):
         parity.assert_f32(oracle.to_vec(a), hip.to_vec(b), "cache")
 
@@ -122,10 +130,10 @@ def leave_nan_in_memory(be, *sizes):
 
 # What a cache's room to grow holds before it is written must not reach a result: an appending step of each decode kernel,
 # whose last range of keys ends inside a tile (one workgroup; split keys; the matrix-core form, with one and two tiles of a
-# pass past the end, merged by the launch itself and by the reader).
+# pass past the end).
 @pytest.mark.gpu
 @pytest.mark.parametrize("mode", ["f32", "bf16"])
-@pytest.mark.parametrize("H,KV,d,T", [(4, 2, 64, 20), (4, 2, 64, 300), (4, 1, 64, 881), (16, 2, 64, 2049), (4, 2, 128, 129), (8, 4, 128, 516)])
+@pytest.mark.parametrize("H,KV,d,T", [(4, 2, 64, 20), (4, 2, 64, 300), (4, 1, 64, 881), (16, 2, 64, 2049), (4, 2, 128, 129), (16, 4, 128, 2565)])
 def test_unwritten_rows_of_a_cache_stay_out(oracle, hip, hip_bf16, mode, H, KV, d, T):
     be, check = (hip, parity.assert_f32) if mode == "f32" else (hip_bf16, parity.assert_bf16)
     cfg = llm.Config(hidden_size=H * d, intermediate_size=64, num_hidden_layers=1, num_attention_heads=H, num_key_value_heads=KV,
