@@ -40,9 +40,9 @@ int try_attn_prefill(cg_backend *be, cg_tensor *n, bool *done) {
     ~Held() { storage_release(s); }
   } vt_made;
   const Storage *vt_of = nullptr;
-  // (few keys and narrow heads: nothing but launch latency, the rotations keep the launches of their own)
-  const bool few_keys = T < (f32 ? 512 : 256) && !(be->flags & CG_FLAG_ATTN_ONE_PASS);
-  if (cg_tensor *kr = few_keys && heads * d < 512 ? nullptr : node_under_repeat_kv(S->in[1])) {
+  // (eight layers of 4 / 2 heads of 64, 48 tokens, each rotation a launch of its own: f32 692 us, 673 in pairs; bf16 413, 356
+  // in the projections' launch)
+  if (cg_tensor *kr = node_under_repeat_kv(S->in[1])) {
     bool paired = false;
     // ... or none at all: the projections still deferred rotate q and k in their epilogue
     if (!f32 && (d == 64 || d == 128)) TRY(try_qkv_rope_gemm(be, q, kr, node_under_repeat_kv(n->in[1]), &vt_made.s, &vt_of, &paired));
@@ -196,8 +196,7 @@ int try_attn_prefill(cg_backend *be, cg_tensor *n, bool *done) {
   }
   {
     const double qo = 2.0 * nb * heads * Sq * d * 4, kvb = 2.0 * nb * Kop.shape[1] * T * d * 4;
-    // (the records tell the plain launches from those of few keys and of mask rows copied for alignment)
-    KernelScope ks(be, T % 8 ? "attn_ragged" : few_keys ? "attn_short" : "attn_prefill", qo + kvb + (mask ? (double)Sq * T * 4 : 0.0), 4.0 * nb * heads * Sq * T * d);
+    KernelScope ks(be, "attn_prefill", qo + kvb + (mask ? (double)Sq * T * 4 : 0.0), 4.0 * nb * heads * Sq * T * d);
     hipError_t ae = launch_attn_prefill(be->lc(), a);
     storage_release(vt);
     HIPCHK(be, ae);
