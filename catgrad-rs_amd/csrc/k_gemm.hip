@@ -2845,14 +2845,15 @@ bool gemm_act_ok(const LaunchCtx &lc, const GemmDesc &g) {
 // not start on 16 bytes) on the direct-to-LDS kernel.  Up to two launches of 3 - 8 us, against a generic kernel that
 // widens and rounds every element on its way into LDS, eight at a time: sigmoid(x W1) W2 of 64 x 128 x 256 x 10 in
 // 57 us without, 34 with the copies; 300 x 500 x 1000 x 50 145, 54; 1000 x 1000 x 1000 x 10 105, 65; 6000 x 1000 x 4100
-// x 100 802, 230 (the product 420 us at 117 TFLOP/s -> 76 us at 650).  Below PACK_MIN_FLOPS nothing was measured; operands
-// that gemm_bf16_nt_kernel reads in 16-byte pieces are copied from PACK_ALIGNED_MIN_FLOPS on only.
-constexpr double PACK_MIN_FLOPS = 1e5, PACK_ALIGNED_MIN_FLOPS = 8e9;
+// x 100 802, 230 (the product 420 us at 117 TFLOP/s -> 76 us at 650); the smallest, one product of 17 x 65 x 8, 12.2 us, 8.5.
+// Operands that gemm_bf16_nt_kernel reads in 16-byte pieces are copied for 64 rows and PACK_ALIGNED_MIN_FLOPS on only (fewer
+// rows do not pay for the copy of a matrix: 8 x 63 x 2048 x 8192 150 us as it lies, 170 with the copy).
+constexpr double PACK_ALIGNED_MIN_FLOPS = 8e9;
 bool gemm_pack_wanted(const GemmDesc &g, bool epilogue) {
   const uint32_t batch = g.nb0 * g.nb1;
   if (!g.bf16_math || g.b_index || !gemm_rows(g.M, g.K) || g.K < 64 || g.N < 8 || batch > 65535) return false;
   if ((g.sak != 1 && g.sam != 1) || (g.sbk != 1 && g.sbn != 1)) return false;
-  if (2.0 * batch * g.M * g.N * g.K < PACK_MIN_FLOPS) return false;
+  epilogue = epilogue && g.N >= 64;  // (fewer columns: not on the kernel that has one - 17 x 64 x 8 with a sigmoid 9.3 us, 12.6)
   GemmDesc t = g;  // (as it would run: f32 operands with unit strides along k are read from their bf16 twins)
   const int asz = g.a_stype == ST_BF16 ? 2 : 4, bsz = g.b_stype == ST_BF16 ? 2 : 4;
   const int av = vec_ok(g.a, asz, g.sak == 1 ? g.sam : g.sak, g.sa_b0, g.sa_b1);
@@ -2862,7 +2863,7 @@ bool gemm_pack_wanted(const GemmDesc &g, bool epilogue) {
   if (as_it_lies && g.sbk == 1) return false;
   if (gemm_dma_bkm_ok(t)) return epilogue;  // (the k-major form has no epilogue)
   // (both operands in 16-byte pieces already: gemm_bf16_nt_kernel reads them where they lie)
-  return epilogue || !gemm_fast_path(t, av, bv) || 2.0 * batch * g.M * g.N * g.K >= PACK_ALIGNED_MIN_FLOPS;
+  return epilogue || !gemm_fast_path(t, av, bv) || (g.M >= 64 && 2.0 * batch * g.M * g.N * g.K >= PACK_ALIGNED_MIN_FLOPS);
 }
 
 bool gemm_rope_epilogue_ok(const LaunchCtx &lc, const GemmDesc &g) {
@@ -2941,9 +2942,12 @@ uint32_t gemm_split_k(const LaunchCtx &lc, const GemmDesc &g) {
     while (tiles * splits <= (uint64_t)lc.n_cus && g.K / (splits * 2) >= 128 && splits < 16) splits *= 2;
     return splits;
   }
-  if (gemm_dma_ok(g) && g.M <= 64) {  // tiles of 64 x 64: a workgroup to every CU, four k-steps at least to each
+  if (gemm_dma_ok(g) && g.M <= 64) {
+    // Tiles of 64 x 64: a workgroup to every CU, four k-steps at least to each - and none below 16 k-steps, where the pass
+    // that sums the slices costs what they save (17 x 512 x 64 9.6 us in two slices, 5.5 in one; 17 x 768 x 256 9.8, 8.0; 40 x
+    // 1024 x 64 9.5, 10.8).
     const uint64_t t64 = (uint64_t)((g.N + 63) / 64) * batch;
-    while (t64 * splits * 2 <= (uint64_t)lc.n_cus && g.K / (splits * 2) >= 256 && splits < 8) splits *= 2;
+    while (g.K >= 1024 && t64 * splits * 2 <= (uint64_t)lc.n_cus && g.K / (splits * 2) >= 256 && splits < 8) splits *= 2;
     return g.N <= 64 && ((uint64_t)batch * g.M * g.N) % 4 ? 1 : splits;
   }
   // (a narrow product - the router of a MoE prefill, 1024 x 60 x 2048: 16 tiles of 64 x 64 walking all of k, 27 us -
@@ -3085,7 +3089,12 @@ hipError_t launch_matmul(const LaunchCtx &lc_in, const GemmDesc &g, const char *
         } else if (g.glu_gate || g.c16 || (g.act_sigmoid && splits == 1)) {
           e = launch_gemm_dma<64, 64, 2, 2, true, 8, false, false, false, 2>(lc, gg, (uint32_t)t64);
         } else {
-          e = launch_gemm_dma<64, 64, 2, 2, false, 8, false, false, false, 2>(lc, gg, (uint32_t)t64);
+          // (More tiles than CUs - batches of small products, or many columns -: two stages and several workgroups to a CU, one's
+          // tail under another's loads.  b x 17 x 64 x 512, 128 and 512 of them 12.3 -> 6.3 us, 42.5 -> 16.1; 128 x 17 x 1024 x
+          // 1024 64.7 -> 44.7; 512 x 33 x 128 x 128 14.3 -> 8.2; 40 x 2048 x 32000 28.9 -> 23.9; three stages 7.0, 18.8, 44.3, 9.2,
+          // 22.7.)
+          e = t64 > (uint64_t)lc.n_cus ? launch_gemm_dma<64, 64, 2, 2>(lc, gg, (uint32_t)t64)
+                                       : launch_gemm_dma<64, 64, 2, 2, false, 8, false, false, false, 2>(lc, gg, (uint32_t)t64);
         }
       } else if (g.dual_b) {  // gate and up stacked: 128 output columns per tile, 256 rows when that still fills the CUs
         if (g.n_group || g.glu_gate || splits != 1) return hipErrorInvalidValue;

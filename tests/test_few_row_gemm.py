@@ -49,3 +49,21 @@ def test_rotation_in_the_projections_launch_of_few_rows(oracle, hip_bf16, tokens
 @pytest.mark.parametrize("batch,tokens,heads", [(1, 40, 4), (3, 20, 4), (3, 41, 4), (1, 128, 4), (1, 101, 16)])
 def test_rotation_of_wide_heads_of_few_rows(oracle, hip_bf16, batch, tokens, heads):
     moe_tests.test_qwen_prefill_biases_and_rotation_in_the_projections_launch(oracle, hip_bf16, batch, tokens, heads, heads, 128)
+
+
+# more 64 x 64 tiles than the device has CUs: the form with two stages - one k-step, an odd number, many -, rows and columns
+# that end inside a tile; and on both sides of the depth from which a product of few tiles is split along k
+@pytest.mark.gpu
+@pytest.mark.parametrize("batch,rows,K,N", [(130, 17, 64, 130), (300, 64, 128, 64), (5, 33, 192, 4001), (1, 40, 320, 16500), (90, 63, 704, 200),
+                                            (1, 17, 960, 64), (1, 64, 1024, 64), (3, 40, 512, 136)])
+def test_many_small_products(hip_bf16, batch, rows, K, N):
+    g = np.random.default_rng(batch + rows)
+    x, w = (vectors.bf16_round(g.standard_normal(s).astype(np.float32)) for s in ((batch, rows, K), (batch, N, K)))
+
+    def f(b, x, w):
+        return [lang.matmul(b, x, lang.transpose(b, 1, 2, w))]
+    (got,) = vectors.run(hip_bf16, f, 1, x, w)
+    exact = x.astype(np.float64) @ w.astype(np.float64).transpose(0, 2, 1)
+    # (the operands are bf16 already: sums of K exact products in f32)
+    err = np.linalg.norm(got - exact, axis=-1) / np.linalg.norm(exact, axis=-1)
+    assert err.max() <= 4 * np.sqrt(K) * 2.0 ** -24, err.max()
