@@ -2938,8 +2938,12 @@ uint32_t gemm_split_k(const LaunchCtx &lc, const GemmDesc &g) {
     if (g.M <= 8 || g.b_index || !g.K) return 1;
     // (two workgroups to a CU, one's loads under the other's products: 700 x 2048 x 8192 357 -> 312 us, 400 x 2048 x 8192
     // 185 -> 168; four k-steps at least to each: 1000 x 1000 x 1000 54 -> 36, 100 x 2048 x 2048 33 -> 27; four workgroups
-    // to a CU were slower throughout)
-    while (tiles * splits <= (uint64_t)lc.n_cus && g.K / (splits * 2) >= 128 && splits < 16) splits *= 2;
+    // to a CU were slower throughout.  A shallow product does not pay for the second workgroup's slices, unless its sums are
+    // those of a few columns: 16 x 512 x 512 x 512 52.6 us in one slice, 61.4 in two, 16 x 200 x 512 x 512 36.8 in two, 39.2
+    // in four; 16 x 300 x 1000 x 300 108, 97; 16 x 700 x 520 x 7 50, 39)
+    while (tiles * splits <= (uint64_t)lc.n_cus && g.K / (splits * 2) >= 128 && splits < 16 &&
+           (tiles * splits * 2 <= (uint64_t)lc.n_cus || g.K >= 768 || g.N <= 64))
+      splits *= 2;
     return splits;
   }
   if (gemm_dma_ok(g) && g.M <= 64) {

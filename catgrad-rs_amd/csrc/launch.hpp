@@ -470,7 +470,9 @@ uint32_t gemv_pro_multi_row_max_k(int b_stype);
 // most input rows any several-row form takes
 enum { GEMV_PRO_MAX_ROWS = 16 };
 // bf16 mode: whether a product of this many rows belongs on the tile kernels.  From 17 rows on; from 9 at depths whose rows
-// do not fit the few-row kernel's LDS (12 rows against a 2048 x 2048 matrix: 25.7 us on what was left, 6.5 on tiles).  Not
+// do not fit the few-row kernel's LDS (12 rows against a 2048 x 2048 matrix: 25.7 us on what was left, 6.5 on tiles; the 9
+// rows of 2048 that do fit take 9.0 there against 14.2, their narrowing included, but a 9-token prompt, whose other fusions
+// go with the tiles, 2.03 ms against 1.21).  Not
 // the 5 to 8 rows of a depth that the few-row kernel does not take: the vector ALUs multiply those as f32, and tiles would
 // round them to bf16 (8 x 8192 x 2048: 26 us, 19 on tiles with the narrowing of the rows and the sum of the k-slices; as
 // three products of bf16 parts that add up to the f32 value, on tiles, no faster at 8 rows and slower at 5).
