@@ -837,7 +837,10 @@ int realize_matmul(cg_backend *be, cg_tensor *n, cg_tensor *addend, bool *added,
     probe.nb0 = nbo[0]; probe.nb1 = nbo[1];
     probe.sa_b0 = sao[0]; probe.sa_b1 = sao[1]; probe.sb_b0 = sbo[0]; probe.sb_b1 = sbo[1];
     probe.bf16_math = (be->flags & CG_FLAG_BF16) ? 1 : 0;
-    if (g.bf16_math && M >= 64 && N >= 64 && K % 64 == 0 && g.a_stype == ST_BF16 && g.sak == 1 && g.sbn == 1 &&
+    // (The 5 to 8 f32 rows of a deep product as well: the kernel that takes a k-major matrix for them reads it a few columns
+    // at a time, 8 x 4096 x 1024 354 us, 8 x 8192 x 2048 765.)
+    const bool few_deep = g.bf16_math && M > 4 && M <= 8 && K >= 4096 && K % 64 == 0 && g.a_stype == ST_F32 && g.b_stype == ST_BF16;
+    if (g.bf16_math && ((M >= 64 && K % 64 == 0 && g.a_stype == ST_BF16) || few_deep) && N >= 64 && g.sak == 1 && g.sbn == 1 &&
         g.sbk != 1 && !ex.w && (g.b_stype == ST_F32 || g.b_stype == ST_BF16) && !gemm_dma_bkm_ok(probe)) {
       // batches that only repeat (stride 0) are transposed once
       const uint32_t tb0 = g.sb_b0 ? g.nb0 : 1, tb1 = g.sb_b1 ? g.nb1 : 1;

@@ -38,6 +38,11 @@ def test_few_rows_of_a_deep_product(hip_bf16, rows, K, N):
     exact = x.reshape(rows, K).astype(np.float64) @ w.astype(np.float64).T
     assert_f32_sums(exact, got, K, f"{rows} x {K} x {N}")
 
+    def k_major(b, x, w):
+        return [lang.matmul(b, lang.reshape(b, lang.make_shape(b, rows, K), x), w)]
+    (got,) = vectors.run(hip_bf16, k_major, 1, x, np.ascontiguousarray(w.T))
+    assert_f32_sums(exact, got, K, f"{rows} x {K} x {N}, k-major")
+
 
 @pytest.mark.gpu
 def test_few_rows_of_a_deep_product_with_a_residual_and_special_values(hip_bf16):
