@@ -82,9 +82,6 @@ class LaunchQueue {
     while (tail_.load(std::memory_order_acquire) < h) pause();
   }
 
-  // Whether the thread sleeps with nothing to do (for the thread that calls launch()).
-  bool asleep() const { return sleeping_.load() && head_.load(std::memory_order_relaxed) == tail_.load(std::memory_order_acquire); }
-
   // First error a launch reported since the last call (hipSuccess if none).
   hipError_t take_error() { return (hipError_t)error_.exchange((int)hipSuccess, std::memory_order_acq_rel); }
 

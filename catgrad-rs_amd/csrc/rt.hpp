@@ -215,13 +215,6 @@ struct cg_backend {
   // kernel launches go through this thread's queue; null when the backend launches inline (CG_FLAG_EAGER)
   cgk::LaunchQueue *queue = nullptr;
   cgk::LaunchCtx lc() const { return cgk::LaunchCtx{stream, n_cus, d_words, cur_start, cur_stop, queue}; }
-  // for a copy to or from the host: made by the caller when the queue's thread sleeps (nothing is queued before it), which
-  // is not worth waking for one launch (64 KB up and a wait, after 5 ms of rest: 55 us through the thread, 34 so)
-  cgk::LaunchCtx copy_lc() const {
-    cgk::LaunchCtx c = lc();
-    if (queue && queue->asleep()) c.queue = nullptr;
-    return c;
-  }
   // the stream, once every launch handed to the queue has reached it: what anything but a kernel launch
   // (copies, events, synchronisation, frees) must use to keep program order
   hipStream_t ordered_stream() const {

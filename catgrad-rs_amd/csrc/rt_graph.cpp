@@ -267,7 +267,7 @@ int wait_host_flag(cg_backend *be, const uint32_t *flag) {
 // wait for the stream and surface device-side error flags
 int sync_and_check(cg_backend *be) {
   be->h_words[2] = HOST_FLAG_PENDING;
-  HIPCHK(be, launch_to_host(be->copy_lc(), nullptr, nullptr, 0, be->d_words, be->h_words, be->d_words + 4));
+  HIPCHK(be, launch_to_host(be->lc(), nullptr, nullptr, 0, be->d_words, be->h_words, be->d_words + 4));
   TRY(wait_host_flag(be, be->h_words + 2));
   return check_error_words(be, be->h_words);
 }
@@ -591,7 +591,9 @@ int upload(cg_backend *be, const void *data, size_t n, const int64_t *shape, int
   if (!narrow && n * 4 <= HOST_IN_BYTES - 64 && be->queue) {
     // A prompt's token ids, a small vector: through a slot of pinned memory, without a wait.  One workgroup takes it, up to
     // the whole slot: until the values are there, and a wait for that, 1 KB 14 us, 64 KB 20, where a copy by the runtime
-    // takes 28 at either size; after 5 ms of rest 29 and 34 against 46 and 48.
+    // takes 28 at either size.  (After a rest, the launch thread asleep, 50 and 55 against 46 and 48; launching from the
+    // caller then, 29 and 34, only moves the thread's waking into the pass that follows: 37 tokens uploaded and run 1.36 ms
+    // either way.)
     const size_t tail = HOST_IN_BYTES - 64;
     if (!be->h_in) {
       e = hipHostMalloc((void **)&be->h_in, HOST_IN_BYTES * HOST_IN_SLOTS, hipHostMallocDefault);
@@ -609,7 +611,7 @@ int upload(cg_backend *be, const void *data, size_t n, const int64_t *shape, int
       }
       std::memcpy(slot, data, n * 4);
       *flag = HOST_FLAG_PENDING;
-      e = launch_from_host(be->copy_lc(), slot, t->st->ptr, (uint32_t)n, flag);
+      e = launch_from_host(be->lc(), slot, t->st->ptr, (uint32_t)n, flag);
       if (e != hipSuccess) *flag = HOST_FLAG_DONE;
       else be->h_in_next = (be->h_in_next + 1) % HOST_IN_SLOTS;
     }
@@ -672,7 +674,7 @@ static int download_through_halves(cg_backend *be, const char *src, char *dst, s
   auto ask = [&](size_t first) -> int {  // for the pieces from `first` that fill one half
     for (size_t i = first; i < std::min(pieces, first + TO_HOST_MAX_PIECES); ++i) words(i)[2] = HOST_FLAG_PENDING;
     const size_t len = std::min(half, bytes - first * piece);
-    HIPCHK(be, launch_to_host(be->copy_lc(), src + first * piece, data(first), len / 4, be->d_words, words(first), be->d_words + 4));
+    HIPCHK(be, launch_to_host(be->lc(), src + first * piece, data(first), len / 4, be->d_words, words(first), be->d_words + 4));
     return CG_OK;
   };
   for (size_t i = 0; i < 2 * TO_HOST_MAX_PIECES && i < pieces; i += TO_HOST_MAX_PIECES) TRY(ask(i));
