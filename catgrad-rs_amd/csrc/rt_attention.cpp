@@ -30,7 +30,11 @@ int try_attn_prefill(cg_backend *be, cg_tensor *n, bool *done) {
   // f32 products of a middling number of keys: the pass walks them one tile after the other with too few workgroups to
   // cover for it (1 x 32 heads x 200 x 200: 37 us), GEMM + softmax + GEMM take 31; at 50 keys it is 13 us against 21,
   // at 700 95 against 155.  bf16: one pass at every length (37 keys: 10 us against 45; 2900: 202 against 1130).
-  if (f32 && T > 128 && T < 512 && !(be->flags & CG_FLAG_ATTN_ONE_PASS)) return CG_OK;
+  // Heads of 256 in f32 hold 64 queries to a workgroup and 32 keys to a step, one wave to a SIMD: behind at every length, until
+  // the scores themselves are what to avoid (Gemma-3 shape, whole prompts: 16 tokens 4.74 ms so, 4.59 in three launches; 128
+  // 8.0, 6.7; 512 18.0, 13.1; 777 24.8, 19.9; 4 x 1000, scores of 64 MB, 77.6, 75.3).
+  const bool three = d == 256 ? nb * heads * Sq * T < ((int64_t)64 << 20) / 4 : T > 128 && T < 512;
+  if (f32 && three && !(be->flags & CG_FLAG_ATTN_ONE_PASS)) return CG_OK;
   if (nb > 65535 || heads > 65535) return CG_OK;
   cg_tensor *q = S->in[0];
   // queries and keys both still to be rotated: one launch for the two (each alone otherwise, below)

@@ -75,9 +75,10 @@ enum {
   /* keep deferring, but never dispatch to the hand-written pattern kernels (softmax, RMSNorm,
    * RoPE, gated activations): everything goes through the generic fused-program kernels */
   CG_FLAG_NO_PATTERNS = 4u,
-  /* use the one-pass attention kernels over several query rows for every number of keys (by default not for 129 to 511
-   * keys without CG_FLAG_BF16, where two products and a softmax are ahead; with CG_FLAG_BF16 they run from 9 queries on at
-   * every number of keys, flag or no flag); bf16 or f32 products, as CG_FLAG_BF16 says */
+  /* use the one-pass attention kernels over several query rows for every number of keys (by default, without CG_FLAG_BF16,
+   * neither for 129 to 511 keys nor for heads of 256 with scores under 64 MB, where two products and a softmax are ahead;
+   * with CG_FLAG_BF16 they run from 9 queries on at every number of keys, flag or no flag); bf16 or f32 products, as
+   * CG_FLAG_BF16 says */
   CG_FLAG_ATTN_ONE_PASS = 8u
 };
 

@@ -46,7 +46,7 @@ def test_attention_of_any_length(oracle, hip, hip_bf16, H, KV, S, d, window):
         be.launch_counts(reset=True)
         (got,) = vectors.run(be, f, 1, q, k, v)
         counts = be.launch_counts(reset=True)
-        three = 128 < S < 512 if be is hip else S <= 8      # (two products and a softmax at these lengths)
+        three = 128 < S < 512 or d == 256 if be is hip else S <= 8      # (two products and a softmax at these lengths)
         assert counts.get("attn_prefill", 0) == (0 if three else 1), counts
         check(ref, got, f"attention over {S} keys")
 
