@@ -25,11 +25,6 @@ namespace cgk {
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 typedef __attribute__((ext_vector_type(16))) float f32x16;
 
-__device__ __forceinline__ uint32_t bf16_rne(float f) {
-  uint32_t u = __float_as_uint(f);
-  if ((u & 0x7FFFFFFFu) > 0x7F800000u) return (u >> 16) | 0x40u;
-  return (u + 0x7FFFu + ((u >> 16) & 1u)) >> 16;
-}
 __device__ __forceinline__ float widen(float v) { return v; }
 __device__ __forceinline__ float widen(uint16_t v) { return __uint_as_float((uint32_t)v << 16); }
 
@@ -165,10 +160,10 @@ __global__ void __launch_bounds__(256) gemm_kernel(GemmDesc g, int a_vec, int b_
       LT *d = S + row * LD + kc;
       if (BF16) {
         uint4 q;
-        q.x = bf16_rne(v[0]) | (bf16_rne(v[1]) << 16);
-        q.y = bf16_rne(v[2]) | (bf16_rne(v[3]) << 16);
-        q.z = bf16_rne(v[4]) | (bf16_rne(v[5]) << 16);
-        q.w = bf16_rne(v[6]) | (bf16_rne(v[7]) << 16);
+        q.x = bf16_pack2(v[0], v[1]);
+        q.y = bf16_pack2(v[2], v[3]);
+        q.z = bf16_pack2(v[4], v[5]);
+        q.w = bf16_pack2(v[6], v[7]);
         *(uint4 *)d = q;
       } else {
         *(float2 *)d = make_float2(v[0], v[1]);
@@ -180,7 +175,7 @@ __global__ void __launch_bounds__(256) gemm_kernel(GemmDesc g, int a_vec, int b_
       const int kk = chunk / (rows_total / 8), rc = (chunk % (rows_total / 8)) * 8;
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
-        if (BF16) S[(rc + j) * LD + kk] = (LT)bf16_rne(v[j]);
+        if (BF16) S[(rc + j) * LD + kk] = (LT)bf16_bits(v[j]);
         else S[(rc + j) * LD + kk] = (LT)v[j];
       }
     }
@@ -1027,8 +1022,8 @@ __global__ void __launch_bounds__(256) transpose_cast_bf16_kernel(const TB *b, u
       if (k < K && n < N) {
         if (sizeof(TB) == 4) {
           const float4 q = *(const float4 *)((const float *)src + (int64_t)k * sbk + n);
-          v[0] = (uint16_t)bf16_rne(q.x); v[1] = (uint16_t)bf16_rne(q.y);
-          v[2] = (uint16_t)bf16_rne(q.z); v[3] = (uint16_t)bf16_rne(q.w);
+          v[0] = (uint16_t)bf16_bits(q.x); v[1] = (uint16_t)bf16_bits(q.y);
+          v[2] = (uint16_t)bf16_bits(q.z); v[3] = (uint16_t)bf16_bits(q.w);
         } else {
           const uint2 q = *(const uint2 *)((const uint16_t *)src + (int64_t)k * sbk + n);
           v[0] = (uint16_t)q.x; v[1] = (uint16_t)(q.x >> 16); v[2] = (uint16_t)q.y; v[3] = (uint16_t)(q.y >> 16);
@@ -1038,7 +1033,7 @@ __global__ void __launch_bounds__(256) transpose_cast_bf16_kernel(const TB *b, u
 #pragma unroll
       for (int j = 0; j < 4; ++j)
         if (k < K && n + j < N) {
-          if (sizeof(TB) == 4) v[j] = (uint16_t)bf16_rne(widen(src[(int64_t)k * sbk + n + j]));
+          if (sizeof(TB) == 4) v[j] = (uint16_t)bf16_bits(widen(src[(int64_t)k * sbk + n + j]));
           else v[j] = (uint16_t)src[(int64_t)k * sbk + n + j];
         }
     }
@@ -3105,17 +3100,18 @@ hipError_t launch_matmul(const LaunchCtx &lc_in, const GemmDesc &g, const char *
         const uint64_t d256 = (uint64_t)((g.M + 255) / 256) * ((g.N + 127) / 128) * batch;
         const uint64_t d128 = (uint64_t)((g.M + 127) / 128) * ((g.N + 127) / 128) * batch;
         // (fewer tiles of 128 than half the CUs: 64 or 32 output columns per tile)
-        if (d256 >= (uint64_t)lc.n_cus) e = launch_gemm_dma<256, 256, 2, 4, true, 2, true>(lc, gg, (uint32_t)d256);
+        if (d256 >= (uint64_t)lc.n_cus && gemm_ring_ok(gg)) e = launch_gemm_ring(lc, gg);
         else if (d128 * 4 <= (uint64_t)lc.n_cus)
           e = launch_gemm_dma<128, 64, 4, 1, true, 5, true, false, false, 2>(lc, gg, (uint32_t)((uint64_t)((g.M + 127) / 128) * ((g.N + 31) / 32) * batch));
         else if (d128 * 2 <= (uint64_t)lc.n_cus)
           e = launch_gemm_dma<128, 128, 4, 2, true, 4, true>(lc, gg, (uint32_t)((uint64_t)((g.M + 127) / 128) * ((g.N + 63) / 64) * batch));
         else e = launch_gemm_dma<128, 256, 2, 4, true, 3, true>(lc, gg, (uint32_t)d128);
       } else if (g.glu_gate || g.c16 || (g.act_sigmoid && splits == 1)) {
-        if (g.act_sigmoid && t256 >= (uint64_t)lc.n_cus) e = launch_gemm_dma<256, 256, 2, 4, true, 2>(lc, gg, (uint32_t)t256);
+        if (g.act_sigmoid && t256 >= (uint64_t)lc.n_cus && gemm_ring_ok(gg)) e = launch_gemm_ring(lc, gg);
+        else if (g.act_sigmoid && t256 >= (uint64_t)lc.n_cus) e = launch_gemm_dma<256, 256, 2, 4, true, 2>(lc, gg, (uint32_t)t256);
         else if (deep) e = launch_gemm_dma<128, 128, 2, 4, true, 4>(lc, gg, (uint32_t)t128);
         else e = launch_gemm_dma<128, 128, 2, 2, true, 2>(lc, gg, (uint32_t)t128);
-      } else if (t256 >= (uint64_t)lc.n_cus && grp256) {
+      } else if (t256 >= (uint64_t)lc.n_cus && grp256 && gemm_ring_ok(gg)) {
         // 256 x 256 tiles run one to a CU, 128 x 128 two to a CU: when the big tiles leave the last round of
         // workgroups mostly empty (320 tiles on 256 CUs), the small ones fill the machine better
         auto fill = [&](uint64_t tiles, uint64_t slots) { return (double)tiles / (double)((tiles + slots - 1) / slots * slots); };
@@ -3135,7 +3131,7 @@ hipError_t launch_matmul(const LaunchCtx &lc_in, const GemmDesc &g, const char *
           LaunchCtx first = lc, second = lc_in;
           first.ev_stop = nullptr;
           second.ev_start = nullptr;
-          e = launch_gemm_dma<256, 256, 2, 4>(first, lead, (uint32_t)(lead_m * tiles_n));
+          e = launch_gemm_ring(first, lead);
           if (e != hipSuccess) return e;
           return launch_matmul(second, rest, nullptr);
         }
@@ -3143,7 +3139,7 @@ hipError_t launch_matmul(const LaunchCtx &lc_in, const GemmDesc &g, const char *
           e = g.K < 2048 ? launch_gemm_dma<128, 128, 2, 4, false, 2>(lc, gg, (uint32_t)t128)  // (as below)
                          : launch_gemm_dma<128, 128, 2, 2>(lc, gg, (uint32_t)t128);
         else
-          e = launch_gemm_dma<256, 256, 2, 4>(lc, gg, (uint32_t)t256);
+          e = launch_gemm_ring(lc, gg);
       } else if (splits == 1 && t128 * 2 <= (uint64_t)lc.n_cus && g.N >= 128) {
         // too few 128 x 128 tiles for the CUs and no split-K to multiply them: halve the tile
         const uint32_t t64 = (uint32_t)((uint64_t)((g.M + 127) / 128) * ((g.N + 63) / 64) * batch);

@@ -1,0 +1,382 @@
+// k_gemm_ring.hip — the bf16 NT product of large problems: 256 x 256 tiles, four wavefronts, one per SIMD.
+//
+// C[m, n] = sum_k A[m, k] B[n, k], both operands bf16 with unit stride along k, K a multiple of 64 and at least 128
+// (Backend::matmul, mod.rs:41; ndarray.rs:549-615).
+//
+// What bounds it: the matrix cores, if nothing else of a k-step of 64 takes longer than its 2048 cycles of MFMAs (64 per
+// wavefront, 32 cycles each).  A wavefront owns 128 x 128 of the tile, so a k-step reads 128 KB of fragments out of LDS
+// and writes 64 KB into it (eight wavefronts of 128 x 64 read 192 KB, all that the LDS delivers in that time), and the
+// CU takes in 64 KB through its one load path of 64 bytes a cycle: 1024 cycles, if the loads are spread evenly.  Issued
+// in one burst at the top of a step - which is what a compiler makes of them, since it moves nothing across their inline
+// assembly - each of them costs its wave 55 to 120 cycles, in which no MFMA is issued.  So the whole main loop is one
+// statement of assembly with a fixed place for everything:
+//   * The tile is four quadrants of 128 x 128, (A half, B half) = (0,0) (0,1) (1,1) (1,0), a phase each; in a quadrant a
+//     wavefront owns 64 x 64, and a phase is 16 MFMAs in four k-slices.
+//   * A unit is half an operand's tile: 128 rows x 128 bytes.  A stage is four units, LDS holds two.  Every phase reads
+//     the fragments of one unit (8 reads) for the phases after it, and requests the same unit of the step after the
+//     next (4 loads of 1 KB by each wavefront), into the place whose last reader was two phases ago.  A load has six
+//     phases, 3072 cycles, to arrive, and there is no point at which everything is waited for.
+//   * One barrier a phase: before it a wavefront has seen its own loads of the unit about to be read (a count) and the
+//     reads of two phases ago (a count); so behind it the unit is there for everyone, and its predecessor's place free.
+// The products of an element are added in the order of k, as in gemm_bf16_dma_kernel: the same bits.
+// Measured against 256 x 256 tiles with eight wavefronts whose loads a compiler placed, on the same box: 16384 x 1152 by 2 x 6912
+// gate and up 531 -> 464 us, 2900 x 2048 by 2 x 8192 184 -> 161; 13056 x 6912 x 1152 203 -> 177, 16384 x 1152 x 1536 77 -> 67
+// (100 MB of result); 6000 x 1024 x 4100 with a sigmoid 77 -> 64.  What is left is power: 8192 cubed takes 1.40 us a step on
+// random operands (1.35 PFLOP/s) and 0.99 on zeros (1.96), with the same loads.  Around the loop a tile takes 0.8 us to set up,
+// 1.1 for its first loads and 5.3 to store.
+#include <hip/hip_runtime.h>
+#include "launch.hpp"
+#include "dev_common.hpp"
+
+namespace cgk {
+
+typedef __attribute__((ext_vector_type(16))) float f32x16;
+
+// ---- the main loop, in pieces -------------------------------------------------------------------------
+// Fragments live in v[128:255]: (half U, 32-row block r, k-slice ks) as below.  s[40:41] points at A, s[42:43] and s[44:45]
+// at the two halves of B, at the step being requested; s46 is this wavefront's place in the stage being requested, s47
+// counts steps.  M0 (a load's place in LDS) is set an instruction ahead of the load.
+#define FR_A0_0_0 "v[128:131]"
+#define FR_A0_0_1 "v[132:135]"
+#define FR_A0_0_2 "v[136:139]"
+#define FR_A0_0_3 "v[140:143]"
+#define FR_A0_1_0 "v[144:147]"
+#define FR_A0_1_1 "v[148:151]"
+#define FR_A0_1_2 "v[152:155]"
+#define FR_A0_1_3 "v[156:159]"
+#define FR_A1_0_0 "v[160:163]"
+#define FR_A1_0_1 "v[164:167]"
+#define FR_A1_0_2 "v[168:171]"
+#define FR_A1_0_3 "v[172:175]"
+#define FR_A1_1_0 "v[176:179]"
+#define FR_A1_1_1 "v[180:183]"
+#define FR_A1_1_2 "v[184:187]"
+#define FR_A1_1_3 "v[188:191]"
+#define FR_B0_0_0 "v[192:195]"
+#define FR_B0_0_1 "v[196:199]"
+#define FR_B0_0_2 "v[200:203]"
+#define FR_B0_0_3 "v[204:207]"
+#define FR_B0_1_0 "v[208:211]"
+#define FR_B0_1_1 "v[212:215]"
+#define FR_B0_1_2 "v[216:219]"
+#define FR_B0_1_3 "v[220:223]"
+#define FR_B1_0_0 "v[224:227]"
+#define FR_B1_0_1 "v[228:231]"
+#define FR_B1_0_2 "v[232:235]"
+#define FR_B1_0_3 "v[236:239]"
+#define FR_B1_1_0 "v[240:243]"
+#define FR_B1_1_1 "v[244:247]"
+#define FR_B1_1_2 "v[248:251]"
+#define FR_B1_1_3 "v[252:255]"
+// byte offset of a 32-row block of a unit in its stage
+#define AT_A0_0 "0"
+#define AT_A0_1 "4096"
+#define AT_B0_0 "16384"
+#define AT_B0_1 "20480"
+#define AT_B1_0 "32768"
+#define AT_B1_1 "36864"
+#define AT_A1_0 "49152"
+#define AT_A1_1 "53248"
+#define BASE_A0(ks) "%[ra" #ks "]"
+#define BASE_A1(ks) "%[ra" #ks "]"
+#define BASE_B0(ks) "%[rb" #ks "]"
+#define BASE_B1(ks) "%[rb" #ks "]"
+#define RD(U, r, ks) "ds_read_b128 " FR_##U##_##r##_##ks ", " BASE_##U(ks) " offset:" AT_##U##_##r "\n\t"
+#define RD_UNIT(U) RD(U, 0, 0) RD(U, 1, 0) RD(U, 0, 1) RD(U, 1, 1) RD(U, 0, 2) RD(U, 1, 2) RD(U, 0, 3) RD(U, 1, 3)
+#define PTR_A0 "s[40:41]"
+#define PTR_A1 "s[40:41]"
+#define PTR_B0 "s[42:43]"
+#define PTR_B1 "s[44:45]"
+// piece i (1 KB, eight rows) of unit U
+#define M0_A0(i) "s_add_u32 m0, s46, " #i "*1024\n\t"
+#define M0_B0(i) "s_add_u32 m0, s46, 16384+" #i "*1024\n\t"
+#define M0_B1(i) "s_add_u32 m0, s46, 32768+" #i "*1024\n\t"
+#define M0_A1(i) "s_add_u32 m0, s46, 49152+" #i "*1024\n\t"
+#define LOAD(U, i) "global_load_lds_dwordx4 %[d" #U #i "], " PTR_##U "\n\t"
+#define LOAD_UNIT(U)                                                                                              \
+  M0_##U(0) "s_nop 0\n\t" LOAD(U, 0) M0_##U(1) "s_nop 0\n\t" LOAD(U, 1) M0_##U(2) "s_nop 0\n\t" LOAD(U, 2) M0_##U(3) \
+  "s_nop 0\n\t" LOAD(U, 3)
+#define NEXT_STEP                                                                                              \
+  "s_add_u32 s40, s40, 128\n\ts_addc_u32 s41, s41, 0\n\ts_add_u32 s42, s42, 128\n\ts_addc_u32 s43, s43, 0\n\t" \
+  "s_add_u32 s44, s44, 128\n\ts_addc_u32 s45, s45, 0\n\t"
+#define OTHER_STAGE_LOADS "s_xor_b32 s46, s46, 0x10000\n\t"
+#define OTHER_STAGE_A                                                                        \
+  "v_xor_b32 %[ra0], 0x10000, %[ra0]\n\tv_xor_b32 %[ra1], 0x10000, %[ra1]\n\t" \
+  "v_xor_b32 %[ra2], 0x10000, %[ra2]\n\tv_xor_b32 %[ra3], 0x10000, %[ra3]\n\t"
+#define OTHER_STAGE_B                                                                        \
+  "v_xor_b32 %[rb0], 0x10000, %[rb0]\n\tv_xor_b32 %[rb1], 0x10000, %[rb1]\n\t" \
+  "v_xor_b32 %[rb2], 0x10000, %[rb2]\n\tv_xor_b32 %[rb3], 0x10000, %[rb3]\n\t"
+#define POINTERS "s_mov_b64 s[40:41], %[pa]\n\ts_mov_b64 s[42:43], %[pb0]\n\ts_mov_b64 s[44:45], %[pb1]\n\ts_mov_b32 s46, %[lds]\n\t"
+// products of row block i of A half a with row block j of B half b.  The operands in this order leave the tile transposed: a
+// lane holds four consecutive columns of a row of C.
+#define PRODUCT(a, b, i, j, UA, UB, ks)                                                                                \
+  "v_mfma_f32_32x32x16_bf16 %[c" #a #b #i #j "], " FR_##UB##_##j##_##ks ", " FR_##UA##_##i##_##ks ", %[c" #a #b #i #j \
+  "]\n\t"
+#define NONE ""
+#define READS_BUT(n) "s_waitcnt lgkmcnt(" #n ")\n\t"
+// a k-slice: its fragments (all but the six youngest reads are there), four products, two reads and one load among them
+#define SLICE(a, b, UA, UB, ks, W, R1, M0, R2, L) \
+  W PRODUCT(a, b, 0, 0, UA, UB, ks) R1 PRODUCT(a, b, 0, 1, UA, UB, ks) R2 M0 PRODUCT(a, b, 1, 0, UA, UB, ks) L PRODUCT(a, b, 1, 1, UA, UB, ks)
+#define SYNC(v) "s_waitcnt vmcnt(" #v ") lgkmcnt(8)\n\ts_barrier\n\t"
+#define ON_M(U, i) M0_##U(i)
+#define ON_L(U, i) LOAD(U, i)
+#define OFF_M(U, i) ""
+#define OFF_L(U, i) ""
+// G: ON while there is a step after the next to request.  v: this wavefront's loads that may still be under way.
+#define PHASE0(G, v)                                                                            \
+  SYNC(v)                                                                                           \
+  SLICE(0, 0, A0, B0, 0, READS_BUT(6), RD(B1, 0, 0), G##_M(A0, 0), RD(B1, 1, 0), G##_L(A0, 0))  \
+  SLICE(0, 0, A0, B0, 1, READS_BUT(6), RD(B1, 0, 1), G##_M(A0, 1), RD(B1, 1, 1), G##_L(A0, 1))  \
+  SLICE(0, 0, A0, B0, 2, READS_BUT(6), RD(B1, 0, 2), G##_M(A0, 2), RD(B1, 1, 2), G##_L(A0, 2))  \
+  SLICE(0, 0, A0, B0, 3, READS_BUT(6), RD(B1, 0, 3), G##_M(A0, 3), RD(B1, 1, 3), G##_L(A0, 3))
+#define PHASE1(G, v)                                                                                           \
+  SYNC(v)                                                                                                          \
+  SLICE(0, 1, A0, B1, 0, READS_BUT(6), RD(A1, 0, 0), G##_M(B0, 0), RD(A1, 1, 0), G##_L(B0, 0))                 \
+  SLICE(0, 1, A0, B1, 1, READS_BUT(6), RD(A1, 0, 1), G##_M(B0, 1), RD(A1, 1, 1), G##_L(B0, 1))                 \
+  SLICE(0, 1, A0, B1, 2, READS_BUT(6), RD(A1, 0, 2), G##_M(B0, 2), RD(A1, 1, 2) OTHER_STAGE_B, G##_L(B0, 2))   \
+  SLICE(0, 1, A0, B1, 3, READS_BUT(6), RD(A1, 0, 3), G##_M(B0, 3), RD(A1, 1, 3) OTHER_STAGE_A, G##_L(B0, 3))
+#define PHASE2(G, v)                                                                            \
+  SYNC(v)                                                                                           \
+  SLICE(1, 1, A1, B1, 0, READS_BUT(6), RD(A0, 0, 0), G##_M(B1, 0), RD(A0, 1, 0), G##_L(B1, 0))  \
+  SLICE(1, 1, A1, B1, 1, READS_BUT(6), RD(A0, 0, 1), G##_M(B1, 1), RD(A0, 1, 1), G##_L(B1, 1))  \
+  SLICE(1, 1, A1, B1, 2, READS_BUT(6), RD(A0, 0, 2), G##_M(B1, 2), RD(A0, 1, 2), G##_L(B1, 2))  \
+  SLICE(1, 1, A1, B1, 3, READS_BUT(6), RD(A0, 0, 3), G##_M(B1, 3), RD(A0, 1, 3), G##_L(B1, 3))
+// (these reads replace fragments of this phase: each comes behind the products that use what it replaces)
+#define PHASE3(G, v)                                                                                  \
+  SYNC(v)                                                                                                 \
+  SLICE(1, 0, A1, B0, 0, NONE, NONE, G##_M(A1, 0), NONE, G##_L(A1, 0))                                \
+  SLICE(1, 0, A1, B0, 1, NONE, RD(B0, 0, 0), G##_M(A1, 1), RD(B0, 1, 0), G##_L(A1, 1))                \
+  SLICE(1, 0, A1, B0, 2, NONE, RD(B0, 0, 1), G##_M(A1, 2), RD(B0, 1, 1), G##_L(A1, 2))                \
+  SLICE(1, 0, A1, B0, 3, NONE, RD(B0, 0, 2), G##_M(A1, 3), RD(B0, 1, 2), G##_L(A1, 3)) RD(B0, 0, 3)   \
+  RD(B0, 1, 3)
+// the last step has nothing further to read in its second half
+#define LAST_HALF                                                            \
+  SLICE(1, 1, A1, B1, 0, READS_BUT(6), NONE, NONE, NONE, NONE)               \
+  SLICE(1, 1, A1, B1, 1, READS_BUT(4), NONE, NONE, NONE, NONE)               \
+  SLICE(1, 1, A1, B1, 2, READS_BUT(2), NONE, NONE, NONE, NONE)               \
+  SLICE(1, 1, A1, B1, 3, READS_BUT(0), NONE, NONE, NONE, NONE)               \
+  SLICE(1, 0, A1, B0, 0, NONE, NONE, NONE, NONE, NONE)                       \
+  SLICE(1, 0, A1, B0, 1, NONE, NONE, NONE, NONE, NONE)                       \
+  SLICE(1, 0, A1, B0, 2, NONE, NONE, NONE, NONE, NONE)                       \
+  SLICE(1, 0, A1, B0, 3, NONE, NONE, NONE, NONE, NONE)
+// steps 0 and 1 requested: 32 loads
+#define FIRST_LOADS                                                                                                   \
+  POINTERS LOAD_UNIT(A0) LOAD_UNIT(B0) LOAD_UNIT(B1) LOAD_UNIT(A1) NEXT_STEP OTHER_STAGE_LOADS LOAD_UNIT(A0) LOAD_UNIT(B0) \
+  LOAD_UNIT(B1) LOAD_UNIT(A1)
+// all n >= 2 steps (the nops: nothing behind this statement may read the accumulators before the last product is done)
+#define MAIN_LOOP                                                                                                    \
+  POINTERS NEXT_STEP NEXT_STEP "s_sub_u32 s47, %[n], 2\n\t"                                                              \
+  "s_waitcnt vmcnt(24)\n\ts_barrier\n\t" RD_UNIT(A0) RD_UNIT(B0)                                                         \
+  "s_cmp_eq_u32 s47, 0\n\ts_cbranch_scc1 2f\n\t"                                                                         \
+  "1:\n\t" PHASE0(ON, 20) PHASE1(ON, 20) PHASE2(ON, 20) PHASE3(ON, 20) NEXT_STEP OTHER_STAGE_LOADS       \
+  "s_sub_u32 s47, s47, 1\n\ts_cmp_lg_u32 s47, 0\n\ts_cbranch_scc1 1b\n\t"                                                \
+  "2:\n\t" PHASE0(OFF, 20) PHASE1(OFF, 16) PHASE2(OFF, 12) PHASE3(OFF, 8) PHASE0(OFF, 4)             \
+  PHASE1(OFF, 0) LAST_HALF "s_nop 15\n\ts_nop 7\n\t"
+
+// RING_PLAIN: C (f32) straight from the accumulators, with the biases of grouped products.  RING_SIGMOID: sigmoid(A . B)
+// as the next product's operand, whole rows of c16_pitch bf16 values with zeros past the last column.  RING_SILU, RING_GELU: half the tile's B rows are gate_proj's, half up_proj's;
+// act(gate) * up, 128 columns a tile, as bf16.  (GemmDesc says what each field means.)
+enum { RING_PLAIN, RING_SIGMOID, RING_SILU, RING_GELU };
+template <int KIND>
+__global__ void __launch_bounds__(256, 1) gemm_bf16_ring_kernel(GemmDesc g) {
+  constexpr bool GATED = KIND == RING_SILU || KIND == RING_GELU;
+  constexpr uint32_t BNO = GATED ? 128 : 256;  // output columns of a tile
+  warm_kernel_arguments<sizeof(GemmDesc)>();
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), wm = wave >> 1, wn = wave & 1;
+  const uint32_t tiles_m = (g.M + 255) / 256, tiles_n = (g.N + BNO - 1) / BNO;
+  const uint32_t per_batch = tiles_m * tiles_n, batch = g.nb0 * g.nb1;
+  // every XCD a contiguous range of tiles, in groups of four tile rows: as in gemm_bf16_dma_kernel
+  uint32_t id = blockIdx.x;
+  if (gridDim.x % 8 == 0) id = (id % 8) * (gridDim.x / 8) + id / 8;
+  const uint32_t zz = id / per_batch, t = id - zz * per_batch;
+  const uint32_t split = zz / batch, bz = zz - split * batch;
+  const uint32_t b0 = bz / g.nb1, b1 = bz - b0 * g.nb1;
+  constexpr uint32_t GM = 4;
+  const uint32_t first_m = t / (GM * tiles_n) * GM, gsz = min(tiles_m - first_m, GM);
+  const uint32_t tg = t % (GM * tiles_n);
+  const uint32_t m0 = (first_m + tg % gsz) * 256;
+  uint32_t n0 = tg / gsz * BNO, Nl = g.N;
+  const uint16_t *B = (const uint16_t *)g.b + b0 * g.sb_b0 + b1 * g.sb_b1;
+  float *C = (g.splits > 1 ? g.workspace + (uint64_t)split * batch * g.M * g.N : g.c) + (uint64_t)bz * g.M * g.N;
+  const float *Bias = nullptr;
+  if (KIND == RING_PLAIN && g.n_group) {  // grouped products: tiles never straddle two
+    uint32_t p = 0;
+    while (p + 1 < g.n_group && n0 >= g.grp_n[p]) {
+      n0 -= g.grp_n[p];
+      ++p;
+    }
+    B = (const uint16_t *)g.grp_b[p];
+    C = g.grp_c[p];
+    Nl = g.grp_n[p];
+    Bias = g.grp_bias[p];
+  }
+  const uint32_t k_begin = split * g.k_per_split, k_end = min(g.K, k_begin + g.k_per_split);
+  const uint32_t n_steps = __builtin_amdgcn_readfirstlane((k_end - k_begin) / 64);
+  // Where this lane's piece of each load comes from: byte offsets from the tile's first row (rows past the end repeat the last
+  // one), the 16-byte chunk swizzled so that the fragment reads are free of bank conflicts.
+  const uint16_t *pa = (const uint16_t *)g.a + b0 * g.sa_b0 + b1 * g.sa_b1 + (int64_t)m0 * g.sam + k_begin;
+  const uint16_t *pb0 = B + (int64_t)n0 * g.sbn + k_begin;
+  const uint16_t *pb1 = GATED ? (const uint16_t *)g.dual_b + b0 * g.sb_b0 + b1 * g.sb_b1 + (int64_t)n0 * g.sbn + k_begin : pb0;
+  const uint32_t sa = (uint32_t)g.sam * 2, sb = (uint32_t)g.sbn * 2, last_a = g.M - 1 - m0, last_b = Nl - 1 - n0;
+  uint32_t dA0[4], dA1[4], dB0[4], dB1[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const uint32_t r = (wave * 4 + i) * 8 + (lane >> 3), c = ((lane & 7) ^ ((r >> 1) & 7)) * 16;
+    dA0[i] = min(r, last_a) * sa + c;
+    dA1[i] = min(r + 128, last_a) * sa + c;
+    dB0[i] = min(r, last_b) * sb + c;
+    dB1[i] = GATED ? dB0[i] : min(r + 128, last_b) * sb + c;
+  }
+  // (the compiler may keep a uniform value in a vector register; the assembly wants scalars)
+  auto scalar = [](const uint16_t *p) {
+    const uint64_t v = (uint64_t)p;
+    return (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)v) | (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(v >> 32)) << 32;
+  };
+  const uint64_t sa0 = scalar(pa), sb0 = scalar(pb0), sb1 = scalar(pb1);
+  const uint32_t lds = wave * 4096;  // (all LDS of this kernel is the two stages, at offset 0)
+#define RING_IN                                                                                                            \
+  [dA00] "v"(dA0[0]), [dA01] "v"(dA0[1]), [dA02] "v"(dA0[2]), [dA03] "v"(dA0[3]), [dA10] "v"(dA1[0]), [dA11] "v"(dA1[1]),  \
+      [dA12] "v"(dA1[2]), [dA13] "v"(dA1[3]), [dB00] "v"(dB0[0]), [dB01] "v"(dB0[1]), [dB02] "v"(dB0[2]),                  \
+      [dB03] "v"(dB0[3]), [dB10] "v"(dB1[0]), [dB11] "v"(dB1[1]), [dB12] "v"(dB1[2]), [dB13] "v"(dB1[3]), [pa] "s"(sa0),   \
+      [pb0] "s"(sb0), [pb1] "s"(sb1), [lds] "s"(lds)
+#define RING_SCALARS "s40", "s41", "s42", "s43", "s44", "s45", "s46", "s47", "m0", "scc", "memory"
+#define RING_V10(d) "v" #d "0", "v" #d "1", "v" #d "2", "v" #d "3", "v" #d "4", "v" #d "5", "v" #d "6", "v" #d "7", "v" #d "8", "v" #d "9"
+#define RING_FRAGMENTS                                                                                                     \
+  "v128", "v129", RING_V10(13), RING_V10(14), RING_V10(15), RING_V10(16), RING_V10(17), RING_V10(18), RING_V10(19),        \
+      RING_V10(20), RING_V10(21), RING_V10(22), RING_V10(23), RING_V10(24), "v250", "v251", "v252", "v253", "v254", "v255"
+  asm volatile(FIRST_LOADS::RING_IN : RING_SCALARS);
+  float zero;
+  asm volatile("v_mov_b32 %0, 0" : "=v"(zero));  // (the accumulators are cleared behind the first loads, not in front of them)
+  f32x16 acc[2][2][2][2];  // [A half][B half][row block][column block]
+#pragma unroll
+  for (int q = 0; q < 16; ++q)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) acc[q >> 3][(q >> 2) & 1][(q >> 1) & 1][q & 1][e] = zero;
+  const uint32_t half = lane >> 5;
+  uint32_t ra[4], rb[4];  // where this lane's fragments of a k-slice start in a unit
+#pragma unroll
+  for (int ks = 0; ks < 4; ++ks) {
+    const uint32_t p = ((ks * 2 + half) ^ ((lane >> 1) & 7)) * 16 + (lane & 31) * 128;
+    ra[ks] = wm * 8192 + p;
+    rb[ks] = wn * 8192 + p;
+  }
+  unsigned long long tick0 = 0, real0 = 0;  // (clock probe only: GemmDesc::clock_ticks)
+  if (KIND == RING_PLAIN && g.clock_ticks) {
+    tick0 = __builtin_amdgcn_s_memtime();
+    real0 = __builtin_amdgcn_s_memrealtime();
+  }
+#define RING_ACC(a, b, i, j) [c##a##b##i##j] "+a"(acc[a][b][i][j])
+#define RING_INOUT                                                                                                       \
+  RING_ACC(0, 0, 0, 0), RING_ACC(0, 0, 0, 1), RING_ACC(0, 0, 1, 0), RING_ACC(0, 0, 1, 1), RING_ACC(0, 1, 0, 0),          \
+      RING_ACC(0, 1, 0, 1), RING_ACC(0, 1, 1, 0), RING_ACC(0, 1, 1, 1), RING_ACC(1, 0, 0, 0), RING_ACC(1, 0, 0, 1),      \
+      RING_ACC(1, 0, 1, 0), RING_ACC(1, 0, 1, 1), RING_ACC(1, 1, 0, 0), RING_ACC(1, 1, 0, 1), RING_ACC(1, 1, 1, 0),      \
+      RING_ACC(1, 1, 1, 1), [ra0] "+v"(ra[0]), [ra1] "+v"(ra[1]), [ra2] "+v"(ra[2]), [ra3] "+v"(ra[3]), [rb0] "+v"(rb[0]), \
+      [rb1] "+v"(rb[1]), [rb2] "+v"(rb[2]), [rb3] "+v"(rb[3])
+  asm volatile(MAIN_LOOP : RING_INOUT : RING_IN, [n] "s"(n_steps) : RING_SCALARS, RING_FRAGMENTS);
+  if (KIND == RING_PLAIN && g.clock_ticks && tid == 0) {
+    atomicAdd(g.clock_ticks, __builtin_amdgcn_s_memtime() - tick0);
+    atomicAdd(g.clock_ticks + 1, __builtin_amdgcn_s_memrealtime() - real0);
+  }
+  // The tile leaves through LDS, a quadrant at a time and each wavefront for itself: a lane holds pieces of four columns in 32
+  // different rows, and stored as they are every instruction would touch 32 lines; out of LDS a store is four rows of 64
+  // columns, whole lines.  (Chunks of 16 bytes swizzled by the row: no bank conflicts either way.)  A tile without edges has
+  // no branch in all of this: with one per store the accumulators' 256 registers leave one at a time, 8 us a tile.
+  __syncthreads();  // every wavefront has read its last fragments
+  extern __shared__ __attribute__((aligned(16))) float ring_smem[];
+  uint16_t *C16 = g.c16 ? g.c16 + (uint64_t)bz * g.M * g.N : nullptr;
+  const bool whole = m0 + 256 <= g.M && n0 + BNO <= Nl && !Bias;
+  constexpr bool F32 = KIND == RING_PLAIN;
+  const uint32_t pitch = KIND == RING_SIGMOID ? g.c16_pitch : Nl;
+  uint32_t to[4];  // where this lane's piece of rows 0-3, 4-7, 8-11, 12-15 of a quadrant goes, in bytes from its corner
+#pragma unroll
+  for (int u = 0; u < 4; ++u) to[u] = ((u * 4 + (lane >> 4)) * pitch + (((lane & 15) ^ (u * 4 + (lane >> 4))) << 2)) * (F32 ? 4u : 2u);
+#pragma unroll
+  for (int qd = 0; qd < (GATED ? 2 : 4); ++qd) {
+    const int a = GATED ? qd : qd >> 1, b = GATED ? 0 : qd & 1;
+    float *tile = ring_smem + wave * 8192 + (qd & 1) * 4096;
+    const uint32_t col0 = n0 + b * 128 + wn * 64, row0 = m0 + a * 128 + wm * 64;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const uint32_t r = i * 32 + (lane & 31), chunk = j * 8 + q * 2 + half;
+          const f32x16 &x = acc[a][b][i][j], &u = acc[a][GATED ? 1 : b][i][j];
+          float4 v = make_float4(x[q * 4], x[q * 4 + 1], x[q * 4 + 2], x[q * 4 + 3]);
+          if (KIND == RING_GELU) v = make_float4(gelu_fast(v.x), gelu_fast(v.y), gelu_fast(v.z), gelu_fast(v.w));
+          if (KIND == RING_SILU) v = make_float4(silu_fast(v.x), silu_fast(v.y), silu_fast(v.z), silu_fast(v.w));
+          if (KIND == RING_SIGMOID) v = make_float4(sigmoid_fast(v.x), sigmoid_fast(v.y), sigmoid_fast(v.z), sigmoid_fast(v.w));
+          if (GATED) { v.x *= u[q * 4]; v.y *= u[q * 4 + 1]; v.z *= u[q * 4 + 2]; v.w *= u[q * 4 + 3]; }
+          *(float4 *)(tile + r * 64 + ((chunk ^ (r & 15)) << 2)) = v;
+        }
+    const float *from = tile + ((lane >> 4) << 6) + ((lane & 15) << 2);
+    if (whole) {
+      float4 out[16];
+#pragma unroll
+      for (int it = 0; it < 16; ++it) out[it] = *(const float4 *)(from + it * 256);
+      char *corner = F32 ? (char *)(C + (uint64_t)row0 * Nl + col0) : (char *)(C16 + (uint64_t)row0 * pitch + col0);
+#pragma unroll
+      for (int it = 0; it < 16; ++it) {
+        char *at = corner + (uint64_t)(it >> 2) * 16 * pitch * (F32 ? 4 : 2) + to[it & 3];
+        if (F32) {
+          __builtin_memcpy(at, &out[it], 16);  // (rows of any length: 4-byte aligned)
+        } else {
+          *(uint2 *)at = bf16_pack4(out[it]);
+        }
+      }
+      continue;
+    }
+#pragma unroll 1
+    for (uint32_t it = 0; it < 16; ++it) {
+      const uint32_t r = it * 4 + (lane >> 4), row = row0 + r, col = col0 + (((lane & 15) ^ (r & 15)) << 2);
+      float4 v = *(const float4 *)(from + it * 256);
+      if (row >= g.M) continue;
+      if (F32) {
+        float *c = C + (uint64_t)row * Nl + col;
+        const float e[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+          if (col + k < Nl) c[k] = Bias ? e[k] + Bias[col + k] : e[k];
+      } else if (col < pitch) {  // (N % 4 == 0, or padded rows: a piece is inside or outside; zeros past the last column)
+        v = make_float4(col < Nl ? v.x : 0.f, col + 1 < Nl ? v.y : 0.f, col + 2 < Nl ? v.z : 0.f, col + 3 < Nl ? v.w : 0.f);
+        *(uint2 *)(C16 + (uint64_t)row * pitch + col) = bf16_pack4(v);
+      }
+    }
+  }
+}
+
+// Operands whose rows lie within 32-bit byte offsets of a tile's first row, two k-steps at least to each slice.
+bool gemm_ring_ok(const GemmDesc &g) {
+  const uint32_t splits = g.splits > 1 ? g.splits : 1, last = splits > 1 ? g.K - (splits - 1) * g.k_per_split : g.K;
+  if (splits > 1 && ((uint64_t)(splits - 1) * g.k_per_split >= g.K || g.k_per_split % 64 || g.k_per_split < 128)) return false;
+  return g.sak == 1 && g.sbk == 1 && last % 64 == 0 && last >= 128 && g.sam >= 0 && g.sbn >= 0 && g.sam <= (1 << 22) &&
+         g.sbn <= (1 << 22) && !g.rope_s && !g.glu_gate && (!g.act_sigmoid || splits > 1 || g.c16_pitch) &&
+         (!g.dual_b || (g.c16 && !g.c));
+}
+
+template <int KIND>
+static hipError_t launch_ring_as(const LaunchCtx &lc, const GemmDesc &g, uint32_t grid) {
+  constexpr int smem = 2 * 65536;
+  static bool configured = false;  // one attribute call per kernel and process
+  if (!configured) {
+    hipError_t e = hipFuncSetAttribute((const void *)gemm_bf16_ring_kernel<KIND>, hipFuncAttributeMaxDynamicSharedMemorySize, smem);
+    if (e != hipSuccess) return e;
+    configured = true;
+  }
+  cg_launch(lc, gemm_bf16_ring_kernel<KIND>, dim3(grid), dim3(256), smem, g);
+  return hipGetLastError();
+}
+
+hipError_t launch_gemm_ring(const LaunchCtx &lc, const GemmDesc &g) {
+  if (!gemm_ring_ok(g)) return hipErrorInvalidValue;
+  const uint32_t bno = g.dual_b ? 128 : 256, batch = g.nb0 * g.nb1 * (g.splits > 1 ? g.splits : 1);
+  const uint64_t grid = (uint64_t)((g.M + 255) / 256) * ((g.N + bno - 1) / bno) * batch;
+  if (grid > 0x7FFFFFFFull) return hipErrorInvalidValue;
+  if (g.dual_b) return g.glu_kind ? launch_ring_as<RING_GELU>(lc, g, (uint32_t)grid) : launch_ring_as<RING_SILU>(lc, g, (uint32_t)grid);
+  if (g.act_sigmoid && g.splits <= 1) return launch_ring_as<RING_SIGMOID>(lc, g, (uint32_t)grid);
+  return launch_ring_as<RING_PLAIN>(lc, g, (uint32_t)grid);
+}
+
+}  // namespace cgk

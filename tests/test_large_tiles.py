@@ -1,0 +1,82 @@
+"""bf16 products that fill the chip with 256 x 256 tiles (gemm_bf16_ring_kernel): two k-steps, an odd number, many; rows and
+columns that end inside a tile and rows of a length that is no multiple of 16 bytes; the stacked gate / up form with either
+activation; grouped products with and without a bias; a sigmoid stored as the next product's operand."""
+import numpy as np
+import pytest
+
+import vectors
+
+lang, nn = vectors.cg.lang, vectors.cg.nn
+
+
+def draw(g, shape, std=1.0):
+    return vectors.bf16_round((g.standard_normal(shape) * std).astype(np.float32))
+
+
+def linear(b, x, w, n, k, bias=None):
+    y = lang.matmul(b, x, lang.reshape(b, lang.make_shape(b, 1, k, n), lang.transpose(b, 0, 1, w)))
+    return y if bias is None else y + lang.broadcast(b, bias, lang.shape(b, y))
+
+
+def product_and_bound(x, w):
+    """x w^T in 64 bits and what K f32 additions of exact bf16 products may be off by."""
+    x, w = x.astype(np.float64), w.astype(np.float64)
+    return x @ w.T, x.shape[-1] * 2.0 ** -24 * (np.abs(x) @ np.abs(w).T)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(4096, 4096, 128), (4097, 4101, 192), (3841, 4353, 256), (8300, 2049, 320), (255, 65600, 448)])
+def test_product(hip_bf16, M, N, K):
+    g = np.random.default_rng(M)
+    x, w = draw(g, (1, M, K)), draw(g, (N, K))
+    (got,) = vectors.run(hip_bf16, lambda b, x, w: [linear(b, x, w, N, K)], 1, x, w)
+    ref, bound = product_and_bound(x[0], w)
+    assert np.all(np.abs(got[0] - ref) <= bound)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("bias", [False, True])
+@pytest.mark.parametrize("M,K", [(21900, 128), (22016, 192)])
+def test_grouped_products(hip_bf16, M, K, bias):
+    g = np.random.default_rng(K)
+    x, ws, bs = draw(g, (1, M, K)), [draw(g, (256, K)) for _ in range(3)], [g.standard_normal(256).astype(np.float32) for _ in range(3)]
+
+    def f(b, x, *p):
+        return [linear(b, x, p[i], 256, K, p[3 + i] if bias else None) for i in range(3)]
+    got = vectors.run(hip_bf16, f, 3, x, *ws, *bs)
+    for w, v, y in zip(ws, bs, got):
+        ref, bound = product_and_bound(x[0], w)
+        if bias:    # one more f32 addition
+            ref, bound = ref + v, bound + 2.0 ** -24 * (np.abs(ref) + np.abs(v))
+        assert np.all(np.abs(y[0] - ref) <= bound)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("act", ["silu", "gelu"])
+@pytest.mark.parametrize("M,F,K", [(4096, 2048, 128), (4100, 2052, 192), (3900, 2184, 320)])
+def test_gated(hip_bf16, M, F, K, act):
+    g = np.random.default_rng(F)
+    x, wg, wu, wd = draw(g, (1, M, K)), draw(g, (F, K), K ** -0.5), draw(g, (F, K), K ** -0.5), np.eye(64, F, dtype=np.float32)
+
+    def f(b, x, wg, wu, wd):    # (wd picks the first 64 gated values out: exact products)
+        x = x + x - x
+        return [linear(b, getattr(nn, act)(b, linear(b, x, wg, F, K)) * linear(b, x, wu, F, K), wd, 64, F)]
+    (got,) = vectors.run(hip_bf16, f, 1, x, wg, wu, np.roll(wd, F - 64, axis=1))
+    gate, up = (x[0].astype(np.float64) @ w[F - 64:].astype(np.float64).T for w in (wg, wu))
+    c = gate if act == "silu" else 2 * np.sqrt(2 / np.pi) * (gate + 0.044715 * gate ** 3)
+    ref = gate / (1 + np.exp(-c)) * up
+    # rounded once to bf16, whose eight significant bits leave half a unit in the last place: 2^-8 of the value at most; the f32
+    # sums of K <= 320 products of rms K^-1/2 in front of it are good to 1e-5
+    assert np.all(np.abs(got[0] - ref) <= 2.0 ** -8 * np.abs(ref) + 1e-5)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,K,H", [(4100, 130, 4099), (4352, 192, 3900)])
+def test_sigmoid_as_the_next_operand(hip_bf16, M, K, H):
+    g = np.random.default_rng(H)
+    x, w1 = draw(g, (M, K)), draw(g, (K, H), K ** -0.5)
+    w2 = np.zeros((H, 64), np.float32)
+    w2[H - 64 + np.arange(64), np.arange(64)] = 1.0
+    (got,) = vectors.run(hip_bf16, lambda b, x, w1, w2: [lang.matmul(b, nn.sigmoid(b, lang.matmul(b, x, w1)), w2)], 1, x, w1, w2)
+    ref = 1 / (1 + np.exp(-(x.astype(np.float64) @ w1[:, H - 64:].astype(np.float64))))
+    assert np.all(np.abs(got - ref) <= 2.0 ** -8 * ref + 1e-5)    # (as above)
