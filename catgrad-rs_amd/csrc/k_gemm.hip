@@ -16,9 +16,11 @@
 //    partial dots meet in a DPP/shuffle reduction; x stays in L2/registers.
 //  * gemv_col_kernel (M <= 8, B n-contiguous): lanes across n, k split over the workgroup.
 #include <hip/hip_runtime.h>
+#include <algorithm>
 #include <cstring>
 #include "launch.hpp"
 #include "dev_common.hpp"
+#include "mfma_step_ring.hpp"
 
 namespace cgk {
 
@@ -519,7 +521,9 @@ template <int N> __device__ __forceinline__ void wait_vmcnt() {
 // sums meet in LDS at the end.  For tiles of a few rows against weights nobody has touched (a prompt of 17 to 128
 // tokens), which are bound by the stream of weights: narrow tiles put a workgroup on every CU, and more wavefronts than
 // such a tile has MFMA columns for share the issue of its loads (a global_load_lds costs its wave 55 - 120 cycles).
-template <int BM_, int BN_, int WR, int WC, bool EPI, int NS, bool DUAL = false, bool BKM = false, bool ROPE = false, int KG = 1>
+// RING: four wavefronts, and the main loop of mfma_step_ring.hpp: every slice of k has NS - 1 k-steps at least.
+template <int BM_, int BN_, int WR, int WC, bool EPI, int NS, bool DUAL = false, bool BKM = false, bool ROPE = false, int KG = 1,
+          bool RING = false>
 __global__ void __launch_bounds__(WR *WC *KG * 64) gemm_bf16_dma_kernel(GemmDesc g) {
   constexpr int NW = WR * WC * KG, BK = 64;
   static_assert(!ROPE || ((BN_ % 64 == 0 || BN_ == 32) && !EPI && !DUAL && !BKM && (BM_ * BN_ / 4) % (NW * 64) == 0),
@@ -590,10 +594,12 @@ __global__ void __launch_bounds__(WR *WC *KG * 64) gemm_bf16_dma_kernel(GemmDesc
       for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
 
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint16_t *)dma_smem;
+  constexpr int PA = BM_ / 32, PB = BN_ / 32;  // RING: this wave's pieces of A and of B
+  auto piece = [&](int i) { return !RING ? wave * LPW + i : i < PA ? wave * PA + i : BM_ / 8 + wave * PB + i - PA; };
   const uint16_t *gp[LPW];  // per-lane source of each of this wave's loads; advances by BK per stage
 #pragma unroll
   for (int i = 0; i < LPW; ++i) {
-    const int q = wave * LPW + i;  // 8-row block of the stacked [A; B] tile
+    const int q = piece(i);  // 8-row block of the stacked [A; B] tile
     const int R = q * 8 + (lane >> 3);
     const int c = (lane & 7) ^ ((R >> 1) & 7);
     if (q * 8 < BM_) {
@@ -611,7 +617,7 @@ __global__ void __launch_bounds__(WR *WC *KG * 64) gemm_bf16_dma_kernel(GemmDesc
   auto issue = [&](int buf) {
 #pragma unroll
     for (int i = 0; i < LPW; ++i) {
-      lds_dma16(gp[i], lds0 + buf * STAGE + (wave * LPW + i) * 1024);
+      lds_dma16(gp[i], lds0 + buf * STAGE + piece(i) * 1024);
       gp[i] += gp_step;
     }
   };
@@ -687,14 +693,57 @@ __global__ void __launch_bounds__(WR *WC *KG * 64) gemm_bf16_dma_kernel(GemmDesc
 #pragma unroll
   for (int s0 = 0; s0 < NS - 1; ++s0)
     if (s0 < n_steps) issue(s0);
-  for (int step = 0; step < n_steps; ++step) {
-    // stage `step` has landed (this wave's part): at most the NS - 2 younger stages are still in
-    // flight; in the tail, where fewer were issued, wait for everything
-    if (step + NS - 1 <= n_steps) wait_vmcnt<(NS - 2) * LPW>();
-    else wait_vmcnt<0>();
-    __syncthreads();   // ... and everyone's; all waves are done reading the buffer refilled next
-    if (step + NS - 1 < n_steps) issue((step + NS - 1) % NS);
-    compute(step % NS);
+  if constexpr (RING) {
+    // (the accumulators are cleared behind the first loads)
+    float zero;
+    asm volatile("v_mov_b32 %0, 0" : "=v"(zero));
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) acc[i][j][e] = zero;
+    uint32_t ra[4], rb[4];  // where this lane's fragments of a slice start in a stage
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) {
+      const uint32_t p = lds0 + (lane & 31) * 128 + ((ks * 2 + half) ^ sw) * 16;
+      ra[ks] = p + wm * WM * 128;
+      rb[ks] = p + BM_ * 128 + wn * (DUAL ? OC : WN) * 128;
+    }
+    uint64_t at[LPW];
+#pragma unroll
+    for (int i = 0; i < LPW; ++i) at[i] = (uint64_t)gp[i];
+    const uint32_t la = lds0 + wave * PA * 1024, ab = (BM_ / 8 + wave * (PB - PA)) * 1024;
+    const uint32_t first = la + (NS - 1) * STAGE, limit = la + NS * STAGE;
+    const uint32_t n = __builtin_amdgcn_readfirstlane((uint32_t)n_steps);
+#define SR_ACC(i, j) [c##i##j] "+a"(acc[i][j])
+#define SR_A4 [ga0] "+v"(at[0]), [ga1] "+v"(at[1]), [ga2] "+v"(at[2]), [ga3] "+v"(at[3])
+#define SR_B4(o) [gb0] "+v"(at[o]), [gb1] "+v"(at[o + 1]), [gb2] "+v"(at[o + 2]), [gb3] "+v"(at[o + 3])
+#define SR_IN                                                                                                              \
+  [ra0] "v"(ra[0]), [ra1] "v"(ra[1]), [ra2] "v"(ra[2]), [ra3] "v"(ra[3]), [rb0] "v"(rb[0]), [rb1] "v"(rb[1]),              \
+      [rb2] "v"(rb[2]), [rb3] "v"(rb[3]), [first] "s"(first), [limit] "s"(limit), [la] "s"(la), [ab] "s"(ab), [n] "s"(n),  \
+      [stage] "i"(STAGE), [all] "i"(NS * STAGE), [held] "i"(NS - 1)
+    if constexpr (TM == 2 && TN == 2) {
+      static_assert(NS == 5 && !EPI, "");
+      asm volatile(SR_LOOP_22 : SR_ACC(0, 0), SR_ACC(0, 1), SR_ACC(1, 0), SR_ACC(1, 1), SR_A4, SR_B4(4) : SR_IN : SR_CLOBBERS);
+    } else {
+      static_assert(TM == 3 && TN == 2 && NS == 4 && !EPI, "");
+      asm volatile(SR_LOOP_32
+                   : SR_ACC(0, 0), SR_ACC(0, 1), SR_ACC(1, 0), SR_ACC(1, 1), SR_ACC(2, 0), SR_ACC(2, 1), SR_A4, [ga4] "+v"(at[4]),
+                     [ga5] "+v"(at[5]), SR_B4(6)
+                   : SR_IN
+                   : SR_CLOBBERS);
+    }
+  } else {
+    for (int step = 0; step < n_steps; ++step) {
+      // stage `step` has landed (this wave's part): at most the NS - 2 younger stages are still in
+      // flight; in the tail, where fewer were issued, wait for everything
+      if (step + NS - 1 <= n_steps) wait_vmcnt<(NS - 2) * LPW>();
+      else wait_vmcnt<0>();
+      __syncthreads();   // ... and everyone's; all waves are done reading the buffer refilled next
+      if (step + NS - 1 < n_steps) issue((step + NS - 1) % NS);
+      compute(step % NS);
+    }
   }
   if (g.clock_ticks && tid == 0) {
     atomicAdd(g.clock_ticks, __builtin_amdgcn_s_memtime() - tick0);
@@ -916,18 +965,19 @@ __global__ void __launch_bounds__(WR *WC *KG * 64) gemm_bf16_dma_kernel(GemmDesc
     }
 }
 
-template <int BM_, int BN_, int WR, int WC, bool EPI = false, int NS = 2, bool DUAL = false, bool BKM = false, bool ROPE = false, int KG = 1>
+template <int BM_, int BN_, int WR, int WC, bool EPI = false, int NS = 2, bool DUAL = false, bool BKM = false, bool ROPE = false, int KG = 1,
+          bool RING = false>
 static hipError_t launch_gemm_dma(const LaunchCtx &lc, const GemmDesc &g, uint32_t grid) {
   // (ROPE: the f32 tile is exchanged through LDS at the end, BN_ + 8 floats per row)
   constexpr int stages = NS * (BM_ + BN_) * 64 * 2, smem = ROPE && BM_ * (BN_ + 8) * 4 > stages ? BM_ * (BN_ + 8) * 4 : stages;
   static bool configured = false;  // one attribute call per kernel and process
   if (!configured) {
-    hipError_t e = hipFuncSetAttribute((const void *)gemm_bf16_dma_kernel<BM_, BN_, WR, WC, EPI, NS, DUAL, BKM, ROPE, KG>,
+    hipError_t e = hipFuncSetAttribute((const void *)gemm_bf16_dma_kernel<BM_, BN_, WR, WC, EPI, NS, DUAL, BKM, ROPE, KG, RING>,
                                        hipFuncAttributeMaxDynamicSharedMemorySize, smem);
     if (e != hipSuccess) return e;
     configured = true;
   }
-  cg_launch(lc, gemm_bf16_dma_kernel<BM_, BN_, WR, WC, EPI, NS, DUAL, BKM, ROPE, KG>, dim3(grid), dim3(WR * WC * KG * 64), smem, g);
+  cg_launch(lc, gemm_bf16_dma_kernel<BM_, BN_, WR, WC, EPI, NS, DUAL, BKM, ROPE, KG, RING>, dim3(grid), dim3(WR * WC * KG * 64), smem, g);
   return hipGetLastError();
 }
 
@@ -3099,13 +3149,17 @@ hipError_t launch_matmul(const LaunchCtx &lc_in, const GemmDesc &g, const char *
         if (g.n_group || g.glu_gate || splits != 1) return hipErrorInvalidValue;
         const uint64_t d256 = (uint64_t)((g.M + 255) / 256) * ((g.N + 127) / 128) * batch;
         const uint64_t d128 = (uint64_t)((g.M + 127) / 128) * ((g.N + 127) / 128) * batch;
-        // (fewer tiles of 128 than half the CUs: 64 or 32 output columns per tile)
-        if (d256 >= (uint64_t)lc.n_cus && gemm_ring_ok(gg)) e = launch_gemm_ring(lc, gg);
-        else if (d128 * 4 <= (uint64_t)lc.n_cus)
+        // Tiles of 256 rows or of 128, by the rounds they take: a round of the large ones costs 1.4 to 1.7 rounds of the small (512 rows
+        // by 2 x 8192, K = 2048, one round either way 56 and 40 us; 700 rows, one round or two, 50 and 60; 1024 rows by 2 x 5632 47 and
+        // 60; 1500 rows, two or three, 92 and 84; 2900 by 2 x 8192, three or six, 159 and 181).  Fewer tiles of 128 than half the
+        // CUs: 64 or 32 output columns per tile.
+        const uint64_t cus = (uint64_t)lc.n_cus, r256 = (d256 + cus - 1) / cus, r128 = (d128 + cus - 1) / cus;
+        if (r256 * 5 <= r128 * 3 && gemm_ring_ok(gg)) e = launch_gemm_ring(lc, gg);
+        else if (d128 * 4 <= cus)
           e = launch_gemm_dma<128, 64, 4, 1, true, 5, true, false, false, 2>(lc, gg, (uint32_t)((uint64_t)((g.M + 127) / 128) * ((g.N + 31) / 32) * batch));
-        else if (d128 * 2 <= (uint64_t)lc.n_cus)
+        else if (d128 * 2 <= cus || g.K < 192 || !gemm_ring_ok(gg))
           e = launch_gemm_dma<128, 128, 4, 2, true, 4, true>(lc, gg, (uint32_t)((uint64_t)((g.M + 127) / 128) * ((g.N + 63) / 64) * batch));
-        else e = launch_gemm_dma<128, 256, 2, 4, true, 3, true>(lc, gg, (uint32_t)d128);
+        else e = launch_gemm_ring(lc, gg, true);
       } else if (g.glu_gate || g.c16 || (g.act_sigmoid && splits == 1)) {
         if (g.act_sigmoid && t256 >= (uint64_t)lc.n_cus && gemm_ring_ok(gg)) e = launch_gemm_ring(lc, gg);
         else if (g.act_sigmoid && t256 >= (uint64_t)lc.n_cus) e = launch_gemm_dma<256, 256, 2, 4, true, 2>(lc, gg, (uint32_t)t256);
@@ -3140,33 +3194,47 @@ hipError_t launch_matmul(const LaunchCtx &lc_in, const GemmDesc &g, const char *
                          : launch_gemm_dma<128, 128, 2, 2>(lc, gg, (uint32_t)t128);
         else
           e = launch_gemm_ring(lc, gg);
-      } else if (splits == 1 && t128 * 2 <= (uint64_t)lc.n_cus && g.N >= 128) {
-        // too few 128 x 128 tiles for the CUs and no split-K to multiply them: halve the tile
-        const uint32_t t64 = (uint32_t)((uint64_t)((g.M + 127) / 128) * ((g.N + 63) / 64) * batch);
-        // (heads of 128 columns need the whole head in one tile)
-        if (g.rope_s && g.rope_hd > 64) e = launch_gemm_dma<128, 128, 2, 4, false, 4, false, false, true>(lc, gg, (uint32_t)t128);
-        else if (g.rope_s) e = launch_gemm_dma<128, 64, 4, 2, false, 4, false, false, true>(lc, gg, t64);
-        else e = launch_gemm_dma<128, 64, 4, 2, false, 4>(lc, gg, t64);
-      } else if (deep) {
-        // more tiles than CUs and an epilogue that takes a while: two workgroups of two stages share a CU, and the
-        // epilogue of one runs under the main loop of the other (1024 x 6144 x 2048: 59.7 -> 47.6 us, what the plain
-        // grouped product takes; the plain product itself gains nothing from it)
-        const bool two = t128 > (uint64_t)lc.n_cus;
-        if (g.rope_s && two) e = launch_gemm_dma<128, 128, 2, 4, false, 2, false, false, true>(lc, gg, (uint32_t)t128);
-        else if (g.rope_s) e = launch_gemm_dma<128, 128, 2, 4, false, 4, false, false, true>(lc, gg, (uint32_t)t128);
-        // (a second round of 128-row tiles that would be mostly empty: 192 rows, if all of those tiles run at once - o_proj and
-        // down_proj of 2900 rows, 2048 columns, 368 tiles or 256: 97 -> 75 us on average, of 2600 rows 95 -> 71)
-        else if (const uint64_t t192 = (uint64_t)((g.M + 191) / 192) * ((g.N + 127) / 128) * batch * splits;
-                 !g.n_group && two && t192 <= (uint64_t)lc.n_cus)
-          e = launch_gemm_dma<192, 128, 2, 4, false, 3>(lc, gg, (uint32_t)t192);
-        else e = launch_gemm_dma<128, 128, 2, 4, false, 4>(lc, gg, (uint32_t)t128);
       } else {
-        // Eight waves share the tail of a tile - a rotation, or stores after few k-steps -, four are ahead in a long main loop:
-        // q / k / v rotated, 2900 rows of 3072 columns: four waves 79 us, eight 69; 1350 rows of 6144 with heads of 128 86, 77;
-        // plain, K = 1152, 16384 rows of 1536 62, 56; 4000 rows of 2048, K = 2048 and 8192 on average, 90, 93.
-        if (g.rope_s) e = launch_gemm_dma<128, 128, 2, 4, false, 2, false, false, true>(lc, gg, (uint32_t)t128);
-        else if (g.K < 2048) e = launch_gemm_dma<128, 128, 2, 4, false, 2>(lc, gg, (uint32_t)t128);
-        else e = launch_gemm_dma<128, 128, 2, 2>(lc, gg, (uint32_t)t128);
+        // Tiles of 128 columns.  One workgroup to a CU with its main loop in one statement (mfma_step_ring.hpp; 128 or 192 rows), or
+        // two to a CU of two stages each, one's tail under the other's main loop, with eight wavefronts where the tail weighs.
+        const uint64_t cus = (uint64_t)lc.n_cus, t192 = (uint64_t)((g.M + 191) / 192) * ((g.N + 127) / 128) * batch * splits;
+        const uint32_t before_last = (splits - 1) * gg.k_per_split;  // (the last slice may be shorter)
+        const uint32_t steps = before_last >= g.K ? 0 : std::min(gg.k_per_split, g.K - before_last) / 64;
+        auto rounds = [&](uint64_t tiles) { return (tiles + cus - 1) / cus; };
+        if (g.rope_s) {
+          // q / k / v rotated.  Up to a round of 128 rows (four stages and eight wavefronts instead: 700 rows of 3072 columns 24.2 us,
+          // 22.4; 600 of 6144 27.3, 26.7), or of 192 (1500 rows of 3072 39.3, 34.3); from there on the long tail - 64 KB of tile
+          // through LDS, table rows from L2 - is worth a second workgroup to the CU (2000 rows 40.2, 43.6 on one; 1024 rows of 6144
+          // 39.6, 46.3).  Few tiles and heads of 64: 64 columns a tile (512 rows 18.3, 21.8).
+          if (splits == 1 && t128 * 2 <= cus && g.rope_hd == 64)
+            e = launch_gemm_dma<128, 64, 4, 2, false, 4, false, false, true>(lc, gg, (uint32_t)((uint64_t)((g.M + 127) / 128) * ((g.N + 63) / 64) * batch));
+          else if (t128 <= cus && steps >= 4) e = launch_gemm_dma<128, 128, 2, 2, false, 5, false, false, true, 1, true>(lc, gg, (uint32_t)t128);
+          else if (t192 <= cus && steps >= 4) e = launch_gemm_dma<192, 128, 2, 2, false, 4, false, false, true, 1, true>(lc, gg, (uint32_t)t192);
+          else e = launch_gemm_dma<128, 128, 2, 4, false, 2, false, false, true>(lc, gg, (uint32_t)t128);
+        } else if (splits == 1 && t128 * 2 <= cus && g.N >= 128) {
+          // too few 128 x 128 tiles for the CUs and no split-K to multiply them: halve the tile
+          e = launch_gemm_dma<128, 64, 4, 2, false, 4>(lc, gg, (uint32_t)((uint64_t)((g.M + 127) / 128) * ((g.N + 63) / 64) * batch));
+        } else if (t128 <= cus) {
+          // A round of 128 rows.  The four wavefronts' longer start and tail pay from 32 k-steps on, or from 16 while CUs are left over
+          // (1500 x 2048 x 8192 71 -> 55 us, x 2048 23 -> 19; 512 x 2048 x 8192 in four slices 25.5 -> 22.2; 8 steps 10.7, 12.4).
+          if (steps >= 32 || (steps >= 16 && t128 * 4 <= cus * 3)) e = launch_gemm_dma<128, 128, 2, 2, false, 5, false, false, false, 1, true>(lc, gg, (uint32_t)t128);
+          else e = launch_gemm_dma<128, 128, 2, 4, false, 4>(lc, gg, (uint32_t)t128);
+        } else if (t192 <= cus && steps >= 4) {
+          // a round of 192 rows (o_proj and down_proj of 2900 rows: 29 and 91 us; 368 tiles of 128 rows two to a CU 35 and 122; 1024
+          // deep 19.7, 21.6)
+          e = launch_gemm_dma<192, 128, 2, 2, false, 4, false, false, false, 1, true>(lc, gg, (uint32_t)t192);
+        } else if (steps >= 64) {
+          // Several rounds of a deep product, a round of 192 rows at 1.42 times one of 128: 8192 x 1152 x 6912 two or three, 134 and 148 us
+          // (two to a CU 167); 4000 x 2048 x 8192 two either way, 149 and 130 (145); 3100 rows 144 and 117 (122).
+          if (rounds(t192) * 10 <= rounds(t128) * 7) e = launch_gemm_dma<192, 128, 2, 2, false, 4, false, false, false, 1, true>(lc, gg, (uint32_t)t192);
+          else e = launch_gemm_dma<128, 128, 2, 2, false, 5, false, false, false, 1, true>(lc, gg, (uint32_t)t128);
+        } else if (g.K < 2048) {
+          // two to a CU; eight waves share the tail, the stores after few k-steps (16384 rows of 1536, K = 1152, 62 -> 56 us), four are
+          // ahead in a long main loop (4000 rows of 2048, K = 2048 40, 43; 3500 rows 38, 40)
+          e = launch_gemm_dma<128, 128, 2, 4, false, 2>(lc, gg, (uint32_t)t128);
+        } else {
+          e = launch_gemm_dma<128, 128, 2, 2>(lc, gg, (uint32_t)t128);
+        }
       }
       if (e != hipSuccess) return e;
     } else if (gemm_dma_bkm_ok(g)) {

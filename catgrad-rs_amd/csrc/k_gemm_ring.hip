@@ -19,6 +19,7 @@
 //   * One barrier a phase: before it a wavefront has seen its own loads of the unit about to be read (a count) and the
 //     reads of two phases ago (a count); so behind it the unit is there for everyone, and its predecessor's place free.
 // The products of an element are added in the order of k, as in gemm_bf16_dma_kernel: the same bits.
+// Tiles of 128 x 256 for the stacked gate / up of fewer rows: see HPHASE0.
 // Measured against 256 x 256 tiles with eight wavefronts whose loads a compiler placed, on the same box: 16384 x 1152 by 2 x 6912
 // gate and up 531 -> 464 us, 2900 x 2048 by 2 x 8192 184 -> 161; 13056 x 6912 x 1152 203 -> 177, 16384 x 1152 x 1536 77 -> 67
 // (100 MB of result); 6000 x 1024 x 4100 with a sigmoid 77 -> 64.  What is left is power: 8192 cubed takes 1.40 us a step on
@@ -173,18 +174,84 @@ typedef __attribute__((ext_vector_type(16))) float f32x16;
   "2:\n\t" PHASE0(OFF, 20) PHASE1(OFF, 16) PHASE2(OFF, 12) PHASE3(OFF, 8) PHASE0(OFF, 4)             \
   PHASE1(OFF, 0) LAST_HALF "s_nop 15\n\ts_nop 7\n\t"
 
+// ---- tiles of 128 x 256: one unit of A, so a step is three units, two phases - (A, B0), (A, B1) - of 16 MFMAs.  LDS holds ten
+// units, in the order A, B0, B1 of every step; the place of the unit 3 s + u is (3 s + u) % 10 (s48 A, s49 B0, s50 B1 of this
+// step, s51 and s52 A and B0 of the next, s53 B1 of the one before).  The second phase of a step reads A and B0 of the next, the
+// first B1 of this one; what they leave is requested again two phases later: A of step s + 3 in the first phase of s, B0 and B1
+// in the second.  Fragments of A are replaced behind the products that use them, a slice late.  Against eight wavefronts with three
+// stages: 400 rows by 2 x 5632, K = 2048, 31 -> 26.5 us, 512 by 2 x 6912, K = 1152, 21.3 -> 18; 512 by 2 x 8192, K = 2048, 38 to 40
+// either way - rows 4 KB apart: with the same weights at a pitch of 4224 bytes 38.6 and 35.7.  (Workgroups of different columns
+// starting at different k: no change.  Loads past the L1: no change.)
+#define HRD(U, B, r, ks) "ds_read_b128 " FR_##U##_##r##_##ks ", " B " offset:" #r "*4096\n\t"
+#define HFROM_A(S, ks) "v_add_u32 v126, " S ", %[ra" #ks "]\n\t"
+#define HFROM_B(S, ks) "v_add_u32 v127, " S ", %[rb" #ks "]\n\t"
+#define HA(r, ks) HRD(A0, "v126", r, ks)
+#define HB0(r, ks) HRD(B0, "v127", r, ks)
+#define HB1(r, ks) HRD(B1, "v127", r, ks)
+#define HM0(i) "s_add_u32 m0, s54, " #i "*1024\n\t"
+#define HON(x) x
+#define HOFF(x) ""
+#define HSYNC(v) "s_waitcnt vmcnt(" #v ")\n\ts_barrier\n\t"
+#define HSLICE(b, UB, ks, W, E0, E1, E2, E3) \
+  W PRODUCT(0, b, 0, 0, A0, UB, ks) E0 PRODUCT(0, b, 0, 1, A0, UB, ks) E1 PRODUCT(0, b, 1, 0, A0, UB, ks) E2 PRODUCT(0, b, 1, 1, A0, UB, ks) E3
+#define HPHASE0(G, v)                                                                                                              \
+  G("s_add_u32 s54, s53, %[lds]\n\t") HSYNC(v)                                                                                     \
+  HFROM_A("s48", 3) HFROM_B("s50", 0)                                                                                              \
+  HSLICE(0, B0, 0, READS_BUT(8), HA(0, 3) G(HM0(0)), HA(1, 3) G(LOAD(A0, 0)), HB1(0, 0), HB1(1, 0)) HFROM_B("s50", 1)          \
+  HSLICE(0, B0, 1, READS_BUT(8), HB1(0, 1) G(HM0(1)), HB1(1, 1) G(LOAD(A0, 1)), "", "") HFROM_B("s50", 2)                          \
+  HSLICE(0, B0, 2, READS_BUT(6), HB1(0, 2) G(HM0(2)), HB1(1, 2) G(LOAD(A0, 2)), "", "") HFROM_B("s50", 3)                          \
+  HSLICE(0, B0, 3, READS_BUT(6), HB1(0, 3) G(HM0(3)), HB1(1, 3) G(LOAD(A0, 3)), "", "")
+#define HPHASE1(G, v)                                                                                                              \
+  G("s_add_u32 s54, s48, %[lds]\n\t") HSYNC(v)                                                                                     \
+  HFROM_B("s52", 0)                                                                                                                \
+  HSLICE(1, B1, 0, READS_BUT(6), HB0(0, 0) G(HM0(0)), HB0(1, 0) G(LOAD(B0, 0) HM0(1)), G(LOAD(B0, 1)), "")                         \
+  HFROM_A("s51", 0) HFROM_B("s52", 1)                                                                                              \
+  HSLICE(1, B1, 1, READS_BUT(6), HB0(0, 1) G(HM0(2)), HB0(1, 1) G(LOAD(B0, 2) HM0(3)), HA(0, 0) G(LOAD(B0, 3)), HA(1, 0))      \
+  HFROM_A("s51", 1) HFROM_B("s52", 2) G("s_add_u32 s54, s49, %[lds]\n\t")                                                          \
+  HSLICE(1, B1, 2, READS_BUT(8), HB0(0, 2) G(HM0(0)), HB0(1, 2) G(LOAD(B1, 0) HM0(1)), HA(0, 1) G(LOAD(B1, 1)), HA(1, 1))      \
+  HFROM_A("s51", 2) HFROM_B("s52", 3)                                                                                              \
+  HSLICE(1, B1, 3, READS_BUT(10), HB0(0, 3) G(HM0(2)), HB0(1, 3) G(LOAD(B1, 2) HM0(3)), HA(0, 2) G(LOAD(B1, 3)), HA(1, 2))
+// (the last step's second phase reads and requests nothing)
+#define HLAST                                                                                                    \
+  HSLICE(1, B1, 0, READS_BUT(6), "", "", "", "") HSLICE(1, B1, 1, READS_BUT(4), "", "", "", "")                  \
+  HSLICE(1, B1, 2, READS_BUT(2), "", "", "", "") HSLICE(1, B1, 3, READS_BUT(0), "", "", "", "")
+#define HNEXT(x, y) "s_add_u32 " x ", " y ", 16384\n\ts_cmp_eq_u32 " x ", 163840\n\ts_cselect_b32 " x ", 0, " x "\n\t"
+#define HNEXT_PLACES \
+  "s_mov_b32 s53, s50\n\ts_mov_b32 s48, s51\n\ts_mov_b32 s49, s52\n\t" HNEXT("s50", "s52") HNEXT("s51", "s50") HNEXT("s52", "s51")
+#define HLOAD_UNIT(U) HM0(0) "s_nop 0\n\t" LOAD(U, 0) HM0(1) "s_nop 0\n\t" LOAD(U, 1) HM0(2) "s_nop 0\n\t" LOAD(U, 2) HM0(3) "s_nop 0\n\t" LOAD(U, 3)
+#define HPOINTERS "s_mov_b64 s[40:41], %[pa]\n\ts_mov_b64 s[42:43], %[pb0]\n\ts_mov_b64 s[44:45], %[pb1]\n\t"
+#define HSTEP_LOADS HLOAD_UNIT(A0) "s_add_u32 s54, s54, 16384\n\t" HLOAD_UNIT(B0) "s_add_u32 s54, s54, 16384\n\t" HLOAD_UNIT(B1) "s_add_u32 s54, s54, 16384\n\t"
+// steps 0 to 2 requested: 36 loads
+#define HFIRST_LOADS HPOINTERS "s_mov_b32 s54, %[lds]\n\t" HSTEP_LOADS NEXT_STEP HSTEP_LOADS NEXT_STEP HSTEP_LOADS
+// n >= 3 steps
+#define HMAIN_LOOP                                                                                                              \
+  HPOINTERS NEXT_STEP NEXT_STEP NEXT_STEP "s_sub_u32 s47, %[n], 3\n\t"                                                          \
+  "s_mov_b32 s48, 0\n\ts_movk_i32 s49, 0x4000\n\ts_mov_b32 s50, 0x8000\n\ts_mov_b32 s51, 0xC000\n\ts_mov_b32 s52, 0x10000\n\t"  \
+  "s_mov_b32 s53, 0x24000\n\t" HSYNC(28)                                                                                        \
+  HFROM_A("s48", 0) HFROM_B("s49", 0) HB0(0, 0) HB0(1, 0) HFROM_B("s49", 1) HB0(0, 1) HB0(1, 1) HA(0, 0) HA(1, 0)           \
+  HFROM_A("s48", 1) HFROM_B("s49", 2) HB0(0, 2) HB0(1, 2) HA(0, 1) HA(1, 1)                                                 \
+  HFROM_A("s48", 2) HFROM_B("s49", 3) HB0(0, 3) HB0(1, 3) HA(0, 2) HA(1, 2)                                                 \
+  "s_cmp_eq_u32 s47, 0\n\ts_cbranch_scc1 2f\n\t"                                                                                \
+  "1:\n\t" HPHASE0(HON, 24) HPHASE1(HON, 20) NEXT_STEP HNEXT_PLACES                                                             \
+  "s_sub_u32 s47, s47, 1\n\ts_cmp_lg_u32 s47, 0\n\ts_cbranch_scc1 1b\n\t"                                                       \
+  "2:\n\t" HPHASE0(HOFF, 24) HPHASE1(HOFF, 16) HNEXT_PLACES HPHASE0(HOFF, 12) HPHASE1(HOFF, 4) HNEXT_PLACES HPHASE0(HOFF, 0)    \
+  HLAST "s_nop 15\n\ts_nop 7\n\t"
+
 // RING_PLAIN: C (f32) straight from the accumulators, with the biases of grouped products.  RING_SIGMOID: sigmoid(A . B)
 // as the next product's operand, whole rows of c16_pitch bf16 values with zeros past the last column.  RING_SILU, RING_GELU: half the tile's B rows are gate_proj's, half up_proj's;
 // act(gate) * up, 128 columns a tile, as bf16.  (GemmDesc says what each field means.)
 enum { RING_PLAIN, RING_SIGMOID, RING_SILU, RING_GELU };
-template <int KIND>
+// AH: halves of 128 rows to a tile, two or (RING_SILU, RING_GELU) one.
+template <int KIND, int AH>
 __global__ void __launch_bounds__(256, 1) gemm_bf16_ring_kernel(GemmDesc g) {
   constexpr bool GATED = KIND == RING_SILU || KIND == RING_GELU;
   constexpr uint32_t BNO = GATED ? 128 : 256;  // output columns of a tile
   warm_kernel_arguments<sizeof(GemmDesc)>();
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), wm = wave >> 1, wn = wave & 1;
-  const uint32_t tiles_m = (g.M + 255) / 256, tiles_n = (g.N + BNO - 1) / BNO;
+  constexpr uint32_t BM = AH * 128;
+  static_assert(AH == 2 || GATED, "the epilogues of 128-row tiles");
+  const uint32_t tiles_m = (g.M + BM - 1) / BM, tiles_n = (g.N + BNO - 1) / BNO;
   const uint32_t per_batch = tiles_m * tiles_n, batch = g.nb0 * g.nb1;
   // every XCD a contiguous range of tiles, in groups of four tile rows: as in gemm_bf16_dma_kernel
   uint32_t id = blockIdx.x;
@@ -195,7 +262,7 @@ __global__ void __launch_bounds__(256, 1) gemm_bf16_ring_kernel(GemmDesc g) {
   constexpr uint32_t GM = 4;
   const uint32_t first_m = t / (GM * tiles_n) * GM, gsz = min(tiles_m - first_m, GM);
   const uint32_t tg = t % (GM * tiles_n);
-  const uint32_t m0 = (first_m + tg % gsz) * 256;
+  const uint32_t m0 = (first_m + tg % gsz) * BM;
   uint32_t n0 = tg / gsz * BNO, Nl = g.N;
   const uint16_t *B = (const uint16_t *)g.b + b0 * g.sb_b0 + b1 * g.sb_b1;
   float *C = (g.splits > 1 ? g.workspace + (uint64_t)split * batch * g.M * g.N : g.c) + (uint64_t)bz * g.M * g.N;
@@ -240,17 +307,18 @@ __global__ void __launch_bounds__(256, 1) gemm_bf16_ring_kernel(GemmDesc g) {
       [dA12] "v"(dA1[2]), [dA13] "v"(dA1[3]), [dB00] "v"(dB0[0]), [dB01] "v"(dB0[1]), [dB02] "v"(dB0[2]),                  \
       [dB03] "v"(dB0[3]), [dB10] "v"(dB1[0]), [dB11] "v"(dB1[1]), [dB12] "v"(dB1[2]), [dB13] "v"(dB1[3]), [pa] "s"(sa0),   \
       [pb0] "s"(sb0), [pb1] "s"(sb1), [lds] "s"(lds)
-#define RING_SCALARS "s40", "s41", "s42", "s43", "s44", "s45", "s46", "s47", "m0", "scc", "memory"
+#define RING_SCALARS "s54", "s40", "s41", "s42", "s43", "s44", "s45", "s46", "s47", "m0", "scc", "memory"
 #define RING_V10(d) "v" #d "0", "v" #d "1", "v" #d "2", "v" #d "3", "v" #d "4", "v" #d "5", "v" #d "6", "v" #d "7", "v" #d "8", "v" #d "9"
 #define RING_FRAGMENTS                                                                                                     \
   "v128", "v129", RING_V10(13), RING_V10(14), RING_V10(15), RING_V10(16), RING_V10(17), RING_V10(18), RING_V10(19),        \
       RING_V10(20), RING_V10(21), RING_V10(22), RING_V10(23), RING_V10(24), "v250", "v251", "v252", "v253", "v254", "v255"
-  asm volatile(FIRST_LOADS::RING_IN : RING_SCALARS);
+  if constexpr (AH == 2) asm volatile(FIRST_LOADS::RING_IN : RING_SCALARS);
+  else asm volatile(HFIRST_LOADS::RING_IN : RING_SCALARS);
   float zero;
   asm volatile("v_mov_b32 %0, 0" : "=v"(zero));  // (the accumulators are cleared behind the first loads, not in front of them)
-  f32x16 acc[2][2][2][2];  // [A half][B half][row block][column block]
+  f32x16 acc[AH][2][2][2];  // [A half][B half][row block][column block]
 #pragma unroll
-  for (int q = 0; q < 16; ++q)
+  for (int q = 0; q < AH * 8; ++q)
 #pragma unroll
     for (int e = 0; e < 16; ++e) acc[q >> 3][(q >> 2) & 1][(q >> 1) & 1][q & 1][e] = zero;
   const uint32_t half = lane >> 5;
@@ -267,13 +335,22 @@ __global__ void __launch_bounds__(256, 1) gemm_bf16_ring_kernel(GemmDesc g) {
     real0 = __builtin_amdgcn_s_memrealtime();
   }
 #define RING_ACC(a, b, i, j) [c##a##b##i##j] "+a"(acc[a][b][i][j])
-#define RING_INOUT                                                                                                       \
+#define RING_ACC0                                                                                                        \
   RING_ACC(0, 0, 0, 0), RING_ACC(0, 0, 0, 1), RING_ACC(0, 0, 1, 0), RING_ACC(0, 0, 1, 1), RING_ACC(0, 1, 0, 0),          \
-      RING_ACC(0, 1, 0, 1), RING_ACC(0, 1, 1, 0), RING_ACC(0, 1, 1, 1), RING_ACC(1, 0, 0, 0), RING_ACC(1, 0, 0, 1),      \
-      RING_ACC(1, 0, 1, 0), RING_ACC(1, 0, 1, 1), RING_ACC(1, 1, 0, 0), RING_ACC(1, 1, 0, 1), RING_ACC(1, 1, 1, 0),      \
-      RING_ACC(1, 1, 1, 1), [ra0] "+v"(ra[0]), [ra1] "+v"(ra[1]), [ra2] "+v"(ra[2]), [ra3] "+v"(ra[3]), [rb0] "+v"(rb[0]), \
-      [rb1] "+v"(rb[1]), [rb2] "+v"(rb[2]), [rb3] "+v"(rb[3])
-  asm volatile(MAIN_LOOP : RING_INOUT : RING_IN, [n] "s"(n_steps) : RING_SCALARS, RING_FRAGMENTS);
+      RING_ACC(0, 1, 0, 1), RING_ACC(0, 1, 1, 0), RING_ACC(0, 1, 1, 1)
+#define RING_ACC1                                                                                                        \
+  RING_ACC(1, 0, 0, 0), RING_ACC(1, 0, 0, 1), RING_ACC(1, 0, 1, 0), RING_ACC(1, 0, 1, 1), RING_ACC(1, 1, 0, 0),          \
+      RING_ACC(1, 1, 0, 1), RING_ACC(1, 1, 1, 0), RING_ACC(1, 1, 1, 1)
+#define RING_PLACES                                                                                                      \
+  [ra0] "+v"(ra[0]), [ra1] "+v"(ra[1]), [ra2] "+v"(ra[2]), [ra3] "+v"(ra[3]), [rb0] "+v"(rb[0]), [rb1] "+v"(rb[1]),      \
+      [rb2] "+v"(rb[2]), [rb3] "+v"(rb[3])
+  if constexpr (AH == 2)
+    asm volatile(MAIN_LOOP : RING_ACC0, RING_ACC1, RING_PLACES : RING_IN, [n] "s"(n_steps) : RING_SCALARS, RING_FRAGMENTS);
+  else
+    asm volatile(HMAIN_LOOP
+                 : RING_ACC0, RING_PLACES
+                 : RING_IN, [n] "s"(n_steps)
+                 : RING_SCALARS, RING_FRAGMENTS, "v126", "v127", "s48", "s49", "s50", "s51", "s52", "s53");
   if (KIND == RING_PLAIN && g.clock_ticks && tid == 0) {
     atomicAdd(g.clock_ticks, __builtin_amdgcn_s_memtime() - tick0);
     atomicAdd(g.clock_ticks + 1, __builtin_amdgcn_s_memrealtime() - real0);
@@ -285,14 +362,14 @@ __global__ void __launch_bounds__(256, 1) gemm_bf16_ring_kernel(GemmDesc g) {
   __syncthreads();  // every wavefront has read its last fragments
   extern __shared__ __attribute__((aligned(16))) float ring_smem[];
   uint16_t *C16 = g.c16 ? g.c16 + (uint64_t)bz * g.M * g.N : nullptr;
-  const bool whole = m0 + 256 <= g.M && n0 + BNO <= Nl && !Bias;
+  const bool whole = m0 + BM <= g.M && n0 + BNO <= Nl && !Bias;
   constexpr bool F32 = KIND == RING_PLAIN;
   const uint32_t pitch = KIND == RING_SIGMOID ? g.c16_pitch : Nl;
   uint32_t to[4];  // where this lane's piece of rows 0-3, 4-7, 8-11, 12-15 of a quadrant goes, in bytes from its corner
 #pragma unroll
   for (int u = 0; u < 4; ++u) to[u] = ((u * 4 + (lane >> 4)) * pitch + (((lane & 15) ^ (u * 4 + (lane >> 4))) << 2)) * (F32 ? 4u : 2u);
 #pragma unroll
-  for (int qd = 0; qd < (GATED ? 2 : 4); ++qd) {
+  for (int qd = 0; qd < (GATED ? AH : 4); ++qd) {
     const int a = GATED ? qd : qd >> 1, b = GATED ? 0 : qd & 1;
     float *tile = ring_smem + wave * 8192 + (qd & 1) * 4096;
     const uint32_t col0 = n0 + b * 128 + wn * 64, row0 = m0 + a * 128 + wm * 64;
@@ -356,21 +433,27 @@ bool gemm_ring_ok(const GemmDesc &g) {
          (!g.dual_b || (g.c16 && !g.c));
 }
 
-template <int KIND>
+template <int KIND, int AH = 2>
 static hipError_t launch_ring_as(const LaunchCtx &lc, const GemmDesc &g, uint32_t grid) {
-  constexpr int smem = 2 * 65536;
+  constexpr int smem = AH == 2 ? 2 * 65536 : 10 * 16384;
   static bool configured = false;  // one attribute call per kernel and process
   if (!configured) {
-    hipError_t e = hipFuncSetAttribute((const void *)gemm_bf16_ring_kernel<KIND>, hipFuncAttributeMaxDynamicSharedMemorySize, smem);
+    hipError_t e = hipFuncSetAttribute((const void *)gemm_bf16_ring_kernel<KIND, AH>, hipFuncAttributeMaxDynamicSharedMemorySize, smem);
     if (e != hipSuccess) return e;
     configured = true;
   }
-  cg_launch(lc, gemm_bf16_ring_kernel<KIND>, dim3(grid), dim3(256), smem, g);
+  cg_launch(lc, gemm_bf16_ring_kernel<KIND, AH>, dim3(grid), dim3(256), smem, g);
   return hipGetLastError();
 }
 
-hipError_t launch_gemm_ring(const LaunchCtx &lc, const GemmDesc &g) {
+hipError_t launch_gemm_ring(const LaunchCtx &lc, const GemmDesc &g, bool half_height) {
   if (!gemm_ring_ok(g)) return hipErrorInvalidValue;
+  if (half_height) {
+    if (!g.dual_b || g.splits > 1 || g.K < 192) return hipErrorInvalidValue;
+    const uint64_t tiles = (uint64_t)((g.M + 127) / 128) * ((g.N + 127) / 128) * g.nb0 * g.nb1;
+    if (tiles > 0x7FFFFFFFull) return hipErrorInvalidValue;
+    return g.glu_kind ? launch_ring_as<RING_GELU, 1>(lc, g, (uint32_t)tiles) : launch_ring_as<RING_SILU, 1>(lc, g, (uint32_t)tiles);
+  }
   const uint32_t bno = g.dual_b ? 128 : 256, batch = g.nb0 * g.nb1 * (g.splits > 1 ? g.splits : 1);
   const uint64_t grid = (uint64_t)((g.M + 255) / 256) * ((g.N + bno - 1) / bno) * batch;
   if (grid > 0x7FFFFFFFull) return hipErrorInvalidValue;

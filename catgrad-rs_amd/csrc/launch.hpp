@@ -359,9 +359,10 @@ struct GemmDesc {
   // the 100 MHz ticks its main loop took to clock_ticks[0] and [1]
   unsigned long long *clock_ticks;
 };
-// k_gemm_ring.hip: the 256 x 256 tiles of large bf16 products (plain or grouped, sigmoid, stacked gate / up)
+// k_gemm_ring.hip: the 256 x 256 tiles of large bf16 products (plain or grouped, sigmoid, stacked gate / up);
+// half_height: the stacked gate / up of fewer rows on tiles of 128 x 256, K >= 192
 bool gemm_ring_ok(const GemmDesc &g);
-hipError_t launch_gemm_ring(const LaunchCtx &lc, const GemmDesc &g);
+hipError_t launch_gemm_ring(const LaunchCtx &lc, const GemmDesc &g, bool half_height = false);
 // split factor launch_matmul should be given for this problem (1 = none)
 uint32_t gemm_split_k(const LaunchCtx &lc, const GemmDesc &g);
 // whether launch_matmul would run this problem (splits as given) on the kernel that honours

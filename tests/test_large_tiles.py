@@ -1,9 +1,12 @@
-"""bf16 products that fill the chip with 256 x 256 tiles (gemm_bf16_ring_kernel): two k-steps, an odd number, many; rows and
-columns that end inside a tile and rows of a length that is no multiple of 16 bytes; the stacked gate / up form with either
-activation; grouped products with and without a bias; a sigmoid stored as the next product's operand."""
+"""bf16 products whose main loop is one statement of assembly (gemm_bf16_ring_kernel, mfma_step_ring.hpp): the fewest k-steps
+each takes, an odd number, many; rows and columns that end inside a tile and rows of a length that is no multiple of 16 bytes;
+the stacked gate / up form with either activation; grouped products with and without a bias, and rotated; a sigmoid stored as
+the next product's operand."""
 import numpy as np
 import pytest
 
+import test_llama_parity as llama_tests
+import test_moe_gemma_parity as moe_tests
 import vectors
 
 lang, nn = vectors.cg.lang, vectors.cg.nn
@@ -24,8 +27,12 @@ def product_and_bound(x, w):
     return x @ w.T, x.shape[-1] * 2.0 ** -24 * (np.abs(x) @ np.abs(w).T)
 
 
+# 256 x 256 tiles; then 128 x 128 in one round of 33 and 17 steps and in two rounds, 192 x 128 in one round of 4, 5 and 32 steps
+# and in two rounds
 @pytest.mark.gpu
-@pytest.mark.parametrize("M,N,K", [(4096, 4096, 128), (4097, 4101, 192), (3841, 4353, 256), (8300, 2049, 320), (255, 65600, 448)])
+@pytest.mark.parametrize("M,N,K", [(4096, 4096, 128), (4097, 4101, 192), (3841, 4353, 256), (8300, 2049, 320), (255, 65600, 448),
+                                   (1500, 2050, 2112), (1400, 1410, 1088), (3100, 2050, 4160),
+                                   (2300, 2050, 256), (2303, 2049, 320), (2305, 2048, 2048), (4200, 2050, 4096)])
 def test_product(hip_bf16, M, N, K):
     g = np.random.default_rng(M)
     x, w = draw(g, (1, M, K)), draw(g, (N, K))
@@ -53,7 +60,8 @@ def test_grouped_products(hip_bf16, M, K, bias):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("act", ["silu", "gelu"])
-@pytest.mark.parametrize("M,F,K", [(4096, 2048, 128), (4100, 2052, 192), (3900, 2184, 320)])
+@pytest.mark.parametrize("M,F,K", [(4096, 2048, 128), (4100, 2052, 192), (3900, 2184, 320),    # tiles of 256 rows
+                                   (1030, 2180, 192), (900, 3000, 256), (1000, 2820, 512)])    # and of 128: three steps, four, more
 def test_gated(hip_bf16, M, F, K, act):
     g = np.random.default_rng(F)
     x, wg, wu, wd = draw(g, (1, M, K)), draw(g, (F, K), K ** -0.5), draw(g, (F, K), K ** -0.5), np.eye(64, F, dtype=np.float32)
@@ -80,3 +88,16 @@ def test_sigmoid_as_the_next_operand(hip_bf16, M, K, H):
     (got,) = vectors.run(hip_bf16, lambda b, x, w1, w2: [lang.matmul(b, nn.sigmoid(b, lang.matmul(b, x, w1)), w2)], 1, x, w1, w2)
     ref = 1 / (1 + np.exp(-(x.astype(np.float64) @ w1[:, H - 64:].astype(np.float64))))
     assert np.all(np.abs(got - ref) <= 2.0 ** -8 * ref + 1e-5)    # (as above)
+
+
+# one round of 128-row tiles and one of 192-row tiles that rotate, heads of 64 and of 128, with and without biases, several
+# sequences, positions in no multiple of four
+@pytest.mark.gpu
+def test_rotated(oracle, hip_bf16):
+    llama_tests.test_llama_prefill_rotates_in_the_projections_launch(oracle, hip_bf16, 1601, 16, 16, 1)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("batch,tokens", [(2, 301), (3, 550)])
+def test_rotated_wide_heads(oracle, hip_bf16, batch, tokens):
+    moe_tests.test_qwen_prefill_biases_and_rotation_in_the_projections_launch(oracle, hip_bf16, batch, tokens, 8, 8, 128)
