@@ -580,6 +580,7 @@ __global__ void __launch_bounds__(WR *WC *KG * 64) gemm_bf16_dma_kernel(GemmDesc
   const uint32_t pair_hd = PAIRS ? g.rope_hd : 64, pair_0 = PAIRS ? n0 / pair_hd * pair_hd + n0 % pair_hd / 2 : 0;
   auto column = [&](uint32_t cl) { return PAIRS ? pair_0 + (cl & 15) + (cl >> 4) * (pair_hd / 2) : n0 + cl; };
   const float *Bias = g.n_group ? g.grp_bias[grp] : nullptr;
+  const float *Cadd = !ROPE && !EPI && g.c_add && g.splits <= 1 ? g.c_add + (uint64_t)bz * g.M * g.N : nullptr;
   const float *Gate = g.glu_gate ? g.glu_gate + (uint64_t)bz * g.M * g.N : nullptr;  // only without split-K
   uint16_t *C16 = g.c16 ? g.c16 + (uint64_t)bz * g.M * g.N : nullptr;
   const uint32_t k_begin = split * g.k_per_split;
@@ -954,6 +955,20 @@ __global__ void __launch_bounds__(WR *WC *KG * 64) gemm_bf16_dma_kernel(GemmDesc
         for (int e = 0; e < 16; ++e) {
           const uint32_t row = m0 + wm * WM + i * 32 + (e >> 2) * 8 + (lane >> 5) * 4 + (e & 3);
           if (row < g.M && col < Nl) C[(uint64_t)row * Nl + col] = acc[i][j][e] + bv;
+        }
+        continue;
+      }
+      if (Cadd) {  // (all sixteen on their way before the first is used; positions clamped)
+        float add[16];
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+          const uint32_t row = m0 + wm * WM + i * 32 + (e >> 2) * 8 + (lane >> 5) * 4 + (e & 3);
+          add[e] = Cadd[(uint64_t)min(row, g.M - 1) * Nl + min(col, Nl - 1)];
+        }
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+          const uint32_t row = m0 + wm * WM + i * 32 + (e >> 2) * 8 + (lane >> 5) * 4 + (e & 3);
+          if (row < g.M && col < Nl) C[(uint64_t)row * Nl + col] = acc[i][j][e] + add[e];
         }
         continue;
       }
@@ -2874,6 +2889,17 @@ bool gemm_epilogue_ok(const GemmDesc &g) {
          (g.N % 4 == 0 || g.c16_pitch);
 }
 
+// More than 64 rows on the direct-to-LDS kernels, not split along k: every plain tile adds c_add as it stores.
+bool gemm_add_ok(const GemmDesc &g) {
+  GemmDesc t = g;
+  t.c_add = nullptr;
+  const int asz = g.a_stype == ST_BF16 ? 2 : 4, bsz = g.b_stype == ST_BF16 ? 2 : 4;
+  const int av = vec_ok(g.a, asz, g.sak == 1 ? g.sam : g.sak, g.sa_b0, g.sa_b1);
+  const int bv = vec_ok(g.b, bsz, g.sbk == 1 ? g.sbn : g.sbk, g.sb_b0, g.sb_b1);
+  return g.M > 64 && g.splits <= 1 && !g.n_group && !g.dual_b && !g.glu_gate && !g.c16 && !g.act_sigmoid && !g.b_index &&
+         gemm_fast_path(t, av, bv) && gemm_dma_ok(t);
+}
+
 bool gemv_rows_plain_ok(const LaunchCtx &lc, const GemmDesc &g);
 bool gemm_act_ok(const LaunchCtx &lc, const GemmDesc &g) {
   if (g.b_index || g.c_add || g.n_group || g.dual_b || g.glu_gate || g.defer_reduce || !g.K || g.M <= 8) return false;
@@ -3023,10 +3049,10 @@ hipError_t launch_matmul(const LaunchCtx &lc_in, const GemmDesc &g, const char *
   const int av = vec_ok(g.a, asz, a_unit_k ? (g.M == 1 ? 0 : g.sam) : (g.K == 1 ? 0 : g.sak), g.sa_b0, g.sa_b1);
   const int bv = vec_ok(g.b, bsz, b_unit_k ? (g.N == 1 ? 0 : g.sbn) : (g.K == 1 ? 0 : g.sbk),
                         g.b_index ? g.sb_index : g.sb_b0, g.sb_b1);
-  // only the one-row kernels follow b_index and c_add (and the k-slice sum of a split GEMM adds c_add)
+  // only the one-row kernels follow b_index; they add c_add, and so do the k-slice sum of a split GEMM and gemm_add_ok's tiles
   const bool one_row = g.M <= 8 && g.a_stype == ST_F32 && g.K > 0 && (b_unit_k || b_unit_n);
   if (g.b_index && !one_row) return hipErrorInvalidValue;
-  if (g.c_add && !one_row && g.splits <= 1) return hipErrorInvalidValue;
+  if (g.c_add && !one_row && g.splits <= 1 && !gemm_add_ok(g)) return hipErrorInvalidValue;
   if ((g.glu_gate || g.c16 || g.n_group || g.dual_b) && !gemm_epilogue_ok(g)) return hipErrorInvalidValue;
   if (g.act_sigmoid && !gemm_act_ok(lc_in, g)) return hipErrorInvalidValue;
   if (g.rope_s && !gemm_rope_epilogue_ok(lc_in, g)) return hipErrorInvalidValue;
@@ -3182,6 +3208,7 @@ hipError_t launch_matmul(const LaunchCtx &lc_in, const GemmDesc &g, const char *
           rest.M = g.M - lead.M;
           rest.a = (const uint16_t *)g.a + (int64_t)lead.M * g.sam;
           rest.c = g.c + (uint64_t)lead.M * g.N;
+          if (g.c_add) rest.c_add = g.c_add + (uint64_t)lead.M * g.N;
           LaunchCtx first = lc, second = lc_in;
           first.ev_stop = nullptr;
           second.ev_start = nullptr;

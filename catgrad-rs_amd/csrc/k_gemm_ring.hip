@@ -266,7 +266,7 @@ __global__ void __launch_bounds__(256, 1) gemm_bf16_ring_kernel(GemmDesc g) {
   uint32_t n0 = tg / gsz * BNO, Nl = g.N;
   const uint16_t *B = (const uint16_t *)g.b + b0 * g.sb_b0 + b1 * g.sb_b1;
   float *C = (g.splits > 1 ? g.workspace + (uint64_t)split * batch * g.M * g.N : g.c) + (uint64_t)bz * g.M * g.N;
-  const float *Bias = nullptr;
+  const float *Bias = nullptr, *Cadd = KIND == RING_PLAIN && g.c_add && g.splits <= 1 ? g.c_add + (uint64_t)bz * g.M * g.N : nullptr;
   if (KIND == RING_PLAIN && g.n_group) {  // grouped products: tiles never straddle two
     uint32_t p = 0;
     while (p + 1 < g.n_group && n0 >= g.grp_n[p]) {
@@ -393,6 +393,14 @@ __global__ void __launch_bounds__(256, 1) gemm_bf16_ring_kernel(GemmDesc g) {
       float4 out[16];
 #pragma unroll
       for (int it = 0; it < 16; ++it) out[it] = *(const float4 *)(from + it * 256);
+      if (F32 && Cadd) {
+        const char *corner = (const char *)(Cadd + (uint64_t)row0 * Nl + col0);
+        float4 add[16];
+#pragma unroll
+        for (int it = 0; it < 16; ++it) __builtin_memcpy(&add[it], corner + (uint64_t)(it >> 2) * 16 * pitch * 4 + to[it & 3], 16);
+#pragma unroll
+        for (int it = 0; it < 16; ++it) { out[it].x += add[it].x; out[it].y += add[it].y; out[it].z += add[it].z; out[it].w += add[it].w; }
+      }
       char *corner = F32 ? (char *)(C + (uint64_t)row0 * Nl + col0) : (char *)(C16 + (uint64_t)row0 * pitch + col0);
 #pragma unroll
       for (int it = 0; it < 16; ++it) {
@@ -415,7 +423,7 @@ __global__ void __launch_bounds__(256, 1) gemm_bf16_ring_kernel(GemmDesc g) {
         const float e[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
         for (int k = 0; k < 4; ++k)
-          if (col + k < Nl) c[k] = Bias ? e[k] + Bias[col + k] : e[k];
+          if (col + k < Nl) c[k] = Bias ? e[k] + Bias[col + k] : Cadd ? e[k] + Cadd[(uint64_t)row * Nl + col + k] : e[k];
       } else if (col < pitch) {  // (N % 4 == 0, or padded rows: a piece is inside or outside; zeros past the last column)
         v = make_float4(col < Nl ? v.x : 0.f, col + 1 < Nl ? v.y : 0.f, col + 2 < Nl ? v.z : 0.f, col + 3 < Nl ? v.w : 0.f);
         *(uint2 *)(C16 + (uint64_t)row * pitch + col) = bf16_pack4(v);

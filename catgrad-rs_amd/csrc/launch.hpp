@@ -305,7 +305,7 @@ struct GemmDesc {
   // split-K (bf16 fast path only): partial products go to workspace[split][batch][M][N]
   float *workspace;
   uint32_t splits, k_per_split;
-  // optional epilogue of the one-row kernels: C = A . B + c_add (c_add laid out like C)
+  // optional (the one-row kernels, the sum of k-slices, gemm_add_ok): C = A . B + c_add (c_add laid out like C)
   const float *c_add;
   // split along k (splits > 1): leave the slices in the workspace; the caller sums them (launch_splitk_sum, or
   // the RMSNorm kernel on its way in)
@@ -368,6 +368,8 @@ uint32_t gemm_split_k(const LaunchCtx &lc, const GemmDesc &g);
 // whether launch_matmul would run this problem (splits as given) on the kernel that honours
 // glu_gate / c16
 bool gemm_epilogue_ok(const GemmDesc &g);
+// whether launch_matmul's kernel for a problem that is not split along k adds c_add (many rows)
+bool gemm_add_ok(const GemmDesc &g);
 // whether launch_matmul's kernel for this problem (splits as given) honours act_sigmoid
 bool gemm_act_ok(const LaunchCtx &lc, const GemmDesc &g);
 // whether a bf16-mode product is worth copies of its operands in the direct-to-LDS kernel's layout (epilogue: it has one

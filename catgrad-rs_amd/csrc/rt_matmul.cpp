@@ -1145,6 +1145,12 @@ int realize_matmul(cg_backend *be, cg_tensor *n, cg_tensor *addend, bool *added,
         if (be->ksum_request && n->size() % 4 == 0 && n->offset == 0) g.defer_reduce = 1;
       }
     }
+    // A product that is not split along k adds the residual as it stores (2900 rows of 2048: an add of its own reads and
+    // writes 72 MB, 11 us at either block end; here it reads 24).
+    if (splits <= 1 && addend && !be->addend_is_row && !*added && !ep && group.empty() && !g.c_add && gemm_add_ok(g)) {
+      g.c_add = (const float *)data_ptr(addend);
+      *added = true;
+    }
     if (dual) {
       if (!g.c_add && batch == 1 && !ex.w && g.sbk == 1 && g.b_stype == ST_BF16 && gemm_epilogue_ok(g)) {
         g.dual_b = g.b;  // this product is up_proj's; the activation goes on the other one

@@ -41,6 +41,29 @@ def test_product(hip_bf16, M, N, K):
     assert np.all(np.abs(got[0] - ref) <= bound)
 
 
+# a residual added as the product is stored: each tile that does so, whole rounds of large tiles with the rest on smaller ones,
+# a batch, and the forms that leave the add to someone else (64 rows, k-slices)
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,M,N,K", [(1, 4097, 4101, 192), (1, 8300, 2050, 2048), (1, 1500, 2050, 2112), (1, 2303, 2049, 320), (1, 3100, 2050, 1024),
+                                     (1, 3300, 2050, 2048), (1, 300, 130, 64), (1, 1000, 1000, 256), (3, 700, 520, 192), (1, 64, 200, 128),
+                                     (1, 200, 300, 2048)])
+def test_product_and_residual(hip_bf16, B, M, N, K):
+    g = np.random.default_rng(M)
+    x, w, r = draw(g, (B, M, K)), draw(g, (N, K) if B == 1 else (B, N, K)), draw(g, (B, M, N), 3.0)
+
+    def f(b, x, w, r):
+        r = r + r - r       # (f32, like a stream of residuals, and read by others too)
+        return [r + (linear(b, x, w, N, K) if B == 1 else lang.matmul(b, x, lang.transpose(b, 1, 2, w))), r]
+    hip_bf16.launch_counts(reset=True)
+    got, _ = vectors.run(hip_bf16, f, 2, x, w, r)
+    counts = hip_bf16.launch_counts(reset=True)
+    assert counts.get("gemm") == 1 and counts.get("ew_fused") == 1 and (M <= 64) == ("binary_f32" in counts), counts     # (ew_fused: r)
+    for i in range(B):
+        ref, bound = product_and_bound(x[i], w if B == 1 else w[i])
+        ref = ref + r[i]
+        assert np.all(np.abs(got[i] - ref) <= bound + 2.0 ** -24 * (np.abs(ref) + bound))
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("bias", [False, True])
 @pytest.mark.parametrize("M,K", [(21900, 128), (22016, 192)])
