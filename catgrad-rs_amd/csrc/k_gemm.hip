@@ -2710,6 +2710,7 @@ hipError_t launch_moe_gemm(const LaunchCtx &lc, const MoeGemmDesc &g) {
     const dim3 grid((max_n + 127) / 128 * (g.route_tiles ? moe_route_max_tiles(g) : g.n_expert), 1, 1);
     return g.fuse_glu ? launch_moe_gemm_dma<2, 3, true>(lc, g, grid) : launch_moe_gemm_dma<1, 3, true>(lc, g, grid);
   }
+  if (moe_ring_ok(g)) return launch_moe_ring(lc, g);
   if (g.fuse_glu) {
     if (g.n_prob != 2 || g.prob[0].N != g.prob[1].N || g.pro != PRO_NONE) return hipErrorInvalidValue;
     if (moe_gemm_pipelined_ok(g))

@@ -189,6 +189,8 @@ typedef __attribute__((ext_vector_type(16))) float f32x16;
 #define HB0(r, ks) HRD(B0, "v127", r, ks)
 #define HB1(r, ks) HRD(B1, "v127", r, ks)
 #define HM0(i) "s_add_u32 m0, s54, " #i "*1024\n\t"
+// (rows of A may be gathered: a pointer to each lane's)
+#define HLOAD_A(i) "global_load_lds_dwordx4 %[ga" #i "], off\n\tv_lshl_add_u64 %[ga" #i "], %[ga" #i "], 0, s[58:59]\n\t"
 #define HON(x) x
 #define HOFF(x) ""
 #define HSYNC(v) "s_waitcnt vmcnt(" #v ")\n\ts_barrier\n\t"
@@ -197,10 +199,10 @@ typedef __attribute__((ext_vector_type(16))) float f32x16;
 #define HPHASE0(G, v)                                                                                                              \
   G("s_add_u32 s54, s53, %[lds]\n\t") HSYNC(v)                                                                                     \
   HFROM_A("s48", 3) HFROM_B("s50", 0)                                                                                              \
-  HSLICE(0, B0, 0, READS_BUT(8), HA(0, 3) G(HM0(0)), HA(1, 3) G(LOAD(A0, 0)), HB1(0, 0), HB1(1, 0)) HFROM_B("s50", 1)          \
-  HSLICE(0, B0, 1, READS_BUT(8), HB1(0, 1) G(HM0(1)), HB1(1, 1) G(LOAD(A0, 1)), "", "") HFROM_B("s50", 2)                          \
-  HSLICE(0, B0, 2, READS_BUT(6), HB1(0, 2) G(HM0(2)), HB1(1, 2) G(LOAD(A0, 2)), "", "") HFROM_B("s50", 3)                          \
-  HSLICE(0, B0, 3, READS_BUT(6), HB1(0, 3) G(HM0(3)), HB1(1, 3) G(LOAD(A0, 3)), "", "")
+  HSLICE(0, B0, 0, READS_BUT(8), HA(0, 3) G(HM0(0)), HA(1, 3) G(HLOAD_A(0)), HB1(0, 0), HB1(1, 0)) HFROM_B("s50", 1)          \
+  HSLICE(0, B0, 1, READS_BUT(8), HB1(0, 1) G(HM0(1)), HB1(1, 1) G(HLOAD_A(1)), "", "") HFROM_B("s50", 2)                          \
+  HSLICE(0, B0, 2, READS_BUT(6), HB1(0, 2) G(HM0(2)), HB1(1, 2) G(HLOAD_A(2)), "", "") HFROM_B("s50", 3)                          \
+  HSLICE(0, B0, 3, READS_BUT(6), HB1(0, 3) G(HM0(3)), HB1(1, 3) G(HLOAD_A(3)), "", "")
 #define HPHASE1(G, v)                                                                                                              \
   G("s_add_u32 s54, s48, %[lds]\n\t") HSYNC(v)                                                                                     \
   HFROM_B("s52", 0)                                                                                                                \
@@ -218,21 +220,26 @@ typedef __attribute__((ext_vector_type(16))) float f32x16;
 #define HNEXT(x, y) "s_add_u32 " x ", " y ", 16384\n\ts_cmp_eq_u32 " x ", 163840\n\ts_cselect_b32 " x ", 0, " x "\n\t"
 #define HNEXT_PLACES \
   "s_mov_b32 s53, s50\n\ts_mov_b32 s48, s51\n\ts_mov_b32 s49, s52\n\t" HNEXT("s50", "s52") HNEXT("s51", "s50") HNEXT("s52", "s51")
-#define HLOAD_UNIT(U) HM0(0) "s_nop 0\n\t" LOAD(U, 0) HM0(1) "s_nop 0\n\t" LOAD(U, 1) HM0(2) "s_nop 0\n\t" LOAD(U, 2) HM0(3) "s_nop 0\n\t" LOAD(U, 3)
-#define HPOINTERS "s_mov_b64 s[40:41], %[pa]\n\ts_mov_b64 s[42:43], %[pb0]\n\ts_mov_b64 s[44:45], %[pb1]\n\t"
-#define HSTEP_LOADS HLOAD_UNIT(A0) "s_add_u32 s54, s54, 16384\n\t" HLOAD_UNIT(B0) "s_add_u32 s54, s54, 16384\n\t" HLOAD_UNIT(B1) "s_add_u32 s54, s54, 16384\n\t"
+#define HLOADS_A \
+  HM0(0) "s_nop 0\n\t" HLOAD_A(0) HM0(1) "s_nop 0\n\t" HLOAD_A(1) HM0(2) "s_nop 0\n\t" HLOAD_A(2) HM0(3) "s_nop 0\n\t" HLOAD_A(3)
+#define HLOADS_B(U) \
+  HM0(0) "s_nop 0\n\t" LOAD(U, 0) HM0(1) "s_nop 0\n\t" LOAD(U, 1) HM0(2) "s_nop 0\n\t" LOAD(U, 2) HM0(3) "s_nop 0\n\t" LOAD(U, 3)
+#define HPOINTERS "s_mov_b64 s[42:43], %[pb0]\n\ts_mov_b64 s[44:45], %[pb1]\n\ts_movk_i32 s58, 128\n\ts_mov_b32 s59, 0\n\t"
+#define HNEXT_STEP "s_add_u32 s42, s42, 128\n\ts_addc_u32 s43, s43, 0\n\ts_add_u32 s44, s44, 128\n\ts_addc_u32 s45, s45, 0\n\t"
+#define HSTEP_LOADS \
+  HLOADS_A "s_add_u32 s54, s54, 16384\n\t" HLOADS_B(B0) "s_add_u32 s54, s54, 16384\n\t" HLOADS_B(B1) "s_add_u32 s54, s54, 16384\n\t"
 // steps 0 to 2 requested: 36 loads
-#define HFIRST_LOADS HPOINTERS "s_mov_b32 s54, %[lds]\n\t" HSTEP_LOADS NEXT_STEP HSTEP_LOADS NEXT_STEP HSTEP_LOADS
+#define HFIRST_LOADS HPOINTERS "s_mov_b32 s54, %[lds]\n\t" HSTEP_LOADS HNEXT_STEP HSTEP_LOADS HNEXT_STEP HSTEP_LOADS
 // n >= 3 steps
 #define HMAIN_LOOP                                                                                                              \
-  HPOINTERS NEXT_STEP NEXT_STEP NEXT_STEP "s_sub_u32 s47, %[n], 3\n\t"                                                          \
+  HPOINTERS HNEXT_STEP HNEXT_STEP HNEXT_STEP "s_sub_u32 s47, %[n], 3\n\t"                                                          \
   "s_mov_b32 s48, 0\n\ts_movk_i32 s49, 0x4000\n\ts_mov_b32 s50, 0x8000\n\ts_mov_b32 s51, 0xC000\n\ts_mov_b32 s52, 0x10000\n\t"  \
   "s_mov_b32 s53, 0x24000\n\t" HSYNC(28)                                                                                        \
   HFROM_A("s48", 0) HFROM_B("s49", 0) HB0(0, 0) HB0(1, 0) HFROM_B("s49", 1) HB0(0, 1) HB0(1, 1) HA(0, 0) HA(1, 0)           \
   HFROM_A("s48", 1) HFROM_B("s49", 2) HB0(0, 2) HB0(1, 2) HA(0, 1) HA(1, 1)                                                 \
   HFROM_A("s48", 2) HFROM_B("s49", 3) HB0(0, 3) HB0(1, 3) HA(0, 2) HA(1, 2)                                                 \
   "s_cmp_eq_u32 s47, 0\n\ts_cbranch_scc1 2f\n\t"                                                                                \
-  "1:\n\t" HPHASE0(HON, 24) HPHASE1(HON, 20) NEXT_STEP HNEXT_PLACES                                                             \
+  "1:\n\t" HPHASE0(HON, 24) HPHASE1(HON, 20) HNEXT_STEP HNEXT_PLACES                                                             \
   "s_sub_u32 s47, s47, 1\n\ts_cmp_lg_u32 s47, 0\n\ts_cbranch_scc1 1b\n\t"                                                       \
   "2:\n\t" HPHASE0(HOFF, 24) HPHASE1(HOFF, 16) HNEXT_PLACES HPHASE0(HOFF, 12) HPHASE1(HOFF, 4) HNEXT_PLACES HPHASE0(HOFF, 0)    \
   HLAST "s_nop 15\n\ts_nop 7\n\t"
@@ -302,18 +309,24 @@ __global__ void __launch_bounds__(256, 1) gemm_bf16_ring_kernel(GemmDesc g) {
   };
   const uint64_t sa0 = scalar(pa), sb0 = scalar(pb0), sb1 = scalar(pb1);
   const uint32_t lds = wave * 4096;  // (all LDS of this kernel is the two stages, at offset 0)
+#define RING_IN_B                                                                                                         \
+  [dB00] "v"(dB0[0]), [dB01] "v"(dB0[1]), [dB02] "v"(dB0[2]), [dB03] "v"(dB0[3]), [dB10] "v"(dB1[0]), [dB11] "v"(dB1[1]), \
+      [dB12] "v"(dB1[2]), [dB13] "v"(dB1[3]), [pb0] "s"(sb0), [pb1] "s"(sb1), [lds] "s"(lds)
 #define RING_IN                                                                                                            \
   [dA00] "v"(dA0[0]), [dA01] "v"(dA0[1]), [dA02] "v"(dA0[2]), [dA03] "v"(dA0[3]), [dA10] "v"(dA1[0]), [dA11] "v"(dA1[1]),  \
-      [dA12] "v"(dA1[2]), [dA13] "v"(dA1[3]), [dB00] "v"(dB0[0]), [dB01] "v"(dB0[1]), [dB02] "v"(dB0[2]),                  \
-      [dB03] "v"(dB0[3]), [dB10] "v"(dB1[0]), [dB11] "v"(dB1[1]), [dB12] "v"(dB1[2]), [dB13] "v"(dB1[3]), [pa] "s"(sa0),   \
-      [pb0] "s"(sb0), [pb1] "s"(sb1), [lds] "s"(lds)
-#define RING_SCALARS "s54", "s40", "s41", "s42", "s43", "s44", "s45", "s46", "s47", "m0", "scc", "memory"
+      [dA12] "v"(dA1[2]), [dA13] "v"(dA1[3]), [pa] "s"(sa0), RING_IN_B
+#define RING_GATHERED [ga0] "+v"(ga[0]), [ga1] "+v"(ga[1]), [ga2] "+v"(ga[2]), [ga3] "+v"(ga[3])
+#define RING_HALF_SCALARS "v126", "v127", "s48", "s49", "s50", "s51", "s52", "s53"
+#define RING_SCALARS "s54", "s58", "s59", "s40", "s41", "s42", "s43", "s44", "s45", "s46", "s47", "m0", "scc", "memory"
 #define RING_V10(d) "v" #d "0", "v" #d "1", "v" #d "2", "v" #d "3", "v" #d "4", "v" #d "5", "v" #d "6", "v" #d "7", "v" #d "8", "v" #d "9"
 #define RING_FRAGMENTS                                                                                                     \
   "v128", "v129", RING_V10(13), RING_V10(14), RING_V10(15), RING_V10(16), RING_V10(17), RING_V10(18), RING_V10(19),        \
       RING_V10(20), RING_V10(21), RING_V10(22), RING_V10(23), RING_V10(24), "v250", "v251", "v252", "v253", "v254", "v255"
+  uint64_t ga[4];  // AH == 1: this lane's pieces of A, a step on after every load
+#pragma unroll
+  for (int i = 0; i < 4; ++i) ga[i] = (uint64_t)pa + dA0[i];
   if constexpr (AH == 2) asm volatile(FIRST_LOADS::RING_IN : RING_SCALARS);
-  else asm volatile(HFIRST_LOADS::RING_IN : RING_SCALARS);
+  else asm volatile(HFIRST_LOADS : RING_GATHERED : RING_IN_B : RING_SCALARS);
   float zero;
   asm volatile("v_mov_b32 %0, 0" : "=v"(zero));  // (the accumulators are cleared behind the first loads, not in front of them)
   f32x16 acc[AH][2][2][2];  // [A half][B half][row block][column block]
@@ -347,10 +360,7 @@ __global__ void __launch_bounds__(256, 1) gemm_bf16_ring_kernel(GemmDesc g) {
   if constexpr (AH == 2)
     asm volatile(MAIN_LOOP : RING_ACC0, RING_ACC1, RING_PLACES : RING_IN, [n] "s"(n_steps) : RING_SCALARS, RING_FRAGMENTS);
   else
-    asm volatile(HMAIN_LOOP
-                 : RING_ACC0, RING_PLACES
-                 : RING_IN, [n] "s"(n_steps)
-                 : RING_SCALARS, RING_FRAGMENTS, "v126", "v127", "s48", "s49", "s50", "s51", "s52", "s53");
+    asm volatile(HMAIN_LOOP : RING_ACC0, RING_PLACES, RING_GATHERED : RING_IN_B, [n] "s"(n_steps) : RING_SCALARS, RING_HALF_SCALARS, RING_FRAGMENTS);
   if (KIND == RING_PLAIN && g.clock_ticks && tid == 0) {
     atomicAdd(g.clock_ticks, __builtin_amdgcn_s_memtime() - tick0);
     atomicAdd(g.clock_ticks + 1, __builtin_amdgcn_s_memrealtime() - real0);
@@ -430,6 +440,150 @@ __global__ void __launch_bounds__(256, 1) gemm_bf16_ring_kernel(GemmDesc g) {
       }
     }
   }
+}
+
+// ---- the routed experts of a prefill: a row tile of 128 (slot, token) pairs of one expert by 256 weight rows ------------------
+// (MoeGemmDesc with route_tiles; the work and its order are those of moe_gemm_dma_kernel, which says how pairs are sorted.)
+// MOE_SILU, MOE_GELU: 128 rows of gate_proj and the same of up_proj, act(gate) * up leaves as bf16; MOE_PLAIN: 256 rows of one
+// matrix, f32.  Rows of A are gathered; pairs past the expert's last repeat it, and are not stored.
+// Bound by the stream of weights in pieces of 128 bytes, rows 4 KB apart (141 us for the load schedule of gate and up alone): 60
+// experts of 2 x 1408 x 2048, 4096 pairs in crowded experts and empty ones, 161 -> 148 us against moe_gemm_dma_kernel, 2048 x 1408
+// 92 -> 82 (streaming loads, which suit that kernel, 150 and 85).
+enum { MOE_PLAIN, MOE_SILU, MOE_GELU };
+template <int KIND>
+__global__ void __launch_bounds__(256, 1) moe_ring_kernel(MoeGemmDesc g) {
+  constexpr bool GATED = KIND != MOE_PLAIN;
+  constexpr uint32_t BNO = GATED ? 128 : 256;
+  warm_kernel_arguments<sizeof(MoeGemmDesc)>();
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), wm = wave >> 1, wn = wave & 1;
+  const uint32_t prob = GATED ? 0 : blockIdx.y, K = g.K, N = g.prob[prob].N;
+  const uint32_t tiles_n = (N + BNO - 1) / BNO, tile = blockIdx.x / tiles_n, n0 = (blockIdx.x - tile * tiles_n) * BNO;
+  if (tile >= g.route_tiles[0]) return;  // the grid is sized for the most tiles there can be, and the wider problem
+  const uint32_t entry = g.route_tiles[1 + tile], e = entry >> 16, m0 = (entry & 0xFFFFu) * 128;
+  if (e >= g.n_expert) return;
+  const uint32_t live = min(g.route_count[e] - m0, 128u), *list = g.route_list + g.route_offset[e] + m0;
+  const uint32_t n_steps = __builtin_amdgcn_readfirstlane(K / 64);
+  const int64_t sbn0 = g.prob[prob].sbn;
+  const uint16_t *pb0 = (const uint16_t *)g.prob[prob].w + (int64_t)e * g.sb_index + (int64_t)n0 * sbn0;
+  const uint16_t *pb1 = GATED ? (const uint16_t *)g.prob[1].w + (int64_t)e * g.sb_index + (int64_t)n0 * g.prob[1].sbn : pb0;
+  const uint32_t sb = (uint32_t)sbn0 * 2, sb1 = GATED ? (uint32_t)g.prob[1].sbn * 2 : sb, last_b = N - 1 - n0;
+  uint64_t ga[4];
+  uint32_t dB0[4], dB1[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const uint32_t r = (wave * 4 + i) * 8 + (lane >> 3), c = ((lane & 7) ^ ((r >> 1) & 7)) * 16;
+    const uint32_t ent = list[min(r, live - 1)], sl = ent >> 16;
+    const uint16_t *rows = g.slot[0].a16;
+    int64_t bs = g.slot[0].a_bs;
+#pragma unroll
+    for (int s = 1; s < 8; ++s)
+      if (sl == (uint32_t)s) {
+        rows = g.slot[s].a16;
+        bs = g.slot[s].a_bs;
+      }
+    ga[i] = (uint64_t)(rows + (int64_t)(ent & 0xFFFFu) * bs) + c;
+    dB0[i] = min(r, last_b) * sb + c;
+    dB1[i] = GATED ? min(r, last_b) * sb1 + c : min(r + 128, last_b) * sb + c;
+  }
+  auto scalar = [](const uint16_t *p) {
+    const uint64_t v = (uint64_t)p;
+    return (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)v) | (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(v >> 32)) << 32;
+  };
+  const uint64_t s_b0 = scalar(pb0), s_b1 = scalar(pb1);
+  const uint32_t lds = wave * 4096;
+#define MOE_IN                                                                                                            \
+  [dB00] "v"(dB0[0]), [dB01] "v"(dB0[1]), [dB02] "v"(dB0[2]), [dB03] "v"(dB0[3]), [dB10] "v"(dB1[0]), [dB11] "v"(dB1[1]), \
+      [dB12] "v"(dB1[2]), [dB13] "v"(dB1[3]), [pb0] "s"(s_b0), [pb1] "s"(s_b1), [lds] "s"(lds)
+  asm volatile(HFIRST_LOADS : RING_GATHERED : MOE_IN : RING_SCALARS);
+  float zero;
+  asm volatile("v_mov_b32 %0, 0" : "=v"(zero));
+  f32x16 acc[1][2][2][2];  // [0][B half][row block][column block]
+#pragma unroll
+  for (int q = 0; q < 8; ++q)
+#pragma unroll
+    for (int k = 0; k < 16; ++k) acc[0][q >> 2][(q >> 1) & 1][q & 1][k] = zero;
+  const uint32_t half = lane >> 5;
+  uint32_t ra[4], rb[4];
+#pragma unroll
+  for (int ks = 0; ks < 4; ++ks) {
+    const uint32_t p = ((ks * 2 + half) ^ ((lane >> 1) & 7)) * 16 + (lane & 31) * 128;
+    ra[ks] = wm * 8192 + p;
+    rb[ks] = wn * 8192 + p;
+  }
+  asm volatile(HMAIN_LOOP : RING_ACC0, RING_PLACES, RING_GATHERED : MOE_IN, [n] "s"(n_steps) : RING_SCALARS, RING_HALF_SCALARS, RING_FRAGMENTS);
+  // Rows back to their slot and token, out of LDS as in gemm_bf16_ring_kernel: a lane finds where the row of its number goes and
+  // hands that to the sixteen lanes that store it.
+  __syncthreads();
+  extern __shared__ __attribute__((aligned(16))) float ring_smem[];
+  const uint32_t my_row = wm * 64 + lane, ent = list[min(my_row, live - 1)], sl = ent >> 16;
+  uint64_t base = (uint64_t)(GATED ? (void *)g.slot[0].h16 : (void *)g.slot[0].c[prob]);
+#pragma unroll
+  for (int s = 1; s < 8; ++s)
+    if (sl == (uint32_t)s) base = (uint64_t)(GATED ? (void *)g.slot[s].h16 : (void *)g.slot[s].c[prob]);
+  base += (uint64_t)(ent & 0xFFFFu) * N * (GATED ? 2 : 4);
+  const int base_lo = (int)base, base_hi = (int)(base >> 32);
+#pragma unroll
+  for (int qd = 0; qd < (GATED ? 1 : 2); ++qd) {
+    float *stage = ring_smem + wave * 8192 + qd * 4096;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const uint32_t r = i * 32 + (lane & 31), chunk = j * 8 + q * 2 + half;
+          const f32x16 &x = acc[0][qd][i][j], &u = acc[0][GATED ? 1 : qd][i][j];
+          float4 v = make_float4(x[q * 4], x[q * 4 + 1], x[q * 4 + 2], x[q * 4 + 3]);
+          if (KIND == MOE_GELU) v = make_float4(gelu_fast(v.x), gelu_fast(v.y), gelu_fast(v.z), gelu_fast(v.w));
+          if (KIND == MOE_SILU) v = make_float4(silu_fast(v.x), silu_fast(v.y), silu_fast(v.z), silu_fast(v.w));
+          if (GATED) { v.x *= u[q * 4]; v.y *= u[q * 4 + 1]; v.z *= u[q * 4 + 2]; v.w *= u[q * 4 + 3]; }
+          *(float4 *)(stage + r * 64 + ((chunk ^ (r & 15)) << 2)) = v;
+        }
+    const uint32_t col0 = n0 + qd * 128 + wn * 64;
+#pragma unroll
+    for (int it = 0; it < 16; ++it) {
+      const int r = it * 4 + (lane >> 4);
+      const uint32_t col = col0 + (((lane & 15) ^ (r & 15)) << 2);
+      const float4 v = *(const float4 *)(stage + r * 64 + ((lane & 15) << 2));
+      const uint64_t to = (uint64_t)(uint32_t)__shfl(base_lo, r, 64) | (uint64_t)(uint32_t)__shfl(base_hi, r, 64) << 32;
+      if (wm * 64 + r < live && col < N) {  // (N % 8 == 0: a piece is inside or outside)
+        if (GATED) *(uint2 *)((uint16_t *)to + col) = bf16_pack4(v);
+        else *(float4 *)((float *)to + col) = v;
+      }
+    }
+  }
+}
+
+// (route_tiles, 32-bit byte offsets within a tile's weight rows, three k-steps; otherwise what moe_gemm_pipelined_ok asks)
+bool moe_ring_ok(const MoeGemmDesc &g) {
+  if (!moe_gemm_pipelined_ok(g) || !g.route_tiles || g.planes || g.K < 192) return false;
+  for (uint32_t p = 0; p < g.n_prob; ++p)
+    if (g.prob[p].sbn < 0 || g.prob[p].sbn > (1 << 22)) return false;
+  return g.fuse_glu ? g.n_prob == 2 && g.prob[0].N == g.prob[1].N : true;
+}
+
+template <int KIND>
+static hipError_t launch_moe_ring_as(const LaunchCtx &lc, const MoeGemmDesc &g, dim3 grid) {
+  constexpr int smem = 10 * 16384;
+  static bool configured = false;  // one attribute call per kernel and process
+  if (!configured) {
+    hipError_t e = hipFuncSetAttribute((const void *)moe_ring_kernel<KIND>, hipFuncAttributeMaxDynamicSharedMemorySize, smem);
+    if (e != hipSuccess) return e;
+    configured = true;
+  }
+  cg_launch(lc, moe_ring_kernel<KIND>, grid, dim3(256), smem, g);
+  return hipGetLastError();
+}
+
+hipError_t launch_moe_ring(const LaunchCtx &lc, const MoeGemmDesc &g) {
+  if (!moe_ring_ok(g)) return hipErrorInvalidValue;
+  uint32_t max_n = 0;
+  for (uint32_t p = 0; p < g.n_prob; ++p) max_n = g.prob[p].N > max_n ? g.prob[p].N : max_n;
+  const uint32_t bno = g.fuse_glu ? 128 : 256;
+  const dim3 grid((max_n + bno - 1) / bno * moe_route_max_tiles(g), g.fuse_glu ? 1 : g.n_prob, 1);
+  if (g.fuse_glu) return g.fuse_glu == PRO_GEGLU ? launch_moe_ring_as<MOE_GELU>(lc, g, grid) : launch_moe_ring_as<MOE_SILU>(lc, g, grid);
+  return launch_moe_ring_as<MOE_PLAIN>(lc, g, grid);
 }
 
 // Operands whose rows lie within 32-bit byte offsets of a tile's first row, two k-steps at least to each slice.

@@ -534,6 +534,9 @@ struct MoeGemmDesc {
   const uint32_t *route_tiles;
 };
 hipError_t launch_moe_gemm(const LaunchCtx &lc, const MoeGemmDesc &g);
+// k_gemm_ring.hip: the same for sorted pairs with a work list
+bool moe_ring_ok(const MoeGemmDesc &g);
+hipError_t launch_moe_ring(const LaunchCtx &lc, const MoeGemmDesc &g);
 // Sorts the S * n_slot (slot, token) pairs of g by expert into count / offset (n_expert words each) and
 // list (S * n_slot words); n_expert <= MOE_ROUTE_MAX_EXPERTS.  With these in g.route_*, bf16 input rows
 // (slot[].a16 for every slot) and K % 64 == 0, launch_moe_gemm streams the weights through a

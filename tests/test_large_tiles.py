@@ -5,6 +5,7 @@ the next product's operand."""
 import numpy as np
 import pytest
 
+import parity
 import test_llama_parity as llama_tests
 import test_moe_gemma_parity as moe_tests
 import vectors
@@ -124,3 +125,30 @@ def test_rotated(oracle, hip_bf16):
 @pytest.mark.parametrize("batch,tokens", [(2, 301), (3, 550)])
 def test_rotated_wide_heads(oracle, hip_bf16, batch, tokens):
     moe_tests.test_qwen_prefill_biases_and_rotation_in_the_projections_launch(oracle, hip_bf16, batch, tokens, 8, 8, 128)
+
+
+# the routed experts of a prefill (moe_ring_kernel): three slots whose choices crowd one expert (several row tiles, the last
+# partly filled) and leave others empty; the fewest k-steps, columns that end inside a tile of 128 and of 256
+@pytest.mark.gpu
+@pytest.mark.parametrize("act", ["silu", "gelu"])
+@pytest.mark.parametrize("S,E,F,H", [(150, 6, 192, 192), (64, 9, 320, 576), (700, 5, 256, 192)])
+def test_routed_experts(oracle, hip_bf16, S, E, F, H, act):
+    g = np.random.default_rng(S)
+    x, k = draw(g, (S, 1, H)), 3
+    wg, wu, wd = draw(g, (E, F, H), H ** -0.5), draw(g, (E, F, H), H ** -0.5), draw(g, (E, H, F), F ** -0.5)
+    idx = np.where(g.random((S, k)) < 0.6, 2, g.integers(0, E - 1, (S, k))).astype(np.uint32)
+    val = g.random((S, k)).astype(np.float32)
+
+    def f(b, x, iv, vv, wg, wu, wd):
+        x = x + x - x
+        total = None
+        for i in range(k):
+            slot = lang.get(b, 1, i, iv)
+            sel = lambda w: lang.transpose(b, 1, 2, lang.index(b, 0, slot, w))
+            y = lang.matmul(b, getattr(nn, act)(b, lang.matmul(b, x, sel(wg))) * lang.matmul(b, x, sel(wu)), sel(wd))
+            y = y * lang.broadcast(b, lang.reshape(b, lang.shape(b, lang.get(b, 2, 0, y)), lang.get(b, 1, i, vv)), lang.shape(b, y))
+            total = y if total is None else total + y
+        return [total]
+    (ref,) = vectors.run(oracle, f, 1, x, idx, val, wg, wu, wd)
+    (got,) = vectors.run(hip_bf16, f, 1, x, idx, val, wg, wu, wd)
+    parity.assert_bf16(ref, got, f"{S} tokens")
