@@ -40,25 +40,42 @@ __device__ __forceinline__ a_bf16x8 pack8(const float *v) {
   return r.h;
 }
 
+// The values of this lane and of the one 32 lanes away, the lower half's first: v_permlane32_swap_b32, two VALU cycles where
+// a trip through the LDS crossbar costs a step of these kernels over a hundred.
+__device__ __forceinline__ float2 both_halves(float v) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return make_float2(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+__device__ __forceinline__ float max_of_halves(float v) {
+  const float2 p = both_halves(v);
+  return fmaxf(p.x, p.y);
+}
+__device__ __forceinline__ float sum_of_halves(float v) {
+  const float2 p = both_halves(v);
+  return p.x + p.y;
+}
+
 // The classes of one query tile's key tiles (AttnPrefillDesc::tile_class), as the kernels walk them.  A row
-// of up to 64 entries is read once, by the lanes of a wave, and kept as two bit masks: finding the next
+// of up to 128 entries is read once, by the lanes of a wave, and kept as bit masks: finding the next
 // live tile is then bit arithmetic, not a chain of dependent loads.
 template <int BN>
 struct KeyTiles {
   const uint8_t *cls;  // null: no table, every tile is visited and reads its mask values
   uint32_t cols, t;
-  uint64_t live, zero;  // bit i: tile i is not dead / needs no mask values
+  uint64_t live[2], zero[2];  // bit i of word w: tile 64 w + i is not dead / needs no mask values
   bool bits;
   __device__ __forceinline__ KeyTiles(const AttnPrefillDesc &a, uint32_t q_tile, int lane) {
     cls = a.tile_class ? a.tile_class + (size_t)q_tile * a.tile_cols : nullptr;
     cols = a.tile_cols;
     t = a.t;
-    bits = cls && cols <= 64;
-    live = zero = 0;
+    bits = cls && cols <= 128;
+    live[0] = live[1] = zero[0] = zero[1] = 0;
     if (bits) {
-      const uint8_t c = (uint32_t)lane < cols ? cls[lane] : 0;
-      live = __ballot(c != 0);
-      zero = __ballot(c == 2);
+      const uint8_t c0 = (uint32_t)lane < cols ? cls[lane] : 0, c1 = (uint32_t)lane + 64 < cols ? cls[lane + 64] : 0;
+      live[0] = __ballot(c0 != 0);
+      live[1] = __ballot(c1 != 0);
+      zero[0] = __ballot(c0 == 2);
+      zero[1] = __ballot(c1 == 2);
     }
   }
   // the first step at or after t0 that is not dead (>= t: none)
@@ -66,16 +83,33 @@ struct KeyTiles {
     if (!cls) return t0;
     uint32_t i = t0 / BN;
     if (bits) {
-      const uint64_t m = i < 64 ? live >> i : 0;
-      return m ? (i + (uint32_t)__builtin_ctzll(m)) * (uint32_t)BN : cols * (uint32_t)BN;
+      if (i < 64) {
+        const uint64_t m = live[0] >> i;
+        if (m) return (i + (uint32_t)__builtin_ctzll(m)) * (uint32_t)BN;
+        i = 64;
+      }
+      const uint64_t m = i < 128 ? live[1] >> (i - 64) : 0;
+      return (m ? i + (uint32_t)__builtin_ctzll(m) : cols) * (uint32_t)BN;
     }
     while (i < cols && cls[i] == 0) ++i;
     return i * (uint32_t)BN;
   }
+  // the n-th live step after the one at t0
+  __device__ __forceinline__ uint32_t skip(uint32_t t0, int n) const {
+    for (int i = 0; i < n && t0 < t; ++i) t0 = next_step(t0 + BN);
+    return t0;
+  }
+  __device__ __forceinline__ uint32_t live_steps() const {
+    if (bits) return (uint32_t)(__builtin_popcountll(live[0]) + __builtin_popcountll(live[1]));
+    uint32_t n = 0;
+    for (uint32_t t0 = next_step(0); t0 < t; t0 = next_step(t0 + BN)) ++n;
+    return n;
+  }
   // does the step at t0 read mask values (given that there is a mask)?
   __device__ __forceinline__ bool reads_mask(uint32_t t0) const {
     if (!cls || t0 >= t) return true;
-    return bits ? !((zero >> (t0 / BN)) & 1) : cls[t0 / BN] != 2;
+    const uint32_t i = t0 / BN;
+    return bits ? !(((i < 64 ? zero[0] : zero[1]) >> (i & 63)) & 1) : cls[i] != 2;
   }
 };
 
@@ -90,8 +124,10 @@ constexpr float ATTN_MAX_SLACK = 8.0f;
 // conversion.  One path with the tail's and the mask's selects took 541 vector instructions for 32 scores a lane; this one
 // takes 110.  With it, one barrier a step and the long query tiles first: 2900 tokens of 32 heads of 64 212 -> 96 us a
 // layer, 8 x 2048 of 4 heads of 256 227 -> 168, 4 x 256 of 16 heads of 128 26.6 -> 22.7, 512 of 32 heads of 64 17.0 -> 14.9.
-template <int KT>
-__device__ __forceinline__ float attn_softmax_step(const AttnPrefillDesc &a, a_f32x16 (&st)[KT], const float4 (&mask)[KT][4],
+// LATE: the mask values are asked for here, not handed in: 32 registers less across the score product, which is a third wavefront to
+// a SIMD for heads of 64 (2900 tokens 97.6 -> 89.8 us, 4000 154 -> 132), and a trip to L2 in the few steps that read a mask.
+template <int KT, bool LATE>
+__device__ __forceinline__ float attn_softmax_step(const AttnPrefillDesc &a, a_f32x16 (&st)[KT], const float *M, const float4 (&early)[KT][4],
                                                    a_bf16x8 (&pf)[KT * 2], float &m_run, float &l_run, float inv_scale, bool plain,
                                                    bool use_mask, uint32_t t0, int half) {
   constexpr float LOG2E = 1.44269504f, LOWEST = -3.40282347e+38f;
@@ -101,7 +137,7 @@ __device__ __forceinline__ float attn_softmax_step(const AttnPrefillDesc &a, a_f
     for (int kt = 0; kt < KT; ++kt)
 #pragma unroll
       for (int e = 0; e < 16; ++e) tmax = fmaxf(tmax, st[kt][e]);
-    tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64)) * inv_scale;
+    tmax = max_of_halves(tmax) * inv_scale;
     const float m_new = tmax > m_run + ATTN_MAX_SLACK ? tmax : m_run;
     alpha = __expf(m_run - m_new);
     m_run = m_new;
@@ -121,12 +157,17 @@ __device__ __forceinline__ float attn_softmax_step(const AttnPrefillDesc &a, a_f
   } else {
     const bool tail = t0 + KT * 32 > a.t;  // the only step with keys past the end (uniform)
 #pragma unroll
-    for (int kt = 0; kt < KT; ++kt)
+    for (int kt = 0; kt < KT; ++kt) {
+      float4 mask[4];
+      if (use_mask) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) mask[j] = LATE ? *(const float4 *)(M + min(t0 + kt * 32 + j * 8 + half * 4, a.m_len - 4)) : early[kt][j];
+      }
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const uint32_t key = t0 + kt * 32 + j * 8 + half * 4;
         float mv[4] = {0.f, 0.f, 0.f, 0.f};
-        if (use_mask) { mv[0] = mask[kt][j].x; mv[1] = mask[kt][j].y; mv[2] = mask[kt][j].z; mv[3] = mask[kt][j].w; }
+        if (use_mask) { mv[0] = mask[j].x; mv[1] = mask[j].y; mv[2] = mask[j].z; mv[3] = mask[j].w; }
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           float v = st[kt][j * 4 + i];
@@ -138,7 +179,8 @@ __device__ __forceinline__ float attn_softmax_step(const AttnPrefillDesc &a, a_f
           tmax = fmaxf(tmax, v);
         }
       }
-    tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
+    }
+    tmax = max_of_halves(tmax);
     const float m_new = tmax > m_run + ATTN_MAX_SLACK ? tmax : m_run;
     alpha = __expf(m_run - m_new);
     m_run = m_new;
@@ -164,28 +206,34 @@ __device__ __forceinline__ float attn_softmax_step(const AttnPrefillDesc &a, a_f
 // BN keys per step.  The K / V rows of step i + 1 are in registers, asked for a step ago, while step i is computed from
 // one LDS buffer, and go to the other buffer behind its first product: one barrier per step.
 // NW waves of 32 queries each per workgroup (4, or 2 when that is what it takes to occupy the CUs).
+// KG = 2: half of the waves share 64 queries with the other half and take every other live step of them, with tiles of their own;
+// the partial results meet once, in LDS.  The longest query tile of a causal mask is then half as long.
 // Workgroups: the query tiles with the most keys first (a causal mask gives the last tile all of them), and the heads of a
 // (batch, kv head) on one XCD, whose L2 then holds their keys and values.
 // (the register budget of two waves to a SIMD keeps the accumulators of heads of 64 and 128 out of the accumulation file,
-// 64 moves a step; three waves spill 20 bytes: 109 us where two take 96)
-#define ATTN_WAVES(D) __attribute__((amdgpu_waves_per_eu(D <= 128 ? 2 : 1, D <= 128 ? 2 : 1)))
-template <int D, int BN, int NW>
-__global__ void __launch_bounds__(NW * 64) ATTN_WAVES(D) attn_prefill_kernel(AttnPrefillDesc a) {
-  constexpr int NT = NW * 64;
+// 64 moves a step.  Heads of 64 have room for three since the mask values are asked for where they are used and the products of a
+// step take turns between accumulators: 2900 tokens of 32 heads, causal, 90 us a layer where two waves and one chain after the
+// other took 97, 4000 tokens 131 for 154)
+#define ATTN_WAVES(n) __attribute__((amdgpu_waves_per_eu(n, n)))
+template <int D, int BN, int NW, int KG = 1>
+__global__ void __launch_bounds__(NW * 64) ATTN_WAVES((D > 128 ? 1 : D == 64 && NW == 4 && (KG == 1 || BN == 32) ? 3 : 2)) attn_prefill_kernel(AttnPrefillDesc a) {
+  constexpr int NT = NW * 64 / KG, QROWS = NW / KG * 32;  // threads of a key group, queries of the workgroup
   constexpr int KP = D + 8;              // K tile row pitch (bf16 elements)
   constexpr int VP = BN + 8;             // V^T tile row pitch
   constexpr int DT = D / 32;             // 32-row tiles of O^T
   constexpr int KT = BN / 32;            // 32-key tiles of S^T
   constexpr int KCH = BN * D / 8 / NT;   // 16-byte chunks of the K tile / of the V^T tile per thread
-  __shared__ __attribute__((aligned(16))) uint16_t tile[2][BN * KP + D * VP];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  constexpr int TILE = BN * KP + D * VP;
+  __shared__ __attribute__((aligned(16))) uint16_t tile[KG][2][TILE];
+  const int lane = threadIdx.x & 63, all_waves = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int kg = KG == 1 ? 0 : all_waves / (NW / KG), wave = KG == 1 ? all_waves : all_waves % (NW / KG), tid = wave * 64 + lane;
   const int col = lane & 31, half = lane >> 5;
-  const uint32_t n_bh = a.heads * a.b, q_tiles = (a.s + NW * 32 - 1) / (NW * 32);
+  const uint32_t n_bh = a.heads * a.b, q_tiles = (a.s + QROWS - 1) / QROWS;
   const uint32_t rank = blockIdx.x / n_bh, slot = blockIdx.x - rank * n_bh, q_tile = q_tiles - 1 - rank;
   const uint32_t bh = n_bh % 8 == 0 ? (slot % 8) * (n_bh / 8) + slot / 8 : slot;
   const uint32_t b = bh / a.heads, h = bh - b * a.heads;
   const uint32_t kvh = h / a.rep, rp = h % a.rep;
-  const uint32_t query = q_tile * (NW * 32) + wave * 32 + col;
+  const uint32_t query = q_tile * QROWS + wave * 32 + col;
   const bool q_ok = query < a.s;
   const uint32_t qc = q_ok ? query : a.s - 1;  // loads of lanes past the end go to a valid row
   const float *Q = a.q + (int64_t)b * a.q_sb + (int64_t)h * a.q_sh + (int64_t)qc * a.q_ss;
@@ -198,36 +246,43 @@ __global__ void __launch_bounds__(NW * 64) ATTN_WAVES(D) attn_prefill_kernel(Att
 
   typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
   u32x4 kreg[KCH], vreg[KCH];  // the step in flight
-  // All loads are unconditional (indices clamped into range) so that they are issued back to back;
-  // chunks past the end are zeroed when the registers are consumed.
-  // With a class table, dead key tiles are never visited and all-zero ones need no mask values.
+  // All loads are unconditional so that they are issued back to back; chunks past the end are zeroed when the registers are
+  // consumed.  With a class table, dead key tiles are never visited and all-zero ones need no mask values.  This thread's first
+  // chunk of each tile is kept as a pointer; a step without the end of the keys in it is a scalar away from there (with every
+  // index clamped and every product taken in every step, a quarter of the step's vector instructions).
   const KeyTiles<BN> tiles(a, q_tile, lane);
-  auto fetch = [&](uint32_t t0) {
+  constexpr int KROWS = NT * 8 / D, VROWS = NT * 8 / BN;  // rows of the K tile, of the V^T tile, between a thread's chunks
+  const uint32_t k_row = tid / (D / 8), k_d8 = (tid % (D / 8)) * 8, v_row = tid / (BN / 8), v_k8 = (tid % (BN / 8)) * 8;
+  const char *kp = (const char *)(K + (int64_t)k_row * a.k_st + k_d8), *vp = (const char *)(VT + (int64_t)v_row * a.vt_st + v_k8);
+  const int64_t k_step = a.k_st * 2, v_chunk = (int64_t)VROWS * a.vt_st * 2;
+  auto fetch = [&](uint32_t at) {
+    const uint32_t t0 = __builtin_amdgcn_readfirstlane(at);
+    if (t0 + BN <= a.t) {
 #pragma unroll
-    for (int c = 0; c < KCH; ++c) {
-      const int ch = tid + c * NT, key = ch / (D / 8), d8 = (ch % (D / 8)) * 8;
-      kreg[c] = *(const u32x4 *)(K + (int64_t)min(t0 + key, a.t - 1) * a.k_st + d8);
+      for (int c = 0; c < KCH; ++c) kreg[c] = *(const u32x4 *)(kp + (int64_t)(t0 + c * KROWS) * k_step);
+#pragma unroll
+      for (int c = 0; c < KCH; ++c) vreg[c] = *(const u32x4 *)(vp + (c * v_chunk + (int64_t)t0 * 2));
+      return;
     }
 #pragma unroll
-    for (int c = 0; c < KCH; ++c) {
-      const int ch = tid + c * NT, dim = ch / (BN / 8), k8 = (ch % (BN / 8)) * 8;
-      vreg[c] = *(const u32x4 *)(VT + (int64_t)dim * a.vt_st + min(t0 + k8, a.vt_st - 8));
-    }
+    for (int c = 0; c < KCH; ++c) kreg[c] = *(const u32x4 *)(K + (int64_t)min(t0 + k_row + c * KROWS, a.t - 1) * a.k_st + k_d8);
+#pragma unroll
+    for (int c = 0; c < KCH; ++c) vreg[c] = *(const u32x4 *)(VT + (int64_t)(v_row + c * VROWS) * a.vt_st + min(t0 + v_k8, a.vt_st - 8));
   };
-  auto stash = [&](uint16_t *to, uint32_t t0) {  // registers -> LDS: K [BN, D] and V^T [D, BN]
+  uint16_t *const k_at = &tile[kg][0][k_row * KP + k_d8], *const v_at = &tile[kg][0][BN * KP + v_row * VP + v_k8];
+  auto stash = [&](int to, uint32_t at) {  // registers -> LDS: K [BN, D] and V^T [D, BN]
+    const uint32_t t0 = __builtin_amdgcn_readfirstlane(at);
 #pragma unroll
-    for (int c = 0; c < KCH; ++c) {
-      const int ch = tid + c * NT, key = ch / (D / 8), d8 = (ch % (D / 8)) * 8;
-      *(u32x4 *)(&to[key * KP + d8]) = kreg[c];  // (rows past the end repeat the last one: their scores are discarded)
-    }
-#pragma unroll
-    for (int c = 0; c < KCH; ++c) {
-      const int ch = tid + c * NT, dim = ch / (BN / 8), k8 = (ch % (BN / 8)) * 8;
+    for (int c = 0; c < KCH; ++c) *(u32x4 *)(k_at + to * TILE + c * KROWS * KP) = kreg[c];  // (rows past the end repeat the last one: their scores are discarded)
+    if (t0 + BN > a.t) {
       const u32x4 none = {0u, 0u, 0u, 0u};
-      *(u32x4 *)(&to[BN * KP + dim * VP + k8]) = t0 + k8 < a.t ? vreg[c] : none;
+#pragma unroll
+      for (int c = 0; c < KCH; ++c) vreg[c] = t0 + v_k8 < a.t ? vreg[c] : none;
     }
+#pragma unroll
+    for (int c = 0; c < KCH; ++c) *(u32x4 *)(v_at + to * TILE + c * VROWS * VP) = vreg[c];
   };
-  uint32_t t0 = tiles.next_step(0), t_next = a.t;
+  uint32_t t0 = tiles.skip(tiles.next_step(0), kg), t_next = a.t;
   if (t0 < a.t) fetch(t0);  // (uniform)
 
   // this lane's query row as B fragments: k-step ks covers dims 16 ks .. 16 ks + 15, half h takes 8
@@ -254,41 +309,47 @@ __global__ void __launch_bounds__(NW * 64) ATTN_WAVES(D) attn_prefill_kernel(Att
   const bool can_be_plain = inv_scale > 0.f && (M || !a.has_mask_const);
 
   if (t0 < a.t) {
-    stash(tile[0], t0);
-    t_next = tiles.next_step(t0 + BN);
+    stash(0, t0);
+    t_next = tiles.skip(t0, KG);
     if (t_next < a.t) fetch(t_next);
   }
   __syncthreads();
-  for (int buf = 0; t0 < a.t; buf ^= 1) {
-    const uint16_t *Ks = tile[buf], *Vt = Ks + BN * KP;
+  const uint32_t turns = KG > 1 ? (tiles.live_steps() + KG - 1) / KG : 0;  // (as many for every group: they share the barrier)
+  for (uint32_t turn = 0, buf = 0; KG > 1 ? turn < turns : t0 < a.t; ++turn, buf ^= 1) {
+    if (KG > 1 && t0 >= a.t) {  // (the last turn of an odd number of steps)
+      __syncthreads();
+      continue;
+    }
+    const uint16_t *Ks = tile[kg][buf], *Vt = Ks + BN * KP;
     const bool use_mask = M && tiles.reads_mask(t0);  // uniform
     const bool plain = can_be_plain && !use_mask && t0 + BN <= a.t;
     // The mask values of this step are asked for here and used after the score product; rows allow 16-byte loads
     // (checked by the host).  A step whose every pair is masked - possible only without a class table - needs no
     // special case: its weights exp(f32::MIN - m) are zero once any live key has been seen, and a row that never
     // sees one is rebuilt at the end.
+    constexpr bool LATE = D == 128 || (D == 64 && NW == 4 && (KG == 1 || BN == 32));
     float4 mcur[KT][4];
-    if (use_mask) {
+    if (use_mask && !LATE) {
 #pragma unroll
       for (int kt = 0; kt < KT; ++kt)
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
-          mcur[kt][j] = *(const float4 *)(M + min(t0 + kt * 32 + j * 8 + half * 4, a.m_len - 4));
+        for (int j = 0; j < 4; ++j) mcur[kt][j] = *(const float4 *)(M + min(t0 + kt * 32 + j * 8 + half * 4, a.m_len - 4));
     }
     // ---- S^T = K . Q^T
     a_f32x16 st[KT];
 #pragma unroll
-    for (int kt = 0; kt < KT; ++kt) {
+    for (int kt = 0; kt < KT; ++kt)
 #pragma unroll
       for (int e = 0; e < 16; ++e) st[kt][e] = 0.f;
 #pragma unroll
-      for (int ks = 0; ks < D / 16; ++ks) {
+    for (int ks = 0; ks < D / 16; ++ks)
+#pragma unroll
+      for (int kt = 0; kt < KT; ++kt) {  // (chains of products that do not wait for each other)
         const a_bf16x8 kf = *(const a_bf16x8 *)(&Ks[(kt * 32 + col) * KP + ks * 16 + half * 8]);
         st[kt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qf[ks], st[kt], 0, 0, 0);
       }
-    }
-    const uint32_t t_cur = t0, t_after = t_next < a.t ? tiles.next_step(t_next + BN) : a.t;
-    if (t_next < a.t) stash(tile[buf ^ 1], t_next);  // (everyone is past the barrier behind the last reads of that buffer)
+    const uint32_t t_cur = t0, t_after = t_next < a.t ? tiles.skip(t_next, KG) : a.t;
+    if (t_next < a.t) stash(buf ^ 1, t_next);  // (everyone is past the barrier behind the last reads of that buffer)
     if (t_after < a.t) fetch(t_after);
     t0 = t_next;
     t_next = t_after;
@@ -297,7 +358,7 @@ __global__ void __launch_bounds__(NW * 64) ATTN_WAVES(D) attn_prefill_kernel(Att
     // ATTN_MAX_SLACK: the quotient O / l at the end does not depend on it, weights of up to e^slack are as
     // exact in f32 and bf16 as weights of up to 1, and O is rescaled on a few steps instead of on most.
     a_bf16x8 pf[KT * 2];
-    const float alpha = attn_softmax_step<KT>(a, st, mcur, pf, m_run, l_run, inv_scale, plain, use_mask, t_cur, half);
+    const float alpha = attn_softmax_step<KT, LATE>(a, st, M, mcur, pf, m_run, l_run, inv_scale, plain, use_mask, t_cur, half);
     // ---- O^T = O^T * alpha + V^T . P^T
     if (__any(alpha != 1.0f)) {  // the running maximum moved for some query of this wave
 #pragma unroll
@@ -306,9 +367,9 @@ __global__ void __launch_bounds__(NW * 64) ATTN_WAVES(D) attn_prefill_kernel(Att
         for (int e = 0; e < 16; ++e) o[t][e] *= alpha;
     }
 #pragma unroll
-    for (int t = 0; t < DT; ++t) {
+    for (int blk = 0; blk < KT * 2; ++blk) {
 #pragma unroll
-      for (int blk = 0; blk < KT * 2; ++blk) {
+      for (int t = 0; t < DT; ++t) {
         // A fragment: row = dim t*32 + col, the lane's eight keys of this block in the permuted order
         const uint16_t *vr = &Vt[(t * 32 + col) * VP + blk * 16 + half * 4];
         union {
@@ -322,7 +383,29 @@ __global__ void __launch_bounds__(NW * 64) ATTN_WAVES(D) attn_prefill_kernel(Att
     }
     __syncthreads();
   }
-  l_run += __shfl_xor(l_run, 32, 64);
+  l_run = sum_of_halves(l_run);
+  if constexpr (KG == 2) {  // the second group's partial results, [register][lane], join the first's
+    float *part = (float *)&tile[0][0][0] + wave * (DT * 16 + 2) * 64;
+    static_assert((NW / 2) * (DT * 16 + 2) * 64 * 4 <= 2 * 2 * TILE * 2, "partial results fit in the tiles");
+    if (kg) {  // (everyone is past the barrier behind the last step)
+      part[lane] = m_run;
+      part[64 + lane] = l_run;
+#pragma unroll
+      for (int t = 0; t < DT; ++t)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) part[(2 + t * 16 + e) * 64 + lane] = o[t][e];
+    }
+    __syncthreads();
+    if (kg) return;
+    const float m_w = part[lane], l_w = part[64 + lane], m_new = fmaxf(m_run, m_w);
+    const float f0 = __expf(m_run - m_new), f1 = __expf(m_w - m_new);
+    l_run = l_run * f0 + l_w * f1;
+    m_run = m_new;
+#pragma unroll
+    for (int t = 0; t < DT; ++t)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) o[t][e] = o[t][e] * f0 + part[(2 + t * 16 + e) * 64 + lane] * f1;
+  }
   // A row whose every key is masked has all scores equal to f32::MIN on the reference path:
   // uniform weights, i.e. the mean of V.  Dead steps were skipped above, so rebuild that here.
   if (M && q_ok && m_run <= -3.0e38f) {
@@ -391,10 +474,6 @@ attn_prefill_keysplit_kernel(AttnPrefillDesc a) {
   const float *M = a.mask ? a.mask + (int64_t)b * a.m_sb + (int64_t)h * a.m_sh + (int64_t)qc * a.m_ss : nullptr;
 
   const KeyTiles<BN> tiles(a, blockIdx.x, lane);
-  auto skip_steps = [&](uint32_t t0, int n) {  // the n-th live step after the one at t0
-    for (int i = 0; i < n && t0 < a.t; ++i) t0 = tiles.next_step(t0 + BN);
-    return t0;
-  };
   auto step_mask = [&](uint32_t t0) { return M && tiles.reads_mask(t0); };
   uint4 kreg[KCH], vreg[KCH];
   auto fetch = [&](uint32_t t0) {
@@ -409,7 +488,7 @@ attn_prefill_keysplit_kernel(AttnPrefillDesc a) {
       vreg[c] = *(const uint4 *)(VT + (int64_t)dim * a.vt_st + min(t0 + k8, a.vt_st - 8));
     }
   };
-  uint32_t t0 = skip_steps(tiles.next_step(0), wave);
+  uint32_t t0 = tiles.skip(tiles.next_step(0), wave);
   if (t0 < a.t) fetch(t0);  // asked for before the queries: one round trip for both
 
   // The queries: each wave converts a quarter of the workgroup's 32 rows (16 bytes of bf16 per lane and
@@ -449,7 +528,7 @@ attn_prefill_keysplit_kernel(AttnPrefillDesc a) {
   const bool can_be_plain = inv_scale > 0.f && (M || !a.has_mask_const);
 
   while (t0 < a.t) {
-    const uint32_t t_next = skip_steps(t0, NW);
+    const uint32_t t_next = tiles.skip(t0, NW);
     const bool use_mask = step_mask(t0);  // uniform over the wave
     const bool tail = t0 + BN > a.t;
     const uint32_t t_cur = t0;
@@ -463,8 +542,7 @@ attn_prefill_keysplit_kernel(AttnPrefillDesc a) {
 #pragma unroll
       for (int kt = 0; kt < KT; ++kt)
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
-          mcur[kt][j] = *(const float4 *)(M + min(t_cur + kt * 32 + j * 8 + half * 4, a.m_len - 4));
+        for (int j = 0; j < 4; ++j) mcur[kt][j] = *(const float4 *)(M + min(t_cur + kt * 32 + j * 8 + half * 4, a.m_len - 4));
     }
     // registers -> this wave's LDS region.  Its LDS instructions run in program order, so the fragment
     // reads of the previous step are behind these writes and the reads below are ahead of them; the
@@ -495,7 +573,7 @@ attn_prefill_keysplit_kernel(AttnPrefillDesc a) {
       }
     }
     a_bf16x8 pf[KT * 2];
-    const float alpha = attn_softmax_step<KT>(a, st, mcur, pf, m_run, l_run, inv_scale, can_be_plain && !use_mask && !tail, use_mask, t_cur, half);
+    const float alpha = attn_softmax_step<KT, false>(a, st, M, mcur, pf, m_run, l_run, inv_scale, can_be_plain && !use_mask && !tail, use_mask, t_cur, half);
     if (__any(alpha != 1.0f)) {
 #pragma unroll
       for (int t = 0; t < DT; ++t)
@@ -517,7 +595,7 @@ attn_prefill_keysplit_kernel(AttnPrefillDesc a) {
       }
     }
   }
-  l_run += __shfl_xor(l_run, 32, 64);
+  l_run = sum_of_halves(l_run);
   // ---- the waves' partial results meet: [register][lane] floats in each wave's own region
   __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
   float *mine = (float *)(lds + wave * REGION);
@@ -750,7 +828,7 @@ __global__ void __launch_bounds__(NW * 64) attn_prefill_f32_kernel(AttnPrefillDe
           tmax = fmaxf(tmax, s);
         }
       }
-    tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
+    tmax = max_of_halves(tmax);
     const float m_new = fmaxf(m_run, tmax);
     const float alpha = expf(m_run - m_new);
     float psum = 0.f;
@@ -764,7 +842,7 @@ __global__ void __launch_bounds__(NW * 64) attn_prefill_f32_kernel(AttnPrefillDe
         st[kt][e] = p;
         psum += p;
       }
-    psum += __shfl_xor(psum, 32, 64);
+    psum = sum_of_halves(psum);
     l_run = l_run * alpha + psum;
     m_run = m_new;
     if (__any(alpha != 1.0f)) {
@@ -828,9 +906,26 @@ __global__ void __launch_bounds__(NW * 64) attn_prefill_f32_kernel(AttnPrefillDe
   }
 }
 
+// Heads of 64 under a mask whose workgroups of 128 queries would all run at once, two to a CU: the one with the most keys is then
+// what the launch takes, and two key groups of 64 queries halve it.  With more of them the long tiles start first and the short
+// ones fill in.  Up to one such workgroup a CU the key-split kernel's 32 queries are ahead.  us a layer, 32 heads, causal, against
+// what the line keeps them from: 512 tokens 16.5 (key-split 14.2), 900 24.8 (34), 1050 25.4 (128 queries 36.7), 1500 38 (50),
+// 2000 50 (61); 2900 93 (90) and 4000 154 (131) lie past it.
+static bool attn_prefill_two_groups(const LaunchCtx &lc, const AttnPrefillDesc &d) {
+  return !d.f32 && d.d == 64 && d.mask && (uint64_t)((d.s + 63) / 64) * d.heads * d.b > (uint64_t)lc.n_cus &&
+         (uint64_t)((d.s + 127) / 128) * d.heads * d.b <= 2 * (uint64_t)lc.n_cus;
+}
+
+// Keys a step of the two groups.  32 leave registers for a third workgroup on the CU, which pays once two and a half are there for
+// each: 1200 tokens 31.6 us (64 keys 29.6), 1500 38.3 (39.8), 1800 47.0 (53.6), 2000 50.7 (60.2).
+static uint32_t attn_prefill_two_groups_keys(const LaunchCtx &lc, const AttnPrefillDesc &d) {
+  return 2 * (uint64_t)((d.s + 63) / 64) * d.heads * d.b > 5 * (uint64_t)lc.n_cus ? 32 : 64;
+}
+
 // bf16 products, few query rows: 64-query workgroups would not give every CU two of them
 static bool attn_prefill_keysplit(const LaunchCtx &lc, const AttnPrefillDesc &d) {
-  return !d.f32 && d.d == 64 && (uint64_t)((d.s + 63) / 64) * d.heads * d.b < 2 * (uint64_t)lc.n_cus;
+  return !d.f32 && d.d == 64 && (uint64_t)((d.s + 63) / 64) * d.heads * d.b < 2 * (uint64_t)lc.n_cus &&
+         !attn_prefill_two_groups(lc, d);
 }
 
 static bool attn_prefill_small_tiles(const LaunchCtx &lc, const AttnPrefillDesc &d) {
@@ -839,8 +934,8 @@ static bool attn_prefill_small_tiles(const LaunchCtx &lc, const AttnPrefillDesc 
 }
 
 void attn_prefill_tiling(const LaunchCtx &lc, const AttnPrefillDesc &d, uint32_t *q_rows, uint32_t *keys) {
-  *q_rows = attn_prefill_keysplit(lc, d) ? 32 : attn_prefill_small_tiles(lc, d) ? 64 : 128;
-  *keys = (d.d == 256 || (d.f32 && d.d == 128)) ? 32 : 64;
+  *q_rows = attn_prefill_keysplit(lc, d) ? 32 : attn_prefill_small_tiles(lc, d) || attn_prefill_two_groups(lc, d) ? 64 : 128;
+  *keys = attn_prefill_two_groups(lc, d) ? attn_prefill_two_groups_keys(lc, d) : (d.d == 256 || (d.f32 && d.d == 128)) ? 32 : 64;
 }
 
 // one workgroup per (key tile, query tile): any value above the masked level, any value that is not zero
@@ -893,6 +988,12 @@ hipError_t launch_attn_prefill(const LaunchCtx &lc, const AttnPrefillDesc &d) {
   if (attn_prefill_keysplit(lc, d)) {
     dim3 g32((d.s + 31) / 32, d.heads, d.b);
     CG_LAUNCH(lc, (attn_prefill_keysplit_kernel<64, 64, 4>), g32, 256, d);
+    return hipGetLastError();
+  }
+  if (attn_prefill_two_groups(lc, d)) {
+    const uint32_t grid = (d.s + 63) / 64 * d.heads * d.b;
+    if (attn_prefill_two_groups_keys(lc, d) == 32) CG_LAUNCH(lc, (attn_prefill_kernel<64, 32, 4, 2>), grid, 256, d);
+    else CG_LAUNCH(lc, (attn_prefill_kernel<64, 64, 4, 2>), grid, 256, d);
     return hipGetLastError();
   }
   const bool small = attn_prefill_small_tiles(lc, d);

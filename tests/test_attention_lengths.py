@@ -169,3 +169,46 @@ def test_what_memory_held_stays_out_of_a_prompt(oracle, hip, hip_bf16, H, KV, S,
         (got,) = vectors.run(be, f, 1, q, k, v)
         assert np.isfinite(got).all()
         check(ref, got, f"attention over {S} keys")
+
+
+def attention_under(S, T, rep):
+    def f(b, q, k, v, hidden):
+        q, k, v = q + q - q, k + k - k, v + v - v
+        attn = lang.matmul(b, q, lang.transpose(b, 2, 3, helpers.repeat_kv(b, rep, k)))
+        sh = lang.shape(b, attn)
+        mask = hidden * lang.constant(b, helpers.F32_MIN, lang.shape(b, hidden))
+        attn = attn / lang.constant(b, 8.0, sh) + lang.broadcast(b, mask, sh)
+        return lang.matmul(b, nn.softmax(b, attn), helpers.repeat_kv(b, rep, v))
+    return f
+
+
+def attention_in_numpy(q, k, v, hidden, rep):
+    out = np.empty_like(q)      # (the oracle takes half a minute for the longest of these)
+    for h in range(q.shape[1]):
+        p = q[0, h] @ k[0, h // rep].T / np.float32(8) + hidden * np.float32(helpers.F32_MIN)
+        p = np.exp(p - p.max(1, keepdims=True))
+        out[0, h] = p @ v[0, h // rep] / p.sum(1, keepdims=True)
+    return out
+
+
+# Two key groups of a query tile: 64 and 32 keys a step (by how many workgroups there are), key tiles seen by none, some or all of
+# a query tile's rows at random (odd numbers of live steps, a group without any), rows that see no key at all, and more key tiles
+# than the bit masks hold (T = 4100), heads that do not divide by the dies.
+@pytest.mark.gpu
+@pytest.mark.parametrize("H,KV,S,T", [(48, 6, 321, 321), (65, 13, 257, 257), (64, 8, 641, 641), (322, 2, 65, 4100)])
+def test_two_key_groups(hip_bf16, H, KV, S, T):
+    g = np.random.default_rng(S + T)
+    q = vectors.bf16_round(g.standard_normal((1, H, S, 64)).astype(np.float32))
+    k, v = (vectors.bf16_round(g.standard_normal((1, KV, T, 64)).astype(np.float32)) for _ in range(2))
+    tiles = g.integers(0, 3, ((S + 63) // 64, (T + 31) // 32))       # 0: hidden, 1: in part, 2: seen
+    tiles[0] = 0
+    tiles[0, (T - 1) // 32] = 2                                       # one live step for the first 64 queries
+    per = np.repeat(np.repeat(tiles, 64, 0)[:S], 32, 1)[:, :T]
+    hidden = np.where(per == 1, g.integers(0, 2, (S, T)), per == 0).astype(np.float32)
+    hidden[[3, S - 1]] = 1
+    f = attention_under(S, T, H // KV)
+    ref = attention_in_numpy(q, k, v, hidden, H // KV)
+    hip_bf16.launch_counts(reset=True)
+    (got,) = vectors.run(hip_bf16, f, 1, q, k, v, hidden)
+    assert hip_bf16.launch_counts(reset=True).get("attn_prefill") == 1
+    parity.assert_bf16(ref, got, f"{S} queries of {T} keys")
