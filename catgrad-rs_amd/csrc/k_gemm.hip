@@ -3230,22 +3230,23 @@ hipError_t launch_matmul(const LaunchCtx &lc_in, const GemmDesc &g, const char *
         const uint32_t steps = before_last >= g.K ? 0 : std::min(gg.k_per_split, g.K - before_last) / 64;
         auto rounds = [&](uint64_t tiles) { return (tiles + cus - 1) / cus; };
         if (g.rope_s) {
-          // q / k / v rotated.  Up to a round of 128 rows (four stages and eight wavefronts instead: 700 rows of 3072 columns 24.2 us,
-          // 22.4; 600 of 6144 27.3, 26.7), or of 192 (1500 rows of 3072 39.3, 34.3); from there on the long tail - 64 KB of tile
-          // through LDS, table rows from L2 - is worth a second workgroup to the CU (2000 rows 40.2, 43.6 on one; 1024 rows of 6144
-          // 39.6, 46.3).  Few tiles and heads of 64: 64 columns a tile (512 rows 18.3, 21.8).
+          // q / k / v rotated: eight wavefronts share the long tail - 64 KB of tile through LDS, table rows from L2 -, and once there
+          // are more tiles than CUs two workgroups of two stages share a CU, one's tail under the other's main loop.  (With four
+          // wavefronts and the main loop in one statement, weights from memory: 700 rows of 3072 columns 27.2 -> 28.8 us, 1300 38.8 ->
+          // 39.6; 6144 columns of heads of 128, 200 rows 27.7 -> 33.4, 600 32.2 -> 40.0, 960 45.2 -> 55.6.)  Few tiles and heads of
+          // 64: 64 columns a tile (512 rows 18.3, 21.8).
           if (splits == 1 && t128 * 2 <= cus && g.rope_hd == 64)
             e = launch_gemm_dma<128, 64, 4, 2, false, 4, false, false, true>(lc, gg, (uint32_t)((uint64_t)((g.M + 127) / 128) * ((g.N + 63) / 64) * batch));
-          else if (t128 <= cus && steps >= 4) e = launch_gemm_dma<128, 128, 2, 2, false, 5, false, false, true, 1, true>(lc, gg, (uint32_t)t128);
-          else if (t192 <= cus && steps >= 4) e = launch_gemm_dma<192, 128, 2, 2, false, 4, false, false, true, 1, true>(lc, gg, (uint32_t)t192);
+          else if (t128 <= cus) e = launch_gemm_dma<128, 128, 2, 4, false, 4, false, false, true>(lc, gg, (uint32_t)t128);
           else e = launch_gemm_dma<128, 128, 2, 4, false, 2, false, false, true>(lc, gg, (uint32_t)t128);
         } else if (splits == 1 && t128 * 2 <= cus && g.N >= 128) {
           // too few 128 x 128 tiles for the CUs and no split-K to multiply them: halve the tile
           e = launch_gemm_dma<128, 64, 4, 2, false, 4>(lc, gg, (uint32_t)((uint64_t)((g.M + 127) / 128) * ((g.N + 63) / 64) * batch));
         } else if (t128 <= cus) {
-          // A round of 128 rows.  The four wavefronts' longer start and tail pay from 32 k-steps on, or from 16 while CUs are left over
-          // (1500 x 2048 x 8192 71 -> 55 us, x 2048 23 -> 19; 512 x 2048 x 8192 in four slices 25.5 -> 22.2; 8 steps 10.7, 12.4).
-          if (steps >= 32 || (steps >= 16 && t128 * 4 <= cus * 3)) e = launch_gemm_dma<128, 128, 2, 2, false, 5, false, false, false, 1, true>(lc, gg, (uint32_t)t128);
+          // A round of 128 rows.  The four wavefronts' longer start and tail pay from about 24 k-steps on (weights from memory: 900 x
+          // 2048 x 8192 in two slices 44.4 -> 37.4 us, 700 40.9 -> 36.3, 300 in four 23.2 -> 21.7, 400 x 1152 x 6912 in four - 27 steps -
+          // 18.9 -> 18.2; 18 steps 14.8, 16.0; 16 steps 14.1, 15.7 and 14.8, 16.6).
+          if (steps >= 24) e = launch_gemm_dma<128, 128, 2, 2, false, 5, false, false, false, 1, true>(lc, gg, (uint32_t)t128);
           else e = launch_gemm_dma<128, 128, 2, 4, false, 4>(lc, gg, (uint32_t)t128);
         } else if (t192 <= cus && steps >= 4) {
           // a round of 192 rows (o_proj and down_proj of 2900 rows: 29 and 91 us; 368 tiles of 128 rows two to a CU 35 and 122; 1024
