@@ -350,6 +350,20 @@ static bool gemm_small_ok(const LaunchCtx &lc, const GemmDesc &g) {
   return t32 <= 2 * (uint64_t)lc.n_cus && (g.M <= 32 || t32 * g.K <= 400 * 1024);
 }
 
+// An f32 product for k_gemm_f32.hip: all that it takes, unless the kernel above is ahead.  That one takes about 3 us and 13.5 ns per
+// k of a workgroup, half as much again when every CU has more than one, and 3 for a sum of slices (us here, 12 to 16 there: 10 x 512 x
+// 2048 9.5, 11; 64 x 256 x 128 4.4, 5.7; 2000 x 20 x 2000 11.5, 17; 300 x 1000 x 500 13.9, 11.2; 17 x 2048 x 2048 15.5, 12.7).
+static uint32_t gemm_small_split(const LaunchCtx &lc, const GemmDesc &g);
+static bool gemm_f32_tiles(const LaunchCtx &lc, const GemmDesc &g) {
+  if (!gemm_f32_ok(g)) return false;
+  if (!gemm_small_ok(lc, g)) return true;
+  const uint32_t s = gemm_small_split(lc, g);
+  const uint64_t wgs = (uint64_t)((g.M + 31) / 32) * ((g.N + 31) / 32) * g.nb0 * g.nb1 * s;
+  double us = 0;
+  gemm_f32_split(lc, g, &us);
+  return us < 3.0 + 0.0135 * g.K / s * (wgs > (uint64_t)lc.n_cus ? 1.5 : 1.0) + (s > 1 ? 3.0 : 0.0);
+}
+
 // ---- bf16 x bf16 "NT" GEMM: the prefill fast path --------------------------------------------------
 // A[M, K] and B[N, K] both bf16 with unit stride along k (activations are narrowed once by
 // cast_bf16_kernel and the copy is shared by every GEMM that reads them; weights are stored
@@ -2989,6 +3003,14 @@ hipError_t launch_splitk_sum(const LaunchCtx &lc, const float *ws, float *c, uin
   return hipGetLastError();
 }
 
+// gemm_small_f32_kernel, deep and tiny: more workgroups along k while each wavefront keeps two 32-wide chunks
+static uint32_t gemm_small_split(const LaunchCtx &lc, const GemmDesc &g) {
+  const uint64_t t32 = (uint64_t)((g.M + 31) / 32) * ((g.N + 31) / 32) * g.nb0 * g.nb1;
+  uint32_t splits = 1;
+  while (t32 * splits * 2 <= (uint64_t)lc.n_cus && g.K / (splits * 2) >= 256 && splits < 64) splits *= 2;
+  return splits;
+}
+
 // Split-K factor for a problem too small to fill the CUs with 128x128 tiles (0/1 = none).
 // The caller provides g.workspace of splits * batch * M * N floats and sets g.splits/k_per_split.
 uint32_t gemm_split_k(const LaunchCtx &lc, const GemmDesc &g) {
@@ -2999,12 +3021,8 @@ uint32_t gemm_split_k(const LaunchCtx &lc, const GemmDesc &g) {
   const uint64_t tiles = (uint64_t)((g.M + 127) / 128) * ((g.N + 127) / 128) * batch;
   uint32_t splits = 1;
   if (gemv_rows_plain_ok(lc, g)) return 1;
-  if (gemm_small_ok(lc, g)) {
-    // deep and tiny: more workgroups along k while each wavefront keeps two 32-wide chunks
-    const uint64_t t32 = (uint64_t)((g.M + 31) / 32) * ((g.N + 31) / 32) * batch;
-    while (t32 * splits * 2 <= (uint64_t)lc.n_cus && g.K / (splits * 2) >= 256 && splits < 64) splits *= 2;
-    return splits;
-  }
+  if (gemm_f32_tiles(lc, g)) return gemm_f32_split(lc, g, nullptr);
+  if (gemm_small_ok(lc, g)) return gemm_small_split(lc, g);
   if (!gemm_fast_path(g, av, bv)) {
     // the generic kernel (f32 products): same idea, shorter k-steps, so thinner slices still pay
     if (g.M <= 8 || g.b_index || !g.K) return 1;
@@ -3302,6 +3320,13 @@ hipError_t launch_matmul(const LaunchCtx &lc_in, const GemmDesc &g, const char *
                 (const float *)g.workspace, g.c, n, gsplits, g.c_add, (int)g.act_sigmoid);
     }
   };
+  if (gemm_f32_tiles(lc, g)) {
+    if (kernel_name) *kernel_name = "gemm_mfma_f32";
+    hipError_t e = launch_gemm_f32(lc, g);
+    if (e != hipSuccess) return e;
+    sum_slices();
+    return hipGetLastError();
+  }
   if (gemm_small_ok(lc, g)) {
     if (kernel_name) *kernel_name = "gemm_mfma_f32";
     dim3 gr((g.N + 31) / 32, (g.M + 31) / 32, batch * gsplits);

@@ -363,6 +363,11 @@ struct GemmDesc {
 // half_height: the stacked gate / up of fewer rows on tiles of 128 x 256, K >= 192
 bool gemm_ring_ok(const GemmDesc &g);
 hipError_t launch_gemm_ring(const LaunchCtx &lc, const GemmDesc &g, bool half_height = false);
+// k_gemm_f32.hip: f32 products of operands in whole 16-byte pieces; gemm_f32_split: the slices of k it is fastest with (and how long
+// it then takes, about)
+bool gemm_f32_ok(const GemmDesc &g);
+uint32_t gemm_f32_split(const LaunchCtx &lc, const GemmDesc &g, double *us);
+hipError_t launch_gemm_f32(const LaunchCtx &lc, const GemmDesc &g);
 // split factor launch_matmul should be given for this problem (1 = none)
 uint32_t gemm_split_k(const LaunchCtx &lc, const GemmDesc &g);
 // whether launch_matmul would run this problem (splits as given) on the kernel that honours

@@ -1,0 +1,48 @@
+"""f32 products on tiles of 32 to 256 rows by 128 columns (k_gemm_f32.hip; Backend::matmul, ndarray.rs:549-615) against sums in
+64 bits: every height of tile, with the right operand along k (a weight) and along n, columns and rows that end inside a tile,
+depths that end inside a step, slices of k of which the last is shorter, batches, a sigmoid on the way out."""
+import numpy as np
+import pytest
+
+import vectors
+from test_f32_operands import assert_f32_sums
+
+lang, nn = vectors.cg.lang, vectors.cg.nn
+
+
+def product(rank, along_k, act=False):
+    def f(b, x, w):
+        y = lang.matmul(b, x, lang.transpose(b, rank - 2, rank - 1, w) if along_k else w)
+        return [nn.sigmoid(b, y) if act else y]
+    return f
+
+
+SIZES = [(1, 33, 132, 1044), (3, 70, 260, 100), (1, 520, 900, 2060), (1, 1000, 1000, 1000),     # 32 and 64 rows
+         (1, 96, 32000, 132), (1, 256, 32000, 60), (1, 155, 32700, 100), (1, 700, 2048, 4100),  # 96, 128, 160, 192 rows
+         (1, 220, 30000, 100), (1, 8190, 4096, 44), (32, 300, 300, 64)]                         # 224, 256 rows; many products
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("along_k", [True, False])
+@pytest.mark.parametrize("B,M,N,K", SIZES)
+def test_product(hip, B, M, N, K, along_k):
+    g = np.random.default_rng(M + K)
+    x = g.standard_normal((B, M, K)).astype(np.float32)
+    w = g.standard_normal((B, N, K) if along_k else (B, K, N)).astype(np.float32)
+    if B == 1:
+        x, w = x[0], w[0]
+    (got,) = vectors.run(hip, product(x.ndim, along_k), 1, x, w)
+    exact = np.matmul(x.astype(np.float64), (np.swapaxes(w, -1, -2) if along_k else w).astype(np.float64))
+    assert_f32_sums(exact, got, K, f"{B} x {M} x {N} x {K}")
+
+
+# one launch and slices whose sum applies it; the error of a sigmoid is at most a quarter of its argument's, and its own rounding
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(1000, 1000, 1000), (300, 1000, 2060)])
+def test_sigmoid(hip, M, N, K):
+    g = np.random.default_rng(M)
+    x, w = g.standard_normal((M, K)).astype(np.float32), (g.standard_normal((K, N)) * K ** -0.5).astype(np.float32)
+    (got,) = vectors.run(hip, product(2, False, True), 1, x, w)
+    exact = 1 / (1 + np.exp(-(x.astype(np.float64) @ w.astype(np.float64))))
+    # (terms of size K^-1/2: their sums are off by 4 sqrt(K) 2^-24 of K^1/2 K^-1/2 at most; f32 exp and division: 4 units)
+    assert np.abs(got - exact).max() <= 0.25 * 4 * np.sqrt(K) * 2.0 ** -24 + 4 * 2.0 ** -24
