@@ -64,14 +64,24 @@ struct KeyTiles {
   uint32_t cols, t;
   uint64_t live[2], zero[2];  // bit i of word w: tile 64 w + i is not dead / needs no mask values
   bool bits;
+  uint32_t c0, c1;
+  // asks for the row; what is asked for between here and arrived() travels with it
   __device__ __forceinline__ KeyTiles(const AttnPrefillDesc &a, uint32_t q_tile, int lane) {
     cls = a.tile_class ? a.tile_class + (size_t)q_tile * a.tile_cols : nullptr;
     cols = a.tile_cols;
     t = a.t;
     bits = cls && cols <= 128;
+    c0 = c1 = 0;
+    if (bits) {
+      c0 = cls[min((uint32_t)lane, cols - 1)];
+      c1 = cls[min((uint32_t)lane + 64, cols - 1)];
+    }
+  }
+  __device__ __forceinline__ void arrived(int lane) {
     live[0] = live[1] = zero[0] = zero[1] = 0;
     if (bits) {
-      const uint8_t c0 = (uint32_t)lane < cols ? cls[lane] : 0, c1 = (uint32_t)lane + 64 < cols ? cls[lane + 64] : 0;
+      if ((uint32_t)lane >= cols) c0 = 0;
+      if ((uint32_t)lane + 64 >= cols) c1 = 0;
       live[0] = __ballot(c0 != 0);
       live[1] = __ballot(c1 != 0);
       zero[0] = __ballot(c0 == 2);
@@ -206,8 +216,9 @@ __device__ __forceinline__ float attn_softmax_step(const AttnPrefillDesc &a, a_f
 // BN keys per step.  The K / V rows of step i + 1 are in registers, asked for a step ago, while step i is computed from
 // one LDS buffer, and go to the other buffer behind its first product: one barrier per step.
 // NW waves of 32 queries each per workgroup (4, or 2 when that is what it takes to occupy the CUs).
-// KG = 2: half of the waves share 64 queries with the other half and take every other live step of them, with tiles of their own;
+// KG = 2: half of the waves share their queries with the other half and take every other live step of them, with tiles of their own;
 // the partial results meet once, in LDS.  The longest query tile of a causal mask is then half as long.
+// DS = 2: two waves share 32 queries, each with half of the values' dims.
 // Workgroups: the query tiles with the most keys first (a causal mask gives the last tile all of them), and the heads of a
 // (batch, kv head) on one XCD, whose L2 then holds their keys and values.
 // (the register budget of two waves to a SIMD keeps the accumulators of heads of 64 and 128 out of the accumulation file,
@@ -215,18 +226,20 @@ __device__ __forceinline__ float attn_softmax_step(const AttnPrefillDesc &a, a_f
 // step take turns between accumulators: 2900 tokens of 32 heads, causal, 90 us a layer where two waves and one chain after the
 // other took 97, 4000 tokens 131 for 154)
 #define ATTN_WAVES(n) __attribute__((amdgpu_waves_per_eu(n, n)))
-template <int D, int BN, int NW, int KG = 1>
-__global__ void __launch_bounds__(NW * 64) ATTN_WAVES((D > 128 ? 1 : D == 64 && NW == 4 && (KG == 1 || BN == 32) ? 3 : 2)) attn_prefill_kernel(AttnPrefillDesc a) {
-  constexpr int NT = NW * 64 / KG, QROWS = NW / KG * 32;  // threads of a key group, queries of the workgroup
+template <int D, int BN, int NW, int KG = 1, int DS = 1>
+__global__ void __launch_bounds__(NW * 64) ATTN_WAVES((D == 64 && NW == 4 && (KG == 1 || BN == 32) ? 3 : 2)) attn_prefill_kernel(AttnPrefillDesc a) {
+  warm_kernel_arguments<sizeof(AttnPrefillDesc)>();
+  constexpr int NT = NW * 64 / KG, NQ = NW / KG / DS, QROWS = NQ * 32;  // threads of a key group; query groups, queries of the workgroup
   constexpr int KP = D + 8;              // K tile row pitch (bf16 elements)
   constexpr int VP = BN + 8;             // V^T tile row pitch
-  constexpr int DT = D / 32;             // 32-row tiles of O^T
+  constexpr int DT = D / 32 / DS;        // 32-row tiles of O^T of a wave
   constexpr int KT = BN / 32;            // 32-key tiles of S^T
   constexpr int KCH = BN * D / 8 / NT;   // 16-byte chunks of the K tile / of the V^T tile per thread
   constexpr int TILE = BN * KP + D * VP;
   __shared__ __attribute__((aligned(16))) uint16_t tile[KG][2][TILE];
   const int lane = threadIdx.x & 63, all_waves = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int kg = KG == 1 ? 0 : all_waves / (NW / KG), wave = KG == 1 ? all_waves : all_waves % (NW / KG), tid = wave * 64 + lane;
+  const int kg = KG == 1 ? 0 : all_waves / (NW / KG), of_group = KG == 1 ? all_waves : all_waves % (NW / KG), tid = of_group * 64 + lane;
+  const int wave = DS == 1 ? of_group : of_group % NQ, dim0 = DS == 1 ? 0 : of_group / NQ * (D / DS);
   const int col = lane & 31, half = lane >> 5;
   const uint32_t n_bh = a.heads * a.b, q_tiles = (a.s + QROWS - 1) / QROWS;
   const uint32_t rank = blockIdx.x / n_bh, slot = blockIdx.x - rank * n_bh, q_tile = q_tiles - 1 - rank;
@@ -250,7 +263,16 @@ __global__ void __launch_bounds__(NW * 64) ATTN_WAVES((D > 128 ? 1 : D == 64 && 
   // consumed.  With a class table, dead key tiles are never visited and all-zero ones need no mask values.  This thread's first
   // chunk of each tile is kept as a pointer; a step without the end of the keys in it is a scalar away from there (with every
   // index clamped and every product taken in every step, a quarter of the step's vector instructions).
-  const KeyTiles<BN> tiles(a, q_tile, lane);
+  KeyTiles<BN> tiles(a, q_tile, lane);
+  // this lane's query row as B fragments: k-step ks covers dims 16 ks .. 16 ks + 15, half h takes 8 (lanes past the end repeat the
+  // last row; what they compute goes nowhere)
+  float4 qx[D / 8];
+#pragma unroll
+  for (int ks = 0; ks < D / 16; ++ks) {
+    qx[2 * ks] = *(const float4 *)(Q + ks * 16 + half * 8);
+    qx[2 * ks + 1] = *(const float4 *)(Q + ks * 16 + half * 8 + 4);
+  }
+  tiles.arrived(lane);
   constexpr int KROWS = NT * 8 / D, VROWS = NT * 8 / BN;  // rows of the K tile, of the V^T tile, between a thread's chunks
   const uint32_t k_row = tid / (D / 8), k_d8 = (tid % (D / 8)) * 8, v_row = tid / (BN / 8), v_k8 = (tid % (BN / 8)) * 8;
   const char *kp = (const char *)(K + (int64_t)k_row * a.k_st + k_d8), *vp = (const char *)(VT + (int64_t)v_row * a.vt_st + v_k8);
@@ -285,18 +307,11 @@ __global__ void __launch_bounds__(NW * 64) ATTN_WAVES((D > 128 ? 1 : D == 64 && 
   uint32_t t0 = tiles.skip(tiles.next_step(0), kg), t_next = a.t;
   if (t0 < a.t) fetch(t0);  // (uniform)
 
-  // this lane's query row as B fragments: k-step ks covers dims 16 ks .. 16 ks + 15, half h takes 8
   a_bf16x8 qf[D / 16];
 #pragma unroll
   for (int ks = 0; ks < D / 16; ++ks) {
-    float v[8];
-    if (q_ok) {
-      const float4 x0 = *(const float4 *)(Q + ks * 16 + half * 8), x1 = *(const float4 *)(Q + ks * 16 + half * 8 + 4);
-      v[0] = x0.x; v[1] = x0.y; v[2] = x0.z; v[3] = x0.w; v[4] = x1.x; v[5] = x1.y; v[6] = x1.z; v[7] = x1.w;
-    } else {
-#pragma unroll
-      for (int i = 0; i < 8; ++i) v[i] = 0.f;
-    }
+    const float4 x0 = qx[2 * ks], x1 = qx[2 * ks + 1];
+    const float v[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
     qf[ks] = pack8(v);
   }
   a_f32x16 o[DT];
@@ -327,7 +342,7 @@ __global__ void __launch_bounds__(NW * 64) ATTN_WAVES((D > 128 ? 1 : D == 64 && 
     // (checked by the host).  A step whose every pair is masked - possible only without a class table - needs no
     // special case: its weights exp(f32::MIN - m) are zero once any live key has been seen, and a row that never
     // sees one is rebuilt at the end.
-    constexpr bool LATE = D == 128 || (D == 64 && NW == 4 && (KG == 1 || BN == 32));
+    constexpr bool LATE = D > 64 || (D == 64 && NW == 4 && (KG == 1 || BN == 32));
     float4 mcur[KT][4];
     if (use_mask && !LATE) {
 #pragma unroll
@@ -371,7 +386,7 @@ __global__ void __launch_bounds__(NW * 64) ATTN_WAVES((D > 128 ? 1 : D == 64 && 
 #pragma unroll
       for (int t = 0; t < DT; ++t) {
         // A fragment: row = dim t*32 + col, the lane's eight keys of this block in the permuted order
-        const uint16_t *vr = &Vt[(t * 32 + col) * VP + blk * 16 + half * 4];
+        const uint16_t *vr = &Vt[(dim0 + t * 32 + col) * VP + blk * 16 + half * 4];
         union {
           uint2 u[2];
           a_bf16x8 hv;
@@ -385,8 +400,8 @@ __global__ void __launch_bounds__(NW * 64) ATTN_WAVES((D > 128 ? 1 : D == 64 && 
   }
   l_run = sum_of_halves(l_run);
   if constexpr (KG == 2) {  // the second group's partial results, [register][lane], join the first's
-    float *part = (float *)&tile[0][0][0] + wave * (DT * 16 + 2) * 64;
-    static_assert((NW / 2) * (DT * 16 + 2) * 64 * 4 <= 2 * 2 * TILE * 2, "partial results fit in the tiles");
+    float *part = (float *)&tile[0][0][0] + of_group * (DT * 16 + 2) * 64;
+    static_assert((NW / KG) * (DT * 16 + 2) * 64 * 4 <= 2 * 2 * TILE * 2, "partial results fit in the tiles");
     if (kg) {  // (everyone is past the barrier behind the last step)
       part[lane] = m_run;
       part[64 + lane] = l_run;
@@ -419,7 +434,7 @@ __global__ void __launch_bounds__(NW * 64) ATTN_WAVES((D > 128 ? 1 : D == 64 && 
       for (int t = 0; t < DT; ++t)
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-          const float4 vv = *(const float4 *)(V + (int64_t)key * a.v_st + t * 32 + j * 8 + half * 4);
+          const float4 vv = *(const float4 *)(V + (int64_t)key * a.v_st + dim0 + t * 32 + j * 8 + half * 4);
           o[t][j * 4 + 0] += vv.x; o[t][j * 4 + 1] += vv.y; o[t][j * 4 + 2] += vv.z; o[t][j * 4 + 3] += vv.w;
         }
   }
@@ -435,7 +450,7 @@ __global__ void __launch_bounds__(NW * 64) ATTN_WAVES((D > 128 ? 1 : D == 64 && 
         float4 r;
         r.x = o[t][j * 4 + 0] / l_run; r.y = o[t][j * 4 + 1] / l_run;
         r.z = o[t][j * 4 + 2] / l_run; r.w = o[t][j * 4 + 3] / l_run;
-        const int dim = t * 32 + j * 8 + half * 4;
+        const int dim = dim0 + t * 32 + j * 8 + half * 4;
         *(float4 *)(out + dim) = r;
         if (out16) *(uint2 *)(out16 + dim) = bf16_pack4(r);
       }
@@ -451,6 +466,7 @@ __global__ void __launch_bounds__(NW * 64) ATTN_WAVES((D > 128 ? 1 : D == 64 && 
 template <int D, int BN, int NW>
 __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))  // two workgroups per CU
 attn_prefill_keysplit_kernel(AttnPrefillDesc a) {
+  warm_kernel_arguments<sizeof(AttnPrefillDesc)>();
   constexpr int KP = D + 8;
   constexpr int VP = BN + 8;
   constexpr int DT = D / 32;
@@ -473,7 +489,20 @@ attn_prefill_keysplit_kernel(AttnPrefillDesc a) {
   const float *V = a.v + (int64_t)b * a.v_sb + (int64_t)kvh * a.v_skv + (int64_t)rp * a.v_srep;
   const float *M = a.mask ? a.mask + (int64_t)b * a.m_sb + (int64_t)h * a.m_sh + (int64_t)qc * a.m_ss : nullptr;
 
-  const KeyTiles<BN> tiles(a, blockIdx.x, lane);
+  KeyTiles<BN> tiles(a, blockIdx.x, lane);
+  // The queries: each wave converts a quarter of the workgroup's 32 rows (16 bytes of bf16 per lane and
+  // piece), the rows meet in LDS, and every wave reads its B fragments from there - a quarter of the loads
+  // of every wave fetching every row.  (Rows past the end repeat the last; what they compute goes nowhere.)
+  constexpr int QP = D + 8, QC = 32 * D / 8 / (NW * 64);  // row pitch (bf16 elements), pieces of a lane
+  float4 qx[QC][2];
+#pragma unroll
+  for (int c = 0; c < QC; ++c) {
+    const int ch = tid + c * NW * 64, r = ch / (D / 8), d8 = (ch % (D / 8)) * 8;
+    const float *qr = a.q + (int64_t)b * a.q_sb + (int64_t)h * a.q_sh + (int64_t)min(blockIdx.x * 32 + r, a.s - 1) * a.q_ss + d8;
+    qx[c][0] = *(const float4 *)qr;
+    qx[c][1] = *(const float4 *)(qr + 4);
+  }
+  tiles.arrived(lane);
   auto step_mask = [&](uint32_t t0) { return M && tiles.reads_mask(t0); };
   uint4 kreg[KCH], vreg[KCH];
   auto fetch = [&](uint32_t t0) {
@@ -489,29 +518,12 @@ attn_prefill_keysplit_kernel(AttnPrefillDesc a) {
     }
   };
   uint32_t t0 = tiles.skip(tiles.next_step(0), wave);
-  if (t0 < a.t) fetch(t0);  // asked for before the queries: one round trip for both
-
-  // The queries: each wave converts a quarter of the workgroup's 32 rows (16 bytes of bf16 per lane and
-  // piece), the rows meet in LDS, and every wave reads its B fragments from there - a quarter of the loads
-  // of every wave fetching every row.
-  constexpr int QP = D + 8;  // row pitch (bf16 elements)
-  {
-    const float *Q0 = a.q + (int64_t)b * a.q_sb + (int64_t)h * a.q_sh;
+  if (t0 < a.t) fetch(t0);
 #pragma unroll
-    for (int c = 0; c < 32 * D / 8 / (NW * 64); ++c) {
-      const int ch = tid + c * NW * 64, r = ch / (D / 8), d8 = (ch % (D / 8)) * 8;
-      const uint32_t row = blockIdx.x * 32 + r;
-      float v[8];
-      if (row < a.s) {
-        const float *qr = Q0 + (int64_t)row * a.q_ss + d8;
-        const float4 x0 = *(const float4 *)qr, x1 = *(const float4 *)(qr + 4);
-        v[0] = x0.x; v[1] = x0.y; v[2] = x0.z; v[3] = x0.w; v[4] = x1.x; v[5] = x1.y; v[6] = x1.z; v[7] = x1.w;
-      } else {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) v[e] = 0.f;
-      }
-      *(a_bf16x8 *)(&qs[r * QP + d8]) = pack8(v);
-    }
+  for (int c = 0; c < QC; ++c) {
+    const int ch = tid + c * NW * 64, r = ch / (D / 8), d8 = (ch % (D / 8)) * 8;
+    const float v[8] = {qx[c][0].x, qx[c][0].y, qx[c][0].z, qx[c][0].w, qx[c][1].x, qx[c][1].y, qx[c][1].z, qx[c][1].w};
+    *(a_bf16x8 *)(&qs[r * QP + d8]) = pack8(v);
   }
   __syncthreads();
   a_bf16x8 qf[D / 16];
@@ -721,7 +733,8 @@ __global__ void __launch_bounds__(NW * 64) attn_prefill_f32_kernel(AttnPrefillDe
 
   float4 treg[CH];
   float4 mreg[KT][4];
-  const KeyTiles<BN> tiles(a, blockIdx.x, lane);
+  KeyTiles<BN> tiles(a, blockIdx.x, lane);
+  tiles.arrived(lane);
   auto next_step = [&](uint32_t t0) { return tiles.next_step(t0); };
   auto step_mask = [&](uint32_t t0) { return M && tiles.reads_mask(t0); };
   // rows of K (or V) of the step at t0 into registers; rows past the end repeat the last one and are
@@ -928,13 +941,31 @@ static bool attn_prefill_keysplit(const LaunchCtx &lc, const AttnPrefillDesc &d)
          !attn_prefill_two_groups(lc, d);
 }
 
+// Heads of 128 and 256: two wavefronts to 32 queries, each with half of the values' dims (both compute the scores; the accumulators of
+// two waves then fit on a SIMD, and one's softmax runs under the other's products).  us a layer, heads of 128, causal, against one
+// wavefront to 32 queries: 16 heads of 400 tokens 24.0 -> 18.5, 1400 61.1 -> 49.2, 3000 109 -> 103, 4 x 256 20.5 -> 17.9; from about
+// one and a half workgroups of 128 queries a CU on the doubled scores weigh more (4 x 1000 52.3, 66.6).  Heads of 256: 4 heads of
+// 2000 tokens 75.5 -> 51.9, 8 x 1000 81.7 -> 61.1, 8 x 2048 152 -> 130.
+static bool attn_prefill_wide(const LaunchCtx &lc, const AttnPrefillDesc &d) {
+  return !d.f32 && (d.d == 256 || (d.d == 128 && 2 * (uint64_t)((d.s + 127) / 128) * d.heads * d.b <= 3 * (uint64_t)lc.n_cus));
+}
+// ... in two key groups of 32 or 64 queries (0: one group) while a CU has at most one such workgroup and the keys are more than a
+// step: 100 tokens of 16 heads of 128 10.5 -> 9.8, 400 18.5 -> 16.7, 900 33.9 -> 27.8; 4 heads of 256, 700 tokens 40.3 -> 34.1, 2000
+// 51.9 -> 44.1, 4 x 1000 45.3 -> 40.4 (64 queries; 32 in two rounds 64).
+static int attn_prefill_wide_groups(const LaunchCtx &lc, const AttnPrefillDesc &d) {
+  if (!attn_prefill_wide(lc, d) || d.t <= (d.d == 128 ? 64u : 32u)) return 0;
+  if ((uint64_t)((d.s + 31) / 32) * d.heads * d.b <= (uint64_t)lc.n_cus) return 32;
+  return (uint64_t)((d.s + 63) / 64) * d.heads * d.b <= (uint64_t)lc.n_cus ? 64 : 0;
+}
+
 static bool attn_prefill_small_tiles(const LaunchCtx &lc, const AttnPrefillDesc &d) {
   if (d.f32 && d.d == 256) return true;  // its queries live in LDS: 64 of them fit beside the K / V tile
   return (uint64_t)((d.s + 127) / 128) * d.heads * d.b < (uint64_t)lc.n_cus;  // too few workgroups of 128 queries: 64 each
 }
 
 void attn_prefill_tiling(const LaunchCtx &lc, const AttnPrefillDesc &d, uint32_t *q_rows, uint32_t *keys) {
-  *q_rows = attn_prefill_keysplit(lc, d) ? 32 : attn_prefill_small_tiles(lc, d) || attn_prefill_two_groups(lc, d) ? 64 : 128;
+  if (attn_prefill_keysplit(lc, d) || attn_prefill_wide_groups(lc, d) == 32) *q_rows = 32;
+  else *q_rows = attn_prefill_wide(lc, d) || attn_prefill_small_tiles(lc, d) || attn_prefill_two_groups(lc, d) ? 64 : 128;
   *keys = attn_prefill_two_groups(lc, d) ? attn_prefill_two_groups_keys(lc, d) : (d.d == 256 || (d.f32 && d.d == 128)) ? 32 : 64;
 }
 
@@ -996,7 +1027,19 @@ hipError_t launch_attn_prefill(const LaunchCtx &lc, const AttnPrefillDesc &d) {
     else CG_LAUNCH(lc, (attn_prefill_kernel<64, 64, 4, 2>), grid, 256, d);
     return hipGetLastError();
   }
-  const bool small = attn_prefill_small_tiles(lc, d);
+  if (attn_prefill_wide(lc, d)) {
+    const int groups = attn_prefill_wide_groups(lc, d);
+    const uint32_t bh = d.heads * d.b, g32 = (d.s + 31) / 32 * bh, g64 = (d.s + 63) / 64 * bh;
+#define CG_ATTN_WIDE(DD, BN)                                                                        \
+    if (groups == 32) CG_LAUNCH(lc, (attn_prefill_kernel<DD, BN, 4, 2, 2>), g32, 256, d);           \
+    else if (groups == 64) CG_LAUNCH(lc, (attn_prefill_kernel<DD, BN, 8, 2, 2>), g64, 512, d);      \
+    else CG_LAUNCH(lc, (attn_prefill_kernel<DD, BN, 4, 1, 2>), g64, 256, d);
+    if (d.d == 128) { CG_ATTN_WIDE(128, 64) }
+    else { CG_ATTN_WIDE(256, 32) }
+#undef CG_ATTN_WIDE
+    return hipGetLastError();
+  }
+  const bool small = attn_prefill_small_tiles(lc, d);  // (f32 only: bf16 products of so few rows are gone by now)
   dim3 grid(small ? (d.s + 63) / 64 : (d.s + 127) / 128, d.heads, d.b);
   if (!d.f32) grid = dim3(grid.x * d.heads * d.b);
 #define CG_ATTN_CASE(DD, ...)                                               \
@@ -1013,9 +1056,8 @@ hipError_t launch_attn_prefill(const LaunchCtx &lc, const AttnPrefillDesc &d) {
     }
   } else {
     switch (d.d) {
-      CG_ATTN_CASE(64, attn_prefill_kernel<64, 64)
-      CG_ATTN_CASE(128, attn_prefill_kernel<128, 64)
-      CG_ATTN_CASE(256, attn_prefill_kernel<256, 32)
+      case 64: CG_LAUNCH(lc, (attn_prefill_kernel<64, 64, 4>), grid, 256, d); break;
+      case 128: CG_LAUNCH(lc, (attn_prefill_kernel<128, 64, 4>), grid, 256, d); break;
       default: return hipErrorInvalidValue;
     }
   }

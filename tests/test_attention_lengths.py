@@ -191,15 +191,18 @@ def attention_in_numpy(q, k, v, hidden, rep):
     return out
 
 
-# Two key groups of a query tile: 64 and 32 keys a step (by how many workgroups there are), key tiles seen by none, some or all of
+# Heads of 64 in two key groups of a query tile, 64 and 32 keys a step (by how many workgroups there are); heads of 128 and 256 as two
+# halves of the values' dims, in two key groups of 32 or 64 queries, in one, and many heads of 128 undivided.  Key tiles seen by none, some or all of
 # a query tile's rows at random (odd numbers of live steps, a group without any), rows that see no key at all, and more key tiles
 # than the bit masks hold (T = 4100), heads that do not divide by the dies.
 @pytest.mark.gpu
-@pytest.mark.parametrize("H,KV,S,T", [(48, 6, 321, 321), (65, 13, 257, 257), (64, 8, 641, 641), (322, 2, 65, 4100)])
-def test_two_key_groups(hip_bf16, H, KV, S, T):
+@pytest.mark.parametrize("H,KV,S,T,d", [(48, 6, 321, 321, 64), (65, 13, 257, 257, 64), (64, 8, 641, 641, 64), (322, 2, 65, 4100, 64),
+                                         (16, 4, 200, 200, 128), (64, 8, 193, 193, 128), (80, 8, 200, 200, 128), (200, 8, 257, 257, 128),
+                                         (4, 1, 200, 200, 256), (62, 2, 193, 193, 256), (80, 8, 131, 131, 256), (4, 4, 40, 33, 256)])
+def test_parts_of_a_query_tile(hip_bf16, H, KV, S, T, d):
     g = np.random.default_rng(S + T)
-    q = vectors.bf16_round(g.standard_normal((1, H, S, 64)).astype(np.float32))
-    k, v = (vectors.bf16_round(g.standard_normal((1, KV, T, 64)).astype(np.float32)) for _ in range(2))
+    q = vectors.bf16_round(g.standard_normal((1, H, S, d)).astype(np.float32))
+    k, v = (vectors.bf16_round(g.standard_normal((1, KV, T, d)).astype(np.float32)) for _ in range(2))
     tiles = g.integers(0, 3, ((S + 63) // 64, (T + 31) // 32))       # 0: hidden, 1: in part, 2: seen
     tiles[0] = 0
     tiles[0, (T - 1) // 32] = 2                                       # one live step for the first 64 queries
