@@ -3251,15 +3251,26 @@ hipError_t launch_matmul(const LaunchCtx &lc_in, const GemmDesc &g, const char *
           // q / k / v rotated: eight wavefronts share the long tail - 64 KB of tile through LDS, table rows from L2 -, and once there
           // are more tiles than CUs two workgroups of two stages share a CU, one's tail under the other's main loop.  (With four
           // wavefronts and the main loop in one statement, weights from memory: 700 rows of 3072 columns 27.2 -> 28.8 us, 1300 38.8 ->
-          // 39.6; 6144 columns of heads of 128, 200 rows 27.7 -> 33.4, 600 32.2 -> 40.0, 960 45.2 -> 55.6.)  Few tiles and heads of
-          // 64: 64 columns a tile (512 rows 18.3, 21.8).
-          if (splits == 1 && t128 * 2 <= cus && g.rope_hd == 64)
+          // 39.6; 6144 columns of heads of 128, 200 rows 27.7 -> 33.4, 600 32.2 -> 40.0, 960 45.2 -> 55.6.)
+          // Less than a round: what a workgroup takes in of both operands is what the launch waits for, so the tile of the fewest rows
+          // and columns of which every CU holds one.  3072 columns of heads of 64 on 64 x 64: 140 rows 16.6 -> 13.6 us, 310 19.4 ->
+          // 16.6 (128 x 64), beyond that 128 x 64 (512 rows 18.3, 128 x 128 21.8); 6144 columns of heads of 128 on 64 x 128: 140
+          // rows 26.0 -> 18.8, 310 30.3 -> 23.9 (128 x 128).  (256 x 128 where 128 x 128 are two to a CU: 1024 rows 46.2 -> 53.1.)
+          const uint64_t m64 = (g.M + 63) / 64, n64 = (g.N + 63) / 64, n128 = (g.N + 127) / 128;
+          if (g.rope_hd == 64 && m64 * n64 <= cus)
+            e = launch_gemm_dma<64, 64, 2, 2, false, 8, false, false, true, 2>(lc, gg, (uint32_t)(m64 * n64));
+          else if (g.rope_hd == 128 && m64 * n128 <= cus)
+            e = launch_gemm_dma<64, 128, 2, 4, false, 6, false, false, true>(lc, gg, (uint32_t)(m64 * n128));
+          else if (splits == 1 && t128 * 2 <= cus && g.rope_hd == 64)
             e = launch_gemm_dma<128, 64, 4, 2, false, 4, false, false, true>(lc, gg, (uint32_t)((uint64_t)((g.M + 127) / 128) * ((g.N + 63) / 64) * batch));
           else if (t128 <= cus) e = launch_gemm_dma<128, 128, 2, 4, false, 4, false, false, true>(lc, gg, (uint32_t)t128);
           else e = launch_gemm_dma<128, 128, 2, 4, false, 2, false, false, true>(lc, gg, (uint32_t)t128);
         } else if (splits == 1 && t128 * 2 <= cus && g.N >= 128) {
-          // too few 128 x 128 tiles for the CUs and no split-K to multiply them: halve the tile
-          e = launch_gemm_dma<128, 64, 4, 2, false, 4>(lc, gg, (uint32_t)((uint64_t)((g.M + 127) / 128) * ((g.N + 63) / 64) * batch));
+          // too few 128 x 128 tiles for the CUs and no split-K to multiply them: halve the tile, or quarter it if every CU still holds
+          // one at most (1536 columns, K = 1152: 100 rows 11.2 -> 9.5 us, 400 11.3 -> 9.6, 640 11.3 -> 10.1)
+          const uint64_t t64 = (uint64_t)((g.M + 63) / 64) * ((g.N + 63) / 64) * batch;
+          e = t64 <= cus ? launch_gemm_dma<64, 64, 2, 2, false, 8, false, false, false, 2>(lc, gg, (uint32_t)t64)
+                         : launch_gemm_dma<128, 64, 4, 2, false, 4>(lc, gg, (uint32_t)((uint64_t)((g.M + 127) / 128) * ((g.N + 63) / 64) * batch));
         } else if (t128 <= cus) {
           // A round of 128 rows.  The four wavefronts' longer start and tail pay from about 24 k-steps on (weights from memory: 900 x
           // 2048 x 8192 in two slices 44.4 -> 37.4 us, 700 40.9 -> 36.3, 300 in four 23.2 -> 21.7, 400 x 1152 x 6912 in four - 27 steps -

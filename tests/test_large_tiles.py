@@ -114,15 +114,16 @@ def test_sigmoid_as_the_next_operand(hip_bf16, M, K, H):
     assert np.all(np.abs(got - ref) <= 2.0 ** -8 * ref + 1e-5)    # (as above)
 
 
-# a round of tiles that rotate and more than one, heads of 64 and of 128, with and without biases, several
+# less than a round of tiles that rotate, one, more than one, heads of 64 and of 128, with and without biases, several
 # sequences, positions in no multiple of four
 @pytest.mark.gpu
-def test_rotated(oracle, hip_bf16):
-    llama_tests.test_llama_prefill_rotates_in_the_projections_launch(oracle, hip_bf16, 1601, 16, 16, 1)
+@pytest.mark.parametrize("tokens", [1601, 318, 130])
+def test_rotated(oracle, hip_bf16, tokens):
+    llama_tests.test_llama_prefill_rotates_in_the_projections_launch(oracle, hip_bf16, tokens, 16, 16, 1)
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("batch,tokens", [(2, 301), (3, 550)])
+@pytest.mark.parametrize("batch,tokens", [(2, 301), (3, 550), (1, 317), (2, 65)])
 def test_rotated_wide_heads(oracle, hip_bf16, batch, tokens):
     moe_tests.test_qwen_prefill_biases_and_rotation_in_the_projections_launch(oracle, hip_bf16, batch, tokens, 8, 8, 128)
 
