@@ -1134,18 +1134,20 @@ struct SumTerm {
   bool sigmoid;
 };
 
-// rows of `d` values with at most one leading axis longer than 1: views between such shapes keep the row order
-bool rows_shape(const cg_tensor *t, int64_t d) {
-  if (t->rank < 1 || t->shape[t->rank - 1] != d) return false;
+// rows of `d` values: reshapes between such shapes keep the row order
+bool rows_shape(const cg_tensor *t, int64_t d) { return t->rank >= 1 && t->shape[t->rank - 1] == d; }
+// ... with at most one leading axis longer than 1: so do transposes
+bool one_rows_axis(const cg_tensor *t) {
   int big = 0;
   for (int i = 0; i + 1 < t->rank; ++i) big += t->shape[i] != 1;
   return big <= 1;
 }
 
-// through deferred reshapes / transposes that nobody else reads and that only move axes of extent 1
+// through deferred reshapes of rows, and transposes that only move axes of extent 1, that nobody else reads
 cg_tensor *under_unit_views(cg_tensor *n, const cg_tensor *root, int64_t d) {
   while ((n->op == N_RESHAPE || n->op == N_TRANSPOSE) && (n == root || refs(n) == 1) && n->in[0] &&
-         n->in[0]->size() == n->size() && rows_shape(n, d) && rows_shape(n->in[0], d))
+         n->in[0]->size() == n->size() && rows_shape(n, d) && rows_shape(n->in[0], d) &&
+         (n->op == N_RESHAPE || (one_rows_axis(n) && one_rows_axis(n->in[0]))))
     n = n->in[0];
   return n;
 }
@@ -1185,7 +1187,8 @@ bool sum_term(cg_tensor *n, const cg_tensor *root, int64_t rows, int64_t d, SumT
     }
     // the same still deferred: views, ending in a broadcast, of a value that takes a launch of its own whoever
     // reads it (the values a top-k chose); the caller checks the strides once the views are realised
-    if (sc->op == N_BROADCAST && refs(sc) == 1) {
+    const bool per_row = sc->op == N_BROADCAST && sc->in[0]->rank >= 1 && sc->in[0]->shape[sc->in[0]->rank - 1] == 1;
+    if (per_row && refs(sc) == 1) {
       const cg_tensor *src = sc->in[0];
       while ((src->op == N_RESHAPE || src->op == N_SLICE || src->op == N_TRANSPOSE || src->op == N_BROADCAST) && src->in[0])
         src = src->in[0];
@@ -1196,7 +1199,7 @@ bool sum_term(cg_tensor *n, const cg_tensor *root, int64_t rows, int64_t d, SumT
       }
     }
     const cg_tensor *arg = nullptr;
-    if (sc->op == N_BROADCAST && refs(sc) == 1 && sc->in[0]->size() == rows && is_sigmoid_of(sc->in[0], &arg) &&
+    if (per_row && refs(sc) == 1 && sc->in[0]->size() == rows && is_sigmoid_of(sc->in[0], &arg) &&
         arg->size() == rows) {
       out->x = x;
       out->s = const_cast<cg_tensor *>(arg);

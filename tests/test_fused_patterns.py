@@ -924,6 +924,40 @@ def test_sum_of_rows_scaled_by_their_own_values(oracle, hip, hip_nopat, rows, d,
     assert np.allclose(got, ref, rtol=1e-6, atol=1e-6)
 
 
+@pytest.mark.parametrize("B,S,d,k", [(2, 3, 64, 2), (4, 16, 64, 4), (3, 7, 260, 1)])
+def test_sum_of_scaled_rows_of_several_sequences(oracle, hip, hip_nopat, B, S, d, k):
+    """The same in a prefill of several sequences: the rows end in [B, S, d], where the residual is.  (4 x 16 rows of 64: a value
+    for each column of d is as many as there are rows, and is no scale of rows.)"""
+    rows = B * S
+    g = np.random.default_rng(rows + d + k)
+    hs = [g.standard_normal((rows, 1, d)).astype(np.float32) for _ in range(k)]
+    vals = g.random((rows, k)).astype(np.float32)
+    shared = g.standard_normal((1, rows, d)).astype(np.float32)
+    gate = g.standard_normal((1, rows, 1)).astype(np.float32)
+    res = g.standard_normal((B, S, d)).astype(np.float32)
+    cols = g.standard_normal((1, 1, d)).astype(np.float32)
+
+    def f(b, *a):
+        h, (v, sh, gt, rs, co) = a[:k], a[k:]
+        acc = h[0] * lang.broadcast(b, helpers.unsqueeze(b, 2, 2, lang.get(b, 1, 0, v)), lang.shape(b, h[0]))
+        for i in range(1, k):
+            acc = acc + h[i] * lang.broadcast(b, helpers.unsqueeze(b, 2, 2, lang.get(b, 1, i, v)), lang.shape(b, h[i]))
+        acc = lang.transpose(b, 0, 1, acc)
+        out = acc + sh * lang.broadcast(b, nn.sigmoid(b, gt), lang.shape(b, sh))
+        return lang.reshape(b, lang.shape(b, rs), out) + rs
+
+    def by_column(b, *a):
+        return f(b, *a) + a[k + 3] * lang.broadcast(b, nn.sigmoid(b, a[k + 4]), lang.shape(b, a[k + 3]))
+    args = (*hs, vals, shared, gate, res, cols)
+    (ref,) = vectors.run(oracle, f, 1, *args)
+    (got,), names = run_traced(hip, f, 1, *args)
+    (gen,) = vectors.run(hip_nopat, f, 1, *args)
+    assert names == {"row_scaled_sum"}, sorted(names)
+    assert got.shape == ref.shape and np.array_equal(got, gen), np.abs(got - gen).max()
+    (got,), (gen,) = vectors.run(hip, by_column, 1, *args), vectors.run(hip_nopat, by_column, 1, *args)
+    assert np.array_equal(got, gen), np.abs(got - gen).max()
+
+
 @pytest.mark.parametrize("variant", ["right_nested", "shared_term", "two_chains", "scale_on_the_left", "nine_terms"])
 def test_sum_of_scaled_rows_in_other_arrangements(hip, hip_nopat, variant):
     """Additions nested to the right, a term somebody else reads too, two chains under one addition, the scale as
