@@ -2340,8 +2340,11 @@ __global__ void __launch_bounds__(256) moe_gemm_kernel(MoeGemmDesc g) {
 }
 
 // ---- the same with the routing done once and the operands streamed like the dense GEMM ------------------
-// One workgroup of 1024 threads sorts the (slot, token) pairs by expert: a histogram in LDS, a scan,
-// and a scatter through per-expert cursors.  The order of an expert's pairs depends on the order
+// One workgroup of 1024 threads sorts the (slot, token) pairs by expert: a histogram in LDS, a scan, and a scatter.  What a
+// launch of one workgroup takes is its chain of round trips, so a thread keeps its first eight pairs - their expert and the
+// place the histogram's atomic gave them - in registers, and the two scans (pairs and row tiles) go together, in a wave and then
+// over the waves.  (60 experts, 4096 pairs 9.3 -> 7.7 us, 400 5.9 -> 4.4; before: a second pass over the choices, scans of twenty barriers.)
+// The order of an expert's pairs depends on the order
 // the atomics land in, which only decides the tile row a token occupies, never its result.
 // tiles (optional): tiles[0] = the number of row tiles (moe_tile_pairs pairs each) over all experts, tiles[1 + t] = expert << 16 |
 // row tile within the expert, expert by expert - the work list of the GEMM, one workgroup per (row tile, column
@@ -2350,7 +2353,9 @@ __global__ void __launch_bounds__(256) moe_gemm_kernel(MoeGemmDesc g) {
 __host__ __device__ constexpr uint32_t moe_tile_pairs(bool planes) { return planes ? 20 : 128; }
 __global__ void __launch_bounds__(1024) moe_route_kernel(MoeGemmDesc g, uint32_t *count, uint32_t *offset, uint32_t *list,
                                                          uint32_t *tiles, uint16_t *planes) {
-  __shared__ uint32_t hist[MOE_ROUTE_MAX_EXPERTS], cursor[MOE_ROUTE_MAX_EXPERTS], scan[1024];
+  constexpr int KEEP = 8;
+  __shared__ uint32_t hist[MOE_ROUTE_MAX_EXPERTS], cursor[MOE_ROUTE_MAX_EXPERTS];
+  __shared__ uint2 wave_sum[16];
   const uint32_t tid = threadIdx.x, E = g.n_expert, S = g.S, pairs = S * g.n_slot;
   if (blockIdx.x) {
     const uint32_t per_row = g.K / 4, n = S * per_row;
@@ -2361,59 +2366,83 @@ __global__ void __launch_bounds__(1024) moe_route_kernel(MoeGemmDesc g, uint32_t
     }
     return;
   }
+  auto expert_of = [&](uint32_t sl, uint32_t t) { return g.slot[sl].idx[(int64_t)t * g.slot[sl].idx_stride]; };
+  uint32_t kept[KEEP], place[KEEP];  // experts of pairs tid, tid + 1024, ..
+#pragma unroll
+  for (int j = 0; j < KEEP; ++j) {
+    const uint32_t p = tid + j * 1024;
+    if (p < pairs) kept[j] = expert_of(p / S, p % S);
+  }
   for (uint32_t i = tid; i < E; i += 1024) hist[i] = 0;
   __syncthreads();
-  for (uint32_t p = tid; p < pairs; p += 1024) {
-    const uint32_t sl = p / S, t = p - sl * S;
-    uint32_t ix = g.slot[sl].idx[(int64_t)t * g.slot[sl].idx_stride];
-    if (ix >= E) {
-      atomicOr(g.err, ERRF_INDEX_OOB);
-      ix = E - 1;
+#pragma unroll
+  for (int j = 0; j < KEEP; ++j)
+    if (tid + j * 1024 < pairs) {
+      if (kept[j] >= E) {
+        atomicOr(g.err, ERRF_INDEX_OOB);
+        kept[j] = E - 1;
+      }
+      place[j] = atomicAdd(&hist[kept[j]], 1u);
     }
-    atomicAdd(&hist[ix], 1u);
-  }
   __syncthreads();
-  const uint32_t per = (E + 1023) / 1024, first = tid * per;
-  uint32_t local = 0;
-  for (uint32_t i = first; i < min(E, first + per); ++i) local += hist[i];
-  scan[tid] = local;
-  __syncthreads();
-  for (uint32_t d = 1; d < 1024; d <<= 1) {
-    const uint32_t v = tid >= d ? scan[tid - d] : 0u;
+  const bool more = pairs > KEEP * 1024;  // (uniform)
+  if (more) {  // the pairs that are not kept lie behind those that are
+    for (uint32_t i = tid; i < E; i += 1024) cursor[i] = hist[i];
     __syncthreads();
-    scan[tid] += v;
+    for (uint32_t p = tid + KEEP * 1024; p < pairs; p += 1024) {
+      uint32_t ix = expert_of(p / S, p % S);
+      if (ix >= E) {
+        atomicOr(g.err, ERRF_INDEX_OOB);
+        ix = E - 1;
+      }
+      atomicAdd(&hist[ix], 1u);
+    }
     __syncthreads();
   }
-  uint32_t at = scan[tid] - local;
+  const uint32_t per = (E + 1023) / 1024, first = tid * per, tp = moe_tile_pairs(g.planes);
+  uint2 local = make_uint2(0, 0);  // pairs, row tiles of this thread's experts
   for (uint32_t i = first; i < min(E, first + per); ++i) {
-    count[i] = hist[i];
+    local.x += hist[i];
+    local.y += (hist[i] + tp - 1) / tp;
+  }
+  uint2 sum = local;
+  const int lane = tid & 63, wave = tid >> 6;
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const uint32_t x = __shfl_up(sum.x, d, 64), y = __shfl_up(sum.y, d, 64);
+    if (lane >= d) {
+      sum.x += x;
+      sum.y += y;
+    }
+  }
+  if (lane == 63) wave_sum[wave] = sum;
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < 15; ++w)
+    if (w < wave) {
+      sum.x += wave_sum[w].x;
+      sum.y += wave_sum[w].y;
+    }
+  uint32_t at = sum.x - local.x, tt = sum.y - local.y;
+  for (uint32_t i = first; i < min(E, first + per); ++i) {
+    const uint32_t n = hist[i];
+    count[i] = n;
     offset[i] = at;
-    cursor[i] = at;
-    at += hist[i];
+    if (more) cursor[i] += at;
+    hist[i] = at;
+    at += n;
+    if (tiles)
+      for (uint32_t j = 0; j < (n + tp - 1) / tp; ++j) tiles[1 + tt++] = i << 16 | j;
   }
+  if (tiles && tid == 1023) tiles[0] = sum.y;
   __syncthreads();
-  for (uint32_t p = tid; p < pairs; p += 1024) {
-    const uint32_t sl = p / S, t = p - sl * S;
-    const uint32_t ix = min(g.slot[sl].idx[(int64_t)t * g.slot[sl].idx_stride], E - 1);
-    list[atomicAdd(&cursor[ix], 1u)] = sl << 16 | t;
+#pragma unroll
+  for (int j = 0; j < KEEP; ++j) {
+    const uint32_t p = tid + j * 1024;
+    if (p < pairs) list[hist[kept[j]] + place[j]] = p / S << 16 | p % S;
   }
-  if (!tiles) return;
-  // the same scan over row tiles per expert
-  const uint32_t tp = moe_tile_pairs(g.planes);
-  uint32_t my_tiles = 0;
-  for (uint32_t i = first; i < min(E, first + per); ++i) my_tiles += (hist[i] + tp - 1) / tp;
-  scan[tid] = my_tiles;
-  __syncthreads();
-  for (uint32_t d = 1; d < 1024; d <<= 1) {
-    const uint32_t v = tid >= d ? scan[tid - d] : 0u;
-    __syncthreads();
-    scan[tid] += v;
-    __syncthreads();
-  }
-  uint32_t tt = scan[tid] - my_tiles;
-  for (uint32_t i = first; i < min(E, first + per); ++i)
-    for (uint32_t j = 0; j < (hist[i] + tp - 1) / tp; ++j) tiles[1 + tt++] = i << 16 | j;
-  if (tid == 1023) tiles[0] = scan[1023];
+  for (uint32_t p = tid + KEEP * 1024; p < pairs; p += 1024)
+    list[atomicAdd(&cursor[min(expert_of(p / S, p % S), E - 1)], 1u)] = p / S << 16 | p % S;
 }
 
 // most row tiles launch_moe_route can list for g: every expert may end in a partly filled one

@@ -129,10 +129,12 @@ def test_rotated_wide_heads(oracle, hip_bf16, batch, tokens):
 
 
 # the routed experts of a prefill, from 44 pairs to an expert on moe_ring_kernel: three slots whose choices crowd one expert (several row tiles, the last
-# partly filled) and leave others empty; the fewest k-steps, columns that end inside a tile of 128 and of 256
+# partly filled) and leave others empty; the fewest k-steps, columns that end inside a tile of 128 and of 256; more pairs than
+# moe_route_kernel keeps in registers, more experts than it has threads
 @pytest.mark.gpu
 @pytest.mark.parametrize("act", ["silu", "gelu"])
-@pytest.mark.parametrize("S,E,F,H", [(150, 6, 192, 192), (64, 9, 320, 576), (140, 9, 320, 576), (700, 5, 256, 192)])
+@pytest.mark.parametrize("S,E,F,H", [(150, 6, 192, 192), (64, 9, 320, 576), (140, 9, 320, 576), (700, 5, 256, 192),
+                                     (2800, 5, 64, 64), (300, 1100, 64, 64)])
 def test_routed_experts(oracle, hip_bf16, S, E, F, H, act):
     g = np.random.default_rng(S)
     x, k = draw(g, (S, 1, H)), 3
