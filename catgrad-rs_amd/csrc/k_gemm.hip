@@ -1038,6 +1038,41 @@ __global__ void __launch_bounds__(256) splitk_reduce_kernel(const float *ws, flo
   }
 }
 
+// One column: C[m] = A[m, :] . b, both bf16 along k (the gate of a MoE block's shared expert).  A wave to a row, four pieces of 16
+// bytes a lane on their way at once; bound by the chain of one row's loads and its sum (1024 x 1 x 2048: 64 x 64 tiles in sixteen
+// slices 4.7 us and their sum 4.8; 4.6 so, which is what a launch that waits for another takes).
+__global__ void __launch_bounds__(256) gemm_bf16_column_kernel(GemmDesc g) {
+  const uint32_t lane = threadIdx.x & 63, row = blockIdx.x * 4 + (threadIdx.x >> 6), bz = blockIdx.y;
+  if (row >= g.M) return;
+  const uint32_t b0 = bz / g.nb1, b1 = bz - b0 * g.nb1;
+  const uint16_t *A = (const uint16_t *)g.a + b0 * g.sa_b0 + b1 * g.sa_b1 + (int64_t)row * g.sam;
+  const uint16_t *B = (const uint16_t *)g.b + b0 * g.sb_b0 + b1 * g.sb_b1;
+  float s = 0.f;
+  for (uint32_t k0 = lane * 8; k0 < g.K; k0 += 2048) {
+    uint4 a[4], b[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const uint32_t k = k0 + u * 512;
+      a[u] = b[u] = make_uint4(0, 0, 0, 0);
+      if (k < g.K) {  // (K % 8 == 0)
+        a[u] = *(const uint4 *)(A + k);
+        b[u] = *(const uint4 *)(B + k);
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const uint32_t x[4] = {a[u].x, a[u].y, a[u].z, a[u].w}, y[4] = {b[u].x, b[u].y, b[u].z, b[u].w};
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        s = __builtin_fmaf(__uint_as_float(x[j] << 16), __uint_as_float(y[j] << 16), s);
+        s = __builtin_fmaf(__uint_as_float(x[j] & 0xFFFF0000u), __uint_as_float(y[j] & 0xFFFF0000u), s);
+      }
+    }
+  }
+  s = wave_sum(s);
+  if (lane == 0) g.c[(uint64_t)bz * g.M + row] = g.act_sigmoid ? sigmoid_ref(s) : s;
+}
+
 // An f32 as the sum of three bf16 values, exactly (8 + 8 + 8 bits of its 24; below 2^-110 the last ones fall under the
 // smallest bf16): against bf16 weights the products of the parts add up to the product of the whole.  Cut, not rounded:
 // every part has the sign of the whole and the largest f32 stays finite.  Infinities and NaN are the first part alone.
@@ -2925,6 +2960,17 @@ static bool gemm_fast_path(const GemmDesc &g, int av, int bv) {
          (g.sbk == 1 || g.sbn == 1) && g.K % 8 == 0 && (g.sbk == 1 || g.N % 8 == 0) && av && bv;
 }
 
+// gemm_bf16_column_kernel's products (not split)
+static bool gemm_column_ok(const GemmDesc &g, int av, int bv) {
+  return g.N == 1 && g.sbk == 1 && gemm_fast_path(g, av, bv) && !g.c_add && !g.c16 && !g.glu_gate && !g.n_group && !g.dual_b &&
+         g.nb0 * g.nb1 <= 65535;
+}
+// Less than 64 columns, more than half of them, on the direct-to-LDS tile of 64 x 64 (the router of a MoE prefill, 1024 x 60 x 2048 in
+// four slices: through registers 9.4 us, 7.6 so; 400 rows 7.8, 6.5).
+static bool gemm_narrow_dma_ok(const GemmDesc &g) {
+  return g.N > 32 && g.N < 64 && g.sak == 1 && g.sbk == 1 && g.K % 64 == 0 && g.K >= 64 && gemm_rows(g.M, g.K) && !g.c_add && !g.n_group && !g.act_sigmoid;
+}
+
 bool gemm_epilogue_ok(const GemmDesc &g) {
   const int asz = g.a_stype == ST_BF16 ? 2 : 4, bsz = g.b_stype == ST_BF16 ? 2 : 4;
   const int av = vec_ok(g.a, asz, g.sak == 1 ? g.sam : g.sak, g.sa_b0, g.sa_b1);
@@ -3046,7 +3092,7 @@ uint32_t gemm_split_k(const LaunchCtx &lc, const GemmDesc &g) {
   const uint32_t batch = g.nb0 * g.nb1;
   const int asz = g.a_stype == ST_BF16 ? 2 : 4, bsz = g.b_stype == ST_BF16 ? 2 : 4;
   const int av = vec_ok(g.a, asz, g.sak == 1 ? g.sam : g.sak, g.sa_b0, g.sa_b1);
-  const int bv = vec_ok(g.b, bsz, g.sbk == 1 ? g.sbn : g.sbk, g.sb_b0, g.sb_b1);
+  const int bv = vec_ok(g.b, bsz, g.sbk == 1 ? (g.N == 1 ? 0 : g.sbn) : g.sbk, g.sb_b0, g.sb_b1);
   const uint64_t tiles = (uint64_t)((g.M + 127) / 128) * ((g.N + 127) / 128) * batch;
   uint32_t splits = 1;
   if (gemv_rows_plain_ok(lc, g)) return 1;
@@ -3065,6 +3111,7 @@ uint32_t gemm_split_k(const LaunchCtx &lc, const GemmDesc &g) {
       splits *= 2;
     return splits;
   }
+  if (gemm_column_ok(g, av, bv)) return 1;
   if (gemm_dma_ok(g) && g.M <= 64) {
     // Tiles of 64 x 64: a workgroup to every CU, four k-steps at least to each - and none below 16 k-steps, where the pass
     // that sums the slices costs what they save (17 x 512 x 64 9.6 us in two slices, 5.5 in one; 17 x 768 x 256 9.8, 8.0; 40 x
@@ -3329,6 +3376,11 @@ hipError_t launch_matmul(const LaunchCtx &lc_in, const GemmDesc &g, const char *
       const uint64_t t128 = (uint64_t)((g.M + 127) / 128) * ((g.N + 127) / 128) * batch * splits;
       hipError_t e = t256 >= (uint64_t)lc.n_cus ? launch_gemm_dma<256, 256, 2, 4, false, 2, false, true>(lc, gg, (uint32_t)t256)
                                                 : launch_gemm_dma<128, 128, 2, 2, false, 2, false, true>(lc, gg, (uint32_t)t128);
+      if (e != hipSuccess) return e;
+    } else if (splits == 1 && gemm_column_ok(g, av, bv)) {
+      CG_LAUNCH(lc, gemm_bf16_column_kernel, dim3((g.M + 3) / 4, batch), 256, gg);
+    } else if (gemm_narrow_dma_ok(g)) {
+      const hipError_t e = launch_gemm_dma<64, 64, 2, 2, false, 8, false, false, false, 2>(lc, gg, (uint32_t)((uint64_t)((g.M + 63) / 64) * batch * splits));
       if (e != hipSuccess) return e;
     } else {
     if (g.n_group) return hipErrorInvalidValue;

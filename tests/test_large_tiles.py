@@ -42,6 +42,14 @@ def test_product(hip_bf16, M, N, K):
     assert np.all(np.abs(got[0] - ref) <= bound)
 
 
+# one column (a wave to a row, its last pieces of k partly past the end), and columns that are most of a 64 x 64 tile, in one slice
+# of k and in several
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(1030, 1, 2048), (17, 1, 200), (300, 1, 2056), (65, 1, 8), (1030, 60, 2048), (65, 33, 64), (129, 63, 1088), (9, 60, 1024)])
+def test_narrow_product(hip_bf16, M, N, K):
+    test_product(hip_bf16, M, N, K)
+
+
 # a residual added as the product is stored: each tile that does so, whole rounds of large tiles with the rest on smaller ones,
 # a batch, and the forms that leave the add to someone else (64 rows, k-slices)
 @pytest.mark.gpu
