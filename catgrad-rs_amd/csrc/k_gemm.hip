@@ -2965,10 +2965,12 @@ static bool gemm_column_ok(const GemmDesc &g, int av, int bv) {
   return g.N == 1 && g.sbk == 1 && gemm_fast_path(g, av, bv) && !g.c_add && !g.c16 && !g.glu_gate && !g.n_group && !g.dual_b &&
          g.nb0 * g.nb1 <= 65535;
 }
-// Less than 64 columns, more than half of them, on the direct-to-LDS tile of 64 x 64 (the router of a MoE prefill, 1024 x 60 x 2048 in
-// four slices: through registers 9.4 us, 7.6 so; 400 rows 7.8, 6.5).
+// Less than 64 columns, more than half of them, not too deep: direct-to-LDS tiles of 32 x 32 with a quarter of each k-step to a
+// wavefront, and no slices - a launch that sums them takes 4.7 us whatever its size (the router of a MoE prefill, K = 2048, 60
+// columns: 1024 rows 9.2 us, 64 x 64 tiles in four slices 7.6 and their sum; 400 rows 8.2, 6.5; 30 rows 8.1, 5.3; through registers
+// 9.4, 7.8, 7.4 and the sum).
 static bool gemm_narrow_dma_ok(const GemmDesc &g) {
-  return g.N > 32 && g.N < 64 && g.sak == 1 && g.sbk == 1 && g.K % 64 == 0 && g.K >= 64 && gemm_rows(g.M, g.K) && !g.c_add && !g.n_group && !g.act_sigmoid;
+  return g.N > 32 && g.N < 64 && g.sak == 1 && g.sbk == 1 && g.K % 64 == 0 && g.K >= 64 && g.K <= 4096 && gemm_rows(g.M, g.K) && !g.c_add && !g.n_group && !g.act_sigmoid;
 }
 
 bool gemm_epilogue_ok(const GemmDesc &g) {
@@ -3111,7 +3113,7 @@ uint32_t gemm_split_k(const LaunchCtx &lc, const GemmDesc &g) {
       splits *= 2;
     return splits;
   }
-  if (gemm_column_ok(g, av, bv)) return 1;
+  if (gemm_column_ok(g, av, bv) || (gemm_fast_path(g, av, bv) && gemm_narrow_dma_ok(g))) return 1;
   if (gemm_dma_ok(g) && g.M <= 64) {
     // Tiles of 64 x 64: a workgroup to every CU, four k-steps at least to each - and none below 16 k-steps, where the pass
     // that sums the slices costs what they save (17 x 512 x 64 9.6 us in two slices, 5.5 in one; 17 x 768 x 256 9.8, 8.0; 40 x
@@ -3380,7 +3382,7 @@ hipError_t launch_matmul(const LaunchCtx &lc_in, const GemmDesc &g, const char *
     } else if (splits == 1 && gemm_column_ok(g, av, bv)) {
       CG_LAUNCH(lc, gemm_bf16_column_kernel, dim3((g.M + 3) / 4, batch), 256, gg);
     } else if (gemm_narrow_dma_ok(g)) {
-      const hipError_t e = launch_gemm_dma<64, 64, 2, 2, false, 8, false, false, false, 2>(lc, gg, (uint32_t)((uint64_t)((g.M + 63) / 64) * batch * splits));
+      const hipError_t e = launch_gemm_dma<32, 32, 1, 1, false, 8, false, false, false, 4>(lc, gg, (uint32_t)((uint64_t)((g.M + 31) / 32) * ((g.N + 31) / 32) * batch * splits));
       if (e != hipSuccess) return e;
     } else {
     if (g.n_group) return hipErrorInvalidValue;
