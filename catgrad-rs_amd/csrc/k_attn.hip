@@ -164,8 +164,39 @@ __device__ __forceinline__ float attn_softmax_step(const AttnPrefillDesc &a, a_f
         }
         pf[kt * 2 + blk] = pack8(p);
       }
-  } else {
-    const bool tail = t0 + KT * 32 > a.t;  // the only step with keys past the end (uniform)
+  } else if (const bool tail = t0 + KT * 32 > a.t; use_mask && !tail) {  // (uniform)
+    // Mask values and no key past the end: the general form below without its selects, half of the vector instructions (us a layer,
+    // causal, with and before: 32 heads of 64, 2900 tokens 87.3, 89.5; 16 heads of 128, 4 x 256 tokens 17.8, 18.5).
+#pragma unroll
+    for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const float4 m = LATE ? *(const float4 *)(M + min(t0 + kt * 32 + j * 8 + half * 4, a.m_len - 4)) : early[kt][j];
+        const float mv[4] = {m.x, m.y, m.z, m.w};
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const float v = st[kt][j * 4 + i] * inv_scale + mv[i];
+          st[kt][j * 4 + i] = v;
+          tmax = fmaxf(tmax, v);
+        }
+      }
+    tmax = max_of_halves(tmax);
+    const float m_new = tmax > m_run + ATTN_MAX_SLACK ? tmax : m_run;
+    alpha = __expf(m_run - m_new);
+    m_run = m_new;
+#pragma unroll
+    for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+      for (int blk = 0; blk < 2; ++blk) {
+        float p[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          p[i] = __expf(st[kt][blk * 8 + i] - m_new);
+          psum += p[i];
+        }
+        pf[kt * 2 + blk] = pack8(p);
+      }
+  } else {  // the only step with keys past the end, or a constant in the mask's place
 #pragma unroll
     for (int kt = 0; kt < KT; ++kt) {
       float4 mask[4];
