@@ -3297,7 +3297,8 @@ hipError_t launch_matmul(const LaunchCtx &lc_in, const GemmDesc &g, const char *
         // their own with the tiling that suits them (347 -> 307 us; with K = 1024 the second launch costs what
         // the idle CUs did)
         const uint64_t tiles_n = (g.N + 255) / 256, tiles_m = (g.M + 255) / 256;
-        const uint64_t lead_m = t256 / (uint64_t)lc.n_cus * (uint64_t)lc.n_cus / tiles_n;  // tile rows of the whole rounds
+        uint64_t lead_m = t256 / (uint64_t)lc.n_cus * (uint64_t)lc.n_cus / tiles_n;  // tile rows of the whole rounds
+        if (g.c_add && lead_m && g.M - std::min<uint64_t>(g.M, lead_m * 256) <= 64) --lead_m;  // (up to 64 rows would not add c_add)
         if (!g.n_group && batch == 1 && splits == 1 && g.K >= 2048 && fill(t256, (uint64_t)lc.n_cus) < 0.8 && lead_m >= 1 &&
             lead_m < tiles_m && g.a_stype == ST_BF16) {
           GemmDesc lead = gg, rest = g;

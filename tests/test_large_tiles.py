@@ -50,11 +50,11 @@ def test_narrow_product(hip_bf16, M, N, K):
     test_product(hip_bf16, M, N, K)
 
 
-# a residual added as the product is stored: each tile that does so, whole rounds of large tiles with the rest on smaller ones,
-# a batch, and the forms that leave the add to someone else (64 rows, k-slices)
+# a residual added as the product is stored: each tile that does so, whole rounds of large tiles with the rest on smaller ones
+# (also where the rounds alone would leave 40 rows), a batch, and the forms that leave the add to someone else (64 rows, k-slices)
 @pytest.mark.gpu
 @pytest.mark.parametrize("B,M,N,K", [(1, 4097, 4101, 192), (1, 8300, 2050, 2048), (1, 1500, 2050, 2112), (1, 2303, 2049, 320), (1, 3100, 2050, 1024),
-                                     (1, 3300, 2050, 2048), (1, 300, 130, 64), (1, 1000, 1000, 256), (3, 700, 520, 192), (1, 64, 200, 128),
+                                     (1, 8232, 2048, 2048), (1, 296, 33000, 2048), (1, 3300, 2050, 2048), (1, 300, 130, 64), (1, 1000, 1000, 256), (3, 700, 520, 192), (1, 64, 200, 128),
                                      (1, 200, 300, 2048)])
 def test_product_and_residual(hip_bf16, B, M, N, K):
     g = np.random.default_rng(M)
