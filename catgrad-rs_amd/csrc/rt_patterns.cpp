@@ -1136,18 +1136,24 @@ struct SumTerm {
 
 // rows of `d` values: reshapes between such shapes keep the row order
 bool rows_shape(const cg_tensor *t, int64_t d) { return t->rank >= 1 && t->shape[t->rank - 1] == d; }
-// ... with at most one leading axis longer than 1: so do transposes
+// ... with at most one leading axis longer than 1: so do transposes of leading axes
 bool one_rows_axis(const cg_tensor *t) {
   int big = 0;
   for (int i = 0; i + 1 < t->rank; ++i) big += t->shape[i] != 1;
   return big <= 1;
 }
 
+// a transpose of leading axes of which at most one is longer than 1 (the last axis may be swapped for another of the same
+// extent: as many rows as columns, and every shape as before)
+bool moves_unit_axes(const cg_tensor *t) {
+  return t->p0 != t->rank - 1 && t->p1 != t->rank - 1 && one_rows_axis(t);
+}
+
 // through deferred reshapes of rows, and transposes that only move axes of extent 1, that nobody else reads
 cg_tensor *under_unit_views(cg_tensor *n, const cg_tensor *root, int64_t d) {
   while ((n->op == N_RESHAPE || n->op == N_TRANSPOSE) && (n == root || refs(n) == 1) && n->in[0] &&
          n->in[0]->size() == n->size() && rows_shape(n, d) && rows_shape(n->in[0], d) &&
-         (n->op == N_RESHAPE || (one_rows_axis(n) && one_rows_axis(n->in[0]))))
+         (n->op == N_RESHAPE || moves_unit_axes(n)))
     n = n->in[0];
   return n;
 }

@@ -958,6 +958,27 @@ def test_sum_of_scaled_rows_of_several_sequences(oracle, hip, hip_nopat, B, S, d
     assert np.array_equal(got, gen), np.abs(got - gen).max()
 
 
+@pytest.mark.parametrize("shape,a0,a1", [((64, 64), 0, 1), ((1, 64, 64), 1, 2), ((1, 64, 64), 2, 1), ((64, 1, 64), 0, 2)])
+@pytest.mark.parametrize("what", ["term", "scale", "sum"])
+def test_sum_of_scaled_rows_beside_a_transpose_of_as_many_columns(oracle, hip, hip_nopat, shape, a0, a1, what):
+    """As many rows as columns: a transpose that swaps the two leaves every shape as it was, and is no view of the same rows."""
+    g = np.random.default_rng(a0 + a1)
+    h, p, q, res = (g.standard_normal(shape).astype(np.float32) for _ in range(4))
+    v = g.standard_normal(shape[:-1] + (1,)).astype(np.float32)
+
+    def f(b, h, v, p, q, res):
+        scale = lang.broadcast(b, v, lang.shape(b, h))
+        if what == "scale":         # a value for every column
+            return h * lang.transpose(b, a0, a1, scale) + (p + q) + res
+        if what == "sum":
+            return lang.transpose(b, a0, a1, h * scale + p + q) + res
+        return h * scale + lang.transpose(b, a0, a1, p + q) + res
+    args = (h, v, p, q, res)
+    (ref,), (got,), (gen,) = (vectors.run(b, f, 1, *args) for b in (oracle, hip, hip_nopat))
+    assert got.shape == ref.shape and np.array_equal(got, gen), np.abs(got - gen).max()
+    assert np.allclose(got, ref, rtol=1e-6, atol=1e-6)
+
+
 @pytest.mark.parametrize("variant", ["right_nested", "shared_term", "two_chains", "scale_on_the_left", "nine_terms"])
 def test_sum_of_scaled_rows_in_other_arrangements(hip, hip_nopat, variant):
     """Additions nested to the right, a term somebody else reads too, two chains under one addition, the scale as
