@@ -41,9 +41,10 @@ struct Storage {
   // shared by every matmul that reads a view of it (q/k/v, gate/up read the same activations)
   Storage *shadow = nullptr;
   // an attention mask's table of tile classes (launch_mask_tiles), made on demand and shared by every
-  // layer that reads the mask; tiles_key = {element offset of the mask, rows, keys, query rows per tile, keys per tile}
+  // layer that reads the mask; tiles_key = {element offset of the mask, rows, keys, row stride, query rows per tile,
+  // keys per tile}
   Storage *tiles = nullptr;
-  int64_t tiles_key[5] = {-1, 0, 0, 0, 0};
+  int64_t tiles_key[6] = {-1, 0, 0, 0, 0, 0};
   // the same mask with rows padded for 16-byte loads (launch_mask_pad), kept like the table above;
   // padded_key = {element offset of the mask, rows, keys, row stride}
   Storage *padded = nullptr;

@@ -108,6 +108,7 @@ int try_attn_prefill(cg_backend *be, cg_tensor *n, bool *done) {
   const bool shared_mask = mask && a.m_sb == 0 && a.m_sh == 0 && a.m_ss > 0 && a.m_st == 1 && mask->st->grow_dim < 0 && Sq <= 65535;
   const bool pad_mask = mask && (!a.m_vec || T % 4);
   a.m_len = (uint32_t)T;
+  const int64_t mask_rows = a.m_ss;  // (two views of one storage may differ in nothing else)
   if ((pad_mask && !shared_mask) || !twin_ok) {
     storage_release(n->st);
     n->st = nullptr;
@@ -115,7 +116,7 @@ int try_attn_prefill(cg_backend *be, cg_tensor *n, bool *done) {
   }
   if (pad_mask) {
     Storage *ms = mask->st;
-    const int64_t key[4] = {mask->offset, Sq, T, a.m_ss}, pitch = (T + 63) / 64 * 64;
+    const int64_t key[4] = {mask->offset, Sq, T, mask_rows}, pitch = (T + 63) / 64 * 64;
     if (!ms->padded || !std::equal(key, key + 4, ms->padded_key)) {
       storage_release(ms->padded);
       ms->padded = nullptr;
@@ -177,9 +178,9 @@ int try_attn_prefill(cg_backend *be, cg_tensor *n, bool *done) {
     uint32_t q_rows = 0, keys = 0;
     attn_prefill_tiling(be->lc(), a, &q_rows, &keys);
     Storage *ms = mask->st;
-    const int64_t key[5] = {mask->offset, Sq, T, q_rows, keys};
+    const int64_t key[6] = {mask->offset, Sq, T, mask_rows, q_rows, keys};
     const size_t rows = (size_t)(Sq + q_rows - 1) / q_rows, cols = (size_t)(T + keys - 1) / keys;
-    if (!ms->tiles || !std::equal(key, key + 5, ms->tiles_key)) {
+    if (!ms->tiles || !std::equal(key, key + 6, ms->tiles_key)) {
       storage_release(ms->tiles);
       ms->tiles = nullptr;
       int st = dev_alloc(be, rows * cols, &ms->tiles);
@@ -187,7 +188,7 @@ int try_attn_prefill(cg_backend *be, cg_tensor *n, bool *done) {
         storage_release(vt);
         return st;
       }
-      std::copy(key, key + 5, ms->tiles_key);
+      std::copy(key, key + 6, ms->tiles_key);
       KernelScope ks(be, "attn_mask_tiles", (double)Sq * T * 4, 0);
       hipError_t me = launch_mask_tiles(be->lc(), a.mask, a.m_ss, (uint32_t)Sq, (uint32_t)T, q_rows, keys, (uint8_t *)ms->tiles->ptr);
       if (me != hipSuccess) {

@@ -215,3 +215,34 @@ def test_parts_of_a_query_tile(hip_bf16, H, KV, S, T, d):
     (got,) = vectors.run(hip_bf16, f, 1, q, k, v, hidden)
     assert hip_bf16.launch_counts(reset=True).get("attn_prefill") == 1
     parity.assert_bf16(ref, got, f"{S} queries of {T} keys")
+
+
+# Two views of one mask, alike but for their row stride: the first T columns of [S, 2 T] and the first S rows of the same values
+# as [2 S, T].  What one of them hides from every query the other shows to half of them.
+@pytest.mark.gpu
+@pytest.mark.parametrize("S,T", [(64, 128), (200, 192), (64, 132)])
+@pytest.mark.parametrize("order", [0, 1])
+def test_views_of_one_mask(oracle, hip, hip_bf16, S, T, order):
+    g = np.random.default_rng(S + T)
+    qkv = [vectors.bf16_round(g.standard_normal((1, h, n, 64)).astype(np.float32)) for h, n in ((4, S), (2, T), (2, T)) * 2]
+    mask = np.zeros((S, 2 * T), np.float32)
+    mask[:, 64:T] = helpers.F32_MIN
+
+    def f(b, *a):     # (the mask is uploaded as a vector: f32)
+        views = [lang.slice(b, 1, 0, T, lang.reshape(b, lang.make_shape(b, S, 2 * T), a[6])),
+                 lang.slice(b, 0, 0, S, lang.reshape(b, lang.make_shape(b, 2 * S, T), a[6]))]
+        out = [None, None]
+        for i in (order, 1 - order):
+            q, k, v = (x + x - x for x in a[3 * i:3 * i + 3])
+            attn = lang.matmul(b, q, lang.transpose(b, 2, 3, helpers.repeat_kv(b, 2, k)))
+            sh = lang.shape(b, attn)
+            attn = attn / lang.constant(b, 8.0, sh) + lang.broadcast(b, views[i], sh)
+            out[i] = lang.matmul(b, nn.softmax(b, attn), helpers.repeat_kv(b, 2, v))
+        return out if order == 0 else out[::-1]
+    ref = vectors.run(oracle, f, 2, *qkv, mask.reshape(-1))
+    for be, check in ((hip, parity.assert_f32), (hip_bf16, parity.assert_bf16)):
+        be.launch_counts(reset=True)
+        both = vectors.run(be, f, 2, *qkv, mask.reshape(-1))
+        assert be.launch_counts(reset=True).get("attn_prefill", 0) == (0 if be is hip and T > 128 else 2)
+        for r, got in zip(ref, both):
+            check(r, got, "one view of the mask")
