@@ -33,6 +33,16 @@ namespace cgk {
 
 typedef __attribute__((ext_vector_type(16))) float f32x16;
 
+// These kernels' places in LDS are constants that start at 0, where a static __shared__ variable would lie too: no kernel that has
+// one is launched.
+static hipError_t whole_lds(const void *kernel, int bytes) {
+  hipFuncAttributes a;
+  const hipError_t e = hipFuncGetAttributes(&a, kernel);
+  if (e != hipSuccess) return e;
+  if (a.sharedSizeBytes) return hipErrorInvalidConfiguration;
+  return hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+}
+
 // ---- the main loop, in pieces -------------------------------------------------------------------------
 // Fragments live in v[128:255]: (half U, 32-row block r, k-slice ks) as below.  s[40:41] points at A, s[42:43] and s[44:45]
 // at the two halves of B, at the step being requested; s46 is this wavefront's place in the stage being requested, s47
@@ -308,7 +318,7 @@ __global__ void __launch_bounds__(256, 1) gemm_bf16_ring_kernel(GemmDesc g) {
     return (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)v) | (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(v >> 32)) << 32;
   };
   const uint64_t sa0 = scalar(pa), sb0 = scalar(pb0), sb1 = scalar(pb1);
-  const uint32_t lds = wave * 4096;  // (all LDS of this kernel is the two stages, at offset 0)
+  const uint32_t lds = wave * 4096;  // (all LDS of this kernel is the stages, at offset 0: whole_lds)
 #define RING_IN_B                                                                                                         \
   [dB00] "v"(dB0[0]), [dB01] "v"(dB0[1]), [dB02] "v"(dB0[2]), [dB03] "v"(dB0[3]), [dB10] "v"(dB1[0]), [dB11] "v"(dB1[1]), \
       [dB12] "v"(dB1[2]), [dB13] "v"(dB1[3]), [pb0] "s"(sb0), [pb1] "s"(sb1), [lds] "s"(lds)
@@ -491,7 +501,7 @@ __global__ void __launch_bounds__(256, 1) moe_ring_kernel(MoeGemmDesc g) {
     return (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)v) | (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(v >> 32)) << 32;
   };
   const uint64_t s_b0 = scalar(pb0), s_b1 = scalar(pb1);
-  const uint32_t lds = wave * 4096;
+  const uint32_t lds = wave * 4096;  // (as above)
 #define MOE_IN                                                                                                            \
   [dB00] "v"(dB0[0]), [dB01] "v"(dB0[1]), [dB02] "v"(dB0[2]), [dB03] "v"(dB0[3]), [dB10] "v"(dB1[0]), [dB11] "v"(dB1[1]), \
       [dB12] "v"(dB1[2]), [dB13] "v"(dB1[3]), [pb0] "s"(s_b0), [pb1] "s"(s_b1), [lds] "s"(lds)
@@ -572,7 +582,7 @@ static hipError_t launch_moe_ring_as(const LaunchCtx &lc, const MoeGemmDesc &g, 
   constexpr int smem = 10 * 16384;
   static bool configured = false;  // one attribute call per kernel and process
   if (!configured) {
-    hipError_t e = hipFuncSetAttribute((const void *)moe_ring_kernel<KIND>, hipFuncAttributeMaxDynamicSharedMemorySize, smem);
+    const hipError_t e = whole_lds((const void *)moe_ring_kernel<KIND>, smem);
     if (e != hipSuccess) return e;
     configured = true;
   }
@@ -604,7 +614,7 @@ static hipError_t launch_ring_as(const LaunchCtx &lc, const GemmDesc &g, uint32_
   constexpr int smem = AH == 2 ? 2 * 65536 : 10 * 16384;
   static bool configured = false;  // one attribute call per kernel and process
   if (!configured) {
-    hipError_t e = hipFuncSetAttribute((const void *)gemm_bf16_ring_kernel<KIND, AH>, hipFuncAttributeMaxDynamicSharedMemorySize, smem);
+    const hipError_t e = whole_lds((const void *)gemm_bf16_ring_kernel<KIND, AH>, smem);
     if (e != hipSuccess) return e;
     configured = true;
   }

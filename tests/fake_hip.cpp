@@ -1,6 +1,7 @@
 // A HIP runtime without a GPU, for tests of what the host does: memory is host memory, a stream is always idle, the two
 // copy kernels are made on the spot and every other launch is none.  fake_hip_refuse(name, n): the n-th launch from now
-// of a kernel whose name holds `name` is refused, as the runtime refuses one that it cannot make.
+// of a kernel whose name holds `name` is refused, as the runtime refuses one that it cannot make.  fake_hip_launched(): the
+// names of the kernels launched since the last call; fake_hip_static_lds(n): what every kernel's own __shared__ variables take.
 // Loaded with RTLD_GLOBAL before the library, whose references to the runtime it then answers.
 #include <hip/hip_runtime.h>
 #include <atomic>
@@ -16,8 +17,8 @@ std::map<const void *, std::string> &names() {
   return m;
 }
 std::mutex lock;
-std::string refuse;
-std::atomic<int> countdown{0}, waits{0};
+std::string refuse, launched;
+std::atomic<int> countdown{0}, waits{0}, static_lds{0};
 thread_local hipError_t last = hipSuccess;
 
 // the argument lists of to_host_kernel and from_host_kernel (k_misc.hip)
@@ -40,6 +41,7 @@ hipError_t launch(const void *f, void **args) {
   const std::string &name = names()[f];
   {
     std::lock_guard<std::mutex> lk(lock);
+    launched += name + "\n";
     if (!refuse.empty() && name.find(refuse) != std::string::npos && countdown.fetch_sub(1) == 1) {
       refuse.clear();
       return last = hipErrorInvalidConfiguration;
@@ -59,6 +61,14 @@ void fake_hip_refuse(const char *name, int n) {
   countdown = n;
 }
 int fake_hip_waits() { return waits; }  // on the stream
+const char *fake_hip_launched() {
+  static std::string since;
+  std::lock_guard<std::mutex> lk(lock);
+  since.clear();
+  since.swap(launched);
+  return since.c_str();
+}
+void fake_hip_static_lds(int n) { static_lds = n; }
 
 void **__hipRegisterFatBinary(const void *) { static void *h[4]; return h; }
 void __hipUnregisterFatBinary(void **) {}
@@ -89,6 +99,11 @@ hipError_t hipEventCreate(hipEvent_t *e) { return *e = nullptr, hipSuccess; }
 hipError_t hipEventDestroy(hipEvent_t) { return hipSuccess; }
 hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
 hipError_t hipEventElapsedTime(float *ms, hipEvent_t, hipEvent_t) { return *ms = 0.f, hipSuccess; }
+hipError_t hipFuncGetAttributes(hipFuncAttributes *a, const void *) {
+  std::memset(a, 0, sizeof(*a));
+  a->sharedSizeBytes = static_lds;
+  return hipSuccess;
+}
 hipError_t hipFuncSetAttribute(const void *, hipFuncAttribute, int) { return hipSuccess; }
 hipError_t hipLaunchKernel(const void *f, dim3, dim3, void **args, size_t, hipStream_t) { return launch(f, args); }
 hipError_t hipExtLaunchKernel(const void *f, dim3, dim3, void **args, size_t, hipStream_t, hipEvent_t, hipEvent_t, int) { return launch(f, args); }

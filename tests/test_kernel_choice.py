@@ -1,0 +1,42 @@
+"""Which kernel a call is given, on the CPU: the library over the stand-in runtime of fake_hip.cpp, which says what was launched."""
+import pytest
+
+from test_host_copies import fake_hip  # noqa: F401 - a fixture
+
+BF16 = 1
+
+LAUNCHED = """
+import importlib
+fake.fake_hip_launched.restype = ctypes.c_char_p
+
+def launched(f):
+    be.sync()
+    fake.fake_hip_launched()
+    be.realize(f())
+    be.sync()
+    return [n for n in fake.fake_hip_launched().decode().split("\\n") if "gem" in n]
+
+def operand(*shape):
+    n = int(np.prod(shape))
+    if int(sys.argv[2]):
+        return be.from_bf16_bits(np.zeros(n, np.uint16), shape)
+    return be.tensor(np.zeros(n, np.float32).reshape(shape))
+
+def product(m, n, k, along_k=True, batch=1, residual=False):
+    lead, r = ((), 2) if batch == 1 else ((batch,), 3)
+    x, w = operand(*lead, m, k), operand(*lead, *((n, k) if along_k else (k, n)))
+    res = be.reshape(be.tensor(np.zeros(batch * m * n, np.float32)), lead + (m, n)) if residual else None
+    def f():
+        y = be.matmul(x, be.transpose(w, r - 2, r - 1) if along_k else w)
+        return be.add(res, y) if residual else y
+    return launched(f)
+"""
+
+
+def test_no_kernel_with_fixed_places_in_lds_beside_variables_of_its_own(fake_hip):  # noqa: F811
+    fake_hip(LAUNCHED + """
+fake.fake_hip_static_lds(64)
+assert fails(lambda: product(4096, 4096, 128))
+fake.fake_hip_static_lds(0)
+assert ["gemm_bf16_ring" in n for n in product(4096, 4096, 128)] == [True]
+""", BF16)
