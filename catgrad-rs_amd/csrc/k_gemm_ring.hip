@@ -379,20 +379,29 @@ __global__ void __launch_bounds__(256, 1) gemm_bf16_ring_kernel(GemmDesc g) {
   // different rows, and stored as they are every instruction would touch 32 lines; out of LDS a store is four rows of 64
   // columns, whole lines.  (Chunks of 16 bytes swizzled by the row: no bank conflicts either way.)  A tile without edges has
   // no branch in all of this: with one per store the accumulators' 256 registers leave one at a time, 8 us a tile.
+  // At an edge the sixteen pieces, and what is added to them, are on their way before the first is stored, as in the middle (one
+  // after the other, and value by value, 13 us more a tile: 16 x 1000 x 1000 x 128 32 -> 19 us, 16 x 257 x 2000 x 128 30 -> 16,
+  // 1500 x 20000 x 1024 90 -> 76, 6000 x 4100 x 256 and a residual 88 -> 55; biases, which took that path in every tile,
+  // 6000 x 3072 x 2048 178 -> 95).
   __syncthreads();  // every wavefront has read its last fragments
   extern __shared__ __attribute__((aligned(16))) float ring_smem[];
   uint16_t *C16 = g.c16 ? g.c16 + (uint64_t)bz * g.M * g.N : nullptr;
-  const bool whole = m0 + BM <= g.M && n0 + BNO <= Nl && !Bias;
+  const bool whole = m0 + BM <= g.M && n0 + BNO <= Nl;
   constexpr bool F32 = KIND == RING_PLAIN;
   const uint32_t pitch = KIND == RING_SIGMOID ? g.c16_pitch : Nl;
-  uint32_t to[4];  // where this lane's piece of rows 0-3, 4-7, 8-11, 12-15 of a quadrant goes, in bytes from its corner
+  uint32_t at_row[4], at_col[4], to[4];  // this lane's piece of rows 0-3, 4-7, 8-11, 12-15 of a quadrant; its bytes from the corner
 #pragma unroll
-  for (int u = 0; u < 4; ++u) to[u] = ((u * 4 + (lane >> 4)) * pitch + (((lane & 15) ^ (u * 4 + (lane >> 4))) << 2)) * (F32 ? 4u : 2u);
+  for (int u = 0; u < 4; ++u) {
+    at_row[u] = u * 4 + (lane >> 4);
+    at_col[u] = ((lane & 15) ^ at_row[u]) << 2;
+    to[u] = (at_row[u] * pitch + at_col[u]) * (F32 ? 4u : 2u);
+  }
 #pragma unroll
   for (int qd = 0; qd < (GATED ? AH : 4); ++qd) {
     const int a = GATED ? qd : qd >> 1, b = GATED ? 0 : qd & 1;
     float *tile = ring_smem + wave * 8192 + (qd & 1) * 4096;
     const uint32_t col0 = n0 + b * 128 + wn * 64, row0 = m0 + a * 128 + wm * 64;
+    if (row0 >= g.M || col0 >= pitch) continue;  // (uniform: nothing of this quadrant is stored)
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
@@ -409,17 +418,25 @@ __global__ void __launch_bounds__(256, 1) gemm_bf16_ring_kernel(GemmDesc g) {
           *(float4 *)(tile + r * 64 + ((chunk ^ (r & 15)) << 2)) = v;
         }
     const float *from = tile + ((lane >> 4) << 6) + ((lane & 15) << 2);
-    if (whole) {
-      float4 out[16];
+    float4 out[16];
 #pragma unroll
-      for (int it = 0; it < 16; ++it) out[it] = *(const float4 *)(from + it * 256);
+    for (int it = 0; it < 16; ++it) out[it] = *(const float4 *)(from + it * 256);
+    auto plus = [](float4 x, float4 y) { return make_float4(x.x + y.x, x.y + y.y, x.z + y.z, x.w + y.w); };
+    if (F32 && Bias) {  // (grouped products: columns in fours, clamped to the last)
+      float4 bias[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) __builtin_memcpy(&bias[u], Bias + min(col0 + at_col[u], Nl - 4), 16);
+#pragma unroll
+      for (int it = 0; it < 16; ++it) out[it] = plus(out[it], bias[it & 3]);
+    }
+    if (whole) {
       if (F32 && Cadd) {
         const char *corner = (const char *)(Cadd + (uint64_t)row0 * Nl + col0);
         float4 add[16];
 #pragma unroll
         for (int it = 0; it < 16; ++it) __builtin_memcpy(&add[it], corner + (uint64_t)(it >> 2) * 16 * pitch * 4 + to[it & 3], 16);
 #pragma unroll
-        for (int it = 0; it < 16; ++it) { out[it].x += add[it].x; out[it].y += add[it].y; out[it].z += add[it].z; out[it].w += add[it].w; }
+        for (int it = 0; it < 16; ++it) out[it] = plus(out[it], add[it]);
       }
       char *corner = F32 ? (char *)(C + (uint64_t)row0 * Nl + col0) : (char *)(C16 + (uint64_t)row0 * pitch + col0);
 #pragma unroll
@@ -433,20 +450,40 @@ __global__ void __launch_bounds__(256, 1) gemm_bf16_ring_kernel(GemmDesc g) {
       }
       continue;
     }
-#pragma unroll 1
-    for (uint32_t it = 0; it < 16; ++it) {
-      const uint32_t r = it * 4 + (lane >> 4), row = row0 + r, col = col0 + (((lane & 15) ^ (r & 15)) << 2);
-      float4 v = *(const float4 *)(from + it * 256);
-      if (row >= g.M) continue;
-      if (F32) {
-        float *c = C + (uint64_t)row * Nl + col;
-        const float e[4] = {v.x, v.y, v.z, v.w};
+    if (F32) {
+      if (Cadd) {  // (rows and columns clamped into the matrix: what is not stored is not used)
+        float4 add[16];
 #pragma unroll
-        for (int k = 0; k < 4; ++k)
-          if (col + k < Nl) c[k] = Bias ? e[k] + Bias[col + k] : Cadd ? e[k] + Cadd[(uint64_t)row * Nl + col + k] : e[k];
-      } else if (col < pitch) {  // (N % 4 == 0, or padded rows: a piece is inside or outside; zeros past the last column)
+        for (int it = 0; it < 16; ++it)
+          __builtin_memcpy(&add[it], Cadd + (uint64_t)min(row0 + (it >> 2) * 16 + at_row[it & 3], g.M - 1) * Nl + min(col0 + at_col[it & 3], Nl - 4), 16);
+#pragma unroll
+        for (int it = 0; it < 16; ++it) out[it] = plus(out[it], add[it]);
+      }
+#pragma unroll
+      for (int it = 0; it < 16; ++it) {
+        const uint32_t row = row0 + (it >> 2) * 16 + at_row[it & 3], col = col0 + at_col[it & 3];
+        if (row < g.M && col + 4 <= Nl) __builtin_memcpy(C + (uint64_t)row * Nl + col, &out[it], 16);
+      }
+      if (Nl % 4 && col0 + 64 > Nl) {  // the last one to three columns (a product that is not grouped)
+#pragma unroll
+        for (int it = 0; it < 16; ++it) {
+          const uint32_t row = row0 + (it >> 2) * 16 + at_row[it & 3], col = col0 + at_col[it & 3];
+          if (row < g.M && col < Nl && col + 4 > Nl) {
+            float4 v = *(const float4 *)(from + it * 256);
+            const float e[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+            for (int k = 0; k < 3; ++k)
+              if (col + k < Nl) C[(uint64_t)row * Nl + col + k] = Cadd ? e[k] + Cadd[(uint64_t)row * Nl + col + k] : e[k];
+          }
+        }
+      }
+    } else {  // (N % 4 == 0, or padded rows: a piece is inside or outside; zeros past the last column)
+#pragma unroll
+      for (int it = 0; it < 16; ++it) {
+        const uint32_t row = row0 + (it >> 2) * 16 + at_row[it & 3], col = col0 + at_col[it & 3];
+        float4 v = out[it];
         v = make_float4(col < Nl ? v.x : 0.f, col + 1 < Nl ? v.y : 0.f, col + 2 < Nl ? v.z : 0.f, col + 3 < Nl ? v.w : 0.f);
-        *(uint2 *)(C16 + (uint64_t)row * pitch + col) = bf16_pack4(v);
+        if (row < g.M && col < pitch) *(uint2 *)(C16 + (uint64_t)row * pitch + col) = bf16_pack4(v);
       }
     }
   }

@@ -40,3 +40,15 @@ assert fails(lambda: product(4096, 4096, 128))
 fake.fake_hip_static_lds(0)
 assert ["gemm_bf16_ring" in n for n in product(4096, 4096, 128)] == [True]
 """, BF16)
+
+
+def test_products_on_256_x_256_tiles(fake_hip):  # noqa: F811
+    """The sizes that test_large_tiles.py gives its edges, and batches."""
+    fake_hip(LAUNCHED + """
+for m, n, k in ((4096, 4096, 128), (4090, 4093, 192), (3841, 3843, 256), (8001, 2046, 320), (255, 65299, 448)):
+    names = product(m, n, k)
+    assert len(names) == 1 and "gemm_bf16_ring_kernelILi0ELi2E" in names[0], (m, n, k, names)
+for b, m, n, k in ((1, 3841, 3843, 128), (1, 4090, 4093, 192), (1, 8001, 2046, 256), (16, 1000, 1002, 128)):
+    names = product(m, n, k, batch=b, residual=True)
+    assert len(names) == 1 and "gemm_bf16_ring_kernelILi0ELi2E" in names[0], (b, m, n, k, names)
+""", BF16)
