@@ -536,8 +536,11 @@ template <int N> __device__ __forceinline__ void wait_vmcnt() {
 // tokens), which are bound by the stream of weights: narrow tiles put a workgroup on every CU, and more wavefronts than
 // such a tile has MFMA columns for share the issue of its loads (a global_load_lds costs its wave 55 - 120 cycles).
 // RING: four wavefronts, and the main loop of mfma_step_ring.hpp: every slice of k has NS - 1 k-steps at least.
+// ADD: a plain product that adds c_add.  (A kernel of its own: the sixteen values and their addresses that are on their way at once
+// take 22 to 42 registers, and what every product paid for them was 4 to 11 %: 4000 rows of 3072 columns, K = 2048, 73.5 us against
+// 65, 6000 x 700 x 192 10.5 against 9.7.)
 template <int BM_, int BN_, int WR, int WC, bool EPI, int NS, bool DUAL = false, bool BKM = false, bool ROPE = false, int KG = 1,
-          bool RING = false>
+          bool RING = false, bool ADD = false>
 __global__ void __launch_bounds__(WR *WC *KG * 64) gemm_bf16_dma_kernel(GemmDesc g) {
   constexpr int NW = WR * WC * KG, BK = 64;
   static_assert(!ROPE || ((BN_ % 64 == 0 || BN_ == 32) && !EPI && !DUAL && !BKM && (BM_ * BN_ / 4) % (NW * 64) == 0),
@@ -594,7 +597,7 @@ __global__ void __launch_bounds__(WR *WC *KG * 64) gemm_bf16_dma_kernel(GemmDesc
   const uint32_t pair_hd = PAIRS ? g.rope_hd : 64, pair_0 = PAIRS ? n0 / pair_hd * pair_hd + n0 % pair_hd / 2 : 0;
   auto column = [&](uint32_t cl) { return PAIRS ? pair_0 + (cl & 15) + (cl >> 4) * (pair_hd / 2) : n0 + cl; };
   const float *Bias = g.n_group ? g.grp_bias[grp] : nullptr;
-  const float *Cadd = !ROPE && !EPI && g.c_add && g.splits <= 1 ? g.c_add + (uint64_t)bz * g.M * g.N : nullptr;
+  const float *Cadd = ADD ? g.c_add + (uint64_t)bz * g.M * g.N : nullptr;
   const float *Gate = g.glu_gate ? g.glu_gate + (uint64_t)bz * g.M * g.N : nullptr;  // only without split-K
   uint16_t *C16 = g.c16 ? g.c16 + (uint64_t)bz * g.M * g.N : nullptr;
   const uint32_t k_begin = split * g.k_per_split;
@@ -972,7 +975,7 @@ __global__ void __launch_bounds__(WR *WC *KG * 64) gemm_bf16_dma_kernel(GemmDesc
         }
         continue;
       }
-      if (Cadd) {  // (all sixteen on their way before the first is used; positions clamped)
+      if (ADD) {  // (all sixteen on their way before the first is used; positions clamped)
         float add[16];
 #pragma unroll
         for (int e = 0; e < 16; ++e) {
@@ -995,19 +998,26 @@ __global__ void __launch_bounds__(WR *WC *KG * 64) gemm_bf16_dma_kernel(GemmDesc
 }
 
 template <int BM_, int BN_, int WR, int WC, bool EPI = false, int NS = 2, bool DUAL = false, bool BKM = false, bool ROPE = false, int KG = 1,
-          bool RING = false>
+          bool RING = false, bool ADD = false>
 static hipError_t launch_gemm_dma(const LaunchCtx &lc, const GemmDesc &g, uint32_t grid) {
   // (ROPE: the f32 tile is exchanged through LDS at the end, BN_ + 8 floats per row)
   constexpr int stages = NS * (BM_ + BN_) * 64 * 2, smem = ROPE && BM_ * (BN_ + 8) * 4 > stages ? BM_ * (BN_ + 8) * 4 : stages;
   static bool configured = false;  // one attribute call per kernel and process
   if (!configured) {
-    hipError_t e = hipFuncSetAttribute((const void *)gemm_bf16_dma_kernel<BM_, BN_, WR, WC, EPI, NS, DUAL, BKM, ROPE, KG, RING>,
+    hipError_t e = hipFuncSetAttribute((const void *)gemm_bf16_dma_kernel<BM_, BN_, WR, WC, EPI, NS, DUAL, BKM, ROPE, KG, RING, ADD>,
                                        hipFuncAttributeMaxDynamicSharedMemorySize, smem);
     if (e != hipSuccess) return e;
     configured = true;
   }
-  cg_launch(lc, gemm_bf16_dma_kernel<BM_, BN_, WR, WC, EPI, NS, DUAL, BKM, ROPE, KG, RING>, dim3(grid), dim3(WR * WC * KG * 64), smem, g);
+  cg_launch(lc, gemm_bf16_dma_kernel<BM_, BN_, WR, WC, EPI, NS, DUAL, BKM, ROPE, KG, RING, ADD>, dim3(grid), dim3(WR * WC * KG * 64), smem, g);
   return hipGetLastError();
+}
+
+// a plain product, with c_add or without
+template <int BM_, int BN_, int WR, int WC, int NS = 2, int KG = 1, bool RING = false>
+static hipError_t launch_gemm_plain(const LaunchCtx &lc, const GemmDesc &g, uint64_t grid) {
+  return g.c_add && g.splits <= 1 ? launch_gemm_dma<BM_, BN_, WR, WC, false, NS, false, false, false, KG, RING, true>(lc, g, (uint32_t)grid)
+                                  : launch_gemm_dma<BM_, BN_, WR, WC, false, NS, false, false, false, KG, RING>(lc, g, (uint32_t)grid);
 }
 
 // C = sum over splits of workspace[split] (float4 per thread; sizes are multiples of 4 or the
@@ -3315,8 +3325,8 @@ hipError_t launch_matmul(const LaunchCtx &lc_in, const GemmDesc &g, const char *
           return launch_matmul(second, rest, nullptr);
         }
         if (!g.n_group && fill(t128, 2 * (uint64_t)lc.n_cus) > 1.15 * fill(t256, (uint64_t)lc.n_cus))
-          e = g.K < 2048 ? launch_gemm_dma<128, 128, 2, 4, false, 2>(lc, gg, (uint32_t)t128)  // (as below)
-                         : launch_gemm_dma<128, 128, 2, 2>(lc, gg, (uint32_t)t128);
+          e = g.K < 2048 ? launch_gemm_plain<128, 128, 2, 4>(lc, gg, t128)  // (as below)
+                         : launch_gemm_plain<128, 128, 2, 2>(lc, gg, t128);
         else
           e = launch_gemm_ring(lc, gg);
       } else {
@@ -3348,29 +3358,29 @@ hipError_t launch_matmul(const LaunchCtx &lc_in, const GemmDesc &g, const char *
           // too few 128 x 128 tiles for the CUs and no split-K to multiply them: halve the tile, or quarter it if every CU still holds
           // one at most (1536 columns, K = 1152: 100 rows 11.2 -> 9.5 us, 400 11.3 -> 9.6, 640 11.3 -> 10.1)
           const uint64_t t64 = (uint64_t)((g.M + 63) / 64) * ((g.N + 63) / 64) * batch;
-          e = t64 <= cus ? launch_gemm_dma<64, 64, 2, 2, false, 8, false, false, false, 2>(lc, gg, (uint32_t)t64)
-                         : launch_gemm_dma<128, 64, 4, 2, false, 4>(lc, gg, (uint32_t)((uint64_t)((g.M + 127) / 128) * ((g.N + 63) / 64) * batch));
+          e = t64 <= cus ? launch_gemm_plain<64, 64, 2, 2, 8, 2>(lc, gg, t64)
+                         : launch_gemm_plain<128, 64, 4, 2, 4>(lc, gg, (uint64_t)((g.M + 127) / 128) * ((g.N + 63) / 64) * batch);
         } else if (t128 <= cus) {
           // A round of 128 rows.  The four wavefronts' longer start and tail pay from about 24 k-steps on (weights from memory: 900 x
           // 2048 x 8192 in two slices 44.4 -> 37.4 us, 700 40.9 -> 36.3, 300 in four 23.2 -> 21.7, 400 x 1152 x 6912 in four - 27 steps -
           // 18.9 -> 18.2; 18 steps 14.8, 16.0; 16 steps 14.1, 15.7 and 14.8, 16.6).
-          if (steps >= 24) e = launch_gemm_dma<128, 128, 2, 2, false, 5, false, false, false, 1, true>(lc, gg, (uint32_t)t128);
-          else e = launch_gemm_dma<128, 128, 2, 4, false, 4>(lc, gg, (uint32_t)t128);
+          if (steps >= 24) e = launch_gemm_plain<128, 128, 2, 2, 5, 1, true>(lc, gg, t128);
+          else e = launch_gemm_plain<128, 128, 2, 4, 4>(lc, gg, t128);
         } else if (t192 <= cus && steps >= 4) {
           // a round of 192 rows (o_proj and down_proj of 2900 rows: 29 and 91 us; 368 tiles of 128 rows two to a CU 35 and 122; 1024
           // deep 19.7, 21.6)
-          e = launch_gemm_dma<192, 128, 2, 2, false, 4, false, false, false, 1, true>(lc, gg, (uint32_t)t192);
+          e = launch_gemm_plain<192, 128, 2, 2, 4, 1, true>(lc, gg, t192);
         } else if (steps >= 64) {
           // Several rounds of a deep product, a round of 192 rows at 1.42 times one of 128: 8192 x 1152 x 6912 two or three, 134 and 148 us
           // (two to a CU 167); 4000 x 2048 x 8192 two either way, 149 and 130 (145); 3100 rows 144 and 117 (122).
-          if (rounds(t192) * 10 <= rounds(t128) * 7) e = launch_gemm_dma<192, 128, 2, 2, false, 4, false, false, false, 1, true>(lc, gg, (uint32_t)t192);
-          else e = launch_gemm_dma<128, 128, 2, 2, false, 5, false, false, false, 1, true>(lc, gg, (uint32_t)t128);
+          if (rounds(t192) * 10 <= rounds(t128) * 7) e = launch_gemm_plain<192, 128, 2, 2, 4, 1, true>(lc, gg, t192);
+          else e = launch_gemm_plain<128, 128, 2, 2, 5, 1, true>(lc, gg, t128);
         } else if (g.K < 2048) {
           // two to a CU; eight waves share the tail, the stores after few k-steps (16384 rows of 1536, K = 1152, 62 -> 56 us), four are
           // ahead in a long main loop (4000 rows of 2048, K = 2048 40, 43; 3500 rows 38, 40)
-          e = launch_gemm_dma<128, 128, 2, 4, false, 2>(lc, gg, (uint32_t)t128);
+          e = launch_gemm_plain<128, 128, 2, 4>(lc, gg, t128);
         } else {
-          e = launch_gemm_dma<128, 128, 2, 2>(lc, gg, (uint32_t)t128);
+          e = launch_gemm_plain<128, 128, 2, 2>(lc, gg, t128);
         }
       }
       if (e != hipSuccess) return e;
