@@ -3366,10 +3366,13 @@ hipError_t launch_matmul(const LaunchCtx &lc_in, const GemmDesc &g, const char *
           // 18.9 -> 18.2; 18 steps 14.8, 16.0; 16 steps 14.1, 15.7 and 14.8, 16.6).
           if (steps >= 24) e = launch_gemm_plain<128, 128, 2, 2, 5, 1, true>(lc, gg, t128);
           else e = launch_gemm_plain<128, 128, 2, 4, 4>(lc, gg, t128);
-        } else if (t192 <= cus && steps >= 4) {
+        } else if (t192 <= cus) {
           // a round of 192 rows (o_proj and down_proj of 2900 rows: 29 and 91 us; 368 tiles of 128 rows two to a CU 35 and 122; 1024
-          // deep 19.7, 21.6)
-          e = launch_gemm_plain<192, 128, 2, 2, 4, 1, true>(lc, gg, t192);
+          // deep 19.7, 21.6).  Up to nine k-steps eight wavefronts, whose start and tail are shorter (2900 x 2048: K = 64 8.4 us - four
+          // wavefronts take three steps at least, 128 rows two to a CU 8.8 -, 256 11.1 and 12.3, 512 14.5 and 14.8, 768 18.3 and 17.7;
+          // 6000 x 700 x 256 10.4, 11.7).
+          if (steps >= 10) e = launch_gemm_plain<192, 128, 2, 2, 4, 1, true>(lc, gg, t192);
+          else e = launch_gemm_plain<192, 128, 2, 4, 3>(lc, gg, t192);
         } else if (steps >= 64) {
           // Several rounds of a deep product, a round of 192 rows at 1.42 times one of 128: 8192 x 1152 x 6912 two or three, 134 and 148 us
           // (two to a CU 167); 4000 x 2048 x 8192 two either way, 149 and 130 (145); 3100 rows 144 and 117 (122).

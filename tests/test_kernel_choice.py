@@ -52,3 +52,14 @@ for b, m, n, k in ((1, 3841, 3843, 128), (1, 4090, 4093, 192), (1, 8001, 2046, 2
     names = product(m, n, k, batch=b, residual=True)
     assert len(names) == 1 and "gemm_bf16_ring_kernelILi0ELi2E" in names[0], (b, m, n, k, names)
 """, BF16)
+
+
+def test_a_round_of_192_rows(fake_hip):  # noqa: F811
+    """Four wavefronts from ten k-steps on, eight below."""
+    fake_hip(LAUNCHED + """
+for m, n, k, waves in ((2305, 2049, 64, 8), (6000, 700, 256, 8), (2303, 2049, 576, 8), (2303, 2049, 640, 4), (2305, 2048, 2048, 4)):
+    for residual in (False, True):
+        names = product(m, n, k, residual=residual)
+        assert len(names) == 1 and "gemm_bf16_dma_kernelILi192ELi128ELi2ELi%dELb0E" % (waves // 2) in names[0], (m, n, k, names)
+        assert names[0].endswith("ELb%dEEEvNS_8GemmDescE" % residual), names
+""", BF16)

@@ -28,12 +28,13 @@ def product_and_bound(x, w):
     return x @ w.T, x.shape[-1] * 2.0 ** -24 * (np.abs(x) @ np.abs(w).T)
 
 
-# 256 x 256 tiles; then 128 x 128 in one round of 33 and 17 steps and in two rounds, 192 x 128 in one round of 4, 5 and 32 steps
-# and in two rounds
+# 256 x 256 tiles and smaller ones; then 128 x 128 in one round of 33 and 17 steps and in two rounds, 192 x 128 in one round of 4, 5
+# and 32 steps and in two rounds
 @pytest.mark.gpu
 @pytest.mark.parametrize("M,N,K", [(4096, 4096, 128), (4097, 4101, 192), (3841, 4353, 256), (8300, 2049, 320), (255, 65600, 448),
                                    (1500, 2050, 2112), (1400, 1410, 1088), (3100, 2050, 4160),
                                    (2300, 2050, 256), (2303, 2049, 320), (2305, 2048, 2048), (4200, 2050, 4096),
+                                   (2305, 2049, 64), (2303, 2049, 576), (2303, 2049, 640),    # ... of one and nine steps on eight wavefronts, of ten on four
                                    # 256 x 256 again, with one to three columns in the last piece and quadrants past both edges
                                    (4090, 4093, 192), (3841, 3843, 256), (8001, 2046, 320), (255, 65299, 448)])
 def test_product(hip_bf16, M, N, K):
@@ -55,7 +56,7 @@ def test_narrow_product(hip_bf16, M, N, K):
 # a residual added as the product is stored: each tile that does so, whole rounds of large tiles with the rest on smaller ones
 # (also where the rounds alone would leave 40 rows), quadrants of a tile past every edge and three columns in the last piece, a batch, and the forms that leave the add to someone else (64 rows, k-slices)
 @pytest.mark.gpu
-@pytest.mark.parametrize("B,M,N,K", [(1, 4097, 4101, 192), (1, 8300, 2050, 2048), (1, 1500, 2050, 2112), (1, 2303, 2049, 320), (1, 3100, 2050, 1024),
+@pytest.mark.parametrize("B,M,N,K", [(1, 4097, 4101, 192), (1, 8300, 2050, 2048), (1, 1500, 2050, 2112), (1, 2303, 2049, 320), (1, 2303, 2049, 640), (1, 3100, 2050, 1024),
                                      (1, 8232, 2048, 2048), (1, 296, 33000, 2048), (1, 3300, 2050, 2048),
                                      (1, 3841, 3843, 128), (1, 4090, 4093, 192), (1, 8001, 2046, 256), (16, 1000, 1002, 128), (1, 300, 130, 64), (1, 1000, 1000, 256), (3, 700, 520, 192), (1, 64, 200, 128),
                                      (1, 200, 300, 2048)])
