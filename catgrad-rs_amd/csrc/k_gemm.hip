@@ -3356,9 +3356,10 @@ hipError_t launch_matmul(const LaunchCtx &lc_in, const GemmDesc &g, const char *
           else e = launch_gemm_dma<128, 128, 2, 4, false, 2, false, false, true>(lc, gg, (uint32_t)t128);
         } else if (splits == 1 && t128 * 2 <= cus && g.N >= 128) {
           // too few 128 x 128 tiles for the CUs and no split-K to multiply them: halve the tile, or quarter it if every CU still holds
-          // one at most (1536 columns, K = 1152: 100 rows 11.2 -> 9.5 us, 400 11.3 -> 9.6, 640 11.3 -> 10.1)
+          // one at most (1536 columns, K = 1152: 100 rows 11.2 -> 9.5 us, 400 11.3 -> 9.6, 640 11.3 -> 10.1; 300 x 2048 x 512 6.9 -> 6.4,
+          // 256 even; below that the halves: 300 x 2048 x 64 4.5 -> 4.3, 900 x 700 x 128 4.8 -> 4.65, 900 x 700 x 192 5.3 -> 5.1)
           const uint64_t t64 = (uint64_t)((g.M + 63) / 64) * ((g.N + 63) / 64) * batch;
-          e = t64 <= cus ? launch_gemm_plain<64, 64, 2, 2, 8, 2>(lc, gg, t64)
+          e = t64 <= cus && g.K >= 256 ? launch_gemm_plain<64, 64, 2, 2, 8, 2>(lc, gg, t64)
                          : launch_gemm_plain<128, 64, 4, 2, 4>(lc, gg, (uint64_t)((g.M + 127) / 128) * ((g.N + 63) / 64) * batch);
         } else if (t128 <= cus) {
           // A round of 128 rows.  The four wavefronts' longer start and tail pay from about 24 k-steps on (weights from memory: 900 x

@@ -63,3 +63,14 @@ for m, n, k, waves in ((2305, 2049, 64, 8), (6000, 700, 256, 8), (2303, 2049, 57
         assert len(names) == 1 and "gemm_bf16_dma_kernelILi192ELi128ELi2ELi%dELb0E" % (waves // 2) in names[0], (m, n, k, names)
         assert names[0].endswith("ELb%dEEEvNS_8GemmDescE" % residual), names
 """, BF16)
+
+
+def test_less_than_a_round(fake_hip):  # noqa: F811
+    """A quarter of a 128 x 128 tile from four k-steps on, half of one below or where the quarters are more than the CUs."""
+    fake_hip(LAUNCHED + """
+for m, n, k, tile in ((140, 700, 192, "Li128ELi64E"), (300, 300, 256, "Li64ELi64E"), (900, 700, 64, "Li128ELi64E"), (1200, 700, 256, "Li64ELi64E"),
+                      (1000, 1100, 256, "Li128ELi64E")):
+    for residual in (False, True):
+        names = product(m, n, k, residual=residual)
+        assert len(names) == 1 and "gemm_bf16_dma_kernelI" + tile in names[0], (m, n, k, names)
+""", BF16)
