@@ -36,21 +36,23 @@ def product(m, n, k, along_k=True, batch=1, residual=False):
 def test_no_kernel_with_fixed_places_in_lds_beside_variables_of_its_own(fake_hip):  # noqa: F811
     fake_hip(LAUNCHED + """
 fake.fake_hip_static_lds(64)
-assert fails(lambda: product(4096, 4096, 128))
+assert fails(lambda: product(4096, 4096, 320))
 fake.fake_hip_static_lds(0)
-assert ["gemm_bf16_ring" in n for n in product(4096, 4096, 128)] == [True]
+assert ["gemm_bf16_ring" in n for n in product(4096, 4096, 320)] == [True]
 """, BF16)
 
 
 def test_products_on_256_x_256_tiles(fake_hip):  # noqa: F811
-    """The sizes that test_large_tiles.py gives its edges, and batches."""
+    """The sizes that test_large_tiles.py gives its edges, and batches: four wavefronts from five k-steps on and for a residual."""
     fake_hip(LAUNCHED + """
-for m, n, k in ((4096, 4096, 128), (4090, 4093, 192), (3841, 3843, 256), (8001, 2046, 320), (255, 65299, 448)):
+four, eight = "gemm_bf16_ring_kernelILi0ELi2E", "gemm_bf16_dma_kernelILi256ELi256ELi2ELi4ELb0ELi2E"
+for m, n, k in ((4096, 4096, 128), (4090, 4093, 192), (3841, 3843, 256), (8001, 2046, 320), (255, 65299, 448), (4096, 4093, 320)):
     names = product(m, n, k)
-    assert len(names) == 1 and "gemm_bf16_ring_kernelILi0ELi2E" in names[0], (m, n, k, names)
+    assert len(names) == 1 and (four if k > 256 else eight) in names[0], (m, n, k, names)
 for b, m, n, k in ((1, 3841, 3843, 128), (1, 4090, 4093, 192), (1, 8001, 2046, 256), (16, 1000, 1002, 128)):
-    names = product(m, n, k, batch=b, residual=True)
-    assert len(names) == 1 and "gemm_bf16_ring_kernelILi0ELi2E" in names[0], (b, m, n, k, names)
+    for residual in (False, True):
+        names = product(m, n, k, batch=b, residual=residual)
+        assert len(names) == 1 and (four if residual else eight) in names[0], (b, m, n, k, names)
 """, BF16)
 
 
