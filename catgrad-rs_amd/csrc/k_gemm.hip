@@ -3327,11 +3327,12 @@ hipError_t launch_matmul(const LaunchCtx &lc_in, const GemmDesc &g, const char *
         if (!g.n_group && fill(t128, 2 * (uint64_t)lc.n_cus) > 1.15 * fill(t256, (uint64_t)lc.n_cus))
           e = g.K < 2048 ? launch_gemm_plain<128, 128, 2, 4>(lc, gg, t128)  // (as below)
                          : launch_gemm_plain<128, 128, 2, 2>(lc, gg, t128);
-        else if (g.K <= 256 && !g.n_group && !g.c_add)
-          // Two to four k-steps: what a tile stores is most of it, and eight wavefronts store it as they come.  16 x 1024 x 1024 x 128
-          // 17.1 us, with four 18.4 us; x 192 19.3, 20.6; 32 x 2048 x 2048 x 128 120, 130, x 256 150, 157; 8192 x 4096 x 128 31, 38, x 256
-          // 38, 45; but 4096 x 8192 x 128 37, 33, and from five steps on four are ahead nearly everywhere (16 x 1024 x 1024 x 512 29.4,
-          // 28.9; 4096 x 8192 x 512 58, 52; 8192 x 4096 x 512 51, 55, whose result lies 16 KB a row).  A residual, or biases, four
+        else if ((g.K < 384 || (g.K <= 512 && batch == 1 && tiles_m > tiles_n && t256 >= 2 * (uint64_t)lc.n_cus)) && !g.n_group && !g.c_add)
+          // Few k-steps: what a tile stores is most of it, and eight wavefronts store it as they come.  16 x 1024 x 1024 x 128 17.1 us,
+          // with four 18.4; x 192 19.3, 20.6; x 320 24, 24 to 30; 32 x 2048 x 2048 x 128 120, 130, x 256 150, 157; 8192 x 4096 x 128 31,
+          // 38, x 256 38, 45, x 384 46, 51 to 59, x 512 52, 55 to 61; but 4096 x 8192 x 128 37, 33.  (The ranges are from box to box, of
+          // the four alone.)  Beyond, four are ahead: 16 x 1024 x 1024 x 512 29.6, 29.4; 4096 x 4096 x 384 25.2, 24.9; 4096 x 8192 x
+          // 512 58 to 62, 52 to 57; tall ones in rounds from K = 576 on (8192 x 4096 x 1024 82, 80).  A residual, or biases, four
           // wavefronts add on their way (8192 x 2048 x 128 and a residual 27, 48 with an add of its own).
           e = launch_gemm_dma<256, 256, 2, 4>(lc, gg, (uint32_t)t256);
         else

@@ -36,19 +36,20 @@ def product(m, n, k, along_k=True, batch=1, residual=False):
 def test_no_kernel_with_fixed_places_in_lds_beside_variables_of_its_own(fake_hip):  # noqa: F811
     fake_hip(LAUNCHED + """
 fake.fake_hip_static_lds(64)
-assert fails(lambda: product(4096, 4096, 320))
+assert fails(lambda: product(4096, 4096, 384))
 fake.fake_hip_static_lds(0)
-assert ["gemm_bf16_ring" in n for n in product(4096, 4096, 320)] == [True]
+assert ["gemm_bf16_ring" in n for n in product(4096, 4096, 384)] == [True]
 """, BF16)
 
 
 def test_products_on_256_x_256_tiles(fake_hip):  # noqa: F811
-    """The sizes that test_large_tiles.py gives its edges, and batches: four wavefronts from five k-steps on and for a residual."""
+    """The sizes that test_large_tiles.py gives its edges, and batches: eight wavefronts for few k-steps, four beyond and for a residual."""
     fake_hip(LAUNCHED + """
 four, eight = "gemm_bf16_ring_kernelILi0ELi2E", "gemm_bf16_dma_kernelILi256ELi256ELi2ELi4ELb0ELi2E"
-for m, n, k in ((4096, 4096, 128), (4090, 4093, 192), (3841, 3843, 256), (8001, 2046, 320), (255, 65299, 448), (4096, 4093, 320)):
+for m, n, k, kernel in ((4096, 4096, 128, eight), (4090, 4093, 192, eight), (3841, 3843, 256, eight), (8001, 2046, 320, eight), (255, 65299, 448, four),
+                        (4096, 4093, 384, four), (8192, 4096, 512, eight), (8192, 4096, 576, four), (4096, 8192, 512, four), (8192, 2048, 512, four)):
     names = product(m, n, k)
-    assert len(names) == 1 and (four if k > 256 else eight) in names[0], (m, n, k, names)
+    assert len(names) == 1 and kernel in names[0], (m, n, k, names)
 for b, m, n, k in ((1, 3841, 3843, 128), (1, 4090, 4093, 192), (1, 8001, 2046, 256), (16, 1000, 1002, 128)):
     for residual in (False, True):
         names = product(m, n, k, batch=b, residual=residual)

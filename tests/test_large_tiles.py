@@ -37,7 +37,7 @@ def product_and_bound(x, w):
                                    (2305, 2049, 64), (2303, 2049, 576), (2303, 2049, 640),    # ... of one and nine steps on eight wavefronts, of ten on four
                                    (140, 700, 192), (300, 300, 256), (1000, 1100, 256),       # less than a round: halves and quarters of 128 x 128
                                    # 256 x 256 again, with one to three columns in the last piece and quadrants past both edges
-                                   (4090, 4093, 192), (3841, 3843, 256), (8001, 2046, 320), (255, 65299, 448), (4096, 4093, 320), (3841, 3843, 576)])
+                                   (4090, 4093, 192), (3841, 3843, 256), (8001, 2046, 320), (255, 65299, 448), (4096, 4093, 384), (3841, 3843, 576), (8191, 4095, 512)])
 def test_product(hip_bf16, M, N, K):
     g = np.random.default_rng(M)
     x, w = draw(g, (1, M, K)), draw(g, (N, K))
