@@ -2970,8 +2970,13 @@ static bool gemm_fast_path(const GemmDesc &g, int av, int bv) {
          (g.sbk == 1 || g.sbn == 1) && g.K % 8 == 0 && (g.sbk == 1 || g.N % 8 == 0) && av && bv;
 }
 
-// gemm_bf16_column_kernel's products (not split)
+// gemm_bf16_column_kernel's products (not split).  A wave to a row costs a workgroup per four rows, 64 x 64 tiles one per 64 and 0.006
+// us per k, so few k of very many rows stay with those (us, column and tiles: K = 72, 300 rows 3.0, 3.8, 6000 3.8, 3.8, 8192 4.4, 3.8,
+// 65000 17, 5.4; K = 256, 33 rows 2.8, 3.4, 8192 4.4, 4.6, 12000 5.3, 4.6; K = 512, 16384 rows 6.9, 7.9, 32000 10.7, 8.6; K = 1024,
+// 65000 rows 23.6, 25.0), and with few rows a launch is no shorter for them (17 rows, K = 72 3.0, 2.5; 160 2.9, 2.8).
 static bool gemm_column_ok(const GemmDesc &g, int av, int bv) {
+  const uint64_t rows = (uint64_t)g.M * g.nb0 * g.nb1;
+  if (!(g.K >= 1024 || (g.K >= 160 && 32 * (uint64_t)g.K >= rows) || (g.M > 64 && rows <= 6000))) return false;
   return g.N == 1 && g.sbk == 1 && gemm_fast_path(g, av, bv) && !g.c_add && !g.c16 && !g.glu_gate && !g.n_group && !g.dual_b &&
          g.nb0 * g.nb1 <= 65535;
 }

@@ -77,3 +77,13 @@ for m, n, k, tile in ((140, 700, 192, "Li128ELi64E"), (300, 300, 256, "Li64ELi64
         names = product(m, n, k, residual=residual)
         assert len(names) == 1 and "gemm_bf16_dma_kernelI" + tile in names[0], (m, n, k, names)
 """, BF16)
+
+
+def test_one_column(fake_hip):  # noqa: F811
+    """A wave to a row unless few k of very many rows, or of one tile's worth, are quicker on 64 x 64 tiles."""
+    fake_hip(LAUNCHED + """
+for b, m, k, column in ((1, 17, 72, 0), (1, 17, 160, 1), (1, 65, 72, 1), (1, 6000, 64, 1), (1, 6001, 176, 0), (1, 6001, 192, 1), (1, 16384, 504, 0),
+                        (1, 16384, 512, 1), (1, 70000, 1016, 0), (1, 70000, 1024, 1), (100, 66, 192, 0), (20, 66, 64, 1)):
+    names = product(m, 1, k, batch=b)
+    assert len(names) == 1 and ("gemm_bf16_column" if column else "gemm_bf16_nt_kernelILi64ELi64E") in names[0], (b, m, k, names)
+""", BF16)
