@@ -2980,12 +2980,19 @@ static bool gemm_column_ok(const GemmDesc &g, int av, int bv) {
   return g.N == 1 && g.sbk == 1 && gemm_fast_path(g, av, bv) && !g.c_add && !g.c16 && !g.glu_gate && !g.n_group && !g.dual_b &&
          g.nb0 * g.nb1 <= 65535;
 }
-// Less than 64 columns, more than half of them, not too deep: direct-to-LDS tiles of 32 x 32 with a quarter of each k-step to a
-// wavefront, and no slices - a launch that sums them takes 4.7 us whatever its size (the router of a MoE prefill, K = 2048, 60
-// columns: 1024 rows 9.2 us, 64 x 64 tiles in four slices 7.6 and their sum; 400 rows 8.2, 6.5; 30 rows 8.1, 5.3; through registers
-// 9.4, 7.8, 7.4 and the sum).
-static bool gemm_narrow_dma_ok(const GemmDesc &g) {
-  return g.N > 32 && g.N < 64 && g.sak == 1 && g.sbk == 1 && g.K % 64 == 0 && g.K >= 64 && g.K <= 4096 && gemm_rows(g.M, g.K) && !g.c_add && !g.n_group && !g.act_sigmoid;
+// Less than 64 columns, more than half of them: direct-to-LDS tiles of 32 x 32 with a quarter of each k-step to a wavefront, and no
+// slices - a launch that sums them takes 2 to 5 us whatever its size.  A tile lasts 3 us and 2.2 ns per k, so they end where the
+// tiles through registers have a few steps only, or slices short enough to make up for their sum, and where a third workgroup would
+// have to wait for a place on its CU (us here and there, 60 columns: K = 256, 200 rows 4.4, 4.1, 1024 4.6, 4.6, 8192 5.5, 5.0; K =
+// 448, 65 rows 4.8, 4.8, 8192 6.0, 6.2; K = 1024, 17 rows 5.2, 7.2, 1024 6.2, 8.7, 8192 7.9, 14.4; K = 2048, 1024 rows 8.3, 9.2, 10000
+// 21.3, 20.3; K = 512, 10000 rows 10.4, 8.3; K = 3584, 65 rows 11.6, 10.7, 200 11.6, 11.3, 1024 12.1, 15.7; K = 4096, 200 rows 13.6, 10.1, 1024 13.5,
+// 12.0, 4096 14.1, 15.5, 8192 17.4, 21.5).  Results of a size that cannot be summed in pieces of 16 bytes have no slices (17 x 63 x
+// 4096 12.7, 27.3).
+static bool gemm_narrow_dma_ok(const LaunchCtx &lc, const GemmDesc &g) {
+  const uint64_t row_tiles = (uint64_t)((g.M + 31) / 32) * g.nb0 * g.nb1, cus = (uint64_t)lc.n_cus;
+  if (row_tiles > cus || g.K < (row_tiles > cus / 2 || (row_tiles > 1 && row_tiles < cus / 16) ? 448u : 320u)) return false;
+  if (g.K > (row_tiles <= cus / 16 ? 3072u : 3584u) && row_tiles < 3 * cus / 8 && (uint64_t)g.M * g.N * g.nb0 * g.nb1 % 4 == 0) return false;
+  return g.N > 32 && g.N < 64 && g.sak == 1 && g.sbk == 1 && g.K % 64 == 0 && g.K <= 4096 && gemm_rows(g.M, g.K) && !g.c_add && !g.n_group && !g.act_sigmoid;
 }
 
 bool gemm_epilogue_ok(const GemmDesc &g) {
@@ -3128,7 +3135,7 @@ uint32_t gemm_split_k(const LaunchCtx &lc, const GemmDesc &g) {
       splits *= 2;
     return splits;
   }
-  if (gemm_column_ok(g, av, bv) || (gemm_fast_path(g, av, bv) && gemm_narrow_dma_ok(g))) return 1;
+  if (gemm_column_ok(g, av, bv) || (gemm_fast_path(g, av, bv) && gemm_narrow_dma_ok(lc, g))) return 1;
   if (gemm_dma_ok(g) && g.M <= 64) {
     // Tiles of 64 x 64: a workgroup to every CU, four k-steps at least to each - and none below 16 k-steps, where the pass
     // that sums the slices costs what they save (17 x 512 x 64 9.6 us in two slices, 5.5 in one; 17 x 768 x 256 9.8, 8.0; 40 x
@@ -3409,7 +3416,7 @@ hipError_t launch_matmul(const LaunchCtx &lc_in, const GemmDesc &g, const char *
       if (e != hipSuccess) return e;
     } else if (splits == 1 && gemm_column_ok(g, av, bv)) {
       CG_LAUNCH(lc, gemm_bf16_column_kernel, dim3((g.M + 3) / 4, batch), 256, gg);
-    } else if (gemm_narrow_dma_ok(g)) {
+    } else if (gemm_narrow_dma_ok(lc, g)) {
       const hipError_t e = launch_gemm_dma<32, 32, 1, 1, false, 8, false, false, false, 4>(lc, gg, (uint32_t)((uint64_t)((g.M + 31) / 32) * ((g.N + 31) / 32) * batch * splits));
       if (e != hipSuccess) return e;
     } else {

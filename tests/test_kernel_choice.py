@@ -87,3 +87,16 @@ for b, m, k, column in ((1, 17, 72, 0), (1, 17, 160, 1), (1, 65, 72, 1), (1, 600
     names = product(m, 1, k, batch=b)
     assert len(names) == 1 and ("gemm_bf16_column" if column else "gemm_bf16_nt_kernelILi64ELi64E") in names[0], (b, m, k, names)
 """, BF16)
+
+
+def test_less_than_64_columns(fake_hip):  # noqa: F811
+    """32 x 32 tiles of the whole of k, or 64 x 64 ones through registers and, deep, in slices."""
+    fake_hip(LAUNCHED + """
+direct, registers = "gemm_bf16_dma_kernelILi32ELi32E", "gemm_bf16_nt_kernelILi64ELi64E"
+for b, m, n, k, kernel in ((1, 17, 60, 256, registers), (1, 17, 60, 320, direct), (1, 65, 33, 384, registers), (1, 65, 33, 448, direct),
+                                     (1, 512, 60, 256, registers), (1, 512, 60, 320, direct), (1, 4096, 60, 320, direct), (1, 4097, 60, 384, registers),
+                                     (1, 8192, 60, 448, direct), (1, 8193, 60, 512, registers), (3, 4096, 60, 512, registers), (1, 512, 60, 3072, direct), (1, 512, 60, 3136, registers), (1, 513, 60, 3584, direct),
+                                     (1, 1024, 60, 4096, registers), (1, 1023, 63, 4096, direct), (1, 3072, 60, 4096, direct), (1, 200, 60, 4160, registers)):
+    names = product(m, n, k, batch=b)
+    assert len(names) == 1 and kernel in names[0], (b, m, n, k, names)
+""", BF16)

@@ -46,11 +46,12 @@ def test_product(hip_bf16, M, N, K):
     assert np.all(np.abs(got[0] - ref) <= bound)
 
 
-# one column (a wave to a row, its last pieces of k partly past the end, or 64 x 64 tiles), and more than 32 columns but less than 64, to
-# the deepest that is one launch and beyond
+# one column (a wave to a row, its last pieces of k partly past the end, or 64 x 64 tiles), and more than 32 columns but less than 64:
+# tiles of 32 x 32 and of 64 x 64 at both ends of either, slices of the deepest
 @pytest.mark.gpu
 @pytest.mark.parametrize("M,N,K", [(1030, 1, 2048), (17, 1, 200), (300, 1, 2056), (65, 1, 8), (17, 1, 72), (6001, 1, 176), (6001, 1, 192), (16385, 1, 504),
-                                   (1030, 60, 2048), (65, 33, 64), (129, 63, 1088), (9, 60, 1024), (200, 60, 4096), (200, 60, 4160)])
+                                   (1030, 60, 2048), (65, 33, 64), (129, 63, 1088), (9, 60, 1024), (200, 60, 4096), (200, 60, 4160),
+                                   (65, 33, 384), (65, 33, 448), (513, 61, 320), (8192, 60, 448), (8193, 60, 512), (1023, 63, 4096), (3072, 60, 4096)])
 def test_narrow_product(hip_bf16, M, N, K):
     test_product(hip_bf16, M, N, K)
 
