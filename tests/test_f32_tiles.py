@@ -17,15 +17,16 @@ def product(rank, along_k, act=False):
     return f
 
 
-SIZES = [(1, 33, 132, 1044), (3, 70, 260, 100), (1, 520, 900, 2060), (1, 1000, 1000, 1000),     # 32 and 64 rows
-         (1, 96, 32000, 132), (1, 256, 32000, 60), (1, 155, 32700, 100), (1, 700, 2048, 4100),  # 96, 128, 160, 192 rows
-         (1, 220, 30000, 100), (1, 8190, 4096, 44), (32, 300, 300, 64)]                         # 224, 256 rows; many products
+# height of the tile in units of 32 rows (test_kernel_choice.py asserts that each size is given it): B, M, N, K
+SIZES = [(1, 1, 40, 8196, 516), (1, 3, 70, 2060, 100), (1, 1, 1000, 1000, 1000), (2, 1, 130, 7312, 52), (2, 1, 520, 900, 2060), (2, 32, 300, 300, 64),
+         (3, 1, 96, 32000, 132), (3, 1, 700, 2048, 4100), (4, 1, 256, 32000, 60), (5, 1, 155, 32700, 100), (6, 1, 185, 5380, 1404),
+         (7, 1, 220, 30000, 100), (8, 1, 8190, 4096, 44), (8, 1, 719, 2820, 1288)]
 
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("along_k", [True, False])
-@pytest.mark.parametrize("B,M,N,K", SIZES)
-def test_product(hip, B, M, N, K, along_k):
+@pytest.mark.parametrize("rows,B,M,N,K", SIZES)
+def test_product(hip, rows, B, M, N, K, along_k):
     g = np.random.default_rng(M + K)
     x = g.standard_normal((B, M, K)).astype(np.float32)
     w = g.standard_normal((B, N, K) if along_k else (B, K, N)).astype(np.float32)

@@ -1,6 +1,7 @@
 """Which kernel a call is given, on the CPU: the library over the stand-in runtime of fake_hip.cpp, which says what was launched."""
 import pytest
 
+from test_f32_tiles import SIZES
 from test_host_copies import fake_hip  # noqa: F401 - a fixture
 
 BF16 = 1
@@ -100,3 +101,16 @@ for b, m, n, k, kernel in ((1, 17, 60, 256, registers), (1, 17, 60, 320, direct)
     names = product(m, n, k, batch=b)
     assert len(names) == 1 and kernel in names[0], (b, m, n, k, names)
 """, BF16)
+
+
+def test_f32_tiles(fake_hip):  # noqa: F811
+    """Every height of tile, with both layouts of the right operand, for the sizes of test_f32_tiles.py; 32 x 32 tiles where these are ahead."""
+    fake_hip(LAUNCHED + f"""
+for rows, b, m, n, k in {SIZES}:
+    for along_k in (True, False):
+        names = product(m, n, k, along_k, b)
+        assert len(names) == 1 and "gemm_f32_dma_kernelILi%dE" % rows in names[0] and names[0].split("ELb")[1][0] == "10"[along_k], (b, m, n, k, along_k, names)
+for b, m, n, k in ((1, 64, 256, 128), (1, 33, 132, 1044), (3, 70, 260, 100), (1, 10, 512, 2048), (1, 2000, 20, 2000)):
+    names = product(m, n, k, batch=b)
+    assert len(names) == 1 and "gemm_small_f32_kernel" in names[0], (b, m, n, k, names)
+""")
