@@ -353,15 +353,25 @@ static bool gemm_small_ok(const LaunchCtx &lc, const GemmDesc &g) {
 // An f32 product for k_gemm_f32.hip: all that it takes, unless the kernel above is ahead.  That one takes about 3 us and 13.5 ns per
 // k of a workgroup, half as much again when every CU has more than one, and 3 for a sum of slices (us here, 12 to 16 there: 10 x 512 x
 // 2048 9.5, 11; 64 x 256 x 128 4.4, 5.7; 2000 x 20 x 2000 11.5, 17; 300 x 1000 x 500 13.9, 11.2; 17 x 2048 x 2048 15.5, 12.7).
+// splits (optional): the slices of k it is fastest with.
 static uint32_t gemm_small_split(const LaunchCtx &lc, const GemmDesc &g);
-static bool gemm_f32_tiles(const LaunchCtx &lc, const GemmDesc &g) {
+static bool gemm_f32_tiles(const LaunchCtx &lc, const GemmDesc &g, uint32_t *splits = nullptr) {
   if (!gemm_f32_ok(g)) return false;
-  if (!gemm_small_ok(lc, g)) return true;
-  const uint32_t s = gemm_small_split(lc, g);
-  const uint64_t wgs = (uint64_t)((g.M + 31) / 32) * ((g.N + 31) / 32) * g.nb0 * g.nb1 * s;
+  double small_us = 1e30;
+  if (gemm_small_ok(lc, g)) {
+    const uint32_t s = gemm_small_split(lc, g);
+    const uint64_t wgs = (uint64_t)((g.M + 31) / 32) * ((g.N + 31) / 32) * g.nb0 * g.nb1 * s;
+    small_us = 3.0 + 0.0135 * g.K / s * (wgs > (uint64_t)lc.n_cus ? 1.5 : 1.0) + (s > 1 ? 3.0 : 0.0);
+    // (gemm_f32_split looks at up to 128 forms: not where none can be ahead)
+    if (small_us <= gemm_f32_least_us(g)) return false;
+  } else if (!splits) {
+    return true;
+  }
   double us = 0;
-  gemm_f32_split(lc, g, &us);
-  return us < 3.0 + 0.0135 * g.K / s * (wgs > (uint64_t)lc.n_cus ? 1.5 : 1.0) + (s > 1 ? 3.0 : 0.0);
+  const uint32_t best = gemm_f32_split(lc, g, &us);
+  if (us >= small_us) return false;
+  if (splits) *splits = best;
+  return true;
 }
 
 // ---- bf16 x bf16 "NT" GEMM: the prefill fast path --------------------------------------------------
@@ -3120,7 +3130,7 @@ uint32_t gemm_split_k(const LaunchCtx &lc, const GemmDesc &g) {
   const uint64_t tiles = (uint64_t)((g.M + 127) / 128) * ((g.N + 127) / 128) * batch;
   uint32_t splits = 1;
   if (gemv_rows_plain_ok(lc, g)) return 1;
-  if (gemm_f32_tiles(lc, g)) return gemm_f32_split(lc, g, nullptr);
+  if (gemm_f32_tiles(lc, g, &splits)) return splits;
   if (gemm_small_ok(lc, g)) return gemm_small_split(lc, g);
   if (!gemm_fast_path(g, av, bv)) {
     // the generic kernel (f32 products): same idea, shorter k-steps, so thinner slices still pay

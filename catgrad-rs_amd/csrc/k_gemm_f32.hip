@@ -191,6 +191,12 @@ static double f32_best(const LaunchCtx &lc, const GemmDesc &g, uint32_t splits, 
   return best;
 }
 
+// No form takes less than f32_cost has it for one round of 32 rows over all of k, or over the 64 that a slice has at least.
+double gemm_f32_least_us(const GemmDesc &g) {
+  const double per_k = 1.08 * 32 / 2300.0 * 1.38;
+  return std::min(6.0 + per_k * g.K, 9.0 + per_k * 64) * (1 - 1e-9);
+}
+
 uint32_t gemm_f32_split(const LaunchCtx &lc, const GemmDesc &g, double *us) {
   uint32_t best_splits = 1, rows = 0;
   double best = 1e30;
@@ -201,7 +207,7 @@ uint32_t gemm_f32_split(const LaunchCtx &lc, const GemmDesc &g, double *us) {
       best_splits = s;
     }
   }
-  if (us) *us = best;
+  *us = best;
   return best_splits;
 }
 

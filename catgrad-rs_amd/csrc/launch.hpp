@@ -364,9 +364,10 @@ struct GemmDesc {
 bool gemm_ring_ok(const GemmDesc &g);
 hipError_t launch_gemm_ring(const LaunchCtx &lc, const GemmDesc &g, bool half_height = false);
 // k_gemm_f32.hip: f32 products of operands in whole 16-byte pieces; gemm_f32_split: the slices of k it is fastest with (and how long
-// it then takes, about)
+// it then takes, about; gemm_f32_least_us: no less than this)
 bool gemm_f32_ok(const GemmDesc &g);
 uint32_t gemm_f32_split(const LaunchCtx &lc, const GemmDesc &g, double *us);
+double gemm_f32_least_us(const GemmDesc &g);
 hipError_t launch_gemm_f32(const LaunchCtx &lc, const GemmDesc &g);
 // split factor launch_matmul should be given for this problem (1 = none)
 uint32_t gemm_split_k(const LaunchCtx &lc, const GemmDesc &g);
