@@ -974,11 +974,13 @@ static bool attn_prefill_keysplit(const LaunchCtx &lc, const AttnPrefillDesc &d)
 
 // Heads of 128 and 256: two wavefronts to 32 queries, each with half of the values' dims (both compute the scores; the accumulators of
 // two waves then fit on a SIMD, and one's softmax runs under the other's products).  us a layer, heads of 128, causal, against one
-// wavefront to 32 queries: 16 heads of 400 tokens 24.0 -> 18.5, 1400 61.1 -> 49.2, 3000 109 -> 103, 4 x 256 20.5 -> 17.9; from about
-// one and a half workgroups of 128 queries a CU on the doubled scores weigh more (4 x 1000 52.3, 66.6).  Heads of 256: 4 heads of
-// 2000 tokens 75.5 -> 51.9, 8 x 1000 81.7 -> 61.1, 8 x 2048 152 -> 130.
+// wavefront to 32 queries: 16 heads of 400 tokens 24.0 -> 18.5, 1400 61.1 -> 49.2, 4 x 256 20.5 -> 17.9.  Beyond one workgroup of 128
+// queries a CU a second round of these begins and the doubled scores weigh more (causal mask, no mask, a mask without dead tiles: 16
+// heads of 2048 tokens 71, 83, 121, with one wavefront 88, 88, 120; 3000 tokens 107, 193, 289 here, 110, 136, 185 there; 2 x 1100 44,
+// 80, 115 and 49, 58, 77; 4 x 700 39, 58, 78 and 36, 43, 55).  Heads of 256, causal: 4 heads of 2000 tokens 75.5 -> 51.9, 8 x 1000
+// 81.7 -> 61.1, 8 x 2048 152 -> 130; without a mask 369 -> 316.
 static bool attn_prefill_wide(const LaunchCtx &lc, const AttnPrefillDesc &d) {
-  return !d.f32 && (d.d == 256 || (d.d == 128 && 2 * (uint64_t)((d.s + 127) / 128) * d.heads * d.b <= 3 * (uint64_t)lc.n_cus));
+  return !d.f32 && (d.d == 256 || (d.d == 128 && (uint64_t)((d.s + 127) / 128) * d.heads * d.b <= (uint64_t)lc.n_cus));
 }
 // ... in two key groups of 32 or 64 queries (0: one group) while a CU has at most one such workgroup and the keys are more than a
 // step: 100 tokens of 16 heads of 128 10.5 -> 9.8, 400 18.5 -> 16.7, 900 33.9 -> 27.8; 4 heads of 256, 700 tokens 40.3 -> 34.1, 2000

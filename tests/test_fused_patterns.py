@@ -1146,7 +1146,7 @@ def test_attention_prefill_with_an_arbitrary_shared_mask(oracle, hip_bf16_flash,
 
 
 @pytest.mark.parametrize("cfg", [(1, 32, 8, 512, 64), (2, 4, 2, 100, 128), (2, 4, 2, 104, 128), (1, 4, 1, 200, 256),
-                                 (1, 8, 8, 33, 64), (1, 2, 1, 1024, 64),
+                                 (1, 8, 8, 33, 64), (1, 2, 1, 1024, 64), (4, 33, 11, 130, 128),  # (more than a workgroup of 128 queries a CU)
                                  (1, 4, 1, 2048, 256)])  # the last: Gemma-3's heads at its prompt length, window 512
 @pytest.mark.parametrize("mask_kind", ["causal", "window"])
 def test_attention_prefill_bf16(oracle, hip_bf16_flash, hip_bf16, hip_nopat, cfg, mask_kind):

@@ -114,3 +114,36 @@ for b, m, n, k in ((1, 64, 256, 128), (1, 33, 132, 1044), (3, 70, 260, 100), (1,
     names = product(m, n, k, batch=b)
     assert len(names) == 1 and "gemm_small_f32_kernel" in names[0], (b, m, n, k, names)
 """)
+
+
+def test_attention_with_heads_of_128(fake_hip):  # noqa: F811
+    """Two wavefronts to 32 queries up to one workgroup of 128 queries a CU, with a mask and without; one beyond."""
+    fake_hip("""
+import importlib
+lang, nn = cg.lang, cg.nn
+helpers = importlib.import_module("catgrad-rs_amd.llm.helpers")
+fake.fake_hip_launched.restype = ctypes.c_char_p
+
+class Attention(lang.Module):
+    def __init__(self, shape, causal): self.shape, self.causal = shape, causal
+    def path(self): return lang.path(["attention", str(self.causal)])
+    def sort(self): return [lang.TENSOR] * 3, [lang.TENSOR]
+    def def_(self, b, args):
+        q, k, v = (lang.reshape(b, lang.make_shape(b, *self.shape), x) for x in args)
+        q, k, v = q + q - q, helpers.repeat_kv(b, 1, k + k - k), helpers.repeat_kv(b, 1, v + v - v)
+        s = lang.matmul(b, q, lang.transpose(b, 2, 3, k))
+        sh = lang.shape(b, s)
+        s = s / lang.constant(b, 11.0, sh)
+        if self.causal: s = s + lang.broadcast(b, helpers.causal_mask(b, lang.to_nat(b, self.shape[2])), sh)
+        return [lang.matmul(b, nn.softmax(b, s), v)]
+
+for shape, wide in (((1, 16, 2048, 128), 1), ((1, 16, 2049, 128), 0), ((4, 16, 512, 128), 1), ((2, 16, 1100, 128), 0)):
+    for causal in (False, True):
+        q, k, v = (be.tensor(np.zeros(int(np.prod(shape)), np.float32)) for _ in range(3))
+        be.sync()
+        fake.fake_hip_launched()
+        be.realize(cg.Interpreter(be, cg.stdlib(), cg.Parameters()).run(Attention(shape, causal).term(), [q, k, v])[0])
+        be.sync()
+        names = [n for n in fake.fake_hip_launched().decode().split("\\n") if "attn_prefill" in n]
+        assert len(names) == 1 and "attn_prefill_kernelILi128ELi64ELi4ELi1ELi%dE" % (wide + 1) in names[0], (shape, causal, names)
+""", BF16)
