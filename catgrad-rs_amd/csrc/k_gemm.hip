@@ -3002,7 +3002,7 @@ static bool gemm_narrow_dma_ok(const LaunchCtx &lc, const GemmDesc &g) {
   const uint64_t row_tiles = (uint64_t)((g.M + 31) / 32) * g.nb0 * g.nb1, cus = (uint64_t)lc.n_cus;
   if (row_tiles > cus || g.K < (row_tiles > cus / 2 || (row_tiles > 1 && row_tiles < cus / 16) ? 448u : 320u)) return false;
   if (g.K > (row_tiles <= cus / 16 ? 3072u : 3584u) && row_tiles < 3 * cus / 8 && (uint64_t)g.M * g.N * g.nb0 * g.nb1 % 4 == 0) return false;
-  return g.N > 32 && g.N < 64 && g.sak == 1 && g.sbk == 1 && g.K % 64 == 0 && g.K <= 4096 && gemm_rows(g.M, g.K) && !g.c_add && !g.n_group && !g.act_sigmoid;
+  return g.N > 32 && g.N < 64 && g.sak == 1 && g.sbk == 1 && g.K % 64 == 0 && g.K <= 4096 && gemm_rows(g.M, g.K) && !g.n_group && !g.act_sigmoid;
 }
 
 bool gemm_epilogue_ok(const GemmDesc &g) {
@@ -3013,15 +3013,17 @@ bool gemm_epilogue_ok(const GemmDesc &g) {
          (g.N % 4 == 0 || g.c16_pitch);
 }
 
-// More than 64 rows on the direct-to-LDS kernels, not split along k: every plain tile adds c_add as it stores.
-bool gemm_add_ok(const GemmDesc &g) {
+// More than 64 rows on the direct-to-LDS kernels, or less than 64 columns on them, not split along k: every plain tile adds c_add as it
+// stores.  (Few columns: their k-slices' sum added it before, and a launch of its own costs 3 to 5 us: 1024 x 60 x 2048 13.2 ->
+// 8.8, 200 x 60 x 1024 10.9 -> 6.8.)
+bool gemm_add_ok(const LaunchCtx &lc, const GemmDesc &g) {
   GemmDesc t = g;
   t.c_add = nullptr;
   const int asz = g.a_stype == ST_BF16 ? 2 : 4, bsz = g.b_stype == ST_BF16 ? 2 : 4;
   const int av = vec_ok(g.a, asz, g.sak == 1 ? g.sam : g.sak, g.sa_b0, g.sa_b1);
   const int bv = vec_ok(g.b, bsz, g.sbk == 1 ? g.sbn : g.sbk, g.sb_b0, g.sb_b1);
-  return g.M > 64 && g.splits <= 1 && !g.n_group && !g.dual_b && !g.glu_gate && !g.c16 && !g.act_sigmoid && !g.b_index &&
-         gemm_fast_path(t, av, bv) && gemm_dma_ok(t);
+  return g.splits <= 1 && !g.n_group && !g.dual_b && !g.glu_gate && !g.c16 && !g.act_sigmoid && !g.b_index && gemm_fast_path(t, av, bv) &&
+         (gemm_dma_ok(t) ? g.M > 64 : gemm_narrow_dma_ok(lc, t));
 }
 
 bool gemv_rows_plain_ok(const LaunchCtx &lc, const GemmDesc &g);
@@ -3181,7 +3183,7 @@ hipError_t launch_matmul(const LaunchCtx &lc_in, const GemmDesc &g, const char *
   // only the one-row kernels follow b_index; they add c_add, and so do the k-slice sum of a split GEMM and gemm_add_ok's tiles
   const bool one_row = g.M <= 8 && g.a_stype == ST_F32 && g.K > 0 && (b_unit_k || b_unit_n);
   if (g.b_index && !one_row) return hipErrorInvalidValue;
-  if (g.c_add && !one_row && g.splits <= 1 && !gemm_add_ok(g)) return hipErrorInvalidValue;
+  if (g.c_add && !one_row && g.splits <= 1 && !gemm_add_ok(lc_in, g)) return hipErrorInvalidValue;
   if ((g.glu_gate || g.c16 || g.n_group || g.dual_b) && !gemm_epilogue_ok(g)) return hipErrorInvalidValue;
   if (g.act_sigmoid && !gemm_act_ok(lc_in, g)) return hipErrorInvalidValue;
   if (g.rope_s && !gemm_rope_epilogue_ok(lc_in, g)) return hipErrorInvalidValue;
@@ -3427,7 +3429,7 @@ hipError_t launch_matmul(const LaunchCtx &lc_in, const GemmDesc &g, const char *
     } else if (splits == 1 && gemm_column_ok(g, av, bv)) {
       CG_LAUNCH(lc, gemm_bf16_column_kernel, dim3((g.M + 3) / 4, batch), 256, gg);
     } else if (gemm_narrow_dma_ok(lc, g)) {
-      const hipError_t e = launch_gemm_dma<32, 32, 1, 1, false, 8, false, false, false, 4>(lc, gg, (uint32_t)((uint64_t)((g.M + 31) / 32) * ((g.N + 31) / 32) * batch * splits));
+      const hipError_t e = launch_gemm_plain<32, 32, 1, 1, 8, 4>(lc, gg, (uint64_t)((g.M + 31) / 32) * ((g.N + 31) / 32) * batch * splits);
       if (e != hipSuccess) return e;
     } else {
     if (g.n_group) return hipErrorInvalidValue;

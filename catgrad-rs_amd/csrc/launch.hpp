@@ -374,8 +374,8 @@ uint32_t gemm_split_k(const LaunchCtx &lc, const GemmDesc &g);
 // whether launch_matmul would run this problem (splits as given) on the kernel that honours
 // glu_gate / c16
 bool gemm_epilogue_ok(const GemmDesc &g);
-// whether launch_matmul's kernel for a problem that is not split along k adds c_add (many rows)
-bool gemm_add_ok(const GemmDesc &g);
+// whether launch_matmul's kernel for a problem that is not split along k adds c_add (many rows, or few columns)
+bool gemm_add_ok(const LaunchCtx &lc, const GemmDesc &g);
 // whether launch_matmul's kernel for this problem (splits as given) honours act_sigmoid
 bool gemm_act_ok(const LaunchCtx &lc, const GemmDesc &g);
 // whether a bf16-mode product is worth copies of its operands in the direct-to-LDS kernel's layout (epilogue: it has one

@@ -1147,7 +1147,7 @@ int realize_matmul(cg_backend *be, cg_tensor *n, cg_tensor *addend, bool *added,
     }
     // A product that is not split along k adds the residual as it stores (2900 rows of 2048: an add of its own reads and
     // writes 72 MB, 11 us at either block end; here it reads 24).
-    if (splits <= 1 && addend && !be->addend_is_row && !*added && !ep && group.empty() && !g.c_add && gemm_add_ok(g)) {
+    if (splits <= 1 && addend && !be->addend_is_row && !*added && !ep && group.empty() && !g.c_add && gemm_add_ok(be->lc(), g)) {
       g.c_add = (const float *)data_ptr(addend);
       *added = true;
     }

@@ -98,8 +98,10 @@ for b, m, n, k, kernel in ((1, 17, 60, 256, registers), (1, 17, 60, 320, direct)
                                      (1, 512, 60, 256, registers), (1, 512, 60, 320, direct), (1, 4096, 60, 320, direct), (1, 4097, 60, 384, registers),
                                      (1, 8192, 60, 448, direct), (1, 8193, 60, 512, registers), (3, 4096, 60, 512, registers), (1, 512, 60, 3072, direct), (1, 512, 60, 3136, registers), (1, 513, 60, 3584, direct),
                                      (1, 1024, 60, 4096, registers), (1, 1023, 63, 4096, direct), (1, 3072, 60, 4096, direct), (1, 200, 60, 4160, registers)):
-    names = product(m, n, k, batch=b)
-    assert len(names) == 1 and kernel in names[0], (b, m, n, k, names)
+    for residual in (False, True):      # (32 x 32 tiles add it as they are stored)
+        names = product(m, n, k, batch=b, residual=residual)
+        assert len(names) == 1 and kernel in names[0], (b, m, n, k, names)
+        assert kernel != direct or names[0].endswith("ELb%dEEEvNS_8GemmDescE" % residual), names
 """, BF16)
 
 

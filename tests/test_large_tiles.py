@@ -62,7 +62,7 @@ def test_narrow_product(hip_bf16, M, N, K):
 @pytest.mark.parametrize("B,M,N,K", [(1, 4097, 4101, 192), (1, 8300, 2050, 2048), (1, 1500, 2050, 2112), (1, 2303, 2049, 320), (1, 2303, 2049, 640), (1, 3100, 2050, 1024),
                                      (1, 8232, 2048, 2048), (1, 296, 33000, 2048), (1, 3300, 2050, 2048),
                                      (1, 3841, 3843, 128), (1, 4090, 4093, 192), (1, 8001, 2046, 256), (16, 1000, 1002, 128), (1, 300, 130, 64), (1, 1000, 1000, 256), (3, 700, 520, 192), (1, 64, 200, 128),
-                                     (1, 200, 300, 2048)])
+                                     (1, 200, 300, 2048), (1, 4816, 35, 3648), (1, 17, 60, 320), (3, 700, 61, 512)])    # (the last three: 32 x 32 tiles)
 def test_product_and_residual(hip_bf16, B, M, N, K):
     g = np.random.default_rng(M)
     x, w, r = draw(g, (B, M, K)), draw(g, (N, K) if B == 1 else (B, N, K)), draw(g, (B, M, N), 3.0)
@@ -73,7 +73,7 @@ def test_product_and_residual(hip_bf16, B, M, N, K):
     hip_bf16.launch_counts(reset=True)
     got, _ = vectors.run(hip_bf16, f, 2, x, w, r)
     counts = hip_bf16.launch_counts(reset=True)
-    assert counts.get("gemm") == 1 and counts.get("ew_fused") == 1 and (M <= 64) == ("binary_f32" in counts), counts     # (ew_fused: r)
+    assert counts.get("gemm") == 1 and counts.get("ew_fused") == 1 and (M <= 64 <= N) == ("binary_f32" in counts), counts     # (ew_fused: r)
     for i in range(B):
         ref, bound = product_and_bound(x[i], w if B == 1 else w[i])
         ref = ref + r[i]
