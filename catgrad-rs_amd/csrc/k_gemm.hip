@@ -2917,6 +2917,16 @@ static int vec_ok(const void *base, int esize, int64_t other_stride, int64_t sb0
   const int64_t q = 16 / esize;
   return aligned16(base) && other_stride % q == 0 && sb0 % q == 0 && sb1 % q == 0;
 }
+// ... of a product's operands, for the launch and for every rule that has to know what it will launch.  (The stride of an axis of
+// length 1 is never used: it must not spoil the test.)
+static int a_vec_ok(const GemmDesc &g) {
+  const bool unit_k = g.sak == 1 || g.K == 1;
+  return vec_ok(g.a, g.a_stype == ST_BF16 ? 2 : 4, unit_k ? (g.M == 1 ? 0 : g.sam) : g.sak, g.sa_b0, g.sa_b1);
+}
+static int b_vec_ok(const GemmDesc &g) {
+  const bool unit_k = g.sbk == 1 || g.K == 1;
+  return vec_ok(g.b, g.b_stype == ST_BF16 ? 2 : 4, unit_k ? (g.N == 1 ? 0 : g.sbn) : g.sbk, g.b_index ? g.sb_index : g.sb_b0, g.sb_b1);
+}
 
 template <typename TA, typename TB, bool BF16>
 static void launch_gemm_layout(const LaunchCtx &lc, const GemmDesc &g, dim3 grid, int av, int bv) {
@@ -3006,9 +3016,7 @@ static bool gemm_narrow_dma_ok(const LaunchCtx &lc, const GemmDesc &g) {
 }
 
 bool gemm_epilogue_ok(const GemmDesc &g) {
-  const int asz = g.a_stype == ST_BF16 ? 2 : 4, bsz = g.b_stype == ST_BF16 ? 2 : 4;
-  const int av = vec_ok(g.a, asz, g.sak == 1 ? g.sam : g.sak, g.sa_b0, g.sa_b1);
-  const int bv = vec_ok(g.b, bsz, g.sbk == 1 ? g.sbn : g.sbk, g.sb_b0, g.sb_b1);
+  const int av = a_vec_ok(g), bv = b_vec_ok(g);
   return gemm_fast_path(g, av, bv) && gemm_dma_ok(g) && g.splits <= 1 && !g.b_index && !g.c_add &&
          (g.N % 4 == 0 || g.c16_pitch);
 }
@@ -3019,9 +3027,7 @@ bool gemm_epilogue_ok(const GemmDesc &g) {
 bool gemm_add_ok(const LaunchCtx &lc, const GemmDesc &g) {
   GemmDesc t = g;
   t.c_add = nullptr;
-  const int asz = g.a_stype == ST_BF16 ? 2 : 4, bsz = g.b_stype == ST_BF16 ? 2 : 4;
-  const int av = vec_ok(g.a, asz, g.sak == 1 ? g.sam : g.sak, g.sa_b0, g.sa_b1);
-  const int bv = vec_ok(g.b, bsz, g.sbk == 1 ? g.sbn : g.sbk, g.sb_b0, g.sb_b1);
+  const int av = a_vec_ok(g), bv = b_vec_ok(g);
   return g.splits <= 1 && !g.n_group && !g.dual_b && !g.glu_gate && !g.c16 && !g.act_sigmoid && !g.b_index && gemm_fast_path(t, av, bv) &&
          (gemm_dma_ok(t) ? g.M > 64 : gemm_narrow_dma_ok(lc, t));
 }
@@ -3032,10 +3038,8 @@ bool gemm_act_ok(const LaunchCtx &lc, const GemmDesc &g) {
   if (g.c16_pitch) return g.nb0 * g.nb1 == 1 && g.c16_pitch % 64 == 0 && g.c16_pitch >= g.N && gemm_epilogue_ok(g);
   if (gemv_rows_plain_ok(lc, g)) return false;
   if (g.splits > 1) return true;  // the pass that sums the slices applies it
-  const int asz = g.a_stype == ST_BF16 ? 2 : 4, bsz = g.b_stype == ST_BF16 ? 2 : 4;
-  const int av = vec_ok(g.a, asz, g.sak == 1 ? g.sam : g.sak, g.sa_b0, g.sa_b1);
-  const int bv = vec_ok(g.b, bsz, g.sbk == 1 ? g.sbn : g.sbk, g.sb_b0, g.sb_b1);
-  return !gemm_fast_path(g, av, bv) || gemm_epilogue_ok(g);
+  const int av = a_vec_ok(g), bv = b_vec_ok(g);
+  return !gemm_fast_path(g, av, bv) || gemm_epilogue_ok(g) || gemm_column_ok(g, av, bv);
 }
 
 // Copies of the operands in rows of a multiple of 64 bf16 values put a product of ragged sizes (K % 64, or rows that do
@@ -3052,9 +3056,7 @@ bool gemm_pack_wanted(const GemmDesc &g, bool epilogue) {
   if ((g.sak != 1 && g.sam != 1) || (g.sbk != 1 && g.sbn != 1)) return false;
   epilogue = epilogue && g.N >= 64;  // (fewer columns: not on the kernel that has one - 17 x 64 x 8 with a sigmoid 9.3 us, 12.6)
   GemmDesc t = g;  // (as it would run: f32 operands with unit strides along k are read from their bf16 twins)
-  const int asz = g.a_stype == ST_BF16 ? 2 : 4, bsz = g.b_stype == ST_BF16 ? 2 : 4;
-  const int av = vec_ok(g.a, asz, g.sak == 1 ? g.sam : g.sak, g.sa_b0, g.sa_b1);
-  const int bv = vec_ok(g.b, bsz, g.sbk == 1 ? g.sbn : g.sbk, g.sb_b0, g.sb_b1);
+  const int av = a_vec_ok(g), bv = b_vec_ok(g);
   t.a_stype = t.b_stype = ST_BF16;
   const bool as_it_lies = g.K % 64 == 0 && av && bv && g.sak == 1;
   if (as_it_lies && g.sbk == 1) return false;
@@ -3126,9 +3128,7 @@ static uint32_t gemm_small_split(const LaunchCtx &lc, const GemmDesc &g) {
 // The caller provides g.workspace of splits * batch * M * N floats and sets g.splits/k_per_split.
 uint32_t gemm_split_k(const LaunchCtx &lc, const GemmDesc &g) {
   const uint32_t batch = g.nb0 * g.nb1;
-  const int asz = g.a_stype == ST_BF16 ? 2 : 4, bsz = g.b_stype == ST_BF16 ? 2 : 4;
-  const int av = vec_ok(g.a, asz, g.sak == 1 ? g.sam : g.sak, g.sa_b0, g.sa_b1);
-  const int bv = vec_ok(g.b, bsz, g.sbk == 1 ? (g.N == 1 ? 0 : g.sbn) : g.sbk, g.sb_b0, g.sb_b1);
+  const int av = a_vec_ok(g), bv = b_vec_ok(g);
   const uint64_t tiles = (uint64_t)((g.M + 127) / 128) * ((g.N + 127) / 128) * batch;
   uint32_t splits = 1;
   if (gemv_rows_plain_ok(lc, g)) return 1;
@@ -3173,13 +3173,9 @@ hipError_t launch_matmul(const LaunchCtx &lc_in, const GemmDesc &g, const char *
     lc.ev_stop = nullptr;
     tail.ev_start = nullptr;
   }
-  const int asz = g.a_stype == ST_BF16 ? 2 : 4, bsz = g.b_stype == ST_BF16 ? 2 : 4;
   const bool a_unit_k = g.sak == 1 || g.K == 1, b_unit_k = g.sbk == 1 || g.K == 1;
   const bool b_unit_n = g.sbn == 1 || g.N == 1;
-  // the stride of an axis of length 1 is never used: it must not spoil the alignment test
-  const int av = vec_ok(g.a, asz, a_unit_k ? (g.M == 1 ? 0 : g.sam) : (g.K == 1 ? 0 : g.sak), g.sa_b0, g.sa_b1);
-  const int bv = vec_ok(g.b, bsz, b_unit_k ? (g.N == 1 ? 0 : g.sbn) : (g.K == 1 ? 0 : g.sbk),
-                        g.b_index ? g.sb_index : g.sb_b0, g.sb_b1);
+  const int av = a_vec_ok(g), bv = b_vec_ok(g);
   // only the one-row kernels follow b_index; they add c_add, and so do the k-slice sum of a split GEMM and gemm_add_ok's tiles
   const bool one_row = g.M <= 8 && g.a_stype == ST_F32 && g.K > 0 && (b_unit_k || b_unit_n);
   if (g.b_index && !one_row) return hipErrorInvalidValue;

@@ -8,6 +8,7 @@ BF16 = 1
 
 LAUNCHED = """
 import importlib
+lang, nn = cg.lang, cg.nn
 fake.fake_hip_launched.restype = ctypes.c_char_p
 
 def launched(f):
@@ -87,6 +88,27 @@ for b, m, k, column in ((1, 17, 72, 0), (1, 17, 160, 1), (1, 65, 72, 1), (1, 600
                         (1, 16384, 512, 1), (1, 70000, 1016, 0), (1, 70000, 1024, 1), (100, 66, 192, 0), (20, 66, 64, 1)):
     names = product(m, 1, k, batch=b)
     assert len(names) == 1 and ("gemm_bf16_column" if column else "gemm_bf16_nt_kernelILi64ELi64E") in names[0], (b, m, k, names)
+""", BF16)
+
+
+def test_one_column_and_a_sigmoid(fake_hip):  # noqa: F811
+    """In the column kernel's launch, and a launch of its own behind the tiles, which have none, from either order of the column."""
+    fake_hip(LAUNCHED + """
+class Sigmoid(lang.Module):
+    def __init__(self, along_k): self.along_k = along_k
+    def path(self): return lang.path(["sigmoid", str(self.along_k)])
+    def sort(self): return [lang.TENSOR] * 2, [lang.TENSOR]
+    def def_(self, b, args): return [nn.sigmoid(b, lang.matmul(b, args[0], lang.transpose(b, 0, 1, args[1]) if self.along_k else args[1]))]
+
+for m, k, column in ((17, 72, 0), (17, 160, 1), (65, 72, 1), (6001, 176, 0), (6001, 192, 1)):
+    for along_k in (True, False):
+        x, w = operand(m, k), operand(*((1, k) if along_k else (k, 1)))
+        be.sync()
+        fake.fake_hip_launched()
+        be.realize(cg.Interpreter(be, cg.stdlib(), cg.Parameters()).run(Sigmoid(along_k).term(), [x, w])[0])
+        be.sync()
+        names = [n for n in fake.fake_hip_launched().decode().split("\\n") if "gem" in n or "ew_" in n]
+        assert len(names) == 2 - column and ("gemm_bf16_column" if column else "gemm_bf16_nt_kernelILi64ELi64E") in names[0], (m, k, along_k, names)
 """, BF16)
 
 

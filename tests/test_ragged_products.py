@@ -60,6 +60,19 @@ def test_sigmoid_of_a_product(oracle, hip, hip_bf16, rows, inner, hidden, bf16):
     (parity.assert_bf16 if bf16 else parity.assert_f32)(ref, got, f"{rows}x{inner}x{hidden}")
 
 
+# both strides of a single column are 1 as it lies, and the kernels for few k or few rows of it have no sigmoid of their own
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,inner", [(9, 16), (64, 64), (65, 64), (100, 200), (6001, 184), (6001, 192), (20, 2048)])
+@pytest.mark.parametrize("batch", [1, 3])
+def test_sigmoid_of_one_column(oracle, hip_bf16, batch, rows, inner):
+    g = np.random.default_rng(rows)
+    x, w = draw(g, (batch, rows, inner), 1.0), draw(g, (batch, inner, 1), inner ** -0.5)
+    for f, right in ((sigmoid_of_product, w), (lambda b, x, w: [nn.sigmoid(b, lang.matmul(b, x, lang.transpose(b, 1, 2, w)))], w.reshape(batch, 1, inner))):
+        (ref,) = vectors.run(oracle, f, 1, x, right)
+        (got,) = vectors.run(hip_bf16, f, 1, x, right)
+        parity.assert_bf16(ref, got, f"{batch} x {rows} x {inner}")
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("batch,m,n,k", [(1, 700, 900, 801), (3, 260, 516, 1002), (2, 1001, 300, 904), (1, 515, 1030, 1024)])
 @pytest.mark.parametrize("turned", [True, False])
