@@ -196,7 +196,7 @@ __device__ __forceinline__ float block_reduce(float v, float *lds) {
 }
 
 // f32 -> bf16, round to nearest even, two values packed low / high by one instruction (v_cvt_pk_bf16_f32; a NaN keeps its
-// upper bits and becomes quiet.  The same bits as the integer form u + 0x7FFF + (u >> 16 & 1) over all 2^32 arguments,
+// upper bits and becomes quiet.  Otherwise the bits of the integer form u + 0x7FFF + (u >> 16 & 1), ties included,
 // which takes six instructions a value).
 typedef __attribute__((ext_vector_type(2))) __bf16 cvt_bf16x2;
 typedef __attribute__((ext_vector_type(2))) float cvt_f32x2;

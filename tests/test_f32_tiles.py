@@ -37,6 +37,38 @@ def test_product(hip, rows, B, M, N, K, along_k):
     assert_f32_sums(exact, got, K, f"{B} x {M} x {N} x {K}")
 
 
+def with_infinities(x, w):
+    """x [.., M, K] and w [.., N, K] with an infinity in row 3, a NaN in the last row and, of several columns, an infinity in the
+    last: at the first and the last k, next to what a tile holds past either edge."""
+    x, w = x.copy(), w.copy()
+    x[..., 3, 0], x[..., -1, -1] = np.inf, np.nan
+    if w.shape[-2] > 1:
+        w[..., -1, -1] = -np.inf
+    return x, w
+
+
+def assert_infinities(x, w, got):
+    """Infinities and NaN where x w^T has them, nowhere else; K f32 additions of rounded products off in the rest."""
+    x, w = x.astype(np.float64), np.swapaxes(w, -1, -2).astype(np.float64)
+    with np.errstate(invalid="ignore"):
+        ref = np.matmul(x, w)
+    finite = np.isfinite(ref)
+    assert np.array_equal(ref[~finite], got[~finite], equal_nan=True)
+    bound = (x.shape[-1] + 1) * 2.0 ** -24 * np.matmul(*(np.abs(np.where(np.isfinite(a), a, 0)) for a in (x, w)))
+    assert np.all(np.abs(got[finite] - ref[finite]) <= bound[finite])      # (a NaN is no less than its bound)
+
+
+# every height of tile, k in one piece and in slices, a last step of one piece
+@pytest.mark.gpu
+@pytest.mark.parametrize("along_k", [True, False])
+@pytest.mark.parametrize("rows,B,M,N,K", [s for s in SIZES if s[2] * s[3] < 5e6])
+def test_infinities(hip, rows, B, M, N, K, along_k):
+    g = np.random.default_rng(M + K)
+    x, w = with_infinities(*(g.standard_normal(s).astype(np.float32) for s in (((B, M, K), (B, N, K)) if B > 1 else ((M, K), (N, K)))))
+    (got,) = vectors.run(hip, product(x.ndim, along_k), 1, x, w if along_k else np.ascontiguousarray(np.swapaxes(w, -1, -2)))
+    assert_infinities(x, w, got)
+
+
 # one launch and slices whose sum applies it; the error of a sigmoid is at most a quarter of its argument's, and its own rounding
 @pytest.mark.gpu
 @pytest.mark.parametrize("M,N,K", [(1000, 1000, 1000), (300, 1000, 2060)])

@@ -9,6 +9,7 @@ import parity
 import test_llama_parity as llama_tests
 import test_moe_gemma_parity as moe_tests
 import vectors
+from test_f32_tiles import assert_infinities, with_infinities
 
 lang, nn = vectors.cg.lang, vectors.cg.nn
 
@@ -54,6 +55,17 @@ def test_product(hip_bf16, M, N, K):
                                    (65, 33, 384), (65, 33, 448), (513, 61, 320), (8192, 60, 448), (8193, 60, 512), (1023, 63, 4096), (3072, 60, 4096)])
 def test_narrow_product(hip_bf16, M, N, K):
     test_product(hip_bf16, M, N, K)
+
+
+# 256 x 256 on four and eight wavefronts, 192 x 128 and 128 x 128 on four, their quarters, a wave to a row, 32 x 32, copied operands
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(3841, 3843, 576), (4090, 4093, 192), (2303, 2049, 640), (1400, 1410, 1088), (300, 300, 256),
+                                   (1030, 1, 2048), (129, 63, 1088), (900, 1100, 1000)])
+def test_infinities(hip_bf16, M, N, K):
+    g = np.random.default_rng(M)
+    x, w = with_infinities(draw(g, (M, K)), draw(g, (N, K)))
+    (got,) = vectors.run(hip_bf16, lambda b, x, w: [linear(b, x, w, N, K)], 1, x[None], w)
+    assert_infinities(x, w, got[0])
 
 
 # a residual added as the product is stored: each tile that does so, whole rounds of large tiles with the rest on smaller ones
@@ -112,9 +124,11 @@ def test_gated(hip_bf16, M, F, K, act):
     gate, up = (x[0].astype(np.float64) @ w[F - 64:].astype(np.float64).T for w in (wg, wu))
     c = gate if act == "silu" else 2 * np.sqrt(2 / np.pi) * (gate + 0.044715 * gate ** 3)
     ref = gate / (1 + np.exp(-c)) * up
-    # rounded once to bf16, whose eight significant bits leave half a unit in the last place: 2^-8 of the value at most; the f32
-    # sums of K <= 320 products of rms K^-1/2 in front of it are good to 1e-5
-    assert np.all(np.abs(got[0] - ref) <= 2.0 ** -8 * np.abs(ref) + 1e-5)
+    # rounded once to bf16, whose eight significant bits leave half a unit in the last place: 2^-8 of the value at most, and 2^-19 for
+    # the hardware's exp2 and reciprocal; the f32 sums in front of it, of K terms of size K^-1/2, are off by 4 sqrt(K) 2^-24 at most
+    # (as in assert_f32_sums), and no slope of an activation is above 1.13
+    sums = 4 * np.sqrt(K) * 2.0 ** -24 * (1.13 * np.abs(up) + np.abs(gate))
+    assert np.all(np.abs(got[0] - ref) <= (2.0 ** -8 + 2.0 ** -19) * np.abs(ref) + sums)
 
 
 @pytest.mark.gpu

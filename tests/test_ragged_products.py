@@ -97,3 +97,16 @@ def test_one_round_of_tall_tiles(oracle, hip_bf16, rows, n, k):
     (ref,) = vectors.run(oracle, f, 1, x, w)
     (got,) = vectors.run(hip_bf16, f, 1, x, w)
     parity.assert_bf16(ref, got, f"{rows}x{n}x{k}")
+
+
+# f32 rows rounded to bf16 on their way into a product: every upper half of a finite normal number, with lower halves around a tie, a
+# row to each sign and exponent; a product with the unit matrix returns what they became
+@pytest.mark.gpu
+@pytest.mark.parametrize("lower", [0x0000, 0x0001, 0x7FFF, 0x8000, 0x8001, 0xFFFF])
+def test_rounding_of_rows(hip_bf16, lower):
+    upper = np.arange(1 << 16, dtype=np.uint32).reshape(-1, 128)
+    upper = upper[((upper[:, 0] >> 7 & 255) > 0) & ((upper[:, 0] >> 7 & 255) < 254)]
+    x = (upper << 16 | lower).view(np.float32)
+    rows = x.shape[0]
+    (got,) = vectors.run(hip_bf16, lambda b, x, w: [lang.matmul(b, lang.reshape(b, lang.make_shape(b, rows, 128), x), w)], 1, x.ravel(), np.eye(128, dtype=np.float32))
+    assert np.array_equal(got, vectors.bf16_round(x))
