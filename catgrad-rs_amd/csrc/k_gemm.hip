@@ -3310,7 +3310,12 @@ hipError_t launch_matmul(const LaunchCtx &lc_in, const GemmDesc &g, const char *
         if (r256 * 5 <= r128 * 3 && gemm_ring_ok(gg)) e = launch_gemm_ring(lc, gg);
         else if (d128 * 4 <= cus)
           e = launch_gemm_dma<128, 64, 4, 1, true, 5, true, false, false, 2>(lc, gg, (uint32_t)((uint64_t)((g.M + 127) / 128) * ((g.N + 31) / 32) * batch));
-        else if (d128 * 2 <= cus || g.K < 192 || !gemm_ring_ok(gg))
+        // One or two k-steps: what a tile stores is most of it, and eight wavefronts store it as they come.  One step, on tiles of 64
+        // output columns and on these: 6920 rows by 2 x 7648 93 and 60 us, 1416 by 2 x 8200 25.5 and 19.3, 3657 by 2 x 792 10.0
+        // and 8.0, 4589 by 2 x 1176 14.5 both; two, 5099 by 2 x 2112 27.6 and 22.1, 1114 by 2 x 2416 10.6 and 8.9.
+        else if (g.K < 192 && d256 >= cus) e = launch_gemm_dma<256, 256, 2, 4, true, 2, true>(lc, gg, (uint32_t)d256);
+        else if (g.K < 192 && d128 * 2 > cus) e = launch_gemm_dma<128, 256, 2, 4, true, 3, true>(lc, gg, (uint32_t)d128);
+        else if (d128 * 2 <= cus || !gemm_ring_ok(gg))
           e = launch_gemm_dma<128, 128, 4, 2, true, 4, true>(lc, gg, (uint32_t)((uint64_t)((g.M + 127) / 128) * ((g.N + 63) / 64) * batch));
         else e = launch_gemm_ring(lc, gg, true);
       } else if (g.glu_gate || g.c16 || (g.act_sigmoid && splits == 1)) {

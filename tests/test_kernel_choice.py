@@ -70,6 +70,32 @@ for m, n, k, waves in ((2305, 2049, 64, 8), (6000, 700, 256, 8), (2303, 2049, 57
 """, BF16)
 
 
+def test_gated_products(fake_hip):  # noqa: F811
+    """gate and up stacked: one and two k-steps on eight wavefronts unless whole rounds of 256 rows are ahead, four wavefronts beyond."""
+    fake_hip(LAUNCHED + """
+class Gated(lang.Module):
+    def __init__(self, m, f, k): self.m, self.f, self.k = m, f, k
+    def path(self): return lang.path(["gated", "%d" % self.m, "%d" % self.f, "%d" % self.k])
+    def sort(self): return [lang.TENSOR] * 4, [lang.TENSOR]
+    def def_(self, b, args):
+        def linear(x, w, n, k): return lang.matmul(b, x, lang.reshape(b, lang.make_shape(b, 1, k, n), lang.transpose(b, 0, 1, w)))
+        x, g, u, d = args
+        return [linear(nn.silu(b, linear(x, g, self.f, self.k)) * linear(x, u, self.f, self.k), d, 64, self.f)]
+
+wide, tall, four, four128 = ("gemm_bf16_dma_kernelILi128ELi256ELi2ELi4ELb1ELi3ELb1E", "gemm_bf16_dma_kernelILi256ELi256ELi2ELi4ELb1ELi2ELb1E",
+                             "gemm_bf16_ring_kernelILi2ELi2E", "gemm_bf16_ring_kernelILi2ELi1E")
+for m, f, k, kernel in ((4100, 2056, 64, tall), (4200, 2600, 128, tall), (4100, 1256, 128, four), (4200, 2600, 192, four128),
+                        (1000, 3000, 64, wide), (1030, 2184, 128, wide), (1030, 2184, 192, four128)):
+    xs = [operand(1, m, k), operand(f, k), operand(f, k), operand(64, f)]
+    be.sync()
+    fake.fake_hip_launched()
+    be.realize(cg.Interpreter(be, cg.stdlib(), cg.Parameters()).run(Gated(m, f, k).term(), xs)[0])
+    be.sync()
+    names = [n for n in fake.fake_hip_launched().decode().split("\\n") if "gem" in n]
+    assert kernel in names[0], (m, f, k, names)
+""", BF16)
+
+
 def test_less_than_a_round(fake_hip):  # noqa: F811
     """A quarter of a 128 x 128 tile from four k-steps on, half of one below or where the quarters are more than the CUs."""
     fake_hip(LAUNCHED + """

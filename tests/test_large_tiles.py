@@ -112,7 +112,8 @@ def test_grouped_products(hip_bf16, M, K, bias):
 @pytest.mark.gpu
 @pytest.mark.parametrize("act", ["silu", "gelu"])
 @pytest.mark.parametrize("M,F,K", [(4096, 2048, 128), (4100, 2052, 192), (3900, 2184, 320),    # tiles of 256 rows
-                                   (1030, 2180, 192), (900, 3000, 256), (1000, 2820, 512)])    # and of 128: three steps, four, more
+                                   (1030, 2180, 192), (900, 3000, 256), (1000, 2820, 512),     # and of 128: three steps, four, more
+                                   (4100, 2056, 64), (4200, 2600, 128), (4100, 1256, 128), (1000, 3000, 64), (1030, 2184, 128)])    # one and two, on eight wavefronts or four
 def test_gated(hip_bf16, M, F, K, act):
     g = np.random.default_rng(F)
     x, wg, wu, wd = draw(g, (1, M, K)), draw(g, (F, K), K ** -0.5), draw(g, (F, K), K ** -0.5), np.eye(64, F, dtype=np.float32)
