@@ -111,9 +111,10 @@ def test_grouped_products(hip_bf16, M, K, bias):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("act", ["silu", "gelu"])
-@pytest.mark.parametrize("M,F,K", [(4096, 2048, 128), (4100, 2052, 192), (3900, 2184, 320),    # tiles of 256 rows
-                                   (1030, 2180, 192), (900, 3000, 256), (1000, 2820, 512),     # and of 128: three steps, four, more
-                                   (4100, 2056, 64), (4200, 2600, 128), (4100, 1256, 128), (1000, 3000, 64), (1030, 2184, 128)])    # one and two, on eight wavefronts or four
+@pytest.mark.parametrize("M,F,K", [(4096, 2048, 128), (4100, 2056, 192), (3900, 2184, 320),    # tiles of 256 rows
+                                   (1030, 2184, 192), (900, 3000, 256), (1000, 2824, 512),     # and of 128: three steps, four, more
+                                   (4100, 2056, 64), (4200, 2600, 128), (4100, 1256, 128), (1000, 3000, 64), (1030, 2184, 128),    # one and two, on eight wavefronts or four
+                                   (4100, 2052, 192), (1030, 2180, 192), (1000, 2820, 512)])   # two products: rows of results off 16 bytes
 def test_gated(hip_bf16, M, F, K, act):
     g = np.random.default_rng(F)
     x, wg, wu, wd = draw(g, (1, M, K)), draw(g, (F, K), K ** -0.5), draw(g, (F, K), K ** -0.5), np.eye(64, F, dtype=np.float32)
@@ -121,7 +122,10 @@ def test_gated(hip_bf16, M, F, K, act):
     def f(b, x, wg, wu, wd):    # (wd picks the first 64 gated values out: exact products)
         x = x + x - x
         return [linear(b, getattr(nn, act)(b, linear(b, x, wg, F, K)) * linear(b, x, wu, F, K), wd, 64, F)]
+    hip_bf16.launch_counts(reset=True)
     (got,) = vectors.run(hip_bf16, f, 1, x, wg, wu, np.roll(wd, F - 64, axis=1))
+    counts = hip_bf16.launch_counts(reset=True)
+    assert counts.get("gemm") == (3 if F % 8 else 2), counts
     gate, up = (x[0].astype(np.float64) @ w[F - 64:].astype(np.float64).T for w in (wg, wu))
     c = gate if act == "silu" else 2 * np.sqrt(2 / np.pi) * (gate + 0.044715 * gate ** 3)
     ref = gate / (1 + np.exp(-c)) * up
