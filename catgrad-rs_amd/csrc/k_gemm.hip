@@ -362,6 +362,11 @@ static bool gemm_f32_tiles(const LaunchCtx &lc, const GemmDesc &g, uint32_t *spl
     const uint32_t s = gemm_small_split(lc, g);
     const uint64_t wgs = (uint64_t)((g.M + 31) / 32) * ((g.N + 31) / 32) * g.nb0 * g.nb1 * s;
     small_us = 3.0 + 0.0135 * g.K / s * (wgs > (uint64_t)lc.n_cus ? 1.5 : 1.0) + (s > 1 ? 3.0 : 0.0);
+    // Up to 32 columns and a workgroup to every other CU or more, but none with two: the kernel above needs two slices at most there,
+    // and these tiles, three quarters of them empty, take 9 to 16, at 8 to 15 % more than they are priced at (4455 x 18 x 2700 37.6 us
+    // above, 41.3 here; 4839 x 21 x 2408 35.1, 40.1; 5 x 469 x 20 x 3576 29.1, 32.5; level at best: 4340 x 10 x 2864 37.5, 37.4; with
+    // four, 3 x 326 x 17 x 7488 34.0, 32.6).
+    if (g.N <= 32 && s <= 2 && 2 * wgs > (uint64_t)lc.n_cus && wgs <= (uint64_t)lc.n_cus) return false;
     // (gemm_f32_split looks at up to 128 forms: not where none can be ahead)
     if (small_us <= gemm_f32_least_us(g)) return false;
   } else if (!splits) {

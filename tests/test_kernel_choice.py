@@ -160,9 +160,12 @@ for rows, b, m, n, k in {SIZES}:
     for along_k in (True, False):
         names = product(m, n, k, along_k, b)
         assert len(names) == 1 and "gemm_f32_dma_kernelILi%dE" % rows in names[0] and names[0].split("ELb")[1][0] == "10"[along_k], (b, m, n, k, along_k, names)
-for b, m, n, k in ((1, 64, 256, 128), (1, 33, 132, 1044), (3, 70, 260, 100), (1, 10, 512, 2048), (1, 2000, 20, 2000)):
+for b, m, n, k in ((1, 64, 256, 128), (1, 33, 132, 1044), (3, 70, 260, 100), (1, 10, 512, 2048), (1, 2000, 20, 2000), (1, 4455, 18, 2700), (1, 4191, 23, 2860), (3, 1355, 11, 2792), (5, 469, 20, 3576)):
     names = product(m, n, k, batch=b)
     assert len(names) == 1 and "gemm_small_f32_kernel" in names[0], (b, m, n, k, names)
+for b, m, n, k in ((1, 4129, 24, 3200), (1, 4129, 40, 3200), (3, 326, 17, 7488)):     # (deeper, of more columns, of four slices)
+    names = product(m, n, k, batch=b)
+    assert len(names) == 1 and "gemm_f32_dma_kernel" in names[0], (b, m, n, k, names)
 """)
 
 
