@@ -3406,7 +3406,7 @@ hipError_t launch_matmul(const LaunchCtx &lc_in, const GemmDesc &g, const char *
           if (steps >= 24) e = launch_gemm_plain<128, 128, 2, 2, 5, 1, true>(lc, gg, t128);
           else e = launch_gemm_plain<128, 128, 2, 4, 4>(lc, gg, t128);
         } else if (t192 <= cus) {
-          // a round of 192 rows (o_proj and down_proj of 2900 rows: 29 and 91 us; 368 tiles of 128 rows two to a CU 35 and 122; 1024
+          // a round of 192 rows (o_proj and down_proj of 2900 rows: 29 and 91 us, 33 and 94 with the residual added as they store; 368 tiles of 128 rows two to a CU 35 and 122; 1024
           // deep 19.7, 21.6).  Up to nine k-steps eight wavefronts, whose start and tail are shorter (2900 x 2048: K = 64 8.4 us - four
           // wavefronts take three steps at least, 128 rows two to a CU 8.8 -, 256 11.1 and 12.3, 512 14.5 and 14.8, 768 18.3 and 17.7;
           // 6000 x 700 x 256 10.4, 11.7).
