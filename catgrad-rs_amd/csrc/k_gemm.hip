@@ -3276,6 +3276,18 @@ hipError_t launch_matmul(const LaunchCtx &lc_in, const GemmDesc &g, const char *
       if (g.n_group && (batch != 1 || splits != 1 || g.glu_gate || g.c16)) return hipErrorInvalidValue;
       const uint64_t t128 = (uint64_t)((g.M + 127) / 128) * ((g.N + 127) / 128) * batch * splits;
       const bool deep = t128 < 2 * (uint64_t)lc.n_cus;  // at most one workgroup per CU at a time: four stages
+      // Tiles of 256 x 288 (stacked: 144 output columns), at 9/8 of the time of 256 x 256, where they need fewer rounds by more than
+      // that.  K = 6912, 16384 x 1152 (one round; whole rounds of 256 x 256 and the rest on smaller tiles) 274 -> 229 us; K = 1024 50.7
+      // -> 40.9, 512 32.6 -> 28.7, 256 23.4 -> 22.2, 128 19.1, 19.2; 8192 x 2304 x 4096 146 -> 122, 4096 x 4608 x 2048 81 -> 68, 15000
+      // x 1100 x 2048 82 -> 66, 64 x 256 x 1152 x 1024 54 -> 43; two rounds for three, 16384 x 2304 x 1152 105 -> 85; three for four,
+      // 16384 x 3456 x 1152 147 -> 132, x 512 87 -> 75; stacked, twelve for fourteen, 16384 x 2 x 6912, K = 1152, 452 -> 442, one for
+      // two or for three of 128 rows (with a small product of 11 us behind them) 4096 x 2 x 2304 x 1152 67 -> 54, x 2048 97 -> 77.  An
+      // equal number of rounds: 8192 x 1152 x 6912 149, and 144 on 256 x 256.
+      auto rounds_of = [&](uint64_t tiles) { return (tiles + lc.n_cus - 1) / lc.n_cus; };
+      auto wide_ahead = [&](uint64_t columns, uint64_t tiles) {  // (`columns` to a wide tile; `tiles` of 256 x 256, or stacked, otherwise)
+        const uint64_t wide = (uint64_t)((g.M + 255) / 256) * ((g.N + columns - 1) / columns) * batch;
+        return splits == 1 && g.K >= 256 && g.N % 4 == 0 && !g.n_group && !g.act_sigmoid && rounds_of(wide) * 9 < rounds_of(tiles) * 8;
+      };
       if (g.rope_s && g.M <= 128) {
         // q / k / v of a few rows: a workgroup takes in its rows of both operands at about 42 GB/s however wide its tile is,
         // and 64 x 64 or 128 x 64 tiles are 48 workgroups for 3072 columns.  32 x 32 tiles, of columns that rotate into
@@ -3311,8 +3323,11 @@ hipError_t launch_matmul(const LaunchCtx &lc_in, const GemmDesc &g, const char *
         // by 2 x 8192, K = 2048, one round either way 56 and 40 us; 700 rows, one round or two, 50 and 60; 1024 rows by 2 x 5632 47 and
         // 60; 1500 rows, two or three, 92 and 84; 2900 by 2 x 8192, three or six, 159 and 181).  Fewer tiles of 128 than half the
         // CUs: 64 or 32 output columns per tile.
+        const uint64_t d256w = (uint64_t)((g.M + 255) / 256) * ((g.N + 143) / 144) * batch;
         const uint64_t cus = (uint64_t)lc.n_cus, r256 = (d256 + cus - 1) / cus, r128 = (d128 + cus - 1) / cus;
-        if (r256 * 5 <= r128 * 3 && gemm_ring_ok(gg)) e = launch_gemm_ring(lc, gg);
+        const bool wide = wide_ahead(144, d256);
+        const uint64_t large = wide ? (d256w + cus - 1) / cus * 9 : r256 * 8;  // (in eighths of a round of 256 rows)
+        if (large * 5 <= r128 * 24 && gemm_ring_ok(gg)) e = launch_gemm_ring(lc, gg, false, wide);
         else if (d128 * 4 <= cus)
           e = launch_gemm_dma<128, 64, 4, 1, true, 5, true, false, false, 2>(lc, gg, (uint32_t)((uint64_t)((g.M + 127) / 128) * ((g.N + 31) / 32) * batch));
         // One or two k-steps: what a tile stores is most of it, and eight wavefronts store it as they come.  One step, on tiles of 64
@@ -3337,9 +3352,10 @@ hipError_t launch_matmul(const LaunchCtx &lc_in, const GemmDesc &g, const char *
         // their own with the tiling that suits them (347 -> 307 us; with K = 1024 the second launch costs what
         // the idle CUs did)
         const uint64_t tiles_n = (g.N + 255) / 256, tiles_m = (g.M + 255) / 256;
+        const bool wide = wide_ahead(288, t256);
         uint64_t lead_m = t256 / (uint64_t)lc.n_cus * (uint64_t)lc.n_cus / tiles_n;  // tile rows of the whole rounds
         if (g.c_add && lead_m && g.M - std::min<uint64_t>(g.M, lead_m * 256) <= 64) --lead_m;  // (up to 64 rows would not add c_add)
-        if (!g.n_group && batch == 1 && splits == 1 && g.K >= 2048 && fill(t256, (uint64_t)lc.n_cus) < 0.8 && lead_m >= 1 &&
+        if (!wide && !g.n_group && batch == 1 && splits == 1 && g.K >= 2048 && fill(t256, (uint64_t)lc.n_cus) < 0.8 && lead_m >= 1 &&
             lead_m < tiles_m && g.a_stype == ST_BF16) {
           GemmDesc lead = gg, rest = g;
           lead.M = (uint32_t)(lead_m * 256);
@@ -3354,7 +3370,8 @@ hipError_t launch_matmul(const LaunchCtx &lc_in, const GemmDesc &g, const char *
           if (e != hipSuccess) return e;
           return launch_matmul(second, rest, nullptr);
         }
-        if (!g.n_group && fill(t128, 2 * (uint64_t)lc.n_cus) > 1.15 * fill(t256, (uint64_t)lc.n_cus))
+        if (wide) e = launch_gemm_ring(lc, gg, false, true);
+        else if (!g.n_group && fill(t128, 2 * (uint64_t)lc.n_cus) > 1.15 * fill(t256, (uint64_t)lc.n_cus))
           e = g.K < 2048 ? launch_gemm_plain<128, 128, 2, 4>(lc, gg, t128)  // (as below)
                          : launch_gemm_plain<128, 128, 2, 2>(lc, gg, t128);
         else if ((g.K < 384 || (g.K <= 512 && batch == 1 && tiles_m > tiles_n && t256 >= 2 * (uint64_t)lc.n_cus)) && !g.n_group && !g.c_add)
@@ -3399,6 +3416,13 @@ hipError_t launch_matmul(const LaunchCtx &lc_in, const GemmDesc &g, const char *
           const uint64_t t64 = (uint64_t)((g.M + 63) / 64) * ((g.N + 63) / 64) * batch;
           e = t64 <= cus && g.K >= 256 ? launch_gemm_plain<64, 64, 2, 2, 8, 2>(lc, gg, t64)
                          : launch_gemm_plain<128, 64, 4, 2, 4>(lc, gg, (uint64_t)((g.M + 127) / 128) * ((g.N + 63) / 64) * batch);
+        } else if (splits == 1 && steps >= 12 && grp256 && t256 <= cus && t128 > 2 * cus && gemm_ring_ok(gg)) {
+          // Less than a round of 256 x 256, but two of 128 x 128 two to a CU (us here and there; the deepest against 128 or 192 rows one
+          // to a CU, below): 3000 x 3000 (144 tiles), K = 256 16.4, 15.6, 512 20.3, 20.7, 1024 29.1, 32.1, 2048 46.8, 57.7, 4096 82.3, 84.8,
+          // 8192 156, 157; 2048 x 6144 (192) 17.0, 16.2; 21.8, 22.2; 31.8, 34.7; 51.1, 61.9; 89.6, 105; 167, 200; 10000 x 1152 (200)
+          // 17.4, 15.7; 21.8, 21.7; 31.5, 34.1; 51.0, 61.3; 89.4, 92.7; 172, 172.  (One round of 128 x 128 two to a CU: 3500 x 2048 x 2048
+          // 44.9, 38.2.)
+          e = launch_gemm_ring(lc, gg);
         } else if (t128 <= cus) {
           // A round of 128 rows.  The four wavefronts' longer start and tail pay from about 24 k-steps on (weights from memory: 900 x
           // 2048 x 8192 in two slices 44.4 -> 37.4 us, 700 40.9 -> 36.3, 300 in four 23.2 -> 21.7, 400 x 1152 x 6912 in four - 27 steps -

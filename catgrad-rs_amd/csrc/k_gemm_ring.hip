@@ -254,15 +254,97 @@ static hipError_t whole_lds(const void *kernel, int bytes) {
   "2:\n\t" HPHASE0(HOFF, 24) HPHASE1(HOFF, 16) HNEXT_PLACES HPHASE0(HOFF, 12) HPHASE1(HOFF, 4) HNEXT_PLACES HPHASE0(HOFF, 0)    \
   HLAST "s_nop 15\n\ts_nop 7\n\t"
 
+// ---- tiles of 256 x 288: the four quadrants and a strip X of 32 columns more, a ninth of the products with no wavefront idle: in each
+// half of A a wavefront multiplies its first row block - rows wn * 32 of its 64, so that the two wavefronts of the same rows share
+// them - by the strip, in the phases (0,1) and (1,1).  The strip's fragments are read in the first phase of a step and requested in the
+// third; a stage's strip lies behind the two stages.  Rows of A are therefore read from two places a slice: rc is the other row block.
+// A step reads 144 KB of fragments and takes in 68 KB for 72 products (128 and 64 for 64).  Bound by power like 256 x 256: 16384 x 1152 x
+// 6912, one round, 229 us with the matrix cores busy 89 % of the time at the 1235 MHz that are left (256 x 256 in whole rounds, and the
+// rest on smaller tiles, 274).
+#define FR_X_0 "v[112:115]"
+#define FR_X_1 "v[116:119]"
+#define FR_X_2 "v[120:123]"
+#define FR_X_3 "v[124:127]"
+#define WRD(U, at, ks) "ds_read_b128 " FR_##U##_0_##ks ", %[ra" #ks "] offset:" at "\n\tds_read_b128 " FR_##U##_1_##ks ", %[rc" #ks "] offset:" at "\n\t"
+#define WRD0(U, at, ks) "ds_read_b128 " FR_##U##_0_##ks ", %[ra" #ks "] offset:" at "\n\t"
+#define WRD1(U, at, ks) "ds_read_b128 " FR_##U##_1_##ks ", %[rc" #ks "] offset:" at "\n\t"
+#define WRDX(ks) "ds_read_b128 " FR_X_##ks ", %[rx" #ks "]\n\t"
+#define WSTRIP(a, UA, ks) "v_mfma_f32_32x32x16_bf16 %[x" #a "], " FR_X_##ks ", " FR_##UA##_0_##ks ", %[x" #a "]\n\t"
+#define WLOADX "global_load_lds_dwordx4 %[dX], s[50:51]\n\t"
+#define WOTHER_STAGE_A OTHER_STAGE_A                                           \
+  "v_xor_b32 %[rc0], 0x10000, %[rc0]\n\tv_xor_b32 %[rc1], 0x10000, %[rc1]\n\t" \
+  "v_xor_b32 %[rc2], 0x10000, %[rc2]\n\tv_xor_b32 %[rc3], 0x10000, %[rc3]\n\t"
+#define WOTHER_STAGE_X                                                       \
+  "v_xor_b32 %[rx0], 0x1000, %[rx0]\n\tv_xor_b32 %[rx1], 0x1000, %[rx1]\n\t" \
+  "v_xor_b32 %[rx2], 0x1000, %[rx2]\n\tv_xor_b32 %[rx3], 0x1000, %[rx3]\n\t"
+#define WNEXT_STEP NEXT_STEP "s_add_u32 s50, s50, 128\n\ts_addc_u32 s51, s51, 0\n\t"
+#define WOTHER_STAGE_LOADS OTHER_STAGE_LOADS "s_xor_b32 s48, s48, 0x1000\n\t"
+#define WPOINTERS POINTERS "s_mov_b64 s[50:51], %[px]\n\ts_mov_b32 s48, %[ldsx]\n\t"
+#define WSYNC(v, r) "s_waitcnt vmcnt(" #v ") lgkmcnt(" #r ")\n\ts_barrier\n\t"
+#define ON_X(x) x
+#define OFF_X(x) ""
+#define WPHASE0(G, v)                                                                                                    \
+  WSYNC(v, 8)                                                                                                            \
+  SLICE(0, 0, A0, B0, 0, READS_BUT(6), RD(B1, 0, 0), G##_M(A0, 0), RD(B1, 1, 0) WRDX(0), G##_L(A0, 0))                   \
+  SLICE(0, 0, A0, B0, 1, READS_BUT(7), RD(B1, 0, 1), G##_M(A0, 1), RD(B1, 1, 1) WRDX(1), G##_L(A0, 1))                   \
+  SLICE(0, 0, A0, B0, 2, READS_BUT(8), RD(B1, 0, 2), G##_M(A0, 2), RD(B1, 1, 2) WRDX(2), G##_L(A0, 2))                   \
+  SLICE(0, 0, A0, B0, 3, READS_BUT(9), RD(B1, 0, 3), G##_M(A0, 3), RD(B1, 1, 3) WRDX(3), G##_L(A0, 3))
+#define WPHASE1(G, v)                                                                                                                    \
+  WSYNC(v, 12)                                                                                                                           \
+  SLICE(0, 1, A0, B1, 0, READS_BUT(9), WRD0(A1, AT_A1_0, 0), G##_M(B0, 0), WRD1(A1, AT_A1_0, 0), G##_L(B0, 0)) WSTRIP(0, A0, 0)          \
+  SLICE(0, 1, A0, B1, 1, READS_BUT(8), WRD0(A1, AT_A1_0, 1), G##_M(B0, 1), WRD1(A1, AT_A1_0, 1), G##_L(B0, 1)) WSTRIP(0, A0, 1)          \
+  SLICE(0, 1, A0, B1, 2, READS_BUT(7), WRD0(A1, AT_A1_0, 2), G##_M(B0, 2), WRD1(A1, AT_A1_0, 2) OTHER_STAGE_B, G##_L(B0, 2))             \
+  WSTRIP(0, A0, 2) WOTHER_STAGE_X                                                                                                        \
+  SLICE(0, 1, A0, B1, 3, READS_BUT(6), WRD0(A1, AT_A1_0, 3), G##_M(B0, 3), WRD1(A1, AT_A1_0, 3) WOTHER_STAGE_A, G##_L(B0, 3))            \
+  WSTRIP(0, A0, 3)
+#define WPHASE2(G, v)                                                                                                                    \
+  WSYNC(v, 8)                                                                                                                            \
+  SLICE(1, 1, A1, B1, 0, READS_BUT(6), WRD0(A0, AT_A0_0, 0), G##_M(B1, 0), WRD1(A0, AT_A0_0, 0), G##_L(B1, 0)) WSTRIP(1, A1, 0)          \
+  SLICE(1, 1, A1, B1, 1, READS_BUT(6), WRD0(A0, AT_A0_0, 1), G##_M(B1, 1), WRD1(A0, AT_A0_0, 1), G##_L(B1, 1)) WSTRIP(1, A1, 1)          \
+  SLICE(1, 1, A1, B1, 2, READS_BUT(6), WRD0(A0, AT_A0_0, 2), G##_M(B1, 2), WRD1(A0, AT_A0_0, 2), G##_L(B1, 2)) WSTRIP(1, A1, 2)          \
+  SLICE(1, 1, A1, B1, 3, READS_BUT(6), WRD0(A0, AT_A0_0, 3), G##_M(B1, 3), WRD1(A0, AT_A0_0, 3), G##_L(B1, 3))                           \
+  G##_X("s_mov_b32 m0, s48\n\t") WSTRIP(1, A1, 3) G##_X(WLOADX)
+#define WPHASE3(G, v)                                                                                 \
+  WSYNC(v, 8)                                                                                         \
+  SLICE(1, 0, A1, B0, 0, NONE, NONE, G##_M(A1, 0), NONE, G##_L(A1, 0))                                \
+  SLICE(1, 0, A1, B0, 1, NONE, RD(B0, 0, 0), G##_M(A1, 1), RD(B0, 1, 0), G##_L(A1, 1))                \
+  SLICE(1, 0, A1, B0, 2, NONE, RD(B0, 0, 1), G##_M(A1, 2), RD(B0, 1, 1), G##_L(A1, 2))                \
+  SLICE(1, 0, A1, B0, 3, NONE, RD(B0, 0, 2), G##_M(A1, 3), RD(B0, 1, 2), G##_L(A1, 3)) RD(B0, 0, 3)   \
+  RD(B0, 1, 3)
+#define WLAST_HALF                                                                            \
+  SLICE(1, 1, A1, B1, 0, READS_BUT(6), NONE, NONE, NONE, NONE) WSTRIP(1, A1, 0)               \
+  SLICE(1, 1, A1, B1, 1, READS_BUT(4), NONE, NONE, NONE, NONE) WSTRIP(1, A1, 1)               \
+  SLICE(1, 1, A1, B1, 2, READS_BUT(2), NONE, NONE, NONE, NONE) WSTRIP(1, A1, 2)               \
+  SLICE(1, 1, A1, B1, 3, READS_BUT(0), NONE, NONE, NONE, NONE) WSTRIP(1, A1, 3)               \
+  SLICE(1, 0, A1, B0, 0, NONE, NONE, NONE, NONE, NONE)                                        \
+  SLICE(1, 0, A1, B0, 1, NONE, NONE, NONE, NONE, NONE)                                        \
+  SLICE(1, 0, A1, B0, 2, NONE, NONE, NONE, NONE, NONE)                                        \
+  SLICE(1, 0, A1, B0, 3, NONE, NONE, NONE, NONE, NONE)
+#define WSTEP_LOADS LOAD_UNIT(A0) LOAD_UNIT(B0) LOAD_UNIT(B1) "s_mov_b32 m0, s48\n\ts_nop 0\n\t" WLOADX LOAD_UNIT(A1)
+// steps 0 and 1 requested: 34 loads
+#define WFIRST_LOADS WPOINTERS WSTEP_LOADS WNEXT_STEP WOTHER_STAGE_LOADS WSTEP_LOADS
+// n >= 2 steps
+#define WMAIN_LOOP                                                                                                       \
+  WPOINTERS WNEXT_STEP WNEXT_STEP "s_sub_u32 s47, %[n], 2\n\t"                                                           \
+  "s_waitcnt vmcnt(26)\n\ts_barrier\n\t" WRD(A0, AT_A0_0, 0) WRD(A0, AT_A0_0, 1) WRD(A0, AT_A0_0, 2)                     \
+  WRD(A0, AT_A0_0, 3) RD_UNIT(B0)                                                                                        \
+  "s_cmp_eq_u32 s47, 0\n\ts_cbranch_scc1 2f\n\t"                                                                         \
+  "1:\n\t" WPHASE0(ON, 21) WPHASE1(ON, 21) WPHASE2(ON, 21) WPHASE3(ON, 22) WNEXT_STEP WOTHER_STAGE_LOADS                 \
+  "s_sub_u32 s47, s47, 1\n\ts_cmp_lg_u32 s47, 0\n\ts_cbranch_scc1 1b\n\t"                                                \
+  "2:\n\t" WPHASE0(OFF, 21) WPHASE1(OFF, 17) WPHASE2(OFF, 13) WPHASE3(OFF, 9) WPHASE0(OFF, 4)                            \
+  WPHASE1(OFF, 0) WLAST_HALF "s_nop 15\n\ts_nop 7\n\t"
+
 // RING_PLAIN: C (f32) straight from the accumulators, with the biases of grouped products.  RING_SIGMOID: sigmoid(A . B)
 // as the next product's operand, whole rows of c16_pitch bf16 values with zeros past the last column.  RING_SILU, RING_GELU: half the tile's B rows are gate_proj's, half up_proj's;
 // act(gate) * up, 128 columns a tile, as bf16.  (GemmDesc says what each field means.)
 enum { RING_PLAIN, RING_SIGMOID, RING_SILU, RING_GELU };
-// AH: halves of 128 rows to a tile, two or (RING_SILU, RING_GELU) one.
-template <int KIND, int AH>
+// AH: halves of 128 rows to a tile, two or (RING_SILU, RING_GELU) one.  WIDE: with the strip of 32 columns (RING_SILU, RING_GELU: 16
+// rows of each matrix), N % 4 == 0.
+template <int KIND, int AH, bool WIDE = false>
 __global__ void __launch_bounds__(256, 1) gemm_bf16_ring_kernel(GemmDesc g) {
   constexpr bool GATED = KIND == RING_SILU || KIND == RING_GELU;
-  constexpr uint32_t BNO = GATED ? 128 : 256;  // output columns of a tile
+  static_assert(!WIDE || (AH == 2 && KIND != RING_SIGMOID), "the strip's epilogues");
+  constexpr uint32_t BNO = (GATED ? 128 : 256) + (WIDE ? (GATED ? 16 : 32) : 0);  // output columns of a tile
   warm_kernel_arguments<sizeof(GemmDesc)>();
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), wm = wave >> 1, wn = wave & 1;
@@ -319,6 +401,11 @@ __global__ void __launch_bounds__(256, 1) gemm_bf16_ring_kernel(GemmDesc g) {
   };
   const uint64_t sa0 = scalar(pa), sb0 = scalar(pb0), sb1 = scalar(pb1);
   const uint32_t lds = wave * 4096;  // (all LDS of this kernel is the stages, at offset 0: whole_lds)
+  // WIDE: eight rows of the strip, behind the columns of the quadrants
+  constexpr uint32_t STRIP_AT = 2 * 65536;
+  const uint32_t ldsx = STRIP_AT + wave * 1024, rx_row = wave * 8 + (lane >> 3);
+  const uint64_t sx = GATED && wave >= 2 ? sb1 : sb0;
+  const uint32_t dX = min((GATED ? 128 : 256) + (GATED ? rx_row & 15 : rx_row), last_b) * sb + ((lane & 7) ^ ((rx_row >> 1) & 7)) * 16;
 #define RING_IN_B                                                                                                         \
   [dB00] "v"(dB0[0]), [dB01] "v"(dB0[1]), [dB02] "v"(dB0[2]), [dB03] "v"(dB0[3]), [dB10] "v"(dB1[0]), [dB11] "v"(dB1[1]), \
       [dB12] "v"(dB1[2]), [dB13] "v"(dB1[3]), [pb0] "s"(sb0), [pb1] "s"(sb1), [lds] "s"(lds)
@@ -335,7 +422,11 @@ __global__ void __launch_bounds__(256, 1) gemm_bf16_ring_kernel(GemmDesc g) {
   uint64_t ga[4];  // AH == 1: this lane's pieces of A, a step on after every load
 #pragma unroll
   for (int i = 0; i < 4; ++i) ga[i] = (uint64_t)pa + dA0[i];
-  if constexpr (AH == 2) asm volatile(FIRST_LOADS::RING_IN : RING_SCALARS);
+#define RING_WIDE_IN [dX] "v"(dX), [px] "s"(sx), [ldsx] "s"(ldsx)
+#define RING_WIDE_SCALARS "s48", "s50", "s51"
+#define RING_STRIP RING_V10(11), "v120", "v121", "v122", "v123", "v124", "v125", "v126", "v127"
+  if constexpr (WIDE) asm volatile(WFIRST_LOADS::RING_IN, RING_WIDE_IN : RING_SCALARS, RING_WIDE_SCALARS);
+  else if constexpr (AH == 2) asm volatile(FIRST_LOADS::RING_IN : RING_SCALARS);
   else asm volatile(HFIRST_LOADS : RING_GATHERED : RING_IN_B : RING_SCALARS);
   float zero;
   asm volatile("v_mov_b32 %0, 0" : "=v"(zero));  // (the accumulators are cleared behind the first loads, not in front of them)
@@ -344,13 +435,19 @@ __global__ void __launch_bounds__(256, 1) gemm_bf16_ring_kernel(GemmDesc g) {
   for (int q = 0; q < AH * 8; ++q)
 #pragma unroll
     for (int e = 0; e < 16; ++e) acc[q >> 3][(q >> 2) & 1][(q >> 1) & 1][q & 1][e] = zero;
+  f32x16 strip[2];  // WIDE: [A half]
+#pragma unroll
+  for (int e = 0; e < 16; ++e) strip[0][e] = strip[1][e] = zero;
   const uint32_t half = lane >> 5;
-  uint32_t ra[4], rb[4];  // where this lane's fragments of a k-slice start in a unit
+  uint32_t ra[4], rb[4], rc[4], rx[4];  // where this lane's fragments of a k-slice start in a unit
+  const uint32_t first = WIDE ? wn : 0;  // (row block 0 of the accumulators is this one of the 64 rows' two)
 #pragma unroll
   for (int ks = 0; ks < 4; ++ks) {
     const uint32_t p = ((ks * 2 + half) ^ ((lane >> 1) & 7)) * 16 + (lane & 31) * 128;
-    ra[ks] = wm * 8192 + p;
+    ra[ks] = wm * 8192 + first * 4096 + p;
+    rc[ks] = wm * 8192 + (1 - first) * 4096 + p;
     rb[ks] = wn * 8192 + p;
+    rx[ks] = STRIP_AT + p;
   }
   unsigned long long tick0 = 0, real0 = 0;  // (clock probe only: GemmDesc::clock_ticks)
   if (KIND == RING_PLAIN && g.clock_ticks) {
@@ -367,7 +464,13 @@ __global__ void __launch_bounds__(256, 1) gemm_bf16_ring_kernel(GemmDesc g) {
 #define RING_PLACES                                                                                                      \
   [ra0] "+v"(ra[0]), [ra1] "+v"(ra[1]), [ra2] "+v"(ra[2]), [ra3] "+v"(ra[3]), [rb0] "+v"(rb[0]), [rb1] "+v"(rb[1]),      \
       [rb2] "+v"(rb[2]), [rb3] "+v"(rb[3])
-  if constexpr (AH == 2)
+#define RING_WIDE_PLACES                                                                                                  \
+  [x0] "+v"(strip[0]), [x1] "+v"(strip[1]), [rc0] "+v"(rc[0]), [rc1] "+v"(rc[1]), [rc2] "+v"(rc[2]), [rc3] "+v"(rc[3]),   \
+      [rx0] "+v"(rx[0]), [rx1] "+v"(rx[1]), [rx2] "+v"(rx[2]), [rx3] "+v"(rx[3])
+  if constexpr (WIDE)
+    asm volatile(WMAIN_LOOP : RING_ACC0, RING_ACC1, RING_PLACES, RING_WIDE_PLACES : RING_IN, RING_WIDE_IN, [n] "s"(n_steps)
+                 : RING_SCALARS, RING_WIDE_SCALARS, RING_STRIP, RING_FRAGMENTS);
+  else if constexpr (AH == 2)
     asm volatile(MAIN_LOOP : RING_ACC0, RING_ACC1, RING_PLACES : RING_IN, [n] "s"(n_steps) : RING_SCALARS, RING_FRAGMENTS);
   else
     asm volatile(HMAIN_LOOP : RING_ACC0, RING_PLACES, RING_GATHERED : RING_IN_B, [n] "s"(n_steps) : RING_SCALARS, RING_HALF_SCALARS, RING_FRAGMENTS);
@@ -408,7 +511,7 @@ __global__ void __launch_bounds__(256, 1) gemm_bf16_ring_kernel(GemmDesc g) {
       for (int j = 0; j < 2; ++j)
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-          const uint32_t r = i * 32 + (lane & 31), chunk = j * 8 + q * 2 + half;
+          const uint32_t r = (i ^ first) * 32 + (lane & 31), chunk = j * 8 + q * 2 + half;
           const f32x16 &x = acc[a][b][i][j], &u = acc[a][GATED ? 1 : b][i][j];
           float4 v = make_float4(x[q * 4], x[q * 4 + 1], x[q * 4 + 2], x[q * 4 + 3]);
           if (KIND == RING_GELU) v = make_float4(gelu_fast(v.x), gelu_fast(v.y), gelu_fast(v.z), gelu_fast(v.w));
@@ -484,6 +587,43 @@ __global__ void __launch_bounds__(256, 1) gemm_bf16_ring_kernel(GemmDesc g) {
         float4 v = out[it];
         v = make_float4(col < Nl ? v.x : 0.f, col + 1 < Nl ? v.y : 0.f, col + 2 < Nl ? v.z : 0.f, col + 3 < Nl ? v.w : 0.f);
         if (row < g.M && col < pitch) *(uint2 *)(C16 + (uint64_t)row * pitch + col) = bf16_pack4(v);
+      }
+    }
+  }
+  if constexpr (WIDE) {
+    // The strip: 32 rows of each half of A, 32 columns (16 where it is gated: of a block's columns the first 16 are gate's, and the
+    // same lane holds up's).  Rows of 128 bytes, out of LDS eight (gated: 32, sixteen) to a store.
+    constexpr int CH = GATED ? 4 : 8, RPS = 64 / CH;  // pieces of four columns to a row, rows to a store
+    constexpr uint32_t Q = GATED ? 2 : 4;
+    float *tile = ring_smem + wave * 8192;
+    const uint32_t col = n0 + (GATED ? 128 : 256) + (lane % CH) * 4;
+#pragma unroll
+    for (int a = 0; a < 2; ++a) {
+#pragma unroll
+      for (uint32_t q = 0; q < Q; ++q) {
+        const f32x16 &x = strip[a];
+        float4 v = make_float4(x[q * 4], x[q * 4 + 1], x[q * 4 + 2], x[q * 4 + 3]);
+        if (KIND == RING_GELU) v = make_float4(gelu_fast(v.x), gelu_fast(v.y), gelu_fast(v.z), gelu_fast(v.w));
+        if (KIND == RING_SILU) v = make_float4(silu_fast(v.x), silu_fast(v.y), silu_fast(v.z), silu_fast(v.w));
+        if (GATED) { v.x *= x[q * 4 + 8]; v.y *= x[q * 4 + 9]; v.z *= x[q * 4 + 10]; v.w *= x[q * 4 + 11]; }
+        *(float4 *)(tile + a * 1024 + (lane & 31) * 32 + (((q * 2 + half) ^ (lane & (CH - 1))) << 2)) = v;
+      }
+      const uint32_t row0 = m0 + a * 128 + wm * 64 + first * 32;
+#pragma unroll
+      for (int it = 0; it < 32 / RPS; ++it) {
+        const uint32_t r = it * RPS + lane / CH, row = row0 + r;
+        float4 v = *(const float4 *)(tile + a * 1024 + r * 32 + (((lane % CH) ^ (r & (CH - 1))) << 2));
+        if (row >= g.M || col >= Nl) continue;  // (N % 4 == 0: a piece is inside or outside)
+        if (GATED) {
+          *(uint2 *)(C16 + (uint64_t)row * pitch + col) = bf16_pack4(v);
+          continue;
+        }
+        if (Cadd) {
+          float4 add;
+          __builtin_memcpy(&add, Cadd + (uint64_t)row * Nl + col, 16);
+          v = make_float4(v.x + add.x, v.y + add.y, v.z + add.z, v.w + add.w);
+        }
+        __builtin_memcpy(C + (uint64_t)row * Nl + col, &v, 16);
       }
     }
   }
@@ -646,20 +786,20 @@ bool gemm_ring_ok(const GemmDesc &g) {
          (!g.dual_b || (g.c16 && !g.c));
 }
 
-template <int KIND, int AH = 2>
+template <int KIND, int AH = 2, bool WIDE = false>
 static hipError_t launch_ring_as(const LaunchCtx &lc, const GemmDesc &g, uint32_t grid) {
-  constexpr int smem = AH == 2 ? 2 * 65536 : 10 * 16384;
+  constexpr int smem = AH == 2 ? 2 * 65536 + (WIDE ? 2 * 4096 : 0) : 10 * 16384;
   static bool configured = false;  // one attribute call per kernel and process
   if (!configured) {
-    const hipError_t e = whole_lds((const void *)gemm_bf16_ring_kernel<KIND, AH>, smem);
+    const hipError_t e = whole_lds((const void *)gemm_bf16_ring_kernel<KIND, AH, WIDE>, smem);
     if (e != hipSuccess) return e;
     configured = true;
   }
-  cg_launch(lc, gemm_bf16_ring_kernel<KIND, AH>, dim3(grid), dim3(256), smem, g);
+  cg_launch(lc, gemm_bf16_ring_kernel<KIND, AH, WIDE>, dim3(grid), dim3(256), smem, g);
   return hipGetLastError();
 }
 
-hipError_t launch_gemm_ring(const LaunchCtx &lc, const GemmDesc &g, bool half_height) {
+hipError_t launch_gemm_ring(const LaunchCtx &lc, const GemmDesc &g, bool half_height, bool wide) {
   if (!gemm_ring_ok(g)) return hipErrorInvalidValue;
   if (half_height) {
     if (!g.dual_b || g.splits > 1 || g.K < 192) return hipErrorInvalidValue;
@@ -667,9 +807,13 @@ hipError_t launch_gemm_ring(const LaunchCtx &lc, const GemmDesc &g, bool half_he
     if (tiles > 0x7FFFFFFFull) return hipErrorInvalidValue;
     return g.glu_kind ? launch_ring_as<RING_GELU, 1>(lc, g, (uint32_t)tiles) : launch_ring_as<RING_SILU, 1>(lc, g, (uint32_t)tiles);
   }
-  const uint32_t bno = g.dual_b ? 128 : 256, batch = g.nb0 * g.nb1 * (g.splits > 1 ? g.splits : 1);
+  if (wide && (g.N % 4 || g.n_group || g.act_sigmoid)) return hipErrorInvalidValue;
+  const uint32_t bno = (g.dual_b ? 128 : 256) + (wide ? (g.dual_b ? 16 : 32) : 0), batch = g.nb0 * g.nb1 * (g.splits > 1 ? g.splits : 1);
   const uint64_t grid = (uint64_t)((g.M + 255) / 256) * ((g.N + bno - 1) / bno) * batch;
   if (grid > 0x7FFFFFFFull) return hipErrorInvalidValue;
+  if (wide && g.dual_b)
+    return g.glu_kind ? launch_ring_as<RING_GELU, 2, true>(lc, g, (uint32_t)grid) : launch_ring_as<RING_SILU, 2, true>(lc, g, (uint32_t)grid);
+  if (wide) return launch_ring_as<RING_PLAIN, 2, true>(lc, g, (uint32_t)grid);
   if (g.dual_b) return g.glu_kind ? launch_ring_as<RING_GELU>(lc, g, (uint32_t)grid) : launch_ring_as<RING_SILU>(lc, g, (uint32_t)grid);
   if (g.act_sigmoid && g.splits <= 1) return launch_ring_as<RING_SIGMOID>(lc, g, (uint32_t)grid);
   return launch_ring_as<RING_PLAIN>(lc, g, (uint32_t)grid);

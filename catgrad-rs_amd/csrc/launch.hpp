@@ -360,9 +360,10 @@ struct GemmDesc {
   unsigned long long *clock_ticks;
 };
 // k_gemm_ring.hip: the 256 x 256 tiles of large bf16 products (plain or grouped, sigmoid, stacked gate / up);
-// half_height: the stacked gate / up of fewer rows on tiles of 128 x 256, K >= 192
+// half_height: the stacked gate / up of fewer rows on tiles of 128 x 256, K >= 192; wide: tiles of 256 x 288 (plain without groups or a
+// sigmoid, stacked gate / up), N % 4 == 0
 bool gemm_ring_ok(const GemmDesc &g);
-hipError_t launch_gemm_ring(const LaunchCtx &lc, const GemmDesc &g, bool half_height = false);
+hipError_t launch_gemm_ring(const LaunchCtx &lc, const GemmDesc &g, bool half_height = false, bool wide = false);
 // k_gemm_f32.hip: f32 products of operands in whole 16-byte pieces; gemm_f32_split: the slices of k it is fastest with (and how long
 // it then takes, about; gemm_f32_least_us: no less than this)
 bool gemm_f32_ok(const GemmDesc &g);

@@ -47,6 +47,32 @@ def test_product(hip_bf16, M, N, K):
     assert np.all(np.abs(got[0] - ref) <= bound)
 
 
+# 256 x 288: one round where 256 x 256 take two, the fewest k-steps it is given, an odd number; rows that end in the first and the second
+# half of a tile, columns that end in the strip and in front of it; and less than a round of 256 x 256 in place of two of 128 x 128
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(4100, 4308, 256), (4250, 4084, 320), (4352, 4320, 576), (3900, 4148, 1088), (3001, 3003, 768), (2100, 4100, 1024)])
+def test_wide_product(hip_bf16, M, N, K):
+    test_product(hip_bf16, M, N, K)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,M,N,K", [(1, 4100, 4308, 256), (1, 4250, 4084, 320), (3, 1300, 4292, 256), (1, 3001, 3003, 768)])
+def test_wide_product_and_residual(hip_bf16, B, M, N, K):
+    test_product_and_residual(hip_bf16, B, M, N, K)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("act", ["silu", "gelu"])
+@pytest.mark.parametrize("M,F,K", [(4100, 2156, 256), (4250, 2052, 320), (3900, 2304, 640)])    # columns that end in the strip, in front of it, with a tile
+def test_wide_gated(hip_bf16, M, F, K, act):
+    test_gated(hip_bf16, M, F, K, act)
+
+
+@pytest.mark.gpu
+def test_wide_infinities(hip_bf16):
+    test_infinities(hip_bf16, 4100, 4308, 256)
+
+
 # one column (a wave to a row, its last pieces of k partly past the end, or 64 x 64 tiles), and more than 32 columns but less than 64:
 # tiles of 32 x 32 and of 64 x 64 at both ends of either, slices of the deepest
 @pytest.mark.gpu
