@@ -3070,9 +3070,23 @@ bool gemm_pack_wanted(const GemmDesc &g, bool epilogue) {
   return epilogue || !gemm_fast_path(t, av, bv) || (g.M >= 64 && 2.0 * batch * g.M * g.N * g.K >= PACK_ALIGNED_MIN_FLOPS);
 }
 
+// Which of a rotating product's tiles: 256 x 256 (ring_store_attention), or those of 128 columns and less.  A round of the large ones is
+// 1.7 rounds of 128 x 128 two to a CU (us, small and large; 3072 columns of heads of 64, K = 2048, two rounds and one: 2700 rows 64.6,
+// 57.4, 2900 63.6, 52.1, 3300 67.6, 58.2, 4090 86.4, 64.1; 6144 columns of heads of 128 with biases: 1400 68.3, 59.8, 5 x 290 78.3, 66.6).
+// Heads of 256 with their norm have no other: against a plain product, the rotation's launch and a transposition, 1536 columns, K =
+// 1152, 3 x 1900 rows 65.3 and 45.6, 6 x 1999 112.6 and 86.9, 8 x 2048 (two rounds) 115 and 96.6; below two rounds of 128 x 128 the plain
+// product's tiles are smaller.
+static bool rope_on_large_tiles(const LaunchCtx &lc, const GemmDesc &g) {
+  if (!gemm_ring_ok(g)) return false;
+  const uint64_t cus = (uint64_t)lc.n_cus, t256 = (uint64_t)((g.M + 255) / 256) * ((g.N + 255) / 256),
+                 t128 = (uint64_t)((g.M + 127) / 128) * ((g.N + 127) / 128);
+  const uint64_t large = (t256 + cus - 1) / cus, small = (t128 + 2 * cus - 1) / (2 * cus);
+  return g.rope_hd == 256 ? t128 > 2 * cus : g.K >= 768 && large * 17 <= small * 10;
+}
+
 bool gemm_rope_epilogue_ok(const LaunchCtx &lc, const GemmDesc &g) {
   if (!g.rope_s || !g.n_group || !gemm_epilogue_ok(g)) return false;
-  if (g.rope_hd != 64 && g.rope_hd != 128) return false;
+  if (g.rope_hd != 64 && g.rope_hd != 128 && g.rope_hd != 256) return false;
   if (g.nb0 * g.nb1 != 1 || g.glu_gate || g.c16 || g.dual_b || g.M % g.rope_s || !gemm_rows(g.M, g.K)) return false;
   bool grp256 = true;
   for (uint32_t p = 0; p < g.n_group; ++p) {
@@ -3086,11 +3100,12 @@ bool gemm_rope_epilogue_ok(const LaunchCtx &lc, const GemmDesc &g) {
       return false;
     }
   }
-  // launch_matmul's tiles of 32 and 128 rows have this epilogue (128 columns, or 64 - for heads of 64 - where those are
-  // too few for the CUs); the 256 x 256 tile of the largest problems has not
+  // launch_matmul's tiles of 32 to 128 rows have this epilogue (128 columns, or 64 - for heads of 64 - where those are
+  // too few for the CUs), and 256 x 256, which alone hold heads of 256 and norm; several rounds of products that are not for those are
+  // better left without
+  if (rope_on_large_tiles(lc, g)) return true;
   const uint64_t t256 = (uint64_t)((g.M + 255) / 256) * ((g.N + 255) / 256);
-  if (t256 >= (uint64_t)lc.n_cus && grp256) return false;
-  return g.N >= 128;
+  return g.rope_hd != 256 && g.N >= 128 && !(t256 >= (uint64_t)lc.n_cus && grp256);
 }
 
 // A plain product of 2 to 16 rows with bf16 weights [N][K] that gemv_rows_mfma_kernel takes.
@@ -3288,7 +3303,9 @@ hipError_t launch_matmul(const LaunchCtx &lc_in, const GemmDesc &g, const char *
         const uint64_t wide = (uint64_t)((g.M + 255) / 256) * ((g.N + columns - 1) / columns) * batch;
         return splits == 1 && g.K >= 256 && g.N % 4 == 0 && !g.n_group && !g.act_sigmoid && rounds_of(wide) * 9 < rounds_of(tiles) * 8;
       };
-      if (g.rope_s && g.M <= 128) {
+      if (g.rope_s && rope_on_large_tiles(lc, g)) {
+        e = launch_gemm_ring(lc, gg);
+      } else if (g.rope_s && g.M <= 128) {
         // q / k / v of a few rows: a workgroup takes in its rows of both operands at about 42 GB/s however wide its tile is,
         // and 64 x 64 or 128 x 64 tiles are 48 workgroups for 3072 columns.  32 x 32 tiles, of columns that rotate into
         // each other: 37 rows 14.5 -> 12.1 us, 64 15.1 -> 10.5, 100 17.4 -> 12.4, 128 18.3 -> 14.6; with heads of 128 and
@@ -3343,7 +3360,7 @@ hipError_t launch_matmul(const LaunchCtx &lc_in, const GemmDesc &g, const char *
         else if (g.act_sigmoid && t256 >= (uint64_t)lc.n_cus) e = launch_gemm_dma<256, 256, 2, 4, true, 2>(lc, gg, (uint32_t)t256);
         else if (deep) e = launch_gemm_dma<128, 128, 2, 4, true, 4>(lc, gg, (uint32_t)t128);
         else e = launch_gemm_dma<128, 128, 2, 2, true, 2>(lc, gg, (uint32_t)t128);
-      } else if (t256 >= (uint64_t)lc.n_cus && grp256 && gemm_ring_ok(gg)) {
+      } else if (t256 >= (uint64_t)lc.n_cus && grp256 && !g.rope_s && gemm_ring_ok(gg)) {
         // 256 x 256 tiles run one to a CU, 128 x 128 two to a CU: when the big tiles leave the last round of
         // workgroups mostly empty (320 tiles on 256 CUs), the small ones fill the machine better
         auto fill = [&](uint64_t tiles, uint64_t slots) { return (double)tiles / (double)((tiles + slots - 1) / slots * slots); };

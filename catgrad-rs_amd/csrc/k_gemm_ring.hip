@@ -27,6 +27,7 @@
 // 1.1 for its first loads and 5.3 to store.
 #include <hip/hip_runtime.h>
 #include "launch.hpp"
+#include <type_traits>
 #include "dev_common.hpp"
 
 namespace cgk {
@@ -337,13 +338,218 @@ static hipError_t whole_lds(const void *kernel, int bytes) {
 // RING_PLAIN: C (f32) straight from the accumulators, with the biases of grouped products.  RING_SIGMOID: sigmoid(A . B)
 // as the next product's operand, whole rows of c16_pitch bf16 values with zeros past the last column.  RING_SILU, RING_GELU: half the tile's B rows are gate_proj's, half up_proj's;
 // act(gate) * up, 128 columns a tile, as bf16.  (GemmDesc says what each field means.)
-enum { RING_PLAIN, RING_SIGMOID, RING_SILU, RING_GELU };
+// RING_ROPE_*: grouped q / k / v, rotated and transposed as they leave (GemmDesc::rope_role; rope_s >= 64, groups of whole tiles), for heads
+// of 64, 128 and 256 columns, those with biases, and with a norm in front of the rotation.
+enum { RING_PLAIN, RING_SIGMOID, RING_SILU, RING_GELU, RING_ROPE_64, RING_ROPE_64_BIAS, RING_ROPE_128, RING_ROPE_128_BIAS, RING_ROPE_256, RING_ROPE_256_NORM };
+// q / k / v of an attention (GemmDesc::rope_role) out of the accumulators of a 256 x 256 tile, half of the rows at a time: every
+// wavefront puts its 64 rows of both column halves into LDS - with a bias, or leaving the sums of their squares -, row r's piece of four
+// columns `chunk` of a column half at place chunk ^ (r & 15).
+struct RingRope {  // one group's part of a GemmDesc
+  const float *cos, *sin, *gamma, *bias;
+  float *out, *c;
+  uint16_t *out16;
+  int64_t cs_ss;
+  float n_as_float, eps, gamma_offset;
+  uint32_t M, N, S;
+};
+__device__ __forceinline__ uint32_t ring_place(uint32_t r, uint32_t chunk) { return r * 64 + ((chunk ^ (r & 15)) << 2); }
+template <bool BIAS, bool SQUARES>
+__device__ __forceinline__ void ring_half_to_lds(const f32x16 (&acc)[2][2][2], const float *bias, float *mine, float *sums) {
+  const uint32_t lane = threadIdx.x & 63, half = lane >> 5;
+  float ss[2] = {0.f, 0.f};
+#pragma unroll
+  for (int b = 0; b < 2; ++b)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        float4 w;
+        if (BIAS) __builtin_memcpy(&w, bias + b * 128 + j * 32 + q * 8 + half * 4, 16);
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          const f32x16 &x = acc[b][i][j];
+          float4 v = make_float4(x[q * 4], x[q * 4 + 1], x[q * 4 + 2], x[q * 4 + 3]);
+          if (BIAS) { v.x += w.x; v.y += w.y; v.z += w.z; v.w += w.w; }
+          if (SQUARES) ss[i] += v.x * v.x + v.y * v.y + v.z * v.z + v.w * v.w;
+          *(float4 *)(mine + b * 4096 + ring_place(i * 32 + (lane & 31), j * 8 + q * 2 + half)) = v;
+        }
+      }
+  if (SQUARES) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      ss[i] += __shfl_xor(ss[i], 32, 64);
+      if (!half) sums[i * 32 + lane] = ss[i];
+    }
+  }
+}
+
+// Queries and keys, heads of HD columns, rotated with the arithmetic of rope_kernel; NORM: normed before that with rmsnorm_kernel's.  A lane
+// takes a piece of the lower half of a head and its partner of the upper - in the same rows (heads of 64), from the neighbouring
+// wavefront (128: each does half of the 64 rows), from the other column half (256) - and stores both.  Table rows serve both column halves
+// (not heads of 256), and are on their way a group of pieces ahead: the first group's (`t`) while the tile goes to LDS.
+template <int HD>
+struct RingPieces {
+  static constexpr uint32_t H = HD / 2, PER = HD == 64 ? 8 : 16, RPU = 64 / PER;  // pieces to half a row, rows to a unit
+  static constexpr int UNITS = HD == 256 ? 16 : 8, GROUP = 4, BS = HD == 256 ? 1 : 2;  // units of a half tile, of a group; pairs to a unit
+  uint32_t row0, sq0, pos0;  // this wavefront's first row, its sequence and position
+  uint32_t chunk, row_in, in_half;  // the piece of its row, the row of the first unit, the piece's column of the lower half of its head
+  float4 t[GROUP][4];  // cos and sin of the lower half, of the upper
+  __device__ __forceinline__ RingPieces(uint32_t first_row, uint32_t S, uint32_t wn, uint32_t lane)
+      : row0(first_row), sq0(first_row / S), pos0(first_row - first_row / S * S), chunk(lane % PER), row_in(lane / PER + (HD == 128 ? wn * 32 : 0)),
+        in_half((HD == 256 ? wn * 64 : 0) + lane % PER * 4) {}
+  __device__ __forceinline__ void tables(const RingRope &d, int u0) {
+#pragma unroll
+    for (int u = 0; u < GROUP; ++u) {
+      const uint32_t r = row_in + (u0 + u) * RPU;
+      uint32_t pos = pos0 + (row0 + r < d.M ? r : 0);
+      if (pos >= d.S) pos -= d.S;
+      const int64_t from = (int64_t)pos * d.cs_ss + in_half;
+      t[u][0] = *(const float4 *)(d.cos + from);
+      t[u][1] = *(const float4 *)(d.sin + from);
+      t[u][2] = *(const float4 *)(d.cos + from + H);
+      t[u][3] = *(const float4 *)(d.sin + from + H);
+    }
+  }
+};
+template <int HD, bool NORM>
+__device__ __forceinline__ void ring_store_rotated(const RingRope &d, RingPieces<HD> &p, uint32_t n0, float *smem, uint32_t wave, uint32_t lane) {
+  typedef RingPieces<HD> P;
+  const uint32_t wn = wave & 1, S = d.S, heads = d.N / HD;
+  const float *mine = smem + wave * 8192;
+  float *sums = smem + 32768 + wave * 128;  // NORM: the sums of squares, then each row's divisor and its inverse
+  float4 g_lo, g_hi;
+  if (NORM) {  // (heads of 256: a row's columns are with two wavefronts)
+    if (d.gamma) {
+      g_lo = *(const float4 *)(d.gamma + p.in_half);
+      g_hi = *(const float4 *)(d.gamma + p.in_half + P::H);
+    }
+    const float sum = sums[lane] + smem[32768 + (wave ^ 1) * 128 + lane];
+    __syncthreads();
+    const float rms = sqrtf(sum / d.n_as_float + d.eps);
+    sums[lane] = rms == INFINITY ? 0.f : rms;  // (then 1 / rms = 0, and every finite value of the row leaves as 0)
+    sums[64 + lane] = 1.f / rms;
+  }
+#pragma unroll 1
+  for (int u0 = 0; u0 < P::UNITS; u0 += P::GROUP) {
+    float4 now[P::GROUP][4];
+#pragma unroll
+    for (int u = 0; u < P::GROUP; ++u)
+#pragma unroll
+      for (int k = 0; k < 4; ++k) now[u][k] = p.t[u][k];
+    if (u0 + P::GROUP < P::UNITS) p.tables(d, u0 + P::GROUP);
+#pragma unroll
+    for (int u = 0; u < P::GROUP; ++u) {
+      const uint32_t r = p.row_in + (u0 + u) * P::RPU;
+#pragma unroll
+      for (int b = 0; b < P::BS; ++b) {
+        const float *lo = HD == 128 ? smem + (wave & ~1u) * 8192 + b * 4096 : mine + b * 4096;
+        const float *hi = HD == 64 ? lo : HD == 128 ? lo + 8192 : lo + 4096;
+        float4 x = *(const float4 *)(lo + ring_place(r, p.chunk)), y = *(const float4 *)(hi + ring_place(r, HD == 64 ? p.chunk + 8 : p.chunk));
+        if (NORM) {
+          // x / rms, rounded once: the quotient by the inverse, and what it leaves of x
+          const float rms = sums[r], inv = sums[64 + r];
+          auto normed = [&](float v, float w) {
+            const float q = v * inv, n = fmaf(fmaf(-q, rms, v), inv, q);
+            return d.gamma ? n * (d.gamma_offset + w) : n;
+          };
+          x = make_float4(normed(x.x, g_lo.x), normed(x.y, g_lo.y), normed(x.z, g_lo.z), normed(x.w, g_lo.w));
+          y = make_float4(normed(y.x, g_hi.x), normed(y.y, g_hi.y), normed(y.z, g_hi.z), normed(y.w, g_hi.w));
+        }
+        const float4 c0 = now[u][0], s0 = now[u][1], c1 = now[u][2], s1 = now[u][3];
+        const float4 l = make_float4(c0.x * x.x + s0.x * -y.x, c0.y * x.y + s0.y * -y.y, c0.z * x.z + s0.z * -y.z, c0.w * x.w + s0.w * -y.w);
+        const float4 h = make_float4(c1.x * y.x + s1.x * x.x, c1.y * y.y + s1.y * x.y, c1.z * y.z + s1.z * x.z, c1.w * y.w + s1.w * x.w);
+        if (p.row0 + r < d.M) {
+          // [sequence][head][position][column]; a position past a sequence's end is the next one's
+          const uint32_t head = (n0 + b * 128 + (HD == 64 ? wn * 64 : 0)) / HD, over = p.pos0 + r >= S ? 1 : 0;
+          const uint64_t to = ((uint64_t)((p.sq0 + over) * heads + head) * S + (p.pos0 + r - over * S)) * HD + p.in_half;
+          *(float4 *)(d.out + to) = l;
+          *(float4 *)(d.out + to + P::H) = h;
+          if (d.out16) {
+            *(uint2 *)(d.out16 + to) = bf16_pack4(l);
+            *(uint2 *)(d.out16 + to + P::H) = bf16_pack4(h);
+          }
+        }
+      }
+    }
+  }
+}
+
+// Values: as they are, and as bf16 [sequence][column][position], rows of positions padded with zeros to a multiple of eight.
+__device__ __forceinline__ void ring_store_values(const RingRope &d, uint32_t row0, uint32_t n0, const float *mine, uint32_t wn, uint32_t lane) {
+  const uint32_t S = d.S, Sp = (S + 7) & ~7u, sq0 = row0 / S, pos0 = row0 - sq0 * S;
+  const uint32_t r0 = (lane >> 2) * 4, row = row0 + r0, over = pos0 + r0 >= S ? 1 : 0, sq = sq0 + over, pos = pos0 + r0 - over * S;
+#pragma unroll 1
+  for (uint32_t b = 0; b < 2; ++b) {
+    const uint32_t col0 = n0 + b * 128 + wn * 64;  // (whole tiles: every column exists)
+    const float *tile = mine + b * 4096;
+#pragma unroll 4
+    for (uint32_t it = 0; it < 16; ++it) {
+      const uint32_t r = it * 4 + (lane >> 4);
+      if (row0 + r < d.M) *(float4 *)(d.c + (uint64_t)(row0 + r) * d.N + col0 + (lane & 15) * 4) = *(const float4 *)(tile + ring_place(r, lane & 15));
+    }
+    // four positions of four columns to a lane
+#pragma unroll 1
+    for (uint32_t it = 0; it < 4; ++it) {
+      const uint32_t chunk = it * 4 + (lane & 3);
+      float4 f[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) f[e] = *(const float4 *)(tile + ring_place(r0 + e, chunk));
+      uint16_t *to = d.out16 + ((uint64_t)sq * d.N + col0 + chunk * 4) * Sp + pos;
+      if (row + 4 <= d.M && pos % 4 == 0 && pos + 4 <= S) {
+        const uint2 w[4] = {bf16_pack4(make_float4(f[0].x, f[1].x, f[2].x, f[3].x)), bf16_pack4(make_float4(f[0].y, f[1].y, f[2].y, f[3].y)),
+                            bf16_pack4(make_float4(f[0].z, f[1].z, f[2].z, f[3].z)), bf16_pack4(make_float4(f[0].w, f[1].w, f[2].w, f[3].w))};
+#pragma unroll
+        for (int x = 0; x < 4; ++x) {
+          *(uint2 *)(to + (uint64_t)x * Sp) = w[x];
+          if (pos + 4 == S && Sp > S) *(uint2 *)(to + (uint64_t)x * Sp + 4) = make_uint2(0u, 0u);
+        }
+      } else {  // the product's last rows, or four that straddle two sequences
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          if (row + e >= d.M) continue;
+          const bool next = pos + e >= S;
+          uint16_t *at = to + e + (next ? (uint64_t)d.N * Sp - S : 0);
+          const uint2 h = bf16_pack4(f[e]);
+          const uint16_t v[4] = {(uint16_t)h.x, (uint16_t)(h.x >> 16), (uint16_t)h.y, (uint16_t)(h.y >> 16)};
+#pragma unroll
+          for (int x = 0; x < 4; ++x) {
+            at[(uint64_t)x * Sp] = v[x];
+            if (pos + e + 1 == (next ? 2 * S : S))
+              for (uint32_t z = 1; z <= Sp - S; ++z) at[(uint64_t)x * Sp + z] = 0;
+          }
+        }
+      }
+    }
+  }
+}
+
+// (one place that reads the accumulators: where two branches do, the compiler spills them)
+template <int HD, bool BIAS, bool NORM>
+__device__ __forceinline__ void ring_store_attention(const RingRope d, bool values, uint32_t m0, uint32_t n0, const f32x16 (&acc)[2][2][2][2], float *smem) {
+  const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wm = wave >> 1, wn = wave & 1;
+  float *mine = smem + wave * 8192;
+  auto half_tile = [&](auto A) __attribute__((always_inline)) {
+    constexpr int a = A;
+    const uint32_t row0 = m0 + a * 128 + wm * 64;
+    RingPieces<HD> p(row0, d.S, wn, lane);
+    if (!values) p.tables(d, 0);
+    if (a) __syncthreads();  // the other half has been read
+    ring_half_to_lds<BIAS, NORM>(acc[a], d.bias + n0 + wn * 64, mine, smem + 32768 + wave * 128);
+    __syncthreads();
+    if (values) ring_store_values(d, row0, n0, mine, wn, lane);
+    else ring_store_rotated<HD, NORM>(d, p, n0, smem, wave, lane);
+  };
+  half_tile(std::integral_constant<int, 0>());
+  half_tile(std::integral_constant<int, 1>());
+}
+
 // AH: halves of 128 rows to a tile, two or (RING_SILU, RING_GELU) one.  WIDE: with the strip of 32 columns (RING_SILU, RING_GELU: 16
 // rows of each matrix), N % 4 == 0.
 template <int KIND, int AH, bool WIDE = false>
 __global__ void __launch_bounds__(256, 1) gemm_bf16_ring_kernel(GemmDesc g) {
   constexpr bool GATED = KIND == RING_SILU || KIND == RING_GELU;
-  static_assert(!WIDE || (AH == 2 && KIND != RING_SIGMOID), "the strip's epilogues");
+  constexpr bool ROPE = KIND >= RING_ROPE_64;
+  static_assert(!WIDE || (AH == 2 && KIND != RING_SIGMOID && !ROPE), "the strip's epilogues");
   constexpr uint32_t BNO = (GATED ? 128 : 256) + (WIDE ? (GATED ? 16 : 32) : 0);  // output columns of a tile
   warm_kernel_arguments<sizeof(GemmDesc)>();
   const int tid = threadIdx.x, lane = tid & 63;
@@ -366,7 +572,8 @@ __global__ void __launch_bounds__(256, 1) gemm_bf16_ring_kernel(GemmDesc g) {
   const uint16_t *B = (const uint16_t *)g.b + b0 * g.sb_b0 + b1 * g.sb_b1;
   float *C = (g.splits > 1 ? g.workspace + (uint64_t)split * batch * g.M * g.N : g.c) + (uint64_t)bz * g.M * g.N;
   const float *Bias = nullptr, *Cadd = KIND == RING_PLAIN && g.c_add && g.splits <= 1 ? g.c_add + (uint64_t)bz * g.M * g.N : nullptr;
-  if (KIND == RING_PLAIN && g.n_group) {  // grouped products: tiles never straddle two
+  uint32_t grp = 0;
+  if ((KIND == RING_PLAIN || ROPE) && g.n_group) {  // grouped products: tiles never straddle two
     uint32_t p = 0;
     while (p + 1 < g.n_group && n0 >= g.grp_n[p]) {
       n0 -= g.grp_n[p];
@@ -376,6 +583,7 @@ __global__ void __launch_bounds__(256, 1) gemm_bf16_ring_kernel(GemmDesc g) {
     C = g.grp_c[p];
     Nl = g.grp_n[p];
     Bias = g.grp_bias[p];
+    grp = p;
   }
   const uint32_t k_begin = split * g.k_per_split, k_end = min(g.K, k_begin + g.k_per_split);
   const uint32_t n_steps = __builtin_amdgcn_readfirstlane((k_end - k_begin) / 64);
@@ -488,6 +696,17 @@ __global__ void __launch_bounds__(256, 1) gemm_bf16_ring_kernel(GemmDesc g) {
   // 6000 x 3072 x 2048 178 -> 95).
   __syncthreads();  // every wavefront has read its last fragments
   extern __shared__ __attribute__((aligned(16))) float ring_smem[];
+  if constexpr (ROPE) {
+    // (read here, not held through the main loop)
+    auto *late = (const __attribute__((address_space(4))) GemmDesc *)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(late));
+    const RingRope d = {late->rope_cos[grp], late->rope_sin[grp], late->rope_gamma[grp], late->grp_bias[grp], late->rope_out[grp], late->grp_c[grp],
+                        late->rope_out16[grp], late->rope_cs_ss[grp], late->rope_n_as_float[grp], late->rope_eps[grp], late->rope_gamma_offset[grp],
+                        late->M, late->grp_n[grp], late->rope_s};
+    constexpr int HD = KIND >= RING_ROPE_256 ? 256 : KIND >= RING_ROPE_128 ? 128 : 64;
+    ring_store_attention<HD, KIND == RING_ROPE_64_BIAS || KIND == RING_ROPE_128_BIAS, KIND == RING_ROPE_256_NORM>(d, late->rope_role[grp] == 2, m0, n0, acc, ring_smem);
+    return;
+  }
   uint16_t *C16 = g.c16 ? g.c16 + (uint64_t)bz * g.M * g.N : nullptr;
   const bool whole = m0 + BM <= g.M && n0 + BNO <= Nl;
   constexpr bool F32 = KIND == RING_PLAIN;
@@ -777,18 +996,30 @@ hipError_t launch_moe_ring(const LaunchCtx &lc, const MoeGemmDesc &g) {
   return launch_moe_ring_as<MOE_PLAIN>(lc, g, grid);
 }
 
+// q / k / v that rotate as they leave: groups of whole tiles (so whole heads), all with a bias or none, all that rotate normed or none
+// (heads of 256, no bias), sequences no shorter than the 64 rows that a wavefront stores at a time.
+static bool gemm_ring_rope_ok(const GemmDesc &g) {
+  if (!g.n_group || g.splits > 1 || g.rope_s < 64 || (g.rope_hd != 64 && g.rope_hd != 128 && g.rope_hd != 256)) return false;
+  bool norm = false, plain = false;
+  for (uint32_t p = 0; p < g.n_group; ++p) {
+    if (!g.rope_role[p] || g.grp_n[p] % 256 || !g.grp_bias[p] != !g.grp_bias[0] || (g.grp_bias[p] && g.rope_hd == 256)) return false;
+    if (g.rope_role[p] == 1) (g.rope_norm[p] ? norm : plain) = true;
+  }
+  return !norm || (!plain && g.rope_hd == 256);
+}
+
 // Operands whose rows lie within 32-bit byte offsets of a tile's first row, two k-steps at least to each slice.
 bool gemm_ring_ok(const GemmDesc &g) {
   const uint32_t splits = g.splits > 1 ? g.splits : 1, last = splits > 1 ? g.K - (splits - 1) * g.k_per_split : g.K;
   if (splits > 1 && ((uint64_t)(splits - 1) * g.k_per_split >= g.K || g.k_per_split % 64 || g.k_per_split < 128)) return false;
   return g.sak == 1 && g.sbk == 1 && last % 64 == 0 && last >= 128 && g.sam >= 0 && g.sbn >= 0 && g.sam <= (1 << 22) &&
-         g.sbn <= (1 << 22) && !g.rope_s && !g.glu_gate && (!g.act_sigmoid || splits > 1 || g.c16_pitch) &&
+         g.sbn <= (1 << 22) && (!g.rope_s || gemm_ring_rope_ok(g)) && !g.glu_gate && (!g.act_sigmoid || splits > 1 || g.c16_pitch) &&
          (!g.dual_b || (g.c16 && !g.c));
 }
 
 template <int KIND, int AH = 2, bool WIDE = false>
 static hipError_t launch_ring_as(const LaunchCtx &lc, const GemmDesc &g, uint32_t grid) {
-  constexpr int smem = AH == 2 ? 2 * 65536 + (WIDE ? 2 * 4096 : 0) : 10 * 16384;
+  constexpr int smem = AH == 2 ? 2 * 65536 + (WIDE ? 2 * 4096 : 0) + (KIND >= RING_ROPE_64 ? 4 * 128 * 4 : 0) : 10 * 16384;  // (ring_store_rotated: sums of squares)
   static bool configured = false;  // one attribute call per kernel and process
   if (!configured) {
     const hipError_t e = whole_lds((const void *)gemm_bf16_ring_kernel<KIND, AH, WIDE>, smem);
@@ -811,6 +1042,13 @@ hipError_t launch_gemm_ring(const LaunchCtx &lc, const GemmDesc &g, bool half_he
   const uint32_t bno = (g.dual_b ? 128 : 256) + (wide ? (g.dual_b ? 16 : 32) : 0), batch = g.nb0 * g.nb1 * (g.splits > 1 ? g.splits : 1);
   const uint64_t grid = (uint64_t)((g.M + 255) / 256) * ((g.N + bno - 1) / bno) * batch;
   if (grid > 0x7FFFFFFFull) return hipErrorInvalidValue;
+  if (g.rope_s) {
+    if (wide) return hipErrorInvalidValue;
+    const bool bias = g.grp_bias[0] != nullptr;
+    if (g.rope_hd == 256) return g.rope_norm[0] || g.rope_norm[1] || g.rope_norm[2] ? launch_ring_as<RING_ROPE_256_NORM>(lc, g, (uint32_t)grid) : launch_ring_as<RING_ROPE_256>(lc, g, (uint32_t)grid);
+    if (g.rope_hd == 128) return bias ? launch_ring_as<RING_ROPE_128_BIAS>(lc, g, (uint32_t)grid) : launch_ring_as<RING_ROPE_128>(lc, g, (uint32_t)grid);
+    return bias ? launch_ring_as<RING_ROPE_64_BIAS>(lc, g, (uint32_t)grid) : launch_ring_as<RING_ROPE_64>(lc, g, (uint32_t)grid);
+  }
   if (wide && g.dual_b)
     return g.glu_kind ? launch_ring_as<RING_GELU, 2, true>(lc, g, (uint32_t)grid) : launch_ring_as<RING_SILU, 2, true>(lc, g, (uint32_t)grid);
   if (wide) return launch_ring_as<RING_PLAIN, 2, true>(lc, g, (uint32_t)grid);

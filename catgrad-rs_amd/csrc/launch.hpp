@@ -344,7 +344,7 @@ struct GemmDesc {
   const float *grp_bias[3];
   // optional, with n_group (gemm_rope_epilogue_ok): the products are the q / k / v projections of M / rope_s
   // sequences of rope_s positions each (row m = sequence m / rope_s, position m % rope_s) with heads of rope_hd
-  // (64 or 128) columns.  A group with rope_role 1 leaves the kernel rotated (apply_rope_embedding, cos / sin
+  // (64, 128 or 256) columns.  A group with rope_role 1 leaves the kernel rotated (apply_rope_embedding, cos / sin
   // rows of rope_hd floats at rope_cs_ss apart, indexed by position) as [sequence][head][position][rope_hd] at
   // rope_out (f32) and rope_out16 (bf16, optional) instead of grp_c; a group with rope_role 2 is stored as usual
   // and also transposed, as bf16 [sequence][head][rope_hd][position], at rope_out16 (rows of positions padded with
@@ -355,6 +355,11 @@ struct GemmDesc {
   uint16_t *rope_out16[3];
   const float *rope_cos[3], *rope_sin[3];
   int64_t rope_cs_ss[3];
+  // ... heads of 256 (256 x 256 tiles only), rope_norm[p] != 0: every head's row is RMS-normed in front of its rotation, the arithmetic
+  // of rmsnorm_kernel - x / sqrt(sum(x * x) / rope_n_as_float + rope_eps) * (rope_gamma_offset + rope_gamma), gamma: rope_hd floats or null
+  int32_t rope_norm[3];
+  const float *rope_gamma[3];
+  float rope_n_as_float[3], rope_eps[3], rope_gamma_offset[3];
   // optional (the direct-to-LDS bf16 GEMM, for the clock probe): every workgroup adds the shader-clock ticks and
   // the 100 MHz ticks its main loop took to clock_ticks[0] and [1]
   unsigned long long *clock_ticks;

@@ -527,6 +527,7 @@ struct RopeGemmRequest {
   uint16_t *out16[3] = {nullptr, nullptr, nullptr};  // their bf16 copies (optional); [2]: v as [sequences][heads][head_dim][positions]
   const float *cos[2] = {nullptr, nullptr}, *sin[2] = {nullptr, nullptr};
   int64_t cs_ss[2] = {0, 0};
+  const RmsNormMatch *norm[2] = {nullptr, nullptr};  // the norm in front of the rotation (its gamma realised), or none
   uint32_t positions = 0, head_dim = 0;
   bool applied = false;
 };

@@ -584,21 +584,34 @@ int rope_operands(cg_backend *be, const RopeMatch &m, bool *ok) {
 // transpose and the rotation.  When the rotated tensor of `m` is such a norm, still deferred and read by nothing
 // but the rotation, the rotation's kernel can norm each row on its way in: *out says so and holds what it reads
 // (the norm's input as a [b, h, s, d] view, realised here, and gamma).  out->on = false: not that shape.
-static int rope_normed_input(cg_backend *be, cg_tensor *root, const RopeMatch &m, RopeNormed *out) {
-  *out = RopeNormed();
-  if (be->flags & CG_FLAG_NO_PATTERNS) return CG_OK;
+// The match alone: *norm's input is reshapes of `*view`, [b, h, s, d]; *sole: the norm is what reads it, and nothing else.
+static bool match_rope_normed(cg_tensor *root, const RopeMatch &m, RmsNormMatch *norm, cg_tensor **view, bool *sole) {
   const int64_t n = root->shape[3];
-  if ((n != 64 && n != 128 && n != 256) || m.x->op == N_REAL || refs(m.x) != 3) return CG_OK;
+  if ((n != 64 && n != 128 && n != 256) || m.x->op == N_REAL || refs(m.x) != 3) return false;
   cg_tensor *t = m.x;
   while (t->op == N_RESHAPE && t->in[0] && (t == m.x || refs(t) == 1) && t->in[0]->rank >= 1 &&
          t->in[0]->shape[t->in[0]->rank - 1] == n)
     t = t->in[0];
-  if (t->op == N_REAL || (t != m.x && refs(t) != 1)) return CG_OK;
+  if (t->op == N_REAL || (t != m.x && refs(t) != 1)) return false;
+  if (!match_rmsnorm(t, norm)) return false;
+  cg_tensor *v = norm->x;
+  *sole = refs(v) == 3;  // (squared, and divided)
+  while (v->op == N_RESHAPE && v->in[0] && v->in[0]->rank >= 1 && v->in[0]->shape[v->in[0]->rank - 1] == n) {
+    v = v->in[0];
+    *sole = *sole && refs(v) == 1;
+  }
+  if (v->rank != 4 || !std::equal(v->shape, v->shape + 4, root->shape) || v->dtype != CG_F32) return false;
+  *view = v;
+  return true;
+}
+
+static int rope_normed_input(cg_backend *be, cg_tensor *root, const RopeMatch &m, RopeNormed *out) {
+  *out = RopeNormed();
+  if (be->flags & CG_FLAG_NO_PATTERNS) return CG_OK;
   RmsNormMatch rm;
-  if (!match_rmsnorm(t, &rm)) return CG_OK;
-  cg_tensor *v = rm.x;
-  while (v->op == N_RESHAPE && v->in[0] && v->in[0]->rank >= 1 && v->in[0]->shape[v->in[0]->rank - 1] == n) v = v->in[0];
-  if (v->rank != 4 || !std::equal(v->shape, v->shape + 4, root->shape) || v->dtype != CG_F32) return CG_OK;
+  cg_tensor *v = nullptr;
+  bool sole = false;
+  if (!match_rope_normed(root, m, &rm, &v, &sole)) return CG_OK;
   if (rm.gamma) {
     bool vec = false;
     TRY(gamma_row_vector(be, rm.gamma, &vec));
@@ -718,7 +731,7 @@ int try_rope_pair(cg_backend *be, cg_tensor *rq, cg_tensor *rk, bool *done) {
   for (int i = 0; i < 2 && !st && ok; ++i) {
     st = alloc_result(be, roots[i], ST_F32);
     uint16_t *y16 = nullptr;
-    if (!st) st = twin_for_result(be, roots[i], &y16);
+    if (!st && i) st = twin_for_result(be, roots[i], &y16);  // (the attention reads its queries as f32)
     if (!st) st = rope_describe(be, roots[i], *ms[i], (float *)roots[i]->st->ptr, roots[i]->strides, y16, &d[i], &xs[i], &ok, &norms[i]);
   }
   if (!st && ok) {
@@ -745,7 +758,8 @@ int try_rope_pair(cg_backend *be, cg_tensor *rq, cg_tensor *rk, bool *done) {
 // three linears on one input - with or without a bias -, `reshape [b, s, heads, d]`, `transpose(1, 2)`, then
 // apply_rope_embedding on q and k): the grouped launch of the three products rotates q and k where they are still
 // accumulators and stores a transposed bf16 copy of v beside v itself, so neither the rotation nor the
-// transposition is a launch of its own.  Heads of 64 or 128 columns; the linears see the batch folded into the rows.
+// transposition is a launch of its own.  Heads of 64, 128 or 256 columns - of 256 also with the RMS norm of every head's row between
+// the head transpose and the rotation (gemma3.rs:99-117) -; the linears see the batch folded into the rows.
 // *done = false: nothing was changed beyond realising the products.  On success *vt owns the transposed values
 // ([sequences][kv heads][d][positions], bf16) of the storage *v_st.
 int try_qkv_rope_gemm(cg_backend *be, cg_tensor *rq, cg_tensor *rk, cg_tensor *v, Storage **vt, const Storage **v_st,
@@ -758,7 +772,24 @@ int try_qkv_rope_gemm(cg_backend *be, cg_tensor *rq, cg_tensor *rk, cg_tensor *v
   RopeMatch mq, mk;
   if (!match_rope(rq, &mq) || !match_rope(rk, &mk)) return CG_OK;
   const int64_t hd = rq->shape[3];
-  if (hd != 64 && hd != 128) return CG_OK;
+  if (hd != 64 && hd != 128 && hd != 256) return CG_OK;
+  RmsNormMatch norms[2];
+  cg_tensor *xs[2] = {mq.x, mk.x};
+  bool sole[2] = {false, false}, normed = false;
+  int readers[2] = {3, 3};
+  if (hd == 256) {
+    const bool nq = match_rope_normed(rq, mq, &norms[0], &xs[0], &sole[0]), nk = match_rope_normed(rk, mk, &norms[1], &xs[1], &sole[1]);
+    if (nq != nk || (nq && (!sole[0] || !sole[1]))) return CG_OK;
+    normed = nq;
+    for (int i = 0; i < 2 && normed; ++i) {
+      readers[i] = xs[i] == norms[i].x ? 3 : 1;
+      if (norms[i].gamma) {
+        bool vec = false;
+        TRY(gamma_row_vector(be, norms[i].gamma, &vec));
+        if (!vec) return CG_OK;
+      }
+    }
+  }
   // x = transpose(1, 2) of reshapes of a deferred product [1, b * s, heads * hd], or of that product plus its bias
   // vector; `readers`: the references x must have (the rotation reads it three times and nobody else may: its
   // product is never stored as such), 0 = any.  *top: the node whose realisation launches the product.
@@ -774,7 +805,7 @@ int try_qkv_rope_gemm(cg_backend *be, cg_tensor *rq, cg_tensor *rk, cg_tensor *v
     return t;
   };
   cg_tensor *top_q = nullptr, *top_k = nullptr, *top_v = nullptr;
-  cg_tensor *pq = product_under(mq.x, 3, &top_q), *pk = product_under(mk.x, 3, &top_k), *pv = product_under(v, 0, &top_v);
+  cg_tensor *pq = product_under(xs[0], readers[0], &top_q), *pk = product_under(xs[1], readers[1], &top_k), *pv = product_under(v, 0, &top_v);
   if (!pq || !pk || !pv || pq == pk || pq == pv || pk == pv) return CG_OK;
   const int64_t positions = rq->shape[2], seqs = rq->shape[0];
   if (rk->shape[2] != positions || rk->shape[0] != seqs || v->shape[2] != positions || v->shape[0] != seqs ||
@@ -790,12 +821,13 @@ int try_qkv_rope_gemm(cg_backend *be, cg_tensor *rq, cg_tensor *rk, cg_tensor *v
   int st = CG_OK;
   for (int i = 0; i < 2 && !st; ++i) {
     st = alloc_result(be, roots[i], ST_F32);
-    if (!st) st = twin_for_result(be, roots[i], &req.out16[i]);
+    if (!st && i) st = twin_for_result(be, roots[i], &req.out16[i]);  // (the attention reads its queries as f32)
     if (!st) {
       req.out[i] = (float *)roots[i]->st->ptr;
       req.cos[i] = (const float *)data_ptr(ms[i]->cb);
       req.sin[i] = (const float *)data_ptr(ms[i]->sb);
       req.cs_ss[i] = positions == 1 ? 0 : ms[i]->cb->strides[2];
+      req.norm[i] = normed ? &norms[i] : nullptr;
     }
   }
   Storage *t = nullptr;

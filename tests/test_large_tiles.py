@@ -11,7 +11,7 @@ import test_moe_gemma_parity as moe_tests
 import vectors
 from test_f32_tiles import assert_infinities, with_infinities
 
-lang, nn = vectors.cg.lang, vectors.cg.nn
+lang, nn, helpers = vectors.cg.lang, vectors.cg.nn, moe_tests.llm.helpers
 
 
 def draw(g, shape, std=1.0):
@@ -186,6 +186,63 @@ def test_rotated(oracle, hip_bf16, tokens):
 @pytest.mark.parametrize("batch,tokens", [(2, 301), (3, 550), (1, 317), (2, 65)])
 def test_rotated_wide_heads(oracle, hip_bf16, batch, tokens):
     moe_tests.test_qwen_prefill_biases_and_rotation_in_the_projections_launch(oracle, hip_bf16, batch, tokens, 8, 8, 128)
+
+
+# q / k / v that leave a 256 x 256 tile rotated: heads of 64, 128 and 256, with biases, with a norm of every head's row in front of the
+# rotation; one sequence that ends inside a tile, several whose length is no multiple of four (pieces of values that straddle two), of eight
+@pytest.mark.gpu
+@pytest.mark.parametrize("hd,batch,S,heads,kv,K,bias,norm", [(64, 1, 2203, 20, 20, 768, False, False), (64, 8, 276, 20, 20, 768, True, False),
+                                                             (128, 5, 271, 16, 16, 768, True, False), (128, 1, 1302, 16, 16, 832, False, False),
+                                                             (256, 21, 257, 4, 1, 192, False, True), (256, 129, 64, 2, 1, 128, False, True),
+                                                             (256, 20, 270, 4, 1, 128, False, False)])
+def test_rotated_on_large_tiles(hip_bf16, hd, batch, S, heads, kv, K, bias, norm):
+    g = np.random.default_rng(S)
+    x, ns = draw(g, (1, batch * S, K)), [heads * hd, kv * hd, kv * hd]
+    ws, bs = [draw(g, (n, K), K ** -0.5) for n in ns], [g.standard_normal(n).astype(np.float32) for n in ns]
+    gammas = [(0.3 * g.standard_normal(hd)).astype(np.float32) for _ in range(2)]
+    h, theta, eps = helpers, 10000.0, 1e-6
+
+    def normed(b, gamma, n_heads, y):   # (gemma3.rs:41-68, folded as in gemma3.rs:99-117)
+        y = lang.reshape(b, lang.make_shape(b, batch * n_heads * S, hd), y)
+        s = lang.sum(b, y * y)
+        mean = s / lang.broadcast(b, lang.cast(b, lang.nat_to_u32(b, lang.to_nat(b, hd)), lang.dtype(b, y)), lang.shape(b, s))
+        rms = nn.sqrt(b, mean + lang.constant(b, eps, lang.shape(b, mean)))
+        y = y / lang.broadcast(b, rms, lang.shape(b, y))
+        gm = lang.broadcast(b, gamma, lang.shape(b, y))
+        y = y * (lang.constant(b, 1.0, lang.shape(b, gm)) + gm)
+        return lang.reshape(b, lang.make_shape(b, batch, n_heads, S, hd), y)
+
+    def f(b, x, *p):
+        x = x + x - x
+        y = [linear(b, x, p[i], ns[i], K, p[3 + i] if bias else None) for i in range(3)]
+        y = [lang.transpose(b, 1, 2, lang.reshape(b, lang.make_shape(b, batch, S, n // hd, hd), t)) for n, t in zip(ns, y)]
+        q, k, v = y if not norm else [normed(b, p[6], heads, y[0]), normed(b, p[7], kv, y[1]), y[2]]
+        q, k = h.rope(b, theta, 0, S, hd, q), h.rope(b, theta, 0, S, hd, k)
+        attn = lang.matmul(b, q, lang.transpose(b, 2, 3, h.repeat_kv(b, heads // kv, k)))
+        sh = lang.shape(b, attn)
+        attn = attn / lang.constant(b, float(np.sqrt(np.float32(hd))), sh) + lang.broadcast(b, h.causal_mask(b, lang.to_nat(b, S)), sh)
+        return [lang.matmul(b, nn.softmax(b, attn), h.repeat_kv(b, heads // kv, v)), k, v]
+    hip_bf16.trace(2)
+    hip_bf16.trace_reset()
+    got, k, v = vectors.run(hip_bf16, f, 3, x, *ws, *bs, *gammas)
+    names = sorted(hip_bf16.trace_report())
+    hip_bf16.trace(False)
+    assert sum("grouped,rope" in n for n in names) == 1 and not any(n.startswith(("rope_fused", "transpose_cast_bf16")) for n in names), names
+    c, s = (t.astype(np.float64) for t in vectors.run(hip_bf16, lambda b, _: h.rope_tables(b, theta, lang.to_nat(b, S), hd), 2, np.zeros(1, np.float32)))
+    y = [x[0].astype(np.float64) @ w.T.astype(np.float64) + (v64 if bias else 0.0) for w, v64 in zip(ws, bs)]
+    y = [t.reshape(batch, S, -1, hd).transpose(0, 2, 1, 3) for t in y]
+    if norm:
+        for i in range(2):
+            y[i] = y[i] / np.sqrt(np.mean(y[i] ** 2, axis=-1, keepdims=True) + eps) * (1.0 + gammas[i].astype(np.float64))
+    for i in range(2):
+        y[i] = c * y[i] + s * np.concatenate([-y[i][..., hd // 2:], y[i][..., :hd // 2]], axis=-1)
+    parity.assert_f32(y[1], k, "rotated keys")
+    parity.assert_f32(y[2], v, "values")
+    keys, values = (np.repeat(t, heads // kv, axis=1).astype(np.float32) for t in y[1:])
+    scores = (y[0].astype(np.float32) @ keys.transpose(0, 1, 3, 2)) / np.sqrt(np.float32(hd))
+    scores = np.where(np.tri(S, dtype=bool), scores, -np.inf)
+    scores = np.exp(scores - scores.max(axis=-1, keepdims=True))
+    parity.assert_bf16((scores / scores.sum(axis=-1, keepdims=True)) @ values, got, "attention")
 
 
 # the routed experts of a prefill, from 44 pairs to an expert on moe_ring_kernel: three slots whose choices crowd one expert (several row tiles, the last
