@@ -250,6 +250,7 @@ __device__ __forceinline__ float attn_softmax_step(const AttnPrefillDesc &a, a_f
 // KG = 2: half of the waves share their queries with the other half and take every other live step of them, with tiles of their own;
 // the partial results meet once, in LDS.  The longest query tile of a causal mask is then half as long.
 // DS = 2: two waves share 32 queries, each with half of the values' dims.
+// LEAN: bf16 in and out (AttnPrefillDesc::q16), for a result that only products read.
 // Workgroups: the query tiles with the most keys first (a causal mask gives the last tile all of them), and the heads of a
 // (batch, kv head) on one XCD, whose L2 then holds their keys and values.
 // (the register budget of two waves to a SIMD keeps the accumulators of heads of 64 and 128 out of the accumulation file,
@@ -257,7 +258,7 @@ __device__ __forceinline__ float attn_softmax_step(const AttnPrefillDesc &a, a_f
 // step take turns between accumulators: 2900 tokens of 32 heads, causal, 90 us a layer where two waves and one chain after the
 // other took 97, 4000 tokens 131 for 154)
 #define ATTN_WAVES(n) __attribute__((amdgpu_waves_per_eu(n, n)))
-template <int D, int BN, int NW, int KG = 1, int DS = 1>
+template <int D, int BN, int NW, int KG = 1, int DS = 1, bool LEAN = false>
 __global__ void __launch_bounds__(NW * 64) ATTN_WAVES((D == 64 && NW == 4 && (KG == 1 || BN == 32) ? 3 : 2)) attn_prefill_kernel(AttnPrefillDesc a) {
   warm_kernel_arguments<sizeof(AttnPrefillDesc)>();
   constexpr int NT = NW * 64 / KG, NQ = NW / KG / DS, QROWS = NQ * 32;  // threads of a key group; query groups, queries of the workgroup
@@ -280,7 +281,7 @@ __global__ void __launch_bounds__(NW * 64) ATTN_WAVES((D == 64 && NW == 4 && (KG
   const uint32_t query = q_tile * QROWS + wave * 32 + col;
   const bool q_ok = query < a.s;
   const uint32_t qc = q_ok ? query : a.s - 1;  // loads of lanes past the end go to a valid row
-  const float *Q = a.q + (int64_t)b * a.q_sb + (int64_t)h * a.q_sh + (int64_t)qc * a.q_ss;
+  const int64_t q_at = (int64_t)b * a.q_sb + (int64_t)h * a.q_sh + (int64_t)qc * a.q_ss;
   // K rows as bf16 (the twin of the rotated keys), V as bf16 V^T [b, kv, d, T]: both were narrowed
   // once, not once per query block
   const uint16_t *K = a.k16 + (int64_t)b * a.k_sb + (int64_t)kvh * a.k_skv + (int64_t)rp * a.k_srep;
@@ -297,11 +298,16 @@ __global__ void __launch_bounds__(NW * 64) ATTN_WAVES((D == 64 && NW == 4 && (KG
   KeyTiles<BN> tiles(a, q_tile, lane);
   // this lane's query row as B fragments: k-step ks covers dims 16 ks .. 16 ks + 15, half h takes 8 (lanes past the end repeat the
   // last row; what they compute goes nowhere)
-  float4 qx[D / 8];
+  float4 qx[LEAN ? 1 : D / 8];
+  a_bf16x8 qf[D / 16];
 #pragma unroll
   for (int ks = 0; ks < D / 16; ++ks) {
-    qx[2 * ks] = *(const float4 *)(Q + ks * 16 + half * 8);
-    qx[2 * ks + 1] = *(const float4 *)(Q + ks * 16 + half * 8 + 4);
+    if constexpr (LEAN) {
+      qf[ks] = *(const a_bf16x8 *)(a.q16 + q_at + ks * 16 + half * 8);
+    } else {
+      qx[2 * ks] = *(const float4 *)(a.q + q_at + ks * 16 + half * 8);
+      qx[2 * ks + 1] = *(const float4 *)(a.q + q_at + ks * 16 + half * 8 + 4);
+    }
   }
   tiles.arrived(lane);
   constexpr int KROWS = NT * 8 / D, VROWS = NT * 8 / BN;  // rows of the K tile, of the V^T tile, between a thread's chunks
@@ -338,12 +344,13 @@ __global__ void __launch_bounds__(NW * 64) ATTN_WAVES((D == 64 && NW == 4 && (KG
   uint32_t t0 = tiles.skip(tiles.next_step(0), kg), t_next = a.t;
   if (t0 < a.t) fetch(t0);  // (uniform)
 
-  a_bf16x8 qf[D / 16];
+  if constexpr (!LEAN) {
 #pragma unroll
-  for (int ks = 0; ks < D / 16; ++ks) {
-    const float4 x0 = qx[2 * ks], x1 = qx[2 * ks + 1];
-    const float v[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
-    qf[ks] = pack8(v);
+    for (int ks = 0; ks < D / 16; ++ks) {
+      const float4 x0 = qx[2 * ks], x1 = qx[2 * ks + 1];
+      const float v[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
+      qf[ks] = pack8(v);
+    }
   }
   a_f32x16 o[DT];
 #pragma unroll
@@ -472,8 +479,8 @@ __global__ void __launch_bounds__(NW * 64) ATTN_WAVES((D == 64 && NW == 4 && (KG
   // ---- normalise and store: O^T register e of tile t is dim t*32 + (e>>2)*8 + half*4 + (e&3)
   if (q_ok) {
     const int64_t o_off = (int64_t)b * a.o_sb + (int64_t)h * a.o_sh + (int64_t)query * a.o_ss;
-    float *out = a.out + o_off;
-    uint16_t *out16 = a.out16 ? a.out16 + o_off : nullptr;
+    float *out = LEAN ? nullptr : a.out + o_off;
+    uint16_t *out16 = LEAN || a.out16 ? a.out16 + o_off : nullptr;
 #pragma unroll
     for (int t = 0; t < DT; ++t)
 #pragma unroll
@@ -482,8 +489,8 @@ __global__ void __launch_bounds__(NW * 64) ATTN_WAVES((D == 64 && NW == 4 && (KG
         r.x = o[t][j * 4 + 0] / l_run; r.y = o[t][j * 4 + 1] / l_run;
         r.z = o[t][j * 4 + 2] / l_run; r.w = o[t][j * 4 + 3] / l_run;
         const int dim = dim0 + t * 32 + j * 8 + half * 4;
-        *(float4 *)(out + dim) = r;
-        if (out16) *(uint2 *)(out16 + dim) = bf16_pack4(r);
+        if (!LEAN) *(float4 *)(out + dim) = r;
+        if (LEAN || out16) *(uint2 *)(out16 + dim) = bf16_pack4(r);
       }
   }
 }
@@ -494,7 +501,7 @@ __global__ void __launch_bounds__(NW * 64) ATTN_WAVES((D == 64 && NW == 4 && (KG
 // the main loop needs no workgroup barrier and the waves' memory waits overlap each other's arithmetic.
 // Each wave ends with its own running maximum, sum and O^T; they meet once, in LDS, and wave 0 merges
 // them (the same rescaling as between two steps of one wave).
-template <int D, int BN, int NW>
+template <int D, int BN, int NW, bool LEAN = false>
 __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))  // two workgroups per CU
 attn_prefill_keysplit_kernel(AttnPrefillDesc a) {
   warm_kernel_arguments<sizeof(AttnPrefillDesc)>();
@@ -526,12 +533,17 @@ attn_prefill_keysplit_kernel(AttnPrefillDesc a) {
   // of every wave fetching every row.  (Rows past the end repeat the last; what they compute goes nowhere.)
   constexpr int QP = D + 8, QC = 32 * D / 8 / (NW * 64);  // row pitch (bf16 elements), pieces of a lane
   float4 qx[QC][2];
+  a_bf16x8 qh[QC];
 #pragma unroll
   for (int c = 0; c < QC; ++c) {
     const int ch = tid + c * NW * 64, r = ch / (D / 8), d8 = (ch % (D / 8)) * 8;
-    const float *qr = a.q + (int64_t)b * a.q_sb + (int64_t)h * a.q_sh + (int64_t)min(blockIdx.x * 32 + r, a.s - 1) * a.q_ss + d8;
-    qx[c][0] = *(const float4 *)qr;
-    qx[c][1] = *(const float4 *)(qr + 4);
+    const int64_t at = (int64_t)b * a.q_sb + (int64_t)h * a.q_sh + (int64_t)min(blockIdx.x * 32 + r, a.s - 1) * a.q_ss + d8;
+    if constexpr (LEAN) {
+      qh[c] = *(const a_bf16x8 *)(a.q16 + at);
+    } else {
+      qx[c][0] = *(const float4 *)(a.q + at);
+      qx[c][1] = *(const float4 *)(a.q + at + 4);
+    }
   }
   tiles.arrived(lane);
   auto step_mask = [&](uint32_t t0) { return M && tiles.reads_mask(t0); };
@@ -553,8 +565,12 @@ attn_prefill_keysplit_kernel(AttnPrefillDesc a) {
 #pragma unroll
   for (int c = 0; c < QC; ++c) {
     const int ch = tid + c * NW * 64, r = ch / (D / 8), d8 = (ch % (D / 8)) * 8;
-    const float v[8] = {qx[c][0].x, qx[c][0].y, qx[c][0].z, qx[c][0].w, qx[c][1].x, qx[c][1].y, qx[c][1].z, qx[c][1].w};
-    *(a_bf16x8 *)(&qs[r * QP + d8]) = pack8(v);
+    if constexpr (LEAN) {
+      *(a_bf16x8 *)(&qs[r * QP + d8]) = qh[c];
+    } else {
+      const float v[8] = {qx[c][0].x, qx[c][0].y, qx[c][0].z, qx[c][0].w, qx[c][1].x, qx[c][1].y, qx[c][1].z, qx[c][1].w};
+      *(a_bf16x8 *)(&qs[r * QP + d8]) = pack8(v);
+    }
   }
   __syncthreads();
   a_bf16x8 qf[D / 16];
@@ -682,8 +698,8 @@ attn_prefill_keysplit_kernel(AttnPrefillDesc a) {
   }
   if (q_ok) {
     const int64_t o_off = (int64_t)b * a.o_sb + (int64_t)h * a.o_sh + (int64_t)query * a.o_ss;
-    float *out = a.out + o_off;
-    uint16_t *out16 = a.out16 ? a.out16 + o_off : nullptr;
+    float *out = LEAN ? nullptr : a.out + o_off;
+    uint16_t *out16 = LEAN || a.out16 ? a.out16 + o_off : nullptr;
     const float inv_l = 1.0f / l_run;  // bf16 products: a reciprocal and a product, not 64 quotients
 #pragma unroll
     for (int t = 0; t < DT; ++t)
@@ -693,8 +709,8 @@ attn_prefill_keysplit_kernel(AttnPrefillDesc a) {
         r.x = o[t][j * 4 + 0] * inv_l; r.y = o[t][j * 4 + 1] * inv_l;
         r.z = o[t][j * 4 + 2] * inv_l; r.w = o[t][j * 4 + 3] * inv_l;
         const int dim = t * 32 + j * 8 + half * 4;
-        *(float4 *)(out + dim) = r;
-        if (out16) *(uint2 *)(out16 + dim) = bf16_pack4(r);
+        if (!LEAN) *(float4 *)(out + dim) = r;
+        if (LEAN || out16) *(uint2 *)(out16 + dim) = bf16_pack4(r);
       }
   }
 }
@@ -1049,24 +1065,30 @@ hipError_t launch_attn_prefill(const LaunchCtx &lc, const AttnPrefillDesc &d) {
   if (!d.b || !d.heads || !d.s) return hipSuccess;
   if (d.f32 ? !d.k : (!d.k16 || !d.vt16 || d.vt_st < d.t || d.vt_st % 8)) return hipErrorInvalidValue;
   if (d.mask && (d.m_len < d.t || d.m_len % 4)) return hipErrorInvalidValue;
+  if (d.q16 ? d.f32 || !d.out16 : !d.q || !d.out) return hipErrorInvalidValue;
+#define CG_ATTN(kernel, grid, block, ...)                                            \
+  do {                                                                               \
+    if (d.q16) CG_LAUNCH(lc, (kernel<__VA_ARGS__, true>), grid, block, d);           \
+    else CG_LAUNCH(lc, (kernel<__VA_ARGS__, false>), grid, block, d);                \
+  } while (0)
   if (attn_prefill_keysplit(lc, d)) {
     dim3 g32((d.s + 31) / 32, d.heads, d.b);
-    CG_LAUNCH(lc, (attn_prefill_keysplit_kernel<64, 64, 4>), g32, 256, d);
+    CG_ATTN(attn_prefill_keysplit_kernel, g32, 256, 64, 64, 4);
     return hipGetLastError();
   }
   if (attn_prefill_two_groups(lc, d)) {
     const uint32_t grid = (d.s + 63) / 64 * d.heads * d.b;
-    if (attn_prefill_two_groups_keys(lc, d) == 32) CG_LAUNCH(lc, (attn_prefill_kernel<64, 32, 4, 2>), grid, 256, d);
-    else CG_LAUNCH(lc, (attn_prefill_kernel<64, 64, 4, 2>), grid, 256, d);
+    if (attn_prefill_two_groups_keys(lc, d) == 32) CG_ATTN(attn_prefill_kernel, grid, 256, 64, 32, 4, 2, 1);
+    else CG_ATTN(attn_prefill_kernel, grid, 256, 64, 64, 4, 2, 1);
     return hipGetLastError();
   }
   if (attn_prefill_wide(lc, d)) {
     const int groups = attn_prefill_wide_groups(lc, d);
     const uint32_t bh = d.heads * d.b, g32 = (d.s + 31) / 32 * bh, g64 = (d.s + 63) / 64 * bh;
 #define CG_ATTN_WIDE(DD, BN)                                                                        \
-    if (groups == 32) CG_LAUNCH(lc, (attn_prefill_kernel<DD, BN, 4, 2, 2>), g32, 256, d);           \
-    else if (groups == 64) CG_LAUNCH(lc, (attn_prefill_kernel<DD, BN, 8, 2, 2>), g64, 512, d);      \
-    else CG_LAUNCH(lc, (attn_prefill_kernel<DD, BN, 4, 1, 2>), g64, 256, d);
+    if (groups == 32) CG_ATTN(attn_prefill_kernel, g32, 256, DD, BN, 4, 2, 2);           \
+    else if (groups == 64) CG_ATTN(attn_prefill_kernel, g64, 512, DD, BN, 8, 2, 2);      \
+    else CG_ATTN(attn_prefill_kernel, g64, 256, DD, BN, 4, 1, 2);
     if (d.d == 128) { CG_ATTN_WIDE(128, 64) }
     else { CG_ATTN_WIDE(256, 32) }
 #undef CG_ATTN_WIDE
@@ -1089,12 +1111,13 @@ hipError_t launch_attn_prefill(const LaunchCtx &lc, const AttnPrefillDesc &d) {
     }
   } else {
     switch (d.d) {
-      case 64: CG_LAUNCH(lc, (attn_prefill_kernel<64, 64, 4>), grid, 256, d); break;
-      case 128: CG_LAUNCH(lc, (attn_prefill_kernel<128, 64, 4>), grid, 256, d); break;
+      case 64: CG_ATTN(attn_prefill_kernel, grid, 256, 64, 64, 4, 1, 1); break;
+      case 128: CG_ATTN(attn_prefill_kernel, grid, 256, 128, 64, 4, 1, 1); break;
       default: return hipErrorInvalidValue;
     }
   }
 #undef CG_ATTN_CASE
+#undef CG_ATTN
   return hipGetLastError();
 }
 

@@ -1136,7 +1136,7 @@ __device__ __forceinline__ void rope_rows(const RopeDesc &d, uint32_t block, uin
     o.x = c.x * xv.x + sn.x * pv.x; o.y = c.y * xv.y + sn.y * pv.y;
     o.z = c.z * xv.z + sn.z * pv.z; o.w = c.w * xv.w + sn.w * pv.w;
     const int64_t oo = (int64_t)b * d.o_sb + (int64_t)h * d.o_sh + (int64_t)s * d.o_ss + j;
-    *(float4 *)(d.out + oo) = o;
+    if (d.out) *(float4 *)(d.out + oo) = o;
     if (d.out16) *(uint2 *)(d.out16 + oo) = bf16_pack4(o);
   }
 }
@@ -1175,7 +1175,7 @@ __device__ __forceinline__ void rope_norm_rows(const RopeDesc &d, uint32_t block
     o.x = c.x * y.x + sn.x * pv.x; o.y = c.y * y.y + sn.y * pv.y;
     o.z = c.z * y.z + sn.z * pv.z; o.w = c.w * y.w + sn.w * pv.w;
     const int64_t oo = (int64_t)b * d.o_sb + (int64_t)h * d.o_sh + (int64_t)s * d.o_ss + j;
-    *(float4 *)(d.out + oo) = o;
+    if (d.out) *(float4 *)(d.out + oo) = o;
     if (d.out16) *(uint2 *)(d.out16 + oo) = bf16_pack4(o);
   }
 }

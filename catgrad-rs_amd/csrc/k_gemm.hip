@@ -934,7 +934,7 @@ __global__ void __launch_bounds__(WR *WC *KG * 64) gemm_bf16_dma_kernel(GemmDesc
         if (row < g.M) {
           const uint32_t sq = row / S, pos = row - sq * S, head = column(c4) / hd;
           const uint64_t at = (((uint64_t)sq * heads + head) * S + pos) * hd + (column(c4) & (hd - 1));
-          *(float4 *)(g.rope_out[grp] + at) = o;
+          if (g.rope_out[grp]) *(float4 *)(g.rope_out[grp] + at) = o;
           if (g.rope_out16[grp]) *(uint2 *)(g.rope_out16[grp] + at) = bf16_pack4(o);
         }
       }
@@ -3092,8 +3092,8 @@ bool gemm_rope_epilogue_ok(const LaunchCtx &lc, const GemmDesc &g) {
   for (uint32_t p = 0; p < g.n_group; ++p) {
     if (g.grp_n[p] % 128) return false;
     grp256 = grp256 && g.grp_n[p] % 256 == 0;
-    if (g.rope_role[p] == 1) {
-      if (!g.rope_out[p] || !g.rope_cos[p] || !g.rope_sin[p]) return false;
+    if (g.rope_role[p] == 1 || g.rope_role[p] == 3) {
+      if ((!g.rope_out[p] && !g.rope_out16[p]) || !g.rope_cos[p] || !g.rope_sin[p]) return false;
     } else if (g.rope_role[p] == 2) {
       if (!g.rope_out16[p] || (uintptr_t)g.rope_out16[p] % 8 || !g.grp_c[p]) return false;
     } else if (g.rope_role[p] != 0 || !g.grp_c[p]) {

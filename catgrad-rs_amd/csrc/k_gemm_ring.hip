@@ -345,7 +345,7 @@ enum { RING_PLAIN, RING_SIGMOID, RING_SILU, RING_GELU, RING_ROPE_64, RING_ROPE_6
 // wavefront puts its 64 rows of both column halves into LDS - with a bias, or leaving the sums of their squares -, row r's piece of four
 // columns `chunk` of a column half at place chunk ^ (r & 15).
 struct RingRope {  // one group's part of a GemmDesc
-  const float *cos, *sin, *gamma, *bias;
+  const float *cos, *sin, *bias;  // (NORM: bias is the norm's gamma)
   float *out, *c;
   uint16_t *out16;
   int64_t cs_ss;
@@ -419,9 +419,9 @@ __device__ __forceinline__ void ring_store_rotated(const RingRope &d, RingPieces
   float *sums = smem + 32768 + wave * 128;  // NORM: the sums of squares, then each row's divisor and its inverse
   float4 g_lo, g_hi;
   if (NORM) {  // (heads of 256: a row's columns are with two wavefronts)
-    if (d.gamma) {
-      g_lo = *(const float4 *)(d.gamma + p.in_half);
-      g_hi = *(const float4 *)(d.gamma + p.in_half + P::H);
+    if (d.bias) {
+      g_lo = *(const float4 *)(d.bias + p.in_half);
+      g_hi = *(const float4 *)(d.bias + p.in_half + P::H);
     }
     const float sum = sums[lane] + smem[32768 + (wave ^ 1) * 128 + lane];
     __syncthreads();
@@ -450,20 +450,23 @@ __device__ __forceinline__ void ring_store_rotated(const RingRope &d, RingPieces
           const float rms = sums[r], inv = sums[64 + r];
           auto normed = [&](float v, float w) {
             const float q = v * inv, n = fmaf(fmaf(-q, rms, v), inv, q);
-            return d.gamma ? n * (d.gamma_offset + w) : n;
+            return d.bias ? n * (d.gamma_offset + w) : n;
           };
           x = make_float4(normed(x.x, g_lo.x), normed(x.y, g_lo.y), normed(x.z, g_lo.z), normed(x.w, g_lo.w));
           y = make_float4(normed(y.x, g_hi.x), normed(y.y, g_hi.y), normed(y.z, g_hi.z), normed(y.w, g_hi.w));
         }
         const float4 c0 = now[u][0], s0 = now[u][1], c1 = now[u][2], s1 = now[u][3];
-        const float4 l = make_float4(c0.x * x.x + s0.x * -y.x, c0.y * x.y + s0.y * -y.y, c0.z * x.z + s0.z * -y.z, c0.w * x.w + s0.w * -y.w);
-        const float4 h = make_float4(c1.x * y.x + s1.x * x.x, c1.y * y.y + s1.y * x.y, c1.z * y.z + s1.z * x.z, c1.w * y.w + s1.w * x.w);
+        // (the compiler's choice in rope_kernel, which product is rounded on its own, written out: the same bits)
+        const float4 l = make_float4(fmaf(c0.x, x.x, s0.x * -y.x), fmaf(c0.y, x.y, s0.y * -y.y), fmaf(c0.z, x.z, s0.z * -y.z), fmaf(c0.w, x.w, s0.w * -y.w));
+        const float4 h = make_float4(fmaf(c1.x, y.x, s1.x * x.x), fmaf(c1.y, y.y, s1.y * x.y), fmaf(c1.z, y.z, s1.z * x.z), fmaf(c1.w, y.w, s1.w * x.w));
         if (p.row0 + r < d.M) {
           // [sequence][head][position][column]; a position past a sequence's end is the next one's
           const uint32_t head = (n0 + b * 128 + (HD == 64 ? wn * 64 : 0)) / HD, over = p.pos0 + r >= S ? 1 : 0;
           const uint64_t to = ((uint64_t)((p.sq0 + over) * heads + head) * S + (p.pos0 + r - over * S)) * HD + p.in_half;
-          *(float4 *)(d.out + to) = l;
-          *(float4 *)(d.out + to + P::H) = h;
+          if (d.out) {
+            *(float4 *)(d.out + to) = l;
+            *(float4 *)(d.out + to + P::H) = h;
+          }
           if (d.out16) {
             *(uint2 *)(d.out16 + to) = bf16_pack4(l);
             *(uint2 *)(d.out16 + to + P::H) = bf16_pack4(h);
@@ -700,8 +703,8 @@ __global__ void __launch_bounds__(256, 1) gemm_bf16_ring_kernel(GemmDesc g) {
     // (read here, not held through the main loop)
     auto *late = (const __attribute__((address_space(4))) GemmDesc *)__builtin_amdgcn_kernarg_segment_ptr();
     asm volatile("" : "+s"(late));
-    const RingRope d = {late->rope_cos[grp], late->rope_sin[grp], late->rope_gamma[grp], late->grp_bias[grp], late->rope_out[grp], late->grp_c[grp],
-                        late->rope_out16[grp], late->rope_cs_ss[grp], late->rope_n_as_float[grp], late->rope_eps[grp], late->rope_gamma_offset[grp],
+    const RingRope d = {late->rope_cos[grp], late->rope_sin[grp], late->grp_bias[grp], late->rope_out[grp], late->grp_c[grp],
+                        late->rope_out16[grp], late->rope_cs_ss[grp], late->rope_n_as_float, late->rope_eps, late->rope_gamma_offset,
                         late->M, late->grp_n[grp], late->rope_s};
     constexpr int HD = KIND >= RING_ROPE_256 ? 256 : KIND >= RING_ROPE_128 ? 128 : 64;
     ring_store_attention<HD, KIND == RING_ROPE_64_BIAS || KIND == RING_ROPE_128_BIAS, KIND == RING_ROPE_256_NORM>(d, late->rope_role[grp] == 2, m0, n0, acc, ring_smem);
@@ -1002,8 +1005,11 @@ static bool gemm_ring_rope_ok(const GemmDesc &g) {
   if (!g.n_group || g.splits > 1 || g.rope_s < 64 || (g.rope_hd != 64 && g.rope_hd != 128 && g.rope_hd != 256)) return false;
   bool norm = false, plain = false;
   for (uint32_t p = 0; p < g.n_group; ++p) {
-    if (!g.rope_role[p] || g.grp_n[p] % 256 || !g.grp_bias[p] != !g.grp_bias[0] || (g.grp_bias[p] && g.rope_hd == 256)) return false;
-    if (g.rope_role[p] == 1) (g.rope_norm[p] ? norm : plain) = true;
+    if (!g.rope_role[p] || g.grp_n[p] % 256) return false;
+    if (g.rope_role[p] != 3 && g.grp_bias[p] && g.rope_hd == 256) return false;
+    if (g.rope_hd != 256 && !g.grp_bias[p] != !g.grp_bias[0]) return false;
+    norm = norm || g.rope_role[p] == 3;
+    plain = plain || g.rope_role[p] == 1;
   }
   return !norm || (!plain && g.rope_hd == 256);
 }
@@ -1045,7 +1051,7 @@ hipError_t launch_gemm_ring(const LaunchCtx &lc, const GemmDesc &g, bool half_he
   if (g.rope_s) {
     if (wide) return hipErrorInvalidValue;
     const bool bias = g.grp_bias[0] != nullptr;
-    if (g.rope_hd == 256) return g.rope_norm[0] || g.rope_norm[1] || g.rope_norm[2] ? launch_ring_as<RING_ROPE_256_NORM>(lc, g, (uint32_t)grid) : launch_ring_as<RING_ROPE_256>(lc, g, (uint32_t)grid);
+    if (g.rope_hd == 256) return g.rope_role[0] == 3 || g.rope_role[1] == 3 || g.rope_role[2] == 3 ? launch_ring_as<RING_ROPE_256_NORM>(lc, g, (uint32_t)grid) : launch_ring_as<RING_ROPE_256>(lc, g, (uint32_t)grid);
     if (g.rope_hd == 128) return bias ? launch_ring_as<RING_ROPE_128_BIAS>(lc, g, (uint32_t)grid) : launch_ring_as<RING_ROPE_128>(lc, g, (uint32_t)grid);
     return bias ? launch_ring_as<RING_ROPE_64_BIAS>(lc, g, (uint32_t)grid) : launch_ring_as<RING_ROPE_64>(lc, g, (uint32_t)grid);
   }

@@ -171,7 +171,7 @@ struct RopeDesc {
   float *out;            // [b, h, s, dim] through o_sb / o_sh / o_ss (e.g. a slot of the KV cache)
   int64_t x_sb, x_sh, x_ss, cs_ss;  // element strides (unit stride along dim everywhere)
   int64_t o_sb, o_sh, o_ss;
-  uint16_t *out16;       // optional bf16 copy, same layout as out, or null
+  uint16_t *out16;       // optional bf16 copy, same layout as out, or null (either may be)
   uint32_t b, h, s, dim, half;
   // optional (norm != 0, dim 64, 128 or 256): every row of x is RMS-normed first, the arithmetic of rmsnorm_kernel -
   // x / sqrt(sum(x * x) / n_as_float + eps) * (gamma_offset + gamma), gamma: dim floats or null
@@ -260,6 +260,8 @@ hipError_t launch_attn_decode(const LaunchCtx &lc, const AttnDecodeDesc &d);
 struct AttnPrefillDesc {
   const float *q, *v, *mask;
   const uint16_t *k16, *vt16;          // bf16 products: keys as bf16 rows, values as bf16 V^T [b, kv, d, T]
+  // bf16 products, optional: the queries as bf16, through the same strides, in place of q; out is then not written (null), out16 is
+  const uint16_t *q16;
   const float *k;                      // f32 products (f32 != 0): keys as f32 rows; k16 / vt16 unused
   int32_t f32;
   float *out;
@@ -346,7 +348,7 @@ struct GemmDesc {
   // sequences of rope_s positions each (row m = sequence m / rope_s, position m % rope_s) with heads of rope_hd
   // (64, 128 or 256) columns.  A group with rope_role 1 leaves the kernel rotated (apply_rope_embedding, cos / sin
   // rows of rope_hd floats at rope_cs_ss apart, indexed by position) as [sequence][head][position][rope_hd] at
-  // rope_out (f32) and rope_out16 (bf16, optional) instead of grp_c; a group with rope_role 2 is stored as usual
+  // rope_out (f32) and rope_out16 (bf16), either optional, instead of grp_c; a group with rope_role 2 is stored as usual
   // and also transposed, as bf16 [sequence][head][rope_hd][position], at rope_out16 (rows of positions padded with
   // zeros to a multiple of 8).
   uint32_t rope_s, rope_hd;
@@ -355,15 +357,16 @@ struct GemmDesc {
   uint16_t *rope_out16[3];
   const float *rope_cos[3], *rope_sin[3];
   int64_t rope_cs_ss[3];
-  // ... heads of 256 (256 x 256 tiles only), rope_norm[p] != 0: every head's row is RMS-normed in front of its rotation, the arithmetic
-  // of rmsnorm_kernel - x / sqrt(sum(x * x) / rope_n_as_float + rope_eps) * (rope_gamma_offset + rope_gamma), gamma: rope_hd floats or null
-  int32_t rope_norm[3];
-  const float *rope_gamma[3];
-  float rope_n_as_float[3], rope_eps[3], rope_gamma_offset[3];
+  // Role 3 (heads of 256, on 256 x 256 tiles only): as 1, every head's row RMS-normed in front of its rotation, the arithmetic of
+  // rmsnorm_kernel - x / sqrt(sum(x * x) / rope_n_as_float + rope_eps) * (rope_gamma_offset + gamma) with gamma, rope_hd floats or null,
+  // in the place of the bias, which it then does not have
+  float rope_n_as_float, rope_eps, rope_gamma_offset;
   // optional (the direct-to-LDS bf16 GEMM, for the clock probe): every workgroup adds the shader-clock ticks and
   // the 100 MHz ticks its main loop took to clock_ticks[0] and [1]
   unsigned long long *clock_ticks;
 };
+// (up to eight lines of 64 bytes a kernel's arguments are touched in one trip: with nine a 37-token prompt took 1242 us, with eight 1218)
+static_assert(sizeof(GemmDesc) <= 512, "a GemmDesc is eight lines of kernel arguments");
 // k_gemm_ring.hip: the 256 x 256 tiles of large bf16 products (plain or grouped, sigmoid, stacked gate / up);
 // half_height: the stacked gate / up of fewer rows on tiles of 128 x 256, K >= 192; wide: tiles of 256 x 288 (plain without groups or a
 // sigmoid, stacked gate / up), N % 4 == 0

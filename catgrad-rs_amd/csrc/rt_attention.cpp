@@ -37,6 +37,9 @@ int try_attn_prefill(cg_backend *be, cg_tensor *n, bool *done) {
   if (f32 && three && !(be->flags & CG_FLAG_ATTN_ONE_PASS)) return CG_OK;
   if (nb > 65535 || heads > 65535) return CG_OK;
   cg_tensor *q = S->in[0];
+  // A result that only a product of many rows reads - through the views that merge the heads - is needed as bf16 only, and so are then
+  // queries that nothing else reads: neither is stored as f32.
+  const bool narrow = !f32 && nb * Sq > 64 && refs(q) == 1 && only_a_product_reads(be, n);
   // queries and keys both still to be rotated: one launch for the two (each alone otherwise, below)
   // (the transposed bf16 values, when the projections' own launch has made them: released on every way out)
   struct Held {
@@ -49,8 +52,8 @@ int try_attn_prefill(cg_backend *be, cg_tensor *n, bool *done) {
   if (cg_tensor *kr = node_under_repeat_kv(S->in[1])) {
     bool paired = false;
     // ... or none at all: the projections still deferred rotate q and k in their epilogue
-    if (!f32) TRY(try_qkv_rope_gemm(be, q, kr, node_under_repeat_kv(n->in[1]), &vt_made.s, &vt_of, &paired));
-    if (!paired) TRY(try_rope_pair(be, q, kr, &paired));
+    if (!f32) TRY(try_qkv_rope_gemm(be, q, kr, node_under_repeat_kv(n->in[1]), narrow, &vt_made.s, &vt_of, &paired));
+    if (!paired) TRY(try_rope_pair(be, q, kr, narrow, &paired));
   }
   MatOperand Kop, Vop;
   bool pk = false, pv = false;
@@ -67,14 +70,16 @@ int try_attn_prefill(cg_backend *be, cg_tensor *n, bool *done) {
     return true;
   };
   if (Kop.shape[2] != Vop.shape[2] || Kop.shape[1] != Vop.shape[1] || Kop.shape[1] * Kop.shape[2] != heads) return CG_OK;
-  if (q->stype != ST_F32 || Kop.t->stype != ST_F32 || Vop.t->stype != ST_F32 || (mask && mask->stype != ST_F32)) return CG_OK;
+  const bool lean = narrow && q->stype == ST_BF16;
+  if ((q->stype != ST_F32 && !lean) || Kop.t->stype != ST_F32 || Vop.t->stype != ST_F32 || (mask && mask->stype != ST_F32)) return CG_OK;
   if (!ok4(data_ptr(q), q->strides[3], {q->strides[0], q->strides[1], q->strides[2]}) ||
       !ok4(data_ptr(Kop.t), Kop.strides[3], {Kop.strides[0], Kop.strides[1], Kop.strides[2], Kop.strides[4]}) ||
       !ok4(data_ptr(Vop.t), Vop.strides[4], {Vop.strides[0], Vop.strides[1], Vop.strides[2], Vop.strides[3]}))
     return CG_OK;
+  if (lean && ((uintptr_t)data_ptr(q) % 16 || q->strides[0] % 8 || q->strides[1] % 8 || q->strides[2] % 8)) return CG_OK;
   // the bf16 keys are read eight at a time
   if (!f32 && (Kop.t->offset % 8 || Kop.strides[0] % 8 || Kop.strides[1] % 8 || Kop.strides[2] % 8 || Kop.strides[4] % 8)) return CG_OK;
-  TRY(alloc_result(be, n, ST_F32));
+  TRY(alloc_result(be, n, lean ? ST_BF16 : ST_F32));
   // The models merge the heads next (`transpose(1, 2)` + `reshape [b, s, heads * d]`, llama.rs:107-109):
   // the result is laid out [b, s, heads, d] in memory and handed back as the [b, heads, s, d] view of
   // it, so that merge is a view and the bf16 twin is already the o_proj operand.
@@ -84,11 +89,16 @@ int try_attn_prefill(cg_backend *be, cg_tensor *n, bool *done) {
   n->strides[3] = 1;
   AttnPrefillDesc a;
   std::memset(&a, 0, sizeof(a));
-  a.q = (const float *)data_ptr(q);
   a.v = (const float *)data_ptr(Vop.t);
-  a.out = (float *)n->st->ptr;
+  if (lean) {
+    a.q16 = (const uint16_t *)data_ptr(q);
+    a.out16 = (uint16_t *)n->st->ptr;
+  } else {
+    a.q = (const float *)data_ptr(q);
+    a.out = (float *)n->st->ptr;
+  }
   a.o_sb = n->strides[0]; a.o_sh = n->strides[1]; a.o_ss = n->strides[2];
-  TRY(twin_for_result(be, n, &a.out16));
+  if (!lean) TRY(twin_for_result(be, n, &a.out16));
   a.q_sb = q->strides[0]; a.q_sh = q->strides[1]; a.q_ss = q->strides[2];
   a.k_sb = Kop.strides[0]; a.k_skv = Kop.strides[1]; a.k_srep = Kop.strides[2]; a.k_st = Kop.strides[4];
   a.v_sb = Vop.strides[0]; a.v_skv = Vop.strides[1]; a.v_srep = Vop.strides[2]; a.v_st = Vop.strides[3];
@@ -202,6 +212,7 @@ int try_attn_prefill(cg_backend *be, cg_tensor *n, bool *done) {
   {
     const double qo = 2.0 * nb * heads * Sq * d * 4, kvb = 2.0 * nb * Kop.shape[1] * T * d * 4;
     KernelScope ks(be, "attn_prefill", qo + kvb + (mask ? (double)Sq * T * 4 : 0.0), 4.0 * nb * heads * Sq * T * d);
+    if (be->trace_shapes && lean) ks.rename("attn_prefill[bf16]");
     hipError_t ae = launch_attn_prefill(be->lc(), a);
     storage_release(vt);
     HIPCHK(be, ae);

@@ -125,8 +125,9 @@ int rope_into(cg_backend *be, cg_tensor *root, const RopeMatch &m, float *out, c
 int try_rope(cg_backend *be, cg_tensor *root, bool *done);
 int rope_describe(cg_backend *be, cg_tensor *root, const RopeMatch &m, float *out, const int64_t *o_strides,
                   uint16_t *out16, RopeDesc *dsc, cg_tensor **xs_out, bool *ok, const RopeNormed *normed = nullptr);
-int try_rope_pair(cg_backend *be, cg_tensor *rq, cg_tensor *rk, bool *done);
-int try_qkv_rope_gemm(cg_backend *be, cg_tensor *rq, cg_tensor *rk, cg_tensor *v, Storage **vt, const Storage **v_st,
+bool only_a_product_reads(cg_backend *be, const cg_tensor *n);
+int try_rope_pair(cg_backend *be, cg_tensor *rq, cg_tensor *rk, bool q_bf16, bool *done);
+int try_qkv_rope_gemm(cg_backend *be, cg_tensor *rq, cg_tensor *rk, cg_tensor *v, bool q_bf16, Storage **vt, const Storage **v_st,
                       bool *done);
 cg_tensor *node_under_repeat_kv(cg_tensor *t);
 bool is_sigmoid_of(const cg_tensor *s, const cg_tensor **arg);

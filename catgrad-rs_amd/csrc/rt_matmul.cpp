@@ -1093,11 +1093,12 @@ int realize_matmul(cg_backend *be, cg_tensor *n, cg_tensor *addend, bool *added,
           t.rope_sin[i] = rq->sin[j];
           t.rope_cs_ss[i] = rq->cs_ss[j];
           if (const RmsNormMatch *nm = rq->norm[j]) {
-            t.rope_norm[i] = 1;
-            t.rope_gamma[i] = nm->gamma ? (const float *)data_ptr(nm->gamma) : nullptr;
-            t.rope_n_as_float[i] = nm->n_as_float;
-            t.rope_eps[i] = nm->eps;
-            t.rope_gamma_offset[i] = nm->gamma_offset;
+            all = !t.grp_bias[i];
+            t.rope_role[i] = 3;
+            t.grp_bias[i] = nm->gamma ? (const float *)data_ptr(nm->gamma) : nullptr;
+            t.rope_n_as_float = nm->n_as_float;
+            t.rope_eps = nm->eps;
+            t.rope_gamma_offset = nm->gamma_offset;
           }
         } else {
           t.rope_role[i] = 2;

@@ -115,6 +115,19 @@ int gemm_readers(cg_backend *be, const cg_tensor *n, bool *all) {
 }
 
 
+// One waiting product of many rows reads n, through reshapes and transpositions that nobody else holds, and nothing else does.
+bool only_a_product_reads(cg_backend *be, const cg_tensor *n) {
+  if (refs(n) != 1) return false;
+  for (const cg_tensor *c : be->gemm_candidates) {
+    if (c->op != N_MATMUL || !c->in[0]) continue;
+    const cg_tensor *a = c->in[0];
+    while (a != n && (a->op == N_RESHAPE || a->op == N_TRANSPOSE) && refs(a) == 1) a = a->in[0];
+    if (a == n) return true;
+  }
+  return false;
+}
+
+
 // a realised f32 tensor usable as contiguous rows: itself or a contiguous copy
 int as_rows(cg_backend *be, cg_tensor *t, cg_tensor **out, int64_t *row_stride) {
   TRY(realize(be, t));
@@ -706,8 +719,9 @@ int rope_into(cg_backend *be, cg_tensor *root, const RopeMatch &m, float *out, c
 }
 
 // The queries and the keys of an attention, both straight from apply_rope_embedding and both still
-// deferred: one launch rotates both.  *done = false: nothing was changed (each is then realised alone).
-int try_rope_pair(cg_backend *be, cg_tensor *rq, cg_tensor *rk, bool *done) {
+// deferred: one launch rotates both.  q_bf16: the queries leave as bf16 only.  *done = false: nothing was changed (each is then realised
+// alone).
+int try_rope_pair(cg_backend *be, cg_tensor *rq, cg_tensor *rk, bool q_bf16, bool *done) {
   *done = false;
   if (be->flags & CG_FLAG_NO_PATTERNS) return CG_OK;
   if (rq == rk || rq->op == N_REAL || rk->op == N_REAL) return CG_OK;
@@ -729,10 +743,12 @@ int try_rope_pair(cg_backend *be, cg_tensor *rq, cg_tensor *rk, bool *done) {
   int st = CG_OK;
   bool ok = true;
   for (int i = 0; i < 2 && !st && ok; ++i) {
-    st = alloc_result(be, roots[i], ST_F32);
+    const bool narrow = q_bf16 && i == 0;
+    st = alloc_result(be, roots[i], narrow ? ST_BF16 : ST_F32);
     uint16_t *y16 = nullptr;
-    if (!st && i) st = twin_for_result(be, roots[i], &y16);  // (the attention reads its queries as f32)
-    if (!st) st = rope_describe(be, roots[i], *ms[i], (float *)roots[i]->st->ptr, roots[i]->strides, y16, &d[i], &xs[i], &ok, &norms[i]);
+    if (!st && narrow) y16 = (uint16_t *)roots[i]->st->ptr;
+    if (!st && i) st = twin_for_result(be, roots[i], &y16);  // (f32 queries are read as such)
+    if (!st) st = rope_describe(be, roots[i], *ms[i], narrow ? nullptr : (float *)roots[i]->st->ptr, roots[i]->strides, y16, &d[i], &xs[i], &ok, &norms[i]);
   }
   if (!st && ok) {
     KernelScope ks(be, "rope_fused", (double)(rq->size() + rk->size()) * 8, 0);
@@ -760,9 +776,9 @@ int try_rope_pair(cg_backend *be, cg_tensor *rq, cg_tensor *rk, bool *done) {
 // accumulators and stores a transposed bf16 copy of v beside v itself, so neither the rotation nor the
 // transposition is a launch of its own.  Heads of 64, 128 or 256 columns - of 256 also with the RMS norm of every head's row between
 // the head transpose and the rotation (gemma3.rs:99-117) -; the linears see the batch folded into the rows.
-// *done = false: nothing was changed beyond realising the products.  On success *vt owns the transposed values
+// q_bf16: the queries leave as bf16 only.  *done = false: nothing was changed beyond realising the products.  On success *vt owns the transposed values
 // ([sequences][kv heads][d][positions], bf16) of the storage *v_st.
-int try_qkv_rope_gemm(cg_backend *be, cg_tensor *rq, cg_tensor *rk, cg_tensor *v, Storage **vt, const Storage **v_st,
+int try_qkv_rope_gemm(cg_backend *be, cg_tensor *rq, cg_tensor *rk, cg_tensor *v, bool q_bf16, Storage **vt, const Storage **v_st,
                       bool *done) {
   *done = false;
   *vt = nullptr;
@@ -781,6 +797,7 @@ int try_qkv_rope_gemm(cg_backend *be, cg_tensor *rq, cg_tensor *rk, cg_tensor *v
     const bool nq = match_rope_normed(rq, mq, &norms[0], &xs[0], &sole[0]), nk = match_rope_normed(rk, mk, &norms[1], &xs[1], &sole[1]);
     if (nq != nk || (nq && (!sole[0] || !sole[1]))) return CG_OK;
     normed = nq;
+    if (normed && (norms[0].n_as_float != norms[1].n_as_float || norms[0].eps != norms[1].eps || norms[0].gamma_offset != norms[1].gamma_offset)) return CG_OK;
     for (int i = 0; i < 2 && normed; ++i) {
       readers[i] = xs[i] == norms[i].x ? 3 : 1;
       if (norms[i].gamma) {
@@ -820,10 +837,12 @@ int try_qkv_rope_gemm(cg_backend *be, cg_tensor *rq, cg_tensor *rk, cg_tensor *v
   const RopeMatch *ms[2] = {&mq, &mk};
   int st = CG_OK;
   for (int i = 0; i < 2 && !st; ++i) {
-    st = alloc_result(be, roots[i], ST_F32);
-    if (!st && i) st = twin_for_result(be, roots[i], &req.out16[i]);  // (the attention reads its queries as f32)
+    const bool narrow = q_bf16 && i == 0;
+    st = alloc_result(be, roots[i], narrow ? ST_BF16 : ST_F32);
+    if (!st && i) st = twin_for_result(be, roots[i], &req.out16[i]);  // (f32 queries are read as such)
     if (!st) {
-      req.out[i] = (float *)roots[i]->st->ptr;
+      if (narrow) req.out16[i] = (uint16_t *)roots[i]->st->ptr;
+      else req.out[i] = (float *)roots[i]->st->ptr;
       req.cos[i] = (const float *)data_ptr(ms[i]->cb);
       req.sin[i] = (const float *)data_ptr(ms[i]->sb);
       req.cs_ss[i] = positions == 1 ? 0 : ms[i]->cb->strides[2];

@@ -245,6 +245,40 @@ def test_rotated_on_large_tiles(hip_bf16, hd, batch, S, heads, kv, K, bias, norm
     parity.assert_bf16((scores / scores.sum(axis=-1, keepdims=True)) @ values, got, "attention")
 
 
+# attention whose result only a product of many rows reads: queries and result as bf16 only.  The product with one is that result, and the
+# same bits as the f32 result rounded, which another reader has it store; every form of the kernel, a batch, keys that end inside a tile
+@pytest.mark.gpu
+@pytest.mark.parametrize("hd,batch,S,heads,kv", [(64, 1, 100, 8, 2), (64, 1, 512, 8, 2), (64, 1, 1502, 8, 2), (64, 1, 2903, 8, 2), (64, 3, 70, 8, 8), (128, 2, 700, 8, 4),
+                                                 (128, 1, 3000, 8, 4), (128, 4, 256, 16, 8), (256, 8, 1000, 4, 1), (256, 1, 703, 4, 1), (256, 2, 100, 4, 1)])
+def test_attention_read_by_a_product(hip_bf16, hd, batch, S, heads, kv):
+    g, K, h = np.random.default_rng(S), 192, helpers
+    ns = [heads * hd, kv * hd, kv * hd]
+    x, ws, eye = draw(g, (1, batch * S, K)), [draw(g, (n, K), K ** -0.5) for n in ns], np.eye(heads * hd, dtype=np.float32)
+
+    def f(b, x, *p, also):
+        x = x + x - x
+        y = [linear(b, x, w, n, K) for w, n in zip(p, ns)]
+        q, k, v = (lang.transpose(b, 1, 2, lang.reshape(b, lang.make_shape(b, batch, S, n // hd, hd), t)) for n, t in zip(ns, y))
+        q, k = h.rope(b, 10000.0, 0, S, hd, q), h.rope(b, 10000.0, 0, S, hd, k)
+        attn = lang.matmul(b, q, lang.transpose(b, 2, 3, h.repeat_kv(b, heads // kv, k)))
+        sh = lang.shape(b, attn)
+        attn = attn / lang.constant(b, float(np.sqrt(np.float32(hd))), sh) + lang.broadcast(b, h.causal_mask(b, lang.to_nat(b, S)), sh)
+        out = lang.matmul(b, nn.softmax(b, attn), h.repeat_kv(b, heads // kv, v))
+        merged = lang.reshape(b, lang.make_shape(b, 1, batch * S, ns[0]), lang.transpose(b, 1, 2, out))
+        return [linear(b, merged, p[3], ns[0], ns[0])] + ([out] if also else [])
+
+    def run(also):
+        hip_bf16.trace(2)
+        hip_bf16.trace_reset()
+        got = vectors.run(hip_bf16, lambda b, *a: f(b, *a, also=also), 2 if also else 1, x, *ws, eye)
+        names = set(hip_bf16.trace_report())
+        hip_bf16.trace(False)
+        assert ("attn_prefill" if also else "attn_prefill[bf16]") in names, sorted(names)
+        return got
+    (narrow,), (_, out) = run(False), run(True)
+    assert np.array_equal(narrow[0].reshape(batch, S, heads, hd), vectors.bf16_round(out).transpose(0, 2, 1, 3))
+
+
 # the routed experts of a prefill, from 44 pairs to an expert on moe_ring_kernel: three slots whose choices crowd one expert (several row tiles, the last
 # partly filled) and leave others empty; the fewest k-steps, columns that end inside a tile of 128 and of 256; more pairs than
 # moe_route_kernel keeps in registers, more experts than it has threads
