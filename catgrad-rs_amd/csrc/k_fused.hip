@@ -343,8 +343,8 @@ hipError_t launch_softmax(const LaunchCtx &lc, const SoftmaxDesc &d) {
 // ---- the largest softmax value of a row (and its column) ----------------------------------------------------
 // max(softmax(x)), what a classifier reports as the confidence of its choice, without the probabilities ever being
 // stored: exp(max - max) / sum exp(x - max) in one pass over x with a running maximum; the same pass finds the column of
-// the largest x when argmax(x) is asked for as well.  Bound by reading x once: 4096 x 4096 f32 197 us in four launches
-// (the exponentials written and read twice) -> 18.  Rows of any length and alignment: 16-byte loads that need no
+// the largest x when argmax(x) is asked for as well.  Bound by reading x once, and by five operations and an exp2 a value: 4096 x 4096 f32
+// 197 us in four launches (the exponentials written and read twice) -> 15.  Rows of any length and alignment: 16-byte loads that need no
 // alignment, a scalar tail.  A wave to a row of up to 1024 values, a workgroup to a longer one, several workgroups
 // when there are fewer rows than CUs.
 struct RowBest {  // what is known of a part of a row
@@ -379,9 +379,16 @@ struct RowBest {  // what is known of a part of a row
   }
 };
 
-template <typename T, int TPR>
+// A group of values costs a value one maximum, a subtraction, a product, the hardware's exp2 and a sum: exp(x - m) is 2 to the rounded
+// product of the rounded difference and log2 e, 6e-8 |x - m| off for one value, with a weight that falls as exp(x - m) does, and of either
+// sign from value to value.  (Error against 64 bits over 4096 x 4096, 300 x 50000, 8000 x 300 values of
+// deviation 2: 5.2e-8 to 5.4e-8, as with expf.  4096 x 4096 f32 17.9 us with expf and every value ordered, 15.3 so; 120 x 131072 19.4, 13.2.)  The column is looked for when the
+// largest value is known, by the threads that hold it, in the group they met it in; a group with a NaN, which no maximum shows but the
+// sum does, is ordered value by value.
+// TPR threads to a row, GROUP values to a thread and turn.
+template <typename T, int TPR, int GROUP = 16>
 __global__ void __launch_bounds__(256) softmax_best_kernel(SoftmaxBestDesc d) {
-  constexpr int W = sizeof(T) == 4 ? 4 : 8, U = sizeof(T) == 4 ? 4 : 2, RPB = 256 / TPR;
+  constexpr int W = sizeof(T) == 4 ? 4 : 8, U = GROUP / W, RPB = 256 / TPR;
   __shared__ float part[4][4];
   const uint32_t rc = blockIdx.x * RPB + (RPB > 1 ? threadIdx.x / TPR : 0), t = threadIdx.x % TPR;
   const uint32_t row = rc / d.chunks, chunk = rc - row * d.chunks;
@@ -390,8 +397,10 @@ __global__ void __launch_bounds__(256) softmax_best_kernel(SoftmaxBestDesc d) {
     const T *x = (const T *)d.x + (int64_t)row * d.x_row_stride;
     const uint32_t c_begin = chunk * d.chunk_len, c_end = min(d.n, c_begin + d.chunk_len);
     float m = -3.40282347e+38f;
-    for (uint32_t c0 = c_begin + t * W; c0 < c_end; c0 += TPR * W * U) {
-      float v[U][W];
+    float v[U][W];
+    uint32_t at = 0, held = 0;  // where the group that holds this thread's largest value starts; the group in v
+    auto fetch = [&](uint32_t c0) __attribute__((always_inline)) {
+      held = c0;
 #pragma unroll
       for (int u = 0; u < U; ++u) {
         const uint32_t c = c0 + u * TPR * W;
@@ -420,6 +429,13 @@ __global__ void __launch_bounds__(256) softmax_best_kernel(SoftmaxBestDesc d) {
           }
         }
       }
+    };
+    auto key_of = [](float f) {  // f32::total_cmp as an order of unsigned words
+      const uint32_t w = __float_as_uint(f);
+      return w ^ ((uint32_t)((int32_t)w >> 31) | 0x80000000u);
+    };
+    for (uint32_t c0 = c_begin + t * W; c0 < c_end; c0 += TPR * W * U) {
+      fetch(c0);
       float gm = -INFINITY;
 #pragma unroll
       for (int u = 0; u < U; ++u)
@@ -429,19 +445,40 @@ __global__ void __launch_bounds__(256) softmax_best_kernel(SoftmaxBestDesc d) {
       const float mn = fmaxf(m, gm);
       b.s *= expf(m - mn);
       m = mn;
+      float part_s[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int u = 0; u < U; ++u)
 #pragma unroll
-        for (int j = 0; j < W; ++j) {
-          b.s += expf(v[u][j] - m);
-          if (d.arg) {  // a thread meets its columns in increasing order: "not smaller" replaces
-            const uint32_t w = __float_as_uint(v[u][j]), o = w ^ ((uint32_t)((int32_t)w >> 31) | 0x80000000u);
-            const uint32_t c = c0 + u * TPR * W + j;
-            const bool take = o >= b.key && c < c_end;
-            b.key = take ? o : b.key;
-            b.col = take ? c : b.col;
-          }
+        for (int j = 0; j < W; ++j) part_s[j & 3] += __builtin_amdgcn_exp2f((v[u][j] - m) * 1.44269504f);
+      const float gs = (part_s[0] + part_s[1]) + (part_s[2] + part_s[3]);
+      b.s += gs;
+      if (d.arg) {  // a thread meets its columns in increasing order: "not smaller" replaces
+        uint32_t key = key_of(gm);
+        // (a sum that is no number: a NaN, or an infinity less itself.  Of zeros of both signs either may be the maximum found.)
+        if (gs != gs || gm == 0.f) {
+          key = 0;
+#pragma unroll
+          for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int j = 0; j < W; ++j)
+              if (c0 + u * TPR * W + j < c_end) key = max(key, key_of(v[u][j]));
         }
+        at = key >= b.key ? c0 : at;
+        b.key = max(b.key, key);
+      }
+    }
+    if (d.arg) {
+      const uint32_t best = (uint32_t)wave_max_i32((int32_t)(b.key ^ 0x80000000u)) ^ 0x80000000u;
+      if (b.key == best && c_begin + t * W < c_end) {  // (usually one thread of the wave)
+        if (at != held) fetch(at);
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+          for (int j = 0; j < W; ++j) {
+            const uint32_t c = at + u * TPR * W + j;
+            if (c < c_end && key_of(v[u][j]) == best) b.col = c;
+          }
+      }
     }
   }
   b.merge_wave();
@@ -492,15 +529,20 @@ hipError_t launch_softmax_best(const LaunchCtx &lc, const SoftmaxBestDesc &in) {
   SoftmaxBestDesc d = in;
   if (!d.chunks || !d.best || (d.chunks > 1 && !d.part)) return hipErrorInvalidValue;
   d.chunk_len = ((d.n + d.chunks - 1) / d.chunks + 15) / 16 * 16;
-  const bool wave = d.chunks == 1 && d.n <= 1024;
+  // A wave to a row while that makes enough waves: no meeting of four, and a whole row of up to 2048 or 4096 values asked for at once (us, a
+  // workgroup to a row and so; f32 8192 x 2000 23.7, 13.3, 1024 x 2000 5.8, 5.2, 512 x 2000 5.0, 5.3, 4096 x 3000 14.9, 12.9, 2048 x 4096
+  // 8.3, 7.7, 1024 x 4000 5.8, 7.3; bf16 8192 x 1500 20.7, 11.1, 4096 x 4096 13.2, 10.4, 1000 x 4000 5.6, 7.9).
+  const uint32_t most = d.rows >= (uint32_t)lc.n_cus * 8 ? 4096 : d.rows >= (uint32_t)lc.n_cus * 4 ? 2048 : 1024;
+  const bool wave = d.chunks == 1 && d.n <= most;
   const unsigned grid = wave ? (d.rows + 3) / 4 : d.rows * d.chunks;
-  if (d.x_bf16) {
-    if (wave) CG_LAUNCH(lc, (softmax_best_kernel<uint16_t, 64>), grid, 256, d);
-    else CG_LAUNCH(lc, (softmax_best_kernel<uint16_t, 256>), grid, 256, d);
-  } else {
-    if (wave) CG_LAUNCH(lc, (softmax_best_kernel<float, 64>), grid, 256, d);
-    else CG_LAUNCH(lc, (softmax_best_kernel<float, 256>), grid, 256, d);
-  }
+#define CG_BEST(T)                                                                                \
+  if (wave && d.n > 2048) CG_LAUNCH(lc, (softmax_best_kernel<T, 64, 64>), grid, 256, d);          \
+  else if (wave && d.n > 1024) CG_LAUNCH(lc, (softmax_best_kernel<T, 64, 32>), grid, 256, d);     \
+  else if (wave) CG_LAUNCH(lc, (softmax_best_kernel<T, 64>), grid, 256, d);                       \
+  else CG_LAUNCH(lc, (softmax_best_kernel<T, 256>), grid, 256, d);
+  if (d.x_bf16) { CG_BEST(uint16_t) }
+  else { CG_BEST(float) }
+#undef CG_BEST
   if (d.chunks > 1) {
     LaunchCtx untimed = lc;  // the events stay with the pass over x
     untimed.ev_start = untimed.ev_stop = nullptr;

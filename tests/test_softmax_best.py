@@ -49,3 +49,37 @@ def test_best_of_rows_with_special_values(oracle, hip):
     (p, a), _ = run(oracle, x)
     (gp, ga), _ = run(hip, x)
     assert np.allclose(gp, p, rtol=1e-5, atol=0, equal_nan=True) and np.array_equal(ga, a), (p, gp, a, ga)
+
+
+# the same in rows of several groups of values to a thread, where the column is looked for in the group the largest was met in: equal
+# largest values in different groups, waves and pieces, zeros of both signs, NaN of both signs beside and behind the largest
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [70, 1000, 1030, 4097, 9001, 40000])
+def test_special_values_in_several_groups(oracle, hip, n):
+    g = np.random.default_rng(n)
+    x = vectors.bf16_round(-np.abs(g.standard_normal((14, n))).astype(np.float32))
+    x[0, [0, n // 2, n - 1]] = 3.0                                         # the last of equal values
+    x[1, [1, n // 3]] = 3.0
+    x[2, [n // 4, n - 2]], x[2, n // 2] = 0.0, -0.0                         # +0 is the larger
+    x[3, n // 2] = -0.0
+    x[4] = np.where(np.arange(n) % 2, 0.0, -0.0)
+    x[5, n // 2] = np.nan
+    x[6, n // 3], x[6, n - 1] = np.float32(-np.nan), 5.0                    # (a NaN with its sign set is below everything)
+    x[7, n - 1], x[7, 0] = np.nan, np.inf
+    x[8, [3, n // 2]] = np.inf
+    x[9] = -np.inf
+    x[9, n // 2] = np.finfo(np.float32).min
+    x[10] = np.float32(-np.nan)
+    x[11, n // 2:] = -np.inf
+    x[12] = np.nan
+    (p, a), _ = run(oracle, x)
+    (gp, ga), _ = run(hip, x)
+    for r in range(len(x)):
+        assert np.allclose(gp[r], p[r], rtol=1e-5, atol=0, equal_nan=True) and np.array_equal(ga[r], a[r]), (r, p[r], gp[r], a[r], ga[r])
+
+
+# a wave to rows of more than 1024 values where there are many of them: 32 and 64 values to a thread
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", [(1030, 1031), (1024, 2048), (2050, 2049), (2048, 4096), (2051, 4095), (2048, 4097)])
+def test_a_wave_to_a_longer_row(oracle, hip, hip_bf16, shape):
+    test_best_of_rows(oracle, hip, hip_bf16, shape)
