@@ -1118,7 +1118,7 @@ int try_gemv_add(cg_backend *be, cg_tensor *root, bool *done) {
       // linear(x) + bias: the grouped product launch adds the vector to every row (few rows: always; many rows:
       // where q / k / v go out as one launch - otherwise *added stays false and the add runs as an op of its own)
       TRY(realize(be, bv));
-      if (!bias_vector_ready(bv)) return CG_OK;
+      if (mm->op != N_MATMUL || !bias_vector_ready(bv)) return CG_OK;  // (mm: as below)
       be->addend_is_row = true;
       int st = realize_matmul(be, mm, bv, &added, nullptr);
       be->addend_is_row = false;
@@ -1128,7 +1128,8 @@ int try_gemv_add(cg_backend *be, cg_tensor *root, bool *done) {
       // now: the norm under this many-row product sums it (realize_matmul sees to it that it is summed by
       // the time it is added).
       if (other->op != N_KSUM || mm->gemv_candidate) TRY(realize(be, other));
-      if (other->stype != ST_F32 || !is_contiguous(other)) return CG_OK;
+      // (a launch that realised `other` may have taken mm along: two slots' products of the same experts)
+      if (mm->op != N_MATMUL || other->stype != ST_F32 || !is_contiguous(other)) return CG_OK;
       be->ksum_request = be->ksum_flush_node == root;
       be->ksum_ws = nullptr;
       const int st = realize_matmul(be, mm, other, &added, nullptr);

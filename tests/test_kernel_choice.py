@@ -200,3 +200,18 @@ for shape, wide in (((1, 16, 2048, 128), 1), ((1, 16, 2049, 128), 0), ((4, 16, 5
         names = [n for n in fake.fake_hip_launched().decode().split("\\n") if "attn_prefill" in n]
         assert len(names) == 1 and "attn_prefill_kernelILi128ELi64ELi4ELi1ELi%dE" % (wide + 1) in names[0], (shape, causal, names)
 """, BF16)
+
+
+def test_sum_of_two_slots_of_the_same_experts(fake_hip):  # noqa: F811
+    """The launch that realises one addend of `y0 + y1` makes the other as well: nothing is left of the product to add to."""
+    fake_hip("""
+import importlib
+lang, vectors = cg.lang, importlib.import_module("tests.vectors")
+
+def total(b, x, idx, w):
+    y = [lang.matmul(b, x, lang.transpose(b, 1, 2, lang.index(b, 0, lang.get(b, 1, i, idx), w))) for i in range(2)]
+    return y[0] + y[1]
+for s in (1, 5, 20, 200):
+    (got,) = vectors.run(be, total, 1, np.zeros((s, 1, 128), np.float32), np.zeros((s, 2), np.uint32), np.zeros((3, 192, 128), np.float32))
+    assert got.shape == (s, 1, 192)
+""", BF16)
