@@ -206,12 +206,15 @@ def test_sum_of_two_slots_of_the_same_experts(fake_hip):  # noqa: F811
     """The launch that realises one addend of `y0 + y1` makes the other as well: nothing is left of the product to add to."""
     fake_hip("""
 import importlib
-lang, vectors = cg.lang, importlib.import_module("tests.vectors")
+lang, nn, vectors = cg.lang, cg.nn, importlib.import_module("tests.vectors")
 
-def total(b, x, idx, w):
-    y = [lang.matmul(b, x, lang.transpose(b, 1, 2, lang.index(b, 0, lang.get(b, 1, i, idx), w))) for i in range(2)]
-    return y[0] + y[1]
+def total(b, x, idx, wg, wu, wd):
+    def slot(i):
+        of = lambda w: lang.transpose(b, 1, 2, lang.index(b, 0, lang.get(b, 1, i, idx), w))
+        return lang.matmul(b, nn.silu(b, lang.matmul(b, x, of(wg))) * lang.matmul(b, x, of(wu)), of(wd))
+    return slot(0) + slot(1)
 for s in (1, 5, 20, 200):
-    (got,) = vectors.run(be, total, 1, np.zeros((s, 1, 128), np.float32), np.zeros((s, 2), np.uint32), np.zeros((3, 192, 128), np.float32))
-    assert got.shape == (s, 1, 192)
+    up = np.zeros((3, 192, 128), np.float32)
+    (got,) = vectors.run(be, total, 1, np.zeros((s, 1, 128), np.float32), np.zeros((s, 2), np.uint32), up, up + 1, np.zeros((3, 128, 192), np.float32))
+    assert got.shape == (s, 1, 128)
 """, BF16)
