@@ -575,20 +575,9 @@ __global__ void __launch_bounds__(WR *WC *KG * 64) gemm_bf16_dma_kernel(GemmDesc
   const int kgrp = KG > 1 ? wave / (WR * WC) : 0, wt = KG > 1 ? wave % (WR * WC) : wave;
   const int wm = wt / WC, wn = wt % WC;
   const uint32_t tiles_m = (g.M + BM_ - 1) / BM_, tiles_n = (g.N + BNO - 1) / BNO;
-  const uint32_t per_batch = tiles_m * tiles_n, batch = g.nb0 * g.nb1;
-  // Workgroups are dealt round-robin to the 8 XCDs (one L2 each): give every XCD a contiguous
-  // range of logical tiles, and walk tiles in groups of 4 tile rows so that the ~32 tiles an
-  // XCD works on at once share their A and B panels in that L2.
-  uint32_t id = blockIdx.x;
-  if (gridDim.x % 8 == 0) id = (id % 8) * (gridDim.x / 8) + id / 8;
-  const uint32_t zz = id / per_batch;  // split * batch + batch index
-  const uint32_t t = id - zz * per_batch;
-  const uint32_t split = zz / batch, bz = zz - split * batch;
-  const uint32_t b0 = bz / g.nb1, b1 = bz - b0 * g.nb1;
-  constexpr uint32_t GM = 4;
-  const uint32_t first_m = t / (GM * tiles_n) * GM, gsz = min(tiles_m - first_m, GM);
-  const uint32_t tg = t % (GM * tiles_n);
-  const uint32_t m0 = (first_m + tg % gsz) * BM_, n0_all = tg / gsz * BNO;
+  const TilePlace place(tiles_m, tiles_n, g.nb0, g.nb1, max(g.splits, 1u));
+  const uint32_t batch = g.nb0 * g.nb1, split = place.split, bz = place.bz, b0 = place.b0, b1 = place.b1;
+  const uint32_t m0 = place.tm * BM_, n0_all = place.tn * BNO;
   const uint16_t *A = (const uint16_t *)g.a + b0 * g.sa_b0 + b1 * g.sa_b1;
   const uint16_t *B = (const uint16_t *)g.b + b0 * g.sb_b0 + b1 * g.sb_b1;
   const uint16_t *B2 = DUAL ? (const uint16_t *)g.dual_b + b0 * g.sb_b0 + b1 * g.sb_b1 : nullptr;
@@ -618,6 +607,10 @@ __global__ void __launch_bounds__(WR *WC *KG * 64) gemm_bf16_dma_kernel(GemmDesc
   const uint32_t k_begin = split * g.k_per_split;
   const uint32_t k_end = min(g.K, k_begin + g.k_per_split);
 
+  const int n_steps = k_end > k_begin ? (int)((k_end - k_begin) / BK) : 0;
+  const KOrder order(BKM || (RING && TM == 3) ? 0u : g.k_rotate, place.tn + tiles_n * place.zz, (uint32_t)n_steps);
+  const uint32_t k_first_step = k_begin + order.first * BK;
+
   f32x16 acc[TM][TN];
 #pragma unroll
   for (int i = 0; i < TM; ++i)
@@ -636,22 +629,24 @@ __global__ void __launch_bounds__(WR *WC *KG * 64) gemm_bf16_dma_kernel(GemmDesc
     const int R = q * 8 + (lane >> 3);
     const int c = (lane & 7) ^ ((R >> 1) & 7);
     if (q * 8 < BM_) {
-      gp[i] = A + (int64_t)min(m0 + R, g.M - 1) * g.sam + k_begin + c * 8;
+      gp[i] = A + (int64_t)min(m0 + R, g.M - 1) * g.sam + k_first_step + c * 8;
     } else if (BKM) {
       // 1 KB of the B tile = 1024 / (2 BN_) k-rows; this lane's 16 bytes: row kr, physical piece pc
       const int qb = q - BM_ / 8, kr = qb * (512 / BN_) + lane / (BN_ / 8), pc = lane % (BN_ / 8);
       const uint32_t n = n0 + (uint32_t)((pc ^ ((kr & 3) << 2)) * 8);
       gp[i] = B + (int64_t)(k_begin + kr) * g.sbk + min(n, Nl - 8);
-    } else if (DUAL) gp[i] = (R - BM_ < BNO ? B : B2) + (int64_t)min(n0 + (uint32_t)((R - BM_) % BNO), Nl - 1) * g.sbn + k_begin + c * 8;
-    else gp[i] = B + (int64_t)min(column(R - BM_), Nl - 1) * g.sbn + k_begin + c * 8;
+    } else if (DUAL) gp[i] = (R - BM_ < BNO ? B : B2) + (int64_t)min(n0 + (uint32_t)((R - BM_) % BNO), Nl - 1) * g.sbn + k_first_step + c * 8;
+    else gp[i] = B + (int64_t)min(column(R - BM_), Nl - 1) * g.sbn + k_first_step + c * 8;
   }
   // (k-major B: a wave's loads are all A's or all B's, and B's step down 64 rows per stage)
   const int64_t gp_step = BKM && wave * LPW * 8 >= BM_ ? (int64_t)BK * g.sbk : (int64_t)BK;
+  uint32_t to_wrap = order.wrap;
   auto issue = [&](int buf) {
+    const int64_t to_next = BKM ? gp_step : --to_wrap ? (int64_t)BK : (int64_t)(int32_t)order.back / 2;
 #pragma unroll
     for (int i = 0; i < LPW; ++i) {
       lds_dma16(gp[i], lds0 + buf * STAGE + piece(i) * 1024);
-      gp[i] += gp_step;
+      gp[i] += to_next;
     }
   };
   const int sw = (lane >> 1) & 7, half = lane >> 5;
@@ -715,7 +710,6 @@ __global__ void __launch_bounds__(WR *WC *KG * 64) gemm_bf16_dma_kernel(GemmDesc
     }
     __builtin_amdgcn_s_setprio(0);
   };
-  const int n_steps = k_end > k_begin ? (int)((k_end - k_begin) / BK) : 0;
   // (clock probe only) s_memtime ticks with the shader clock, s_memrealtime with a constant 100 MHz: their ratio
   // over the main loop is the clock this kernel really ran at
   unsigned long long tick0 = 0, real0 = 0;
@@ -749,13 +743,15 @@ __global__ void __launch_bounds__(WR *WC *KG * 64) gemm_bf16_dma_kernel(GemmDesc
     const uint32_t la = lds0 + wave * PA * 1024, ab = (BM_ / 8 + wave * (PB - PA)) * 1024;
     const uint32_t first = la + (NS - 1) * STAGE, limit = la + NS * STAGE;
     const uint32_t n = __builtin_amdgcn_readfirstlane((uint32_t)n_steps);
+    // (steps to request before the order goes back; none to come, or gone back already: never)
+    const uint32_t wrap = __builtin_amdgcn_readfirstlane((int)to_wrap > 0 ? to_wrap : 0x7FFFFFFFu);
 #define SR_ACC(i, j) [c##i##j] "+a"(acc[i][j])
 #define SR_A4 [ga0] "+v"(at[0]), [ga1] "+v"(at[1]), [ga2] "+v"(at[2]), [ga3] "+v"(at[3])
 #define SR_B4(o) [gb0] "+v"(at[o]), [gb1] "+v"(at[o + 1]), [gb2] "+v"(at[o + 2]), [gb3] "+v"(at[o + 3])
 #define SR_IN                                                                                                              \
   [ra0] "v"(ra[0]), [ra1] "v"(ra[1]), [ra2] "v"(ra[2]), [ra3] "v"(ra[3]), [rb0] "v"(rb[0]), [rb1] "v"(rb[1]),              \
       [rb2] "v"(rb[2]), [rb3] "v"(rb[3]), [first] "s"(first), [limit] "s"(limit), [la] "s"(la), [ab] "s"(ab), [n] "s"(n),  \
-      [stage] "i"(STAGE), [all] "i"(NS * STAGE), [held] "i"(NS - 1)
+      [wrap] "s"(wrap), [back] "s"(order.back), [stage] "i"(STAGE), [all] "i"(NS * STAGE), [held] "i"(NS - 1)
     if constexpr (TM == 2 && TN == 2) {
       static_assert(NS == 5 && !EPI, "");
       asm volatile(SR_LOOP_22 : SR_ACC(0, 0), SR_ACC(0, 1), SR_ACC(1, 0), SR_ACC(1, 1), SR_A4, SR_B4(4) : SR_IN : SR_CLOBBERS);
@@ -2573,6 +2569,7 @@ __global__ void __launch_bounds__(256) moe_gemm_dma_kernel(MoeGemmDesc g) {
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint16_t *)dma_smem;
   const int sw = (lane >> 1) & 7, half = lane >> 5;
   const int n_steps = (int)(K / BK);
+  const KOrder order(g.k_rotate, e * tiles_n + n0 / BN_, (uint32_t)n_steps);
   const int64_t plane = PLANES ? (int64_t)g.S * K : 0;
   for (uint32_t m0 = m_first; m0 < cnt; m0 += PAIRS) {
     const int live_tiles = (int)min((uint32_t)MT, (cnt - m0 + TPAIRS - 1) / TPAIRS);  // wave-uniform
@@ -2607,18 +2604,20 @@ __global__ void __launch_bounds__(256) moe_gemm_dma_kernel(MoeGemmDesc g) {
             rows = g.slot[s].a16;
             bs = g.slot[s].a_bs;
           }
-        gp[i] = rows + part * plane + (int64_t)tok * bs + c * 8;
+        gp[i] = rows + part * plane + (int64_t)tok * bs + order.first * BK + c * 8;
       } else {
         const int rb = R - BM_, p = rb / BN_, col = rb - p * BN_;
-        gp[i] = W[p < NP ? p : 0] + (int64_t)min(n0 + (uint32_t)col, N - 1) * sbn[p < NP ? p : 0] + c * 8;
+        gp[i] = W[p < NP ? p : 0] + (int64_t)min(n0 + (uint32_t)col, N - 1) * sbn[p < NP ? p : 0] + order.first * BK + c * 8;
       }
     }
+    uint32_t to_wrap = order.wrap;
     auto issue = [&](int buf) {
+      const int64_t to_next = --to_wrap ? (int64_t)BK : (int64_t)(int32_t)order.back / 2;
 #pragma unroll
       for (int i = 0; i < LPW; ++i) {
         if (i >= MT) lds_dma16_stream(gp[i], lds0 + buf * STAGE + block_of(i) * 1024);
         else if (i < live_tiles) lds_dma16(gp[i], lds0 + buf * STAGE + block_of(i) * 1024);
-        gp[i] += BK;
+        gp[i] += to_next;
       }
     };
     auto compute = [&](int buf) {
@@ -2799,7 +2798,13 @@ static hipError_t launch_moe_gemm_dma(const LaunchCtx &lc, const MoeGemmDesc &g,
   return hipGetLastError();
 }
 
-hipError_t launch_moe_gemm(const LaunchCtx &lc, const MoeGemmDesc &g) {
+hipError_t launch_moe_gemm(const LaunchCtx &lc, const MoeGemmDesc &given) {
+  MoeGemmDesc g = given;
+  // As in launch_matmul, up to two row tiles to an expert, which start at the same k.  Gate and up of 60 experts, 2 x 1408 x 2048, 4 of
+  // them to a token: 100 tokens 123 -> 116 us, 256 124 -> 114, 512 135 -> 129, 1024 147 -> 138, 1500 150 -> 146, 2048 215 -> 212; 4096
+  // 360, 366.
+  g.k_rotate = g.K >= 2048 && (uint64_t)g.S * g.n_slot <= 192 * (uint64_t)g.n_expert;
+  for (uint32_t i = 0; i < g.n_prob && i < 2; ++i) g.k_rotate = g.k_rotate && g.prob[i].sbn % 2048 == 0;
   if (!g.S || !g.n_prob || !g.n_slot || !g.n_expert) return hipSuccess;
   if (g.S > 65535 || g.n_slot > 8 || g.n_prob > 2 || g.n_expert > 65535 || g.K % 8 || g.pro == PRO_RMSNORM)
     return hipErrorInvalidValue;
@@ -3283,6 +3288,14 @@ hipError_t launch_matmul(const LaunchCtx &lc_in, const GemmDesc &g, const char *
     GemmDesc gg = g;
     gg.splits = splits;
     if (splits == 1) gg.k_per_split = g.K;
+    // Weight rows a multiple of 4 KB apart (and slices of a whole one): workgroups that all start at k = 0 ask the same few channels of
+    // the L2s and of memory for 128 bytes of every row, step for step, so up to 128 rows, where the stream of weights is what a
+    // product waits for, column tiles start at different k.  Weights from memory, us: 37 rows of gate and up, 2 x 8192, K = 2048
+    // 18.5 -> 15.6, 100 20.1 -> 18.5; 17 x 16384 x 2048 18.3 -> 15.2, x 8192 58.7 -> 49.8; 64 x 32000 x 8192 134 -> 114; 128 x 32000 x
+    // 4096 65 -> 56; 64 x 4096 x 8192 in four slices 19.7 -> 17.5.  Slices of half of 4 KB start at different k as they are (37 x 2048
+    // x 8192 in eight 10.7, 11.3); rows an odd number of KB apart meet all channels (64 x 2 x 4096 x 2560 20.8, 21.1); more row tiles
+    // share the weights, and their rows are then in the L2s for one step only (2900 x 2048 x 8192 95 and 134, 8192^3 745 and 805).
+    gg.k_rotate = g.M <= 128 && g.sbk == 1 && g.sbn % 2048 == 0 && gg.k_per_split >= 2048;
     if (gemm_dma_ok(g)) {
       const uint64_t t256 = (uint64_t)((g.M + 255) / 256) * ((g.N + 255) / 256) * batch * splits;
       hipError_t e;

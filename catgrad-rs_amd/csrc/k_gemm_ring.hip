@@ -207,6 +207,10 @@ static hipError_t whole_lds(const void *kernel, int bytes) {
 #define HSYNC(v) "s_waitcnt vmcnt(" #v ")\n\ts_barrier\n\t"
 #define HSLICE(b, UB, ks, W, E0, E1, E2, E3) \
   W PRODUCT(0, b, 0, 0, A0, UB, ks) E0 PRODUCT(0, b, 0, 1, A0, UB, ks) E1 PRODUCT(0, b, 1, 0, A0, UB, ks) E2 PRODUCT(0, b, 1, 1, A0, UB, ks) E3
+// s[58:59]: bytes from the step being requested to the next - behind a slice's last step back to its first (KOrder) -, s55 the steps
+// until then; the main loop finds the next size out among its products
+#define HSTEP_SIZE_AT(lo, hi) "s_sub_u32 s55, s55, 1\n\ts_cmp_eq_u32 s55, 0\n\ts_cselect_b32 " lo ", %[back], 128\n\ts_cselect_b32 " hi ", -1, 0\n\t"
+#define HSTEP_SIZE HSTEP_SIZE_AT("s58", "s59")
 #define HPHASE0(G, v)                                                                                                              \
   G("s_add_u32 s54, s53, %[lds]\n\t") HSYNC(v)                                                                                     \
   HFROM_A("s48", 3) HFROM_B("s50", 0)                                                                                              \
@@ -217,7 +221,7 @@ static hipError_t whole_lds(const void *kernel, int bytes) {
 #define HPHASE1(G, v)                                                                                                              \
   G("s_add_u32 s54, s48, %[lds]\n\t") HSYNC(v)                                                                                     \
   HFROM_B("s52", 0)                                                                                                                \
-  HSLICE(1, B1, 0, READS_BUT(6), HB0(0, 0) G(HM0(0)), HB0(1, 0) G(LOAD(B0, 0) HM0(1)), G(LOAD(B0, 1)), "")                         \
+  HSLICE(1, B1, 0, READS_BUT(6), HB0(0, 0) G(HM0(0)), HB0(1, 0) G(LOAD(B0, 0) HM0(1)), G(LOAD(B0, 1)), G(HSTEP_SIZE_AT("s56", "s57"))) \
   HFROM_A("s51", 0) HFROM_B("s52", 1)                                                                                              \
   HSLICE(1, B1, 1, READS_BUT(6), HB0(0, 1) G(HM0(2)), HB0(1, 1) G(LOAD(B0, 2) HM0(3)), HA(0, 0) G(LOAD(B0, 3)), HA(1, 0))      \
   HFROM_A("s51", 1) HFROM_B("s52", 2) G("s_add_u32 s54, s49, %[lds]\n\t")                                                          \
@@ -235,8 +239,9 @@ static hipError_t whole_lds(const void *kernel, int bytes) {
   HM0(0) "s_nop 0\n\t" HLOAD_A(0) HM0(1) "s_nop 0\n\t" HLOAD_A(1) HM0(2) "s_nop 0\n\t" HLOAD_A(2) HM0(3) "s_nop 0\n\t" HLOAD_A(3)
 #define HLOADS_B(U) \
   HM0(0) "s_nop 0\n\t" LOAD(U, 0) HM0(1) "s_nop 0\n\t" LOAD(U, 1) HM0(2) "s_nop 0\n\t" LOAD(U, 2) HM0(3) "s_nop 0\n\t" LOAD(U, 3)
-#define HPOINTERS "s_mov_b64 s[42:43], %[pb0]\n\ts_mov_b64 s[44:45], %[pb1]\n\ts_movk_i32 s58, 128\n\ts_mov_b32 s59, 0\n\t"
-#define HNEXT_STEP "s_add_u32 s42, s42, 128\n\ts_addc_u32 s43, s43, 0\n\ts_add_u32 s44, s44, 128\n\ts_addc_u32 s45, s45, 0\n\t"
+#define HPOINTERS "s_mov_b64 s[42:43], %[pb0]\n\ts_mov_b64 s[44:45], %[pb1]\n\ts_mov_b32 s55, %[wrap]\n\t" HSTEP_SIZE
+#define HNEXT_B "s_add_u32 s42, s42, s58\n\ts_addc_u32 s43, s43, s59\n\ts_add_u32 s44, s44, s58\n\ts_addc_u32 s45, s45, s59\n\t"
+#define HNEXT_STEP HNEXT_B HSTEP_SIZE
 #define HSTEP_LOADS \
   HLOADS_A "s_add_u32 s54, s54, 16384\n\t" HLOADS_B(B0) "s_add_u32 s54, s54, 16384\n\t" HLOADS_B(B1) "s_add_u32 s54, s54, 16384\n\t"
 // steps 0 to 2 requested: 36 loads
@@ -250,7 +255,7 @@ static hipError_t whole_lds(const void *kernel, int bytes) {
   HFROM_A("s48", 1) HFROM_B("s49", 2) HB0(0, 2) HB0(1, 2) HA(0, 1) HA(1, 1)                                                 \
   HFROM_A("s48", 2) HFROM_B("s49", 3) HB0(0, 3) HB0(1, 3) HA(0, 2) HA(1, 2)                                                 \
   "s_cmp_eq_u32 s47, 0\n\ts_cbranch_scc1 2f\n\t"                                                                                \
-  "1:\n\t" HPHASE0(HON, 24) HPHASE1(HON, 20) HNEXT_STEP HNEXT_PLACES                                                             \
+  "1:\n\t" HPHASE0(HON, 24) HPHASE1(HON, 20) HNEXT_B "s_mov_b64 s[58:59], s[56:57]\n\t" HNEXT_PLACES                                                             \
   "s_sub_u32 s47, s47, 1\n\ts_cmp_lg_u32 s47, 0\n\ts_cbranch_scc1 1b\n\t"                                                       \
   "2:\n\t" HPHASE0(HOFF, 24) HPHASE1(HOFF, 16) HNEXT_PLACES HPHASE0(HOFF, 12) HPHASE1(HOFF, 4) HNEXT_PLACES HPHASE0(HOFF, 0)    \
   HLAST "s_nop 15\n\ts_nop 7\n\t"
@@ -560,18 +565,10 @@ __global__ void __launch_bounds__(256, 1) gemm_bf16_ring_kernel(GemmDesc g) {
   constexpr uint32_t BM = AH * 128;
   static_assert(AH == 2 || GATED, "the epilogues of 128-row tiles");
   const uint32_t tiles_m = (g.M + BM - 1) / BM, tiles_n = (g.N + BNO - 1) / BNO;
-  const uint32_t per_batch = tiles_m * tiles_n, batch = g.nb0 * g.nb1;
-  // every XCD a contiguous range of tiles, in groups of four tile rows: as in gemm_bf16_dma_kernel
-  uint32_t id = blockIdx.x;
-  if (gridDim.x % 8 == 0) id = (id % 8) * (gridDim.x / 8) + id / 8;
-  const uint32_t zz = id / per_batch, t = id - zz * per_batch;
-  const uint32_t split = zz / batch, bz = zz - split * batch;
-  const uint32_t b0 = bz / g.nb1, b1 = bz - b0 * g.nb1;
-  constexpr uint32_t GM = 4;
-  const uint32_t first_m = t / (GM * tiles_n) * GM, gsz = min(tiles_m - first_m, GM);
-  const uint32_t tg = t % (GM * tiles_n);
-  const uint32_t m0 = (first_m + tg % gsz) * BM;
-  uint32_t n0 = tg / gsz * BNO, Nl = g.N;
+  const TilePlace place(tiles_m, tiles_n, g.nb0, g.nb1, max(g.splits, 1u));
+  const uint32_t batch = g.nb0 * g.nb1, split = place.split, bz = place.bz, b0 = place.b0, b1 = place.b1;
+  const uint32_t m0 = place.tm * BM;
+  uint32_t n0 = place.tn * BNO, Nl = g.N;
   const uint16_t *B = (const uint16_t *)g.b + b0 * g.sb_b0 + b1 * g.sb_b1;
   float *C = (g.splits > 1 ? g.workspace + (uint64_t)split * batch * g.M * g.N : g.c) + (uint64_t)bz * g.M * g.N;
   const float *Bias = nullptr, *Cadd = KIND == RING_PLAIN && g.c_add && g.splits <= 1 ? g.c_add + (uint64_t)bz * g.M * g.N : nullptr;
@@ -592,9 +589,11 @@ __global__ void __launch_bounds__(256, 1) gemm_bf16_ring_kernel(GemmDesc g) {
   const uint32_t n_steps = __builtin_amdgcn_readfirstlane((k_end - k_begin) / 64);
   // Where this lane's piece of each load comes from: byte offsets from the tile's first row (rows past the end repeat the last
   // one), the 16-byte chunk swizzled so that the fragment reads are free of bank conflicts.
-  const uint16_t *pa = (const uint16_t *)g.a + b0 * g.sa_b0 + b1 * g.sa_b1 + (int64_t)m0 * g.sam + k_begin;
-  const uint16_t *pb0 = B + (int64_t)n0 * g.sbn + k_begin;
-  const uint16_t *pb1 = GATED ? (const uint16_t *)g.dual_b + b0 * g.sb_b0 + b1 * g.sb_b1 + (int64_t)n0 * g.sbn + k_begin : pb0;
+  const KOrder order(AH == 1 ? g.k_rotate : 0u, place.tn + tiles_n * place.zz, n_steps);  // (tiles of 256 rows have more than 128)
+  const uint32_t k_first = k_begin + order.first * 64;
+  const uint16_t *pa = (const uint16_t *)g.a + b0 * g.sa_b0 + b1 * g.sa_b1 + (int64_t)m0 * g.sam + k_first;
+  const uint16_t *pb0 = B + (int64_t)n0 * g.sbn + k_first;
+  const uint16_t *pb1 = GATED ? (const uint16_t *)g.dual_b + b0 * g.sb_b0 + b1 * g.sb_b1 + (int64_t)n0 * g.sbn + k_first : pb0;
   const uint32_t sa = (uint32_t)g.sam * 2, sb = (uint32_t)g.sbn * 2, last_a = g.M - 1 - m0, last_b = Nl - 1 - n0;
   uint32_t dA0[4], dA1[4], dB0[4], dB1[4];
 #pragma unroll
@@ -623,9 +622,10 @@ __global__ void __launch_bounds__(256, 1) gemm_bf16_ring_kernel(GemmDesc g) {
 #define RING_IN                                                                                                            \
   [dA00] "v"(dA0[0]), [dA01] "v"(dA0[1]), [dA02] "v"(dA0[2]), [dA03] "v"(dA0[3]), [dA10] "v"(dA1[0]), [dA11] "v"(dA1[1]),  \
       [dA12] "v"(dA1[2]), [dA13] "v"(dA1[3]), [pa] "s"(sa0), RING_IN_B
+#define RING_ORDER [wrap] "s"(order.wrap), [back] "s"(order.back)
 #define RING_GATHERED [ga0] "+v"(ga[0]), [ga1] "+v"(ga[1]), [ga2] "+v"(ga[2]), [ga3] "+v"(ga[3])
 #define RING_HALF_SCALARS "v126", "v127", "s48", "s49", "s50", "s51", "s52", "s53"
-#define RING_SCALARS "s54", "s58", "s59", "s40", "s41", "s42", "s43", "s44", "s45", "s46", "s47", "m0", "scc", "memory"
+#define RING_SCALARS "s54", "s55", "s56", "s57", "s58", "s59", "s40", "s41", "s42", "s43", "s44", "s45", "s46", "s47", "m0", "scc", "memory"
 #define RING_V10(d) "v" #d "0", "v" #d "1", "v" #d "2", "v" #d "3", "v" #d "4", "v" #d "5", "v" #d "6", "v" #d "7", "v" #d "8", "v" #d "9"
 #define RING_FRAGMENTS                                                                                                     \
   "v128", "v129", RING_V10(13), RING_V10(14), RING_V10(15), RING_V10(16), RING_V10(17), RING_V10(18), RING_V10(19),        \
@@ -638,7 +638,7 @@ __global__ void __launch_bounds__(256, 1) gemm_bf16_ring_kernel(GemmDesc g) {
 #define RING_STRIP RING_V10(11), "v120", "v121", "v122", "v123", "v124", "v125", "v126", "v127"
   if constexpr (WIDE) asm volatile(WFIRST_LOADS::RING_IN, RING_WIDE_IN : RING_SCALARS, RING_WIDE_SCALARS);
   else if constexpr (AH == 2) asm volatile(FIRST_LOADS::RING_IN : RING_SCALARS);
-  else asm volatile(HFIRST_LOADS : RING_GATHERED : RING_IN_B : RING_SCALARS);
+  else asm volatile(HFIRST_LOADS : RING_GATHERED : RING_IN_B, RING_ORDER : RING_SCALARS);
   float zero;
   asm volatile("v_mov_b32 %0, 0" : "=v"(zero));  // (the accumulators are cleared behind the first loads, not in front of them)
   f32x16 acc[AH][2][2][2];  // [A half][B half][row block][column block]
@@ -684,7 +684,7 @@ __global__ void __launch_bounds__(256, 1) gemm_bf16_ring_kernel(GemmDesc g) {
   else if constexpr (AH == 2)
     asm volatile(MAIN_LOOP : RING_ACC0, RING_ACC1, RING_PLACES : RING_IN, [n] "s"(n_steps) : RING_SCALARS, RING_FRAGMENTS);
   else
-    asm volatile(HMAIN_LOOP : RING_ACC0, RING_PLACES, RING_GATHERED : RING_IN_B, [n] "s"(n_steps) : RING_SCALARS, RING_HALF_SCALARS, RING_FRAGMENTS);
+    asm volatile(HMAIN_LOOP : RING_ACC0, RING_PLACES, RING_GATHERED : RING_IN_B, RING_ORDER, [n] "s"(n_steps) : RING_SCALARS, RING_HALF_SCALARS, RING_FRAGMENTS);
   if (KIND == RING_PLAIN && g.clock_ticks && tid == 0) {
     atomicAdd(g.clock_ticks, __builtin_amdgcn_s_memtime() - tick0);
     atomicAdd(g.clock_ticks + 1, __builtin_amdgcn_s_memrealtime() - real0);
@@ -874,8 +874,9 @@ __global__ void __launch_bounds__(256, 1) moe_ring_kernel(MoeGemmDesc g) {
   const uint32_t live = min(g.route_count[e] - m0, 128u), *list = g.route_list + g.route_offset[e] + m0;
   const uint32_t n_steps = __builtin_amdgcn_readfirstlane(K / 64);
   const int64_t sbn0 = g.prob[prob].sbn;
-  const uint16_t *pb0 = (const uint16_t *)g.prob[prob].w + (int64_t)e * g.sb_index + (int64_t)n0 * sbn0;
-  const uint16_t *pb1 = GATED ? (const uint16_t *)g.prob[1].w + (int64_t)e * g.sb_index + (int64_t)n0 * g.prob[1].sbn : pb0;
+  const KOrder order(g.k_rotate, e * tiles_n + n0 / BNO, n_steps);
+  const uint16_t *pb0 = (const uint16_t *)g.prob[prob].w + (int64_t)e * g.sb_index + (int64_t)n0 * sbn0 + order.first * 64;
+  const uint16_t *pb1 = GATED ? (const uint16_t *)g.prob[1].w + (int64_t)e * g.sb_index + (int64_t)n0 * g.prob[1].sbn + order.first * 64 : pb0;
   const uint32_t sb = (uint32_t)sbn0 * 2, sb1 = GATED ? (uint32_t)g.prob[1].sbn * 2 : sb, last_b = N - 1 - n0;
   uint64_t ga[4];
   uint32_t dB0[4], dB1[4];
@@ -891,7 +892,7 @@ __global__ void __launch_bounds__(256, 1) moe_ring_kernel(MoeGemmDesc g) {
         rows = g.slot[s].a16;
         bs = g.slot[s].a_bs;
       }
-    ga[i] = (uint64_t)(rows + (int64_t)(ent & 0xFFFFu) * bs) + c;
+    ga[i] = (uint64_t)(rows + (int64_t)(ent & 0xFFFFu) * bs) + order.first * 128 + c;
     dB0[i] = min(r, last_b) * sb + c;
     dB1[i] = GATED ? min(r, last_b) * sb1 + c : min(r + 128, last_b) * sb + c;
   }
@@ -904,7 +905,7 @@ __global__ void __launch_bounds__(256, 1) moe_ring_kernel(MoeGemmDesc g) {
 #define MOE_IN                                                                                                            \
   [dB00] "v"(dB0[0]), [dB01] "v"(dB0[1]), [dB02] "v"(dB0[2]), [dB03] "v"(dB0[3]), [dB10] "v"(dB1[0]), [dB11] "v"(dB1[1]), \
       [dB12] "v"(dB1[2]), [dB13] "v"(dB1[3]), [pb0] "s"(s_b0), [pb1] "s"(s_b1), [lds] "s"(lds)
-  asm volatile(HFIRST_LOADS : RING_GATHERED : MOE_IN : RING_SCALARS);
+  asm volatile(HFIRST_LOADS : RING_GATHERED : MOE_IN, RING_ORDER : RING_SCALARS);
   float zero;
   asm volatile("v_mov_b32 %0, 0" : "=v"(zero));
   f32x16 acc[1][2][2][2];  // [0][B half][row block][column block]
@@ -920,7 +921,7 @@ __global__ void __launch_bounds__(256, 1) moe_ring_kernel(MoeGemmDesc g) {
     ra[ks] = wm * 8192 + p;
     rb[ks] = wn * 8192 + p;
   }
-  asm volatile(HMAIN_LOOP : RING_ACC0, RING_PLACES, RING_GATHERED : MOE_IN, [n] "s"(n_steps) : RING_SCALARS, RING_HALF_SCALARS, RING_FRAGMENTS);
+  asm volatile(HMAIN_LOOP : RING_ACC0, RING_PLACES, RING_GATHERED : MOE_IN, RING_ORDER, [n] "s"(n_steps) : RING_SCALARS, RING_HALF_SCALARS, RING_FRAGMENTS);
   // Rows back to their slot and token, out of LDS as in gemm_bf16_ring_kernel: a lane finds where the row of its number goes and
   // hands that to the sixteen lanes that store it.
   __syncthreads();

@@ -307,6 +307,7 @@ struct GemmDesc {
   // split-K (bf16 fast path only): partial products go to workspace[split][batch][M][N]
   float *workspace;
   uint32_t splits, k_per_split;
+  uint32_t k_rotate;  // (set by launch_matmul) column tiles start at different k (KOrder in dev_common.hpp)
   // optional (the one-row kernels, the sum of k-slices, gemm_add_ok): C = A . B + c_add (c_add laid out like C)
   const float *c_add;
   // split along k (splits > 1): leave the slices in the workspace; the caller sums them (launch_splitk_sum, or
@@ -547,6 +548,7 @@ struct MoeGemmDesc {
   const uint32_t *route_count, *route_offset, *route_list;
   // optional, with the above: the row tiles of all experts as a work list (launch_moe_route's `tiles`)
   const uint32_t *route_tiles;
+  uint32_t k_rotate;  // (set by launch_moe_gemm) as GemmDesc::k_rotate
 };
 hipError_t launch_moe_gemm(const LaunchCtx &lc, const MoeGemmDesc &g);
 // k_gemm_ring.hip: the same for sorted pairs with a work list

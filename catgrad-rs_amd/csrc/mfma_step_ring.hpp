@@ -44,6 +44,12 @@
 #define SR_LA(i) "global_load_lds_dwordx4 %[ga" #i "], off\n\tv_lshl_add_u64 %[ga" #i "], %[ga" #i "], 0, s[44:45]\n\t"
 #define SR_LB(i) "global_load_lds_dwordx4 %[gb" #i "], off\n\tv_lshl_add_u64 %[gb" #i "], %[gb" #i "], 0, s[44:45]\n\t"
 #define SR_NEXT_READ "s_add_u32 s48, s48, %[stage]\n\ts_cmp_eq_u32 s48, %[all]\n\ts_cselect_b32 s48, 0, s48\n\t"
+// bytes from the step being requested to the next (KOrder; a product of up to 128 rows is on 128 x 128, so the others go straight on)
+#define SR_STEP_SIZE "s_sub_u32 s51, s51, 1\n\ts_cmp_eq_u32 s51, 0\n\ts_cselect_b32 s44, %[back], 128\n\ts_cselect_b32 s45, -1, 0\n\t"
+#define SR_STEP_22 SR_STEP_SIZE
+#define SR_STEP_32 ""
+#define SR_FIRST_STEP_22 "s_mov_b32 s51, %[wrap]\n\t" SR_STEP_SIZE
+#define SR_FIRST_STEP_32 "s_movk_i32 s44, 128\n\ts_mov_b32 s45, 0\n\t"
 #define SR_NEXT_LOAD                                                                                                     \
   "s_add_u32 s46, s46, %[stage]\n\ts_cmp_eq_u32 s46, %[limit]\n\ts_cselect_b32 s46, %[la], s46\n\ts_add_u32 s50, s46, " \
   "%[ab]\n\t"
@@ -84,9 +90,9 @@
 // n >= NS - 1 steps, NS - 1 of them requested already: v0 counts the loads of NS - 2 steps, v those of NS - 3; TAIL: the NS - 2
 // steps before the last, which request nothing
 #define SR_LOOP(R, v0, v, TAIL)                                                                                             \
-  "s_movk_i32 s44, 128\n\ts_mov_b32 s45, 0\n\ts_mov_b32 s46, %[first]\n\ts_add_u32 s50, s46, %[ab]\n\ts_mov_b32 s48, 0\n\t"    \
+  SR_FIRST_STEP_##R "s_mov_b32 s46, %[first]\n\ts_add_u32 s50, s46, %[ab]\n\ts_mov_b32 s48, 0\n\t"    \
   "s_sub_u32 s47, %[n], %[held]\n\t" SR_SYNC(v0) SR_FIRST_##R "s_cmp_eq_u32 s47, 0\n\ts_cbranch_scc1 2f\n\t"                   \
-  "1:\n\t" SR_HEAD_##R SR_REST_##R(SR_ON, v) SR_NEXT_LOAD                                                                \
+  "1:\n\t" SR_HEAD_##R SR_REST_##R(SR_ON, v) SR_NEXT_LOAD SR_STEP_##R                                                                \
   "s_sub_u32 s47, s47, 1\n\ts_cmp_lg_u32 s47, 0\n\ts_cbranch_scc1 1b\n\t"                                                      \
   "2:\n\t" TAIL SR_HEAD_##R SR_LAST_##R "s_nop 15\n\ts_nop 7\n\t"
 #define SR_QUIET(R, v) SR_HEAD_##R SR_REST_##R(SR_OFF, v)
@@ -95,4 +101,4 @@
 #define SR_V10(d) "v" #d "0", "v" #d "1", "v" #d "2", "v" #d "3", "v" #d "4", "v" #d "5", "v" #d "6", "v" #d "7", "v" #d "8", "v" #d "9"
 #define SR_CLOBBERS                                                                                                            \
   "v142", "v143", "v144", "v145", "v146", "v147", "v148", "v149", SR_V10(15), SR_V10(16), SR_V10(17), SR_V10(18), SR_V10(19),  \
-      SR_V10(20), SR_V10(21), "v220", "v221", "v222", "v223", "s44", "s45", "s46", "s47", "s48", "s50", "m0", "scc", "memory"
+      SR_V10(20), SR_V10(21), "v220", "v221", "v222", "v223", "s44", "s45", "s46", "s47", "s48", "s50", "s51", "m0", "scc", "memory"
