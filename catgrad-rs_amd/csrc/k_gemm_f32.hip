@@ -46,15 +46,9 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int half = lane >> 5;
   const uint32_t tiles_m = (g.M + 32 * R - 1) / (32 * R), tiles_n = (g.N + 127) / 128;
-  const uint32_t per_batch = tiles_m * tiles_n, batch = g.nb0 * g.nb1;
-  // a contiguous range of tiles to each XCD, walked in groups of four tile rows (as in gemm_bf16_dma_kernel)
-  uint32_t id = blockIdx.x;
-  if (gridDim.x % 8 == 0) id = (id % 8) * (gridDim.x / 8) + id / 8;
-  const uint32_t zz = id / per_batch, t = id - zz * per_batch;
-  const uint32_t split = zz / batch, bz = zz - split * batch;
-  const uint32_t b0 = bz / g.nb1, b1 = bz - b0 * g.nb1;
-  const uint32_t first_m = t / (4 * tiles_n) * 4, gsz = min(tiles_m - first_m, 4u), tg = t % (4 * tiles_n);
-  const uint32_t m0 = (first_m + tg % gsz) * (32 * R), n0 = tg / gsz * 128;
+  const TilePlace place(tiles_m, tiles_n, g.nb0, g.nb1, max(g.splits, 1u));
+  const uint32_t batch = g.nb0 * g.nb1, split = place.split, bz = place.bz, b0 = place.b0, b1 = place.b1;
+  const uint32_t m0 = place.tm * (32 * R), n0 = place.tn * 128;
   const float *A = (const float *)g.a + b0 * g.sa_b0 + b1 * g.sa_b1;
   const float *B = (const float *)g.b + b0 * g.sb_b0 + b1 * g.sb_b1;
   const uint32_t k_begin = g.splits > 1 ? min(g.K, split * g.k_per_split) : 0;

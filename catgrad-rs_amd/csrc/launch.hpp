@@ -303,16 +303,16 @@ struct GemmDesc {
   int64_t sbk, sbn;          // element strides of B[k, n]
   uint32_t nb0, nb1;         // batch = nb0 * nb1 (row-major)
   int64_t sa_b0, sa_b1, sb_b0, sb_b1;  // batch strides (0 = broadcast)
-  int32_t bf16_math;         // 1: operands rounded to bf16, bf16 MFMA; 0: f32 MFMA
+  uint8_t bf16_math;         // 1: operands rounded to bf16, bf16 MFMA; 0: f32 MFMA
+  uint8_t defer_reduce, glu_kind, act_sigmoid, rope_role[3];  // (below)
+  uint8_t k_rotate;          // (set by launch_matmul) column tiles start at different k (KOrder in dev_common.hpp)
   // split-K (bf16 fast path only): partial products go to workspace[split][batch][M][N]
   float *workspace;
   uint32_t splits, k_per_split;
-  uint32_t k_rotate;  // (set by launch_matmul) column tiles start at different k (KOrder in dev_common.hpp)
   // optional (the one-row kernels, the sum of k-slices, gemm_add_ok): C = A . B + c_add (c_add laid out like C)
   const float *c_add;
-  // split along k (splits > 1): leave the slices in the workspace; the caller sums them (launch_splitk_sum, or
+  // defer_reduce, split along k (splits > 1): leave the slices in the workspace; the caller sums them (launch_splitk_sum, or
   // the RMSNorm kernel on its way in)
-  int32_t defer_reduce;
   // expert-indirect batches (one-row kernels only): when b_index is set, batch z reads its B
   // matrix at b + b_index[z * b_index_stride] * sb_index instead of the batch strides; an
   // index >= b_index_limit raises ERRF_INDEX_OOB in *err and is clamped
@@ -325,12 +325,10 @@ struct GemmDesc {
   // gated activation of an MLP applied where up_proj's product is still in registers;
   // c16: a bf16 copy of C, same indexing
   const float *glu_gate;
-  int32_t glu_kind;
   uint16_t *c16;
-  // optional (gemm_act_ok): C = sigmoid(A . B).  With c16_pitch the sigmoid leaves as bf16 only, in rows of c16_pitch
+  // act_sigmoid (gemm_act_ok): C = sigmoid(A . B).  With c16_pitch the sigmoid leaves as bf16 only, in rows of c16_pitch
   // (a multiple of 64, at least N) values at c16 with zeros past column N: the left operand of the next product as the
   // direct-to-LDS kernel reads it (c is not written; gemm_epilogue_ok, one batch)
-  int32_t act_sigmoid;
   uint32_t c16_pitch;
   // optional (same conditions): a second B matrix laid out like b (same strides, same N).  The kernel computes
   // both products and stores C = act(A . b) * (A . dual_b) - gate_proj, up_proj and the gated activation of an
@@ -353,11 +351,10 @@ struct GemmDesc {
   // and also transposed, as bf16 [sequence][head][rope_hd][position], at rope_out16 (rows of positions padded with
   // zeros to a multiple of 8).
   uint32_t rope_s, rope_hd;
-  uint32_t rope_role[3];
   float *rope_out[3];
   uint16_t *rope_out16[3];
   const float *rope_cos[3], *rope_sin[3];
-  int64_t rope_cs_ss[3];
+  uint32_t rope_cs_ss[3];
   // Role 3 (heads of 256, on 256 x 256 tiles only): as 1, every head's row RMS-normed in front of its rotation, the arithmetic of
   // rmsnorm_kernel - x / sqrt(sum(x * x) / rope_n_as_float + rope_eps) * (rope_gamma_offset + gamma) with gamma, rope_hd floats or null,
   // in the place of the bias, which it then does not have
@@ -366,8 +363,9 @@ struct GemmDesc {
   // the 100 MHz ticks its main loop took to clock_ticks[0] and [1]
   unsigned long long *clock_ticks;
 };
-// (up to eight lines of 64 bytes a kernel's arguments are touched in one trip: with nine a 37-token prompt took 1242 us, with eight 1218)
-static_assert(sizeof(GemmDesc) <= 512, "a GemmDesc is eight lines of kernel arguments");
+// (up to eight lines of 64 bytes a kernel's arguments are touched in one trip: with nine a 37-token prompt took 1242 us, with eight 1218.
+// The one-row kernels' two other arguments and the grid's size lie behind the descriptor, 20 bytes that are to be in the eighth.)
+static_assert(sizeof(GemmDesc) <= 488, "a GemmDesc and what lies behind it are eight lines of kernel arguments");
 // k_gemm_ring.hip: the 256 x 256 tiles of large bf16 products (plain or grouped, sigmoid, stacked gate / up);
 // half_height: the stacked gate / up of fewer rows on tiles of 128 x 256, K >= 192; wide: tiles of 256 x 288 (plain without groups or a
 // sigmoid, stacked gate / up), N % 4 == 0

@@ -1086,14 +1086,15 @@ int realize_matmul(cg_backend *be, cg_tensor *n, cg_tensor *addend, bool *added,
         while (j < 3 && rq->mm[j] != members[i]) ++j;
         if (j == 3) all = false;
         else if (j < 2) {
+          all = rq->cs_ss[j] >= 0 && rq->cs_ss[j] <= INT32_MAX;
           t.rope_role[i] = 1;
           t.rope_out[i] = rq->out[j];
           t.rope_out16[i] = rq->out16[j];
           t.rope_cos[i] = rq->cos[j];
           t.rope_sin[i] = rq->sin[j];
-          t.rope_cs_ss[i] = rq->cs_ss[j];
+          t.rope_cs_ss[i] = (uint32_t)rq->cs_ss[j];
           if (const RmsNormMatch *nm = rq->norm[j]) {
-            all = !t.grp_bias[i];
+            all = all && !t.grp_bias[i];
             t.rope_role[i] = 3;
             t.grp_bias[i] = nm->gamma ? (const float *)data_ptr(nm->gamma) : nullptr;
             t.rope_n_as_float = nm->n_as_float;
