@@ -79,3 +79,23 @@ def test_sigmoid(hip, M, N, K):
     exact = 1 / (1 + np.exp(-(x.astype(np.float64) @ w.astype(np.float64))))
     # (terms of size K^-1/2: their sums are off by 4 sqrt(K) 2^-24 of K^1/2 K^-1/2 at most; f32 exp and division: 4 units)
     assert np.abs(got - exact).max() <= 0.25 * 4 * np.sqrt(K) * 2.0 ** -24 + 4 * 2.0 ** -24
+
+
+# heights of an odd number of 16 rows: their last rows, the first past them, columns that end in either half of a wavefront's 32, a last
+# step of one piece, slices of k, a batch (test_kernel_choice.py asserts the heights)
+ODD_SIZES = [(1, 1, 33, 2048, 4100), (1, 1, 48, 4108, 1000), (2, 1, 65, 5380, 1404), (2, 1, 79, 4100, 2060), (3, 1, 97, 4100, 2060), (3, 2, 112, 2068, 1028),
+             (4, 1, 144, 2052, 4100), (5, 1, 175, 8196, 2060), (6, 1, 207, 5380, 1404), (7, 1, 225, 5380, 1404), (7, 1, 240, 5380, 1404)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("along_k", [True, False])
+@pytest.mark.parametrize("rows,B,M,N,K", ODD_SIZES)
+def test_product_of_an_odd_height(hip, rows, B, M, N, K, along_k):
+    test_product(hip, rows, B, M, N, K, along_k)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("along_k", [True, False])
+@pytest.mark.parametrize("rows,B,M,N,K", [s for s in ODD_SIZES if s[2] * s[3] < 1e6])
+def test_infinities_of_an_odd_height(hip, rows, B, M, N, K, along_k):
+    test_infinities(hip, rows, B, M, N, K, along_k)

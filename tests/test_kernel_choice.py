@@ -1,7 +1,7 @@
 """Which kernel a call is given, on the CPU: the library over the stand-in runtime of fake_hip.cpp, which says what was launched."""
 import pytest
 
-from test_f32_tiles import SIZES
+from test_f32_tiles import ODD_SIZES, SIZES
 from test_host_copies import fake_hip  # noqa: F401 - a fixture
 
 BF16 = 1
@@ -218,3 +218,15 @@ for s in (1, 5, 20, 200):
     (got,) = vectors.run(be, total, 1, np.zeros((s, 1, 128), np.float32), np.zeros((s, 2), np.uint32), up, up + 1, np.zeros((3, 128, 192), np.float32))
     assert got.shape == (s, 1, 128)
 """, BF16)
+
+
+def test_f32_tiles_of_odd_heights(fake_hip):  # noqa: F811
+    """16 rows more than a multiple of 32 for up to 512 rows; none beyond, nor for few k."""
+    fake_hip(LAUNCHED + f"""
+for rows, b, m, n, k in {ODD_SIZES}:
+    for along_k in (True, False):
+        (name,) = [x for x in product(m, n, k, along_k, b) if "gemm" in x and "splitk" not in x]
+        assert "gemm_f32_dma_kernelILi%dE" % rows in name and name.endswith("ELb%dELb1EEEvNS_8GemmDescE" % (not along_k)), (b, m, n, k, along_k, name)
+for b, m, n, k in ((1, 700, 2048, 8192), (1, 1000, 8192, 2048), (1, 130, 7312, 52), (1, 220, 30000, 100)):
+    assert all(x.endswith("ELb0EEEvNS_8GemmDescE") for x in product(m, n, k) if "dma" in x)
+""")
