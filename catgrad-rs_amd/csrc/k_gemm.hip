@@ -3078,7 +3078,7 @@ bool gemm_pack_wanted(const GemmDesc &g, bool epilogue) {
 // Which of a rotating product's tiles: 256 x 256 (ring_store_attention), or those of 128 columns and less.  A round of the large ones is
 // 1.7 rounds of 128 x 128 two to a CU (us, small and large; 3072 columns of heads of 64, K = 2048, two rounds and one: 2700 rows 64.6,
 // 57.4, 2900 63.6, 52.1, 3300 67.6, 58.2, 4090 86.4, 64.1; 6144 columns of heads of 128 with biases: 1400 68.3, 59.8, 5 x 290 78.3, 66.6).
-// Heads of 256 with their norm have no other: against a plain product, the rotation's launch and a transposition, 1536 columns, K =
+// Heads of 256 with their norm have no other but halves of them: against a plain product, the rotation's launch and a transposition, 1536 columns, K =
 // 1152, 3 x 1900 rows 65.3 and 45.6, 6 x 1999 112.6 and 86.9, 8 x 2048 (two rounds) 115 and 96.6; below two rounds of 128 x 128 the plain
 // product's tiles are smaller.
 static bool rope_on_large_tiles(const LaunchCtx &lc, const GemmDesc &g) {
@@ -3087,6 +3087,16 @@ static bool rope_on_large_tiles(const LaunchCtx &lc, const GemmDesc &g) {
                  t128 = (uint64_t)((g.M + 127) / 128) * ((g.N + 127) / 128);
   const uint64_t large = (t256 + cus - 1) / cus, small = (t128 + 2 * cus - 1) / (2 * cus);
   return g.rope_hd == 256 ? t128 > 2 * cus : g.K >= 768 && large * 17 <= small * 10;
+}
+
+// ... or those of 128 x 256 in one round, where 128 x 128 are two to a CU (us, 128 x 128 and 128 x 256, K = 2048: 3072 columns of heads of 64,
+// 1290 rows 41.0, 35.4, 1700 40.4, 34.5, 2048 42.7, 36.4, 2688 44.3, 38.8; 6144 of heads of 128 with biases, 650 54.3, 37.2, 800 42.5, 35.9,
+// 1024 45.4, 37.0, 1280 47.1, 40.5; 1536 of heads of 256 with their norm, K = 1152, 2700 rows 25.0, 4096 26.8, 5376 28.7, where the plain
+// product took 18.7, 24.3 and 26.1 and the rotation and a transposition launches of their own).
+static bool rope_on_half_tiles(const LaunchCtx &lc, const GemmDesc &g) {
+  if (!gemm_ring_ok(g) || g.K < 768) return false;
+  const uint64_t cus = (uint64_t)lc.n_cus, m128 = (g.M + 127) / 128;
+  return m128 * ((g.N + 127) / 128) > cus && m128 * ((g.N + 255) / 256) <= cus;
 }
 
 bool gemm_rope_epilogue_ok(const LaunchCtx &lc, const GemmDesc &g) {
@@ -3106,9 +3116,9 @@ bool gemm_rope_epilogue_ok(const LaunchCtx &lc, const GemmDesc &g) {
     }
   }
   // launch_matmul's tiles of 32 to 128 rows have this epilogue (128 columns, or 64 - for heads of 64 - where those are
-  // too few for the CUs), and 256 x 256, which alone hold heads of 256 and norm; several rounds of products that are not for those are
+  // too few for the CUs), and 128 or 256 x 256, which alone hold heads of 256 and norm; several rounds of products that are not for those are
   // better left without
-  if (rope_on_large_tiles(lc, g)) return true;
+  if (rope_on_large_tiles(lc, g) || rope_on_half_tiles(lc, g)) return true;
   const uint64_t t256 = (uint64_t)((g.M + 255) / 256) * ((g.N + 255) / 256);
   return g.rope_hd != 256 && g.N >= 128 && !(t256 >= (uint64_t)lc.n_cus && grp256);
 }
@@ -3318,6 +3328,8 @@ hipError_t launch_matmul(const LaunchCtx &lc_in, const GemmDesc &g, const char *
       };
       if (g.rope_s && rope_on_large_tiles(lc, g)) {
         e = launch_gemm_ring(lc, gg);
+      } else if (g.rope_s && rope_on_half_tiles(lc, g)) {
+        e = launch_gemm_ring(lc, gg, true);
       } else if (g.rope_s && g.M <= 128) {
         // q / k / v of a few rows: a workgroup takes in its rows of both operands at about 42 GB/s however wide its tile is,
         // and 64 x 64 or 128 x 64 tiles are 48 workgroups for 3072 columns.  32 x 32 tiles, of columns that rotate into
@@ -3466,6 +3478,11 @@ hipError_t launch_matmul(const LaunchCtx &lc_in, const GemmDesc &g, const char *
           // 6000 x 700 x 256 10.4, 11.7).
           if (steps >= 10) e = launch_gemm_plain<192, 128, 2, 2, 4, 1, true>(lc, gg, t192);
           else e = launch_gemm_plain<192, 128, 2, 4, 3>(lc, gg, t192);
+        } else if (splits == 1 && steps >= 16 && grp256 && gemm_ring_ok(gg) && (uint64_t)((g.M + 127) / 128) * ((g.N + 255) / 256) * batch <= cus) {
+          // A round of 128 x 256 where 128 x 128 are two to a CU and 192 rows more than a round (us there and here: 3100 x 2048, K = 512 14.5,
+          // 14.2, 768 17.4, 17.6, 1024 20.7, 20.0, 2048 35.1, 30.4, 8192 117, 98; 4000 rows 15.7, 15.9; 19.4, 19.3; 23.0, 22.0; 39, 34; 128, 108;
+          // 1000 x 6144 x 2048 39.3, 31.2; 2300 x 3000 x 2048 39.5, 32.4, x 512 14.5, 15.5; 6400 x 1152 x 6912 111, 96.8).
+          e = launch_gemm_ring(lc, gg, true);
         } else if (steps >= 64) {
           // Several rounds of a deep product, a round of 192 rows at 1.42 times one of 128: 8192 x 1152 x 6912 two or three, 134 and 148 us
           // (two to a CU 167); 4000 x 2048 x 8192 two either way, 149 and 130 (145); 3100 rows 144 and 117 (122).

@@ -532,8 +532,8 @@ __device__ __forceinline__ void ring_store_values(const RingRope &d, uint32_t ro
 }
 
 // (one place that reads the accumulators: where two branches do, the compiler spills them)
-template <int HD, bool BIAS, bool NORM>
-__device__ __forceinline__ void ring_store_attention(const RingRope d, bool values, uint32_t m0, uint32_t n0, const f32x16 (&acc)[2][2][2][2], float *smem) {
+template <int HD, bool BIAS, bool NORM, int AH>
+__device__ __forceinline__ void ring_store_attention(const RingRope d, bool values, uint32_t m0, uint32_t n0, const f32x16 (&acc)[AH][2][2][2], float *smem) {
   const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wm = wave >> 1, wn = wave & 1;
   float *mine = smem + wave * 8192;
   auto half_tile = [&](auto A) __attribute__((always_inline)) {
@@ -548,10 +548,10 @@ __device__ __forceinline__ void ring_store_attention(const RingRope d, bool valu
     else ring_store_rotated<HD, NORM>(d, p, n0, smem, wave, lane);
   };
   half_tile(std::integral_constant<int, 0>());
-  half_tile(std::integral_constant<int, 1>());
+  if constexpr (AH == 2) half_tile(std::integral_constant<int, 1>());
 }
 
-// AH: halves of 128 rows to a tile, two or (RING_SILU, RING_GELU) one.  WIDE: with the strip of 32 columns (RING_SILU, RING_GELU: 16
+// AH: halves of 128 rows to a tile, two or (not RING_SIGMOID) one.  WIDE: with the strip of 32 columns (RING_SILU, RING_GELU: 16
 // rows of each matrix), N % 4 == 0.
 template <int KIND, int AH, bool WIDE = false>
 __global__ void __launch_bounds__(256, 1) gemm_bf16_ring_kernel(GemmDesc g) {
@@ -563,7 +563,7 @@ __global__ void __launch_bounds__(256, 1) gemm_bf16_ring_kernel(GemmDesc g) {
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), wm = wave >> 1, wn = wave & 1;
   constexpr uint32_t BM = AH * 128;
-  static_assert(AH == 2 || GATED, "the epilogues of 128-row tiles");
+  static_assert(AH == 2 || KIND != RING_SIGMOID, "the epilogues of 128-row tiles");
   const uint32_t tiles_m = (g.M + BM - 1) / BM, tiles_n = (g.N + BNO - 1) / BNO;
   const TilePlace place(tiles_m, tiles_n, g.nb0, g.nb1, max(g.splits, 1u));
   const uint32_t batch = g.nb0 * g.nb1, split = place.split, bz = place.bz, b0 = place.b0, b1 = place.b1;
@@ -707,7 +707,7 @@ __global__ void __launch_bounds__(256, 1) gemm_bf16_ring_kernel(GemmDesc g) {
                         late->rope_out16[grp], late->rope_cs_ss[grp], late->rope_n_as_float, late->rope_eps, late->rope_gamma_offset,
                         late->M, late->grp_n[grp], late->rope_s};
     constexpr int HD = KIND >= RING_ROPE_256 ? 256 : KIND >= RING_ROPE_128 ? 128 : 64;
-    ring_store_attention<HD, KIND == RING_ROPE_64_BIAS || KIND == RING_ROPE_128_BIAS, KIND == RING_ROPE_256_NORM>(d, late->rope_role[grp] == 2, m0, n0, acc, ring_smem);
+    ring_store_attention<HD, KIND == RING_ROPE_64_BIAS || KIND == RING_ROPE_128_BIAS, KIND == RING_ROPE_256_NORM, AH>(d, late->rope_role[grp] == 2, m0, n0, acc, ring_smem);
     return;
   }
   uint16_t *C16 = g.c16 ? g.c16 + (uint64_t)bz * g.M * g.N : nullptr;
@@ -722,7 +722,7 @@ __global__ void __launch_bounds__(256, 1) gemm_bf16_ring_kernel(GemmDesc g) {
     to[u] = (at_row[u] * pitch + at_col[u]) * (F32 ? 4u : 2u);
   }
 #pragma unroll
-  for (int qd = 0; qd < (GATED ? AH : 4); ++qd) {
+  for (int qd = 0; qd < (GATED ? AH : 2 * AH); ++qd) {
     const int a = GATED ? qd : qd >> 1, b = GATED ? 0 : qd & 1;
     float *tile = ring_smem + wave * 8192 + (qd & 1) * 4096;
     const uint32_t col0 = n0 + b * 128 + wn * 64, row0 = m0 + a * 128 + wm * 64;
@@ -1037,25 +1037,30 @@ static hipError_t launch_ring_as(const LaunchCtx &lc, const GemmDesc &g, uint32_
   return hipGetLastError();
 }
 
+template <int AH>
+static hipError_t launch_ring_rope(const LaunchCtx &lc, const GemmDesc &g, uint32_t grid) {
+  const bool bias = g.grp_bias[0] != nullptr, norm = g.rope_role[0] == 3 || g.rope_role[1] == 3 || g.rope_role[2] == 3;
+  if (g.rope_hd == 256) return norm ? launch_ring_as<RING_ROPE_256_NORM, AH>(lc, g, grid) : launch_ring_as<RING_ROPE_256, AH>(lc, g, grid);
+  if (g.rope_hd == 128) return bias ? launch_ring_as<RING_ROPE_128_BIAS, AH>(lc, g, grid) : launch_ring_as<RING_ROPE_128, AH>(lc, g, grid);
+  return bias ? launch_ring_as<RING_ROPE_64_BIAS, AH>(lc, g, grid) : launch_ring_as<RING_ROPE_64, AH>(lc, g, grid);
+}
+
 hipError_t launch_gemm_ring(const LaunchCtx &lc, const GemmDesc &g, bool half_height, bool wide) {
   if (!gemm_ring_ok(g)) return hipErrorInvalidValue;
   if (half_height) {
-    if (!g.dual_b || g.splits > 1 || g.K < 192) return hipErrorInvalidValue;
-    const uint64_t tiles = (uint64_t)((g.M + 127) / 128) * ((g.N + 127) / 128) * g.nb0 * g.nb1;
+    if (g.act_sigmoid || g.splits > 1 || g.K < 192) return hipErrorInvalidValue;
+    const uint32_t bno = g.dual_b ? 128 : 256;
+    const uint64_t tiles = (uint64_t)((g.M + 127) / 128) * ((g.N + bno - 1) / bno) * g.nb0 * g.nb1;
     if (tiles > 0x7FFFFFFFull) return hipErrorInvalidValue;
+    if (g.rope_s) return launch_ring_rope<1>(lc, g, (uint32_t)tiles);
+    if (!g.dual_b) return launch_ring_as<RING_PLAIN, 1>(lc, g, (uint32_t)tiles);
     return g.glu_kind ? launch_ring_as<RING_GELU, 1>(lc, g, (uint32_t)tiles) : launch_ring_as<RING_SILU, 1>(lc, g, (uint32_t)tiles);
   }
   if (wide && (g.N % 4 || g.n_group || g.act_sigmoid)) return hipErrorInvalidValue;
   const uint32_t bno = (g.dual_b ? 128 : 256) + (wide ? (g.dual_b ? 16 : 32) : 0), batch = g.nb0 * g.nb1 * (g.splits > 1 ? g.splits : 1);
   const uint64_t grid = (uint64_t)((g.M + 255) / 256) * ((g.N + bno - 1) / bno) * batch;
   if (grid > 0x7FFFFFFFull) return hipErrorInvalidValue;
-  if (g.rope_s) {
-    if (wide) return hipErrorInvalidValue;
-    const bool bias = g.grp_bias[0] != nullptr;
-    if (g.rope_hd == 256) return g.rope_role[0] == 3 || g.rope_role[1] == 3 || g.rope_role[2] == 3 ? launch_ring_as<RING_ROPE_256_NORM>(lc, g, (uint32_t)grid) : launch_ring_as<RING_ROPE_256>(lc, g, (uint32_t)grid);
-    if (g.rope_hd == 128) return bias ? launch_ring_as<RING_ROPE_128_BIAS>(lc, g, (uint32_t)grid) : launch_ring_as<RING_ROPE_128>(lc, g, (uint32_t)grid);
-    return bias ? launch_ring_as<RING_ROPE_64_BIAS>(lc, g, (uint32_t)grid) : launch_ring_as<RING_ROPE_64>(lc, g, (uint32_t)grid);
-  }
+  if (g.rope_s) return wide ? hipErrorInvalidValue : launch_ring_rope<2>(lc, g, (uint32_t)grid);
   if (wide && g.dual_b)
     return g.glu_kind ? launch_ring_as<RING_GELU, 2, true>(lc, g, (uint32_t)grid) : launch_ring_as<RING_SILU, 2, true>(lc, g, (uint32_t)grid);
   if (wide) return launch_ring_as<RING_PLAIN, 2, true>(lc, g, (uint32_t)grid);

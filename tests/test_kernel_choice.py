@@ -230,3 +230,14 @@ for rows, b, m, n, k in {ODD_SIZES}:
 for b, m, n, k in ((1, 700, 2048, 8192), (1, 1000, 8192, 2048), (1, 130, 7312, 52), (1, 220, 30000, 100)):
     assert all(x.endswith("ELb0EEEvNS_8GemmDescE") for x in product(m, n, k) if "dma" in x)
 """)
+
+
+def test_tiles_of_128_x_256(fake_hip):  # noqa: F811
+    """One round of them where 128 x 128 are two to a CU and 192 rows more than a round, from 16 k-steps on; the sizes of test_large_tiles.py."""
+    fake_hip(LAUNCHED + """
+for m, n, k, half in ((3100, 2050, 1024, True), (3333, 2049, 1088, True), (2300, 3001, 2048, True), (1000, 6143, 1152, True), (4096, 2048, 4160, True),
+                      (3100, 2050, 960, False), (2900, 2048, 2048, False), (4100, 2050, 2048, False)):
+    for residual in (False, True):
+        names = product(m, n, k, residual=residual)
+        assert len(names) == 1 and ("gemm_bf16_ring_kernelILi0ELi1E" in names[0]) == half, (m, n, k, names)
+""", BF16)

@@ -245,6 +245,34 @@ def test_rotated_on_large_tiles(hip_bf16, hd, batch, S, heads, kv, K, bias, norm
     parity.assert_bf16((scores / scores.sum(axis=-1, keepdims=True)) @ values, got, "attention")
 
 
+# ... and on tiles of 128 x 256, where those are one round
+@pytest.mark.gpu
+@pytest.mark.parametrize("hd,batch,S,heads,kv,K,bias,norm", [(64, 1, 1203, 20, 20, 768, False, False), (64, 6, 203, 20, 20, 832, True, False),
+                                                             (128, 5, 151, 16, 16, 768, True, False), (128, 1, 1202, 16, 16, 832, False, False),
+                                                             (256, 11, 257, 4, 1, 768, False, True), (256, 45, 64, 4, 1, 832, False, True),
+                                                             (256, 11, 270, 4, 1, 768, False, False)])
+def test_rotated_on_half_tiles(hip_bf16, hd, batch, S, heads, kv, K, bias, norm):
+    test_rotated_on_large_tiles(hip_bf16, hd, batch, S, heads, kv, K, bias, norm)
+
+
+# 128 x 256 in one round: the fewest k-steps, an odd number, rows and columns that end inside a tile, rows of results off 16 bytes, a batch
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(3100, 2050, 1024), (3333, 2049, 1088), (2300, 3001, 2048), (1000, 6143, 1152), (4096, 2048, 4160)])
+def test_half_height_product(hip_bf16, M, N, K):
+    test_product(hip_bf16, M, N, K)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,M,N,K", [(1, 3100, 2050, 1024), (1, 4000, 2048, 1088), (2, 1601, 2047, 1024)])
+def test_half_height_product_and_residual(hip_bf16, B, M, N, K):
+    test_product_and_residual(hip_bf16, B, M, N, K)
+
+
+@pytest.mark.gpu
+def test_half_height_infinities(hip_bf16):
+    test_infinities(hip_bf16, 3333, 2049, 1088)
+
+
 # attention whose result only a product of many rows reads: queries and result as bf16 only.  The product with one is that result, and the
 # same bits as the f32 result rounded, which another reader has it store; every form of the kernel, a batch, keys that end inside a tile
 @pytest.mark.gpu
