@@ -382,11 +382,15 @@ struct RowBest {  // what is known of a part of a row
 // A group of values costs a value one maximum, a subtraction, a product, the hardware's exp2 and a sum: exp(x - m) is 2 to the rounded
 // product of the rounded difference and log2 e, 6e-8 |x - m| off for one value, with a weight that falls as exp(x - m) does, and of either
 // sign from value to value.  (Error against 64 bits over 4096 x 4096, 300 x 50000, 8000 x 300 values of
-// deviation 2: 5.2e-8 to 5.4e-8, as with expf.  4096 x 4096 f32 17.9 us with expf and every value ordered, 15.3 so; 120 x 131072 19.4, 13.2.)  The column is looked for when the
-// largest value is known, by the threads that hold it, in the group they met it in; a group with a NaN, which no maximum shows but the
-// sum does, is ordered value by value.
-// TPR threads to a row, GROUP values to a thread and turn.
-template <typename T, int TPR, int GROUP = 16>
+// deviation 2: 5.2e-8 to 5.4e-8, as with expf.  4096 x 4096 f32 17.9 us with expf and every value ordered, 15.3 so; 120 x 131072 19.4, 13.2.)
+// The column is looked for when the largest value is known, by the threads that hold it, in the group they met it in: every wave does that
+// for all of its registers, so the value is compared as it is, a comparison and a move, and by its place in the order only where several
+// values share it or compare as nothing does (zeros, NaN; 4096 x 4096 16.6 -> 15.4 us, 8192 x 1500 13.5 -> 12.0).  A group with a NaN, which
+// no maximum shows but the sum does, is ordered value by value.
+// TPR threads to a row, GROUP values to a thread and turn.  WHOLE: a turn that ends inside the row asks for its pieces without a look at each
+// (rows that have such turns: the two ways to the values cost the others 64 moves.  us without and with: f32 4096 x 4096 15.5, 14.4, 8192 x
+// 2048 14.3, 13.8, bf16 12.1, 10.4 and 12.0, 9.2; f32 8192 x 1500 11.9, 12.7, 2000 x 4000 9.1, 10.1.)
+template <typename T, int TPR, int GROUP, bool WHOLE>
 __global__ void __launch_bounds__(256) softmax_best_kernel(SoftmaxBestDesc d) {
   constexpr int W = sizeof(T) == 4 ? 4 : 8, U = GROUP / W, RPB = 256 / TPR;
   __shared__ float part[4][4];
@@ -399,25 +403,28 @@ __global__ void __launch_bounds__(256) softmax_best_kernel(SoftmaxBestDesc d) {
     float m = -3.40282347e+38f;
     float v[U][W];
     uint32_t at = 0, held = 0;  // where the group that holds this thread's largest value starts; the group in v
+    auto piece = [&](int u, const T *from) __attribute__((always_inline)) {
+      uint4 q;
+      __builtin_memcpy(&q, __builtin_assume_aligned(from, sizeof(T)), 16);
+      const uint32_t h[4] = {q.x, q.y, q.z, q.w};
+      if constexpr (sizeof(T) == 4) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[u][j] = __uint_as_float(h[j]);
+      } else {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          v[u][2 * j] = __uint_as_float(h[j] << 16);
+          v[u][2 * j + 1] = __uint_as_float(h[j] & 0xFFFF0000u);
+        }
+      }
+    };
     auto fetch = [&](uint32_t c0) __attribute__((always_inline)) {
       held = c0;
 #pragma unroll
       for (int u = 0; u < U; ++u) {
         const uint32_t c = c0 + u * TPR * W;
         if (c + W <= c_end) {
-          uint4 q;
-          __builtin_memcpy(&q, __builtin_assume_aligned(x + c, sizeof(T)), 16);
-          const uint32_t h[4] = {q.x, q.y, q.z, q.w};
-          if constexpr (sizeof(T) == 4) {
-#pragma unroll
-            for (int j = 0; j < 4; ++j) v[u][j] = __uint_as_float(h[j]);
-          } else {
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-              v[u][2 * j] = __uint_as_float(h[j] << 16);
-              v[u][2 * j + 1] = __uint_as_float(h[j] & 0xFFFF0000u);
-            }
-          }
+          piece(u, x + c);
         } else {
 #pragma unroll
           for (int j = 0; j < W; ++j) {
@@ -435,7 +442,13 @@ __global__ void __launch_bounds__(256) softmax_best_kernel(SoftmaxBestDesc d) {
       return w ^ ((uint32_t)((int32_t)w >> 31) | 0x80000000u);
     };
     for (uint32_t c0 = c_begin + t * W; c0 < c_end; c0 += TPR * W * U) {
-      fetch(c0);
+      if (WHOLE && __builtin_amdgcn_readfirstlane(c0 - t * W) + U * TPR * W <= c_end) {
+        held = c0;
+#pragma unroll
+        for (int u = 0; u < U; ++u) piece(u, x + c0 + u * TPR * W);
+      } else {
+        fetch(c0);
+      }
       float gm = -INFINITY;
 #pragma unroll
       for (int u = 0; u < U; ++u)
@@ -471,13 +484,22 @@ __global__ void __launch_bounds__(256) softmax_best_kernel(SoftmaxBestDesc d) {
       const uint32_t best = (uint32_t)wave_max_i32((int32_t)(b.key ^ 0x80000000u)) ^ 0x80000000u;
       if (b.key == best && c_begin + t * W < c_end) {  // (usually one thread of the wave)
         if (at != held) fetch(at);
+        const float value = __uint_as_float(best & 0x80000000u ? best ^ 0x80000000u : ~best);
+        if (value != 0.f && value == value && value > -INFINITY) {  // the value whose key it is, and no other (past the end of a row are -inf)
 #pragma unroll
-        for (int u = 0; u < U; ++u)
+          for (int u = 0; u < U; ++u)
 #pragma unroll
-          for (int j = 0; j < W; ++j) {
-            const uint32_t c = at + u * TPR * W + j;
-            if (c < c_end && key_of(v[u][j]) == best) b.col = c;
-          }
+            for (int j = 0; j < W; ++j)
+              if (v[u][j] == value) b.col = at + u * TPR * W + j;
+        } else {
+#pragma unroll
+          for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int j = 0; j < W; ++j) {
+              const uint32_t c = at + u * TPR * W + j;
+              if (c < c_end && key_of(v[u][j]) == best) b.col = c;
+            }
+        }
       }
     }
   }
@@ -535,14 +557,20 @@ hipError_t launch_softmax_best(const LaunchCtx &lc, const SoftmaxBestDesc &in) {
   const uint32_t most = d.rows >= (uint32_t)lc.n_cus * 8 ? 4096 : d.rows >= (uint32_t)lc.n_cus * 4 ? 2048 : 1024;
   const bool wave = d.chunks == 1 && d.n <= most;
   const unsigned grid = wave ? (d.rows + 3) / 4 : d.rows * d.chunks;
-#define CG_BEST(T)                                                                                \
-  if (wave && d.n > 2048) CG_LAUNCH(lc, (softmax_best_kernel<T, 64, 64>), grid, 256, d);          \
-  else if (wave && d.n > 1024) CG_LAUNCH(lc, (softmax_best_kernel<T, 64, 32>), grid, 256, d);     \
-  else if (wave) CG_LAUNCH(lc, (softmax_best_kernel<T, 64>), grid, 256, d);                       \
-  else CG_LAUNCH(lc, (softmax_best_kernel<T, 256>), grid, 256, d);
+#define CG_BEST_AS(T, TPR, GROUP)                                                                                          \
+  do {                                                                                                                     \
+    if (std::min(d.n, d.chunk_len) >= TPR * GROUP) CG_LAUNCH(lc, (softmax_best_kernel<T, TPR, GROUP, true>), grid, 256, d);  \
+    else CG_LAUNCH(lc, (softmax_best_kernel<T, TPR, GROUP, false>), grid, 256, d);                                         \
+  } while (0)
+#define CG_BEST(T)                                        \
+  if (wave && d.n > 2048) CG_BEST_AS(T, 64, 64);          \
+  else if (wave && d.n > 1024) CG_BEST_AS(T, 64, 32);     \
+  else if (wave) CG_BEST_AS(T, 64, 16);                   \
+  else CG_BEST_AS(T, 256, 16);
   if (d.x_bf16) { CG_BEST(uint16_t) }
   else { CG_BEST(float) }
 #undef CG_BEST
+#undef CG_BEST_AS
   if (d.chunks > 1) {
     LaunchCtx untimed = lc;  // the events stay with the pass over x
     untimed.ev_start = untimed.ev_stop = nullptr;

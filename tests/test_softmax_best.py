@@ -83,3 +83,16 @@ def test_special_values_in_several_groups(oracle, hip, n):
 @pytest.mark.parametrize("shape", [(1030, 1031), (1024, 2048), (2050, 2049), (2048, 4096), (2051, 4095), (2048, 4097)])
 def test_a_wave_to_a_longer_row(oracle, hip, hip_bf16, shape):
     test_best_of_rows(oracle, hip, hip_bf16, shape)
+
+
+# turns that end inside the row: exactly one, several, one and a part, of a wave and of a workgroup
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", [(40, 1024), (1024, 1024), (2100, 2048), (9, 4096), (5, 12288), (7, 12289), (3, 4103), (2, 65536)])
+def test_whole_turns(oracle, hip, hip_bf16, shape):
+    test_best_of_rows(oracle, hip, hip_bf16, shape)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [1024, 4096, 8192, 8200])
+def test_special_values_in_whole_turns(oracle, hip, n):
+    test_special_values_in_several_groups(oracle, hip, n)
