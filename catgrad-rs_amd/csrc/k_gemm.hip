@@ -2852,28 +2852,64 @@ __global__ void __launch_bounds__(16 * KS) gemv_col_kernel(GemmDesc g, int b_vec
   for (int m = 0; m < MROWS; ++m)
 #pragma unroll
     for (int j = 0; j < 4; ++j) acc[m][j] = 0.f;
-  for (uint32_t k = ks; k < g.K; k += KS) {
-    const TB *brow = B + (int64_t)k * g.sbk + n;
-    float w[4];
-    if (b_vec && n + 4 <= g.N) {
-      if (sizeof(TB) == 4) {
-        float4 q = *(const float4 *)brow;
-        w[0] = q.x; w[1] = q.y; w[2] = q.z; w[3] = q.w;
+  // One row: the compiler asks for several steps' values ahead by itself (14.8 us for 1 x 2048 x 64, 30.5 in fours).  More rows: four steps'
+  // values, all asked for before the first is used; one step at a time was a trip to memory each (5 rows f32 of 1073 x 743 54 -> 27 us, 1024
+  // x 2048 40 -> 26, 2048 x 64 110 -> 44, bf16 weights 743 x 69 52 -> 29).
+  if constexpr (MROWS == 1) {
+    for (uint32_t k = ks; k < g.K; k += KS) {
+      const TB *brow = B + (int64_t)k * g.sbk + n;
+      float w[4];
+      if (b_vec && n + 4 <= g.N) {
+        if (sizeof(TB) == 4) {
+          float4 q = *(const float4 *)brow;
+          w[0] = q.x; w[1] = q.y; w[2] = q.z; w[3] = q.w;
+        } else {
+          uint2 q = *(const uint2 *)brow;
+          w[0] = __uint_as_float(q.x << 16); w[1] = __uint_as_float(q.x & 0xFFFF0000u);
+          w[2] = __uint_as_float(q.y << 16); w[3] = __uint_as_float(q.y & 0xFFFF0000u);
+        }
       } else {
-        uint2 q = *(const uint2 *)brow;
-        w[0] = __uint_as_float(q.x << 16); w[1] = __uint_as_float(q.x & 0xFFFF0000u);
-        w[2] = __uint_as_float(q.y << 16); w[3] = __uint_as_float(q.y & 0xFFFF0000u);
-      }
-    } else {
 #pragma unroll
-      for (int j = 0; j < 4; ++j) w[j] = n + j < g.N ? widen(brow[j]) : 0.f;
+        for (int j = 0; j < 4; ++j) w[j] = n + j < g.N ? widen(brow[j]) : 0.f;
+      }
+      const float xv = A[(int64_t)k * g.sak];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) acc[0][j] += xv * w[j];
+    }
+  }
+  constexpr int U = 4;
+  for (uint32_t k0 = ks; MROWS > 1 && k0 < g.K; k0 += KS * U) {
+    float w[U][4], xv[U][MROWS];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const uint32_t k = min(k0 + u * KS, g.K - 1);
+      const TB *brow = B + (int64_t)k * g.sbk;
+      if (b_vec && n + 4 <= g.N) {
+        if (sizeof(TB) == 4) {
+          float4 q = *(const float4 *)(brow + n);
+          w[u][0] = q.x; w[u][1] = q.y; w[u][2] = q.z; w[u][3] = q.w;
+        } else {
+          uint2 q = *(const uint2 *)(brow + n);
+          w[u][0] = __uint_as_float(q.x << 16); w[u][1] = __uint_as_float(q.x & 0xFFFF0000u);
+          w[u][2] = __uint_as_float(q.y << 16); w[u][3] = __uint_as_float(q.y & 0xFFFF0000u);
+        }
+      } else {  // (columns past the end repeat the last one: their sums are not stored)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) w[u][j] = widen(brow[min(n + j, g.N - 1)]);
+      }
+#pragma unroll
+      for (int m = 0; m < MROWS; ++m)
+        if ((uint32_t)m < g.M) xv[u][m] = A[(int64_t)m * g.sam + (int64_t)k * g.sak];
     }
 #pragma unroll
-    for (int m = 0; m < MROWS; ++m) {
-      if ((uint32_t)m < g.M) {
-        const float xv = A[(int64_t)m * g.sam + (int64_t)k * g.sak];
+    for (int u = 0; u < U; ++u) {
+      if (k0 + u * KS >= g.K) break;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) acc[m][j] += xv * w[j];
+      for (int m = 0; m < MROWS; ++m) {
+        if ((uint32_t)m < g.M) {
+#pragma unroll
+          for (int j = 0; j < 4; ++j) acc[m][j] += xv[u][m] * w[u][j];
+        }
       }
     }
   }
@@ -3171,7 +3207,9 @@ uint32_t gemm_split_k(const LaunchCtx &lc, const GemmDesc &g) {
   if (gemm_small_ok(lc, g)) return gemm_small_split(lc, g);
   if (!gemm_fast_path(g, av, bv)) {
     // the generic kernel (f32 products): same idea, shorter k-steps, so thinner slices still pay
-    if (g.M <= 8 || g.b_index || !g.K) return 1;
+    // (the one-row kernels, which take f32 rows only; 5 bf16 rows of 1073 values by 743 columns 119 us in one slice, 30 in eight
+    // and their sum, 1 or 5 of 1024 by 2048 67, 17)
+    if ((g.M <= 8 && g.a_stype == ST_F32 && (g.sbk == 1 || g.sbn == 1 || g.K == 1 || g.N == 1)) || g.b_index || !g.K) return 1;
     // (two workgroups to a CU, one's loads under the other's products: 700 x 2048 x 8192 357 -> 312 us, 400 x 2048 x 8192
     // 185 -> 168; four k-steps at least to each: 1000 x 1000 x 1000 54 -> 36, 100 x 2048 x 2048 33 -> 27; four workgroups
     // to a CU were slower throughout.  A shallow product does not pay for the second workgroup's slices, unless its sums are

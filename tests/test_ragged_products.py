@@ -110,3 +110,27 @@ def test_rounding_of_rows(hip_bf16, lower):
     rows = x.shape[0]
     (got,) = vectors.run(hip_bf16, lambda b, x, w: [lang.matmul(b, lang.reshape(b, lang.make_shape(b, rows, 128), x), w)], 1, x.ravel(), np.eye(128, dtype=np.float32))
     assert np.array_equal(got, vectors.bf16_round(x))
+
+
+# 1 to 8 rows: bf16 rows in slices of k, f32 rows a few steps of k at a time; columns that end inside a piece and inside 64, k off every
+# step, infinities at either end of k
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,K,H,N", [(1, 1073, 743, 69), (5, 1073, 743, 69), (8, 257, 130, 65), (2, 63, 66, 3), (7, 2048, 515, 10), (3, 129, 64, 64)])
+@pytest.mark.parametrize("mode", ["hip", "hip_bf16"])
+def test_a_few_ragged_rows(request, mode, M, K, H, N):
+    be, g = request.getfixturevalue(mode), np.random.default_rng(M * K)
+    rounded = lambda s, std: vectors.bf16_round((g.standard_normal(s) * std).astype(np.float32))
+    x, w1, w2 = rounded((M, K), 1.0), rounded((K, H), K ** -0.5), rounded((H, N), H ** -0.5)
+    y, h = vectors.run(be, lambda b, x, w1, w2: [lang.matmul(b, lang.matmul(b, x, w1) * lang.matmul(b, x, w1), w2), lang.matmul(b, x, w1)], 2, x, w1, w2)
+    x64, w64 = x.astype(np.float64), w1.astype(np.float64)
+    ref, bound = x64 @ w64, K * 2.0 ** -24 * (np.abs(x64) @ np.abs(w64))     # K f32 additions of exact products
+    assert np.all(np.abs(h - ref) <= bound)
+    rows = (h * h).astype(np.float64)
+    # (f32 rows as they are, or rounded to bf16 where the product does that)
+    bound = ((2.0 ** -8 if be.name.startswith("hip") and mode == "hip_bf16" else 0) + (H + 1) * 2.0 ** -24) * (rows @ np.abs(w2.astype(np.float64)))
+    assert np.all(np.abs(y - rows @ w2.astype(np.float64)) <= bound)
+    x[0, 0], x[-1, -1] = np.inf, np.nan
+    (h,) = vectors.run(be, lambda b, x, w1: [lang.matmul(b, x, w1)], 1, x, w1)
+    with np.errstate(invalid="ignore"):
+        ref = x.astype(np.float64) @ w64
+    assert np.array_equal(np.isnan(h), np.isnan(ref)) and np.array_equal(np.isinf(h), np.isinf(ref))
