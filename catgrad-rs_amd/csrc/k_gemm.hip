@@ -3342,8 +3342,9 @@ hipError_t launch_matmul(const LaunchCtx &lc_in, const GemmDesc &g, const char *
     // 18.5 -> 15.6, 100 20.1 -> 18.5; 17 x 16384 x 2048 18.3 -> 15.2, x 8192 58.7 -> 49.8; 64 x 32000 x 8192 134 -> 114; 128 x 32000 x
     // 4096 65 -> 56; 64 x 4096 x 8192 in four slices 19.7 -> 17.5.  Slices of half of 4 KB start at different k as they are (37 x 2048
     // x 8192 in eight 10.7, 11.3); rows an odd number of KB apart meet all channels (64 x 2 x 4096 x 2560 20.8, 21.1); more row tiles
-    // share the weights, and their rows are then in the L2s for one step only (2900 x 2048 x 8192 95 and 134, 8192^3 745 and 805).
-    gg.k_rotate = g.M <= 128 && g.sbk == 1 && g.sbn % 2048 == 0 && gg.k_per_split >= 2048;
+    // share the weights, and their rows are then in the L2s for one step only (2900 x 2048 x 8192 95 and 134, 8192^3 745 and 805).  q / k / v
+    // that rotate, tiles of 32 columns: 37 rows 12.0 us as they are, 12.6 so, 100 rows 12.3, 13.3.
+    gg.k_rotate = g.M <= 128 && !g.rope_s && g.sbk == 1 && g.sbn % 2048 == 0 && gg.k_per_split >= 2048;
     if (gemm_dma_ok(g)) {
       const uint64_t t256 = (uint64_t)((g.M + 255) / 256) * ((g.N + 255) / 256) * batch * splits;
       hipError_t e;
