@@ -2844,8 +2844,11 @@ __global__ void __launch_bounds__(16 * KS) gemv_col_kernel(GemmDesc g, int b_vec
   const uint32_t bz = blockIdx.y, b0 = bz / g.nb1, b1 = bz - b0 * g.nb1;
   const float *A = (const float *)g.a + b0 * g.sa_b0 + b1 * g.sa_b1;
   const TB *B = (const TB *)g.b + b_batch_offset(g, bz, b0, b1);
-  float *C = g.c + (uint64_t)bz * g.M * g.N;
-  const float *Cadd = g.c_add ? g.c_add + (uint64_t)bz * g.M * g.N : nullptr;
+  // (several rows: slices of k, summed by splitk_reduce_kernel)
+  const bool sliced = MROWS > 1 && g.splits > 1;
+  const uint32_t k_lo = sliced ? min(g.K, blockIdx.z * g.k_per_split) : 0, k_hi = sliced ? min(g.K, k_lo + g.k_per_split) : g.K;
+  float *C = (sliced ? g.workspace + (uint64_t)blockIdx.z * g.nb0 * g.nb1 * g.M * g.N : g.c) + (uint64_t)bz * g.M * g.N;
+  const float *Cadd = g.c_add && !sliced ? g.c_add + (uint64_t)bz * g.M * g.N : nullptr;
   const uint32_t n = blockIdx.x * 64 + cg * 4;
   float acc[MROWS][4];
 #pragma unroll
@@ -2854,7 +2857,7 @@ __global__ void __launch_bounds__(16 * KS) gemv_col_kernel(GemmDesc g, int b_vec
     for (int j = 0; j < 4; ++j) acc[m][j] = 0.f;
   // One row: the compiler asks for several steps' values ahead by itself (14.8 us for 1 x 2048 x 64, 30.5 in fours).  More rows: four steps'
   // values, all asked for before the first is used; one step at a time was a trip to memory each (5 rows f32 of 1073 x 743 54 -> 27 us, 1024
-  // x 2048 40 -> 26, 2048 x 64 110 -> 44, bf16 weights 743 x 69 52 -> 29).
+  // x 2048 40 -> 26, 2048 x 64 110 -> 44, bf16 weights 743 x 69 52 -> 29, all in one slice of k; gemm_split_k has what slices give).
   if constexpr (MROWS == 1) {
     for (uint32_t k = ks; k < g.K; k += KS) {
       const TB *brow = B + (int64_t)k * g.sbk + n;
@@ -2878,11 +2881,11 @@ __global__ void __launch_bounds__(16 * KS) gemv_col_kernel(GemmDesc g, int b_vec
     }
   }
   constexpr int U = 4;
-  for (uint32_t k0 = ks; MROWS > 1 && k0 < g.K; k0 += KS * U) {
+  for (uint32_t k0 = k_lo + ks; MROWS > 1 && k0 < k_hi; k0 += KS * U) {
     float w[U][4], xv[U][MROWS];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const uint32_t k = min(k0 + u * KS, g.K - 1);
+      const uint32_t k = min(k0 + u * KS, k_hi - 1);
       const TB *brow = B + (int64_t)k * g.sbk;
       if (b_vec && n + 4 <= g.N) {
         if (sizeof(TB) == 4) {
@@ -2903,7 +2906,7 @@ __global__ void __launch_bounds__(16 * KS) gemv_col_kernel(GemmDesc g, int b_vec
     }
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      if (k0 + u * KS >= g.K) break;
+      if (k0 + u * KS >= k_hi) break;
 #pragma unroll
       for (int m = 0; m < MROWS; ++m) {
         if ((uint32_t)m < g.M) {
@@ -3209,7 +3212,16 @@ uint32_t gemm_split_k(const LaunchCtx &lc, const GemmDesc &g) {
     // the generic kernel (f32 products): same idea, shorter k-steps, so thinner slices still pay
     // (the one-row kernels, which take f32 rows only; 5 bf16 rows of 1073 values by 743 columns 119 us in one slice, 30 in eight
     // and their sum, 1 or 5 of 1024 by 2048 67, 17)
-    if ((g.M <= 8 && g.a_stype == ST_F32 && (g.sbk == 1 || g.sbn == 1 || g.K == 1 || g.N == 1)) || g.b_index || !g.K) return 1;
+    if (g.b_index || !g.K) return 1;
+    if (g.M <= 8 && g.a_stype == ST_F32 && (g.sbk == 1 || g.sbn == 1 || g.K == 1 || g.N == 1)) {
+      // k-major weights for 2 to 8 rows: a workgroup to 64 columns walks k 64 values at a time, so slices for up to half of the CUs,
+      // of 256 values at least (5 f32 rows of 2048 x 64 45.9 us in one slice, 8.8 in eight and 4.6 for their sum; 743 x 69 19.7, 11.7
+      // and 2.8 in two; 1073 x 743 26.9, 11.2 and 4.0 in four; bf16 weights 2048 x 64 62.7, 11.1 and 2.9, 743 x 69 28.2, 16.3 and 3.8)
+      // (the sum reads and writes 16 bytes at a time)
+      if (g.M > 1 && g.sbk != 1 && g.K > 1 && (uintptr_t)g.c % 16 == 0 && (uintptr_t)g.c_add % 16 == 0)
+        while ((uint64_t)((g.N + 63) / 64) * batch * splits * 4 <= (uint64_t)lc.n_cus && g.K / (splits * 2) >= 256 && splits < 16) splits *= 2;
+      return splits;
+    }
     // (two workgroups to a CU, one's loads under the other's products: 700 x 2048 x 8192 357 -> 312 us, 400 x 2048 x 8192
     // 185 -> 168; four k-steps at least to each: 1000 x 1000 x 1000 54 -> 36, 100 x 2048 x 2048 33 -> 27; four workgroups
     // to a CU were slower throughout.  A shallow product does not pay for the second workgroup's slices, unless its sums are
@@ -3316,7 +3328,8 @@ hipError_t launch_matmul(const LaunchCtx &lc_in, const GemmDesc &g, const char *
     }
     if (b_unit_n) {
       if (kernel_name) *kernel_name = g.b_stype == ST_BF16 ? "gemv_col_bf16" : "gemv_col_f32";
-      dim3 grid((g.N + 63) / 64, batch);
+      const uint32_t slices = g.M > 1 && g.splits > 1 ? g.splits : 1;
+      dim3 grid((g.N + 63) / 64, batch, slices);
       if (g.M == 1) {
         // one output row: 64 k-slices per workgroup keep enough loads in flight
         if (g.b_stype == ST_BF16) CG_LAUNCH(lc, (gemv_col_kernel<uint16_t, 1, 64>), grid, 1024, g, bv);
@@ -3324,6 +3337,11 @@ hipError_t launch_matmul(const LaunchCtx &lc_in, const GemmDesc &g, const char *
       } else {
         if (g.b_stype == ST_BF16) CG_LAUNCH(lc, (gemv_col_kernel<uint16_t, 8, 16>), grid, 256, g, bv);
         else CG_LAUNCH(lc, (gemv_col_kernel<float, 8, 16>), grid, 256, g, bv);
+      }
+      if (slices > 1 && !g.defer_reduce) {
+        const uint64_t n = (uint64_t)batch * g.M * g.N;
+        CG_LAUNCH(tail, (splitk_reduce_kernel), (unsigned)((n / 4 + 255) / 256 + (n < 4)), 256, (const float *)g.workspace, g.c, n, slices, g.c_add,
+                  (int)g.act_sigmoid);
       }
       return hipGetLastError();
     }

@@ -134,3 +134,24 @@ def test_a_few_ragged_rows(request, mode, M, K, H, N):
     with np.errstate(invalid="ignore"):
         ref = x.astype(np.float64) @ w64
     assert np.array_equal(np.isnan(h), np.isnan(ref)) and np.array_equal(np.isinf(h), np.isinf(ref))
+
+
+# 2 to 8 f32 rows against k-major weights in slices of k: one slice and the first two, the last one short, some empty; sums that do and do
+# not fill pieces of 16 bytes; batches, and a residual that starts on one or off
+@pytest.mark.gpu
+@pytest.mark.parametrize("batch,M,K,N", [(1, 5, 511, 7), (1, 5, 512, 7), (1, 3, 4112, 5), (1, 8, 1100, 130), (3, 2, 1073, 66), (2, 7, 5000, 1), (40, 4, 600, 64)])
+@pytest.mark.parametrize("mode", ["hip", "hip_bf16"])
+@pytest.mark.parametrize("residual", [None, 0, 1])
+def test_a_few_rows_in_slices_of_k(request, mode, residual, batch, M, K, N):
+    be, g = request.getfixturevalue(mode), np.random.default_rng(K)
+    rounded = lambda s, std: vectors.bf16_round((g.standard_normal(s) * std).astype(np.float32))
+    x, w, r = rounded((batch, M, K), 1.0), rounded((batch, K, N), K ** -0.5), rounded((batch * M * N + 1,), 1.0)
+    if residual is not None:
+        f = lambda b, x, w, r: [lang.reshape(b, lang.make_shape(b, batch, M, N), lang.slice(b, 0, residual, batch * M * N, r)) + lang.matmul(b, x, w)]
+        (y,) = vectors.run(be, f, 1, x, w, r)
+    else:
+        (y,) = vectors.run(be, plain, 1, x, w)
+    x64, w64 = x.astype(np.float64), w.astype(np.float64)
+    add = 0.0 if residual is None else r[residual:][:batch * M * N].reshape(batch, M, N).astype(np.float64)
+    # K f32 additions of exact products, and one of the residual
+    assert np.all(np.abs(y - (x64 @ w64 + add)) <= (K + 1) * 2.0 ** -24 * (np.abs(x64) @ np.abs(w64) + np.abs(add)))
