@@ -1,7 +1,9 @@
 // A HIP runtime without a GPU, for tests of what the host does: memory is host memory, a stream is always idle, the two
 // copy kernels are made on the spot and every other launch is none.  fake_hip_refuse(name, n): the n-th launch from now
 // of a kernel whose name holds `name` is refused, as the runtime refuses one that it cannot make.  fake_hip_launched(): the
-// names of the kernels launched since the last call; fake_hip_static_lds(n): what every kernel's own __shared__ variables take.
+// names of the kernels launched since the last call; fake_hip_products(): of the matrix products among them a line each, the name and what
+// the kernel is told of its walk along k - slices, values to a slice, whether column tiles start at different ones -; fake_hip_static_lds(n):
+// what every kernel's own __shared__ variables take.
 // Loaded with RTLD_GLOBAL before the library, whose references to the runtime it then answers.
 #include <hip/hip_runtime.h>
 #include <atomic>
@@ -10,6 +12,8 @@
 #include <map>
 #include <mutex>
 #include <string>
+#define HIP_INCLUDE_HIP_HIP_EXT_H  // (templates that only a HIP compiler takes, of which the descriptors need nothing)
+#include "launch.hpp"
 
 namespace {
 std::map<const void *, std::string> &names() {
@@ -17,7 +21,7 @@ std::map<const void *, std::string> &names() {
   return m;
 }
 std::mutex lock;
-std::string refuse, launched;
+std::string refuse, launched, products;
 std::atomic<int> countdown{0}, waits{0}, static_lds{0};
 thread_local hipError_t last = hipSuccess;
 
@@ -42,6 +46,15 @@ hipError_t launch(const void *f, void **args) {
   {
     std::lock_guard<std::mutex> lk(lock);
     launched += name + "\n";
+    if (name.find("NS_8GemmDescE") != std::string::npos) {
+      const auto &g = *(const cgk::GemmDesc *)args[0];
+      const uint32_t splits = g.splits > 1 ? g.splits : 1;
+      products += name + " " + std::to_string(splits) + " " + std::to_string(splits > 1 ? g.k_per_split : g.K) + " " + std::to_string(g.k_rotate) + "\n";
+    }
+    if (name.find("NS_11MoeGemmDescE") != std::string::npos) {
+      const auto &g = *(const cgk::MoeGemmDesc *)args[0];
+      products += name + " 1 " + std::to_string(g.K) + " " + std::to_string(g.k_rotate) + "\n";
+    }
     if (!refuse.empty() && name.find(refuse) != std::string::npos && countdown.fetch_sub(1) == 1) {
       refuse.clear();
       return last = hipErrorInvalidConfiguration;
@@ -61,13 +74,15 @@ void fake_hip_refuse(const char *name, int n) {
   countdown = n;
 }
 int fake_hip_waits() { return waits; }  // on the stream
-const char *fake_hip_launched() {
-  static std::string since;
+static const char *taken(std::string &lines) {
+  static thread_local std::string since;
   std::lock_guard<std::mutex> lk(lock);
   since.clear();
-  since.swap(launched);
+  since.swap(lines);
   return since.c_str();
 }
+const char *fake_hip_launched() { return taken(launched); }
+const char *fake_hip_products() { return taken(products); }
 void fake_hip_static_lds(int n) { static_lds = n; }
 
 void **__hipRegisterFatBinary(const void *) { static void *h[4]; return h; }

@@ -61,7 +61,7 @@ works()
 def fake_hip(tmp_path_factory):
     here, rocm = os.path.dirname(os.path.abspath(__file__)), os.environ.get("ROCM_PATH", "/opt/rocm")
     so = str(tmp_path_factory.mktemp("fake") / "libfake_hip.so")
-    subprocess.check_call(["g++", "-std=c++17", "-O1", "-shared", "-fPIC", "-w", "-D__HIP_PLATFORM_AMD__", "-I" + os.path.join(rocm, "include"),
+    subprocess.check_call(["g++", "-std=c++17", "-O1", "-shared", "-fPIC", "-w", "-D__HIP_PLATFORM_AMD__", "-I" + os.path.join(rocm, "include"), "-I" + os.path.join(os.path.dirname(here), "catgrad-rs_amd", "csrc"),
                            os.path.join(here, "fake_hip.cpp"), "-o", so])
 
     def run(script, flags=0):

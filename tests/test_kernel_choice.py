@@ -1,6 +1,7 @@
 """Which kernel a call is given, on the CPU: the library over the stand-in runtime of fake_hip.cpp, which says what was launched."""
 import pytest
 
+import test_k_order as k_order
 from test_f32_tiles import ODD_SIZES, SIZES
 from test_host_copies import fake_hip  # noqa: F401 - a fixture
 
@@ -9,7 +10,7 @@ BF16 = 1
 LAUNCHED = """
 import importlib
 lang, nn = cg.lang, cg.nn
-fake.fake_hip_launched.restype = ctypes.c_char_p
+fake.fake_hip_launched.restype = fake.fake_hip_products.restype = ctypes.c_char_p
 
 def launched(f):
     be.sync()
@@ -32,6 +33,18 @@ def product(m, n, k, along_k=True, batch=1, residual=False):
         y = be.matmul(x, be.transpose(w, r - 2, r - 1) if along_k else w)
         return be.add(res, y) if residual else y
     return launched(f)
+
+class Term(lang.Module):
+    def __init__(self, n_in, f): self.n_in, self.f = n_in, f
+    def path(self): return lang.path(["choice"])
+    def sort(self): return [lang.TENSOR] * self.n_in, [lang.TENSOR]
+    def def_(self, b, args): return [self.f(b, *args)]
+
+def run(f, *args):
+    return cg.Interpreter(be, cg.stdlib(), cg.Parameters()).run(Term(len(args), f).term(), list(args))[0]
+
+def linear(b, x, w, n, k):
+    return lang.matmul(b, x, lang.reshape(b, lang.make_shape(b, 1, k, n), lang.transpose(b, 0, 1, w)))
 """
 
 
@@ -240,4 +253,51 @@ for m, n, k, half in ((3100, 2050, 1024, True), (3333, 2049, 1088, True), (2300,
     for residual in (False, True):
         names = product(m, n, k, residual=residual)
         assert len(names) == 1 and ("gemm_bf16_ring_kernelILi0ELi1E" in names[0]) == half, (m, n, k, names)
+""", BF16)
+
+
+def test_where_column_tiles_start_at_different_k(fake_hip):  # noqa: F811
+    """The lists of test_k_order.py: kernel, slices of k, and the order as the kernel is told of it."""
+    fake_hip(LAUNCHED + f"""
+def products(f, *args):     # (kernel, slices, values to a slice, order)
+    be.sync()
+    fake.fake_hip_products()
+    be.realize(run(f, *args))
+    be.sync()
+    lines = [line.rsplit(" ", 3) for line in fake.fake_hip_products().decode().splitlines()]
+    return [(name, int(s), int(k), int(o)) for name, s, k, o in lines if "route" not in name]
+
+def check(what, got, kernel, slices, on):
+    assert (kernel % 0 if "%d" in kernel else kernel) in got[0] and got[1] == slices and got[3] == on, (what, got)
+
+for on, sizes in ((1, {k_order.PRODUCTS}), (0, {k_order.OTHER_PRODUCTS})):
+    for m, n, k, kernel, slices in sizes:
+        (got,) = products(lambda b, x, w: linear(b, x, w, n, k), operand(1, m, k), operand(n, k))
+        check((m, n, k), got, kernel, slices, on)
+for on, sizes in ((1, {k_order.PARTS_OF_ROWS}), (0, {k_order.OTHER_PARTS_OF_ROWS})):
+    for m, n, k, apart, kernel, slices in sizes:
+        (got,) = products(lambda b, x, w: linear(b, x, lang.slice(b, 1, 64, k, w), n, k), operand(1, m, k), operand(n, apart))
+        check((m, n, k, apart), got, kernel, slices, on)
+        assert got[2] // 64 % 2 == 1 or not on, got
+for m, n, k, kernel in {k_order.SIGMOIDS}:
+    (got,) = products(lambda b, x, w: nn.sigmoid(b, linear(b, x, w, n, k)), operand(1, m, k), operand(n, k))
+    check((m, n, k), got, kernel % 1, 1, 1)
+for on, sizes in ((1, {k_order.GATED}), (0, {k_order.OTHER_GATED})):
+    for m, f, k, kernel in sizes:
+        got = products(lambda b, x, g, u, d: linear(b, nn.silu(b, linear(b, x, g, f, k)) * linear(b, x, u, f, k), d, 64, f),
+                       operand(1, m, k), operand(f, k), operand(f, k), operand(64, f))
+        check((m, f, k), got[0], kernel % 2 if "%d" in kernel else kernel, 1, on)
+
+def experts(b, x, idx, gs, us, ds):
+    x, total = x + x - x, None
+    for i in range(2):
+        slot = lang.get(b, 1, i, idx)
+        of = lambda w: lang.transpose(b, 1, 2, lang.index(b, 0, slot, w))
+        y = lang.matmul(b, nn.silu(b, lang.matmul(b, x, of(gs))) * lang.matmul(b, x, of(us)), of(ds))
+        total = y if total is None else total + y
+    return total
+for s, kernel, on in {k_order.EXPERTS}:
+    for f, h in ((192, 2048), (2048, 192)):
+        got = products(experts, operand(s, 1, h), be.tensor(np.zeros((s, 2), np.uint32)), operand(5, f, h), operand(5, f, h), operand(5, h, f))
+        assert len(got) == 2 and all(kernel in g[0] and g[3] == (on if g[2] == 2048 else 0) for g in got), (s, f, h, got)
 """, BF16)
