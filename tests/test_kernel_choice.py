@@ -2,6 +2,7 @@
 import pytest
 
 import test_k_order as k_order
+import test_large_tiles as large
 from test_f32_tiles import ODD_SIZES, SIZES
 from test_host_copies import fake_hip  # noqa: F401 - a fixture
 
@@ -300,4 +301,55 @@ for s, kernel, on in {k_order.EXPERTS}:
     for f, h in ((192, 2048), (2048, 192)):
         got = products(experts, operand(s, 1, h), be.tensor(np.zeros((s, 2), np.uint32)), operand(5, f, h), operand(5, f, h), operand(5, h, f))
         assert len(got) == 2 and all(kernel in g[0] and g[3] == (on if g[2] == 2048 else 0) for g in got), (s, f, h, got)
+""", BF16)
+
+
+def test_tiles_of_256_x_288(fake_hip):  # noqa: F811
+    """Where they need fewer rounds, plain with and without a residual, in a batch, stacked; the sizes of test_large_tiles.py."""
+    fake_hip(LAUNCHED + f"""
+tall, wide = "gemm_bf16_ring_kernelILi%dELi2ELb0E", "gemm_bf16_ring_kernelILi%dELi2ELb1E"
+for kernel, sizes in ((wide, {large.WIDE}), (tall, {large.NOT_WIDE}), (wide, [(16384, 1152, 1024)]), (tall, [(8192, 1152, 6912), (4096, 4096, 2048)])):
+    for m, n, k in sizes:
+        for residual in (False, True):
+            (name,) = product(m, n, k, residual=residual)
+            assert kernel % 0 in name or (m, n, k) == (8192, 1152, 6912), (m, n, k, name)
+            assert (wide % 0 in name) == (kernel is wide), (m, n, k, name)
+b, m, n, k = {large.WIDE_BATCH}
+for residual in (False, True):
+    (name,) = product(m, n, k, batch=b, residual=residual)
+    assert wide % 0 in name, name
+for kernel, sizes in ((wide, {large.WIDE_GATED}), (tall, [(4096, 2048, 320)])):
+    for m, f, k in sizes:
+        for kind, act in ((2, nn.silu), (3, nn.gelu)):
+            (first, *_) = launched(lambda: run(lambda b, x, g, u, d: linear(b, act(b, linear(b, x, g, f, k)) * linear(b, x, u, f, k), d, 64, f),
+                                               operand(1, m, k), operand(f, k), operand(f, k), operand(64, f)))
+            assert kernel % kind in first, (m, f, k, first)
+""", BF16)
+
+
+def test_q_k_v_that_rotate_on_large_tiles(fake_hip):  # noqa: F811
+    """256 x 256 and 128 x 256 tiles for the sizes of test_large_tiles.py, with biases and norm; smaller ones, and no rotation, beyond."""
+    fake_hip(LAUNCHED + f"""
+sys.path.insert(0, "tests")
+import test_large_tiles as large
+ring = "gemm_bf16_ring_kernelILi%dELi%dE"
+
+def names(hd, batch, s, heads, kv, k, bias, norm, gamma=True):
+    ns = [heads * hd, kv * hd, kv * hd]
+    args = [operand(1, batch * s, k)] + [operand(n, k) for n in ns]
+    args += [be.tensor(np.zeros(n, np.float32)) for n in ns + ([hd] * 2 if gamma else [])]
+    return launched(lambda: run(lambda b, x, *p: large.attention_of_projections(b, x + x - x, p, hd, batch, s, heads, kv, k, bias, norm)[0], *args))
+
+for height, sizes in ((2, {large.ROTATED_LARGE}), (1, {large.ROTATED_HALF})):
+    for c in sizes:
+        hd, bias, norm = c[0], c[6], c[7]
+        kind = {{64: 4, 128: 6, 256: 8}}[hd] + (bias or norm)
+        for gamma in (True, False) if norm else (True,):
+            got = names(*c, gamma=gamma)
+            assert len(got) == 1 and ring % (kind, height) in got[0], (c, got)
+for c in ((64, 1, 703, 20, 20, 768, False, False), (128, 1, 1202, 16, 16, 704, False, False)):       # few rows; few k
+    (got,) = names(*c)
+    assert "gemm_bf16_dma_kernel" in got, (c, got)
+(got,) = names(256, 4, 257, 4, 1, 768, False, True)
+assert "ring_kernelILi9E" not in got, got
 """, BF16)

@@ -49,21 +49,32 @@ def test_product(hip_bf16, M, N, K):
 
 # 256 x 288: one round where 256 x 256 take two, the fewest k-steps it is given, an odd number; rows that end in the first and the second
 # half of a tile, columns that end in the strip and in front of it; and less than a round of 256 x 256 in place of two of 128 x 128
+# (test_kernel_choice.py holds these lists, and those of tiles that rotate, to the kernel they are meant for)
+WIDE = [(4100, 4308, 256), (4250, 4084, 320), (4352, 4320, 576), (3900, 4148, 1088)]
+NOT_WIDE = [(3001, 3003, 768), (2100, 4100, 1024)]
+
+
 @pytest.mark.gpu
-@pytest.mark.parametrize("M,N,K", [(4100, 4308, 256), (4250, 4084, 320), (4352, 4320, 576), (3900, 4148, 1088), (3001, 3003, 768), (2100, 4100, 1024)])
+@pytest.mark.parametrize("M,N,K", WIDE + NOT_WIDE)
 def test_wide_product(hip_bf16, M, N, K):
     test_product(hip_bf16, M, N, K)
 
 
+WIDE_BATCH = (3, 1300, 4028, 256)
+
+
 @pytest.mark.gpu
-@pytest.mark.parametrize("B,M,N,K", [(1, 4100, 4308, 256), (1, 4250, 4084, 320), (3, 1300, 4292, 256), (1, 3001, 3003, 768)])
+@pytest.mark.parametrize("B,M,N,K", [(1, *WIDE[0]), (1, *WIDE[1]), WIDE_BATCH, (1, *NOT_WIDE[0])])
 def test_wide_product_and_residual(hip_bf16, B, M, N, K):
     test_product_and_residual(hip_bf16, B, M, N, K)
 
 
+WIDE_GATED = [(4100, 2152, 256), (4250, 2056, 320), (3900, 2304, 640)]    # columns that end in the strip, in front of it, with a tile
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("act", ["silu", "gelu"])
-@pytest.mark.parametrize("M,F,K", [(4100, 2156, 256), (4250, 2052, 320), (3900, 2304, 640)])    # columns that end in the strip, in front of it, with a tile
+@pytest.mark.parametrize("M,F,K", WIDE_GATED)
 def test_wide_gated(hip_bf16, M, F, K, act):
     test_gated(hip_bf16, M, F, K, act)
 
@@ -190,11 +201,40 @@ def test_rotated_wide_heads(oracle, hip_bf16, batch, tokens):
 
 # q / k / v that leave a 256 x 256 tile rotated: heads of 64, 128 and 256, with biases, with a norm of every head's row in front of the
 # rotation; one sequence that ends inside a tile, several whose length is no multiple of four (pieces of values that straddle two), of eight
+ROTATED_LARGE = [(64, 1, 2203, 20, 20, 768, False, False), (64, 8, 276, 20, 20, 768, True, False),
+                 (128, 5, 271, 16, 16, 768, True, False), (128, 1, 1302, 16, 16, 832, False, False),
+                 (256, 21, 257, 4, 1, 192, False, True), (256, 129, 64, 2, 1, 128, False, True),
+                 (256, 20, 270, 4, 1, 128, False, False)]
+
+
+def attention_of_projections(b, x, p, hd, batch, S, heads, kv, K, bias, norm, eps=1e-6, theta=10000.0):
+    """Attention, rotated keys and values of x; p: the three weights, their biases, the gammas of queries and keys (none: no gamma)."""
+    h, ns = helpers, [heads * hd, kv * hd, kv * hd]
+
+    def normed(gamma, n_heads, y):   # (gemma3.rs:41-68, folded as in gemma3.rs:99-117)
+        y = lang.reshape(b, lang.make_shape(b, batch * n_heads * S, hd), y)
+        s = lang.sum(b, y * y)
+        mean = s / lang.broadcast(b, lang.cast(b, lang.nat_to_u32(b, lang.to_nat(b, hd)), lang.dtype(b, y)), lang.shape(b, s))
+        rms = nn.sqrt(b, mean + lang.constant(b, eps, lang.shape(b, mean)))
+        y = y / lang.broadcast(b, rms, lang.shape(b, y))
+        if gamma is not None:
+            gm = lang.broadcast(b, gamma, lang.shape(b, y))
+            y = y * (lang.constant(b, 1.0, lang.shape(b, gm)) + gm)
+        return lang.reshape(b, lang.make_shape(b, batch, n_heads, S, hd), y)
+
+    y = [linear(b, x, p[i], ns[i], K, p[3 + i] if bias else None) for i in range(3)]
+    y = [lang.transpose(b, 1, 2, lang.reshape(b, lang.make_shape(b, batch, S, n // hd, hd), t)) for n, t in zip(ns, y)]
+    gammas = p[6:8] if len(p) > 6 else [None, None]
+    q, k, v = y if not norm else [normed(gammas[0], heads, y[0]), normed(gammas[1], kv, y[1]), y[2]]
+    q, k = h.rope(b, theta, 0, S, hd, q), h.rope(b, theta, 0, S, hd, k)
+    attn = lang.matmul(b, q, lang.transpose(b, 2, 3, h.repeat_kv(b, heads // kv, k)))
+    sh = lang.shape(b, attn)
+    attn = attn / lang.constant(b, float(np.sqrt(np.float32(hd))), sh) + lang.broadcast(b, h.causal_mask(b, lang.to_nat(b, S)), sh)
+    return [lang.matmul(b, nn.softmax(b, attn), h.repeat_kv(b, heads // kv, v)), k, v]
+
+
 @pytest.mark.gpu
-@pytest.mark.parametrize("hd,batch,S,heads,kv,K,bias,norm", [(64, 1, 2203, 20, 20, 768, False, False), (64, 8, 276, 20, 20, 768, True, False),
-                                                             (128, 5, 271, 16, 16, 768, True, False), (128, 1, 1302, 16, 16, 832, False, False),
-                                                             (256, 21, 257, 4, 1, 192, False, True), (256, 129, 64, 2, 1, 128, False, True),
-                                                             (256, 20, 270, 4, 1, 128, False, False)])
+@pytest.mark.parametrize("hd,batch,S,heads,kv,K,bias,norm", ROTATED_LARGE)
 def test_rotated_on_large_tiles(hip_bf16, hd, batch, S, heads, kv, K, bias, norm):
     g = np.random.default_rng(S)
     x, ns = draw(g, (1, batch * S, K)), [heads * hd, kv * hd, kv * hd]
@@ -202,26 +242,8 @@ def test_rotated_on_large_tiles(hip_bf16, hd, batch, S, heads, kv, K, bias, norm
     gammas = [(0.3 * g.standard_normal(hd)).astype(np.float32) for _ in range(2)]
     h, theta, eps = helpers, 10000.0, 1e-6
 
-    def normed(b, gamma, n_heads, y):   # (gemma3.rs:41-68, folded as in gemma3.rs:99-117)
-        y = lang.reshape(b, lang.make_shape(b, batch * n_heads * S, hd), y)
-        s = lang.sum(b, y * y)
-        mean = s / lang.broadcast(b, lang.cast(b, lang.nat_to_u32(b, lang.to_nat(b, hd)), lang.dtype(b, y)), lang.shape(b, s))
-        rms = nn.sqrt(b, mean + lang.constant(b, eps, lang.shape(b, mean)))
-        y = y / lang.broadcast(b, rms, lang.shape(b, y))
-        gm = lang.broadcast(b, gamma, lang.shape(b, y))
-        y = y * (lang.constant(b, 1.0, lang.shape(b, gm)) + gm)
-        return lang.reshape(b, lang.make_shape(b, batch, n_heads, S, hd), y)
-
     def f(b, x, *p):
-        x = x + x - x
-        y = [linear(b, x, p[i], ns[i], K, p[3 + i] if bias else None) for i in range(3)]
-        y = [lang.transpose(b, 1, 2, lang.reshape(b, lang.make_shape(b, batch, S, n // hd, hd), t)) for n, t in zip(ns, y)]
-        q, k, v = y if not norm else [normed(b, p[6], heads, y[0]), normed(b, p[7], kv, y[1]), y[2]]
-        q, k = h.rope(b, theta, 0, S, hd, q), h.rope(b, theta, 0, S, hd, k)
-        attn = lang.matmul(b, q, lang.transpose(b, 2, 3, h.repeat_kv(b, heads // kv, k)))
-        sh = lang.shape(b, attn)
-        attn = attn / lang.constant(b, float(np.sqrt(np.float32(hd))), sh) + lang.broadcast(b, h.causal_mask(b, lang.to_nat(b, S)), sh)
-        return [lang.matmul(b, nn.softmax(b, attn), h.repeat_kv(b, heads // kv, v)), k, v]
+        return attention_of_projections(b, x + x - x, p, hd, batch, S, heads, kv, K, bias, norm, eps, theta)
     hip_bf16.trace(2)
     hip_bf16.trace_reset()
     got, k, v = vectors.run(hip_bf16, f, 3, x, *ws, *bs, *gammas)
@@ -246,11 +268,14 @@ def test_rotated_on_large_tiles(hip_bf16, hd, batch, S, heads, kv, K, bias, norm
 
 
 # ... and on tiles of 128 x 256, where those are one round
+ROTATED_HALF = [(64, 1, 1203, 20, 20, 768, False, False), (64, 6, 203, 20, 20, 832, True, False),
+                (128, 5, 151, 16, 16, 768, True, False), (128, 1, 1202, 16, 16, 832, False, False),
+                (256, 11, 257, 4, 1, 768, False, True), (256, 45, 64, 4, 1, 832, False, True),
+                (256, 11, 270, 4, 1, 768, False, False)]
+
+
 @pytest.mark.gpu
-@pytest.mark.parametrize("hd,batch,S,heads,kv,K,bias,norm", [(64, 1, 1203, 20, 20, 768, False, False), (64, 6, 203, 20, 20, 832, True, False),
-                                                             (128, 5, 151, 16, 16, 768, True, False), (128, 1, 1202, 16, 16, 832, False, False),
-                                                             (256, 11, 257, 4, 1, 768, False, True), (256, 45, 64, 4, 1, 832, False, True),
-                                                             (256, 11, 270, 4, 1, 768, False, False)])
+@pytest.mark.parametrize("hd,batch,S,heads,kv,K,bias,norm", ROTATED_HALF)
 def test_rotated_on_half_tiles(hip_bf16, hd, batch, S, heads, kv, K, bias, norm):
     test_rotated_on_large_tiles(hip_bf16, hd, batch, S, heads, kv, K, bias, norm)
 
