@@ -280,6 +280,47 @@ def test_rotated_on_half_tiles(hip_bf16, hd, batch, S, heads, kv, K, bias, norm)
     test_rotated_on_large_tiles(hip_bf16, hd, batch, S, heads, kv, K, bias, norm)
 
 
+# ... the norm in front of the rotation on rows that it treats specially, with gamma and without: zeros, values whose squares vanish or
+# overflow (the quotient by infinity is 0), infinities and a NaN (the quotient is none), beside rows of neither kind
+@pytest.mark.gpu
+@pytest.mark.parametrize("gamma", [True, False])
+@pytest.mark.parametrize("batch,S,K", [(21, 257, 192), (11, 257, 768)])
+def test_special_rows_normed_and_rotated(hip_bf16, batch, S, K, gamma):
+    g, hd, heads, eps, theta = np.random.default_rng(S + K), 256, 4, 1e-6, 10000.0
+    x = draw(g, (1, batch * S, K))
+    rows = g.permutation(batch * S)[:30].reshape(6, 5)      # (any place of a tile and of a wavefront's rows)
+    x[0, rows[0]] = 0.0
+    x[0, rows[1]] *= np.float32(2.0 ** -80)
+    x[0, rows[2]] *= np.float32(2.0 ** 70)
+    x[0, rows[3], 0] = np.inf
+    x[0, rows[4], K - 1] = -np.inf
+    x[0, rows[5], 1] = np.nan
+    ns = [heads * hd, hd, hd]
+    ws, bs = [draw(g, (n, K), K ** -0.5) for n in ns], [np.zeros(n, np.float32) for n in ns]
+    ws[1][:, [0, K - 1]] = np.where(ws[1][:, [0, K - 1]] == 0, np.float32(0.5), ws[1][:, [0, K - 1]])
+    gammas = [(0.3 * g.standard_normal(hd)).astype(np.float32) for _ in range(2)] if gamma else []
+    hip_bf16.trace(2)
+    hip_bf16.trace_reset()
+    def f(b, x, *p):
+        x = x * lang.constant(b, 1.0, lang.shape(b, x))     # (f32, and infinities stay)
+        return attention_of_projections(b, x, p, hd, batch, S, heads, 1, K, False, True, eps, theta)
+    _, k, _ = vectors.run(hip_bf16, f, 3, x, *ws, *bs, *gammas)
+    names = sorted(hip_bf16.trace_report())
+    hip_bf16.trace(False)
+    assert sum("grouped,rope" in n for n in names) == 1 and not any(n.startswith("rope_fused") for n in names), names
+    k = k.reshape(batch * S, hd)
+    assert np.all(k[rows[[0, 2]].ravel()] == 0) and np.all(np.isnan(k[rows[3:].ravel()]))
+    finite = np.setdiff1d(np.arange(batch * S), rows[2:].ravel())
+    c, s = (t.astype(np.float64) for t in vectors.run(hip_bf16, lambda b, _: helpers.rope_tables(b, theta, lang.to_nat(b, S), hd), 2, np.zeros(1, np.float32)))
+    y = x[0, finite].astype(np.float64) @ ws[1].T.astype(np.float64)
+    y = y / np.sqrt(np.mean(y ** 2, axis=-1, keepdims=True) + eps) * (1.0 + gammas[1].astype(np.float64) if gamma else 1.0)
+    c, s = (t.reshape(S, hd)[finite % S] for t in (c, s))
+    ref = c * y + s * np.concatenate([-y[:, hd // 2:], y[:, :hd // 2]], axis=-1)
+    tiny = np.isin(finite, rows[1])     # (on a scale of their own)
+    parity.assert_f32(ref[~tiny], k[finite[~tiny]], "rotated keys")
+    parity.assert_f32(ref[tiny] * 2.0 ** 80, k[finite[tiny]].astype(np.float64) * 2.0 ** 80, "rotated keys of tiny rows")
+
+
 # 128 x 256 in one round: the fewest k-steps, an odd number, rows and columns that end inside a tile, rows of results off 16 bytes, a batch
 @pytest.mark.gpu
 @pytest.mark.parametrize("M,N,K", [(3100, 2050, 1024), (3333, 2049, 1088), (2300, 3001, 2048), (1000, 6143, 1152), (4096, 2048, 4160)])
