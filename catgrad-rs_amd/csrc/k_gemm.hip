@@ -1031,24 +1031,29 @@ static hipError_t launch_gemm_plain(const LaunchCtx &lc, const GemmDesc &g, uint
                                   : launch_gemm_dma<BM_, BN_, WR, WC, false, NS, false, false, false, KG, RING>(lc, g, (uint32_t)grid);
 }
 
-// C = sum over splits of workspace[split] (float4 per thread; sizes are multiples of 4 or the
-// tail is handled scalar)
+// C = sum over splits of workspace[split], four values per thread, the tail by value.  A sum of n values that is no multiple of four
+// puts every slice but the first off 16 bytes, and a residual may start anywhere: the pieces need four bytes only.
+__device__ __forceinline__ float4 any_float4(const float *p) {
+  float4 v;
+  __builtin_memcpy(&v, p, 16);
+  return v;
+}
 __global__ void __launch_bounds__(256) splitk_reduce_kernel(const float *ws, float *c, uint64_t n,
                                                             uint32_t splits, const float *cadd, int act) {
   const uint64_t n4 = n / 4;
   for (uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x; i < n4;
        i += (uint64_t)gridDim.x * 256) {
-    float4 s = ((const float4 *)ws)[i];
+    float4 s = any_float4(ws + i * 4);
     for (uint32_t k = 1; k < splits; ++k) {
-      const float4 v = ((const float4 *)(ws + (uint64_t)k * n))[i];
+      const float4 v = any_float4(ws + (uint64_t)k * n + i * 4);
       s.x += v.x; s.y += v.y; s.z += v.z; s.w += v.w;
     }
     if (cadd) {
-      const float4 v = ((const float4 *)cadd)[i];
+      const float4 v = any_float4(cadd + i * 4);
       s.x += v.x; s.y += v.y; s.z += v.z; s.w += v.w;
     }
     if (act) s = make_float4(sigmoid_ref(s.x), sigmoid_ref(s.y), sigmoid_ref(s.z), sigmoid_ref(s.w));
-    ((float4 *)c)[i] = s;
+    __builtin_memcpy(c + i * 4, &s, 16);
   }
   if (blockIdx.x == 0 && threadIdx.x < (n & 3)) {
     const uint64_t i = n4 * 4 + threadIdx.x;
@@ -3217,8 +3222,7 @@ uint32_t gemm_split_k(const LaunchCtx &lc, const GemmDesc &g) {
       // k-major weights for 2 to 8 rows: a workgroup to 64 columns walks k 64 values at a time, so slices for up to half of the CUs,
       // of 256 values at least (5 f32 rows of 2048 x 64 45.9 us in one slice, 8.8 in eight and 4.6 for their sum; 743 x 69 19.7, 11.7
       // and 2.8 in two; 1073 x 743 26.9, 11.2 and 4.0 in four; bf16 weights 2048 x 64 62.7, 11.1 and 2.9, 743 x 69 28.2, 16.3 and 3.8)
-      // (the sum reads and writes 16 bytes at a time)
-      if (g.M > 1 && g.sbk != 1 && g.K > 1 && (uintptr_t)g.c % 16 == 0 && (uintptr_t)g.c_add % 16 == 0)
+      if (g.M > 1 && g.sbk != 1 && g.K > 1)
         while ((uint64_t)((g.N + 63) / 64) * batch * splits * 4 <= (uint64_t)lc.n_cus && g.K / (splits * 2) >= 256 && splits < 16) splits *= 2;
       return splits;
     }
