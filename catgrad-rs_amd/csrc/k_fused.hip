@@ -344,9 +344,9 @@ hipError_t launch_softmax(const LaunchCtx &lc, const SoftmaxDesc &d) {
 // max(softmax(x)), what a classifier reports as the confidence of its choice, without the probabilities ever being
 // stored: exp(max - max) / sum exp(x - max) in one pass over x with a running maximum; the same pass finds the column of
 // the largest x when argmax(x) is asked for as well.  Bound by reading x once, and by five operations and an exp2 a value: 4096 x 4096 f32
-// 197 us in four launches (the exponentials written and read twice) -> 15.  Rows of any length and alignment: 16-byte loads that need no
-// alignment, a scalar tail.  A wave to a row of up to 1024 values, a workgroup to a longer one, several workgroups
-// when there are fewer rows than CUs.
+// 197 us in four launches (the exponentials written and read twice) -> 14.  Rows of any length and alignment: 16-byte loads that need no
+// alignment, a scalar tail.  A wave to a row of up to 1024 to 4096 values, the longer the more rows there are (launch_softmax_best), a
+// workgroup to a longer one, several workgroups when there are fewer rows than CUs.
 struct RowBest {  // what is known of a part of a row
   float xm = -INFINITY, s = 0.f;       // largest value (NaN ignored), sum of exp(x - max(xm, f32::MIN))
   uint32_t key = 0, col = 0;           // f32::total_cmp order of the largest value as an unsigned word, its (last) column
@@ -380,9 +380,14 @@ struct RowBest {  // what is known of a part of a row
 };
 
 // A group of values costs a value one maximum, a subtraction, a product, the hardware's exp2 and a sum: exp(x - m) is 2 to the rounded
-// product of the rounded difference and log2 e, 6e-8 |x - m| off for one value, with a weight that falls as exp(x - m) does, and of either
-// sign from value to value.  (Error against 64 bits over 4096 x 4096, 300 x 50000, 8000 x 300 values of
-// deviation 2: 5.2e-8 to 5.4e-8, as with expf.  4096 x 4096 f32 17.9 us with expf and every value ordered, 15.3 so; 120 x 131072 19.4, 13.2.)
+// product of the rounded difference and log2 e, which itself is 1.3e-8 off, so a term is up to 7.4e-8 |x - m| off beside exp2's own 1.2e-7.
+// Unequal values are off to either side and those far below the largest weigh little; many equal ones err alike.  The sum weighs more: four
+// partial sums to a group, then one addition a group, where a sum value by value rounds every addition of equal terms alike.  Largest
+// relative error against 64 bits, with expf and a sum value by value, and so: normal values of deviation 2, 4096 x 4096 1.8e-7, 1.7e-7, 300 x
+// 50000 1.6e-7, 1.6e-7; the largest value in every thread's first piece and equal ones 0.25 to 14 below it behind, rows of 300 2.5e-7,
+// 1.8e-7, 4096 9.0e-7, 2.2e-7, 20000 4.6e-6, 4.1e-7, 131072 3.0e-5, 1.9e-6; four distinct values, 300 1.5e-7, 1.4e-7, 20000 6.0e-7, 1.5e-7,
+// 131072 4.2e-6, 2.2e-7.  (With the low parts of product and constant carried the same figures; 4096 x 4096 f32 14.2 us so, 15.2, bf16
+// 11.2, 12.5.  4096 x 4096 f32 17.9 us with expf and every value ordered, 15.3 so; 120 x 131072 19.4, 13.2.)
 // The column is looked for when the largest value is known, by the threads that hold it, in the group they met it in: every wave does that
 // for all of its registers, so the value is compared as it is, a comparison and a move, and by its place in the order only where several
 // values share it or compare as nothing does (zeros, NaN; 4096 x 4096 16.6 -> 15.4 us, 8192 x 1500 13.5 -> 12.0).  A group with a NaN, which

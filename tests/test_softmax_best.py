@@ -96,3 +96,26 @@ def test_whole_turns(oracle, hip, hip_bf16, shape):
 @pytest.mark.parametrize("n", [1024, 4096, 8192, 8200])
 def test_special_values_in_whole_turns(oracle, hip, n):
     test_special_values_in_several_groups(oracle, hip, n)
+
+
+# rows whose sum lies in many equal terms, which are all off to the same side: the largest value in front of every thread's others, or four
+# distinct values.  Against 64 bits a term with d = x - max is off by 2^-23 for exp2, 2^-23 |d| for the rounded difference and product and
+# 1.4e-8 |d| for log2 e; a sum goes through at most 16 additions to a partial sum of a group, two, one for each group that a thread meets
+# (4096 values of a row), and 16 between threads and workgroups, with four more exponentials
+@pytest.mark.gpu
+@pytest.mark.parametrize("mode", ["hip", "hip_bf16"])
+@pytest.mark.parametrize("rows,n", [(64, 300), (64, 1024), (1024, 2000), (2048, 4000), (64, 4096), (256, 20000), (300, 131072), (3, 128256)])
+def test_error_on_rows_of_few_values(request, mode, rows, n):
+    be, g = request.getfixturevalue(mode), np.random.default_rng(n)
+    below = np.linspace(0.25, 14, rows).astype(np.float32)[:, None]
+    behind = np.repeat(-below, n, axis=1)
+    behind[:, :min(n, 1024):4] = 0
+    for x in (behind, -below * g.integers(0, 4, (rows, n)).astype(np.float32) / 3):
+        x = vectors.bf16_round(x)
+        (p, _), counts = run(be, x)
+        assert counts.get("softmax_best") == 1, counts
+        d = x.astype(np.float64)
+        d -= d.max(axis=1, keepdims=True)
+        e = np.exp(d)
+        terms = (e * (2.0 ** -23 + np.abs(d) * (2.0 ** -23 + 1.4e-8))).sum(axis=1) / e.sum(axis=1)
+        assert np.all(np.abs(p.ravel() * e.sum(axis=1) - 1) <= terms + (34 + n / 4096) * 2.0 ** -24 + 4 * 2.0 ** -23)
