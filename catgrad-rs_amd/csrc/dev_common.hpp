@@ -231,7 +231,9 @@ __device__ __forceinline__ float gelu_fast(float x) {
 
 
 // The order in which a tile takes the k-steps of its slice, 64 bf16 values each: `first` up to the last, then the others from the
-// slice's first on; `wrap` steps are taken before it goes back by -`back` bytes (from the last step's place).
+// slice's first on; `wrap` steps are taken before it goes back by -`back` bytes (from the last step's place).  Which sum comes first then
+// depends on the column tile: the same f32 additions in another order, so neither equal columns of weights in two tiles nor a row on its own
+// and among more than 128 need have the same bits.
 struct KOrder {
   uint32_t first, wrap, back;
   __device__ __forceinline__ KOrder(uint32_t rotate, uint32_t tile, uint32_t n_steps) {

@@ -18,8 +18,10 @@
 //     phases, 3072 cycles, to arrive, and there is no point at which everything is waited for.
 //   * One barrier a phase: before it a wavefront has seen its own loads of the unit about to be read (a count) and the
 //     reads of two phases ago (a count); so behind it the unit is there for everyone, and its predecessor's place free.
-// The products of an element are added in the order of k, as in gemm_bf16_dma_kernel: the same bits.
-// Tiles of 128 x 256 for the stacked gate / up of fewer rows: see HPHASE0.
+// On tiles of 256 rows the products of an element are added in the order of k, the same bits as gemm_bf16_dma_kernel's for products of
+// more than 128 rows; on tiles of 128, which up to 128 rows and the routed experts may be given with an order of their own, see KOrder.
+// Tiles of 128 x 256, for the stacked gate / up of fewer rows, for one round of plain, grouped and rotating products, and for the routed
+// experts: see HPHASE0.
 // Measured against 256 x 256 tiles with eight wavefronts whose loads a compiler placed, on the same box: 16384 x 1152 by 2 x 6912
 // gate and up 531 -> 464 us, 2900 x 2048 by 2 x 8192 184 -> 161; 13056 x 6912 x 1152 203 -> 177, 16384 x 1152 x 1536 77 -> 67
 // (100 MB of result); 6000 x 1024 x 4100 with a sigmoid 77 -> 64.  What is left is power: 8192 cubed takes 1.40 us a step on

@@ -355,7 +355,7 @@ struct GemmDesc {
   uint16_t *rope_out16[3];
   const float *rope_cos[3], *rope_sin[3];
   uint32_t rope_cs_ss[3];
-  // Role 3 (heads of 256, on 256 x 256 tiles only): as 1, every head's row RMS-normed in front of its rotation, the arithmetic of
+  // Role 3 (heads of 256, on tiles of 256 columns only): as 1, every head's row RMS-normed in front of its rotation, the arithmetic of
   // rmsnorm_kernel - x / sqrt(sum(x * x) / rope_n_as_float + rope_eps) * (rope_gamma_offset + gamma) with gamma, rope_hd floats or null,
   // in the place of the bias, which it then does not have
   float rope_n_as_float, rope_eps, rope_gamma_offset;
@@ -366,9 +366,9 @@ struct GemmDesc {
 // (up to eight lines of 64 bytes a kernel's arguments are touched in one trip: with nine a 37-token prompt took 1242 us, with eight 1218.
 // The one-row kernels' two other arguments and the grid's size lie behind the descriptor, 20 bytes that are to be in the eighth.)
 static_assert(sizeof(GemmDesc) <= 488, "a GemmDesc and what lies behind it are eight lines of kernel arguments");
-// k_gemm_ring.hip: the 256 x 256 tiles of large bf16 products (plain or grouped, sigmoid, stacked gate / up);
-// half_height: the stacked gate / up of fewer rows on tiles of 128 x 256, K >= 192; wide: tiles of 256 x 288 (plain without groups or a
-// sigmoid, stacked gate / up), N % 4 == 0
+// k_gemm_ring.hip: the 256 x 256 tiles of large bf16 products (plain or grouped, rotating, sigmoid, stacked gate / up);
+// half_height: tiles of 128 x 256 (all of these but a sigmoid, without slices), K >= 192; wide: tiles of 256 x 288 (plain without groups
+// or a sigmoid, stacked gate / up), N % 4 == 0
 bool gemm_ring_ok(const GemmDesc &g);
 hipError_t launch_gemm_ring(const LaunchCtx &lc, const GemmDesc &g, bool half_height = false, bool wide = false);
 // k_gemm_f32.hip: f32 products of operands in whole 16-byte pieces; gemm_f32_split: the slices of k it is fastest with (and how long
