@@ -2403,12 +2403,14 @@ __global__ void __launch_bounds__(256) moe_gemm_kernel(MoeGemmDesc g) {
 // ---- the same with the routing done once and the operands streamed like the dense GEMM ------------------
 // One workgroup of 1024 threads sorts the (slot, token) pairs by expert: a histogram in LDS, a scan, and a scatter.  What a
 // launch of one workgroup takes is its chain of round trips, so a thread keeps its first eight pairs - their expert and the
-// place the histogram's atomic gave them - in registers, and the two scans (pairs and row tiles) go together, in a wave and then
-// over the waves.  (60 experts, 4096 pairs 9.3 -> 7.7 us, 400 5.9 -> 4.4; before: a second pass over the choices, scans of twenty barriers.)
-// The order of an expert's pairs depends on the order
-// the atomics land in, which only decides the tile row a token occupies, never its result.
-// tiles (optional): tiles[0] = the number of row tiles (moe_tile_pairs pairs each) over all experts, tiles[1 + t] = expert << 16 |
-// row tile within the expert, expert by expert - the work list of the GEMM, one workgroup per (row tile, column
+// place the histogram's atomic gave them - in registers, and the scan (of row tiles) goes on in a wave and then over the waves.  (60 experts,
+// 4096 pairs 9.3 -> 7.7 us, 400 5.9 -> 4.4; before: a second pass over the choices, scans of twenty barriers.)
+// The order of an expert's pairs depends on the order the atomics land in, which only decides the tile row a token occupies, never its
+// result.
+// Where an expert's pairs start in the list is its first row tile's number times the pairs of one, so that a row tile's pairs are found
+// without its expert.
+// tiles: tiles[0] = the number of row tiles (moe_tile_pairs pairs each) over all experts, tiles[1 + t] = expert, its row
+// tiles and the row tile within the expert (moe_entry), expert by expert - the work list of the GEMM, one workgroup per (row tile, column
 // tile), so that an expert most tokens chose is spread over the device instead of walked by one workgroup.
 // The workgroups behind the first, if any, split the S rows of slot 0's f32 input into the three planes at `planes`.
 __host__ __device__ constexpr uint32_t moe_tile_pairs(bool planes) { return planes ? 20 : 128; }
@@ -2416,7 +2418,7 @@ __global__ void __launch_bounds__(1024) moe_route_kernel(MoeGemmDesc g, uint32_t
                                                          uint32_t *tiles, uint16_t *planes) {
   constexpr int KEEP = 8;
   __shared__ uint32_t hist[MOE_ROUTE_MAX_EXPERTS], cursor[MOE_ROUTE_MAX_EXPERTS];
-  __shared__ uint2 wave_sum[16];
+  __shared__ uint32_t wave_sum[16];
   const uint32_t tid = threadIdx.x, E = g.n_expert, S = g.S, pairs = S * g.n_slot;
   if (blockIdx.x) {
     const uint32_t per_row = g.K / 4, n = S * per_row;
@@ -2461,41 +2463,31 @@ __global__ void __launch_bounds__(1024) moe_route_kernel(MoeGemmDesc g, uint32_t
     __syncthreads();
   }
   const uint32_t per = (E + 1023) / 1024, first = tid * per, tp = moe_tile_pairs(g.planes);
-  uint2 local = make_uint2(0, 0);  // pairs, row tiles of this thread's experts
-  for (uint32_t i = first; i < min(E, first + per); ++i) {
-    local.x += hist[i];
-    local.y += (hist[i] + tp - 1) / tp;
-  }
-  uint2 sum = local;
+  uint32_t local = 0;  // row tiles of this thread's experts
+  for (uint32_t i = first; i < min(E, first + per); ++i) local += (hist[i] + tp - 1) / tp;
+  uint32_t sum = local;
   const int lane = tid & 63, wave = tid >> 6;
 #pragma unroll
   for (int d = 1; d < 64; d <<= 1) {
-    const uint32_t x = __shfl_up(sum.x, d, 64), y = __shfl_up(sum.y, d, 64);
-    if (lane >= d) {
-      sum.x += x;
-      sum.y += y;
-    }
+    const uint32_t x = __shfl_up(sum, d, 64);
+    if (lane >= d) sum += x;
   }
   if (lane == 63) wave_sum[wave] = sum;
   __syncthreads();
 #pragma unroll
   for (int w = 0; w < 15; ++w)
-    if (w < wave) {
-      sum.x += wave_sum[w].x;
-      sum.y += wave_sum[w].y;
-    }
-  uint32_t at = sum.x - local.x, tt = sum.y - local.y;
+    if (w < wave) sum += wave_sum[w];
+  uint32_t tt = sum - local;
   for (uint32_t i = first; i < min(E, first + per); ++i) {
-    const uint32_t n = hist[i];
+    const uint32_t n = hist[i], at = tt * tp;
     count[i] = n;
     offset[i] = at;
     if (more) cursor[i] += at;
     hist[i] = at;
-    at += n;
-    if (tiles)
-      for (uint32_t j = 0; j < (n + tp - 1) / tp; ++j) tiles[1 + tt++] = i << 16 | j;
+    const uint32_t n_tiles = (n + tp - 1) / tp;
+    for (uint32_t j = 0; j < n_tiles; ++j) tiles[1 + tt++] = moe_entry(i, n_tiles, j);
   }
-  if (tiles && tid == 1023) tiles[0] = sum.y;
+  if (tid == 1023) tiles[0] = sum;
   __syncthreads();
 #pragma unroll
   for (int j = 0; j < KEEP; ++j) {
@@ -2506,6 +2498,8 @@ __global__ void __launch_bounds__(1024) moe_route_kernel(MoeGemmDesc g, uint32_t
     list[atomicAdd(&cursor[min(expert_of(p / S, p % S), E - 1)], 1u)] = p / S << 16 | p % S;
 }
 
+size_t moe_route_list_words(const MoeGemmDesc &g) { return (size_t)moe_route_max_tiles(g) * moe_tile_pairs(g.planes); }
+
 // most row tiles launch_moe_route can list for g: every expert may end in a partly filled one
 uint32_t moe_route_max_tiles(const MoeGemmDesc &g) {
   return (g.S * g.n_slot + moe_tile_pairs(g.planes) - 1) / moe_tile_pairs(g.planes) + g.n_expert;
@@ -2514,7 +2508,7 @@ uint32_t moe_route_max_tiles(const MoeGemmDesc &g) {
 hipError_t launch_moe_route(const LaunchCtx &lc, const MoeGemmDesc &g, uint32_t *count, uint32_t *offset, uint32_t *list,
                             uint32_t *tiles, uint16_t *planes) {
   if (!g.S || !g.n_slot || !g.n_expert) return hipSuccess;
-  if (g.n_expert > MOE_ROUTE_MAX_EXPERTS || g.S > 65535 || g.n_slot > 8) return hipErrorInvalidValue;
+  if (!tiles || g.n_expert > MOE_ROUTE_MAX_EXPERTS || g.S > 65535 || g.n_slot > 8) return hipErrorInvalidValue;
   if (planes && (!g.slot[0].a || (uintptr_t)g.slot[0].a % 16 || g.slot[0].a_bs % 4 || g.K % 8 || (uintptr_t)planes % 16)) return hipErrorInvalidValue;
   const uint32_t split = planes ? (g.S * (g.K / 4) + 1023) / 1024 : 0;
   CG_LAUNCH(lc, moe_route_kernel, 1 + split, 1024, g, count, offset, list, tiles, planes);
@@ -2557,8 +2551,8 @@ __global__ void __launch_bounds__(256) moe_gemm_dma_kernel(MoeGemmDesc g) {
   if (g.route_tiles) {  // one row tile of one expert
     if (e >= g.route_tiles[0]) return;  // the grid is sized for the most tiles there can be
     const uint32_t ent = g.route_tiles[1 + e];
-    e = ent >> 16;
-    m_first = (ent & 0xFFFFu) * PAIRS;
+    e = moe_entry_expert(ent);
+    m_first = moe_entry_row(ent) * PAIRS;
     m_last = m_first + PAIRS;
   }
   if (e >= g.n_expert) return;  // the grid is sized for the wider problem

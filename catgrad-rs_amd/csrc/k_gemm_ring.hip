@@ -35,6 +35,8 @@
 namespace cgk {
 
 typedef __attribute__((ext_vector_type(16))) float f32x16;
+typedef __attribute__((ext_vector_type(4))) float f32x4;
+typedef __attribute__((ext_vector_type(4))) uint32_t u32x4;
 
 // These kernels' places in LDS are constants that start at 0, where a static __shared__ variable would lie too: no kernel that has
 // one is launched.
@@ -107,6 +109,7 @@ static hipError_t whole_lds(const void *kernel, int bytes) {
 #define M0_B1(i) "s_add_u32 m0, s46, 32768+" #i "*1024\n\t"
 #define M0_A1(i) "s_add_u32 m0, s46, 49152+" #i "*1024\n\t"
 #define LOAD(U, i) "global_load_lds_dwordx4 %[d" #U #i "], " PTR_##U "\n\t"
+#define LOAD_AS(U, i, HINT) "global_load_lds_dwordx4 %[d" #U #i "], " PTR_##U HINT "\n\t"
 #define LOAD_UNIT(U)                                                                                              \
   M0_##U(0) "s_nop 0\n\t" LOAD(U, 0) M0_##U(1) "s_nop 0\n\t" LOAD(U, 1) M0_##U(2) "s_nop 0\n\t" LOAD(U, 2) M0_##U(3) \
   "s_nop 0\n\t" LOAD(U, 3)
@@ -220,16 +223,16 @@ static hipError_t whole_lds(const void *kernel, int bytes) {
   HSLICE(0, B0, 1, READS_BUT(8), HB1(0, 1) G(HM0(1)), HB1(1, 1) G(HLOAD_A(1)), "", "") HFROM_B("s50", 2)                          \
   HSLICE(0, B0, 2, READS_BUT(6), HB1(0, 2) G(HM0(2)), HB1(1, 2) G(HLOAD_A(2)), "", "") HFROM_B("s50", 3)                          \
   HSLICE(0, B0, 3, READS_BUT(6), HB1(0, 3) G(HM0(3)), HB1(1, 3) G(HLOAD_A(3)), "", "")
-#define HPHASE1(G, v)                                                                                                              \
+#define HPHASE1(G, v, HINT)                                                                                                              \
   G("s_add_u32 s54, s48, %[lds]\n\t") HSYNC(v)                                                                                     \
   HFROM_B("s52", 0)                                                                                                                \
-  HSLICE(1, B1, 0, READS_BUT(6), HB0(0, 0) G(HM0(0)), HB0(1, 0) G(LOAD(B0, 0) HM0(1)), G(LOAD(B0, 1)), G(HSTEP_SIZE_AT("s56", "s57"))) \
+  HSLICE(1, B1, 0, READS_BUT(6), HB0(0, 0) G(HM0(0)), HB0(1, 0) G(LOAD_AS(B0, 0, HINT) HM0(1)), G(LOAD_AS(B0, 1, HINT)), G(HSTEP_SIZE_AT("s56", "s57"))) \
   HFROM_A("s51", 0) HFROM_B("s52", 1)                                                                                              \
-  HSLICE(1, B1, 1, READS_BUT(6), HB0(0, 1) G(HM0(2)), HB0(1, 1) G(LOAD(B0, 2) HM0(3)), HA(0, 0) G(LOAD(B0, 3)), HA(1, 0))      \
+  HSLICE(1, B1, 1, READS_BUT(6), HB0(0, 1) G(HM0(2)), HB0(1, 1) G(LOAD_AS(B0, 2, HINT) HM0(3)), HA(0, 0) G(LOAD_AS(B0, 3, HINT)), HA(1, 0))      \
   HFROM_A("s51", 1) HFROM_B("s52", 2) G("s_add_u32 s54, s49, %[lds]\n\t")                                                          \
-  HSLICE(1, B1, 2, READS_BUT(8), HB0(0, 2) G(HM0(0)), HB0(1, 2) G(LOAD(B1, 0) HM0(1)), HA(0, 1) G(LOAD(B1, 1)), HA(1, 1))      \
+  HSLICE(1, B1, 2, READS_BUT(8), HB0(0, 2) G(HM0(0)), HB0(1, 2) G(LOAD_AS(B1, 0, HINT) HM0(1)), HA(0, 1) G(LOAD_AS(B1, 1, HINT)), HA(1, 1))      \
   HFROM_A("s51", 2) HFROM_B("s52", 3)                                                                                              \
-  HSLICE(1, B1, 3, READS_BUT(10), HB0(0, 3) G(HM0(2)), HB0(1, 3) G(LOAD(B1, 2) HM0(3)), HA(0, 2) G(LOAD(B1, 3)), HA(1, 2))
+  HSLICE(1, B1, 3, READS_BUT(10), HB0(0, 3) G(HM0(2)), HB0(1, 3) G(LOAD_AS(B1, 2, HINT) HM0(3)), HA(0, 2) G(LOAD_AS(B1, 3, HINT)), HA(1, 2))
 // (the last step's second phase reads and requests nothing)
 #define HLAST                                                                                                    \
   HSLICE(1, B1, 0, READS_BUT(6), "", "", "", "") HSLICE(1, B1, 1, READS_BUT(4), "", "", "", "")                  \
@@ -239,17 +242,17 @@ static hipError_t whole_lds(const void *kernel, int bytes) {
   "s_mov_b32 s53, s50\n\ts_mov_b32 s48, s51\n\ts_mov_b32 s49, s52\n\t" HNEXT("s50", "s52") HNEXT("s51", "s50") HNEXT("s52", "s51")
 #define HLOADS_A \
   HM0(0) "s_nop 0\n\t" HLOAD_A(0) HM0(1) "s_nop 0\n\t" HLOAD_A(1) HM0(2) "s_nop 0\n\t" HLOAD_A(2) HM0(3) "s_nop 0\n\t" HLOAD_A(3)
-#define HLOADS_B(U) \
-  HM0(0) "s_nop 0\n\t" LOAD(U, 0) HM0(1) "s_nop 0\n\t" LOAD(U, 1) HM0(2) "s_nop 0\n\t" LOAD(U, 2) HM0(3) "s_nop 0\n\t" LOAD(U, 3)
+#define HLOADS_B(U, HINT) \
+  HM0(0) "s_nop 0\n\t" LOAD_AS(U, 0, HINT) HM0(1) "s_nop 0\n\t" LOAD_AS(U, 1, HINT) HM0(2) "s_nop 0\n\t" LOAD_AS(U, 2, HINT) HM0(3) "s_nop 0\n\t" LOAD_AS(U, 3, HINT)
 #define HPOINTERS "s_mov_b64 s[42:43], %[pb0]\n\ts_mov_b64 s[44:45], %[pb1]\n\ts_mov_b32 s55, %[wrap]\n\t" HSTEP_SIZE
 #define HNEXT_B "s_add_u32 s42, s42, s58\n\ts_addc_u32 s43, s43, s59\n\ts_add_u32 s44, s44, s58\n\ts_addc_u32 s45, s45, s59\n\t"
 #define HNEXT_STEP HNEXT_B HSTEP_SIZE
-#define HSTEP_LOADS \
-  HLOADS_A "s_add_u32 s54, s54, 16384\n\t" HLOADS_B(B0) "s_add_u32 s54, s54, 16384\n\t" HLOADS_B(B1) "s_add_u32 s54, s54, 16384\n\t"
+#define HSTEP_LOADS(HINT) \
+  HLOADS_A "s_add_u32 s54, s54, 16384\n\t" HLOADS_B(B0, HINT) "s_add_u32 s54, s54, 16384\n\t" HLOADS_B(B1, HINT) "s_add_u32 s54, s54, 16384\n\t"
 // steps 0 to 2 requested: 36 loads
-#define HFIRST_LOADS HPOINTERS "s_mov_b32 s54, %[lds]\n\t" HSTEP_LOADS HNEXT_STEP HSTEP_LOADS HNEXT_STEP HSTEP_LOADS
+#define HFIRST_LOADS(HINT) HPOINTERS "s_mov_b32 s54, %[lds]\n\t" HSTEP_LOADS(HINT) HNEXT_STEP HSTEP_LOADS(HINT) HNEXT_STEP HSTEP_LOADS(HINT)
 // n >= 3 steps
-#define HMAIN_LOOP                                                                                                              \
+#define HMAIN_LOOP(HINT)                                                                                                              \
   HPOINTERS HNEXT_STEP HNEXT_STEP HNEXT_STEP "s_sub_u32 s47, %[n], 3\n\t"                                                          \
   "s_mov_b32 s48, 0\n\ts_movk_i32 s49, 0x4000\n\ts_mov_b32 s50, 0x8000\n\ts_mov_b32 s51, 0xC000\n\ts_mov_b32 s52, 0x10000\n\t"  \
   "s_mov_b32 s53, 0x24000\n\t" HSYNC(28)                                                                                        \
@@ -257,9 +260,9 @@ static hipError_t whole_lds(const void *kernel, int bytes) {
   HFROM_A("s48", 1) HFROM_B("s49", 2) HB0(0, 2) HB0(1, 2) HA(0, 1) HA(1, 1)                                                 \
   HFROM_A("s48", 2) HFROM_B("s49", 3) HB0(0, 3) HB0(1, 3) HA(0, 2) HA(1, 2)                                                 \
   "s_cmp_eq_u32 s47, 0\n\ts_cbranch_scc1 2f\n\t"                                                                                \
-  "1:\n\t" HPHASE0(HON, 24) HPHASE1(HON, 20) HNEXT_B "s_mov_b64 s[58:59], s[56:57]\n\t" HNEXT_PLACES                                                             \
+  "1:\n\t" HPHASE0(HON, 24) HPHASE1(HON, 20, HINT) HNEXT_B "s_mov_b64 s[58:59], s[56:57]\n\t" HNEXT_PLACES                                                             \
   "s_sub_u32 s47, s47, 1\n\ts_cmp_lg_u32 s47, 0\n\ts_cbranch_scc1 1b\n\t"                                                       \
-  "2:\n\t" HPHASE0(HOFF, 24) HPHASE1(HOFF, 16) HNEXT_PLACES HPHASE0(HOFF, 12) HPHASE1(HOFF, 4) HNEXT_PLACES HPHASE0(HOFF, 0)    \
+  "2:\n\t" HPHASE0(HOFF, 24) HPHASE1(HOFF, 16, HINT) HNEXT_PLACES HPHASE0(HOFF, 12) HPHASE1(HOFF, 4, HINT) HNEXT_PLACES HPHASE0(HOFF, 0)    \
   HLAST "s_nop 15\n\ts_nop 7\n\t"
 
 // ---- tiles of 256 x 288: the four quadrants and a strip X of 32 columns more, a ninth of the products with no wavefront idle: in each
@@ -640,7 +643,7 @@ __global__ void __launch_bounds__(256, 1) gemm_bf16_ring_kernel(GemmDesc g) {
 #define RING_STRIP RING_V10(11), "v120", "v121", "v122", "v123", "v124", "v125", "v126", "v127"
   if constexpr (WIDE) asm volatile(WFIRST_LOADS::RING_IN, RING_WIDE_IN : RING_SCALARS, RING_WIDE_SCALARS);
   else if constexpr (AH == 2) asm volatile(FIRST_LOADS::RING_IN : RING_SCALARS);
-  else asm volatile(HFIRST_LOADS : RING_GATHERED : RING_IN_B, RING_ORDER : RING_SCALARS);
+  else asm volatile(HFIRST_LOADS("") : RING_GATHERED : RING_IN_B, RING_ORDER : RING_SCALARS);
   float zero;
   asm volatile("v_mov_b32 %0, 0" : "=v"(zero));  // (the accumulators are cleared behind the first loads, not in front of them)
   f32x16 acc[AH][2][2][2];  // [A half][B half][row block][column block]
@@ -686,7 +689,7 @@ __global__ void __launch_bounds__(256, 1) gemm_bf16_ring_kernel(GemmDesc g) {
   else if constexpr (AH == 2)
     asm volatile(MAIN_LOOP : RING_ACC0, RING_ACC1, RING_PLACES : RING_IN, [n] "s"(n_steps) : RING_SCALARS, RING_FRAGMENTS);
   else
-    asm volatile(HMAIN_LOOP : RING_ACC0, RING_PLACES, RING_GATHERED : RING_IN_B, RING_ORDER, [n] "s"(n_steps) : RING_SCALARS, RING_HALF_SCALARS, RING_FRAGMENTS);
+    asm volatile(HMAIN_LOOP("") : RING_ACC0, RING_PLACES, RING_GATHERED : RING_IN_B, RING_ORDER, [n] "s"(n_steps) : RING_SCALARS, RING_HALF_SCALARS, RING_FRAGMENTS);
   if (KIND == RING_PLAIN && g.clock_ticks && tid == 0) {
     atomicAdd(g.clock_ticks, __builtin_amdgcn_s_memtime() - tick0);
     atomicAdd(g.clock_ticks + 1, __builtin_amdgcn_s_memrealtime() - real0);
@@ -856,45 +859,99 @@ __global__ void __launch_bounds__(256, 1) gemm_bf16_ring_kernel(GemmDesc g) {
 // ---- the routed experts of a prefill: a row tile of 128 (slot, token) pairs of one expert by 256 weight rows ------------------
 // (MoeGemmDesc with route_tiles; the work and its order are those of moe_gemm_dma_kernel, which says how pairs are sorted.)
 // MOE_SILU, MOE_GELU: 128 rows of gate_proj and the same of up_proj, act(gate) * up leaves as bf16; MOE_PLAIN: 256 rows of one
-// matrix, f32.  Rows of A are gathered; pairs past the expert's last repeat it, and are not stored.
-// Bound by the stream of weights in pieces of 128 bytes, rows 4 KB apart (141 us for the load schedule of gate and up alone): 60
-// experts of 2 x 1408 x 2048, 4096 pairs in crowded experts and empty ones, 161 -> 148 us against moe_gemm_dma_kernel, 2048 x 1408
-// 92 -> 82 (streaming loads, which suit that kernel, 150 and 85).  As a router deals 4096 pairs, more evenly, 158 to 169 and 87 to 90.
+// matrix, f32.  Rows of A are gathered; those past the expert's last pair are some token's, and are not stored.
+//
+// MoeGemmDesc::dense is one more expert that all tokens pass through, tiles of the same launch: the routed ones wait for memory (68 rows
+// to 256 of weights), its tiles for the matrix cores, and neither launch has a last round of its own.  60 experts of 2 x 1408 x 2048 and
+// 2048 x 1408, 4 to a token, a dense one of 5632, 1024 tokens, both launches: 338 us in four launches and a sum of k-slices, 252 so; 1500
+// tokens 380, 293; 660 309, 247; 2600 590, 510.
+//
+// Bound by the stream of weights, which the loads alone take 117 and 60 us for (692 and 346 MB; 256 workgroups that load these tiles into
+// LDS and do nothing else).  What it reaches of that, without the dense expert, 140 and 76 us (before: 158 and 84):
+//   * Weights that one row tile reads are loaded with the hint that they are used once, what others will read is not (60 experts, 1024
+//     tokens 236 -> 216 us in both launches, the dense tiles' weights with it 277 instead of 253; 2048 tokens, two row tiles to most
+//     experts, 334 and 347 with it).
+//   * Results leave with that hint, whole lines at a time: 83 -> 76 us for the f32 result of 33 MB, 144 -> 140 for gate and up.
+//   * What a tile needs to know comes in two trips to memory in front of its first load - the place of a row tile's pairs in the list
+//     follows from the work list's entry -, and where its rows go with them: under the weights' stream a trip is 2 to 4 us.
+//   * The row tiles of a crowded expert stand next to each other (2048 tokens, both launches with the dense expert 440 -> 424 us, 4096 708
+//     -> 677, 1024 in crowded experts 301 -> 293; by expert and row tile before).
+//   * A loop over tiles that requests the next one's first steps in front of the stores of this one: no change (217 and 216 us).
 enum { MOE_PLAIN, MOE_SILU, MOE_GELU };
 template <int KIND>
 __global__ void __launch_bounds__(256, 1) moe_ring_kernel(MoeGemmDesc g) {
   constexpr bool GATED = KIND != MOE_PLAIN;
   constexpr uint32_t BNO = GATED ? 128 : 256;
+  typedef const __attribute__((address_space(4))) uint32_t *Uniform;  // (read by scalar loads: written by the launch before)
   warm_kernel_arguments<sizeof(MoeGemmDesc)>();
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), wm = wave >> 1, wn = wave & 1;
-  const uint32_t prob = GATED ? 0 : blockIdx.y, K = g.K, N = g.prob[prob].N;
-  const uint32_t tiles_n = (N + BNO - 1) / BNO, tile = blockIdx.x / tiles_n, n0 = (blockIdx.x - tile * tiles_n) * BNO;
-  if (tile >= g.route_tiles[0]) return;  // the grid is sized for the most tiles there can be, and the wider problem
-  const uint32_t entry = g.route_tiles[1 + tile], e = entry >> 16, m0 = (entry & 0xFFFFu) * 128;
-  if (e >= g.n_expert) return;
-  const uint32_t live = min(g.route_count[e] - m0, 128u), *list = g.route_list + g.route_offset[e] + m0;
+  const uint32_t prob = GATED ? 0 : blockIdx.y, tiles_n = (g.prob[prob].N + BNO - 1) / BNO;
+  // This XCD's tiles: its columns of the dense expert, all row tiles of a column one after the other, and a contiguous range of the
+  // routed experts' that makes the numbers of all XCDs equal.
+  const uint32_t dense_m = (g.S + 127) / 128, dense_n = (g.dense.N + BNO - 1) / BNO, xcd = blockIdx.x & 7, at = blockIdx.x >> 3;
+  const uint32_t total = ((Uniform)g.route_tiles)[0] * tiles_n + dense_m * dense_n, mine = total / 8 + (xcd < total % 8);
+  const uint32_t mine_dense = dense_m * (dense_n / 8 + (xcd < dense_n % 8));
+  if (at >= mine) return;  // the grid is sized for the most tiles there can be, and the wider problem
+  uint32_t before;  // dense tiles in front of this one
+  bool dense;
+  if (g.dense.K > g.K) {  // the longer tiles first
+    before = min(at, mine_dense);
+    dense = at < mine_dense;
+  } else {  // spread evenly: what waits for the matrix cores among what waits for memory
+    before = uniform_quotient(at * mine_dense, mine);
+    dense = uniform_quotient((at + 1) * mine_dense, mine) > before;
+  }
+  const uint32_t *list = g.route_list;
+  uint32_t e = 0, m0, n0, live, N = g.prob[prob].N, K = g.K;
+  bool once = false;  // no other row tile reads these weights
+  if (dense) {
+    const uint32_t col = uniform_quotient(before, dense_m);
+    m0 = (before - col * dense_m) * 128;
+    n0 = (col * 8 + xcd) * BNO;
+    live = min(g.S - m0, 128u);
+    N = g.dense.N;
+    K = g.dense.K;
+  } else {
+    const uint32_t t = xcd * (total / 8) + min(xcd, total % 8) - dense_m * (xcd * (dense_n / 8) + min(xcd, dense_n % 8)) + at - before;
+    const uint32_t tile = uniform_quotient(t, tiles_n), entry = ((Uniform)g.route_tiles)[1 + tile], many = moe_entry_tiles(entry);
+    e = moe_entry_expert(entry);
+    uint32_t row = moe_entry_row(entry), col = t - tile * tiles_n;
+    list += (tile - row) * 128;
+    if (many > 1) {  // an expert's column tiles one after the other, all row tiles at each: they share the weights
+      const uint32_t place = row * tiles_n + col;
+      col = uniform_quotient(place, many);
+      row = place - col * many;
+    }
+    n0 = col * BNO;
+    m0 = row * 128;
+    list += m0;
+    const uint32_t pairs = ((Uniform)g.route_count)[e];
+    live = min(pairs - m0, 128u);
+    once = pairs <= 128;
+  }
+  uint32_t ent[5];  // slot << 16 | token of this lane's rows of A, and of the row it sends off
+#pragma unroll
+  for (int i = 0; i < 5; ++i) {
+    const uint32_t r = i < 4 ? (wave * 4 + i) * 8 + (lane >> 3) : wm * 64 + lane, in_list = list[r];
+    ent[i] = dense ? m0 + r : in_list;
+    if (r >= live) ent[i] = 0;  // past the expert's last pair, where the list is not written: some token's row, not stored
+  }
   const uint32_t n_steps = __builtin_amdgcn_readfirstlane(K / 64);
-  const int64_t sbn0 = g.prob[prob].sbn;
-  const KOrder order(g.k_rotate, e * tiles_n + n0 / BNO, n_steps);
-  const uint16_t *pb0 = (const uint16_t *)g.prob[prob].w + (int64_t)e * g.sb_index + (int64_t)n0 * sbn0 + order.first * 64;
-  const uint16_t *pb1 = GATED ? (const uint16_t *)g.prob[1].w + (int64_t)e * g.sb_index + (int64_t)n0 * g.prob[1].sbn + order.first * 64 : pb0;
-  const uint32_t sb = (uint32_t)sbn0 * 2, sb1 = GATED ? (uint32_t)g.prob[1].sbn * 2 : sb, last_b = N - 1 - n0;
+  const int64_t sbn0 = dense ? g.dense.sbn : g.prob[prob].sbn, sbn1 = dense || !GATED ? sbn0 : g.prob[1].sbn;
+  const KOrder order(dense ? 0u : g.k_rotate, e * tiles_n + n0 / BNO, n_steps);
+  const uint16_t *w0 = dense ? (const uint16_t *)g.dense.w[0] : (const uint16_t *)g.prob[prob].w + (int64_t)e * g.sb_index;
+  const uint16_t *w1 = dense ? (const uint16_t *)g.dense.w[1] : (const uint16_t *)g.prob[1].w + (int64_t)e * g.sb_index;
+  const uint16_t *pb0 = w0 + (int64_t)n0 * sbn0 + order.first * 64, *pb1 = GATED ? w1 + (int64_t)n0 * sbn1 + order.first * 64 : pb0;
+  const uint32_t sb = (uint32_t)sbn0 * 2, sb1 = (uint32_t)sbn1 * 2, last_b = N - 1 - n0;
+  const uint16_t *rows = dense ? g.dense.a16 : g.slot[0].a16;
+  const int64_t row_pitch = dense ? g.dense.a_bs : g.slot[0].a_bs;
   uint64_t ga[4];
   uint32_t dB0[4], dB1[4];
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const uint32_t r = (wave * 4 + i) * 8 + (lane >> 3), c = ((lane & 7) ^ ((r >> 1) & 7)) * 16;
-    const uint32_t ent = list[min(r, live - 1)], sl = ent >> 16;
-    const uint16_t *rows = g.slot[0].a16;
-    int64_t bs = g.slot[0].a_bs;
-#pragma unroll
-    for (int s = 1; s < 8; ++s)
-      if (sl == (uint32_t)s) {
-        rows = g.slot[s].a16;
-        bs = g.slot[s].a_bs;
-      }
-    ga[i] = (uint64_t)(rows + (int64_t)(ent & 0xFFFFu) * bs) + order.first * 128 + c;
+    ga[i] = (uint64_t)(rows + (ent[i] >> 16) * g.a_slot + (ent[i] & 0xFFFFu) * row_pitch) + order.first * 128 + c;
     dB0[i] = min(r, last_b) * sb + c;
     dB1[i] = GATED ? min(r, last_b) * sb1 + c : min(r + 128, last_b) * sb + c;
   }
@@ -907,7 +964,10 @@ __global__ void __launch_bounds__(256, 1) moe_ring_kernel(MoeGemmDesc g) {
 #define MOE_IN                                                                                                            \
   [dB00] "v"(dB0[0]), [dB01] "v"(dB0[1]), [dB02] "v"(dB0[2]), [dB03] "v"(dB0[3]), [dB10] "v"(dB1[0]), [dB11] "v"(dB1[1]), \
       [dB12] "v"(dB1[2]), [dB13] "v"(dB1[3]), [pb0] "s"(s_b0), [pb1] "s"(s_b1), [lds] "s"(lds)
-  asm volatile(HFIRST_LOADS : RING_GATHERED : MOE_IN, RING_ORDER : RING_SCALARS);
+  if (once) asm volatile(HFIRST_LOADS(" nt") : RING_GATHERED : MOE_IN, RING_ORDER : RING_SCALARS);
+  else asm volatile(HFIRST_LOADS("") : RING_GATHERED : MOE_IN, RING_ORDER : RING_SCALARS);
+  const uint64_t out = (uint64_t)(GATED ? (void *)(dense ? g.dense.h16 : g.slot[0].h16) : (void *)(dense ? g.dense.c : g.slot[0].c[prob]));
+  const uint64_t base = out + ((ent[4] >> 16) * g.out_slot + (ent[4] & 0xFFFFu) * (uint64_t)N) * (GATED ? 2 : 4);
   float zero;
   asm volatile("v_mov_b32 %0, 0" : "=v"(zero));
   f32x16 acc[1][2][2][2];  // [0][B half][row block][column block]
@@ -923,48 +983,77 @@ __global__ void __launch_bounds__(256, 1) moe_ring_kernel(MoeGemmDesc g) {
     ra[ks] = wm * 8192 + p;
     rb[ks] = wn * 8192 + p;
   }
-  asm volatile(HMAIN_LOOP : RING_ACC0, RING_PLACES, RING_GATHERED : MOE_IN, RING_ORDER, [n] "s"(n_steps) : RING_SCALARS, RING_HALF_SCALARS, RING_FRAGMENTS);
-  // Rows back to their slot and token, out of LDS as in gemm_bf16_ring_kernel: a lane finds where the row of its number goes and
-  // hands that to the sixteen lanes that store it.
-  __syncthreads();
+  if (once)
+    asm volatile(HMAIN_LOOP(" nt") : RING_ACC0, RING_PLACES, RING_GATHERED : MOE_IN, RING_ORDER, [n] "s"(n_steps) : RING_SCALARS, RING_HALF_SCALARS, RING_FRAGMENTS);
+  else
+    asm volatile(HMAIN_LOOP("") : RING_ACC0, RING_PLACES, RING_GATHERED : MOE_IN, RING_ORDER, [n] "s"(n_steps) : RING_SCALARS, RING_HALF_SCALARS, RING_FRAGMENTS);
+  // Rows back to their slot and token, through 4 KB of LDS of each wavefront's own: 32 rows of 64 bf16 or of 32 f32 values at a time, of
+  // which eight lanes store a line.  A lane knows where the row of its number goes, and hands that to the eight.
+  __syncthreads();  // every wavefront has read its last fragments
   extern __shared__ __attribute__((aligned(16))) float ring_smem[];
-  const uint32_t my_row = wm * 64 + lane, ent = list[min(my_row, live - 1)], sl = ent >> 16;
-  uint64_t base = (uint64_t)(GATED ? (void *)g.slot[0].h16 : (void *)g.slot[0].c[prob]);
-#pragma unroll
-  for (int s = 1; s < 8; ++s)
-    if (sl == (uint32_t)s) base = (uint64_t)(GATED ? (void *)g.slot[s].h16 : (void *)g.slot[s].c[prob]);
-  base += (uint64_t)(ent & 0xFFFFu) * N * (GATED ? 2 : 4);
+  float *stage = ring_smem + wave * 1024;
+  const uint32_t my_rows = live > wm * 64u ? live - wm * 64u : 0u, piece = (lane & 7) ^ (lane >> 3);
   const int base_lo = (int)base, base_hi = (int)(base >> 32);
 #pragma unroll
-  for (int qd = 0; qd < (GATED ? 1 : 2); ++qd) {
-    float *stage = ring_smem + wave * 8192 + qd * 4096;
+  for (int i = 0; i < 2; ++i) {
+    uint64_t to[4];
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int it = 0; it < 4; ++it) {
+      const int r = i * 32 + it * 8 + (lane >> 3);
+      to[it] = (uint64_t)(uint32_t)__shfl(base_lo, r, 64) | (uint64_t)(uint32_t)__shfl(base_hi, r, 64) << 32;
+    }
+    if constexpr (GATED) {
 #pragma unroll
       for (int j = 0; j < 2; ++j)
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-          const uint32_t r = i * 32 + (lane & 31), chunk = j * 8 + q * 2 + half;
-          const f32x16 &x = acc[0][qd][i][j], &u = acc[0][GATED ? 1 : qd][i][j];
+          const uint32_t r = lane & 31, chunk = j * 8 + q * 2 + half;  // four columns
+          const f32x16 &x = acc[0][0][i][j], &u = acc[0][1][i][j];
           float4 v = make_float4(x[q * 4], x[q * 4 + 1], x[q * 4 + 2], x[q * 4 + 3]);
           if (KIND == MOE_GELU) v = make_float4(gelu_fast(v.x), gelu_fast(v.y), gelu_fast(v.z), gelu_fast(v.w));
           if (KIND == MOE_SILU) v = make_float4(silu_fast(v.x), silu_fast(v.y), silu_fast(v.z), silu_fast(v.w));
-          if (GATED) { v.x *= u[q * 4]; v.y *= u[q * 4 + 1]; v.z *= u[q * 4 + 2]; v.w *= u[q * 4 + 3]; }
-          *(float4 *)(stage + r * 64 + ((chunk ^ (r & 15)) << 2)) = v;
+          v.x *= u[q * 4]; v.y *= u[q * 4 + 1]; v.z *= u[q * 4 + 2]; v.w *= u[q * 4 + 3];
+          *(uint2 *)((char *)stage + r * 128 + ((chunk ^ ((r & 7) << 1)) << 3)) = bf16_pack4(v);
         }
-    const uint32_t col0 = n0 + qd * 128 + wn * 64;
+      const uint32_t col = n0 + wn * 64 + (lane & 7) * 8;
 #pragma unroll
-    for (int it = 0; it < 16; ++it) {
-      const int r = it * 4 + (lane >> 4);
-      const uint32_t col = col0 + (((lane & 15) ^ (r & 15)) << 2);
-      const float4 v = *(const float4 *)(stage + r * 64 + ((lane & 15) << 2));
-      const uint64_t to = (uint64_t)(uint32_t)__shfl(base_lo, r, 64) | (uint64_t)(uint32_t)__shfl(base_hi, r, 64) << 32;
-      if (wm * 64 + r < live && col < N) {  // (N % 8 == 0: a piece is inside or outside)
-        if (GATED) *(uint2 *)((uint16_t *)to + col) = bf16_pack4(v);
-        else *(float4 *)((float *)to + col) = v;
+      for (int it = 0; it < 4; ++it) {
+        const u32x4 v = *(const u32x4 *)((const char *)stage + (it * 8 + (lane >> 3)) * 128 + piece * 16);
+        if (i * 32 + it * 8 + (lane >> 3) < my_rows && col < N)  // (N % 8 == 0: a piece is inside or outside)
+          __builtin_nontemporal_store(v, (u32x4 *)((uint16_t *)to[it] + col));
+      }
+    } else {
+#pragma unroll
+      for (int b = 0; b < 4; ++b) {  // column half, block of 32 columns
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const f32x16 &x = acc[0][b >> 1][i][b & 1];
+          *(float4 *)(stage + (lane & 31) * 32 + (((q * 2 + half) ^ (lane & 7)) << 2)) = make_float4(x[q * 4], x[q * 4 + 1], x[q * 4 + 2], x[q * 4 + 3]);
+        }
+        const uint32_t col = n0 + (b >> 1) * 128 + wn * 64 + (b & 1) * 32 + (lane & 7) * 4;
+#pragma unroll
+        for (int it = 0; it < 4; ++it) {
+          const f32x4 v = *(const f32x4 *)(stage + (it * 8 + (lane >> 3)) * 32 + piece * 4);
+          if (i * 32 + it * 8 + (lane >> 3) < my_rows && col < N) __builtin_nontemporal_store(v, (f32x4 *)((float *)to[it] + col));
+        }
       }
     }
   }
+}
+
+// what lies between the rows and between the results of consecutive slots, in values
+static bool moe_slot_pitches(const MoeGemmDesc &g, int64_t *a, int64_t *out) {
+  const int64_t ob = g.fuse_glu ? 2 : 4;
+  auto out_of = [&](uint32_t s, uint32_t p) { return g.fuse_glu ? (int64_t)(intptr_t)g.slot[s].h16 : (int64_t)(intptr_t)g.slot[s].c[p]; };
+  const int64_t ab = g.n_slot > 1 ? (int64_t)(intptr_t)g.slot[1].a16 - (int64_t)(intptr_t)g.slot[0].a16 : 0, cb = g.n_slot > 1 ? out_of(1, 0) - out_of(0, 0) : 0;
+  for (uint32_t s = 0; s < g.n_slot; ++s) {
+    if ((int64_t)(intptr_t)g.slot[s].a16 != (int64_t)(intptr_t)g.slot[0].a16 + s * ab || g.slot[s].a_bs != g.slot[0].a_bs) return false;
+    for (uint32_t p = 0; p < (g.fuse_glu ? 1 : g.n_prob); ++p)
+      if (out_of(s, p) != out_of(0, p) + s * cb) return false;
+  }
+  *a = ab / 2;
+  *out = cb / ob;
+  return ab % 2 == 0 && cb % ob == 0;
 }
 
 // (route_tiles, 32-bit byte offsets within a tile's weight rows, three k-steps; otherwise what moe_gemm_pipelined_ok asks)
@@ -973,10 +1062,23 @@ bool moe_ring_ok(const MoeGemmDesc &g) {
   // wait for weights either way (a whole prefill of 60 experts, 4 to a token: 17 pairs to an expert 7.85 -> 8.55 ms, 34 9.49 ->
   // 9.77, 40 9.73 -> 9.82; 47 10.9 -> 10.3, 73 13.8 -> 12.4).
   if ((uint64_t)g.S * g.n_slot < 44 * (uint64_t)g.n_expert) return false;
-  if (!moe_gemm_pipelined_ok(g) || !g.route_tiles || g.planes || g.K < 192) return false;
+  int64_t a, out;
+  if (!moe_gemm_pipelined_ok(g) || !g.route_tiles || g.planes || g.K < 192 || !moe_slot_pitches(g, &a, &out)) return false;
   for (uint32_t p = 0; p < g.n_prob; ++p)
     if (g.prob[p].sbn < 0 || g.prob[p].sbn > (1 << 22)) return false;
   return g.fuse_glu ? g.n_prob == 2 && g.prob[0].N == g.prob[1].N : true;
+}
+
+// The dense expert's tiles are dealt to the XCDs by whole columns, and the others even that out: there have to be enough of those (eight
+// columns' worth), and few enough of all for the products of their numbers.
+bool moe_dense_ok(const MoeGemmDesc &g) {
+  const auto &d = g.dense;
+  const uint64_t bno = g.fuse_glu ? 128 : 256, rows = (g.S + 127) / 128, cols = (d.N + bno - 1) / bno, tiles_n = (g.prob[0].N + bno - 1) / bno;
+  const uint64_t fewest = ((uint64_t)g.S * g.n_slot + 127) / 128 * tiles_n, most = moe_route_max_tiles(g) * tiles_n + rows * cols;
+  if (!d.N || !moe_ring_ok(g) || (!g.fuse_glu && g.n_prob != 1) || fewest < 8 * rows || most / 8 >= 65535 || rows * (cols / 8 + 1) >= 65535) return false;
+  return d.N % 8 == 0 && d.K % 64 == 0 && d.K >= 192 && d.a16 && (uintptr_t)d.a16 % 16 == 0 && d.a_bs % 8 == 0 && (uintptr_t)d.w[0] % 16 == 0 &&
+         (!g.fuse_glu || (uintptr_t)d.w[1] % 16 == 0) && d.sbn % 8 == 0 && d.sbn >= 0 && d.sbn <= (1 << 22) &&
+         (g.fuse_glu ? d.h16 && (uintptr_t)d.h16 % 16 == 0 : d.c && (uintptr_t)d.c % 16 == 0);
 }
 
 template <int KIND>
@@ -992,12 +1094,14 @@ static hipError_t launch_moe_ring_as(const LaunchCtx &lc, const MoeGemmDesc &g, 
   return hipGetLastError();
 }
 
-hipError_t launch_moe_ring(const LaunchCtx &lc, const MoeGemmDesc &g) {
-  if (!moe_ring_ok(g)) return hipErrorInvalidValue;
+hipError_t launch_moe_ring(const LaunchCtx &lc, const MoeGemmDesc &given) {
+  MoeGemmDesc g = given;
+  if (!moe_ring_ok(g) || (g.dense.N && !moe_dense_ok(g)) || !moe_slot_pitches(g, &g.a_slot, &g.out_slot)) return hipErrorInvalidValue;
   uint32_t max_n = 0;
   for (uint32_t p = 0; p < g.n_prob; ++p) max_n = g.prob[p].N > max_n ? g.prob[p].N : max_n;
   const uint32_t bno = g.fuse_glu ? 128 : 256;
-  const dim3 grid((max_n + bno - 1) / bno * moe_route_max_tiles(g), g.fuse_glu ? 1 : g.n_prob, 1);
+  const uint32_t most = (max_n + bno - 1) / bno * moe_route_max_tiles(g) + (g.S + 127) / 128 * ((g.dense.N + bno - 1) / bno);
+  const dim3 grid((most + 7) / 8 * 8, g.fuse_glu ? 1 : g.n_prob, 1);
   if (g.fuse_glu) return g.fuse_glu == PRO_GEGLU ? launch_moe_ring_as<MOE_GELU>(lc, g, grid) : launch_moe_ring_as<MOE_SILU>(lc, g, grid);
   return launch_moe_ring_as<MOE_PLAIN>(lc, g, grid);
 }

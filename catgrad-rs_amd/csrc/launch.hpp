@@ -546,24 +546,41 @@ struct MoeGemmDesc {
   const uint32_t *route_count, *route_offset, *route_list;
   // optional, with the above: the row tiles of all experts as a work list (launch_moe_route's `tiles`)
   const uint32_t *route_tiles;
+  int64_t a_slot, out_slot;  // (set by launch_moe_ring) values between the rows, and between the results, of consecutive slots
   uint32_t k_rotate;  // (set by launch_moe_gemm) as GemmDesc::k_rotate
+  // optional (N != 0, moe_dense_ok): one more expert, which every token passes through (a shared expert), in the same launch: its rows a16,
+  // its matrices [N, K] - gate_proj and up_proj with fuse_glu, down_proj in w[0] without - and what h16 or c get, contiguous [S, N]
+  struct {
+    const void *w[2];
+    int64_t sbn, a_bs;
+    const uint16_t *a16;
+    uint16_t *h16;
+    float *c;
+    uint32_t N, K;
+  } dense;
 };
 hipError_t launch_moe_gemm(const LaunchCtx &lc, const MoeGemmDesc &g);
 // k_gemm_ring.hip: the same for sorted pairs with a work list
 bool moe_ring_ok(const MoeGemmDesc &g);
+bool moe_dense_ok(const MoeGemmDesc &g);  // ... and g.dense among them
 hipError_t launch_moe_ring(const LaunchCtx &lc, const MoeGemmDesc &g);
 // Sorts the S * n_slot (slot, token) pairs of g by expert into count / offset (n_expert words each) and
-// list (S * n_slot words); n_expert <= MOE_ROUTE_MAX_EXPERTS.  With these in g.route_*, bf16 input rows
+// list (moe_route_list_words; every expert's pairs start at a row tile's); n_expert <= MOE_ROUTE_MAX_EXPERTS.  With these in g.route_*, bf16 input rows
 // (slot[].a16 for every slot) and K % 64 == 0, launch_moe_gemm streams the weights through a
 // multi-stage direct-to-LDS pipeline.
 enum { MOE_ROUTE_MAX_EXPERTS = 4096 };
-// tiles (optional, 1 + moe_route_max_tiles(g) words): the number of row tiles (128 pairs, 20 of planes) over all experts, then
-// expert << 16 | row tile for each; with it in g.route_tiles a workgroup of launch_moe_gemm owns one row tile
+// tiles (1 + moe_route_max_tiles(g) words): the number of row tiles (128 pairs, 20 of planes) over all experts, then
+// for each its expert, the number of that expert's row tiles (1 if they are more than 255) and its own number among them (moe_entry); with it in g.route_tiles a workgroup of launch_moe_gemm owns one row tile
 // of one expert, so the launch stays balanced when most tokens choose the same few experts.
 // planes (optional): the S rows of K f32 values at slot[0].a, as the planes that launch_moe_gemm takes
 hipError_t launch_moe_route(const LaunchCtx &lc, const MoeGemmDesc &g, uint32_t *count, uint32_t *offset, uint32_t *list,
                             uint32_t *tiles, uint16_t *planes);
+__host__ __device__ constexpr uint32_t moe_entry(uint32_t expert, uint32_t tiles, uint32_t row) { return expert << 20 | (tiles < 256 ? tiles : 1u) << 12 | row; }
+__host__ __device__ constexpr uint32_t moe_entry_expert(uint32_t e) { return e >> 20; }
+__host__ __device__ constexpr uint32_t moe_entry_tiles(uint32_t e) { return e >> 12 & 255u; }
+__host__ __device__ constexpr uint32_t moe_entry_row(uint32_t e) { return e & 0xFFFu; }
 uint32_t moe_route_max_tiles(const MoeGemmDesc &g);
+size_t moe_route_list_words(const MoeGemmDesc &g);
 bool moe_gemm_pipelined_ok(const MoeGemmDesc &g);
 // wrapping u32 matmul (ndarray's generic dot); all operands contiguous
 hipError_t launch_matmul_u32(const LaunchCtx &lc, const uint32_t *a, const uint32_t *b, uint32_t *c,

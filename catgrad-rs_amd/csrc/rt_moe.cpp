@@ -17,6 +17,47 @@ bool match_expert_operand(const cg_tensor *t, int64_t S, ExpertOperand *o) {
 }
 
 
+// An expert that every token passes through, still waiting: down_proj(act(gate_proj(x)) * up_proj(x)) of rows x that the routed experts
+// read too (`x` is their input, realised).
+struct DenseExpert {
+  cg_tensor *down = nullptr, *wg = nullptr, *wu = nullptr, *wd = nullptr;
+};
+static int find_dense_expert(cg_backend *be, const cg_tensor *x, int gelu, DenseExpert *out) {
+  const int64_t S = x->shape[0], H = x->shape[2];
+  auto weight_ok = [](const cg_tensor *w) {
+    return w->rank == 3 && w->shape[0] == 1 && w->stype == ST_BF16 && w->strides[1] == 1 && (uintptr_t)data_ptr(w) % 16 == 0 && w->strides[2] % 8 == 0;
+  };
+  auto in_memory = [](const cg_tensor *t) {  // a view of a value there is
+    while ((t->op == N_RESHAPE || t->op == N_TRANSPOSE || t->op == N_BROADCAST) && t->in[0]) t = t->in[0];
+    return t->op == N_REAL ? t : nullptr;
+  };
+  for (cg_tensor *c : std::vector<cg_tensor *>(be->gemm_candidates)) {
+    if (c->op != N_MATMUL || c->bias_user || c->dtype != CG_F32 || c->rank != 3 || c->shape[0] != 1 || c->shape[1] != S) continue;
+    cg_tensor *glu = c->in[0], *g = nullptr, *u = nullptr;
+    int ge = 0;
+    if (glu->op == N_REAL || refs(glu) != 1 || !match_glu(glu, &g, &u, &ge) || ge != gelu) continue;
+    if (g->op != N_MATMUL || u->op != N_MATMUL || g == u || refs(g) != (ge ? 3 : 2) || refs(u) != 1 || !same_rows(g->in[0], u->in[0]) ||
+        !g->gemm_candidate || !u->gemm_candidate || !std::equal(g->shape, g->shape + 3, u->shape) || g->in[0]->shape[2] != H)
+      continue;
+    cg_tensor *a = g->in[0];
+    const cg_tensor *rows = in_memory(a);
+    if (!rows || rows->st != x->st || !in_memory(g->in[1]) || !in_memory(u->in[1]) || !in_memory(c->in[1])) continue;
+    TRY(realize(be, a));
+    if (a->st != x->st || a->offset != x->offset || a->stype != ST_F32 || a->strides[2] != 1 || a->strides[1] != x->strides[0]) continue;
+    TRY(realize(be, g->in[1]));
+    TRY(realize(be, u->in[1]));
+    TRY(realize(be, c->in[1]));
+    if (!weight_ok(g->in[1]) || !weight_ok(u->in[1]) || !weight_ok(c->in[1]) || g->in[1]->strides[2] != u->in[1]->strides[2]) continue;
+    out->down = c;
+    out->wg = g->in[1];
+    out->wu = u->in[1];
+    out->wd = c->in[1];
+    return CG_OK;
+  }
+  return CG_OK;
+}
+
+
 // The same products over many tokens (a prefill, bf16 mode): expert by expert instead of token by
 // token, and all k slots of the layer in one launch - every deferred expert product on the same
 // stacked weights joins, with its own indices, input rows and output (launch_moe_gemm).
@@ -171,21 +212,18 @@ int try_moe_gemm(cg_backend *be, cg_tensor *n, bool *done) {
       if (planes && (H % 64 || F % 64 || d.n_expert > MOE_ROUTE_MAX_EXPERTS)) return CG_OK;  // token by token
       if (H % 8 == 0 && x->stype == ST_F32 && x->strides[2] == 1 && x->strides[0] % 8 == 0 && x->offset % 8 == 0 &&
           x->st->bytes % 32 == 0 && x->st->grow_dim < 0 && w_ok(wg, F, H) && w_ok(wu, F, H) && wg->strides[0] == wu->strides[0]) {
-        Storage *xsh = nullptr, *xplanes = nullptr;
-        if (!planes) TRY(bf16_shadow(be, x->st, &xsh));
-        std::vector<Storage *> hbuf(slot_a.size(), nullptr);
-        auto drop_h = [&]() {
-          for (Storage *h : hbuf) storage_release(h);
-          storage_release(xplanes);
-        };
-        int st = planes ? dev_alloc(be, (size_t)S * H * 6, &xplanes) : CG_OK;
-        for (size_t sl = 0; sl < hbuf.size() && !st; ++sl) st = dev_alloc(be, (size_t)S * F * (planes ? 6 : 2), &hbuf[sl]);
-        for (const Member &m : members)
-          if (!st) st = alloc_result(be, m.c, ST_F32);
-        if (st) {
-          drop_h();
+        const int64_t N = d.prob[0].N, c_slot = (S * N + 63) / 64 * 64, h_slot = S * F * (planes ? 3 : 1);
+        Storage *xsh = nullptr, *xplanes = nullptr, *hbuf = nullptr, *cbuf = nullptr, *route = nullptr, *dense_h = nullptr, *dense_c = nullptr;
+        auto drop = [&](int st) {
+          for (Storage *b : {xplanes, hbuf, cbuf, route, dense_h, dense_c}) storage_release(b);
           return st;
-        }
+        };
+        if (!planes) TRY(bf16_shadow(be, x->st, &xsh));
+        int st = planes ? dev_alloc(be, (size_t)S * H * 6, &xplanes) : CG_OK;
+        // the slots' gated rows, and their results, behind one another at one distance
+        if (!st) st = dev_alloc(be, (size_t)d.n_slot * h_slot * 2, &hbuf);
+        if (!st) st = dev_alloc(be, (size_t)d.n_slot * c_slot * 4, &cbuf);
+        if (st) return drop(st);
         MoeGemmDesc f = d;  // same slots' indices and experts; products gate and up over x
         f.K = (uint32_t)H;
         f.n_prob = 2;
@@ -194,27 +232,23 @@ int try_moe_gemm(cg_backend *be, cg_tensor *n, bool *done) {
         f.sb_index = wg->strides[0];
         f.prob[0].w = data_ptr(wg); f.prob[0].sbn = wg->strides[1]; f.prob[0].N = (uint32_t)F;
         f.prob[1].w = data_ptr(wu); f.prob[1].sbn = wu->strides[1]; f.prob[1].N = (uint32_t)F;
-        for (size_t sl = 0; sl < hbuf.size(); ++sl) {
+        for (size_t sl = 0; sl < slot_a.size(); ++sl) {
           f.slot[sl].a16 = planes ? (const uint16_t *)xplanes->ptr : (const uint16_t *)xsh->ptr + x->offset;
           f.slot[sl].a_bs = planes ? H : x->strides[0];
-          f.slot[sl].h16 = (uint16_t *)hbuf[sl]->ptr;
-          d.slot[sl].a16 = (const uint16_t *)hbuf[sl]->ptr;
+          f.slot[sl].h16 = (uint16_t *)hbuf->ptr + sl * h_slot;
+          d.slot[sl].a16 = f.slot[sl].h16;
           d.slot[sl].a_bs = F;
+          d.slot[sl].c[0] = (float *)cbuf->ptr + sl * c_slot;
         }
         d.pro = PRO_NONE;
         f.planes = d.planes = planes;
-        for (const Member &m : members) d.slot[m.slot].c[0] = (float *)m.c->st->ptr;
         hipError_t e = hipSuccess;
-        // the pairs sorted by expert once, for both launches: count, offset (one word per expert), list
-        Storage *route = nullptr;
+        // the pairs sorted by expert once, for both launches: count, offset (one word per expert), list, row tiles
         if (d.n_expert <= MOE_ROUTE_MAX_EXPERTS && H % 64 == 0 && F % 64 == 0) {
-          const size_t words = 2 * (size_t)d.n_expert + (size_t)S * d.n_slot + 1 + moe_route_max_tiles(d);
+          const size_t words = 2 * (size_t)d.n_expert + moe_route_list_words(d) + 1 + moe_route_max_tiles(d);
           st = dev_alloc(be, words * 4, &route);
-          if (st) {
-            drop_h();
-            return st;
-          }
-          uint32_t *rc = (uint32_t *)route->ptr, *ro = rc + d.n_expert, *rl = ro + d.n_expert, *rt = rl + (size_t)S * d.n_slot;
+          if (st) return drop(st);
+          uint32_t *rc = (uint32_t *)route->ptr, *ro = rc + d.n_expert, *rl = ro + d.n_expert, *rt = rl + moe_route_list_words(d);
           {
             KernelScope ks(be, "experts_route", (double)S * d.n_slot * 8 + (planes ? (double)S * H * 10 : 0), 0);
             MoeGemmDesc rd = f;
@@ -227,29 +261,76 @@ int try_moe_gemm(cg_backend *be, cg_tensor *n, bool *done) {
           f.route_offset = d.route_offset = ro;
           f.route_list = d.route_list = rl;
         }
+        // an expert of all tokens that waits for the same rows: in the same launches
+        DenseExpert de;
+        double dense_bytes[2] = {0, 0}, dense_flops[2] = {0, 0};
+        if (moe_ring_ok(f) && moe_ring_ok(d)) {
+          st = find_dense_expert(be, x, gelu, &de);
+          if (st) return drop(st);
+          if (de.down) {
+            const int64_t FS = de.wg->shape[2], HO = de.wd->shape[2];
+            st = dev_alloc(be, (size_t)S * FS * 2, &dense_h);
+            if (!st) st = dev_alloc(be, (size_t)S * HO * 4, &dense_c);
+            if (st) return drop(st);
+            f.dense.w[0] = data_ptr(de.wg);
+            f.dense.w[1] = data_ptr(de.wu);
+            f.dense.sbn = de.wg->strides[2];
+            f.dense.a16 = f.slot[0].a16;
+            f.dense.a_bs = f.slot[0].a_bs;
+            f.dense.h16 = (uint16_t *)dense_h->ptr;
+            f.dense.N = (uint32_t)FS;
+            f.dense.K = (uint32_t)H;
+            d.dense.w[0] = data_ptr(de.wd);
+            d.dense.sbn = de.wd->strides[2];
+            d.dense.a16 = f.dense.h16;
+            d.dense.a_bs = FS;
+            d.dense.c = (float *)dense_c->ptr;
+            d.dense.N = (uint32_t)HO;
+            d.dense.K = (uint32_t)FS;
+            if (moe_dense_ok(f) && moe_dense_ok(d)) {
+              dense_bytes[0] = 4.0 * FS * H + 2.0 * S * FS;
+              dense_bytes[1] = 2.0 * FS * HO + (double)S * (2 * FS + 4 * HO);
+              dense_flops[0] = 4.0 * S * FS * H;
+              dense_flops[1] = 2.0 * S * FS * HO;
+            } else {
+              f.dense.N = d.dense.N = 0;
+              de.down = nullptr;
+            }
+          }
+        }
         if (e == hipSuccess) {
-          KernelScope ks(be, "gemm_experts_bf16", 2.0 * d.n_expert * F * H * 2 + (double)S * H * 2 + (double)d.n_slot * S * F * 2,
-                         4.0 * d.n_slot * S * F * H);
+          KernelScope ks(be, "gemm_experts_bf16", 2.0 * d.n_expert * F * H * 2 + (double)S * H * 2 + (double)d.n_slot * S * F * 2 + dense_bytes[0],
+                         4.0 * d.n_slot * S * F * H + dense_flops[0]);
           if (be->trace_shapes) ks.rename("gemm_experts_bf16[gate*up]");
           e = launch_moe_gemm(be->lc(), f);
         }
         if (e == hipSuccess) {
           KernelScope ks(be, "gemm_experts_bf16",
-                         (double)d.n_expert * d.prob[0].N * F * 2 + (double)d.n_slot * S * (F * 2 + d.prob[0].N * 4),
-                         2.0 * d.n_slot * S * d.prob[0].N * F);
+                         (double)d.n_expert * N * F * 2 + (double)d.n_slot * S * (F * 2 + N * 4) + dense_bytes[1],
+                         2.0 * d.n_slot * S * N * F + dense_flops[1]);
           if (be->trace_shapes) ks.rename("gemm_experts_bf16[down]");
           e = launch_moe_gemm(be->lc(), d);
         }
-        drop_h();
-        storage_release(route);
-        if (e != hipSuccess) return fail(be, CG_ERR_DEVICE, hipGetErrorString(e));
+        if (e != hipSuccess) return drop(fail(be, CG_ERR_DEVICE, hipGetErrorString(e)));
+        auto take = [&](cg_tensor *c, Storage *st, int64_t offset) {
+          c->st = st;
+          st->rc.fetch_add(1);
+          c->stype = ST_F32;
+          c->offset = offset;
+          contiguous_strides(c->rank, c->shape, c->strides);
+          c->op = N_REAL;
+          drop_inputs(c);  // the products under it were never needed as tensors
+        };
         for (const Member &m : members) {
           forget_gemv_candidate(m.c);
-          m.c->op = N_REAL;
-          drop_inputs(m.c);  // the gate and up products under it were never needed as tensors
+          take(m.c, cbuf, m.slot * c_slot);
+        }
+        if (de.down) {
+          forget_gemm_candidate(de.down);
+          take(de.down, dense_c, 0);
         }
         *done = true;
-        return CG_OK;
+        return drop(CG_OK);
       }
     }
   }
