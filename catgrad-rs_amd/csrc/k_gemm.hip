@@ -608,8 +608,8 @@ __global__ void __launch_bounds__(WR *WC *KG * 64) gemm_bf16_dma_kernel(GemmDesc
   const uint32_t k_end = min(g.K, k_begin + g.k_per_split);
 
   const int n_steps = k_end > k_begin ? (int)((k_end - k_begin) / BK) : 0;
-  const KOrder order(BKM || (RING && TM == 3) ? 0u : g.k_rotate, place.tn + tiles_n * place.zz, (uint32_t)n_steps);
-  const uint32_t k_first_step = k_begin + order.first * BK;
+  KOrder order(BKM ? 0u : g.k_rotate, place.tn + tiles_n * place.zz, (uint32_t)n_steps, BKM || g.M <= 128 ? 0u : place.tm + place.tn);
+  const uint32_t k_first_step = k_begin + order.step() * BK;
 
   f32x16 acc[TM][TN];
 #pragma unroll
@@ -640,9 +640,8 @@ __global__ void __launch_bounds__(WR *WC *KG * 64) gemm_bf16_dma_kernel(GemmDesc
   }
   // (k-major B: a wave's loads are all A's or all B's, and B's step down 64 rows per stage)
   const int64_t gp_step = BKM && wave * LPW * 8 >= BM_ ? (int64_t)BK * g.sbk : (int64_t)BK;
-  uint32_t to_wrap = order.wrap;
   auto issue = [&](int buf) {
-    const int64_t to_next = BKM ? gp_step : --to_wrap ? (int64_t)BK : (int64_t)(int32_t)order.back / 2;
+    const int64_t to_next = BKM ? gp_step : (int64_t)order.advance() * BK;
 #pragma unroll
     for (int i = 0; i < LPW; ++i) {
       lds_dma16(gp[i], lds0 + buf * STAGE + piece(i) * 1024);
@@ -743,15 +742,14 @@ __global__ void __launch_bounds__(WR *WC *KG * 64) gemm_bf16_dma_kernel(GemmDesc
     const uint32_t la = lds0 + wave * PA * 1024, ab = (BM_ / 8 + wave * (PB - PA)) * 1024;
     const uint32_t first = la + (NS - 1) * STAGE, limit = la + NS * STAGE;
     const uint32_t n = __builtin_amdgcn_readfirstlane((uint32_t)n_steps);
-    // (steps to request before the order goes back; none to come, or gone back already: never)
-    const uint32_t wrap = __builtin_amdgcn_readfirstlane((int)to_wrap > 0 ? to_wrap : 0x7FFFFFFFu);
+    const uint32_t next = __builtin_amdgcn_readfirstlane(order.at), flip = __builtin_amdgcn_readfirstlane(order.flip);
 #define SR_ACC(i, j) [c##i##j] "+a"(acc[i][j])
 #define SR_A4 [ga0] "+v"(at[0]), [ga1] "+v"(at[1]), [ga2] "+v"(at[2]), [ga3] "+v"(at[3])
 #define SR_B4(o) [gb0] "+v"(at[o]), [gb1] "+v"(at[o + 1]), [gb2] "+v"(at[o + 2]), [gb3] "+v"(at[o + 3])
 #define SR_IN                                                                                                              \
   [ra0] "v"(ra[0]), [ra1] "v"(ra[1]), [ra2] "v"(ra[2]), [ra3] "v"(ra[3]), [rb0] "v"(rb[0]), [rb1] "v"(rb[1]),              \
       [rb2] "v"(rb[2]), [rb3] "v"(rb[3]), [first] "s"(first), [limit] "s"(limit), [la] "s"(la), [ab] "s"(ab), [n] "s"(n),  \
-      [wrap] "s"(wrap), [back] "s"(order.back), [stage] "i"(STAGE), [all] "i"(NS * STAGE), [held] "i"(NS - 1)
+      [next] "s"(next), [flip] "s"(flip), [stage] "i"(STAGE), [all] "i"(NS * STAGE), [held] "i"(NS - 1)
     if constexpr (TM == 2 && TN == 2) {
       static_assert(NS == 5 && !EPI, "");
       asm volatile(SR_LOOP_22 : SR_ACC(0, 0), SR_ACC(0, 1), SR_ACC(1, 0), SR_ACC(1, 1), SR_A4, SR_B4(4) : SR_IN : SR_CLOBBERS);
@@ -2568,10 +2566,11 @@ __global__ void __launch_bounds__(256) moe_gemm_dma_kernel(MoeGemmDesc g) {
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint16_t *)dma_smem;
   const int sw = (lane >> 1) & 7, half = lane >> 5;
   const int n_steps = (int)(K / BK);
-  const KOrder order(g.k_rotate, e * tiles_n + n0 / BN_, (uint32_t)n_steps);
+  const KOrder first_order(g.k_rotate, e * tiles_n + n0 / BN_, (uint32_t)n_steps);
   const int64_t plane = PLANES ? (int64_t)g.S * K : 0;
   for (uint32_t m0 = m_first; m0 < cnt; m0 += PAIRS) {
     const int live_tiles = (int)min((uint32_t)MT, (cnt - m0 + TPAIRS - 1) / TPAIRS);  // wave-uniform
+    KOrder order = first_order;
     f32x16 acc[NP][MT], run[PLANES ? NP : 1][PLANES ? MT : 1];  // run: the sum over the k-steps so far
 #pragma unroll
     for (int p = 0; p < NP; ++p)
@@ -2603,15 +2602,14 @@ __global__ void __launch_bounds__(256) moe_gemm_dma_kernel(MoeGemmDesc g) {
             rows = g.slot[s].a16;
             bs = g.slot[s].a_bs;
           }
-        gp[i] = rows + part * plane + (int64_t)tok * bs + order.first * BK + c * 8;
+        gp[i] = rows + part * plane + (int64_t)tok * bs + order.step() * BK + c * 8;
       } else {
         const int rb = R - BM_, p = rb / BN_, col = rb - p * BN_;
-        gp[i] = W[p < NP ? p : 0] + (int64_t)min(n0 + (uint32_t)col, N - 1) * sbn[p < NP ? p : 0] + order.first * BK + c * 8;
+        gp[i] = W[p < NP ? p : 0] + (int64_t)min(n0 + (uint32_t)col, N - 1) * sbn[p < NP ? p : 0] + order.step() * BK + c * 8;
       }
     }
-    uint32_t to_wrap = order.wrap;
     auto issue = [&](int buf) {
-      const int64_t to_next = --to_wrap ? (int64_t)BK : (int64_t)(int32_t)order.back / 2;
+      const int64_t to_next = (int64_t)order.advance() * BK;
 #pragma unroll
       for (int i = 0; i < LPW; ++i) {
         if (i >= MT) lds_dma16_stream(gp[i], lds0 + buf * STAGE + block_of(i) * 1024);

@@ -18,8 +18,7 @@
 //     phases, 3072 cycles, to arrive, and there is no point at which everything is waited for.
 //   * One barrier a phase: before it a wavefront has seen its own loads of the unit about to be read (a count) and the
 //     reads of two phases ago (a count); so behind it the unit is there for everyone, and its predecessor's place free.
-// On tiles of 256 rows the products of an element are added in the order of k, the same bits as gemm_bf16_dma_kernel's for products of
-// more than 128 rows; on tiles of 128, which up to 128 rows and the routed experts may be given with an order of their own, see KOrder.
+// On tiles of 256 rows the products of an element are added in the order of k; on tiles of 128 in an order of the tile's own (KOrder).
 // Tiles of 128 x 256, for the stacked gate / up of fewer rows, for one round of plain, grouped and rotating products, and for the routed
 // experts: see HPHASE0.
 // Measured against 256 x 256 tiles with eight wavefronts whose loads a compiler placed, on the same box: 16384 x 1152 by 2 x 6912
@@ -196,8 +195,9 @@ static hipError_t whole_lds(const void *kernel, int bytes) {
 // first B1 of this one; what they leave is requested again two phases later: A of step s + 3 in the first phase of s, B0 and B1
 // in the second.  Fragments of A are replaced behind the products that use them, a slice late.  Against eight wavefronts with three
 // stages: 400 rows by 2 x 5632, K = 2048, 31 -> 26.5 us, 512 by 2 x 6912, K = 1152, 21.3 -> 18; 512 by 2 x 8192, K = 2048, 38 to 40
-// either way - rows 4 KB apart: with the same weights at a pitch of 4224 bytes 38.6 and 35.7.  (Workgroups of different columns
-// starting at different k: no change.  Loads past the L1: no change.)
+// either way.  (Workgroups of different columns starting at different k: no change.  Loads past the L1: no change.  Four wavefronts that
+// only load beside four that only multiply: 41 us a launch of twelve in a row against 41.)  What bounds it in a row of such launches is
+// power: a step takes 1300 cycles, 1024 of them MFMAs, at 1.36 to 1.4 GHz; without the MFMAs 1360 at 2.1, without the loads 1210 at 1.9.
 #define HRD(U, B, r, ks) "ds_read_b128 " FR_##U##_##r##_##ks ", " B " offset:" #r "*4096\n\t"
 #define HFROM_A(S, ks) "v_add_u32 v126, " S ", %[ra" #ks "]\n\t"
 #define HFROM_B(S, ks) "v_add_u32 v127, " S ", %[rb" #ks "]\n\t"
@@ -212,10 +212,13 @@ static hipError_t whole_lds(const void *kernel, int bytes) {
 #define HSYNC(v) "s_waitcnt vmcnt(" #v ")\n\ts_barrier\n\t"
 #define HSLICE(b, UB, ks, W, E0, E1, E2, E3) \
   W PRODUCT(0, b, 0, 0, A0, UB, ks) E0 PRODUCT(0, b, 0, 1, A0, UB, ks) E1 PRODUCT(0, b, 1, 0, A0, UB, ks) E2 PRODUCT(0, b, 1, 1, A0, UB, ks) E3
-// s[58:59]: bytes from the step being requested to the next - behind a slice's last step back to its first (KOrder) -, s55 the steps
-// until then; the main loop finds the next size out among its products
-#define HSTEP_SIZE_AT(lo, hi) "s_sub_u32 s55, s55, 1\n\ts_cmp_eq_u32 s55, 0\n\ts_cselect_b32 " lo ", %[back], 128\n\ts_cselect_b32 " hi ", -1, 0\n\t"
-#define HSTEP_SIZE HSTEP_SIZE_AT("s58", "s59")
+// s[58:59]: bytes from the step being requested to the next (KOrder::advance; s55 is its place in the order); the main loop finds the
+// next size out among its products
+#define HSTEP_A "s_xor_b32 s40, s55, %[flip]\n\ts_add_u32 s55, s55, 1\n\t"
+#define HSTEP_B "s_cmp_eq_u32 s55, %[n]\n\ts_cselect_b32 s55, 0, s55\n\t"
+#define HSTEP_C "s_xor_b32 s41, s55, %[flip]\n\ts_sub_u32 s41, s41, s40\n\t"
+#define HSTEP_D(lo, hi) "s_lshl_b32 " lo ", s41, 7\n\ts_ashr_i32 " hi ", s41, 31\n\t"
+#define HSTEP_SIZE HSTEP_A HSTEP_B HSTEP_C HSTEP_D("s58", "s59")
 #define HPHASE0(G, v)                                                                                                              \
   G("s_add_u32 s54, s53, %[lds]\n\t") HSYNC(v)                                                                                     \
   HFROM_A("s48", 3) HFROM_B("s50", 0)                                                                                              \
@@ -226,9 +229,9 @@ static hipError_t whole_lds(const void *kernel, int bytes) {
 #define HPHASE1(G, v, HINT)                                                                                                              \
   G("s_add_u32 s54, s48, %[lds]\n\t") HSYNC(v)                                                                                     \
   HFROM_B("s52", 0)                                                                                                                \
-  HSLICE(1, B1, 0, READS_BUT(6), HB0(0, 0) G(HM0(0)), HB0(1, 0) G(LOAD_AS(B0, 0, HINT) HM0(1)), G(LOAD_AS(B0, 1, HINT)), G(HSTEP_SIZE_AT("s56", "s57"))) \
+  HSLICE(1, B1, 0, READS_BUT(6), HB0(0, 0) G(HM0(0)), HB0(1, 0) G(LOAD_AS(B0, 0, HINT) HM0(1)), G(LOAD_AS(B0, 1, HINT)), G(HSTEP_A HSTEP_B)) \
   HFROM_A("s51", 0) HFROM_B("s52", 1)                                                                                              \
-  HSLICE(1, B1, 1, READS_BUT(6), HB0(0, 1) G(HM0(2)), HB0(1, 1) G(LOAD_AS(B0, 2, HINT) HM0(3)), HA(0, 0) G(LOAD_AS(B0, 3, HINT)), HA(1, 0))      \
+  HSLICE(1, B1, 1, READS_BUT(6), HB0(0, 1) G(HM0(2)), HB0(1, 1) G(LOAD_AS(B0, 2, HINT) HM0(3)), HA(0, 0) G(LOAD_AS(B0, 3, HINT)), HA(1, 0) G(HSTEP_C HSTEP_D("s56", "s57")))      \
   HFROM_A("s51", 1) HFROM_B("s52", 2) G("s_add_u32 s54, s49, %[lds]\n\t")                                                          \
   HSLICE(1, B1, 2, READS_BUT(8), HB0(0, 2) G(HM0(0)), HB0(1, 2) G(LOAD_AS(B1, 0, HINT) HM0(1)), HA(0, 1) G(LOAD_AS(B1, 1, HINT)), HA(1, 1))      \
   HFROM_A("s51", 2) HFROM_B("s52", 3)                                                                                              \
@@ -244,7 +247,7 @@ static hipError_t whole_lds(const void *kernel, int bytes) {
   HM0(0) "s_nop 0\n\t" HLOAD_A(0) HM0(1) "s_nop 0\n\t" HLOAD_A(1) HM0(2) "s_nop 0\n\t" HLOAD_A(2) HM0(3) "s_nop 0\n\t" HLOAD_A(3)
 #define HLOADS_B(U, HINT) \
   HM0(0) "s_nop 0\n\t" LOAD_AS(U, 0, HINT) HM0(1) "s_nop 0\n\t" LOAD_AS(U, 1, HINT) HM0(2) "s_nop 0\n\t" LOAD_AS(U, 2, HINT) HM0(3) "s_nop 0\n\t" LOAD_AS(U, 3, HINT)
-#define HPOINTERS "s_mov_b64 s[42:43], %[pb0]\n\ts_mov_b64 s[44:45], %[pb1]\n\ts_mov_b32 s55, %[wrap]\n\t" HSTEP_SIZE
+#define HPOINTERS "s_mov_b64 s[42:43], %[pb0]\n\ts_mov_b64 s[44:45], %[pb1]\n\ts_mov_b32 s55, %[first]\n\t" HSTEP_SIZE
 #define HNEXT_B "s_add_u32 s42, s42, s58\n\ts_addc_u32 s43, s43, s59\n\ts_add_u32 s44, s44, s58\n\ts_addc_u32 s45, s45, s59\n\t"
 #define HNEXT_STEP HNEXT_B HSTEP_SIZE
 #define HSTEP_LOADS(HINT) \
@@ -594,8 +597,9 @@ __global__ void __launch_bounds__(256, 1) gemm_bf16_ring_kernel(GemmDesc g) {
   const uint32_t n_steps = __builtin_amdgcn_readfirstlane((k_end - k_begin) / 64);
   // Where this lane's piece of each load comes from: byte offsets from the tile's first row (rows past the end repeat the last
   // one), the 16-byte chunk swizzled so that the fragment reads are free of bank conflicts.
-  const KOrder order(AH == 1 ? g.k_rotate : 0u, place.tn + tiles_n * place.zz, n_steps);  // (tiles of 256 rows have more than 128)
-  const uint32_t k_first = k_begin + order.first * 64;
+  // (tiles of 256 rows: in the order of k)
+  const KOrder order(AH == 1 ? g.k_rotate : 0u, place.tn + tiles_n * place.zz, n_steps, AH == 1 && g.M > 128 ? place.tm + place.tn : 0u);
+  const uint32_t k_first = k_begin + order.step() * 64;
   const uint16_t *pa = (const uint16_t *)g.a + b0 * g.sa_b0 + b1 * g.sa_b1 + (int64_t)m0 * g.sam + k_first;
   const uint16_t *pb0 = B + (int64_t)n0 * g.sbn + k_first;
   const uint16_t *pb1 = GATED ? (const uint16_t *)g.dual_b + b0 * g.sb_b0 + b1 * g.sb_b1 + (int64_t)n0 * g.sbn + k_first : pb0;
@@ -627,7 +631,7 @@ __global__ void __launch_bounds__(256, 1) gemm_bf16_ring_kernel(GemmDesc g) {
 #define RING_IN                                                                                                            \
   [dA00] "v"(dA0[0]), [dA01] "v"(dA0[1]), [dA02] "v"(dA0[2]), [dA03] "v"(dA0[3]), [dA10] "v"(dA1[0]), [dA11] "v"(dA1[1]),  \
       [dA12] "v"(dA1[2]), [dA13] "v"(dA1[3]), [pa] "s"(sa0), RING_IN_B
-#define RING_ORDER [wrap] "s"(order.wrap), [back] "s"(order.back)
+#define RING_ORDER [first] "s"(order.at), [flip] "s"(order.flip), [n] "s"(n_steps)
 #define RING_GATHERED [ga0] "+v"(ga[0]), [ga1] "+v"(ga[1]), [ga2] "+v"(ga[2]), [ga3] "+v"(ga[3])
 #define RING_HALF_SCALARS "v126", "v127", "s48", "s49", "s50", "s51", "s52", "s53"
 #define RING_SCALARS "s54", "s55", "s56", "s57", "s58", "s59", "s40", "s41", "s42", "s43", "s44", "s45", "s46", "s47", "m0", "scc", "memory"
@@ -689,7 +693,7 @@ __global__ void __launch_bounds__(256, 1) gemm_bf16_ring_kernel(GemmDesc g) {
   else if constexpr (AH == 2)
     asm volatile(MAIN_LOOP : RING_ACC0, RING_ACC1, RING_PLACES : RING_IN, [n] "s"(n_steps) : RING_SCALARS, RING_FRAGMENTS);
   else
-    asm volatile(HMAIN_LOOP("") : RING_ACC0, RING_PLACES, RING_GATHERED : RING_IN_B, RING_ORDER, [n] "s"(n_steps) : RING_SCALARS, RING_HALF_SCALARS, RING_FRAGMENTS);
+    asm volatile(HMAIN_LOOP("") : RING_ACC0, RING_PLACES, RING_GATHERED : RING_IN_B, RING_ORDER : RING_SCALARS, RING_HALF_SCALARS, RING_FRAGMENTS);
   if (KIND == RING_PLAIN && g.clock_ticks && tid == 0) {
     atomicAdd(g.clock_ticks, __builtin_amdgcn_s_memtime() - tick0);
     atomicAdd(g.clock_ticks + 1, __builtin_amdgcn_s_memrealtime() - real0);
@@ -939,10 +943,10 @@ __global__ void __launch_bounds__(256, 1) moe_ring_kernel(MoeGemmDesc g) {
   }
   const uint32_t n_steps = __builtin_amdgcn_readfirstlane(K / 64);
   const int64_t sbn0 = dense ? g.dense.sbn : g.prob[prob].sbn, sbn1 = dense || !GATED ? sbn0 : g.prob[1].sbn;
-  const KOrder order(dense ? 0u : g.k_rotate, e * tiles_n + n0 / BNO, n_steps);
+  const KOrder order(dense ? 0u : g.k_rotate, e * tiles_n + n0 / BNO, n_steps, once ? 0u : m0 / 128 + n0 / BNO);
   const uint16_t *w0 = dense ? (const uint16_t *)g.dense.w[0] : (const uint16_t *)g.prob[prob].w + (int64_t)e * g.sb_index;
   const uint16_t *w1 = dense ? (const uint16_t *)g.dense.w[1] : (const uint16_t *)g.prob[1].w + (int64_t)e * g.sb_index;
-  const uint16_t *pb0 = w0 + (int64_t)n0 * sbn0 + order.first * 64, *pb1 = GATED ? w1 + (int64_t)n0 * sbn1 + order.first * 64 : pb0;
+  const uint16_t *pb0 = w0 + (int64_t)n0 * sbn0 + order.step() * 64, *pb1 = GATED ? w1 + (int64_t)n0 * sbn1 + order.step() * 64 : pb0;
   const uint32_t sb = (uint32_t)sbn0 * 2, sb1 = (uint32_t)sbn1 * 2, last_b = N - 1 - n0;
   const uint16_t *rows = dense ? g.dense.a16 : g.slot[0].a16;
   const int64_t row_pitch = dense ? g.dense.a_bs : g.slot[0].a_bs;
@@ -951,7 +955,7 @@ __global__ void __launch_bounds__(256, 1) moe_ring_kernel(MoeGemmDesc g) {
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const uint32_t r = (wave * 4 + i) * 8 + (lane >> 3), c = ((lane & 7) ^ ((r >> 1) & 7)) * 16;
-    ga[i] = (uint64_t)(rows + (ent[i] >> 16) * g.a_slot + (ent[i] & 0xFFFFu) * row_pitch) + order.first * 128 + c;
+    ga[i] = (uint64_t)(rows + (ent[i] >> 16) * g.a_slot + (ent[i] & 0xFFFFu) * row_pitch) + order.step() * 128 + c;
     dB0[i] = min(r, last_b) * sb + c;
     dB1[i] = GATED ? min(r, last_b) * sb1 + c : min(r + 128, last_b) * sb + c;
   }
@@ -984,9 +988,9 @@ __global__ void __launch_bounds__(256, 1) moe_ring_kernel(MoeGemmDesc g) {
     rb[ks] = wn * 8192 + p;
   }
   if (once)
-    asm volatile(HMAIN_LOOP(" nt") : RING_ACC0, RING_PLACES, RING_GATHERED : MOE_IN, RING_ORDER, [n] "s"(n_steps) : RING_SCALARS, RING_HALF_SCALARS, RING_FRAGMENTS);
+    asm volatile(HMAIN_LOOP(" nt") : RING_ACC0, RING_PLACES, RING_GATHERED : MOE_IN, RING_ORDER : RING_SCALARS, RING_HALF_SCALARS, RING_FRAGMENTS);
   else
-    asm volatile(HMAIN_LOOP("") : RING_ACC0, RING_PLACES, RING_GATHERED : MOE_IN, RING_ORDER, [n] "s"(n_steps) : RING_SCALARS, RING_HALF_SCALARS, RING_FRAGMENTS);
+    asm volatile(HMAIN_LOOP("") : RING_ACC0, RING_PLACES, RING_GATHERED : MOE_IN, RING_ORDER : RING_SCALARS, RING_HALF_SCALARS, RING_FRAGMENTS);
   // Rows back to their slot and token, through 4 KB of LDS of each wavefront's own: 32 rows of 64 bf16 or of 32 f32 values at a time, of
   // which eight lanes store a line.  A lane knows where the row of its number goes, and hands that to the eight.
   __syncthreads();  // every wavefront has read its last fragments
