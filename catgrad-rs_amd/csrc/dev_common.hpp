@@ -239,7 +239,10 @@ __device__ __forceinline__ float gelu_fast(float x) {
 // memory, 120 to 140 from its XCD's L2 (256 workgroups that only load tiles of 128 x 256 of 512 rows by 16384 of 2048 values: 39.4 us
 // with two stages and with three).  Tiles in step wait for memory with every load, since each piece is new to all of them; so, only with the
 // one step in four that they are the first to take: 30.3 us, 128 x 128 of 8192 30.7 -> 22.6, 128 x 64 of 3072 27 -> 18.6, 256 x 256 of 3072
-// rows 120 -> 92 (numbered by row tile alone 34.2, 26.1, 18.6 and 100; of eight steps 35.0, 27.2, 23.2 and 103).
+// rows 120 -> 92 (numbered by row tile alone 34.2, 26.1, 18.6 and 100; of eight steps 35.0, 27.2, 23.2 and 103).  For the routed experts of
+// several row tiles and the dense expert (1024 tokens 177 + 112 -> 173 + 104 us a layer).  Dense products do not gain: 512 x 2048 x 8192 on
+// 128 x 128 26.8 -> 25.5 us, but the kernels around it lose that (the clock), 512 x 2 x 8192 x 2048 on 128 x 256 36.0 -> 37.1, 2900 on
+// 256 x 256 168 -> 170, q / k / v of 37 rows 12.4 -> 12.7.
 struct KOrder {
   uint32_t at, flip, n;  // at: the next step to request, before the flip
   __device__ __forceinline__ KOrder(uint32_t rotate, uint32_t tile, uint32_t n_steps, uint32_t share = 0) {

@@ -608,7 +608,7 @@ __global__ void __launch_bounds__(WR *WC *KG * 64) gemm_bf16_dma_kernel(GemmDesc
   const uint32_t k_end = min(g.K, k_begin + g.k_per_split);
 
   const int n_steps = k_end > k_begin ? (int)((k_end - k_begin) / BK) : 0;
-  KOrder order(BKM ? 0u : g.k_rotate, place.tn + tiles_n * place.zz, (uint32_t)n_steps, BKM || g.M <= 128 ? 0u : place.tm + place.tn);
+  KOrder order(BKM || (RING && TM == 3) ? 0u : g.k_rotate, place.tn + tiles_n * place.zz, (uint32_t)n_steps);
   const uint32_t k_first_step = k_begin + order.step() * BK;
 
   f32x16 acc[TM][TN];
@@ -742,14 +742,14 @@ __global__ void __launch_bounds__(WR *WC *KG * 64) gemm_bf16_dma_kernel(GemmDesc
     const uint32_t la = lds0 + wave * PA * 1024, ab = (BM_ / 8 + wave * (PB - PA)) * 1024;
     const uint32_t first = la + (NS - 1) * STAGE, limit = la + NS * STAGE;
     const uint32_t n = __builtin_amdgcn_readfirstlane((uint32_t)n_steps);
-    const uint32_t next = __builtin_amdgcn_readfirstlane(order.at), flip = __builtin_amdgcn_readfirstlane(order.flip);
+    const uint32_t wrap = __builtin_amdgcn_readfirstlane(n - order.at), back = __builtin_amdgcn_readfirstlane(128u - n * 128u);  // steps to request before the order goes back, by so many bytes
 #define SR_ACC(i, j) [c##i##j] "+a"(acc[i][j])
 #define SR_A4 [ga0] "+v"(at[0]), [ga1] "+v"(at[1]), [ga2] "+v"(at[2]), [ga3] "+v"(at[3])
 #define SR_B4(o) [gb0] "+v"(at[o]), [gb1] "+v"(at[o + 1]), [gb2] "+v"(at[o + 2]), [gb3] "+v"(at[o + 3])
 #define SR_IN                                                                                                              \
   [ra0] "v"(ra[0]), [ra1] "v"(ra[1]), [ra2] "v"(ra[2]), [ra3] "v"(ra[3]), [rb0] "v"(rb[0]), [rb1] "v"(rb[1]),              \
       [rb2] "v"(rb[2]), [rb3] "v"(rb[3]), [first] "s"(first), [limit] "s"(limit), [la] "s"(la), [ab] "s"(ab), [n] "s"(n),  \
-      [next] "s"(next), [flip] "s"(flip), [stage] "i"(STAGE), [all] "i"(NS * STAGE), [held] "i"(NS - 1)
+      [wrap] "s"(wrap), [back] "s"(back), [stage] "i"(STAGE), [all] "i"(NS * STAGE), [held] "i"(NS - 1)
     if constexpr (TM == 2 && TN == 2) {
       static_assert(NS == 5 && !EPI, "");
       asm volatile(SR_LOOP_22 : SR_ACC(0, 0), SR_ACC(0, 1), SR_ACC(1, 0), SR_ACC(1, 1), SR_A4, SR_B4(4) : SR_IN : SR_CLOBBERS);

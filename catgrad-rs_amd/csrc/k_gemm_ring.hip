@@ -18,7 +18,9 @@
 //     phases, 3072 cycles, to arrive, and there is no point at which everything is waited for.
 //   * One barrier a phase: before it a wavefront has seen its own loads of the unit about to be read (a count) and the
 //     reads of two phases ago (a count); so behind it the unit is there for everyone, and its predecessor's place free.
-// On tiles of 256 rows the products of an element are added in the order of k; on tiles of 128 in an order of the tile's own (KOrder).
+// On tiles of 256 rows the products of an element are added in the order of k, the same bits as gemm_bf16_dma_kernel's for products of
+// more than 128 rows (but for its tiles of 128 x 128 and 192 x 128 with the scheduled loop); on tiles of 128, which up to 128 rows and the
+// routed experts may be given with an order of their own, see KOrder.
 // Tiles of 128 x 256, for the stacked gate / up of fewer rows, for one round of plain, grouped and rotating products, and for the routed
 // experts: see HPHASE0.
 // Measured against 256 x 256 tiles with eight wavefronts whose loads a compiler placed, on the same box: 16384 x 1152 by 2 x 6912
@@ -597,8 +599,7 @@ __global__ void __launch_bounds__(256, 1) gemm_bf16_ring_kernel(GemmDesc g) {
   const uint32_t n_steps = __builtin_amdgcn_readfirstlane((k_end - k_begin) / 64);
   // Where this lane's piece of each load comes from: byte offsets from the tile's first row (rows past the end repeat the last
   // one), the 16-byte chunk swizzled so that the fragment reads are free of bank conflicts.
-  // (tiles of 256 rows: in the order of k)
-  const KOrder order(AH == 1 ? g.k_rotate : 0u, place.tn + tiles_n * place.zz, n_steps, AH == 1 && g.M > 128 ? place.tm + place.tn : 0u);
+  const KOrder order(AH == 1 ? g.k_rotate : 0u, place.tn + tiles_n * place.zz, n_steps);  // (tiles of 256 rows have more than 128)
   const uint32_t k_first = k_begin + order.step() * 64;
   const uint16_t *pa = (const uint16_t *)g.a + b0 * g.sa_b0 + b1 * g.sa_b1 + (int64_t)m0 * g.sam + k_first;
   const uint16_t *pb0 = B + (int64_t)n0 * g.sbn + k_first;

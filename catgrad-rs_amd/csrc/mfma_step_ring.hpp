@@ -9,7 +9,7 @@
 // into the stage that step s - 1 has left.  One barrier a step, between slices 0 and 1: before it a wavefront has seen its own
 // loads of step s + 1 (a count of younger ones may be under way), behind it that stage is there for everyone.
 // Registers: fragments in v[144:223], addresses of a slice's reads in v142 / v143; s46 and s50 are this wavefront's places for
-// loads of A and B in the stage being requested, s47 counts steps, s48 is the stage being read.
+// loads of A and B in the stage being requested, s47 counts steps, s48 is the stage being read, s[44:45] a step's bytes.
 #pragma once
 
 #define SR_A_0_0 "v[144:147]"
@@ -44,11 +44,12 @@
 #define SR_LA(i) "global_load_lds_dwordx4 %[ga" #i "], off\n\tv_lshl_add_u64 %[ga" #i "], %[ga" #i "], 0, s[44:45]\n\t"
 #define SR_LB(i) "global_load_lds_dwordx4 %[gb" #i "], off\n\tv_lshl_add_u64 %[gb" #i "], %[gb" #i "], 0, s[44:45]\n\t"
 #define SR_NEXT_READ "s_add_u32 s48, s48, %[stage]\n\ts_cmp_eq_u32 s48, %[all]\n\ts_cselect_b32 s48, 0, s48\n\t"
-// s[44:45]: bytes from the step being requested to the next (KOrder::advance; s51 is its place in the order), found out in a step's first slice
-#define SR_STEP_A "s_xor_b32 s44, s51, %[flip]\n\ts_add_u32 s51, s51, 1\n\t"
-#define SR_STEP_B "s_cmp_eq_u32 s51, %[n]\n\ts_cselect_b32 s51, 0, s51\n\t"
-#define SR_STEP_C "s_xor_b32 s45, s51, %[flip]\n\ts_sub_u32 s44, s45, s44\n\t"
-#define SR_STEP_D "s_lshl_b32 s44, s44, 7\n\ts_ashr_i32 s45, s44, 31\n\t"
+// bytes from the step being requested to the next (KOrder; a product of up to 128 rows is on 128 x 128, so the others go straight on)
+#define SR_STEP_SIZE "s_sub_u32 s51, s51, 1\n\ts_cmp_eq_u32 s51, 0\n\ts_cselect_b32 s44, %[back], 128\n\ts_cselect_b32 s45, -1, 0\n\t"
+#define SR_STEP_22 SR_STEP_SIZE
+#define SR_STEP_32 ""
+#define SR_FIRST_STEP_22 "s_mov_b32 s51, %[wrap]\n\t" SR_STEP_SIZE
+#define SR_FIRST_STEP_32 "s_movk_i32 s44, 128\n\ts_mov_b32 s45, 0\n\t"
 #define SR_NEXT_LOAD                                                                                                     \
   "s_add_u32 s46, s46, %[stage]\n\ts_cmp_eq_u32 s46, %[limit]\n\ts_cselect_b32 s46, %[la], s46\n\ts_add_u32 s50, s46, " \
   "%[ab]\n\t"
@@ -57,8 +58,7 @@
 #define SR_ON(x) x
 #define SR_OFF(x) ""
 // 128 x 128 (four reads a slice, 4 + 4 loads a step) and 192 x 128 (five, 6 + 4).  D: loads on or off
-#define SR_HEAD_22 \
-  SR_W(8) SR_FROM(3) SR_S22(0, SR_RDA(0, 3) SR_STEP_A, SR_RDA(1, 3) SR_STEP_B, SR_RDB(0, 3) SR_STEP_C, SR_RDB(1, 3) SR_STEP_D) SR_NEXT_READ
+#define SR_HEAD_22 SR_W(8) SR_FROM(3) SR_S22(0, SR_RDA(0, 3), SR_RDA(1, 3), SR_RDB(0, 3), SR_RDB(1, 3)) SR_NEXT_READ
 #define SR_REST_22(D, v)                                                                                                       \
   SR_SYNC(v)                                                                                                                      \
   SR_W(8) SR_FROM(0) SR_S22(1, SR_RDA(0, 0) D(SR_MA(0)), SR_RDA(1, 0) D(SR_LA(0) SR_MA(1)), SR_RDB(0, 0) D(SR_LA(1) SR_MA(2)), \
@@ -72,7 +72,7 @@
   SR_FROM(0) SR_RDA(0, 0) SR_RDA(1, 0) SR_RDB(0, 0) SR_RDB(1, 0) SR_FROM(1) SR_RDA(0, 1) SR_RDA(1, 1) SR_RDB(0, 1) \
   SR_RDB(1, 1) SR_FROM(2) SR_RDA(0, 2) SR_RDA(1, 2) SR_RDB(0, 2) SR_RDB(1, 2)
 #define SR_HEAD_32 \
-  SR_W(10) SR_FROM(3) SR_S32(0, SR_RDA(0, 3) SR_STEP_A, SR_RDA(1, 3) SR_STEP_B, SR_RDA(2, 3) SR_STEP_C, SR_RDB(0, 3) SR_STEP_D, SR_RDB(1, 3), "") SR_NEXT_READ
+  SR_W(10) SR_FROM(3) SR_S32(0, SR_RDA(0, 3), SR_RDA(1, 3), SR_RDA(2, 3), SR_RDB(0, 3), SR_RDB(1, 3), "") SR_NEXT_READ
 #define SR_REST_32(D, v)                                                                                                         \
   SR_SYNC(v)                                                                                                                        \
   SR_W(10) SR_FROM(0) SR_S32(1, SR_RDA(0, 0) D(SR_MA(0)), SR_RDA(1, 0) D(SR_LA(0) SR_MA(1)), SR_RDA(2, 0) D(SR_LA(1) SR_MA(2)),  \
@@ -90,9 +90,9 @@
 // n >= NS - 1 steps, NS - 1 of them requested already: v0 counts the loads of NS - 2 steps, v those of NS - 3; TAIL: the NS - 2
 // steps before the last, which request nothing
 #define SR_LOOP(R, v0, v, TAIL)                                                                                             \
-  "s_mov_b32 s51, %[next]\n\ts_mov_b32 s46, %[first]\n\ts_add_u32 s50, s46, %[ab]\n\ts_mov_b32 s48, 0\n\t"    \
+  SR_FIRST_STEP_##R "s_mov_b32 s46, %[first]\n\ts_add_u32 s50, s46, %[ab]\n\ts_mov_b32 s48, 0\n\t"    \
   "s_sub_u32 s47, %[n], %[held]\n\t" SR_SYNC(v0) SR_FIRST_##R "s_cmp_eq_u32 s47, 0\n\ts_cbranch_scc1 2f\n\t"                   \
-  "1:\n\t" SR_HEAD_##R SR_REST_##R(SR_ON, v) SR_NEXT_LOAD                                                                \
+  "1:\n\t" SR_HEAD_##R SR_REST_##R(SR_ON, v) SR_NEXT_LOAD SR_STEP_##R                                                                \
   "s_sub_u32 s47, s47, 1\n\ts_cmp_lg_u32 s47, 0\n\ts_cbranch_scc1 1b\n\t"                                                      \
   "2:\n\t" TAIL SR_HEAD_##R SR_LAST_##R "s_nop 15\n\ts_nop 7\n\t"
 #define SR_QUIET(R, v) SR_HEAD_##R SR_REST_##R(SR_OFF, v)
