@@ -20,6 +20,7 @@
 #include <cstring>
 #include "launch.hpp"
 #include "dev_common.hpp"
+#include <type_traits>
 #include "mfma_step_ring.hpp"
 
 namespace cgk {
@@ -649,11 +650,14 @@ __global__ void __launch_bounds__(WR *WC *KG * 64) gemm_bf16_dma_kernel(GemmDesc
     }
   };
   const int sw = (lane >> 1) & 7, half = lane >> 5;
-  auto compute = [&](int buf) {
-    const uint16_t *As = dma_smem + buf * (STAGE / 2), *Bs = As + BM_ * BK;
+  constexpr int KS = BK / 16 / KG;  // k-slices of a step that this wave's group takes
+  const int k_first = KG > 1 ? kgrp * KS : 0;
+  auto compute = [&](int buf, auto steps) __attribute__((always_inline)) {  // `steps` stages from this one on
+    constexpr int SLICES = decltype(steps)::value * KS;
     bf16x8 af[2][TM], bfr[2][TN];
-    auto frags = [&](int ks, int set) {
-      const int p = ((ks * 2 + half) ^ sw) * 8;
+    auto frags = [&](int slice, int set) __attribute__((always_inline)) {
+      const uint16_t *As = dma_smem + (slice < KS ? buf : (buf + slice / KS) % NS) * (STAGE / 2), *Bs = As + BM_ * BK;
+      const int ks = k_first + slice % KS, p = ((ks * 2 + half) ^ sw) * 8;
 #pragma unroll
       for (int i = 0; i < TM; ++i)
         af[set][i] = *(const bf16x8 *)(&As[(wm * WM + i * 32 + (lane & 31)) * BK + p]);
@@ -677,14 +681,12 @@ __global__ void __launch_bounds__(WR *WC *KG * 64) gemm_bf16_dma_kernel(GemmDesc
         }
       }
     };
-    constexpr int KS = BK / 16 / KG;  // k-slices of this wave's group
-    const int k_first = KG > 1 ? kgrp * KS : 0;
-    frags(k_first, 0);
+    frags(0, 0);
     // the wave that is in its MFMA phase goes first when both waves of a SIMD have something to issue
     __builtin_amdgcn_s_setprio(1);
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-      if (ks + 1 < KS) frags(k_first + ks + 1, (ks + 1) & 1);
+    for (int ks = 0; ks < SLICES; ++ks) {
+      if (ks + 1 < SLICES) frags(ks + 1, (ks + 1) & 1);
 #pragma unroll
       for (int i = 0; i < TM; ++i)
 #pragma unroll
@@ -696,7 +698,7 @@ __global__ void __launch_bounds__(WR *WC *KG * 64) gemm_bf16_dma_kernel(GemmDesc
       // Issue order within the slice: one LDS read behind each of the first MFMAs, so that the reads of
       // the next slice go out while the matrix pipe is busy instead of in a block during which it drains
       // (measured on 4096^3: 0.93 -> 1.06 PFLOP/s).
-      if (ks + 1 < KS) {
+      if (ks + 1 < SLICES) {
         constexpr int READS = TM + TN < TM * TN ? TM + TN : TM * TN;
 #pragma unroll
         for (int q = 0; q < READS; ++q) {
@@ -716,8 +718,12 @@ __global__ void __launch_bounds__(WR *WC *KG * 64) gemm_bf16_dma_kernel(GemmDesc
     tick0 = __builtin_amdgcn_s_memtime();
     real0 = __builtin_amdgcn_s_memrealtime();
   }
+  // K-steps between two barriers.  A tile of a few rows does little in a step but wait for the barrier, for its first fragments and for its
+  // loads to be issued; two steps share the first and the fragments of the second come among the products of the first (37 rows, the
+  // split products of 2048 x 2048 and 2048 x 8192 8.75 -> 8.1 us on average; the whole prompt 1.175 -> 1.145 ms).
+  constexpr int SPB = NS == 8 ? 2 : 1;
 #pragma unroll
-  for (int s0 = 0; s0 < NS - 1; ++s0)
+  for (int s0 = 0; s0 < NS - SPB; ++s0)
     if (s0 < n_steps) issue(s0);
   if constexpr (RING) {
     // (the accumulators are cleared behind the first loads)
@@ -762,14 +768,22 @@ __global__ void __launch_bounds__(WR *WC *KG * 64) gemm_bf16_dma_kernel(GemmDesc
                    : SR_CLOBBERS);
     }
   } else {
-    for (int step = 0; step < n_steps; ++step) {
-      // stage `step` has landed (this wave's part): at most the NS - 2 younger stages are still in
+    int step = 0;
+    for (; step + SPB <= n_steps; step += SPB) {
+      // stages `step` .. have landed (this wave's part): at most the NS - 2 SPB younger ones are still in
       // flight; in the tail, where fewer were issued, wait for everything
-      if (step + NS - 1 <= n_steps) wait_vmcnt<(NS - 2) * LPW>();
+      if (step + NS - SPB <= n_steps) wait_vmcnt<(NS - 2 * SPB) * LPW>();
       else wait_vmcnt<0>();
-      __syncthreads();   // ... and everyone's; all waves are done reading the buffer refilled next
-      if (step + NS - 1 < n_steps) issue((step + NS - 1) % NS);
-      compute(step % NS);
+      __syncthreads();   // ... and everyone's; all waves are done reading the buffers refilled next
+#pragma unroll
+      for (int s = 0; s < SPB; ++s)
+        if (step + NS - SPB + s < n_steps) issue((step + NS - SPB + s) % NS);
+      compute(step % NS, std::integral_constant<int, SPB>());
+    }
+    if (SPB == 2 && step < n_steps) {
+      wait_vmcnt<0>();
+      __syncthreads();
+      compute(step % NS, std::integral_constant<int, 1>());
     }
   }
   if (g.clock_ticks && tid == 0) {
