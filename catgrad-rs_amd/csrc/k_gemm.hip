@@ -3149,6 +3149,13 @@ static bool rope_on_half_tiles(const LaunchCtx &lc, const GemmDesc &g) {
   return m128 * ((g.N + 127) / 128) > cus && m128 * ((g.N + 255) / 256) <= cus;
 }
 
+// ... or of 192 x 256 in the place of 256 x 256, at 0.8 of a round's time and more (3072 columns of heads of 64, K = 2048, one round either
+// way: 2700 rows 59.7 -> 50.1 us, 2900 58.6 -> 49.9, 3500 61.5 -> 53.8, 4000 63.3 -> 56.4).
+static bool rope_on_192_tiles(const LaunchCtx &lc, const GemmDesc &g) {
+  const uint64_t cus = (uint64_t)lc.n_cus, n256 = (g.N + 255) / 256, t256 = (g.M + 255) / 256 * n256, t192 = (g.M + 191) / 192 * n256;
+  return gemm_ring_192_ok(g) && (t192 + cus - 1) / cus * 4 < (t256 + cus - 1) / cus * 5;
+}
+
 bool gemm_rope_epilogue_ok(const LaunchCtx &lc, const GemmDesc &g) {
   if (!g.rope_s || !g.n_group || !gemm_epilogue_ok(g)) return false;
   if (g.rope_hd != 64 && g.rope_hd != 128 && g.rope_hd != 256) return false;
@@ -3394,9 +3401,9 @@ hipError_t launch_matmul(const LaunchCtx &lc_in, const GemmDesc &g, const char *
         return splits == 1 && g.K >= 256 && g.N % 4 == 0 && !g.n_group && !g.act_sigmoid && rounds_of(wide) * 9 < rounds_of(tiles) * 8;
       };
       if (g.rope_s && rope_on_large_tiles(lc, g)) {
-        e = launch_gemm_ring(lc, gg);
+        e = launch_gemm_ring(lc, gg, rope_on_192_tiles(lc, g) ? RING_192 : RING_256);
       } else if (g.rope_s && rope_on_half_tiles(lc, g)) {
-        e = launch_gemm_ring(lc, gg, true);
+        e = launch_gemm_ring(lc, gg, RING_128);
       } else if (g.rope_s && g.M <= 128) {
         // q / k / v of a few rows: a workgroup takes in its rows of both operands at about 42 GB/s however wide its tile is,
         // and 64 x 64 or 128 x 64 tiles are 48 workgroups for 3072 columns.  32 x 32 tiles, of columns that rotate into
@@ -3431,12 +3438,16 @@ hipError_t launch_matmul(const LaunchCtx &lc_in, const GemmDesc &g, const char *
         // Tiles of 256 rows or of 128, by the rounds they take: a round of the large ones costs 1.4 to 1.7 rounds of the small (512 rows
         // by 2 x 8192, K = 2048, one round either way 56 and 40 us; 700 rows, one round or two, 50 and 60; 1024 rows by 2 x 5632 47 and
         // 60; 1500 rows, two or three, 92 and 84; 2900 by 2 x 8192, three or six, 159 and 181).  Fewer tiles of 128 than half the
-        // CUs: 64 or 32 output columns per tile.
+        // CUs: 64 or 32 output columns per tile.  A round of 192 rows is 0.8 to 0.92 of one of 256 (2 x 8192, K = 2048: 700 rows, one round
+        // either way, 49.0 and 44.6 us; 2100, three either way, 149 and 124; 2300 149 and 133) and 1.25 to 1.4 of one of 128 (1100, two or
+        // three, 89.3 and 78.5; 1459 98.8 and 88.3).
         const uint64_t d256w = (uint64_t)((g.M + 255) / 256) * ((g.N + 143) / 144) * batch;
         const uint64_t cus = (uint64_t)lc.n_cus, r256 = (d256 + cus - 1) / cus, r128 = (d128 + cus - 1) / cus;
         const bool wide = wide_ahead(144, d256);
         const uint64_t large = wide ? (d256w + cus - 1) / cus * 9 : r256 * 8;  // (in eighths of a round of 256 rows)
-        if (large * 5 <= r128 * 24 && gemm_ring_ok(gg)) e = launch_gemm_ring(lc, gg, false, wide);
+        const uint64_t r192 = ((uint64_t)((g.M + 191) / 192) * ((g.N + 127) / 128) * batch + cus - 1) / cus;
+        if (r192 * 32 < std::min(large * 5, r128 * 24) && g.K >= 192 && gemm_ring_192_ok(gg)) e = launch_gemm_ring(lc, gg, RING_192);
+        else if (large * 5 <= r128 * 24 && gemm_ring_ok(gg)) e = launch_gemm_ring(lc, gg, wide ? RING_288 : RING_256);
         else if (d128 * 4 <= cus)
           e = launch_gemm_dma<128, 64, 4, 1, true, 5, true, false, false, 2>(lc, gg, (uint32_t)((uint64_t)((g.M + 127) / 128) * ((g.N + 31) / 32) * batch));
         // One or two k-steps: what a tile stores is most of it, and eight wavefronts store it as they come.  One step, on tiles of 64
@@ -3446,7 +3457,7 @@ hipError_t launch_matmul(const LaunchCtx &lc_in, const GemmDesc &g, const char *
         else if (g.K < 192 && d128 * 2 > cus) e = launch_gemm_dma<128, 256, 2, 4, true, 3, true>(lc, gg, (uint32_t)d128);
         else if (d128 * 2 <= cus || !gemm_ring_ok(gg))
           e = launch_gemm_dma<128, 128, 4, 2, true, 4, true>(lc, gg, (uint32_t)((uint64_t)((g.M + 127) / 128) * ((g.N + 63) / 64) * batch));
-        else e = launch_gemm_ring(lc, gg, true);
+        else e = launch_gemm_ring(lc, gg, RING_128);
       } else if (g.glu_gate || g.c16 || (g.act_sigmoid && splits == 1)) {
         if (g.act_sigmoid && t256 >= (uint64_t)lc.n_cus && gemm_ring_ok(gg)) e = launch_gemm_ring(lc, gg);
         else if (g.act_sigmoid && t256 >= (uint64_t)lc.n_cus) e = launch_gemm_dma<256, 256, 2, 4, true, 2>(lc, gg, (uint32_t)t256);
@@ -3479,7 +3490,7 @@ hipError_t launch_matmul(const LaunchCtx &lc_in, const GemmDesc &g, const char *
           if (e != hipSuccess) return e;
           return launch_matmul(second, rest, nullptr);
         }
-        if (wide) e = launch_gemm_ring(lc, gg, false, true);
+        if (wide) e = launch_gemm_ring(lc, gg, RING_288);
         else if (!g.n_group && fill(t128, 2 * (uint64_t)lc.n_cus) > 1.15 * fill(t256, (uint64_t)lc.n_cus))
           e = g.K < 2048 ? launch_gemm_plain<128, 128, 2, 4>(lc, gg, t128)  // (as below)
                          : launch_gemm_plain<128, 128, 2, 2>(lc, gg, t128);
@@ -3549,7 +3560,7 @@ hipError_t launch_matmul(const LaunchCtx &lc_in, const GemmDesc &g, const char *
           // A round of 128 x 256 where 128 x 128 are two to a CU and 192 rows more than a round (us there and here: 3100 x 2048, K = 512 14.5,
           // 14.2, 768 17.4, 17.6, 1024 20.7, 20.0, 2048 35.1, 30.4, 8192 117, 98; 4000 rows 15.7, 15.9; 19.4, 19.3; 23.0, 22.0; 39, 34; 128, 108;
           // 1000 x 6144 x 2048 39.3, 31.2; 2300 x 3000 x 2048 39.5, 32.4, x 512 14.5, 15.5; 6400 x 1152 x 6912 111, 96.8).
-          e = launch_gemm_ring(lc, gg, true);
+          e = launch_gemm_ring(lc, gg, RING_128);
         } else if (steps >= 64) {
           // Several rounds of a deep product, a round of 192 rows at 1.42 times one of 128: 8192 x 1152 x 6912 two or three, 134 and 148 us
           // (two to a CU 167); 4000 x 2048 x 8192 two either way, 149 and 130 (145); 3100 rows 144 and 117 (122).

@@ -21,6 +21,7 @@
 // On tiles of 256 rows the products of an element are added in the order of k, the same bits as gemm_bf16_dma_kernel's for products of
 // more than 128 rows (but for its tiles of 128 x 128 and 192 x 128 with the scheduled loop); on tiles of 128, which up to 128 rows and the
 // routed experts may be given with an order of their own, see KOrder.
+// Tiles of 192 x 256, for gate / up and rotating products: see SPHASE1.
 // Tiles of 128 x 256, for the stacked gate / up of fewer rows, for one round of plain, grouped and rotating products, and for the routed
 // experts: see HPHASE0.
 // Measured against 256 x 256 tiles with eight wavefronts whose loads a compiler placed, on the same box: 16384 x 1152 by 2 x 6912
@@ -190,6 +191,53 @@ static hipError_t whole_lds(const void *kernel, int bytes) {
   "s_sub_u32 s47, s47, 1\n\ts_cmp_lg_u32 s47, 0\n\ts_cbranch_scc1 1b\n\t"                                                \
   "2:\n\t" PHASE0(OFF, 20) PHASE1(OFF, 16) PHASE2(OFF, 12) PHASE3(OFF, 8) PHASE0(OFF, 4)             \
   PHASE1(OFF, 0) LAST_HALF "s_nop 15\n\ts_nop 7\n\t"
+
+// ---- tiles of 192 x 256: half of A1 (its unit is 64 rows, 32 of each wavefront's row half, eight KB in two pieces 8192 bytes apart, as
+// the fragments of 256 rows lie), so the phases (1,1) and (1,0) have eight products, A1 four reads a step and two loads.  For rows
+// that 256 to a tile put in as many rounds: gate and up of 2100 rows by 2 x 8192, K = 2048, 149 -> 124 us, q / k / v of 2900 58.6 -> 49.9.
+#define SM0_A1(i) "s_add_u32 m0, s48, 49152+" #i "*1024\n\t"
+#define SSLICE(b, UB, ks, W, R1, M0, R2, L) W PRODUCT(1, b, 0, 0, A1, UB, ks) R1 M0 PRODUCT(1, b, 0, 1, A1, UB, ks) R2 L
+#define SSYNC(v, r) "s_waitcnt vmcnt(" #v ") lgkmcnt(" #r ")\n\ts_barrier\n\t"
+#define ON_S(x) x
+#define OFF_S(x) ""
+#define SPHASE1(G, v)                                                                                    \
+  SSYNC(v, 8)                                                                                            \
+  SLICE(0, 1, A0, B1, 0, READS_BUT(6), RD(A1, 0, 0), G##_M(B0, 0), NONE, G##_L(B0, 0))                   \
+  SLICE(0, 1, A0, B1, 1, READS_BUT(5), RD(A1, 0, 1), G##_M(B0, 1), NONE, G##_L(B0, 1))                   \
+  SLICE(0, 1, A0, B1, 2, READS_BUT(4), RD(A1, 0, 2), G##_M(B0, 2), OTHER_STAGE_B, G##_L(B0, 2))          \
+  SLICE(0, 1, A0, B1, 3, READS_BUT(3), RD(A1, 0, 3), G##_M(B0, 3), OTHER_STAGE_A, G##_L(B0, 3))
+#define SPHASE2(G, v)                                                                                    \
+  SSYNC(v, 4)                                                                                            \
+  SSLICE(1, B1, 0, READS_BUT(3), RD(A0, 0, 0), G##_M(B1, 0), RD(A0, 1, 0), G##_L(B1, 0))                 \
+  SSLICE(1, B1, 1, READS_BUT(4), RD(A0, 0, 1), G##_M(B1, 1), RD(A0, 1, 1), G##_L(B1, 1))                 \
+  SSLICE(1, B1, 2, READS_BUT(5), RD(A0, 0, 2), G##_M(B1, 2), RD(A0, 1, 2), G##_L(B1, 2))                 \
+  SSLICE(1, B1, 3, READS_BUT(6), RD(A0, 0, 3), G##_M(B1, 3), RD(A0, 1, 3), G##_L(B1, 3))
+#define SPHASE3(G, v)                                                                                    \
+  SSYNC(v, 8)                                                                                            \
+  SSLICE(0, B0, 0, NONE, NONE, G##_S(SM0_A1(0)), NONE, G##_L(A1, 0))                                     \
+  SSLICE(0, B0, 1, NONE, RD(B0, 0, 0), G##_S(SM0_A1(1)), RD(B0, 1, 0), G##_L(A1, 1))                     \
+  SSLICE(0, B0, 2, NONE, RD(B0, 0, 1), NONE, RD(B0, 1, 1), NONE)                                         \
+  SSLICE(0, B0, 3, NONE, RD(B0, 0, 2), NONE, RD(B0, 1, 2), NONE) RD(B0, 0, 3) RD(B0, 1, 3)
+#define SLAST_HALF                                                                                       \
+  SSLICE(1, B1, 0, READS_BUT(3), NONE, NONE, NONE, NONE) SSLICE(1, B1, 1, READS_BUT(2), NONE, NONE, NONE, NONE) \
+  SSLICE(1, B1, 2, READS_BUT(1), NONE, NONE, NONE, NONE) SSLICE(1, B1, 3, READS_BUT(0), NONE, NONE, NONE, NONE) \
+  SSLICE(0, B0, 0, NONE, NONE, NONE, NONE, NONE) SSLICE(0, B0, 1, NONE, NONE, NONE, NONE, NONE)          \
+  SSLICE(0, B0, 2, NONE, NONE, NONE, NONE, NONE) SSLICE(0, B0, 3, NONE, NONE, NONE, NONE, NONE)
+#define SPOINTERS POINTERS "s_mov_b32 s48, %[lds1]\n\t"
+#define SOTHER_STAGE_LOADS OTHER_STAGE_LOADS "s_xor_b32 s48, s48, 0x10000\n\t"
+#define SSTEP_LOADS \
+  LOAD_UNIT(A0) LOAD_UNIT(B0) LOAD_UNIT(B1) SM0_A1(0) "s_nop 0\n\t" LOAD(A1, 0) SM0_A1(1) "s_nop 0\n\t" LOAD(A1, 1)
+// steps 0 and 1 requested: 28 loads
+#define SFIRST_LOADS SPOINTERS SSTEP_LOADS NEXT_STEP SOTHER_STAGE_LOADS SSTEP_LOADS
+// n >= 2 steps
+#define SMAIN_LOOP                                                                                                   \
+  SPOINTERS NEXT_STEP NEXT_STEP "s_sub_u32 s47, %[n], 2\n\t"                                                        \
+  "s_waitcnt vmcnt(20)\n\ts_barrier\n\t" RD_UNIT(A0) RD_UNIT(B0)                                                  \
+  "s_cmp_eq_u32 s47, 0\n\ts_cbranch_scc1 2f\n\t"                                                                  \
+  "1:\n\t" PHASE0(ON, 16) SPHASE1(ON, 18) SPHASE2(ON, 18) SPHASE3(ON, 18) NEXT_STEP SOTHER_STAGE_LOADS            \
+  "s_sub_u32 s47, s47, 1\n\ts_cmp_lg_u32 s47, 0\n\ts_cbranch_scc1 1b\n\t"                                        \
+  "2:\n\t" PHASE0(OFF, 16) SPHASE1(OFF, 14) SPHASE2(OFF, 10) SPHASE3(OFF, 6) PHASE0(OFF, 2)                        \
+  SPHASE1(OFF, 0) SLAST_HALF "s_nop 15\n\ts_nop 7\n\t"
 
 // ---- tiles of 128 x 256: one unit of A, so a step is three units, two phases - (A, B0), (A, B1) - of 16 MFMAs.  LDS holds ten
 // units, in the order A, B0, B1 of every step; the place of the unit 3 s + u is (3 s + u) % 10 (s48 A, s49 B0, s50 B1 of this
@@ -368,7 +416,8 @@ struct RingRope {  // one group's part of a GemmDesc
   uint32_t M, N, S;
 };
 __device__ __forceinline__ uint32_t ring_place(uint32_t r, uint32_t chunk) { return r * 64 + ((chunk ^ (r & 15)) << 2); }
-template <bool BIAS, bool SQUARES>
+// (IB: blocks of 32 rows that a wavefront has of the half tile, two, or one of 192 rows' second)
+template <bool BIAS, bool SQUARES, int IB>
 __device__ __forceinline__ void ring_half_to_lds(const f32x16 (&acc)[2][2][2], const float *bias, float *mine, float *sums) {
   const uint32_t lane = threadIdx.x & 63, half = lane >> 5;
   float ss[2] = {0.f, 0.f};
@@ -381,7 +430,7 @@ __device__ __forceinline__ void ring_half_to_lds(const f32x16 (&acc)[2][2][2], c
         float4 w;
         if (BIAS) __builtin_memcpy(&w, bias + b * 128 + j * 32 + q * 8 + half * 4, 16);
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {
+        for (int i = 0; i < IB; ++i) {
           const f32x16 &x = acc[b][i][j];
           float4 v = make_float4(x[q * 4], x[q * 4 + 1], x[q * 4 + 2], x[q * 4 + 3]);
           if (BIAS) { v.x += w.x; v.y += w.y; v.z += w.z; v.w += w.w; }
@@ -391,7 +440,7 @@ __device__ __forceinline__ void ring_half_to_lds(const f32x16 (&acc)[2][2][2], c
       }
   if (SQUARES) {
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
+    for (int i = 0; i < IB; ++i) {
       ss[i] += __shfl_xor(ss[i], 32, 64);
       if (!half) sums[i * 32 + lane] = ss[i];
     }
@@ -402,15 +451,15 @@ __device__ __forceinline__ void ring_half_to_lds(const f32x16 (&acc)[2][2][2], c
 // takes a piece of the lower half of a head and its partner of the upper - in the same rows (heads of 64), from the neighbouring
 // wavefront (128: each does half of the 64 rows), from the other column half (256) - and stores both.  Table rows serve both column halves
 // (not heads of 256), and are on their way a group of pieces ahead: the first group's (`t`) while the tile goes to LDS.
-template <int HD>
+template <int HD, int IB>
 struct RingPieces {
   static constexpr uint32_t H = HD / 2, PER = HD == 64 ? 8 : 16, RPU = 64 / PER;  // pieces to half a row, rows to a unit
-  static constexpr int UNITS = HD == 256 ? 16 : 8, GROUP = 4, BS = HD == 256 ? 1 : 2;  // units of a half tile, of a group; pairs to a unit
+  static constexpr int UNITS = (HD == 256 ? 8 : 4) * IB, GROUP = 4, BS = HD == 256 ? 1 : 2;  // units of a half tile, of a group; pairs to a unit
   uint32_t row0, sq0, pos0;  // this wavefront's first row, its sequence and position
   uint32_t chunk, row_in, in_half;  // the piece of its row, the row of the first unit, the piece's column of the lower half of its head
   float4 t[GROUP][4];  // cos and sin of the lower half, of the upper
   __device__ __forceinline__ RingPieces(uint32_t first_row, uint32_t S, uint32_t wn, uint32_t lane)
-      : row0(first_row), sq0(first_row / S), pos0(first_row - first_row / S * S), chunk(lane % PER), row_in(lane / PER + (HD == 128 ? wn * 32 : 0)),
+      : row0(first_row), sq0(first_row / S), pos0(first_row - first_row / S * S), chunk(lane % PER), row_in(lane / PER + (HD == 128 ? wn * IB * 16 : 0)),
         in_half((HD == 256 ? wn * 64 : 0) + lane % PER * 4) {}
   __device__ __forceinline__ void tables(const RingRope &d, int u0) {
 #pragma unroll
@@ -426,9 +475,9 @@ struct RingPieces {
     }
   }
 };
-template <int HD, bool NORM>
-__device__ __forceinline__ void ring_store_rotated(const RingRope &d, RingPieces<HD> &p, uint32_t n0, float *smem, uint32_t wave, uint32_t lane) {
-  typedef RingPieces<HD> P;
+template <int HD, bool NORM, int IB>
+__device__ __forceinline__ void ring_store_rotated(const RingRope &d, RingPieces<HD, IB> &p, uint32_t n0, float *smem, uint32_t wave, uint32_t lane) {
+  typedef RingPieces<HD, IB> P;
   const uint32_t wn = wave & 1, S = d.S, heads = d.N / HD;
   const float *mine = smem + wave * 8192;
   float *sums = smem + 32768 + wave * 128;  // NORM: the sums of squares, then each row's divisor and its inverse
@@ -493,6 +542,7 @@ __device__ __forceinline__ void ring_store_rotated(const RingRope &d, RingPieces
 }
 
 // Values: as they are, and as bf16 [sequence][column][position], rows of positions padded with zeros to a multiple of eight.
+template <int IB>
 __device__ __forceinline__ void ring_store_values(const RingRope &d, uint32_t row0, uint32_t n0, const float *mine, uint32_t wn, uint32_t lane) {
   const uint32_t S = d.S, Sp = (S + 7) & ~7u, sq0 = row0 / S, pos0 = row0 - sq0 * S;
   const uint32_t r0 = (lane >> 2) * 4, row = row0 + r0, over = pos0 + r0 >= S ? 1 : 0, sq = sq0 + over, pos = pos0 + r0 - over * S;
@@ -501,11 +551,12 @@ __device__ __forceinline__ void ring_store_values(const RingRope &d, uint32_t ro
     const uint32_t col0 = n0 + b * 128 + wn * 64;  // (whole tiles: every column exists)
     const float *tile = mine + b * 4096;
 #pragma unroll 4
-    for (uint32_t it = 0; it < 16; ++it) {
+    for (uint32_t it = 0; it < 8 * IB; ++it) {
       const uint32_t r = it * 4 + (lane >> 4);
       if (row0 + r < d.M) *(float4 *)(d.c + (uint64_t)(row0 + r) * d.N + col0 + (lane & 15) * 4) = *(const float4 *)(tile + ring_place(r, lane & 15));
     }
     // four positions of four columns to a lane
+    if (IB == 1 && lane >= 32) continue;
 #pragma unroll 1
     for (uint32_t it = 0; it < 4; ++it) {
       const uint32_t chunk = it * 4 + (lane & 3);
@@ -542,28 +593,28 @@ __device__ __forceinline__ void ring_store_values(const RingRope &d, uint32_t ro
 }
 
 // (one place that reads the accumulators: where two branches do, the compiler spills them)
-template <int HD, bool BIAS, bool NORM, int AH>
+template <int HD, bool BIAS, bool NORM, int AH, bool SHORT>
 __device__ __forceinline__ void ring_store_attention(const RingRope d, bool values, uint32_t m0, uint32_t n0, const f32x16 (&acc)[AH][2][2][2], float *smem) {
   const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wm = wave >> 1, wn = wave & 1;
   float *mine = smem + wave * 8192;
   auto half_tile = [&](auto A) __attribute__((always_inline)) {
-    constexpr int a = A;
-    const uint32_t row0 = m0 + a * 128 + wm * 64;
-    RingPieces<HD> p(row0, d.S, wn, lane);
+    constexpr int a = A, IB = SHORT && a ? 1 : 2;
+    const uint32_t row0 = m0 + a * 128 + wm * IB * 32;
+    RingPieces<HD, IB> p(row0, d.S, wn, lane);
     if (!values) p.tables(d, 0);
     if (a) __syncthreads();  // the other half has been read
-    ring_half_to_lds<BIAS, NORM>(acc[a], d.bias + n0 + wn * 64, mine, smem + 32768 + wave * 128);
+    ring_half_to_lds<BIAS, NORM, IB>(acc[a], d.bias + n0 + wn * 64, mine, smem + 32768 + wave * 128);
     __syncthreads();
-    if (values) ring_store_values(d, row0, n0, mine, wn, lane);
-    else ring_store_rotated<HD, NORM>(d, p, n0, smem, wave, lane);
+    if (values) ring_store_values<IB>(d, row0, n0, mine, wn, lane);
+    else ring_store_rotated<HD, NORM, IB>(d, p, n0, smem, wave, lane);
   };
   half_tile(std::integral_constant<int, 0>());
   if constexpr (AH == 2) half_tile(std::integral_constant<int, 1>());
 }
 
 // AH: halves of 128 rows to a tile, two or (not RING_SIGMOID) one.  WIDE: with the strip of 32 columns (RING_SILU, RING_GELU: 16
-// rows of each matrix), N % 4 == 0.
-template <int KIND, int AH, bool WIDE = false>
+// rows of each matrix), N % 4 == 0.  SHORT: 192 rows, the second half is 64.
+template <int KIND, int AH, bool WIDE = false, bool SHORT = false>
 __global__ void __launch_bounds__(256, 1) gemm_bf16_ring_kernel(GemmDesc g) {
   constexpr bool GATED = KIND == RING_SILU || KIND == RING_GELU;
   constexpr bool ROPE = KIND >= RING_ROPE_64;
@@ -572,7 +623,8 @@ __global__ void __launch_bounds__(256, 1) gemm_bf16_ring_kernel(GemmDesc g) {
   warm_kernel_arguments<sizeof(GemmDesc)>();
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), wm = wave >> 1, wn = wave & 1;
-  constexpr uint32_t BM = AH * 128;
+  constexpr uint32_t BM = SHORT ? 192 : AH * 128;
+  static_assert(!SHORT || (AH == 2 && !WIDE && (GATED || (ROPE && KIND < RING_ROPE_256))), "the epilogues of 192-row tiles");
   static_assert(AH == 2 || KIND != RING_SIGMOID, "the epilogues of 128-row tiles");
   const uint32_t tiles_m = (g.M + BM - 1) / BM, tiles_n = (g.N + BNO - 1) / BNO;
   const TilePlace place(tiles_m, tiles_n, g.nb0, g.nb1, max(g.splits, 1u));
@@ -610,7 +662,7 @@ __global__ void __launch_bounds__(256, 1) gemm_bf16_ring_kernel(GemmDesc g) {
   for (int i = 0; i < 4; ++i) {
     const uint32_t r = (wave * 4 + i) * 8 + (lane >> 3), c = ((lane & 7) ^ ((r >> 1) & 7)) * 16;
     dA0[i] = min(r, last_a) * sa + c;
-    dA1[i] = min(r + 128, last_a) * sa + c;
+    dA1[i] = min(SHORT ? 128 + (wave * 2 + i) * 8 + (lane >> 3) : r + 128, last_a) * sa + c;  // (SHORT: two pieces)
     dB0[i] = min(r, last_b) * sb + c;
     dB1[i] = GATED ? dB0[i] : min(r + 128, last_b) * sb + c;
   }
@@ -646,7 +698,13 @@ __global__ void __launch_bounds__(256, 1) gemm_bf16_ring_kernel(GemmDesc g) {
 #define RING_WIDE_IN [dX] "v"(dX), [px] "s"(sx), [ldsx] "s"(ldsx)
 #define RING_WIDE_SCALARS "s48", "s50", "s51"
 #define RING_STRIP RING_V10(11), "v120", "v121", "v122", "v123", "v124", "v125", "v126", "v127"
+  // SHORT: this wavefront's place for A1 in a stage
+  const uint32_t lds1 = lds - (wave & 1) * 2048;
+#define RING_SHORT_IN                                                                                                      \
+  [dA00] "v"(dA0[0]), [dA01] "v"(dA0[1]), [dA02] "v"(dA0[2]), [dA03] "v"(dA0[3]), [dA10] "v"(dA1[0]), [dA11] "v"(dA1[1]),  \
+      [lds1] "s"(lds1), [pa] "s"(sa0), RING_IN_B
   if constexpr (WIDE) asm volatile(WFIRST_LOADS::RING_IN, RING_WIDE_IN : RING_SCALARS, RING_WIDE_SCALARS);
+  else if constexpr (SHORT) asm volatile(SFIRST_LOADS::RING_SHORT_IN : RING_SCALARS, "s48");
   else if constexpr (AH == 2) asm volatile(FIRST_LOADS::RING_IN : RING_SCALARS);
   else asm volatile(HFIRST_LOADS("") : RING_GATHERED : RING_IN_B, RING_ORDER : RING_SCALARS);
   float zero;
@@ -682,6 +740,7 @@ __global__ void __launch_bounds__(256, 1) gemm_bf16_ring_kernel(GemmDesc g) {
 #define RING_ACC1                                                                                                        \
   RING_ACC(1, 0, 0, 0), RING_ACC(1, 0, 0, 1), RING_ACC(1, 0, 1, 0), RING_ACC(1, 0, 1, 1), RING_ACC(1, 1, 0, 0),          \
       RING_ACC(1, 1, 0, 1), RING_ACC(1, 1, 1, 0), RING_ACC(1, 1, 1, 1)
+#define RING_ACC_SHORT RING_ACC(1, 0, 0, 0), RING_ACC(1, 0, 0, 1), RING_ACC(1, 1, 0, 0), RING_ACC(1, 1, 0, 1)
 #define RING_PLACES                                                                                                      \
   [ra0] "+v"(ra[0]), [ra1] "+v"(ra[1]), [ra2] "+v"(ra[2]), [ra3] "+v"(ra[3]), [rb0] "+v"(rb[0]), [rb1] "+v"(rb[1]),      \
       [rb2] "+v"(rb[2]), [rb3] "+v"(rb[3])
@@ -691,6 +750,8 @@ __global__ void __launch_bounds__(256, 1) gemm_bf16_ring_kernel(GemmDesc g) {
   if constexpr (WIDE)
     asm volatile(WMAIN_LOOP : RING_ACC0, RING_ACC1, RING_PLACES, RING_WIDE_PLACES : RING_IN, RING_WIDE_IN, [n] "s"(n_steps)
                  : RING_SCALARS, RING_WIDE_SCALARS, RING_STRIP, RING_FRAGMENTS);
+  else if constexpr (SHORT)
+    asm volatile(SMAIN_LOOP : RING_ACC0, RING_ACC_SHORT, RING_PLACES : RING_SHORT_IN, [n] "s"(n_steps) : RING_SCALARS, "s48", RING_FRAGMENTS);
   else if constexpr (AH == 2)
     asm volatile(MAIN_LOOP : RING_ACC0, RING_ACC1, RING_PLACES : RING_IN, [n] "s"(n_steps) : RING_SCALARS, RING_FRAGMENTS);
   else
@@ -717,7 +778,7 @@ __global__ void __launch_bounds__(256, 1) gemm_bf16_ring_kernel(GemmDesc g) {
                         late->rope_out16[grp], late->rope_cs_ss[grp], late->rope_n_as_float, late->rope_eps, late->rope_gamma_offset,
                         late->M, late->grp_n[grp], late->rope_s};
     constexpr int HD = KIND >= RING_ROPE_256 ? 256 : KIND >= RING_ROPE_128 ? 128 : 64;
-    ring_store_attention<HD, KIND == RING_ROPE_64_BIAS || KIND == RING_ROPE_128_BIAS, KIND == RING_ROPE_256_NORM, AH>(d, late->rope_role[grp] == 2, m0, n0, acc, ring_smem);
+    ring_store_attention<HD, KIND == RING_ROPE_64_BIAS || KIND == RING_ROPE_128_BIAS, KIND == RING_ROPE_256_NORM, AH, SHORT>(d, late->rope_role[grp] == 2, m0, n0, acc, ring_smem);
     return;
   }
   uint16_t *C16 = g.c16 ? g.c16 + (uint64_t)bz * g.M * g.N : nullptr;
@@ -735,7 +796,8 @@ __global__ void __launch_bounds__(256, 1) gemm_bf16_ring_kernel(GemmDesc g) {
   for (int qd = 0; qd < (GATED ? AH : 2 * AH); ++qd) {
     const int a = GATED ? qd : qd >> 1, b = GATED ? 0 : qd & 1;
     float *tile = ring_smem + wave * 8192 + (qd & 1) * 4096;
-    const uint32_t col0 = n0 + b * 128 + wn * 64, row0 = m0 + a * 128 + wm * 64;
+    const int blocks = SHORT && a ? 1 : 2;  // of 32 rows (guards in loops of a fixed length: registers are not indexed)
+    const uint32_t col0 = n0 + b * 128 + wn * 64, row0 = m0 + a * 128 + wm * blocks * 32;
     if (row0 >= g.M || col0 >= pitch) continue;  // (uniform: nothing of this quadrant is stored)
 #pragma unroll
     for (int i = 0; i < 2; ++i)
@@ -743,6 +805,7 @@ __global__ void __launch_bounds__(256, 1) gemm_bf16_ring_kernel(GemmDesc g) {
       for (int j = 0; j < 2; ++j)
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
+          if (i >= blocks) continue;
           const uint32_t r = (i ^ first) * 32 + (lane & 31), chunk = j * 8 + q * 2 + half;
           const f32x16 &x = acc[a][b][i][j], &u = acc[a][GATED ? 1 : b][i][j];
           float4 v = make_float4(x[q * 4], x[q * 4 + 1], x[q * 4 + 2], x[q * 4 + 3]);
@@ -755,7 +818,8 @@ __global__ void __launch_bounds__(256, 1) gemm_bf16_ring_kernel(GemmDesc g) {
     const float *from = tile + ((lane >> 4) << 6) + ((lane & 15) << 2);
     float4 out[16];
 #pragma unroll
-    for (int it = 0; it < 16; ++it) out[it] = *(const float4 *)(from + it * 256);
+    for (int it = 0; it < 16; ++it)
+      if (it < blocks * 8) out[it] = *(const float4 *)(from + it * 256);
     auto plus = [](float4 x, float4 y) { return make_float4(x.x + y.x, x.y + y.y, x.z + y.z, x.w + y.w); };
     if (F32 && Bias) {  // (grouped products: columns in fours, clamped to the last)
       float4 bias[4];
@@ -776,6 +840,7 @@ __global__ void __launch_bounds__(256, 1) gemm_bf16_ring_kernel(GemmDesc g) {
       char *corner = F32 ? (char *)(C + (uint64_t)row0 * Nl + col0) : (char *)(C16 + (uint64_t)row0 * pitch + col0);
 #pragma unroll
       for (int it = 0; it < 16; ++it) {
+        if (it >= blocks * 8) continue;
         char *at = corner + (uint64_t)(it >> 2) * 16 * pitch * (F32 ? 4 : 2) + to[it & 3];
         if (F32) {
           __builtin_memcpy(at, &out[it], 16);  // (rows of any length: 4-byte aligned)
@@ -815,6 +880,7 @@ __global__ void __launch_bounds__(256, 1) gemm_bf16_ring_kernel(GemmDesc g) {
     } else {  // (N % 4 == 0, or padded rows: a piece is inside or outside; zeros past the last column)
 #pragma unroll
       for (int it = 0; it < 16; ++it) {
+        if (it >= blocks * 8) continue;
         const uint32_t row = row0 + (it >> 2) * 16 + at_row[it & 3], col = col0 + at_col[it & 3];
         float4 v = out[it];
         v = make_float4(col < Nl ? v.x : 0.f, col + 1 < Nl ? v.y : 0.f, col + 2 < Nl ? v.z : 0.f, col + 3 < Nl ? v.w : 0.f);
@@ -1135,16 +1201,16 @@ bool gemm_ring_ok(const GemmDesc &g) {
          (!g.dual_b || (g.c16 && !g.c));
 }
 
-template <int KIND, int AH = 2, bool WIDE = false>
+template <int KIND, int AH = 2, bool WIDE = false, bool SHORT = false>
 static hipError_t launch_ring_as(const LaunchCtx &lc, const GemmDesc &g, uint32_t grid) {
   constexpr int smem = AH == 2 ? 2 * 65536 + (WIDE ? 2 * 4096 : 0) + (KIND >= RING_ROPE_64 ? 4 * 128 * 4 : 0) : 10 * 16384;  // (ring_store_rotated: sums of squares)
   static bool configured = false;  // one attribute call per kernel and process
   if (!configured) {
-    const hipError_t e = whole_lds((const void *)gemm_bf16_ring_kernel<KIND, AH, WIDE>, smem);
+    const hipError_t e = whole_lds((const void *)gemm_bf16_ring_kernel<KIND, AH, WIDE, SHORT>, smem);
     if (e != hipSuccess) return e;
     configured = true;
   }
-  cg_launch(lc, gemm_bf16_ring_kernel<KIND, AH, WIDE>, dim3(grid), dim3(256), smem, g);
+  cg_launch(lc, gemm_bf16_ring_kernel<KIND, AH, WIDE, SHORT>, dim3(grid), dim3(256), smem, g);
   return hipGetLastError();
 }
 
@@ -1156,28 +1222,39 @@ static hipError_t launch_ring_rope(const LaunchCtx &lc, const GemmDesc &g, uint3
   return bias ? launch_ring_as<RING_ROPE_64_BIAS, AH>(lc, g, grid) : launch_ring_as<RING_ROPE_64, AH>(lc, g, grid);
 }
 
-hipError_t launch_gemm_ring(const LaunchCtx &lc, const GemmDesc &g, bool half_height, bool wide) {
+bool gemm_ring_192_ok(const GemmDesc &g) {
+  return gemm_ring_ok(g) && g.splits <= 1 && !g.act_sigmoid && (g.dual_b || (g.rope_s && g.rope_hd != 256));
+}
+
+hipError_t launch_gemm_ring(const LaunchCtx &lc, const GemmDesc &g, RingTile tile) {
   if (!gemm_ring_ok(g)) return hipErrorInvalidValue;
-  if (half_height) {
-    if (g.act_sigmoid || g.splits > 1 || g.K < 192) return hipErrorInvalidValue;
-    const uint32_t bno = g.dual_b ? 128 : 256;
-    const uint64_t tiles = (uint64_t)((g.M + 127) / 128) * ((g.N + bno - 1) / bno) * g.nb0 * g.nb1;
-    if (tiles > 0x7FFFFFFFull) return hipErrorInvalidValue;
-    if (g.rope_s) return launch_ring_rope<1>(lc, g, (uint32_t)tiles);
-    if (!g.dual_b) return launch_ring_as<RING_PLAIN, 1>(lc, g, (uint32_t)tiles);
-    return g.glu_kind ? launch_ring_as<RING_GELU, 1>(lc, g, (uint32_t)tiles) : launch_ring_as<RING_SILU, 1>(lc, g, (uint32_t)tiles);
+  if (tile == RING_128 && (g.act_sigmoid || g.splits > 1 || g.K < 192)) return hipErrorInvalidValue;
+  if (tile == RING_192 && !gemm_ring_192_ok(g)) return hipErrorInvalidValue;
+  if (tile == RING_288 && (g.N % 4 || g.n_group || g.act_sigmoid || g.rope_s)) return hipErrorInvalidValue;
+  const uint32_t bm = tile == RING_128 ? 128 : tile == RING_192 ? 192 : 256, bn = tile == RING_288 ? 288 : 256, bno = g.dual_b ? bn / 2 : bn;
+  const uint64_t tiles = (uint64_t)((g.M + bm - 1) / bm) * ((g.N + bno - 1) / bno) * g.nb0 * g.nb1 * (g.splits > 1 ? g.splits : 1);
+  if (tiles > 0x7FFFFFFFull) return hipErrorInvalidValue;
+  const uint32_t grid = (uint32_t)tiles;
+  if (tile == RING_192) {
+    if (g.dual_b) return g.glu_kind ? launch_ring_as<RING_GELU, 2, false, true>(lc, g, grid) : launch_ring_as<RING_SILU, 2, false, true>(lc, g, grid);
+    const bool bias = g.grp_bias[0] != nullptr;
+    if (g.rope_hd == 128)
+      return bias ? launch_ring_as<RING_ROPE_128_BIAS, 2, false, true>(lc, g, grid) : launch_ring_as<RING_ROPE_128, 2, false, true>(lc, g, grid);
+    return bias ? launch_ring_as<RING_ROPE_64_BIAS, 2, false, true>(lc, g, grid) : launch_ring_as<RING_ROPE_64, 2, false, true>(lc, g, grid);
   }
-  if (wide && (g.N % 4 || g.n_group || g.act_sigmoid)) return hipErrorInvalidValue;
-  const uint32_t bno = (g.dual_b ? 128 : 256) + (wide ? (g.dual_b ? 16 : 32) : 0), batch = g.nb0 * g.nb1 * (g.splits > 1 ? g.splits : 1);
-  const uint64_t grid = (uint64_t)((g.M + 255) / 256) * ((g.N + bno - 1) / bno) * batch;
-  if (grid > 0x7FFFFFFFull) return hipErrorInvalidValue;
-  if (g.rope_s) return wide ? hipErrorInvalidValue : launch_ring_rope<2>(lc, g, (uint32_t)grid);
-  if (wide && g.dual_b)
-    return g.glu_kind ? launch_ring_as<RING_GELU, 2, true>(lc, g, (uint32_t)grid) : launch_ring_as<RING_SILU, 2, true>(lc, g, (uint32_t)grid);
-  if (wide) return launch_ring_as<RING_PLAIN, 2, true>(lc, g, (uint32_t)grid);
-  if (g.dual_b) return g.glu_kind ? launch_ring_as<RING_GELU>(lc, g, (uint32_t)grid) : launch_ring_as<RING_SILU>(lc, g, (uint32_t)grid);
-  if (g.act_sigmoid && g.splits <= 1) return launch_ring_as<RING_SIGMOID>(lc, g, (uint32_t)grid);
-  return launch_ring_as<RING_PLAIN>(lc, g, (uint32_t)grid);
+  if (tile == RING_128) {
+    if (g.rope_s) return launch_ring_rope<1>(lc, g, grid);
+    if (!g.dual_b) return launch_ring_as<RING_PLAIN, 1>(lc, g, grid);
+    return g.glu_kind ? launch_ring_as<RING_GELU, 1>(lc, g, grid) : launch_ring_as<RING_SILU, 1>(lc, g, grid);
+  }
+  if (tile == RING_288) {
+    if (!g.dual_b) return launch_ring_as<RING_PLAIN, 2, true>(lc, g, grid);
+    return g.glu_kind ? launch_ring_as<RING_GELU, 2, true>(lc, g, grid) : launch_ring_as<RING_SILU, 2, true>(lc, g, grid);
+  }
+  if (g.rope_s) return launch_ring_rope<2>(lc, g, grid);
+  if (g.dual_b) return g.glu_kind ? launch_ring_as<RING_GELU>(lc, g, grid) : launch_ring_as<RING_SILU>(lc, g, grid);
+  if (g.act_sigmoid && g.splits <= 1) return launch_ring_as<RING_SIGMOID>(lc, g, grid);
+  return launch_ring_as<RING_PLAIN>(lc, g, grid);
 }
 
 }  // namespace cgk

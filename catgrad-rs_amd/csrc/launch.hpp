@@ -367,10 +367,12 @@ struct GemmDesc {
 // The one-row kernels' two other arguments and the grid's size lie behind the descriptor, 20 bytes that are to be in the eighth.)
 static_assert(sizeof(GemmDesc) <= 488, "a GemmDesc and what lies behind it are eight lines of kernel arguments");
 // k_gemm_ring.hip: the 256 x 256 tiles of large bf16 products (plain or grouped, rotating, sigmoid, stacked gate / up);
-// half_height: tiles of 128 x 256 (all of these but a sigmoid, without slices), K >= 192; wide: tiles of 256 x 288 (plain without groups
-// or a sigmoid, stacked gate / up), N % 4 == 0
+// RING_128: tiles of 128 x 256 (all of these but a sigmoid, without slices), K >= 192; RING_192: 192 x 256 (gemm_ring_192_ok); RING_288:
+// 256 x 288 (plain without groups or a sigmoid, stacked gate / up), N % 4 == 0
+enum RingTile { RING_256, RING_128, RING_192, RING_288 };
 bool gemm_ring_ok(const GemmDesc &g);
-hipError_t launch_gemm_ring(const LaunchCtx &lc, const GemmDesc &g, bool half_height = false, bool wide = false);
+bool gemm_ring_192_ok(const GemmDesc &g);
+hipError_t launch_gemm_ring(const LaunchCtx &lc, const GemmDesc &g, RingTile tile = RING_256);
 // k_gemm_f32.hip: f32 products of operands in whole 16-byte pieces; gemm_f32_split: the slices of k it is fastest with (and how long
 // it then takes, about; gemm_f32_least_us: no less than this)
 bool gemm_f32_ok(const GemmDesc &g);

@@ -151,6 +151,7 @@ def test_grouped_products(hip_bf16, M, K, bias):
 @pytest.mark.parametrize("M,F,K", [(4096, 2048, 128), (4100, 2056, 192), (3900, 2184, 320),    # tiles of 256 rows
                                    (1030, 2184, 192), (900, 3000, 256), (1000, 2824, 512),     # and of 128: three steps, four, more
                                    (4100, 2056, 64), (4200, 2600, 128), (4100, 1256, 128), (1000, 3000, 64), (1030, 2184, 128),    # one and two, on eight wavefronts or four
+                                   (700, 8192, 192), (577, 7688, 256), (768, 6920, 320), (1153, 8200, 192),    # of 192: three steps, four, five; three rounds
                                    (4100, 2052, 192), (1030, 2180, 192), (1000, 2820, 512)])   # two products: rows of results off 16 bytes
 def test_gated(hip_bf16, M, F, K, act):
     g = np.random.default_rng(F)
@@ -265,6 +266,17 @@ def test_rotated_on_large_tiles(hip_bf16, hd, batch, S, heads, kv, K, bias, norm
     scores = np.where(np.tri(S, dtype=bool), scores, -np.inf)
     scores = np.exp(scores - scores.max(axis=-1, keepdims=True))
     parity.assert_bf16((scores / scores.sum(axis=-1, keepdims=True)) @ values, got, "attention")
+
+
+# ... (of those, the heads of 64 and of 128 above are in one round of 192 x 256; here, in none)
+ROTATED_256 = [(64, 1, 3301, 20, 20, 768, False, False), (64, 12, 277, 20, 20, 832, True, False),
+               (128, 7, 279, 16, 16, 768, True, False), (128, 1, 1930, 16, 16, 832, False, False)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("hd,batch,S,heads,kv,K,bias,norm", ROTATED_256)
+def test_rotated_on_256_rows(hip_bf16, hd, batch, S, heads, kv, K, bias, norm):
+    test_rotated_on_large_tiles(hip_bf16, hd, batch, S, heads, kv, K, bias, norm)
 
 
 # ... and on tiles of 128 x 256, where those are one round
