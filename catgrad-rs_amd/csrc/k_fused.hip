@@ -1187,6 +1187,37 @@ hipError_t launch_attn_decode(const LaunchCtx &lc, const AttnDecodeDesc &d) {
   return hipGetLastError();
 }
 
+// Bound by memory: four 16-byte pieces to a thread, all asked for before the first is stored.  8 x 4000 rows of 64, keys and values, 7.8 us,
+// 512 rows 3.3 (a copy of each 8.0 and 3.9 before, two launches of 2.8 to 3.0 for the new rows, and the key's rotation).  Each piece has a
+// name: an array of them the compiler put into LDS, by a kernel argument that lies in host memory (20 and 12.1 us).
+__global__ void __launch_bounds__(256) cache_grow_kernel(CacheGrowDesc g) {
+  typedef __attribute__((ext_vector_type(4))) float f32x4;
+  const bool c = blockIdx.z != 0;
+  const uint32_t bi = blockIdx.y / g.h, hi = blockIdx.y - bi * g.h, d4 = g.d / 4, n = g.t * d4;
+  const float *src = (c ? g.src[1] : g.src[0]) + bi * (c ? g.s_b[1] : g.s_b[0]) + hi * (c ? g.s_h[1] : g.s_h[0]);
+  float *dst = (c ? g.dst[1] : g.dst[0]) + bi * (c ? g.d_b[1] : g.d_b[0]) + hi * (c ? g.d_h[1] : g.d_h[0]);
+  const int64_t s_t = c ? g.s_t[1] : g.s_t[0];
+  const uint32_t i0 = blockIdx.x * 1024 + threadIdx.x, i1 = i0 + 256, i2 = i0 + 512, i3 = i0 + 768;
+  auto piece = [&](uint32_t i) {  // (past the end: the last)
+    i = min(i, n - 1);
+    const uint32_t t = i / d4;
+    return *(const f32x4 *)(src + t * s_t + (i - t * d4) * 4);
+  };
+  const f32x4 v0 = piece(i0), v1 = piece(i1), v2 = piece(i2), v3 = piece(i3);
+  if (i0 < n) *(f32x4 *)(dst + (uint64_t)i0 * 4) = v0;
+  if (i1 < n) *(f32x4 *)(dst + (uint64_t)i1 * 4) = v1;
+  if (i2 < n) *(f32x4 *)(dst + (uint64_t)i2 * 4) = v2;
+  if (i3 < n) *(f32x4 *)(dst + (uint64_t)i3 * 4) = v3;
+}
+
+hipError_t launch_cache_grow(const LaunchCtx &lc, const CacheGrowDesc &g) {
+  if (!g.n || !g.b || !g.h || !g.t || !g.d) return hipSuccess;
+  if (g.n > 2 || g.d % 4 || (uint64_t)g.b * g.h > 65535 || (uint64_t)g.t * g.d > 0xFFFFFFFFull) return hipErrorInvalidValue;
+  const uint32_t pieces = g.t * (g.d / 4);
+  CG_LAUNCH(lc, cache_grow_kernel, dim3((pieces + 1023) / 1024, g.b * g.h, g.n), 256, g);
+  return hipGetLastError();
+}
+
 // ---- rope -------------------------------------------------------------------------------------------
 // out[b,h,s,j] = cos[s,j] * x[b,h,s,j] + sin[s,j] * rot, rot = j < half ? -x[..,j+half] : x[..,j-half]
 // x is read through (b, h, s) strides with a unit stride along j, so the transposed view of the

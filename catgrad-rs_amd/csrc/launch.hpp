@@ -207,6 +207,16 @@ hipError_t launch_glu(const LaunchCtx &lc, int gelu, const float *gate, const fl
 hipError_t launch_binary_f32(const LaunchCtx &lc, int op, const float *a, const float *b, float *out,
                              uint64_t n, uint32_t b_period, bool a_bf16 = false);  // a_bf16: a points at bf16 values
 
+// The rows of a pair of caches ([b, h, t, d] through their strides, unit stride along d) copied to storage with room for more, rows d
+// floats apart: one launch.  d % 4 == 0, everything 16-byte aligned, b * h <= 65535.
+struct CacheGrowDesc {
+  const float *src[2];
+  float *dst[2];
+  int64_t s_b[2], s_h[2], s_t[2], d_b[2], d_h[2];
+  uint32_t n, b, h, t, d;  // n: one cache or two
+};
+hipError_t launch_cache_grow(const LaunchCtx &lc, const CacheGrowDesc &g);
+
 // One-query attention (a decode step): out[b, h, :] = softmax(q[b, h, :] . K[b, h, t, :] / scale + mask_const) . V
 // K and V rows are read in place from the (growable) cache through strides; head h of a
 // grouped-query model reads kv head h / rep (stride 0 along the repeat axis).

@@ -4,6 +4,26 @@
 namespace cgrt {
 
 
+// Storage for `n` with room to grow along `dim`, laid out for it (Storage::grow_*)
+int alloc_growable(cg_backend *be, const cg_tensor *n, int dim, Storage **out) {
+  int64_t cap = 64;
+  while (cap < 2 * n->shape[dim]) cap <<= 1;
+  int64_t cshape[CG_MAX_RANK];
+  std::copy(n->shape, n->shape + n->rank, cshape);
+  cshape[dim] = cap;
+  int64_t total = 1;
+  for (int i = 0; i < n->rank; ++i) total *= cshape[i];
+  Storage *s = nullptr;
+  TRY(dev_alloc(be, (size_t)total * 4, &s));
+  s->grow_dim = dim;
+  s->grow_cap = cap;
+  s->grow_rank = n->rank;
+  contiguous_strides(n->rank, cshape, s->grow_strides);
+  *out = s;
+  return CG_OK;
+}
+
+
 // concat(x, y, dim).  The KV cache grows by `concat(2, cached, new)` once per decode step
 // (catgrad-llm/src/legacy/models/utils.rs:210-228): copying the whole cache every step would cost
 // O(T) traffic per layer, so a small y appended to a large x gets storage with room to grow along
@@ -50,23 +70,12 @@ int realize_concat(cg_backend *be, cg_tensor *n) {
   // (2) an append-shaped concat: allocate with capacity along dim
   if (xd > 0 && yd > 0 && yd * 4 <= xd && x->stype != ST_BF16 && y->stype != ST_BF16 &&
       n->size() < ((int64_t)1 << 30)) {
-    int64_t cap = 64;
-    while (cap < 2 * (xd + yd)) cap <<= 1;
-    int64_t cshape[CG_MAX_RANK];
-    std::copy(n->shape, n->shape + n->rank, cshape);
-    cshape[dim] = cap;
-    int64_t total = 1;
-    for (int i = 0; i < n->rank; ++i) total *= cshape[i];
     Storage *s = nullptr;
-    TRY(dev_alloc(be, (size_t)total * 4, &s));
-    s->grow_dim = dim;
-    s->grow_cap = cap;
+    TRY(alloc_growable(be, n, dim, &s));
     n->st = s;
     n->stype = plain;
     n->offset = 0;
-    contiguous_strides(n->rank, cshape, n->strides);
-    s->grow_rank = n->rank;
-    std::copy(n->strides, n->strides + n->rank, s->grow_strides);
+    std::copy(s->grow_strides, s->grow_strides + n->rank, n->strides);
     TRY(run_ew(be, x, true, s->ptr, n->strides, plain, "ew_concat"));
     char *dst = (char *)s->ptr + xd * n->strides[dim] * 4;
     TRY(run_ew(be, y, true, dst, n->strides, plain, "ew_concat"));

@@ -155,7 +155,9 @@ int attn_decode_scratch(cg_backend *be, size_t part_floats, size_t count_words);
 bool has_grow_layout(const cg_tensor *x);
 cg_tensor *kv_concat_under(cg_tensor *t);
 int row_append_candidate(cg_backend *be, cg_tensor *c, bool allow_rope, RowAppend *out, bool *ok);
-void commit_row_append(cg_tensor *c);
+int grow_caches(cg_backend *be, RowAppend *ka, RowAppend *va, bool *ok);
+void commit_row_append(RowAppend *ra);
+int alloc_growable(cg_backend *be, const cg_tensor *n, int dim, Storage **out);
 int write_row_append(cg_backend *be, const RowAppend &ra);
 // later (optional): when the launch divides the keys over workgroups and the caller can merge the
 // partials itself (launch_gemv_pro with PRO_ATTN_MERGE), the attention stops at its partials, *later
@@ -586,7 +588,10 @@ struct RowAppend {
   cg_tensor *src = nullptr;  // retained: the tensor the rows are read from
   const float *cos = nullptr, *sin = nullptr;
   cg_tensor *cos_t = nullptr, *sin_t = nullptr;  // retained
+  bool grow = false;         // the cache has no room, or has other readers: its rows go to storage of their own first
+  Storage *grown = nullptr;  // that storage, until commit_row_append
   ~RowAppend() {
+    storage_release(grown);
     node_release(src);
     node_release(cos_t);
     node_release(sin_t);

@@ -545,6 +545,53 @@ def test_attention_decode_that_cannot_be_fused_still_appends_its_rows(oracle, hi
     assert np.max(np.abs(go - ro)) <= 2e-2 * np.abs(ro).max()
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("b,H,KV,T0,d", [(1, 4, 2, 5, 64), (2, 4, 4, 37, 128), (1, 8, 2, 900, 64), (3, 2, 1, 257, 16), (1, 4, 2, 64, 12)])
+@pytest.mark.parametrize("view", [False, True])
+def test_decode_from_a_kept_cache_copies_it_in_one_launch(oracle, hip, cg, b, H, KV, T0, d, view):
+    """A step whose caches somebody else holds too (a kept prefix), rows one after the other or a transposed view, and then one that appends
+    in place: the rows of both caches go to storage with room in one launch, the new ones with the attention's; the prefix stays as it was."""
+    g = np.random.default_rng(T0)
+    shape = (b, T0, KV, d) if view else (b, KV, T0, d)
+    k0, v0 = (g.standard_normal(shape).astype(np.float32) for _ in range(2))
+    new = [g.standard_normal((b, h, 1, d)).astype(np.float32) for h in (H, KV, KV)]
+
+    def step(bd, qv, kc, vc, kx, vx):
+        k, v = lang.concat(bd, 2, kc, kx), lang.concat(bd, 2, vc, vx)
+        kr, vr = helpers.repeat_kv(bd, H // KV, k), helpers.repeat_kv(bd, H // KV, v)
+        attn = lang.matmul(bd, qv, lang.transpose(bd, 2, 3, kr))
+        sh = lang.shape(bd, attn)
+        attn = attn / lang.constant(bd, float(np.sqrt(np.float32(d))), sh)
+        attn = attn + lang.broadcast(bd, helpers.causal_mask(bd, lang.to_nat(bd, 1)), sh)
+        return lang.matmul(bd, nn.softmax(bd, attn), vr), k, v
+
+    res = []
+    for be in (oracle, hip):
+        it = cg.Interpreter(be, cg.stdlib())
+        turn = vectors.Fn("turn", 1, 1, lambda bd, x: [lang.transpose(bd, 1, 2, x) if view else x + x - x]).term()
+        ((kc,), (vc,)) = (it.run(turn, [be.tensor(t)]) for t in (k0, v0))
+        be.realize(kc), be.realize(vc)
+        st = vectors.Fn("step", 5, 3, step).term()
+        args = [be.tensor(t) for t in new]
+        if be is hip:
+            be.trace(True)
+            be.trace_reset()
+        out1, k1, v1 = it.run(st, [args[0], kc, vc, args[1], args[2]])
+        be.realize(out1)
+        if be is hip:
+            names = be.trace_report()
+            be.trace(False)
+            assert names["cache_grow"]["launches"] == 1 and not any(n.startswith(("ew_concat", "kv_append")) for n in names), names
+        first = [be.numpy(t) for t in (out1, k1, v1)]
+        out2, k2, v2 = it.run(st, [args[0], k1, v1, args[1], args[2]], moved=(1, 2))
+        res.append(first + [be.numpy(t) for t in (out2, k2, v2, kc, vc)])
+    for i, (r, t) in enumerate(zip(*res)):
+        if i in (0, 3):
+            assert np.max(np.abs(t - r)) <= 1e-4 * np.abs(r).max()
+        else:
+            assert np.array_equal(t, r)
+
+
 @pytest.mark.parametrize("K", [2048, 256, 1152])
 @pytest.mark.parametrize("variant", ["llama", "gemma", "extra_consumer"])
 def test_rmsnorm_in_projection_prologue(oracle, hip, hip_bf16, hip_nopat, K, variant):
