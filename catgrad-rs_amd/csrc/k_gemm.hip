@@ -3440,13 +3440,13 @@ hipError_t launch_matmul(const LaunchCtx &lc_in, const GemmDesc &g, const char *
         // 60; 1500 rows, two or three, 92 and 84; 2900 by 2 x 8192, three or six, 159 and 181).  Fewer tiles of 128 than half the
         // CUs: 64 or 32 output columns per tile.  A round of 192 rows is 0.8 to 0.92 of one of 256 (2 x 8192, K = 2048: 700 rows, one round
         // either way, 49.0 and 44.6 us; 2100, three either way, 149 and 124; 2300 149 and 133) and 1.25 to 1.4 of one of 128 (1100, two or
-        // three, 89.3 and 78.5; 1459 98.8 and 88.3).
+        // three, 89.3 and 78.5; 1459 98.8 and 88.3).  (Fewer k-steps than eight: not measured.)
         const uint64_t d256w = (uint64_t)((g.M + 255) / 256) * ((g.N + 143) / 144) * batch;
         const uint64_t cus = (uint64_t)lc.n_cus, r256 = (d256 + cus - 1) / cus, r128 = (d128 + cus - 1) / cus;
         const bool wide = wide_ahead(144, d256);
         const uint64_t large = wide ? (d256w + cus - 1) / cus * 9 : r256 * 8;  // (in eighths of a round of 256 rows)
         const uint64_t r192 = ((uint64_t)((g.M + 191) / 192) * ((g.N + 127) / 128) * batch + cus - 1) / cus;
-        if (r192 * 32 < std::min(large * 5, r128 * 24) && g.K >= 192 && gemm_ring_192_ok(gg)) e = launch_gemm_ring(lc, gg, RING_192);
+        if (r192 * 32 < std::min(large * 5, r128 * 24) && g.K >= 512 && gemm_ring_192_ok(gg)) e = launch_gemm_ring(lc, gg, RING_192);
         else if (large * 5 <= r128 * 24 && gemm_ring_ok(gg)) e = launch_gemm_ring(lc, gg, wide ? RING_288 : RING_256);
         else if (d128 * 4 <= cus)
           e = launch_gemm_dma<128, 64, 4, 1, true, 5, true, false, false, 2>(lc, gg, (uint32_t)((uint64_t)((g.M + 127) / 128) * ((g.N + 31) / 32) * batch));

@@ -327,6 +327,28 @@ for kernel, sizes in ((wide, {large.WIDE_GATED}), (tall, [(4096, 2048, 320)])):
 """, BF16)
 
 
+def test_tiles_of_192_x_256(fake_hip):  # noqa: F811
+    """Gate and up from eight k-steps on, and q / k / v, where 256 rows to a tile, or 128, put in as many rounds; the sizes of test_large_tiles.py."""
+    fake_hip(LAUNCHED + f"""
+sys.path.insert(0, "tests")
+import test_large_tiles as large
+short, ring = "gemm_bf16_ring_kernelILi%dELi2ELb0ELb1E", "gemm_bf16_ring_kernelILi%dE"
+for m, f, k, on in ((700, 8192, 512, True), (577, 7688, 576, True), (768, 6920, 640, True), (1153, 8200, 512, True), (2100, 8192, 2048, True),
+                    (700, 8192, 448, False), (512, 8192, 2048, False), (769, 8192, 2048, False), (2900, 8192, 2048, False)):
+    for kind, act in ((2, nn.silu), (3, nn.gelu)):
+        (first, *_) = launched(lambda: run(lambda b, x, g, u, d: linear(b, act(b, linear(b, x, g, f, k)) * linear(b, x, u, f, k), d, 64, f),
+                                           operand(1, m, k), operand(f, k), operand(f, k), operand(64, f)))
+        assert ring % kind in first and (short % kind in first) == on, (m, f, k, first)
+for on, sizes in ((True, {large.ROTATED_LARGE}), (False, {large.ROTATED_256}), (False, {large.ROTATED_HALF})):
+    for hd, batch, s, heads, kv, k, bias, norm in sizes:
+        if hd == 256: continue
+        ns, kind = [heads * hd, kv * hd, kv * hd], {{64: 4, 128: 6}}[hd] + bias
+        args = [operand(1, batch * s, k)] + [operand(n, k) for n in ns] + [be.tensor(np.zeros(n, np.float32)) for n in ns]
+        (name,) = launched(lambda: run(lambda b, x, *p: large.attention_of_projections(b, x + x - x, p, hd, batch, s, heads, kv, k, bias, norm)[0], *args))
+        assert ring % kind in name and (short % kind in name) == on, (hd, batch, s, name)
+""", BF16)
+
+
 def test_q_k_v_that_rotate_on_large_tiles(fake_hip):  # noqa: F811
     """256 x 256 and 128 x 256 tiles for the sizes of test_large_tiles.py, with biases and norm; smaller ones, and no rotation, beyond."""
     fake_hip(LAUNCHED + f"""

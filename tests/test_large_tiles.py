@@ -151,7 +151,7 @@ def test_grouped_products(hip_bf16, M, K, bias):
 @pytest.mark.parametrize("M,F,K", [(4096, 2048, 128), (4100, 2056, 192), (3900, 2184, 320),    # tiles of 256 rows
                                    (1030, 2184, 192), (900, 3000, 256), (1000, 2824, 512),     # and of 128: three steps, four, more
                                    (4100, 2056, 64), (4200, 2600, 128), (4100, 1256, 128), (1000, 3000, 64), (1030, 2184, 128),    # one and two, on eight wavefronts or four
-                                   (700, 8192, 192), (577, 7688, 256), (768, 6920, 320), (1153, 8200, 192),    # of 192: three steps, four, five; three rounds
+                                   (700, 8192, 512), (577, 7688, 576), (768, 6920, 640), (1153, 8200, 512),    # of 192: eight steps, nine, ten; two rounds
                                    (4100, 2052, 192), (1030, 2180, 192), (1000, 2820, 512)])   # two products: rows of results off 16 bytes
 def test_gated(hip_bf16, M, F, K, act):
     g = np.random.default_rng(F)
