@@ -341,6 +341,64 @@ __global__ void __launch_bounds__(256) gemm_small_f32_kernel(GemmDesc g, int a_v
   }
 }
 
+// The same for the smallest: 16 x 16 tiles, eight wavefronts that share k in chunks of 16, so that a wavefront has a few loads, all asked for
+// at once, and a few short MFMAs (v_mfma_f32_16x16x4_f32; lane (r, kb) holds k = 4 kb .. 4 kb + 3 of row or column r, component j goes
+// into the j-th product).  Bound by latency: launch, one trip to memory, the sum of eight wavefronts through LDS.
+template <bool A_KC, bool B_KC>
+__global__ void __launch_bounds__(512) gemm_small_f32_kernel_16(GemmDesc g, int a_vec, int b_vec) {
+  typedef __attribute__((ext_vector_type(4))) float f32x4;
+  __shared__ float part[8][256];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r = lane & 15, kb = lane >> 4;
+  const uint32_t m0 = blockIdx.y * 16, n0 = blockIdx.x * 16, bz = blockIdx.z, b0 = bz / g.nb1, b1 = bz - b0 * g.nb1, K = g.K;
+  // (rows and columns past the end repeat the last: what they compute is not stored)
+  const float *Ar = (const float *)g.a + b0 * g.sa_b0 + b1 * g.sa_b1 + (int64_t)min(m0 + r, g.M - 1) * g.sam;
+  const float *Bc = (const float *)g.b + b0 * g.sb_b0 + b1 * g.sb_b1 + (int64_t)min(n0 + r, g.N - 1) * g.sbn;
+  const int64_t sak = A_KC ? 1 : g.sak, sbk = B_KC ? 1 : g.sbk;
+  const uint32_t chunks = (K + 15) / 16, per = (chunks + 7) / 8, c_begin = min(chunks, wave * per), c_end = min(chunks, c_begin + per);
+  auto four = [&](const float *p, int64_t s, bool vec, uint32_t k) {
+    f32x4 v;
+    if (k + 4 <= K) {
+      if (vec) return *(const f32x4 *)(p + k);
+      v[0] = p[k * s];
+      v[1] = p[(k + 1) * s];
+      v[2] = p[(k + 2) * s];
+      v[3] = p[(k + 3) * s];
+      return v;
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = k + e < K ? p[(k + e) * s] : 0.f;
+    return v;
+  };
+  f32x4 acc[4];  // (four chains of sums: their error is that of a quarter of the length)
+#pragma unroll
+  for (int u = 0; u < 4; ++u) acc[u] = (f32x4){0.f, 0.f, 0.f, 0.f};
+  for (uint32_t c = c_begin; c < c_end; c += 4) {
+    f32x4 a[4], b[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      if (c + u < c_end) {  // (uniform)
+        a[u] = four(Ar, sak, A_KC && a_vec, (c + u) * 16 + kb * 4);
+        b[u] = four(Bc, sbk, B_KC && b_vec, (c + u) * 16 + kb * 4);
+      }
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      if (c + u < c_end) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[u][j], b[u][j], acc[u], 0, 0, 0);
+      }
+  }
+#pragma unroll
+  for (int e = 0; e < 4; ++e) part[wave][(kb * 4 + e) * 16 + r] = (acc[0][e] + acc[1][e]) + (acc[2][e] + acc[3][e]);
+  __syncthreads();
+  const uint32_t row = m0 + tid / 16, col = n0 + tid % 16;
+  if (tid < 256 && row < g.M && col < g.N) {
+    const uint64_t at = (uint64_t)bz * g.M * g.N + (uint64_t)row * g.N + col;
+    float v = ((part[0][tid] + part[1][tid]) + (part[2][tid] + part[3][tid])) + ((part[4][tid] + part[5][tid]) + (part[6][tid] + part[7][tid]));
+    if (g.c_add) v += g.c_add[at];
+    g.c[at] = g.act_sigmoid ? sigmoid_ref(v) : v;
+  }
+}
+
 // Few enough 32 x 32 tiles that the kernel above has the machine to itself, and each not too deep: a tile reads its 64 rows
 // of operands by itself, and 128 x 128 tiles split along k are ahead from tiles * K of about 400 000 on (500 x 1000 x 500
 // 18 us here, 30 there; 200 x 512 x 2048 21, 24; 400 x 512 x 2048 33, 27; 200 x 2048 x 2048 64, 36; 200 x 2048 x 8192 237,
@@ -351,8 +409,18 @@ static bool gemm_small_ok(const LaunchCtx &lc, const GemmDesc &g) {
   return t32 <= 2 * (uint64_t)lc.n_cus && (g.M <= 32 || t32 * g.K <= 400 * 1024);
 }
 
+// Of those, the ones in 16 x 16 tiles, at most one to a CU and none of them deep (us, 32 x 32 with the sum of its slices, if any, and 16 x 16:
+// 64 x 256 x 128 4.5, 3.1; 64 x 10 x 256 5.5, 3.2; 250 x 250 x 256 6.1, 3.7; 64 x 256 x 512 8.6, 4.3; 33 x 100 x 499, rows off 16 bytes,
+// 13.5, 4.3; 40 x 100 x 743 11.7, 4.9; 256 x 256 x 1024 9.7, 6.3; 16 x 512 x 1024 8.8, 5.7; 128 x 256 x 2048 10.7, 9.4 - from there on a
+// weight's rows come from memory, and slices, which the norm behind them may sum, ask for them with more CUs).  Errors against 64-bit
+// sums of normal operands: 0.9 to 1.2e-7 for K = 128 to 1024, 1.1 to 1.8e-7 on 32 x 32.
+static bool gemm_small_16_ok(const LaunchCtx &lc, const GemmDesc &g) {
+  const uint64_t t16 = (uint64_t)((g.M + 15) / 16) * ((g.N + 15) / 16) * g.nb0 * g.nb1;
+  return gemm_small_ok(lc, g) && t16 <= (uint64_t)lc.n_cus && g.K <= 1024;
+}
+
 // An f32 product for k_gemm_f32.hip: all that it takes, unless the kernel above is ahead.  That one takes about 3 us and 13.5 ns per
-// k of a workgroup, half as much again when every CU has more than one, and 3 for a sum of slices (us here, 12 to 16 there: 10 x 512 x
+// k of a workgroup, half as much again when every CU has more than one, and 3 for a sum of slices - or, in 16 x 16 tiles, 2.6 us and 3.6 ns per k - (us here, on 32 x 32, 12 to 16 there: 10 x 512 x
 // 2048 9.5, 11; 64 x 256 x 128 4.4, 5.7; 2000 x 20 x 2000 11.5, 17; 300 x 1000 x 500 13.9, 11.2; 17 x 2048 x 2048 15.5, 12.7).
 // splits (optional): the slices of k it is fastest with.
 static uint32_t gemm_small_split(const LaunchCtx &lc, const GemmDesc &g);
@@ -362,7 +430,8 @@ static bool gemm_f32_tiles(const LaunchCtx &lc, const GemmDesc &g, uint32_t *spl
   if (gemm_small_ok(lc, g)) {
     const uint32_t s = gemm_small_split(lc, g);
     const uint64_t wgs = (uint64_t)((g.M + 31) / 32) * ((g.N + 31) / 32) * g.nb0 * g.nb1 * s;
-    small_us = 3.0 + 0.0135 * g.K / s * (wgs > (uint64_t)lc.n_cus ? 1.5 : 1.0) + (s > 1 ? 3.0 : 0.0);
+    if (gemm_small_16_ok(lc, g)) small_us = 2.6 + 0.0036 * g.K;
+    else small_us = 3.0 + 0.0135 * g.K / s * (wgs > (uint64_t)lc.n_cus ? 1.5 : 1.0) + (s > 1 ? 3.0 : 0.0);
     // Up to 32 columns and a workgroup to every other CU or more, but none with two: the kernel above needs two slices at most there,
     // and these tiles, three quarters of them empty, take 9 to 16, at 8 to 15 % more than they are priced at (4455 x 18 x 2700 37.6 us
     // above, 41.3 here; 4839 x 21 x 2408 35.1, 40.1; 5 x 469 x 20 x 3576 29.1, 32.5; level at best: 4340 x 10 x 2864 37.5, 37.4; with
@@ -3087,6 +3156,8 @@ bool gemm_epilogue_ok(const GemmDesc &g) {
 bool gemm_add_ok(const LaunchCtx &lc, const GemmDesc &g) {
   GemmDesc t = g;
   t.c_add = nullptr;
+  // (f32 products in 16 x 16 tiles, too: up to 1024 deep they were in slices from 512 on)
+  if (g.splits <= 1 && !g.act_sigmoid && !gemm_f32_tiles(lc, t) && gemm_small_16_ok(lc, t)) return true;
   const int av = a_vec_ok(g), bv = b_vec_ok(g);
   return g.splits <= 1 && !g.n_group && !g.dual_b && !g.glu_gate && !g.c16 && !g.act_sigmoid && !g.b_index && gemm_fast_path(t, av, bv) &&
          (gemm_dma_ok(t) ? g.M > 64 : gemm_narrow_dma_ok(lc, t));
@@ -3212,6 +3283,7 @@ hipError_t launch_splitk_sum(const LaunchCtx &lc, const float *ws, float *c, uin
 static uint32_t gemm_small_split(const LaunchCtx &lc, const GemmDesc &g) {
   const uint64_t t32 = (uint64_t)((g.M + 31) / 32) * ((g.N + 31) / 32) * g.nb0 * g.nb1;
   uint32_t splits = 1;
+  if (gemm_small_16_ok(lc, g)) return 1;
   while (t32 * splits * 2 <= (uint64_t)lc.n_cus && g.K / (splits * 2) >= 256 && splits < 64) splits *= 2;
   return splits;
 }
@@ -3625,8 +3697,16 @@ hipError_t launch_matmul(const LaunchCtx &lc_in, const GemmDesc &g, const char *
   }
   if (gemm_small_ok(lc, g)) {
     if (kernel_name) *kernel_name = "gemm_mfma_f32";
-    dim3 gr((g.N + 31) / 32, (g.M + 31) / 32, batch * gsplits);
     const bool akc = a_unit_k, bkc = b_unit_k;
+    if (gsplits == 1 && gemm_small_16_ok(lc, g)) {
+      const dim3 gr((g.N + 15) / 16, (g.M + 15) / 16, batch);
+      if (akc && bkc) CG_LAUNCH(lc, (gemm_small_f32_kernel_16<true, true>), gr, 512, g, av, bv);
+      else if (akc) CG_LAUNCH(lc, (gemm_small_f32_kernel_16<true, false>), gr, 512, g, av, 0);
+      else if (bkc) CG_LAUNCH(lc, (gemm_small_f32_kernel_16<false, true>), gr, 512, g, 0, bv);
+      else CG_LAUNCH(lc, (gemm_small_f32_kernel_16<false, false>), gr, 512, g, 0, 0);
+      return hipGetLastError();
+    }
+    dim3 gr((g.N + 31) / 32, (g.M + 31) / 32, batch * gsplits);
     if (akc && bkc) CG_LAUNCH(lc, (gemm_small_f32_kernel<true, true>), gr, 256, g, av, bv);
     else if (akc) CG_LAUNCH(lc, (gemm_small_f32_kernel<true, false>), gr, 256, g, av, 0);
     else if (bkc) CG_LAUNCH(lc, (gemm_small_f32_kernel<false, true>), gr, 256, g, 0, bv);

@@ -58,6 +58,42 @@ def assert_infinities(x, w, got):
     assert np.all(np.abs(got[finite] - ref[finite]) <= bound[finite])      # (a NaN is no less than its bound)
 
 
+# the smallest, on 16 x 16 tiles (test_kernel_choice.py asserts so): rows and columns that end inside one, k that ends inside a chunk of 16
+# or a lane's four, gives some wavefronts nothing, or takes more than one group of chunks; a batch
+SMALLEST = [(1, 9, 1, 1), (1, 64, 256, 128), (1, 64, 10, 256), (1, 17, 33, 5), (1, 31, 15, 127), (3, 70, 60, 100), (1, 40, 100, 743), (2, 16, 17, 1023),
+            (1, 250, 250, 512), (1, 13, 500, 1024)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("along_k", [True, False])
+@pytest.mark.parametrize("B,M,N,K", SMALLEST)
+def test_smallest_product(hip, B, M, N, K, along_k):
+    test_product(hip, 0, B, M, N, K, along_k)
+    if N > 1 and K > 1:
+        test_infinities(hip, 0, B, M, N, K, along_k)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(64, 256, 128), (33, 31, 1000)])
+def test_smallest_sigmoid(hip, M, N, K):
+    test_sigmoid(hip, M, N, K)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,M,N,K", [(1, 64, 256, 128), (3, 33, 31, 1000)])
+def test_smallest_product_of_columns_and_residual(hip, B, M, N, K):
+    """A left operand whose rows lie across memory, and a residual, added by the product's launch."""
+    g = np.random.default_rng(K)
+    x, w, r = (g.standard_normal(s).astype(np.float32) for s in ((B, K, M), (B, K, N), (B, M, N)))
+    hip.launch_counts(reset=True)
+    (got,) = vectors.run(hip, lambda b, r, x, w: [r + lang.matmul(b, lang.transpose(b, 1, 2, x), w)], 1, r, x, w)
+    counts = hip.launch_counts(reset=True)
+    assert sum(counts.values()) == 1, counts
+    exact = np.matmul(np.swapaxes(x, 1, 2).astype(np.float64), w.astype(np.float64))
+    bound = (K + 1) * 2.0 ** -24 * np.matmul(np.abs(np.swapaxes(x, 1, 2)), np.abs(w)) + 2.0 ** -24 * np.abs(exact + r)
+    assert np.all(np.abs(got - (exact + r)) <= bound)
+
+
 # every height of tile, k in one piece and in slices, a last step of one piece
 @pytest.mark.gpu
 @pytest.mark.parametrize("along_k", [True, False])

@@ -3,7 +3,7 @@ import pytest
 
 import test_k_order as k_order
 import test_large_tiles as large
-from test_f32_tiles import ODD_SIZES, SIZES
+from test_f32_tiles import ODD_SIZES, SIZES, SMALLEST
 from test_host_copies import fake_hip  # noqa: F401 - a fixture
 
 BF16 = 1
@@ -177,6 +177,13 @@ for rows, b, m, n, k in {SIZES}:
 for b, m, n, k in ((1, 64, 256, 128), (1, 33, 132, 1044), (3, 70, 260, 100), (1, 10, 512, 2048), (1, 2000, 20, 2000), (1, 4455, 18, 2700), (1, 4191, 23, 2860), (3, 1355, 11, 2792), (5, 469, 20, 3576)):
     names = product(m, n, k, batch=b)
     assert len(names) == 1 and "gemm_small_f32_kernel" in names[0], (b, m, n, k, names)
+for b, m, n, k in {SMALLEST}:
+    for along_k in (True, False):
+        names = product(m, n, k, along_k, b)
+        assert len(names) == 1 and "gemm_small_f32_kernel_16" in names[0], (b, m, n, k, names)
+for b, m, n, k in ((1, 33, 132, 1044), (1, 10, 512, 2048), (1, 2000, 40, 256)):     # (deep; more tiles than CUs)
+    names = product(m, n, k, batch=b)
+    assert len(names) == 1 and "gemm_small_f32_kernelI" in names[0], (b, m, n, k, names)
 for b, m, n, k in ((1, 4129, 24, 3200), (1, 4129, 40, 3200), (3, 326, 17, 7488)):     # (deeper, of more columns, of four slices)
     names = product(m, n, k, batch=b)
     assert len(names) == 1 and "gemm_f32_dma_kernel" in names[0], (b, m, n, k, names)
