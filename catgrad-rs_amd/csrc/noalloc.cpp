@@ -96,5 +96,9 @@ extern "C" int cg_argmax_into(cg_backend *be, cg_tensor *x, cg_tensor *out) {
     return fail_with(be, CG_ERR_DEVICE, "cg_argmax_into: every scratch slice of this device belongs to another live "
                                         "backend (8 per device)");
   if (hipSetDevice(be->device) != hipSuccess) return fail_with(be, CG_ERR_DEVICE, "hipSetDevice failed");
+  // (written here, now and in every replay of a graph: no host copy of its storage, kept or to come)
+  out->st->together = 0;
+  if (out->st->mirror) be->mirror_pool.push_back(out->st->mirror);
+  out->st->mirror = nullptr;
   return cgrt::reduce_into(be, x->dtype == CG_F32 ? R_ARGMAX_F : R_ARGMAX_U, x, out, ptr, SCRATCH_BYTES);
 }

@@ -49,6 +49,10 @@ struct Storage {
   // padded_key = {element offset of the mask, rows, keys, row stride}
   Storage *padded = nullptr;
   int64_t padded_key[4] = {-1, 0, 0, 0};
+  // results of one launch that lie one behind the other and are read one after the other (max(softmax(x)) and argmax(x)): the first read
+  // of either brings all `together` words, into a pinned buffer of cg_backend::mirror_pool that stays with the storage (0: each by itself)
+  uint32_t together = 0;
+  void *mirror = nullptr;
 };
 
 enum NodeOp : uint8_t {
@@ -207,6 +211,9 @@ struct cg_backend {
   // pinned buffers (PREFETCH_BYTES each) of cg_tensor_prefetch no tensor holds any more; the copy into the
   // last ones given back may still be in flight (its flag says)
   std::deque<void *> pinned_pool;
+  // the same of Storage::mirror (MIRROR_BYTES each, MIRROR_MAX at most)
+  std::deque<void *> mirror_pool;
+  int mirrors = 0;
   // scratch of the decode attention that divides the keys over several workgroups: partial results
   // and one counter per (batch, head); the counters are zero whenever no launch is running
   float *attn_part = nullptr;

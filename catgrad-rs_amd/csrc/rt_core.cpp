@@ -100,6 +100,7 @@ void storage_release(Storage *s) {
   storage_release(s->tiles);
   storage_release(s->padded);
   cg_backend *be = s->be;
+  if (s->mirror) be->mirror_pool.push_back(s->mirror);  // (used again once its copy has landed)
   // Safe to recycle at once: every consumer was enqueued on the backend's only stream.
   be->pool[s->bytes].push_back(s->ptr);
   be->pool_bytes += s->bytes;
@@ -117,6 +118,7 @@ void backend_release(cg_backend *be) {
   }
   trim_pool(be);
   for (void *p : be->pinned_pool) (void)hipHostFree(p);
+  for (void *p : be->mirror_pool) (void)hipHostFree(p);
   if (be->d_words) (void)hipFree(be->d_words);
   if (be->attn_part) (void)hipFree(be->attn_part);
   if (be->attn_count) (void)hipFree(be->attn_count);

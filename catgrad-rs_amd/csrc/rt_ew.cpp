@@ -408,11 +408,29 @@ static int try_softmax_best(cg_backend *be, cg_tensor *n, bool *done) {
   d.chunks = softmax_best_chunks(be->lc(), d.rows, d.n);
   Storage *part = nullptr;
   if (d.chunks > 1) TRY(dev_alloc(be, (size_t)rows * d.chunks * 16, &part));
-  int st = alloc_result(be, n, ST_F32);
-  if (!st && arg) st = alloc_result(be, arg, ST_U32);
+  // (a few rows' results lie in one storage: read one after the other, they cross the bus together)
+  const uint64_t behind = ((uint64_t)rows + 63) / 64 * 64, both = behind + (uint64_t)rows;
+  int st = CG_OK;
+  if (arg && both * 4 <= MIRROR_BYTES) {
+    st = dev_alloc(be, both * 4, &n->st);
+    if (!st) {
+      n->st->together = (uint32_t)both;
+      arg->st = n->st;
+      arg->st->rc.fetch_add(1);
+      n->stype = ST_F32;
+      arg->stype = ST_U32;
+      n->offset = 0;
+      arg->offset = (int64_t)behind;
+      contiguous_strides(n->rank, n->shape, n->strides);
+      contiguous_strides(arg->rank, arg->shape, arg->strides);
+    }
+  } else {
+    st = alloc_result(be, n, ST_F32);
+    if (!st && arg) st = alloc_result(be, arg, ST_U32);
+  }
   if (!st) {
-    d.best = (float *)n->st->ptr;
-    d.arg = arg ? (uint32_t *)arg->st->ptr : nullptr;
+    d.best = (float *)data_ptr(n);
+    d.arg = arg ? (uint32_t *)data_ptr(arg) : nullptr;
     d.part = part ? (float *)part->ptr : nullptr;
     KernelScope ks(be, "softmax_best", (double)x->size() * esize(x->stype) + (double)rows * (arg ? 8 : 4), 0);
     const hipError_t e = launch_softmax_best(be->lc(), d);

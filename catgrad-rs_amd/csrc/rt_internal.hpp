@@ -38,6 +38,7 @@ using namespace cgk;
   } while (0)
 
 
+enum : uint32_t { MIRROR_BYTES = 65536, MIRROR_TAIL = 64, MIRROR_MAX = 16 };  // pinned buffer of a Storage::mirror, behind it its error words and flag
 enum { PREFETCH_BYTES = 4096, PREFETCH_TAIL = 16 };  // pinned buffer of a prefetched tensor: data, error words and flag
 enum : size_t { HOST_IN_BYTES = (64 << 10) + 64, HOST_IN_SLOTS = 8 };
 enum : uint32_t { F_ONE = 0x3F800000u, F_HALF = 0x3F000000u, F_E = 0x402DF854u, F_TWO = 0x40000000u };
@@ -64,6 +65,7 @@ size_t size_class(size_t bytes);
 void trim_pool(cg_backend *be);
 void cap_pool(cg_backend *be);
 int dev_alloc(cg_backend *be, size_t bytes, Storage **out);
+inline uint32_t *mirror_words(void *mirror) { return (uint32_t *)((char *)mirror + MIRROR_BYTES); }
 void storage_release(Storage *s);
 void backend_release(cg_backend *be);
 cg_tensor *new_node(cg_backend *be, cg_dtype dt, int rank, const int64_t *shape);

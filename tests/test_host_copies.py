@@ -128,3 +128,49 @@ for i in range(40):
     assert np.array_equal(be.to_vec(t), a[:500] + np.uint32(i))
 works()
 """)
+
+
+def test_results_of_one_launch_cross_the_bus_together(fake_hip):
+    """max(softmax(x)) and argmax(x): one copy for both, each by itself for many rows; a copy that was not launched, and one given up unread."""
+    fake_hip("""
+lang, nn = cg.lang, cg.nn
+fake.fake_hip_launched.restype = ctypes.c_char_p
+
+class Best(lang.Module):
+    def path(self): return lang.path(["best"])
+    def sort(self): return [lang.TENSOR], [lang.TENSOR] * 2
+    def def_(self, b, args): return [lang.max(b, nn.softmax(b, args[0])), lang.argmax(b, args[0])]
+
+it = cg.Interpreter(be, cg.stdlib())
+term = Best().term()
+run = lambda rows: it.run(term, [be.tensor(np.zeros((rows, 8), np.float32))])
+
+def copies(reads):
+    be.sync()
+    fake.fake_hip_launched()
+    for t in reads: be.to_vec(t)
+    return fake.fake_hip_launched().decode().count("to_host_kernel")
+
+for rows, n in ((5, 1), (8192, 1), (8193, 2)):
+    p, a = run(rows)
+    c = copies([p, a]), copies([p, a])
+    assert c == ((1, 0) if n == 1 else (2, 2)), (rows, c)
+    p, a = run(rows)
+    be.realize(p)       # (asked for first, the column is found by itself)
+    assert copies([a, p, a]) == (1 if n == 1 else 3), rows
+held = [run(5) for i in range(20)]      # more than there are buffers
+c = [copies(r) for r in held]
+assert c[:15] == [1] * 15 and c[16:] == [2] * 4, c
+del held, p, a
+p, a = run(5)
+be.realize(p)
+be.sync()
+refuse("to_host_kernel")
+assert fails(lambda: be.to_vec(p))
+assert copies([p, a]) == 1
+for i in range(40):
+    p, a = run(5)
+    be.realize(p)
+    assert copies([a]) == 1
+works()
+""")

@@ -119,3 +119,34 @@ def test_error_on_rows_of_few_values(request, mode, rows, n):
         e = np.exp(d)
         terms = (e * (2.0 ** -23 + np.abs(d) * (2.0 ** -23 + 1.4e-8))).sum(axis=1) / e.sum(axis=1)
         assert np.all(np.abs(p.ravel() * e.sum(axis=1) - 1) <= terms + (34 + n / 4096) * 2.0 ** -24 + 4 * 2.0 ** -23)
+
+
+# what the two leave in memory is read back together where the rows are few: in either order, through a view, with more results held than
+# there are buffers, again after their storage has served others, and by itself once cg_argmax_into has written it
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows", [1, 63, 64, 4096, 8192, 8193])
+def test_results_read_one_after_the_other(hip, rows):
+    cg = vectors.cg
+    it, term = cg.Interpreter(hip, cg.stdlib()), vectors.Fn("best", 1, 2, best).term()
+    g = np.random.default_rng(rows)
+    xs = [g.standard_normal((rows, 8)).astype(np.float32) for _ in range(18 if rows == 63 else 3)]
+
+    def check(out, x, order):
+        e = np.exp(x.astype(np.float64) - x.max(1, keepdims=True))
+        for i in order:
+            got = hip.to_vec(out[i])
+            assert np.array_equal(got, x.argmax(1)) if i else np.allclose(got, 1 / e.sum(1), rtol=1e-5, atol=0)
+    for again in range(2):
+        held = [it.run(term, [hip.tensor(x)]) for x in xs]
+        for j, (out, x) in enumerate(zip(held, xs)):
+            hip.realize(out[0])     # (asked for first, the column is found by itself)
+            check(out, x, ((0, 1), (1, 0), (1, 1, 0, 0))[j % 3])
+        del out
+    seen = hip.reshape(held[0][1], (rows,))
+    assert np.array_equal(hip.to_vec(seen), xs[0].argmax(1))
+    other = hip.realize(hip.tensor(xs[1]))
+    hip.argmax_into(other, held[0][1])
+    assert np.array_equal(hip.to_vec(held[0][1]), xs[1].argmax(1)) and np.array_equal(hip.to_vec(seen), xs[1].argmax(1))
+    check(held[0], xs[0], (0,))
+    hip.argmax_into(hip.realize(hip.tensor(xs[2])), held[0][1])
+    assert np.array_equal(hip.to_vec(held[0][1]), xs[2].argmax(1))
