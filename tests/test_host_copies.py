@@ -152,25 +152,25 @@ def copies(reads):
     return fake.fake_hip_launched().decode().count("to_host_kernel")
 
 for rows, n in ((5, 1), (8192, 1), (8193, 2)):
-    p, a = run(rows)
-    c = copies([p, a]), copies([p, a])
+    p, k = run(rows)
+    c = copies([p, k]), copies([p, k])
     assert c == ((1, 0) if n == 1 else (2, 2)), (rows, c)
-    p, a = run(rows)
+    p, k = run(rows)
     be.realize(p)       # (asked for first, the column is found by itself)
-    assert copies([a, p, a]) == (1 if n == 1 else 3), rows
+    assert copies([k, p, k]) == (1 if n == 1 else 3), rows
 held = [run(5) for i in range(20)]      # more than there are buffers
 c = [copies(r) for r in held]
 assert c[:15] == [1] * 15 and c[16:] == [2] * 4, c
-del held, p, a
-p, a = run(5)
+del held, p, k
+p, k = run(5)
 be.realize(p)
 be.sync()
 refuse("to_host_kernel")
 assert fails(lambda: be.to_vec(p))
-assert copies([p, a]) == 1
+assert copies([p, k]) == 1
 for i in range(40):
-    p, a = run(5)
+    p, k = run(5)
     be.realize(p)
-    assert copies([a]) == 1
+    assert copies([k]) == 1
 works()
 """)
