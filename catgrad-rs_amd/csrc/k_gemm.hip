@@ -657,8 +657,10 @@ __global__ void __launch_bounds__(WR *WC *KG * 64) gemm_bf16_dma_kernel(GemmDesc
   uint32_t n0 = n0_all, Nl = g.N, grp = 0;
   if (g.n_group) {
     uint32_t p = 0;
-    while (p + 1 < g.n_group && n0 >= g.grp_n[p]) {
-      n0 -= g.grp_n[p];
+    // (32 x 32, gemm_with_column_ok: a product's last tile may be partly filled)
+    auto width = [&](uint32_t q) { return BM_ == 32 && !ROPE ? (g.grp_n[q] + BNO - 1) / BNO * BNO : g.grp_n[q]; };
+    while (p + 1 < g.n_group && n0 >= width(p)) {
+      n0 -= width(p);
       ++p;
     }
     B = (const uint16_t *)g.grp_b[p];
@@ -3144,6 +3146,20 @@ static bool gemm_narrow_dma_ok(const LaunchCtx &lc, const GemmDesc &g) {
   return g.N > 32 && g.N < 64 && g.sak == 1 && g.sbk == 1 && g.K % 64 == 0 && g.K <= 4096 && gemm_rows(g.M, g.K) && !g.n_group && !g.act_sigmoid;
 }
 
+// The router of a MoE prefill and the shared expert's gate, a column tile more: 1024 x 60 x 2048 9.1 us, and 4.9 for the column's own launch
+// (gemm_bf16_column_kernel), together 9.3.  While two workgroups to a CU hold every tile.
+bool gemm_with_column_ok(const LaunchCtx &lc, const GemmDesc &g) {
+  if (g.n_group != 2 || g.grp_n[1] != 1 || g.grp_bias[0] || g.grp_bias[1] || g.rope_s || g.nb0 * g.nb1 != 1 || g.splits > 1 || g.c_add || g.c16 ||
+      g.glu_gate || g.dual_b || g.act_sigmoid || g.b_index)
+    return false;
+  GemmDesc t = g;
+  t.n_group = 0;
+  t.N = g.grp_n[0];
+  t.b = g.grp_b[0];
+  if (3 * (uint64_t)((g.M + 31) / 32) > 2 * (uint64_t)lc.n_cus) return false;
+  return gemm_fast_path(t, a_vec_ok(t), b_vec_ok(t)) && gemm_narrow_dma_ok(lc, t) && aligned16(g.grp_b[1]);
+}
+
 bool gemm_epilogue_ok(const GemmDesc &g) {
   const int av = a_vec_ok(g), bv = b_vec_ok(g);
   return gemm_fast_path(g, av, bv) && gemm_dma_ok(g) && g.splits <= 1 && !g.b_index && !g.c_add &&
@@ -3354,7 +3370,8 @@ hipError_t launch_matmul(const LaunchCtx &lc_in, const GemmDesc &g, const char *
   const bool one_row = g.M <= 8 && g.a_stype == ST_F32 && g.K > 0 && (b_unit_k || b_unit_n);
   if (g.b_index && !one_row) return hipErrorInvalidValue;
   if (g.c_add && !one_row && g.splits <= 1 && !gemm_add_ok(lc_in, g)) return hipErrorInvalidValue;
-  if ((g.glu_gate || g.c16 || g.n_group || g.dual_b) && !gemm_epilogue_ok(g)) return hipErrorInvalidValue;
+  const bool with_column = g.n_group && gemm_with_column_ok(lc_in, g);
+  if ((g.glu_gate || g.c16 || g.n_group || g.dual_b) && !with_column && !gemm_epilogue_ok(g)) return hipErrorInvalidValue;
   if (g.act_sigmoid && !gemm_act_ok(lc_in, g)) return hipErrorInvalidValue;
   if (g.rope_s && !gemm_rope_epilogue_ok(lc_in, g)) return hipErrorInvalidValue;
 
@@ -3452,7 +3469,11 @@ hipError_t launch_matmul(const LaunchCtx &lc_in, const GemmDesc &g, const char *
     // share the weights, and their rows are then in the L2s for one step only (2900 x 2048 x 8192 95 and 134, 8192^3 745 and 805).  q / k / v
     // that rotate, tiles of 32 columns: 37 rows 12.0 us as they are, 12.6 so, 100 rows 12.3, 13.3.
     gg.k_rotate = g.M <= 128 && !g.rope_s && g.sbk == 1 && g.sbn % 2048 == 0 && gg.k_per_split >= 2048;
-    if (gemm_dma_ok(g)) {
+    if (with_column) {
+      gg.N = (g.grp_n[0] + 31) / 32 * 32 + 32;
+      const hipError_t e = launch_gemm_dma<32, 32, 1, 1, false, 8, false, false, false, 4>(lc, gg, (g.M + 31) / 32 * (gg.N / 32));
+      if (e != hipSuccess) return e;
+    } else if (gemm_dma_ok(g)) {
       const uint64_t t256 = (uint64_t)((g.M + 255) / 256) * ((g.N + 255) / 256) * batch * splits;
       hipError_t e;
       bool grp256 = true;  // 256-column tiles must not straddle two grouped products

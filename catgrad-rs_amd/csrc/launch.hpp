@@ -346,7 +346,7 @@ struct GemmDesc {
   const void *dual_b;
   // optional (same kernel, one batch, no split-K): n_group products that share A, K and the strides of
   // B (q/k/v of a prefill) as one launch.  N is the sum of grp_n; columns [0, grp_n[0]) belong to the
-  // first product, and so on; every grp_n is a multiple of 128; b and c are ignored.
+  // first product, and so on; every grp_n is a multiple of 128 (or: gemm_with_column_ok); b and c are ignored.
   uint32_t n_group;
   const void *grp_b[3];
   float *grp_c[3];
@@ -379,6 +379,8 @@ static_assert(sizeof(GemmDesc) <= 488, "a GemmDesc and what lies behind it are e
 // k_gemm_ring.hip: the 256 x 256 tiles of large bf16 products (plain or grouped, rotating, sigmoid, stacked gate / up);
 // RING_128: tiles of 128 x 256 (all of these but a sigmoid, without slices), K >= 192; RING_192: 192 x 256 (gemm_ring_192_ok); RING_288:
 // 256 x 288 (plain without groups or a sigmoid, stacked gate / up), N % 4 == 0
+// a product of 33 to 63 columns and one of a single column (n_group 2) in one launch of 32 x 32 tiles
+bool gemm_with_column_ok(const LaunchCtx &lc, const GemmDesc &g);
 enum RingTile { RING_256, RING_128, RING_192, RING_288 };
 bool gemm_ring_ok(const GemmDesc &g);
 bool gemm_ring_192_ok(const GemmDesc &g);

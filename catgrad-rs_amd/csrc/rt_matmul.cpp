@@ -1018,23 +1018,23 @@ int realize_matmul(cg_backend *be, cg_tensor *n, cg_tensor *addend, bool *added,
     // launch as further column ranges (their own weights, their own outputs)
     std::vector<cg_tensor *> group, group_add, group_bias;  // a member, the add that takes its value, its bias vector
     const bool bias_row = addend && be->addend_is_row;  // `addend` is a vector added to every row
+    // the same rows: one node, or - each linear folding the batch itself - dense reshapes of one value
+    auto dense_view = [](const cg_tensor *t, const Storage **st, int64_t *off) {
+      const cg_tensor *base = t->op == N_RESHAPE && t->in[0] ? t->in[0] : t;
+      if (base->op != N_REAL || !is_contiguous(base) || (t != base && t->size() != base->size())) return false;
+      *st = base->st;
+      *off = base->offset;
+      return true;
+    };
+    auto same_matrix = [&](const cg_tensor *a, const cg_tensor *b) {
+      if (a == b) return true;
+      const Storage *sa = nullptr, *sb = nullptr;
+      int64_t oa = 0, ob = 0;
+      return a->rank == b->rank && std::equal(a->shape, a->shape + a->rank, b->shape) && dense_view(a, &sa, &oa) &&
+             dense_view(b, &sb, &ob) && sa == sb && oa == ob;
+    };
     if (n->gemm_candidate && (!addend || bias_row) && !ep && !ex.w && batch == 1 && g.bf16_math && g.a_stype == ST_BF16 &&
         g.b_stype == ST_BF16 && g.sbk == 1 && N % 128 == 0 && gemm_epilogue_ok(g)) {
-      // the same rows: one node, or - each linear folding the batch itself - dense reshapes of one value
-      auto dense_view = [](const cg_tensor *t, const Storage **st, int64_t *off) {
-        const cg_tensor *base = t->op == N_RESHAPE && t->in[0] ? t->in[0] : t;
-        if (base->op != N_REAL || !is_contiguous(base) || (t != base && t->size() != base->size())) return false;
-        *st = base->st;
-        *off = base->offset;
-        return true;
-      };
-      auto same_matrix = [&](const cg_tensor *a, const cg_tensor *b) {
-        if (a == b) return true;
-        const Storage *sa = nullptr, *sb = nullptr;
-        int64_t oa = 0, ob = 0;
-        return a->rank == b->rank && std::equal(a->shape, a->shape + a->rank, b->shape) && dense_view(a, &sa, &oa) &&
-               dense_view(b, &sb, &ob) && sa == sb && oa == ob;
-      };
       for (cg_tensor *c : std::vector<cg_tensor *>(be->gemm_candidates)) {
         if (c == n || group.size() >= 2 || c->op != N_MATMUL || !same_matrix(c->in[0], n->in[0]) || c->rank != n->rank) continue;
         cg_tensor *w = c->in[1];
@@ -1055,6 +1055,27 @@ int realize_matmul(cg_backend *be, cg_tensor *n, cg_tensor *addend, bool *added,
         group_bias.push_back(bv);
       }
       if (group.size() < 2) group.clear();  // pairs (gate / up) keep their own launches and epilogues
+    }
+    // ... and a product of one column that of a few dozen: the shared expert's gate the router's (gemm_with_column_ok)
+    if (group.empty() && n->gemm_candidate && !addend && !ep && !ex.w && batch == 1 && N < 64) {
+      for (cg_tensor *c : std::vector<cg_tensor *>(be->gemm_candidates)) {
+        if (c == n || c->op != N_MATMUL || c->shape[c->rank - 1] != 1 || c->bias_user || !same_matrix(c->in[0], n->in[0])) continue;
+        cg_tensor *w = c->in[1];
+        if (w->rank != 3 || w->shape[0] != 1 || w->shape[1] != (int64_t)K) continue;
+        TRY(realize(be, w));  // a view of the parameter
+        if (w->stype != ST_BF16 || w->strides[1] != 1) continue;
+        GemmDesc t = g;
+        t.n_group = 2;
+        t.grp_n[0] = N;
+        t.grp_n[1] = 1;
+        t.grp_b[0] = g.b;
+        t.grp_b[1] = data_ptr(w);
+        if (!gemm_with_column_ok(be->lc(), t)) continue;
+        group.push_back(c);
+        group_add.push_back(nullptr);
+        group_bias.push_back(nullptr);
+        break;
+      }
     }
     if (!group.empty()) {
       g.n_group = 1;

@@ -412,3 +412,26 @@ def test_routed_experts(oracle, hip_bf16, S, E, F, H, act):
     (ref,) = vectors.run(oracle, f, 1, x, idx, val, wg, wu, wd)
     (got,) = vectors.run(hip_bf16, f, 1, x, idx, val, wg, wu, wd)
     parity.assert_bf16(ref, got, f"{S} tokens")
+
+
+# a product of a few dozen columns and one of a single column of the same rows (a MoE layer's router and its shared expert's gate): one
+# launch, a tile more; partly filled tiles of rows and columns, the fewest k, and more rows than two workgroups to a CU hold
+WITH_COLUMN = [(1024, 60, 2048, True), (17, 60, 1024, True), (33, 34, 448, True), (65, 63, 512, True), (5440, 60, 448, True), (5473, 60, 448, False)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K,joined", WITH_COLUMN)
+def test_product_with_a_column(hip_bf16, M, N, K, joined):
+    g = np.random.default_rng(M)
+    x, w, col = draw(g, (1, M, K)), draw(g, (N, K), K ** -0.5), draw(g, (1, K), K ** -0.5)
+
+    def f(b, x, w, col):
+        x = x + x - x
+        return [linear(b, x, w, N, K), linear(b, x, col, 1, K)]
+    hip_bf16.launch_counts(reset=True)
+    got = vectors.run(hip_bf16, f, 2, x, w, col)
+    counts = hip_bf16.launch_counts(reset=True)
+    assert sum(c for n, c in counts.items() if n.startswith("gem")) == 2 - joined, counts
+    for y, weight in zip(got, (w, col)):
+        ref, bound = product_and_bound(x[0], weight)
+        assert np.all(np.abs(y[0] - ref) <= bound)
