@@ -139,7 +139,7 @@ constexpr float ATTN_MAX_SLACK = 8.0f;
 template <int KT, bool LATE>
 __device__ __forceinline__ float attn_softmax_step(const AttnPrefillDesc &a, a_f32x16 (&st)[KT], const float *M, const float4 (&early)[KT][4],
                                                    a_bf16x8 (&pf)[KT * 2], float &m_run, float &l_run, float inv_scale, bool plain,
-                                                   bool use_mask, uint32_t t0, int half) {
+                                                   bool use_mask, uint32_t t0, int half, bool mask_covers = false) {
   constexpr float LOG2E = 1.44269504f, LOWEST = -3.40282347e+38f;
   float tmax = LOWEST, alpha, psum = 0.f;
   if (plain) {
@@ -164,7 +164,8 @@ __device__ __forceinline__ float attn_softmax_step(const AttnPrefillDesc &a, a_f
         }
         pf[kt * 2 + blk] = pack8(p);
       }
-  } else if (const bool tail = t0 + KT * 32 > a.t; use_mask && !tail) {  // (uniform)
+  } else if (const bool tail = t0 + KT * 32 > a.t; use_mask && (!tail || mask_covers)) {  // (uniform)
+    // (mask_covers: the keys past the end are zeros, and the mask's padded row has f32::MIN for them)
     // Mask values and no key past the end: the general form below without its selects, half of the vector instructions (us a layer,
     // causal, with and before: 32 heads of 64, 2900 tokens 87.3, 89.5; 16 heads of 128, 4 x 256 tokens 17.8, 18.5).
 #pragma unroll
@@ -501,7 +502,9 @@ __global__ void __launch_bounds__(NW * 64) ATTN_WAVES((D == 64 && NW == 4 && (KG
 // the main loop needs no workgroup barrier and the waves' memory waits overlap each other's arithmetic.
 // Each wave ends with its own running maximum, sum and O^T; they meet once, in LDS, and wave 0 merges
 // them (the same rescaling as between two steps of one wave).
-template <int D, int BN, int NW, bool LEAN = false>
+// ONE: all keys are one step, of one wave; nothing waits for the class table, the mask values travel with the keys, and the waves that had no
+// step, and their merge, are gone (us a layer, causal, 32 heads of 64: 20 tokens 7.9 -> 4.9, 37 7.9 -> 4.8, 64 7.4 -> 5.1).
+template <int D, int BN, int NW, bool LEAN = false, bool ONE = false>
 __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))  // two workgroups per CU
 attn_prefill_keysplit_kernel(AttnPrefillDesc a) {
   warm_kernel_arguments<sizeof(AttnPrefillDesc)>();
@@ -546,7 +549,8 @@ attn_prefill_keysplit_kernel(AttnPrefillDesc a) {
     }
   }
   tiles.arrived(lane);
-  auto step_mask = [&](uint32_t t0) { return M && tiles.reads_mask(t0); };
+  static_assert(!ONE || NW == 1, "one step, one wave");
+  auto step_mask = [&](uint32_t t0) { return M && (ONE || tiles.reads_mask(t0)); };
   uint4 kreg[KCH], vreg[KCH];
   auto fetch = [&](uint32_t t0) {
 #pragma unroll
@@ -560,8 +564,15 @@ attn_prefill_keysplit_kernel(AttnPrefillDesc a) {
       vreg[c] = *(const uint4 *)(VT + (int64_t)dim * a.vt_st + min(t0 + k8, a.vt_st - 8));
     }
   };
-  uint32_t t0 = tiles.skip(tiles.next_step(0), wave);
+  uint32_t t0 = ONE ? 0 : tiles.skip(tiles.next_step(0), wave);
   if (t0 < a.t) fetch(t0);
+  float4 first_mask[ONE ? KT : 1][4];
+  if (ONE && M) {
+#pragma unroll
+    for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) first_mask[ONE ? kt : 0][j] = *(const float4 *)(M + min(kt * 32u + j * 8 + half * 4, a.m_len - 4));
+  }
 #pragma unroll
   for (int c = 0; c < QC; ++c) {
     const int ch = tid + c * NW * 64, r = ch / (D / 8), d8 = (ch % (D / 8)) * 8;
@@ -587,7 +598,7 @@ attn_prefill_keysplit_kernel(AttnPrefillDesc a) {
   const bool can_be_plain = inv_scale > 0.f && (M || !a.has_mask_const);
 
   while (t0 < a.t) {
-    const uint32_t t_next = tiles.skip(t0, NW);
+    const uint32_t t_next = ONE ? a.t : tiles.skip(t0, NW);
     const bool use_mask = step_mask(t0);  // uniform over the wave
     const bool tail = t0 + BN > a.t;
     const uint32_t t_cur = t0;
@@ -601,7 +612,7 @@ attn_prefill_keysplit_kernel(AttnPrefillDesc a) {
 #pragma unroll
       for (int kt = 0; kt < KT; ++kt)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) mcur[kt][j] = *(const float4 *)(M + min(t_cur + kt * 32 + j * 8 + half * 4, a.m_len - 4));
+        for (int j = 0; j < 4; ++j) mcur[kt][j] = ONE ? first_mask[ONE ? kt : 0][j] : *(const float4 *)(M + min(t_cur + kt * 32 + j * 8 + half * 4, a.m_len - 4));
     }
     // registers -> this wave's LDS region.  Its LDS instructions run in program order, so the fragment
     // reads of the previous step are behind these writes and the reads below are ahead of them; the
@@ -632,7 +643,7 @@ attn_prefill_keysplit_kernel(AttnPrefillDesc a) {
       }
     }
     a_bf16x8 pf[KT * 2];
-    const float alpha = attn_softmax_step<KT, false>(a, st, M, mcur, pf, m_run, l_run, inv_scale, can_be_plain && !use_mask && !tail, use_mask, t_cur, half);
+    const float alpha = attn_softmax_step<KT, false>(a, st, M, mcur, pf, m_run, l_run, inv_scale, can_be_plain && !use_mask && !tail, use_mask, t_cur, half, ONE && a.m_len >= BN);
     if (__any(alpha != 1.0f)) {
 #pragma unroll
       for (int t = 0; t < DT; ++t)
@@ -988,6 +999,8 @@ static bool attn_prefill_keysplit(const LaunchCtx &lc, const AttnPrefillDesc &d)
          !attn_prefill_two_groups(lc, d);
 }
 
+bool attn_prefill_one_step(const LaunchCtx &lc, const AttnPrefillDesc &d) { return d.t <= 64 && attn_prefill_keysplit(lc, d); }
+
 // Heads of 128 and 256: two wavefronts to 32 queries, each with half of the values' dims (both compute the scores; the accumulators of
 // two waves then fit on a SIMD, and one's softmax runs under the other's products).  us a layer, heads of 128, causal, against one
 // wavefront to 32 queries: 16 heads of 400 tokens 24.0 -> 18.5, 1400 61.1 -> 49.2, 4 x 256 20.5 -> 17.9.  Beyond one workgroup of 128
@@ -1073,6 +1086,11 @@ hipError_t launch_attn_prefill(const LaunchCtx &lc, const AttnPrefillDesc &d) {
   } while (0)
   if (attn_prefill_keysplit(lc, d)) {
     dim3 g32((d.s + 31) / 32, d.heads, d.b);
+    if (attn_prefill_one_step(lc, d)) {
+      if (d.q16) CG_LAUNCH(lc, (attn_prefill_keysplit_kernel<64, 64, 1, true, true>), g32, 64, d);
+      else CG_LAUNCH(lc, (attn_prefill_keysplit_kernel<64, 64, 1, false, true>), g32, 64, d);
+      return hipGetLastError();
+    }
     CG_ATTN(attn_prefill_keysplit_kernel, g32, 256, 64, 64, 4);
     return hipGetLastError();
   }

@@ -296,6 +296,8 @@ struct AttnPrefillDesc {
 hipError_t launch_attn_prefill(const LaunchCtx &lc, const AttnPrefillDesc &d);
 // query rows and keys per tile that launch_attn_prefill uses for this problem
 void attn_prefill_tiling(const LaunchCtx &lc, const AttnPrefillDesc &d, uint32_t *q_rows, uint32_t *keys);
+// all keys are one step, of a kernel that looks at no class table
+bool attn_prefill_one_step(const LaunchCtx &lc, const AttnPrefillDesc &d);
 // out[qt * ceil(t / keys) + kt] = class of mask[qt * q_rows .., kt * keys ..] (values <= -3e38 count as masked);
 // mask is [s, t] with unit stride along t and row stride m_ss
 // mask [s, t] copied to rows of `pitch` >= t floats, f32::MIN from t on

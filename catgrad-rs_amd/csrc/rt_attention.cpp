@@ -116,7 +116,8 @@ int try_attn_prefill(cg_backend *be, cg_tensor *n, bool *done) {
   Storage *ksh = nullptr;
   const bool twin_ok = f32 || (Kop.t->st->grow_dim < 0 && Kop.t->st->bytes % 32 == 0);
   const bool shared_mask = mask && a.m_sb == 0 && a.m_sh == 0 && a.m_ss > 0 && a.m_st == 1 && mask->st->grow_dim < 0 && Sq <= 65535;
-  const bool pad_mask = mask && (!a.m_vec || T % 4);
+  // (... nor is it short of one step: the kernel then needs no look at where the keys end, attn_softmax_step)
+  const bool pad_mask = mask && (!a.m_vec || T % 4 || (T < 64 && shared_mask && !f32));
   a.m_len = (uint32_t)T;
   const int64_t mask_rows = a.m_ss;  // (two views of one storage may differ in nothing else)
   if ((pad_mask && !shared_mask) || !twin_ok) {
@@ -184,7 +185,7 @@ int try_attn_prefill(cg_backend *be, cg_tensor *n, bool *done) {
   // One mask for every batch and head (the causal or sliding-window mask of a model): classify its
   // tiles once - the table stays with the mask's storage, so every layer of the run finds it - and let
   // the kernel skip the key tiles no query of a tile can see.
-  if (mask && a.m_sb == 0 && a.m_sh == 0 && a.m_ss > 0 && mask->st->grow_dim < 0) {
+  if (mask && a.m_sb == 0 && a.m_sh == 0 && a.m_ss > 0 && mask->st->grow_dim < 0 && !attn_prefill_one_step(be->lc(), a)) {
     uint32_t q_rows = 0, keys = 0;
     attn_prefill_tiling(be->lc(), a, &q_rows, &keys);
     Storage *ms = mask->st;

@@ -217,6 +217,26 @@ def test_parts_of_a_query_tile(hip_bf16, H, KV, S, T, d):
     parity.assert_bf16(ref, got, f"{S} queries of {T} keys")
 
 
+# Heads of 64 whose keys are one step (test_kernel_choice.py asserts its kernel): full, ragged, of a length that is no multiple of four and of
+# one that is; more queries than keys; pairs hidden at random, rows that see no key, a key that no row sees
+@pytest.mark.gpu
+@pytest.mark.parametrize("H,KV,S,T", [(4, 2, 37, 37), (8, 8, 64, 64), (2, 1, 200, 40), (6, 3, 17, 63), (4, 4, 33, 36), (32, 8, 9, 10)])
+def test_keys_of_one_step(hip_bf16, H, KV, S, T):
+    g = np.random.default_rng(S + T)
+    q = vectors.bf16_round(g.standard_normal((1, H, S, 64)).astype(np.float32))
+    k, v = (vectors.bf16_round(g.standard_normal((1, KV, T, 64)).astype(np.float32)) for _ in range(2))
+    hidden = g.integers(0, 2, (S, T)).astype(np.float32)
+    hidden[:, T - 2], hidden[:, 1] = 1, 0
+    hidden[[3, S - 1]] = 1
+    f = attention_under(S, T, H // KV)
+    leave_nan_in_memory(hip_bf16, *(256 << i for i in range(13)), 1 << 20, 2 << 20)
+    hip_bf16.launch_counts(reset=True)
+    (got,) = vectors.run(hip_bf16, f, 1, q, k, v, hidden)
+    counts = hip_bf16.launch_counts(reset=True)
+    assert counts.get("attn_prefill") == 1 and "attn_mask_tiles" not in counts, counts
+    parity.assert_bf16(attention_in_numpy(q, k, v, hidden, H // KV), got, f"{S} queries of {T} keys")
+
+
 # Two views of one mask, alike but for their row stride: the first T columns of [S, 2 T] and the first S rows of the same values
 # as [2 S, T].  What one of them hides from every query the other shows to half of them.
 @pytest.mark.gpu

@@ -223,6 +223,40 @@ for shape, wide in (((1, 16, 2048, 128), 1), ((1, 16, 2049, 128), 0), ((4, 16, 5
 """, BF16)
 
 
+def test_attention_over_one_step_of_keys(fake_hip):  # noqa: F811
+    """Heads of 64: a wavefront to a tile up to 64 keys, with a mask and without; the keys of four beyond, and where tiles of 64 queries fill the CUs."""
+    fake_hip("""
+import importlib
+lang, nn = cg.lang, cg.nn
+helpers = importlib.import_module("catgrad-rs_amd.llm.helpers")
+fake.fake_hip_launched.restype = ctypes.c_char_p
+
+class Attention(lang.Module):
+    def __init__(self, shape, causal): self.shape, self.causal = shape, causal
+    def path(self): return lang.path(["attention", str(self.causal)])
+    def sort(self): return [lang.TENSOR] * 3, [lang.TENSOR]
+    def def_(self, b, args):
+        q, k, v = (lang.reshape(b, lang.make_shape(b, *self.shape), x) for x in args)
+        q, k, v = q + q - q, helpers.repeat_kv(b, 1, k + k - k), helpers.repeat_kv(b, 1, v + v - v)
+        s = lang.matmul(b, q, lang.transpose(b, 2, 3, k))
+        sh = lang.shape(b, s)
+        s = s / lang.constant(b, 11.0, sh)
+        if self.causal: s = s + lang.broadcast(b, helpers.causal_mask(b, lang.to_nat(b, self.shape[2])), sh)
+        return [lang.matmul(b, nn.softmax(b, s), v)]
+
+for shape, kernel in (((1, 32, 37, 64), "keysplit_kernelILi64ELi64ELi1E"), ((1, 32, 64, 64), "keysplit_kernelILi64ELi64ELi1E"),
+                      ((1, 32, 65, 64), "keysplit_kernelILi64ELi64ELi4E"), ((20, 32, 64, 64), "attn_prefill_kernelILi64E")):
+    for causal in (False, True):
+        q, k, v = (be.tensor(np.zeros(int(np.prod(shape)), np.float32)) for _ in range(3))
+        be.sync()
+        fake.fake_hip_launched()
+        be.realize(cg.Interpreter(be, cg.stdlib(), cg.Parameters()).run(Attention(shape, causal).term(), [q, k, v])[0])
+        be.sync()
+        names = [n for n in fake.fake_hip_launched().decode().split("\\n") if "attn_prefill" in n]
+        assert len(names) == 1 and kernel in names[0], (shape, causal, names)
+""", BF16)
+
+
 def test_sum_of_two_slots_of_the_same_experts(fake_hip):  # noqa: F811
     """The launch that realises one addend of `y0 + y1` makes the other as well: nothing is left of the product to add to."""
     fake_hip("""
