@@ -239,8 +239,10 @@ __device__ __forceinline__ float gelu_fast(float x) {
 // memory, 120 to 140 from its XCD's L2 (256 workgroups that only load tiles of 128 x 256 of 512 rows by 16384 of 2048 values: 39.4 us
 // with two stages and with three).  Tiles in step wait for memory with every load, since each piece is new to all of them; so, only with the
 // one step in four that they are the first to take: 30.3 us, 128 x 128 of 8192 30.7 -> 22.6, 128 x 64 of 3072 27 -> 18.6, 256 x 256 of 3072
-// rows 120 -> 92 (numbered by row tile alone 34.2, 26.1, 18.6 and 100; of eight steps 35.0, 27.2, 23.2 and 103).  For the routed experts of
-// several row tiles and the dense expert (1024 tokens 177 + 112 -> 173 + 104 us a layer).  Dense products do not gain: 512 x 2048 x 8192 on
+// rows 120 -> 92 (numbered by row tile alone 34.2, 26.1, 18.6 and 100; of eight steps 35.0, 27.2, 23.2 and 103).  For the dense expert's tiles
+// in the routed experts' launches (24 layers, 1024 tokens 9.70 -> 9.28 ms, 1400 10.68 -> 10.50, 4096 24.2 -> 23.7).  Not the routed experts' of several
+// row tiles: which of them a pair lies in follows from the order in which the sort's atomics land, and a result must not (nor do they gain: 9.28 and
+// 9.29 ms, 10.50 and 10.55, 23.7 and 23.55).  Other products do not gain: 512 x 2048 x 8192 on
 // 128 x 128 26.8 -> 25.5 us, but the kernels around it lose that (the clock), 512 x 2 x 8192 x 2048 on 128 x 256 36.0 -> 37.1, 2900 on
 // 256 x 256 168 -> 170, q / k / v of 37 rows 12.4 -> 12.7.
 struct KOrder {

@@ -1010,7 +1010,8 @@ __global__ void __launch_bounds__(256, 1) moe_ring_kernel(MoeGemmDesc g) {
   }
   const uint32_t n_steps = __builtin_amdgcn_readfirstlane(K / 64);
   const int64_t sbn0 = dense ? g.dense.sbn : g.prob[prob].sbn, sbn1 = dense || !GATED ? sbn0 : g.prob[1].sbn;
-  const KOrder order(dense ? 0u : g.k_rotate, e * tiles_n + n0 / BNO, n_steps, once ? 0u : m0 / 128 + n0 / BNO);
+  // (routed experts: no flip, since the row tile that a pair lies in depends on the order in which the sort's atomics land)
+  const KOrder order(dense ? 0u : g.k_rotate, e * tiles_n + n0 / BNO, n_steps, dense ? m0 / 128 + n0 / BNO : 0u);
   const uint16_t *w0 = dense ? (const uint16_t *)g.dense.w[0] : (const uint16_t *)g.prob[prob].w + (int64_t)e * g.sb_index;
   const uint16_t *w1 = dense ? (const uint16_t *)g.dense.w[1] : (const uint16_t *)g.prob[1].w + (int64_t)e * g.sb_index;
   const uint16_t *pb0 = w0 + (int64_t)n0 * sbn0 + order.step() * 64, *pb1 = GATED ? w1 + (int64_t)n0 * sbn1 + order.step() * 64 : pb0;

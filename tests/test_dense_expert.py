@@ -14,16 +14,7 @@ CASES = [(300, 768, 1280, 320, True), (300, 768, 1280, 768, True), (257, 1024, 1
          (128, 512, 2112, 192, True), (300, 768, 256, 320, False), (300, 768, 1280, 1000, False)]
 
 
-@pytest.mark.gpu
-@pytest.mark.parametrize("S,F,H,FS,joined", CASES)
-@pytest.mark.parametrize("act", ["silu", "gelu"])
-def test_dense_expert(hip_bf16, S, F, H, FS, joined, act):
-    E, k = 5, 2
-    g = np.random.default_rng(S + FS)
-    x = large.draw(g, (1, S, H))
-    wg, wu, sg, su = (large.draw(g, s, H ** -0.5) for s in ((E, F, H), (E, F, H), (FS, H), (FS, H)))
-    wd, sd = large.draw(g, (E, H, F), F ** -0.5), large.draw(g, (H, FS), FS ** -0.5)
-    idx = np.stack([g.choice(np.array([0, 2, 3]), S, p=[.2, .7, .1]), np.full(S, 4)], 1).astype(np.uint32)
+def layer(act, k, F, H, FS):
     gate = nn.silu if act == "silu" else nn.gelu
 
     def f(b, xv, iv, g_all, u_all, d_all, sg, su, sd):
@@ -36,6 +27,20 @@ def test_dense_expert(hip_bf16, S, F, H, FS, joined, act):
             total = y if total is None else total + y
         y = gate(b, large.linear(b, xv, sg, FS, H)) * large.linear(b, xv, su, FS, H)
         return [total, large.linear(b, y, sd, H, FS)]
+    return f
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("S,F,H,FS,joined", CASES)
+@pytest.mark.parametrize("act", ["silu", "gelu"])
+def test_dense_expert(hip_bf16, S, F, H, FS, joined, act):
+    E, k = 5, 2
+    g = np.random.default_rng(S + FS)
+    x = large.draw(g, (1, S, H))
+    wg, wu, sg, su = (large.draw(g, s, H ** -0.5) for s in ((E, F, H), (E, F, H), (FS, H), (FS, H)))
+    wd, sd = large.draw(g, (E, H, F), F ** -0.5), large.draw(g, (H, FS), FS ** -0.5)
+    idx = np.stack([g.choice(np.array([0, 2, 3]), S, p=[.2, .7, .1]), np.full(S, 4)], 1).astype(np.uint32)
+    f = layer(act, k, F, H, FS)
     hip_bf16.launch_counts(reset=True)
     routed, dense = vectors.run(hip_bf16, f, 2, x, idx, wg, wu, wd, sg, su, sd)
     counts = hip_bf16.launch_counts()
@@ -59,3 +64,22 @@ def test_dense_expert(hip_bf16, S, F, H, FS, joined, act):
         times = (idx == e).sum(1)[:, None]
         ref, bound = ref + times * y, bound + times * dy
     assert np.all(np.abs(routed[:, 0] - ref) <= bound + 2.0 ** -23 * np.abs(ref))
+
+
+# Experts of several row tiles: which of them a pair lies in follows from the order in which the sort's atomics land, and from the other tokens.
+# A routed row's sums come in the same order wherever it lies: the same bits in every run, and for the same tokens in another order.
+@pytest.mark.gpu
+@pytest.mark.parametrize("S,F,H,FS", [c[:4] for c in CASES[:4]] + [(2100, 512, 1024, 256)])
+def test_the_same_bits_wherever_a_pair_lies(hip_bf16, S, F, H, FS):
+    E, k = 5, 2
+    g = np.random.default_rng(S + F)
+    x = large.draw(g, (1, S, H))
+    weights = [large.draw(g, s, s[-1] ** -0.5) for s in ((E, F, H), (E, F, H), (E, H, F), (FS, H), (FS, H), (H, FS))]
+    idx = np.stack([g.choice(np.array([0, 2, 3]), S, p=[.2, .7, .1]), np.full(S, 4)], 1).astype(np.uint32)
+    run = lambda order: vectors.run(hip_bf16, layer("silu", k, F, H, FS), 2, x[:, order], idx[order], *weights)
+    routed, dense = run(np.arange(S))
+    for again in range(4):
+        r, d = run(np.arange(S))
+        assert np.array_equal(r, routed) and np.array_equal(d, dense), again
+        order = g.permutation(S)
+        assert np.array_equal(run(order)[0], routed[order]), again
