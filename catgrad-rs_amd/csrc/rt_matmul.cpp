@@ -150,6 +150,22 @@ cg_tensor *rows_base(cg_tensor *t) {
 }
 
 
+// Whether a product is among what t still waits for (or all that cannot be looked through quickly).  A product that joins the launch of
+// another has its operands realised while that one is on its way: an operand that waits for a product may wait for the very one, or for a
+// third that would take it along.
+static bool waits_for_product(const cg_tensor *t, int *looks) {
+  if (t->op == N_REAL) return false;
+  if (t->op == N_MATMUL || t->op == N_KSUM || --*looks < 0) return true;
+  for (const cg_tensor *in : t->in)
+    if (in && waits_for_product(in, looks)) return true;
+  return false;
+}
+bool waits_for_product(const cg_tensor *t) {
+  int looks = 64;
+  return waits_for_product(t, &looks);
+}
+
+
 // A deferred RMSNorm row A (or a reshape of one that regroups its rows) whose every reader can compute the norm
 // on its own way in, so that the norm needs no launch and its value is never stored: few-row products reading
 // A directly - at most one gated pair (`glu`, with its gate and up products) and narrow plain ones - and
@@ -957,7 +973,7 @@ int realize_matmul(cg_backend *be, cg_tensor *n, cg_tensor *addend, bool *added,
         cg_tensor *w = c->in[1];
         const int64_t nc = w->shape[w->rank - 1];
         if (w->rank != n->rank || w->shape[w->rank - 2] != (int64_t)K || nc < 1 || nc >= 64 ||  // (wide ones have fusions of their own)
-            c->size() != (int64_t)M * nc)
+            c->size() != (int64_t)M * nc || waits_for_product(w))
           continue;
         TRY(realize(be, w));  // a view of the parameter
         if (w->stype != ST_BF16 || w->strides[w->rank - 2] != 1) continue;
@@ -1057,20 +1073,19 @@ int realize_matmul(cg_backend *be, cg_tensor *n, cg_tensor *addend, bool *added,
       if (group.size() < 2) group.clear();  // pairs (gate / up) keep their own launches and epilogues
     }
     // ... and a product of one column that of a few dozen: the shared expert's gate the router's (gemm_with_column_ok)
-    if (group.empty() && n->gemm_candidate && !addend && !ep && !ex.w && batch == 1 && N < 64) {
+    GemmDesc with = g;
+    with.n_group = 2;
+    with.grp_n[0] = N;
+    with.grp_n[1] = 1;
+    with.grp_b[0] = with.grp_b[1] = g.b;
+    if (group.empty() && n->gemm_candidate && !addend && !ep && !ex.w && batch == 1 && N < 64 && gemm_with_column_ok(be->lc(), with)) {
       for (cg_tensor *c : std::vector<cg_tensor *>(be->gemm_candidates)) {
         if (c == n || c->op != N_MATMUL || c->shape[c->rank - 1] != 1 || c->bias_user || !same_matrix(c->in[0], n->in[0])) continue;
         cg_tensor *w = c->in[1];
-        if (w->rank != 3 || w->shape[0] != 1 || w->shape[1] != (int64_t)K) continue;
+        if (w->rank != 3 || w->shape[0] != 1 || w->shape[1] != (int64_t)K || waits_for_product(w)) continue;
         TRY(realize(be, w));  // a view of the parameter
-        if (w->stype != ST_BF16 || w->strides[1] != 1) continue;
-        GemmDesc t = g;
-        t.n_group = 2;
-        t.grp_n[0] = N;
-        t.grp_n[1] = 1;
-        t.grp_b[0] = g.b;
-        t.grp_b[1] = data_ptr(w);
-        if (!gemm_with_column_ok(be->lc(), t)) continue;
+        with.grp_b[1] = data_ptr(w);
+        if (w->stype != ST_BF16 || w->strides[1] != 1 || !gemm_with_column_ok(be->lc(), with)) continue;
         group.push_back(c);
         group_add.push_back(nullptr);
         group_bias.push_back(nullptr);

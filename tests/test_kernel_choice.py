@@ -416,3 +416,46 @@ for c in ((64, 1, 703, 20, 20, 768, False, False), (128, 1, 1202, 16, 16, 704, F
 (got,) = names(256, 4, 257, 4, 1, 768, False, True)
 assert "ring_kernelILi9E" not in got, got
 """, BF16)
+
+
+DEPENDENT = LAUNCHED + """
+helpers = importlib.import_module("catgrad-rs_amd.llm.helpers")
+def rows_of(b, y): return lang.transpose(b, 1, 2, lang.max(b, lang.transpose(b, 1, 2, y)))     # the largest of every column, a row
+def column(b, q): return lang.transpose(b, 1, 2, q)
+def graph(f, *args):
+    for outputs in range(2):
+        be.realize(run(lambda b, *a: f(b, *a)[outputs], *args))
+        both = cg.Interpreter(be, cg.stdlib(), cg.Parameters()).run(Both(len(args), f).term(), list(args))
+        for o in both[::-1] if outputs else both: be.realize(o)
+    be.sync()
+
+class Both(Term):
+    def sort(self): return [lang.TENSOR] * self.n_in, [lang.TENSOR] * 2
+    def def_(self, b, args): return self.f(b, *args)
+"""
+
+
+@pytest.mark.parametrize("rows", [4, 16, 300, 512])
+@pytest.mark.parametrize("columns", [8, 40])
+def test_a_column_that_comes_from_another_product_of_the_same_rows(fake_hip, rows, columns):  # noqa: F811
+    """A narrow product takes others of the same rows along, unless their matrices wait for a product: for itself, or for a third."""
+    fake_hip(DEPENDENT + f"""
+rows, n, k = {rows}, {columns}, 512
+x, w, v, u = operand(1, rows, k), operand(n, k), operand(n, k), operand(k, n)
+f32 = lambda x: x + x - x
+def pooled(b, x, w, u):
+    x = f32(x)
+    y = linear(b, x, w, n, k)
+    return [lang.matmul(b, x, column(b, linear(b, rows_of(b, y), u, k, n))), y]
+def largest(b, x, w):
+    x = f32(x)
+    y = linear(b, x, w, n, rows)
+    return [lang.matmul(b, x, lang.reshape(b, lang.make_shape(b, 1, rows, 1), lang.max(b, y))), y]
+def third(b, x, w, v, u):
+    x = f32(x)
+    y, p = linear(b, x, w, n, k), linear(b, x, v, n, k)
+    return [y + y, lang.matmul(b, x, column(b, linear(b, rows_of(b, p), u, k, n)))]
+graph(pooled, x, w, u)
+graph(third, x, w, v, u)
+graph(largest, operand(1, rows, rows), operand(n, rows))
+""", BF16)
