@@ -153,16 +153,24 @@ cg_tensor *rows_base(cg_tensor *t) {
 // Whether a product is among what t still waits for (or all that cannot be looked through quickly).  A product that joins the launch of
 // another has its operands realised while that one is on its way: an operand that waits for a product may wait for the very one, or for a
 // third that would take it along.
-static bool waits_for_product(const cg_tensor *t, int *looks) {
+static bool waits_for_product(const cg_tensor *t, bool experts, int *looks) {
   if (t->op == N_REAL) return false;
-  if (t->op == N_MATMUL || t->op == N_KSUM || --*looks < 0) return true;
+  ExpertOperand eo;
+  if ((t->op == N_MATMUL && (!experts || (t->rank == 3 && match_expert_operand(t->in[1], t->shape[0], &eo)))) ||
+      (t->op == N_KSUM && !experts) || --*looks < 0)
+    return true;
   for (const cg_tensor *in : t->in)
-    if (in && waits_for_product(in, looks)) return true;
+    if (in && waits_for_product(in, experts, looks)) return true;
   return false;
 }
 bool waits_for_product(const cg_tensor *t) {
   int looks = 64;
-  return waits_for_product(t, &looks);
+  return waits_for_product(t, false, &looks);
+}
+// ... of routed experts.  (Their indices wait for the router's product, which takes no expert's along.)
+bool waits_for_expert(const cg_tensor *t) {
+  int looks = 256;
+  return waits_for_product(t, true, &looks);
 }
 
 
@@ -286,6 +294,10 @@ int try_gate_up_glu(cg_backend *be, cg_tensor *glu, cg_tensor *g, cg_tensor *u, 
       for (cg_tensor *c : nr.plain) {
         cg_tensor *w = c->in[1];
         const int64_t nc = w->rank >= 2 ? w->shape[w->rank - 1] : 0;
+        if (waits_for_product(w)) {
+          shared_norm = false;
+          break;
+        }
         TRY(realize(be, w));
         bool ok = w->rank >= 2 && w->shape[w->rank - 2] == K && nc >= 1 && nc < 64 && c->size() == rows * nc && c->dtype == CG_F32 &&
                   w->stype == ST_BF16 && w->strides[w->rank - 2] == 1 && (uintptr_t)data_ptr(w) % 16 == 0 &&
@@ -387,6 +399,7 @@ int try_norm_reader_group(cg_backend *be, cg_tensor *n, bool *done) {
   NormReaders nr;
   if (!norm_readers(be, A, &nr) || !nr.glu) return CG_OK;
   if (std::find(nr.plain.begin(), nr.plain.end(), n) == nr.plain.end()) return CG_OK;
+  if (waits_for_product(rows_base(nr.gate)->in[1]) || waits_for_product(rows_base(nr.up)->in[1])) return CG_OK;
   bool fused = false;
   TRY(try_gate_up_glu(be, nr.glu, nr.gate, nr.up, nr.gelu, &fused));
   *done = fused && n->op == N_REAL;
@@ -421,6 +434,8 @@ int try_gemv_prologue(cg_backend *be, cg_tensor *n, cg_tensor *addend, bool *add
   for (cg_tensor *c : be->gemv_candidates)
     if (c != n && c->op == N_MATMUL && rows_base(c->in[0]) == A) members.push_back(c);
   if ((int)members.size() != refs(A) || members.size() > 4) return CG_OK;
+  for (const cg_tensor *c : members)
+    if (c != n && waits_for_product(c->in[1])) return CG_OK;
   GemvProDesc d;
   std::memset(&d, 0, sizeof(d));
   int b_stype = -1;
@@ -481,7 +496,7 @@ int try_gemv_prologue(cg_backend *be, cg_tensor *n, cg_tensor *addend, bool *add
     cg_tensor *c = members[i], *add = c->bias_user;
     if (c == n || !add || refs(c) != 1 || add->op != N_BIN || add->bias_of != c || add->size() != c->size()) continue;
     cg_tensor *bv = bias_vector_of(add->in[add->in[0] == c ? 1 : 0], add);
-    if (!bv) continue;
+    if (!bv || waits_for_product(bv)) continue;
     st = realize(be, bv);
     if (st) break;
     if (!bias_vector_ready(bv)) continue;
@@ -644,6 +659,15 @@ int realize_matmul(cg_backend *be, cg_tensor *n, cg_tensor *addend, bool *added,
     if (done) return CG_OK;
   }
   if (n->dtype == CG_F32 && n->gemv_candidate && !(be->flags & CG_FLAG_NO_PATTERNS)) {
+    // (a matrix that waits for products first: these may be of the same rows, and would find n on its way)
+    ExpertOperand own;
+    if (n->rank == 3 && match_expert_operand(n->in[1], n->shape[0], &own)) {
+      if (waits_for_expert(own.idx)) TRY(realize(be, own.idx));
+      if (waits_for_expert(own.w)) TRY(realize(be, own.w));
+    } else if (n->rank <= 3 && waits_for_product(n->in[1])) {
+      TRY(realize(be, n->in[1]));
+    }
+    if (n->op != N_MATMUL) return CG_OK;
     bool done = false;
     if (!addend) TRY(try_moe_gemv(be, n, &done));
     if (done) return CG_OK;
@@ -1062,7 +1086,7 @@ int realize_matmul(cg_backend *be, cg_tensor *n, cg_tensor *addend, bool *added,
         if (add) {
           if (refs(c) != 1 || add->op != N_BIN || add->bias_of != c || add->size() != c->size()) continue;
           bv = bias_vector_of(add->in[add->in[0] == c ? 1 : 0], add);
-          if (!bv) continue;
+          if (!bv || waits_for_product(bv)) continue;
           TRY(realize(be, bv));
           if (!bias_vector_ready(bv)) continue;
         }

@@ -4,6 +4,7 @@ for having actually been dispatched (by kernel name in the backend's trace)."""
 import numpy as np
 import pytest
 
+import parity
 import vectors
 
 pytestmark = pytest.mark.gpu
@@ -590,6 +591,31 @@ def test_decode_from_a_kept_cache_copies_it_in_one_launch(oracle, hip, cg, b, H,
             assert np.max(np.abs(t - r)) <= 1e-4 * np.abs(r).max()
         else:
             assert np.array_equal(t, r)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows", [1, 4, 20, 300])
+def test_products_whose_matrix_or_bias_comes_from_another_of_the_same_rows(oracle, hip, hip_bf16, rows):
+    """Products of the same rows that would share a launch, but one's matrix, or its bias, is computed from the other."""
+    n, k = 40, 512
+    g = np.random.default_rng(rows)
+    x = g.standard_normal((1, rows, k)).astype(np.float32)
+    w, v, u = (g.standard_normal(s).astype(np.float32) * s[-1] ** -0.5 for s in ((n, k), (n, k), (k, n)))
+
+    def f(b, x, w, v, u):
+        linear = lambda x, w, n, k: lang.matmul(b, x, lang.reshape(b, lang.make_shape(b, 1, k, n), lang.transpose(b, 0, 1, w)))
+        largest = lambda y: lang.transpose(b, 1, 2, lang.max(b, lang.transpose(b, 1, 2, y)))    # of every column, a row
+        out = []
+        for h in (x + x - x, helpers.rmsnorm_raw(b, 1e-5, x + x)):
+            y, z = linear(h, w, n, k), linear(h, v, n, k)
+            pooled = lang.matmul(b, h, lang.transpose(b, 1, 2, linear(largest(y), u, k, n)))
+            out += [pooled, y, z + lang.broadcast(b, lang.reshape(b, lang.make_shape(b, n), largest(y)), lang.shape(b, z))]
+        return out
+    ref = vectors.run(oracle, f, 6, x, w, v, u)
+    for be, check in ((hip, parity.assert_f32), (hip_bf16, parity.assert_bf16)):
+        for i, (r, t) in enumerate(zip(ref, vectors.run(be, f, 6, x, w, v, u))):
+            # (a row of one value is measured against all of them)
+            check(r.reshape(1, -1) if r.shape[-1] == 1 else r, t.reshape(1, -1) if r.shape[-1] == 1 else t, str(i))
 
 
 @pytest.mark.parametrize("K", [2048, 256, 1152])

@@ -459,3 +459,74 @@ graph(pooled, x, w, u)
 graph(third, x, w, v, u)
 graph(largest, operand(1, rows, rows), operand(n, rows))
 """, BF16)
+
+
+@pytest.mark.parametrize("flags", [0, BF16])
+@pytest.mark.parametrize("rows", [1, 4, 16, 300])
+def test_matrices_and_biases_that_come_from_another_product_of_the_same_rows(fake_hip, rows, flags):  # noqa: F811
+    """The readers of a norm that is computed on the way in, of a gated pair's rows, of q / k / v with biases: none joins that waits for a product."""
+    fake_hip(DEPENDENT + f"""
+rows, n, k = {rows}, 256, 512
+x, w, v, u, one = operand(1, rows, k), operand(n, k), operand(n, k), operand(k, n), operand(1, k)
+norm = lambda b, x: helpers.rmsnorm_raw(b, 1e-5, x + x)
+def normed(b, x, w, u):
+    h = norm(b, x)
+    y = linear(b, h, w, n, k)
+    return [lang.matmul(b, h, column(b, linear(b, rows_of(b, y), u, k, n))), y]
+def third(b, x, w, v, u):
+    h = norm(b, x)
+    y, p = linear(b, h, w, n, k), linear(b, h, v, n, k)
+    return [y + y, lang.matmul(b, h, column(b, linear(b, rows_of(b, p), u, k, n)))]
+def biased(rows_in):
+    def f(b, x, w, v):
+        h = rows_in(b, x)
+        y, z, t = linear(b, h, w, n, k), linear(b, h, v, n, k), linear(b, h, v, n, k)
+        return [z + lang.broadcast(b, lang.reshape(b, lang.make_shape(b, n), rows_of(b, y)), lang.shape(b, z)), y * t]
+    return f
+def gated(b, x, w, v, u, one):      # a gated pair and a column that comes from its gate's weights, or they from the column
+    h = norm(b, x)
+    c = linear(b, h, one, 1, k)
+    pair = nn.silu(b, linear(b, h, w, n, k)) * linear(b, h, v, n, k)
+    late = lang.matmul(b, h, column(b, linear(b, rows_of(b, lang.broadcast(b, c, lang.shape(b, pair))), u, k, n)))
+    return [pair, c + late]
+def gated_late(b, x, w, v, u, one):
+    h = norm(b, x)
+    c = linear(b, h, one, 1, k)
+    row = linear(b, rows_of(b, lang.broadcast(b, c, lang.make_shape(b, 1, rows, n))), u, k, n)
+    w = lang.transpose(b, 0, 1, w) + lang.broadcast(b, lang.reshape(b, lang.make_shape(b, k, 1), row), lang.make_shape(b, k, n))
+    pair = nn.silu(b, lang.matmul(b, h, lang.reshape(b, lang.make_shape(b, 1, k, n), w))) * linear(b, h, v, n, k)
+    return [pair, c]
+graph(normed, x, w, u)
+graph(third, x, w, v, u)
+graph(biased(norm), x, w, v)
+graph(biased(lambda b, x: x + x - x), x, w, v)
+graph(gated, x, w, v, u, one)
+graph(gated_late, x, w, v, u, one)
+""", flags)
+
+
+@pytest.mark.parametrize("flags", [0, BF16])
+@pytest.mark.parametrize("rows", [1, 4, 20, 300])
+def test_experts_chosen_by_another_expert(fake_hip, rows, flags):  # noqa: F811
+    """Routed experts' products of the same rows join each other's launches, unless their indices or matrices wait for an expert's product."""
+    fake_hip(DEPENDENT + f"""
+s, f, k = {rows}, 256, 512
+x, idx = be.tensor(np.zeros((s, 1, k), np.float32)), be.tensor(np.zeros((s, 2), np.uint32))
+up, down = [operand(5, f, k) for i in range(2)], operand(5, k, f)
+of = lambda b, i, w: lang.transpose(b, 1, 2, lang.index(b, 0, i, w))
+first = lambda b, idx: lang.reshape(b, lang.make_shape(b, s), lang.get(b, 1, 0, idx))
+def plain(b, x, idx, w):
+    y = lang.matmul(b, x, of(b, first(b, idx), w))
+    return [y + lang.matmul(b, x, of(b, lang.reshape(b, lang.make_shape(b, s), lang.argmax(b, y)), w)), y]
+def matrices(b, x, idx, w):
+    y = lang.matmul(b, x, of(b, first(b, idx), w))
+    t = lang.broadcast(b, lang.slice(b, 0, 0, 1, y), lang.make_shape(b, 5, k, f))
+    return [lang.matmul(b, x, of(b, first(b, idx), lang.transpose(b, 1, 2, t))), y]
+def whole(b, x, idx, g, u, d):
+    expert = lambda i: lang.matmul(b, nn.silu(b, lang.matmul(b, x, of(b, i, g))) * lang.matmul(b, x, of(b, i, u)), of(b, i, d))
+    y = expert(first(b, idx))
+    return [y + expert(lang.reshape(b, lang.make_shape(b, s), lang.argmax(b, y))), y]
+graph(plain, x, idx, up[0])
+graph(matrices, x, idx, up[0])
+graph(whole, x, idx, *up, down)
+""", flags)
