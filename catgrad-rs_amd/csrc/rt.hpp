@@ -53,6 +53,7 @@ struct Storage {
   // of either brings all `together` words, into a pinned buffer of cg_backend::mirror_pool that stays with the storage (0: each by itself)
   uint32_t together = 0;
   void *mirror = nullptr;
+  uint64_t mirror_at = 0;  // cg_backend::contexts when that copy was asked for
 };
 
 enum NodeOp : uint8_t {
@@ -222,7 +223,12 @@ struct cg_backend {
 
   // kernel launches go through this thread's queue; null when the backend launches inline (CG_FLAG_EAGER)
   cgk::LaunchQueue *queue = nullptr;
-  cgk::LaunchCtx lc() const { return cgk::LaunchCtx{stream, n_cus, d_words, cur_start, cur_stop, queue}; }
+  cgk::LaunchCtx lc() const {
+    ++contexts;
+    return copy_lc();
+  }
+  cgk::LaunchCtx copy_lc() const { return cgk::LaunchCtx{stream, n_cus, d_words, cur_start, cur_stop, queue}; }  // of a copy to the host
+  mutable uint64_t contexts = 0;  // contexts handed out for anything else: while it stays, nothing on the device has changed
   // the stream, once every launch handed to the queue has reached it: what anything but a kernel launch
   // (copies, events, synchronisation, frees) must use to keep program order
   hipStream_t ordered_stream() const {

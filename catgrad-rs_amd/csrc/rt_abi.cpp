@@ -113,7 +113,7 @@ int cg_tensor_prefetch(cg_backend *be, cg_tensor *t) {
     HIPCHK(be, hipHostMalloc(&buf, PREFETCH_BYTES, hipHostMallocDefault));
   }
   *flag_of(buf) = HOST_FLAG_PENDING;
-  const hipError_t e = launch_to_host(be->lc(), data_ptr(t), buf, bytes / 4, be->d_words, flag_of(buf) - 2, be->d_words + 4);
+  const hipError_t e = launch_to_host(be->copy_lc(), data_ptr(t), buf, bytes / 4, be->d_words, flag_of(buf) - 2, be->d_words + 4);
   if (e != hipSuccess) {
     *flag_of(buf) = HOST_FLAG_DONE;
     be->pinned_pool.push_back(buf);

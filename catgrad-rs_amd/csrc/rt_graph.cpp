@@ -276,7 +276,7 @@ int wait_host_flag(cg_backend *be, const uint32_t *flag) {
 // wait for the stream and surface device-side error flags
 int sync_and_check(cg_backend *be) {
   be->h_words[2] = HOST_FLAG_PENDING;
-  HIPCHK(be, launch_to_host(be->lc(), nullptr, nullptr, 0, be->d_words, be->h_words, be->d_words + 4));
+  HIPCHK(be, launch_to_host(be->copy_lc(), nullptr, nullptr, 0, be->d_words, be->h_words, be->d_words + 4));
   TRY(wait_host_flag(be, be->h_words + 2));
   return check_error_words(be, be->h_words);
 }
@@ -683,7 +683,7 @@ static int download_through_halves(cg_backend *be, const char *src, char *dst, s
   auto ask = [&](size_t first) -> int {  // for the pieces from `first` that fill one half
     for (size_t i = first; i < std::min(pieces, first + TO_HOST_MAX_PIECES); ++i) words(i)[2] = HOST_FLAG_PENDING;
     const size_t len = std::min(half, bytes - first * piece);
-    HIPCHK(be, launch_to_host(be->lc(), src + first * piece, data(first), len / 4, be->d_words, words(first), be->d_words + 4));
+    HIPCHK(be, launch_to_host(be->copy_lc(), src + first * piece, data(first), len / 4, be->d_words, words(first), be->d_words + 4));
     return CG_OK;
   };
   for (size_t i = 0; i < 2 * TO_HOST_MAX_PIECES && i < pieces; i += TO_HOST_MAX_PIECES) TRY(ask(i));
@@ -705,10 +705,16 @@ static int download_pieces(cg_backend *be, const char *src, char *dst, size_t by
 
 
 // A part of a storage whose parts are read together (Storage::together): the first read waits for all of it - a launch and a trip across
-// the bus more cost 9 us, 16 KB more on the way nothing -, later ones find it on the host.  *done stays false where the read has to go
-// the usual way: no buffer is left, or a kernel flagged an error since.
+// the bus more cost 9 us, 16 KB more on the way nothing -, the next ones find it on the host as long as nothing has been launched since
+// but copies to the host.  *done stays false where the read has to go the usual way: something was launched, which may have flagged an error
+// or stored here, what came was flagged, or there is no buffer.
 static int download_together(cg_backend *be, const cg_tensor *c, void *dst, size_t bytes, bool *done) {
   Storage *s = c->st;
+  if (s->mirror && (s->mirror_at != be->contexts || mirror_words(s->mirror)[0])) {
+    be->mirror_pool.push_back(s->mirror);
+    s->mirror = nullptr;
+    return CG_OK;
+  }
   const bool first = !s->mirror;
   if (first) {
     void *buf = nullptr;
@@ -721,17 +727,18 @@ static int download_together(cg_backend *be, const cg_tensor *c, void *dst, size
       ++be->mirrors;
     }
     mirror_words(buf)[2] = HOST_FLAG_PENDING;
-    const hipError_t e = launch_to_host(be->lc(), s->ptr, buf, s->together, be->d_words, mirror_words(buf), be->d_words + 4);
+    const hipError_t e = launch_to_host(be->copy_lc(), s->ptr, buf, s->together, be->d_words, mirror_words(buf), be->d_words + 4);
     if (e != hipSuccess) {
       mirror_words(buf)[2] = HOST_FLAG_DONE;
       be->mirror_pool.push_back(buf);
       return fail(be, CG_ERR_DEVICE, hipGetErrorString(e));
     }
     s->mirror = buf;
+    s->mirror_at = be->contexts;
   }
   uint32_t *words = mirror_words(s->mirror);
   const int st = wait_host_flag(be, words + 2);
-  if (st || (!first && words[0])) {  // nothing came and nothing will, or what came was flagged: the next read asks again
+  if (st) {  // nothing came and nothing will: the next read asks again
     words[2] = HOST_FLAG_DONE;
     be->mirror_pool.push_back(s->mirror);
     s->mirror = nullptr;

@@ -174,3 +174,39 @@ for i in range(40):
     assert copies([k]) == 1
 works()
 """)
+
+
+def test_a_kept_copy_is_not_read_once_something_was_launched(fake_hip):
+    """Between the reads of two results that crossed together: a launch, which may have flagged an error, and copies to the host, which cannot."""
+    fake_hip("""
+lang, nn = cg.lang, cg.nn
+fake.fake_hip_launched.restype = ctypes.c_char_p
+
+class Best(lang.Module):
+    def path(self): return lang.path(["best"])
+    def sort(self): return [lang.TENSOR], [lang.TENSOR] * 2
+    def def_(self, b, args): return [lang.max(b, nn.softmax(b, args[0])), lang.argmax(b, args[0])]
+
+it = cg.Interpreter(be, cg.stdlib())
+term = Best().term()
+other, third = be.tensor(a[:64]), be.tensor(a[64:128])
+be.realize(other), be.realize(third)
+
+def copies(f):
+    fake.fake_hip_launched()
+    f()
+    return fake.fake_hip_launched().decode().count("to_host_kernel")
+
+for again in range(40):     # (more often than there are buffers)
+    p, k = it.run(term, [be.tensor(np.zeros((5, 8), np.float32))])
+    assert copies(lambda: be.to_vec(p)) == 1
+    assert copies(lambda: be.to_vec(k)) == 0
+    be.to_vec(other), be.prefetch(third), be.sync()
+    assert copies(lambda: be.to_vec(k)) == 0
+    be.realize(be.add(other, third))
+    assert copies(lambda: be.to_vec(k)) == 1
+    be.realize(be.add(other, third))
+    assert copies(lambda: (be.to_vec(p), be.to_vec(k))) == 1
+    assert copies(lambda: (be.to_vec(p), be.to_vec(k))) == 0
+works()
+""")

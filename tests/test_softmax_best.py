@@ -150,3 +150,19 @@ def test_results_read_one_after_the_other(hip, rows):
     check(held[0], xs[0], (0,))
     hip.argmax_into(hip.realize(hip.tensor(xs[2])), held[0][1])
     assert np.array_equal(hip.to_vec(held[0][1]), xs[2].argmax(1))
+
+
+# an error that a kernel flags between the two reads is reported by the second, as if it crossed the bus by itself; the next ones are clean
+@pytest.mark.gpu
+@pytest.mark.parametrize("first", [0, 1])
+def test_an_error_between_two_reads(hip, first):
+    cg = vectors.cg
+    x = np.random.default_rng(5).standard_normal((70, 9)).astype(np.float32)
+    out = cg.Interpreter(hip, cg.stdlib()).run(vectors.Fn("best", 1, 2, best).term(), [hip.tensor(x)])
+    a, zero = hip.realize(hip.tensor(np.arange(4, dtype=np.uint32))), hip.realize(hip.tensor(np.zeros(4, np.uint32)))
+    hip.to_vec(out[first])
+    hip.realize(hip.div(a, zero))
+    with pytest.raises(cg.BackendPanic, match="divide by zero"):
+        hip.to_vec(out[1 - first])
+    assert np.array_equal(hip.to_vec(out[1]), x.argmax(1)) and hip.to_vec(out[0]).shape == (70,)
+    hip.sync()
