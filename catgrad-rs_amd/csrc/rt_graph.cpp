@@ -723,7 +723,10 @@ static int download_together(cg_backend *be, const cg_tensor *c, void *dst, size
       be->mirror_pool.pop_front();
     } else {
       if (be->mirrors >= (int)MIRROR_MAX) return CG_OK;
-      HIPCHK(be, hipHostMalloc(&buf, MIRROR_BYTES + MIRROR_TAIL, hipHostMallocDefault));
+      if (hipHostMalloc(&buf, MIRROR_BYTES + MIRROR_TAIL, hipHostMallocDefault) != hipSuccess) {
+        (void)hipGetLastError();
+        return CG_OK;
+      }
       ++be->mirrors;
     }
     mirror_words(buf)[2] = HOST_FLAG_PENDING;

@@ -1,6 +1,7 @@
 // A HIP runtime without a GPU, for tests of what the host does: memory is host memory, a stream is always idle, the two
 // copy kernels are made on the spot and every other launch is none.  fake_hip_refuse(name, n): the n-th launch from now
-// of a kernel whose name holds `name` is refused, as the runtime refuses one that it cannot make.  fake_hip_launched(): the
+// of a kernel whose name holds `name` is refused, as the runtime refuses one that it cannot make
+// ("hipHostMalloc": the n-th such call).  fake_hip_launched(): the
 // names of the kernels launched since the last call; fake_hip_products(): of the matrix products among them a line each, the name and what
 // the kernel is told of its walk along k - slices, values to a slice, whether column tiles start at different ones -; fake_hip_static_lds(n):
 // what every kernel's own __shared__ variables take.
@@ -101,7 +102,14 @@ hipError_t hipGetSymbolAddress(void **p, const void *) { static char room[1 << 1
 hipError_t hipGetLastError() { const hipError_t e = last; return last = hipSuccess, e; }
 const char *hipGetErrorString(hipError_t e) { return e == hipSuccess ? "no error" : "launch refused"; }
 hipError_t hipMalloc(void **p, size_t n) { return memory(p, n); }
-hipError_t hipHostMalloc(void **p, size_t n, unsigned) { return memory(p, n); }
+hipError_t hipHostMalloc(void **p, size_t n, unsigned) {
+  std::lock_guard<std::mutex> lk(lock);
+  if (refuse == "hipHostMalloc" && countdown.fetch_sub(1) == 1) {
+    refuse.clear();
+    return last = hipErrorOutOfMemory;
+  }
+  return memory(p, n);
+}
 hipError_t hipFree(void *p) { return free(p), hipSuccess; }
 hipError_t hipHostFree(void *p) { return free(p), hipSuccess; }
 hipError_t hipMemcpy(void *d, const void *s, size_t n, hipMemcpyKind) { return std::memcpy(d, s, n), hipSuccess; }

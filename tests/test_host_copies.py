@@ -210,3 +210,21 @@ for again in range(40):     # (more often than there are buffers)
     assert copies(lambda: (be.to_vec(p), be.to_vec(k))) == 0
 works()
 """)
+
+
+def test_results_are_read_one_by_one_without_room_for_them_on_the_host(fake_hip):
+    fake_hip("""
+lang, nn = cg.lang, cg.nn
+
+class Best(lang.Module):
+    def path(self): return lang.path(["best"])
+    def sort(self): return [lang.TENSOR], [lang.TENSOR] * 2
+    def def_(self, b, args): return [lang.max(b, nn.softmax(b, args[0])), lang.argmax(b, args[0])]
+
+p, k = cg.Interpreter(be, cg.stdlib()).run(Best().term(), [be.tensor(np.zeros((5, 8), np.float32))])
+be.realize(p)
+be.sync()
+refuse("hipHostMalloc")
+assert not fails(lambda: be.to_vec(p)) and not fails(lambda: be.to_vec(k))
+works()
+""")
