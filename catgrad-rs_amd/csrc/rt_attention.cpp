@@ -89,6 +89,13 @@ int try_attn_prefill(cg_backend *be, cg_tensor *n, bool *done) {
   n->strides[3] = 1;
   AttnPrefillDesc a;
   std::memset(&a, 0, sizeof(a));
+  a.b = (uint32_t)nb;
+  a.heads = (uint32_t)heads;
+  a.rep = (uint32_t)Kop.shape[2];
+  a.s = (uint32_t)Sq;
+  a.t = (uint32_t)T;
+  a.d = (uint32_t)d;
+  a.f32 = f32 ? 1 : 0;
   a.v = (const float *)data_ptr(Vop.t);
   if (lean) {
     a.q16 = (const uint16_t *)data_ptr(q);
@@ -116,8 +123,8 @@ int try_attn_prefill(cg_backend *be, cg_tensor *n, bool *done) {
   Storage *ksh = nullptr;
   const bool twin_ok = f32 || (Kop.t->st->grow_dim < 0 && Kop.t->st->bytes % 32 == 0);
   const bool shared_mask = mask && a.m_sb == 0 && a.m_sh == 0 && a.m_ss > 0 && a.m_st == 1 && mask->st->grow_dim < 0 && Sq <= 65535;
-  // (... nor is it short of one step: the kernel then needs no look at where the keys end, attn_softmax_step)
-  const bool pad_mask = mask && (!a.m_vec || T % 4 || (T < 64 && shared_mask && !f32));
+  // (... nor is it short of the step of the kernel that takes one only: that needs no look at where the keys end, attn_softmax_step)
+  const bool pad_mask = mask && (!a.m_vec || T % 4 || (T < 64 && shared_mask && attn_prefill_one_step(be->lc(), a)));
   a.m_len = (uint32_t)T;
   const int64_t mask_rows = a.m_ss;  // (two views of one storage may differ in nothing else)
   if ((pad_mask && !shared_mask) || !twin_ok) {
@@ -147,7 +154,6 @@ int try_attn_prefill(cg_backend *be, cg_tensor *n, bool *done) {
   bool vt_ready = false;
   const int64_t kvh = Kop.shape[1];
   if (f32) {
-    a.f32 = 1;
     a.k = (const float *)data_ptr(Kop.t);
   } else {
     TRY(bf16_shadow(be, Kop.t->st, &ksh));
@@ -172,12 +178,6 @@ int try_attn_prefill(cg_backend *be, cg_tensor *n, bool *done) {
     }
   }
   if (vt) a.vt16 = (const uint16_t *)vt->ptr;
-  a.b = (uint32_t)nb;
-  a.heads = (uint32_t)heads;
-  a.rep = (uint32_t)Kop.shape[2];
-  a.s = (uint32_t)Sq;
-  a.t = (uint32_t)T;
-  a.d = (uint32_t)d;
   a.has_scale = m.has_scale;
   a.scale = m.scale;
   a.has_mask_const = m.has_mask_const;

@@ -257,6 +257,38 @@ for shape, kernel in (((1, 32, 37, 64), "keysplit_kernelILi64ELi64ELi1E"), ((1, 
 """, BF16)
 
 
+def test_masks_that_are_read_as_they_are(fake_hip):  # noqa: F811
+    """Rows of a multiple of four keys are copied to longer ones for the kernel of one step alone; others always."""
+    fake_hip("""
+import importlib
+lang, nn = cg.lang, cg.nn
+helpers = importlib.import_module("catgrad-rs_amd.llm.helpers")
+fake.fake_hip_launched.restype = ctypes.c_char_p
+
+class Attention(lang.Module):
+    def __init__(self, shape): self.shape = shape
+    def path(self): return lang.path(["attention"])
+    def sort(self): return [lang.TENSOR] * 3, [lang.TENSOR]
+    def def_(self, b, args):
+        q, k, v = (lang.reshape(b, lang.make_shape(b, *self.shape), x) for x in args)
+        q, k, v = q + q - q, helpers.repeat_kv(b, 1, k + k - k), helpers.repeat_kv(b, 1, v + v - v)
+        s = lang.matmul(b, q, lang.transpose(b, 2, 3, k))
+        sh = lang.shape(b, s)
+        s = s / lang.constant(b, 11.0, sh) + lang.broadcast(b, helpers.causal_mask(b, lang.to_nat(b, self.shape[2])), sh)
+        return [lang.matmul(b, nn.softmax(b, s), v)]
+
+for shape, padded in (((1, 32, 36, 64), 1), ((1, 32, 64, 64), 0), ((1, 32, 68, 64), 0), ((1, 32, 70, 64), 1), ((20, 32, 60, 64), 0),
+                      ((1, 16, 36, 128), 0), ((1, 16, 37, 128), 1), ((1, 4, 60, 256), 0), ((1, 4, 61, 256), 1), ((4, 16, 32, 128), 0)):
+    q, k, v = (be.tensor(np.zeros(int(np.prod(shape)), np.float32)) for _ in range(3))
+    be.sync()
+    fake.fake_hip_launched()
+    be.realize(cg.Interpreter(be, cg.stdlib(), cg.Parameters()).run(Attention(shape).term(), [q, k, v])[0])
+    be.sync()
+    names = fake.fake_hip_launched().decode().split("\\n")
+    assert sum("attn_prefill" in n for n in names) == 1 and sum("mask_pad" in n for n in names) == padded, (shape, names)
+""", BF16)
+
+
 def test_sum_of_two_slots_of_the_same_experts(fake_hip):  # noqa: F811
     """The launch that realises one addend of `y0 + y1` makes the other as well: nothing is left of the product to add to."""
     fake_hip("""
