@@ -3243,11 +3243,14 @@ static bool rope_on_half_tiles(const LaunchCtx &lc, const GemmDesc &g) {
   return m128 * ((g.N + 127) / 128) > cus && m128 * ((g.N + 255) / 256) <= cus;
 }
 
-// ... or of 192 x 256 in the place of 256 x 256, at 0.8 of a round's time and more (3072 columns of heads of 64, K = 2048, one round either
-// way: 2700 rows 59.7 -> 50.1 us, 2900 58.6 -> 49.9, 3500 61.5 -> 53.8, 4000 63.3 -> 56.4).
+// ... or of 192 x 256 in the place of 256 x 256, at 0.8 of a round's time and more - more rounds of them only where the grid is dealt to the
+// XCDs in eight equal parts (TilePlace; below, at gate / up, both sides).  One round either way, 3072 columns: heads of 64, K = 2048, 2700 rows
+// 57.9 -> 50.8 us, 2904 52.9 -> 45.5, 3510 60.8 -> 54.4, 3990 63.7 -> 58.4; heads of 128 2904 rows 53.1 -> 45.0; K = 1024 2904 rows 35.8 -> 30.7,
+// 3510 42.3 -> 38.4; 768 3510 rows 38.0 -> 34.7, heads of 128, 1355 x 6144 38.0 -> 34.3.  (Fewer k: rope_on_large_tiles.)
 static bool rope_on_192_tiles(const LaunchCtx &lc, const GemmDesc &g) {
   const uint64_t cus = (uint64_t)lc.n_cus, n256 = (g.N + 255) / 256, t256 = (g.M + 255) / 256 * n256, t192 = (g.M + 191) / 192 * n256;
-  return gemm_ring_192_ok(g) && (t192 + cus - 1) / cus * 4 < (t256 + cus - 1) / cus * 5;
+  const uint64_t r256 = (t256 + cus - 1) / cus, r192 = (t192 + cus - 1) / cus;
+  return gemm_ring_192_ok(g) && r192 * 4 < r256 * 5 && (r192 <= r256 || t192 % 8 == 0);
 }
 
 bool gemm_rope_epilogue_ok(const LaunchCtx &lc, const GemmDesc &g) {
@@ -3538,15 +3541,19 @@ hipError_t launch_matmul(const LaunchCtx &lc_in, const GemmDesc &g, const char *
         // Tiles of 256 rows or of 128, by the rounds they take: a round of the large ones costs 1.4 to 1.7 rounds of the small (512 rows
         // by 2 x 8192, K = 2048, one round either way 56 and 40 us; 700 rows, one round or two, 50 and 60; 1024 rows by 2 x 5632 47 and
         // 60; 1500 rows, two or three, 92 and 84; 2900 by 2 x 8192, three or six, 159 and 181).  Fewer tiles of 128 than half the
-        // CUs: 64 or 32 output columns per tile.  A round of 192 rows is 0.8 to 0.92 of one of 256 (2 x 8192, K = 2048: 700 rows, one round
-        // either way, 49.0 and 44.6 us; 2100, three either way, 149 and 124; 2300 149 and 133) and 1.25 to 1.4 of one of 128 (1100, two or
-        // three, 89.3 and 78.5; 1459 98.8 and 88.3).  (Fewer k-steps than eight: not measured.)
+        // CUs: 64 or 32 output columns per tile.  A round of 192 rows is 0.74 to 0.92 of one of 256 (2 x 8192, K = 2048: 700 rows, one round
+        // either way, 50.0 and 43.4 us; 2100, three either way, 139 and 115; 8705 by 2 x 5632, 6.75 rounds' worth of 256 x 288 or eight, 329 and
+        // 311; 5153 by 2 x 8192, 5.6 or seven, 287 and 271) and 1.25 to 1.4 of one of 128 (1100 by 2 x 8192, two or three, 83.7 and 72.7).
+        // More rounds of them only where the grid is dealt to the XCDs in eight equal parts (TilePlace): 5900 by 2 x 6912, K = 1152, 5.6
+        // or seven, 171 and 185, 6144, the same rounds but a grid of 216 x 8, 171 and 168; 3585 by 2 x 11008, K = 4096, 518 and 571, 5985
+        // 806 and 779; as many rounds gain on any grid (1601 by 2 x 6912 67.7 and 54.0).  (Fewer k-steps than eight: not measured.)
         const uint64_t d256w = (uint64_t)((g.M + 255) / 256) * ((g.N + 143) / 144) * batch;
         const uint64_t cus = (uint64_t)lc.n_cus, r256 = (d256 + cus - 1) / cus, r128 = (d128 + cus - 1) / cus;
         const bool wide = wide_ahead(144, d256);
         const uint64_t large = wide ? (d256w + cus - 1) / cus * 9 : r256 * 8;  // (in eighths of a round of 256 rows)
-        const uint64_t r192 = ((uint64_t)((g.M + 191) / 192) * ((g.N + 127) / 128) * batch + cus - 1) / cus;
-        if (r192 * 32 < std::min(large * 5, r128 * 24) && g.K >= 512 && gemm_ring_192_ok(gg)) e = launch_gemm_ring(lc, gg, RING_192);
+        const uint64_t t192 = (uint64_t)((g.M + 191) / 192) * ((g.N + 127) / 128) * batch, r192 = (t192 + cus - 1) / cus;
+        if (r192 * 32 < std::min(large * 5, r128 * 24) && (r192 * 8 <= large || t192 % 8 == 0) && g.K >= 512 && gemm_ring_192_ok(gg))
+          e = launch_gemm_ring(lc, gg, RING_192);
         else if (large * 5 <= r128 * 24 && gemm_ring_ok(gg)) e = launch_gemm_ring(lc, gg, wide ? RING_288 : RING_256);
         else if (d128 * 4 <= cus)
           e = launch_gemm_dma<128, 64, 4, 1, true, 5, true, false, false, 2>(lc, gg, (uint32_t)((uint64_t)((g.M + 127) / 128) * ((g.N + 31) / 32) * batch));

@@ -401,13 +401,16 @@ for kernel, sizes in ((wide, {large.WIDE_GATED}), (tall, [(4096, 2048, 320)])):
 
 
 def test_tiles_of_192_x_256(fake_hip):  # noqa: F811
-    """Gate and up from eight k-steps on, and q / k / v, where 256 rows to a tile, or 128, put in as many rounds; the sizes of test_large_tiles.py."""
+    """Gate and up from eight k-steps on, and q / k / v, where 256 rows to a tile, or 128, put in as many rounds, or a few less and the grid is
+    dealt evenly; the sizes of test_large_tiles.py."""
     fake_hip(LAUNCHED + f"""
 sys.path.insert(0, "tests")
 import test_large_tiles as large
 short, ring = "gemm_bf16_ring_kernelILi%dELi2ELb0ELb1E", "gemm_bf16_ring_kernelILi%dE"
 for m, f, k, on in ((700, 8192, 512, True), (577, 7688, 576, True), (768, 6920, 640, True), (1153, 8200, 512, True), (2100, 8192, 2048, True),
-                    (700, 8192, 448, False), (512, 8192, 2048, False), (769, 8192, 2048, False), (2900, 8192, 2048, False)):
+                    (700, 8192, 448, False), (512, 8192, 2048, False), (769, 8192, 2048, False), (2900, 8192, 2048, False),
+                    # more rounds than on other tiles, a grid of a multiple of eight tiles and others; as many rounds
+                    (6144, 6912, 1152, True), (5900, 6912, 1152, False), (6208, 6912, 1152, False), (5153, 8192, 2048, True), (1601, 6912, 1152, True)):
     for kind, act in ((2, nn.silu), (3, nn.gelu)):
         (first, *_) = launched(lambda: run(lambda b, x, g, u, d: linear(b, act(b, linear(b, x, g, f, k)) * linear(b, x, u, f, k), d, 64, f),
                                            operand(1, m, k), operand(f, k), operand(f, k), operand(64, f)))
