@@ -1143,11 +1143,15 @@ bool moe_ring_ok(const MoeGemmDesc &g) {
 
 // The dense expert's tiles are dealt to the XCDs by whole columns, and the others even that out: there have to be enough of those (eight
 // columns' worth), and few enough of all for the products of their numbers.
+// Up to 3072 tokens: beyond, the routed experts' tiles wait for the matrix cores too, and 256 x 256 tiles are as fast for the dense one (24 layers
+// of 60 experts of 2 x 1408 x 2048 and 2048 x 1408, 4 to a token, a dense one of 5632, ms with it in launches of its own and in these: 660 tokens
+// 8.26, 7.52; 1024 10.5, 9.73; 1400 11.8, 10.96; 2048 15.3, 14.6; 2600 18.6, 18.2; 4096 24.9, 24.7; 6144 39.6, 39.6; 8192 48.3, 48.9; 16384 93.8
+// either way).
 bool moe_dense_ok(const MoeGemmDesc &g) {
   const auto &d = g.dense;
   const uint64_t bno = g.fuse_glu ? 128 : 256, rows = (g.S + 127) / 128, cols = (d.N + bno - 1) / bno, tiles_n = (g.prob[0].N + bno - 1) / bno;
   const uint64_t fewest = ((uint64_t)g.S * g.n_slot + 127) / 128 * tiles_n, most = moe_route_max_tiles(g) * tiles_n + rows * cols;
-  if (!d.N || !moe_ring_ok(g) || (!g.fuse_glu && g.n_prob != 1) || fewest < 8 * rows || most / 8 >= 65535 || rows * (cols / 8 + 1) >= 65535) return false;
+  if (!d.N || !moe_ring_ok(g) || g.S > 3072 || (!g.fuse_glu && g.n_prob != 1) || fewest < 8 * rows || most / 8 >= 65535 || rows * (cols / 8 + 1) >= 65535) return false;
   return d.N % 8 == 0 && d.K % 64 == 0 && d.K >= 192 && d.a16 && (uintptr_t)d.a16 % 16 == 0 && d.a_bs % 8 == 0 && (uintptr_t)d.w[0] % 16 == 0 &&
          (!g.fuse_glu || (uintptr_t)d.w[1] % 16 == 0) && d.sbn % 8 == 0 && d.sbn >= 0 && d.sbn <= (1 << 22) &&
          (g.fuse_glu ? d.h16 && (uintptr_t)d.h16 % 16 == 0 : d.c && (uintptr_t)d.c % 16 == 0);

@@ -565,3 +565,22 @@ graph(plain, x, idx, up[0])
 graph(matrices, x, idx, up[0])
 graph(whole, x, idx, *up, down)
 """, flags)
+
+
+def test_a_dense_expert_in_the_routed_experts_launches(fake_hip):  # noqa: F811
+    """Up to 3072 tokens; launches of its own beyond."""
+    fake_hip(LAUNCHED + """
+sys.path.insert(0, "tests")
+import test_dense_expert as dense
+e, f, h, fs = 5, 768, 1280, 320
+weights = [operand(*s) for s in ((e, f, h), (e, f, h), (e, h, f), (fs, h), (fs, h), (h, fs))]
+for s, joined in ((300, True), (3072, True), (3073, False)):
+    be.sync()
+    fake.fake_hip_launched()
+    term = type("Layer", (Term,), {"sort": lambda self: ([lang.TENSOR] * 8, [lang.TENSOR] * 2), "def_": lambda self, b, args: dense.layer("silu", 2, f, h, fs)(b, *args)})
+    for t in cg.Interpreter(be, cg.stdlib(), cg.Parameters()).run(term(8, None).term(), [operand(1, s, h), be.tensor(np.zeros((s, 2), np.uint32))] + weights):
+        be.realize(t)
+    be.sync()
+    names = [n for n in fake.fake_hip_launched().decode().split("\\n") if "gem" in n or "moe_ring" in n]
+    assert sum("moe_ring" in n for n in names) == 2 and (len(names) == 2) == joined, (s, names)
+""", BF16)
