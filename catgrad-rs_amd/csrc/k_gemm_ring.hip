@@ -260,8 +260,9 @@ static hipError_t whole_lds(const void *kernel, int bytes) {
 #define HON(x) x
 #define HOFF(x) ""
 #define HSYNC(v) "s_waitcnt vmcnt(" #v ")\n\ts_barrier\n\t"
-#define HSLICE(b, UB, ks, W, E0, E1, E2, E3) \
-  W PRODUCT(0, b, 0, 0, A0, UB, ks) E0 PRODUCT(0, b, 0, 1, A0, UB, ks) E1 PRODUCT(0, b, 1, 0, A0, UB, ks) E2 PRODUCT(0, b, 1, 1, A0, UB, ks) E3
+// (C: the accumulators, of a step's two phases alike)
+#define HSLICE(C, b, UB, ks, W, E0, E1, E2, E3) \
+  W PRODUCT(C, b, 0, 0, A0, UB, ks) E0 PRODUCT(C, b, 0, 1, A0, UB, ks) E1 PRODUCT(C, b, 1, 0, A0, UB, ks) E2 PRODUCT(C, b, 1, 1, A0, UB, ks) E3
 // s[58:59]: bytes from the step being requested to the next (KOrder::advance; s55 is its place in the order); the main loop finds the
 // next size out among its products
 #define HSTEP_A "s_xor_b32 s40, s55, %[flip]\n\ts_add_u32 s55, s55, 1\n\t"
@@ -269,27 +270,27 @@ static hipError_t whole_lds(const void *kernel, int bytes) {
 #define HSTEP_C "s_xor_b32 s41, s55, %[flip]\n\ts_sub_u32 s41, s41, s40\n\t"
 #define HSTEP_D(lo, hi) "s_lshl_b32 " lo ", s41, 7\n\ts_ashr_i32 " hi ", s41, 31\n\t"
 #define HSTEP_SIZE HSTEP_A HSTEP_B HSTEP_C HSTEP_D("s58", "s59")
-#define HPHASE0(G, v)                                                                                                              \
+#define HPHASE0(C, G, v)                                                                                                              \
   G("s_add_u32 s54, s53, %[lds]\n\t") HSYNC(v)                                                                                     \
   HFROM_A("s48", 3) HFROM_B("s50", 0)                                                                                              \
-  HSLICE(0, B0, 0, READS_BUT(8), HA(0, 3) G(HM0(0)), HA(1, 3) G(HLOAD_A(0)), HB1(0, 0), HB1(1, 0)) HFROM_B("s50", 1)          \
-  HSLICE(0, B0, 1, READS_BUT(8), HB1(0, 1) G(HM0(1)), HB1(1, 1) G(HLOAD_A(1)), "", "") HFROM_B("s50", 2)                          \
-  HSLICE(0, B0, 2, READS_BUT(6), HB1(0, 2) G(HM0(2)), HB1(1, 2) G(HLOAD_A(2)), "", "") HFROM_B("s50", 3)                          \
-  HSLICE(0, B0, 3, READS_BUT(6), HB1(0, 3) G(HM0(3)), HB1(1, 3) G(HLOAD_A(3)), "", "")
-#define HPHASE1(G, v, HINT)                                                                                                              \
+  HSLICE(C, 0, B0, 0, READS_BUT(8), HA(0, 3) G(HM0(0)), HA(1, 3) G(HLOAD_A(0)), HB1(0, 0), HB1(1, 0)) HFROM_B("s50", 1)          \
+  HSLICE(C, 0, B0, 1, READS_BUT(8), HB1(0, 1) G(HM0(1)), HB1(1, 1) G(HLOAD_A(1)), "", "") HFROM_B("s50", 2)                          \
+  HSLICE(C, 0, B0, 2, READS_BUT(6), HB1(0, 2) G(HM0(2)), HB1(1, 2) G(HLOAD_A(2)), "", "") HFROM_B("s50", 3)                          \
+  HSLICE(C, 0, B0, 3, READS_BUT(6), HB1(0, 3) G(HM0(3)), HB1(1, 3) G(HLOAD_A(3)), "", "")
+#define HPHASE1(C, G, v, HINT)                                                                                                              \
   G("s_add_u32 s54, s48, %[lds]\n\t") HSYNC(v)                                                                                     \
   HFROM_B("s52", 0)                                                                                                                \
-  HSLICE(1, B1, 0, READS_BUT(6), HB0(0, 0) G(HM0(0)), HB0(1, 0) G(LOAD_AS(B0, 0, HINT) HM0(1)), G(LOAD_AS(B0, 1, HINT)), G(HSTEP_A HSTEP_B)) \
+  HSLICE(C, 1, B1, 0, READS_BUT(6), HB0(0, 0) G(HM0(0)), HB0(1, 0) G(LOAD_AS(B0, 0, HINT) HM0(1)), G(LOAD_AS(B0, 1, HINT)), G(HSTEP_A HSTEP_B)) \
   HFROM_A("s51", 0) HFROM_B("s52", 1)                                                                                              \
-  HSLICE(1, B1, 1, READS_BUT(6), HB0(0, 1) G(HM0(2)), HB0(1, 1) G(LOAD_AS(B0, 2, HINT) HM0(3)), HA(0, 0) G(LOAD_AS(B0, 3, HINT)), HA(1, 0) G(HSTEP_C HSTEP_D("s56", "s57")))      \
+  HSLICE(C, 1, B1, 1, READS_BUT(6), HB0(0, 1) G(HM0(2)), HB0(1, 1) G(LOAD_AS(B0, 2, HINT) HM0(3)), HA(0, 0) G(LOAD_AS(B0, 3, HINT)), HA(1, 0) G(HSTEP_C HSTEP_D("s56", "s57")))      \
   HFROM_A("s51", 1) HFROM_B("s52", 2) G("s_add_u32 s54, s49, %[lds]\n\t")                                                          \
-  HSLICE(1, B1, 2, READS_BUT(8), HB0(0, 2) G(HM0(0)), HB0(1, 2) G(LOAD_AS(B1, 0, HINT) HM0(1)), HA(0, 1) G(LOAD_AS(B1, 1, HINT)), HA(1, 1))      \
+  HSLICE(C, 1, B1, 2, READS_BUT(8), HB0(0, 2) G(HM0(0)), HB0(1, 2) G(LOAD_AS(B1, 0, HINT) HM0(1)), HA(0, 1) G(LOAD_AS(B1, 1, HINT)), HA(1, 1))      \
   HFROM_A("s51", 2) HFROM_B("s52", 3)                                                                                              \
-  HSLICE(1, B1, 3, READS_BUT(10), HB0(0, 3) G(HM0(2)), HB0(1, 3) G(LOAD_AS(B1, 2, HINT) HM0(3)), HA(0, 2) G(LOAD_AS(B1, 3, HINT)), HA(1, 2))
+  HSLICE(C, 1, B1, 3, READS_BUT(10), HB0(0, 3) G(HM0(2)), HB0(1, 3) G(LOAD_AS(B1, 2, HINT) HM0(3)), HA(0, 2) G(LOAD_AS(B1, 3, HINT)), HA(1, 2))
 // (the last step's second phase reads and requests nothing)
-#define HLAST                                                                                                    \
-  HSLICE(1, B1, 0, READS_BUT(6), "", "", "", "") HSLICE(1, B1, 1, READS_BUT(4), "", "", "", "")                  \
-  HSLICE(1, B1, 2, READS_BUT(2), "", "", "", "") HSLICE(1, B1, 3, READS_BUT(0), "", "", "", "")
+#define HLAST(C)                                                                                                    \
+  HSLICE(C, 1, B1, 0, READS_BUT(6), "", "", "", "") HSLICE(C, 1, B1, 1, READS_BUT(4), "", "", "", "")                  \
+  HSLICE(C, 1, B1, 2, READS_BUT(2), "", "", "", "") HSLICE(C, 1, B1, 3, READS_BUT(0), "", "", "", "")
 #define HNEXT(x, y) "s_add_u32 " x ", " y ", 16384\n\ts_cmp_eq_u32 " x ", 163840\n\ts_cselect_b32 " x ", 0, " x "\n\t"
 #define HNEXT_PLACES \
   "s_mov_b32 s53, s50\n\ts_mov_b32 s48, s51\n\ts_mov_b32 s49, s52\n\t" HNEXT("s50", "s52") HNEXT("s51", "s50") HNEXT("s52", "s51")
@@ -305,18 +306,25 @@ static hipError_t whole_lds(const void *kernel, int bytes) {
 // steps 0 to 2 requested: 36 loads
 #define HFIRST_LOADS(HINT) HPOINTERS "s_mov_b32 s54, %[lds]\n\t" HSTEP_LOADS(HINT) HNEXT_STEP HSTEP_LOADS(HINT) HNEXT_STEP HSTEP_LOADS(HINT)
 // n >= 3 steps
-#define HMAIN_LOOP(HINT)                                                                                                              \
+#define HMAIN_START                                                                                                              \
   HPOINTERS HNEXT_STEP HNEXT_STEP HNEXT_STEP "s_sub_u32 s47, %[n], 3\n\t"                                                          \
   "s_mov_b32 s48, 0\n\ts_movk_i32 s49, 0x4000\n\ts_mov_b32 s50, 0x8000\n\ts_mov_b32 s51, 0xC000\n\ts_mov_b32 s52, 0x10000\n\t"  \
   "s_mov_b32 s53, 0x24000\n\t" HSYNC(28)                                                                                        \
   HFROM_A("s48", 0) HFROM_B("s49", 0) HB0(0, 0) HB0(1, 0) HFROM_B("s49", 1) HB0(0, 1) HB0(1, 1) HA(0, 0) HA(1, 0)           \
   HFROM_A("s48", 1) HFROM_B("s49", 2) HB0(0, 2) HB0(1, 2) HA(0, 1) HA(1, 1)                                                 \
   HFROM_A("s48", 2) HFROM_B("s49", 3) HB0(0, 3) HB0(1, 3) HA(0, 2) HA(1, 2)                                                 \
-  "s_cmp_eq_u32 s47, 0\n\ts_cbranch_scc1 2f\n\t"                                                                                \
-  "1:\n\t" HPHASE0(HON, 24) HPHASE1(HON, 20, HINT) HNEXT_B "s_mov_b64 s[58:59], s[56:57]\n\t" HNEXT_PLACES                                                             \
-  "s_sub_u32 s47, s47, 1\n\ts_cmp_lg_u32 s47, 0\n\ts_cbranch_scc1 1b\n\t"                                                       \
-  "2:\n\t" HPHASE0(HOFF, 24) HPHASE1(HOFF, 16, HINT) HNEXT_PLACES HPHASE0(HOFF, 12) HPHASE1(HOFF, 4, HINT) HNEXT_PLACES HPHASE0(HOFF, 0)    \
-  HLAST "s_nop 15\n\ts_nop 7\n\t"
+  "s_cmp_eq_u32 s47, 0\n\ts_cbranch_scc1 2f\n\t"
+#define HMAIN_STEP(C, HINT) \
+  HPHASE0(C, HON, 24) HPHASE1(C, HON, 20, HINT) HNEXT_B "s_mov_b64 s[58:59], s[56:57]\n\t" HNEXT_PLACES "s_sub_u32 s47, s47, 1\n\t"
+#define HMAIN_END(C0, C1, C2, HINT)                                                                                              \
+  "2:\n\t" HPHASE0(C0, HOFF, 24) HPHASE1(C0, HOFF, 16, HINT) HNEXT_PLACES HPHASE0(C1, HOFF, 12) HPHASE1(C1, HOFF, 4, HINT)        \
+  HNEXT_PLACES HPHASE0(C2, HOFF, 0) HLAST(C2) "s_nop 15\n\ts_nop 7\n\t"
+#define HMAIN_LOOP(HINT) \
+  HMAIN_START "1:\n\t" HMAIN_STEP(0, HINT) "s_cmp_lg_u32 s47, 0\n\ts_cbranch_scc1 1b\n\t" HMAIN_END(0, 0, 0, HINT)
+// ... every other step in accumulators of its own (an odd number in front of the last three starts with the second of a pair)
+#define HMAIN_LOOP_2(HINT)                                                                                                       \
+  HMAIN_START "s_bitcmp1_b32 s47, 0\n\ts_cbranch_scc1 3f\n\t" "1:\n\t" HMAIN_STEP(1, HINT) "3:\n\t" HMAIN_STEP(0, HINT)          \
+  "s_cmp_lg_u32 s47, 0\n\ts_cbranch_scc1 1b\n\t" HMAIN_END(1, 0, 1, HINT)
 
 // ---- tiles of 256 x 288: the four quadrants and a strip X of 32 columns more, a ninth of the products with no wavefront idle: in each
 // half of A a wavefront multiplies its first row block - rows wn * 32 of its 64, so that the two wavefronts of the same rows share
@@ -948,6 +956,8 @@ __global__ void __launch_bounds__(256, 1) gemm_bf16_ring_kernel(GemmDesc g) {
 //   * The row tiles of a crowded expert stand next to each other (2048 tokens, both launches with the dense expert 440 -> 424 us, 4096 708
 //     -> 677, 1024 in crowded experts 301 -> 293; by expert and row tile before).
 //   * A loop over tiles that requests the next one's first steps in front of the stores of this one: no change (217 and 216 us).
+// A dense expert's down_proj is deep, and in slices of k by itself: every other step of it has accumulators of its own, so that its sums
+// are no longer chains than in two slices (5632 values off by 3.24e-7 of the 64-bit sum, in one chain 4.69e-7; the same time).
 enum { MOE_PLAIN, MOE_SILU, MOE_GELU };
 template <int KIND>
 __global__ void __launch_bounds__(256, 1) moe_ring_kernel(MoeGemmDesc g) {
@@ -1042,7 +1052,7 @@ __global__ void __launch_bounds__(256, 1) moe_ring_kernel(MoeGemmDesc g) {
   const uint64_t base = out + ((ent[4] >> 16) * g.out_slot + (ent[4] & 0xFFFFu) * (uint64_t)N) * (GATED ? 2 : 4);
   float zero;
   asm volatile("v_mov_b32 %0, 0" : "=v"(zero));
-  f32x16 acc[1][2][2][2];  // [0][B half][row block][column block]
+  f32x16 acc[GATED ? 1 : 2][2][2][2];  // [0, or every other step's][B half][row block][column block]
 #pragma unroll
   for (int q = 0; q < 8; ++q)
 #pragma unroll
@@ -1055,10 +1065,23 @@ __global__ void __launch_bounds__(256, 1) moe_ring_kernel(MoeGemmDesc g) {
     ra[ks] = wm * 8192 + p;
     rb[ks] = wn * 8192 + p;
   }
-  if (once)
+  if (once) {
     asm volatile(HMAIN_LOOP(" nt") : RING_ACC0, RING_PLACES, RING_GATHERED : MOE_IN, RING_ORDER : RING_SCALARS, RING_HALF_SCALARS, RING_FRAGMENTS);
-  else
+  } else if (!GATED && dense) {
+    if constexpr (!GATED) {
+#pragma unroll
+      for (int q = 0; q < 8; ++q)
+#pragma unroll
+        for (int k = 0; k < 16; ++k) acc[1][q >> 2][(q >> 1) & 1][q & 1][k] = zero;
+      asm volatile(HMAIN_LOOP_2("") : RING_ACC0, RING_ACC1, RING_PLACES, RING_GATHERED : MOE_IN, RING_ORDER : RING_SCALARS, RING_HALF_SCALARS, RING_FRAGMENTS);
+#pragma unroll
+      for (int q = 0; q < 8; ++q)
+#pragma unroll
+        for (int k = 0; k < 16; ++k) acc[0][q >> 2][(q >> 1) & 1][q & 1][k] += acc[1][q >> 2][(q >> 1) & 1][q & 1][k];
+    }
+  } else {
     asm volatile(HMAIN_LOOP("") : RING_ACC0, RING_PLACES, RING_GATHERED : MOE_IN, RING_ORDER : RING_SCALARS, RING_HALF_SCALARS, RING_FRAGMENTS);
+  }
   // Rows back to their slot and token, through 4 KB of LDS of each wavefront's own: 32 rows of 64 bf16 or of 32 f32 values at a time, of
   // which eight lanes store a line.  A lane knows where the row of its number goes, and hands that to the eight.
   __syncthreads();  // every wavefront has read its last fragments

@@ -83,3 +83,28 @@ def test_the_same_bits_wherever_a_pair_lies(hip_bf16, S, F, H, FS):
         assert np.array_equal(r, routed) and np.array_equal(d, dense), again
         order = g.permutation(S)
         assert np.array_equal(run(order)[0], routed[order]), again
+
+
+# The dense expert's down_proj on operands that are known exactly: gates of 64 (whose silu is 64 to the last bit) and up projections that pick
+# a value of the token.  A sum of random terms in chains of n additions is off by 0.42 2^-24 sqrt(n / 2) - a rounding is 0.42 2^-24 of the
+# partial sum, whose square grows evenly -, and an MFMA makes two additions for 16 values: 3.3e-7 for 5632 values in two chains, which is what
+# they were in two slices, 4.7e-7 in one.
+@pytest.mark.gpu
+@pytest.mark.parametrize("S,FS", [(300, 5632), (300, 5696), (131, 2816)])
+def test_the_sums_of_a_deep_down_projection(hip_bf16, S, FS):
+    E, k, F, H = 5, 2, 768, 2048
+    g = np.random.default_rng(FS)
+    x = large.draw(g, (1, S, H))
+    x[..., 0] = 1
+    idx = np.stack([g.choice(np.array([0, 2, 3]), S), np.full(S, 4)], 1).astype(np.uint32)
+    routed = [large.draw(g, s, s[-1] ** -0.5) for s in ((E, F, H), (E, F, H), (E, H, F))]
+    sg, su, pick = np.zeros((FS, H), np.float32), np.zeros((FS, H), np.float32), g.integers(1, H, FS)
+    sg[:, 0], su[np.arange(FS), pick] = 64, 1
+    sd = large.draw(g, (H, FS), FS ** -0.5)
+    hip_bf16.launch_counts(reset=True)
+    _, dense = vectors.run(hip_bf16, layer("silu", k, F, H, FS), 2, x, idx, *routed, sg, su, sd)
+    counts = hip_bf16.launch_counts()
+    assert counts["gemm_experts_bf16"] == 2 and "gemm" not in counts, counts
+    ref = 64 * x[0][:, pick].astype(np.float64) @ sd.T.astype(np.float64)
+    off = np.linalg.norm(dense[0] - ref) / np.linalg.norm(ref)
+    assert off <= 1.15 * 0.42 * 2.0 ** -24 * np.sqrt(FS / 16 / 2), off
