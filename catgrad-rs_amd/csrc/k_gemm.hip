@@ -2605,8 +2605,7 @@ hipError_t launch_moe_route(const LaunchCtx &lc, const MoeGemmDesc &g, uint32_t 
   return hipGetLastError();
 }
 
-// A workgroup owns (128 output columns of NP problems, one expert) and walks that expert's pairs 128
-// at a time.  Token rows (gathered through the sorted list, bf16) and weight rows travel to LDS with
+// A workgroup owns (128 output columns of NP problems, a row tile of one expert's pairs).  Token rows (gathered through the sorted list, bf16) and weight rows travel to LDS with
 // global_load_lds_dwordx4 exactly as in gemm_bf16_dma_kernel - same 1 KB wave loads, same XOR
 // swizzle, NS stages in flight - so a k-step no longer waits out a trip to memory.  Wavefront w
 // computes columns [32 w, 32 w + 32) of every 32-row tile that has a live row.
@@ -2636,17 +2635,10 @@ __global__ void __launch_bounds__(256) moe_gemm_dma_kernel(MoeGemmDesc g) {
   // consecutive workgroups (dealt round-robin to the 8 XCDs) take the column tiles of one expert: giving an
   // XCD a contiguous range of experts instead measured 10 % slower
   const uint32_t id = blockIdx.x;
-  uint32_t e = id / tiles_n, m_first = 0, m_last = UINT32_MAX;
-  const uint32_t n0 = (id - e * tiles_n) * BN_;
-  if (g.route_tiles) {  // one row tile of one expert
-    if (e >= g.route_tiles[0]) return;  // the grid is sized for the most tiles there can be
-    const uint32_t ent = g.route_tiles[1 + e];
-    e = moe_entry_expert(ent);
-    m_first = moe_entry_row(ent) * PAIRS;
-    m_last = m_first + PAIRS;
-  }
-  if (e >= g.n_expert) return;  // the grid is sized for the wider problem
-  const uint32_t cnt = min(g.route_count[e], m_last);
+  const uint32_t tile = id / tiles_n, n0 = (id - tile * tiles_n) * BN_;
+  if (tile >= g.route_tiles[0]) return;  // the grid is sized for the most row tiles there can be, and the wider problem
+  const uint32_t entry = g.route_tiles[1 + tile], e = moe_entry_expert(entry), m0 = moe_entry_row(entry) * PAIRS;
+  const uint32_t cnt = min(g.route_count[e], m0 + PAIRS);
   const uint32_t *list = g.route_list + g.route_offset[e];
   const uint16_t *W[NP];
   int64_t sbn[NP];
@@ -2658,209 +2650,202 @@ __global__ void __launch_bounds__(256) moe_gemm_dma_kernel(MoeGemmDesc g) {
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint16_t *)dma_smem;
   const int sw = (lane >> 1) & 7, half = lane >> 5;
   const int n_steps = (int)(K / BK);
-  const KOrder first_order(g.k_rotate, e * tiles_n + n0 / BN_, (uint32_t)n_steps);
+  KOrder order(g.k_rotate, e * tiles_n + n0 / BN_, (uint32_t)n_steps);
   const int64_t plane = PLANES ? (int64_t)g.S * K : 0;
-  for (uint32_t m0 = m_first; m0 < cnt; m0 += PAIRS) {
-    const int live_tiles = (int)min((uint32_t)MT, (cnt - m0 + TPAIRS - 1) / TPAIRS);  // wave-uniform
-    KOrder order = first_order;
-    f32x16 acc[NP][MT], run[PLANES ? NP : 1][PLANES ? MT : 1];  // run: the sum over the k-steps so far
+  const int live_tiles = (int)min((uint32_t)MT, (cnt - m0 + TPAIRS - 1) / TPAIRS);  // wave-uniform
+  f32x16 acc[NP][MT], run[PLANES ? NP : 1][PLANES ? MT : 1];  // run: the sum over the k-steps so far
 #pragma unroll
-    for (int p = 0; p < NP; ++p)
+  for (int p = 0; p < NP; ++p)
 #pragma unroll
-      for (int h = 0; h < MT; ++h)
+    for (int h = 0; h < MT; ++h)
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-          acc[p][h][i] = 0.f;
-          if constexpr (PLANES) run[p][h][i] = 0.f;
+      for (int i = 0; i < 16; ++i) {
+        acc[p][h][i] = 0.f;
+        if constexpr (PLANES) run[p][h][i] = 0.f;
+      }
+  // Load i of a wave: i < MT: its eight rows of the i-th 32-row tile of token rows (not made when no pair is in
+  // that tile: an expert of a few pairs moves its weights and 32 rows, not 128), then its share of the weight rows.
+  const uint16_t *gp[LPW];  // per-lane source; advances by BK per stage
+  auto block_of = [&](int i) { return i < MT ? i * 4 + wave : BM_ / 8 + wave * (LPW - MT) + i - MT; };  // 8-row block of the stacked tile
+#pragma unroll
+  for (int i = 0; i < LPW; ++i) {
+    const int q = block_of(i);
+    const int R = q * 8 + (lane >> 3);
+    const int c = (lane & 7) ^ ((R >> 1) & 7);
+    if (i < MT) {
+      // rows past the expert's last pair repeat it: loaded, multiplied, never stored
+      const int part = PLANES ? min((R & 31) / TPAIRS, 2) : 0, pair = PLANES ? (R >> 5) * TPAIRS + (R & 31) % TPAIRS : R;
+      const uint32_t ent = list[min(m0 + (uint32_t)pair, cnt - 1)], sl = ent >> 16, tok = ent & 0xFFFFu;
+      const uint16_t *rows = g.slot[0].a16;
+      int64_t bs = g.slot[0].a_bs;
+#pragma unroll
+      for (int s = 1; s < 8; ++s)
+        if (sl == (uint32_t)s) {
+          rows = g.slot[s].a16;
+          bs = g.slot[s].a_bs;
         }
-    // Load i of a wave: i < MT: its eight rows of the i-th 32-row tile of token rows (not made when no pair is in
-    // that tile: an expert of a few pairs moves its weights and 32 rows, not 128), then its share of the weight rows.
-    const uint16_t *gp[LPW];  // per-lane source; advances by BK per stage
-    auto block_of = [&](int i) { return i < MT ? i * 4 + wave : BM_ / 8 + wave * (LPW - MT) + i - MT; };  // 8-row block of the stacked tile
+      gp[i] = rows + part * plane + (int64_t)tok * bs + order.step() * BK + c * 8;
+    } else {
+      const int rb = R - BM_, p = rb / BN_, col = rb - p * BN_;
+      gp[i] = W[p < NP ? p : 0] + (int64_t)min(n0 + (uint32_t)col, N - 1) * sbn[p < NP ? p : 0] + order.step() * BK + c * 8;
+    }
+  }
+  auto issue = [&](int buf) {
+    const int64_t to_next = (int64_t)order.advance() * BK;
 #pragma unroll
     for (int i = 0; i < LPW; ++i) {
-      const int q = block_of(i);
-      const int R = q * 8 + (lane >> 3);
-      const int c = (lane & 7) ^ ((R >> 1) & 7);
-      if (i < MT) {
-        // rows past the expert's last pair repeat it: loaded, multiplied, never stored
-        const int part = PLANES ? min((R & 31) / TPAIRS, 2) : 0, pair = PLANES ? (R >> 5) * TPAIRS + (R & 31) % TPAIRS : R;
-        const uint32_t ent = list[min(m0 + (uint32_t)pair, cnt - 1)], sl = ent >> 16, tok = ent & 0xFFFFu;
-        const uint16_t *rows = g.slot[0].a16;
-        int64_t bs = g.slot[0].a_bs;
-#pragma unroll
-        for (int s = 1; s < 8; ++s)
-          if (sl == (uint32_t)s) {
-            rows = g.slot[s].a16;
-            bs = g.slot[s].a_bs;
-          }
-        gp[i] = rows + part * plane + (int64_t)tok * bs + order.step() * BK + c * 8;
-      } else {
-        const int rb = R - BM_, p = rb / BN_, col = rb - p * BN_;
-        gp[i] = W[p < NP ? p : 0] + (int64_t)min(n0 + (uint32_t)col, N - 1) * sbn[p < NP ? p : 0] + order.step() * BK + c * 8;
-      }
+      if (i >= MT) lds_dma16_stream(gp[i], lds0 + buf * STAGE + block_of(i) * 1024);
+      else if (i < live_tiles) lds_dma16(gp[i], lds0 + buf * STAGE + block_of(i) * 1024);
+      gp[i] += to_next;
     }
-    auto issue = [&](int buf) {
-      const int64_t to_next = (int64_t)order.advance() * BK;
+  };
+  auto compute = [&](int buf) {
+    const uint16_t *As = dma_smem + buf * (STAGE / 2), *Bs = As + BM_ * BK;
+    bf16x8 af[2][MT], bfr[2][NP];
+    auto frags = [&](int ks, int set) {
+      const int o = ((ks * 2 + half) ^ sw) * 8;
 #pragma unroll
-      for (int i = 0; i < LPW; ++i) {
-        if (i >= MT) lds_dma16_stream(gp[i], lds0 + buf * STAGE + block_of(i) * 1024);
-        else if (i < live_tiles) lds_dma16(gp[i], lds0 + buf * STAGE + block_of(i) * 1024);
-        gp[i] += to_next;
-      }
+      for (int h = 0; h < MT; ++h)
+        if (h < live_tiles) af[set][h] = *(const bf16x8 *)(&As[(h * 32 + (lane & 31)) * BK + o]);
+#pragma unroll
+      for (int p = 0; p < NP; ++p) bfr[set][p] = *(const bf16x8 *)(&Bs[(p * BN_ + wave * 32 + (lane & 31)) * BK + o]);
     };
-    auto compute = [&](int buf) {
-      const uint16_t *As = dma_smem + buf * (STAGE / 2), *Bs = As + BM_ * BK;
-      bf16x8 af[2][MT], bfr[2][NP];
-      auto frags = [&](int ks, int set) {
-        const int o = ((ks * 2 + half) ^ sw) * 8;
+    frags(0, 0);
 #pragma unroll
-        for (int h = 0; h < MT; ++h)
-          if (h < live_tiles) af[set][h] = *(const bf16x8 *)(&As[(h * 32 + (lane & 31)) * BK + o]);
+    for (int ks = 0; ks < BK / 16; ++ks) {
+      if (ks + 1 < BK / 16) frags(ks + 1, (ks + 1) & 1);
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int p = 0; p < NP; ++p) bfr[set][p] = *(const bf16x8 *)(&Bs[(p * BN_ + wave * 32 + (lane & 31)) * BK + o]);
-      };
-      frags(0, 0);
+      for (int h = 0; h < MT; ++h)
+        if (h < live_tiles)
 #pragma unroll
-      for (int ks = 0; ks < BK / 16; ++ks) {
-        if (ks + 1 < BK / 16) frags(ks + 1, (ks + 1) & 1);
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int h = 0; h < MT; ++h)
-          if (h < live_tiles)
-#pragma unroll
-            for (int p = 0; p < NP; ++p)
-              acc[p][h] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[ks & 1][h], bfr[ks & 1][p], acc[p][h], 0, 0, 0);
-        __builtin_amdgcn_sched_barrier(0);
-      }
-      if constexpr (PLANES) {
-#pragma unroll
-        for (int p = 0; p < NP; ++p)
-#pragma unroll
-          for (int h = 0; h < MT; ++h)
-#pragma unroll
-            for (int i = 0; i < 16; ++i) {
-              run[p][h][i] += acc[p][h][i];
-              acc[p][h][i] = 0.f;
-            }
-      }
-    };
-#pragma unroll
-    for (int s0 = 0; s0 < NS - 1; ++s0)
-      if (s0 < n_steps) issue(s0);
-    for (int step = 0; step < n_steps; ++step) {
-      // (a stage is as many loads as there are weight pieces and live row tiles)
-      if (step + NS - 1 > n_steps || NS == 2) wait_vmcnt<0>();
-      else if (live_tiles == 1) wait_vmcnt<(NS - 2) * (LPW - MT + 1)>();
-      else if (live_tiles == 2) wait_vmcnt<(NS - 2) * (LPW - MT + 2)>();
-      else if (live_tiles == 3) wait_vmcnt<(NS - 2) * (LPW - MT + 3)>();
-      else wait_vmcnt<(NS - 2) * LPW>();
-      __syncthreads();
-      if (step + NS - 1 < n_steps) issue((step + NS - 1) % NS);
-      compute(step % NS);
+          for (int p = 0; p < NP; ++p)
+            acc[p][h] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[ks & 1][h], bfr[ks & 1][p], acc[p][h], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
     }
-    // ---- rows back to their slot and token.  Register i of tile h is row
-    // h * 32 + (i >> 2) * 8 + (lane >> 5) * 4 + (i & 3), column lane & 31.  The tile is staged in LDS
-    // (the operand stages are free now) so that a row leaves as 16-byte pieces: f32 for a plain
-    // product, bf16 act(gate) * up for the fused pair.
-    __syncthreads();  // every wave is done reading the last stage
     if constexpr (PLANES) {
-      constexpr int P = BN_ + 4;
-      float *T = (float *)dma_smem;
 #pragma unroll
       for (int p = 0; p < NP; ++p)
 #pragma unroll
         for (int h = 0; h < MT; ++h)
 #pragma unroll
-          for (int i = 0; i < 16; ++i)
-            T[(p * BM_ + h * 32 + (i >> 2) * 8 + (lane >> 5) * 4 + (i & 3)) * P + wave * 32 + (lane & 31)] = run[p][h][i];
-      __syncthreads();
-      const uint32_t pairs_here = min((uint32_t)PAIRS, cnt - m0);
-      for (uint32_t idx = tid; idx < pairs_here * (BN_ / 4); idx += 256) {
-        const uint32_t j = idx / (BN_ / 4), c = (idx - j * (BN_ / 4)) * 4;
-        if (n0 + c >= N) continue;
-        const uint32_t ent = list[m0 + j], sl = ent >> 16;
-        const uint64_t at = (uint64_t)(ent & 0xFFFFu) * N + n0 + c;
-        float4 v[NP];
-#pragma unroll
-        for (int p = 0; p < NP; ++p) {  // the parts' products, the smallest first
-          const float *t = T + (p * BM_ + j / TPAIRS * 32 + j % TPAIRS) * P + c;
-          const float4 hi = *(const float4 *)t, mid = *(const float4 *)(t + TPAIRS * P), lo = *(const float4 *)(t + 2 * TPAIRS * P);
-          v[p] = make_float4((lo.x + mid.x) + hi.x, (lo.y + mid.y) + hi.y, (lo.z + mid.z) + hi.z, (lo.w + mid.w) + hi.w);
-        }
-        if constexpr (NP == 2) {
-          auto act = [&](float x) { return g.fuse_glu == PRO_GEGLU ? gelu_ref(x) : x * sigmoid_ref(x); };
-          uint16_t *out = g.slot[0].h16;
-#pragma unroll
-          for (int s2 = 1; s2 < 8; ++s2)
-            if (sl == (uint32_t)s2) out = g.slot[s2].h16;
-          bf16_planes4(make_float4(act(v[0].x) * v[1].x, act(v[0].y) * v[1].y, act(v[0].z) * v[1].z, act(v[0].w) * v[1].w), out + at,
-                       (uint64_t)g.S * N);
-        } else {
-          float *out = g.slot[0].c[prob];
-#pragma unroll
-          for (int s2 = 1; s2 < 8; ++s2)
-            if (sl == (uint32_t)s2) out = g.slot[s2].c[prob];
-          *(float4 *)(out + at) = v[0];
-        }
-      }
-      wait_vmcnt<0>();
-      __syncthreads();
-      continue;
-    }
-    constexpr int TP = NP == 2 ? BN_ + 8 : BN_ + 4;  // row pitch in elements (keeps 16-byte alignment)
-    if (NP == 2) {
-      uint16_t *T = dma_smem;
-#pragma unroll
-      for (int h = 0; h < MT; ++h)
-        if (h < live_tiles)
-#pragma unroll
           for (int i = 0; i < 16; ++i) {
-            const float gt = acc[0][h][i];
-            const float hv = (g.fuse_glu == PRO_GEGLU ? gelu_fast(gt) : silu_fast(gt)) * acc[NP - 1][h][i];  // (leaves as bf16)
-            T[(h * 32 + (i >> 2) * 8 + (lane >> 5) * 4 + (i & 3)) * TP + wave * 32 + (lane & 31)] = (uint16_t)bf16_bits(hv);
+            run[p][h][i] += acc[p][h][i];
+            acc[p][h][i] = 0.f;
           }
-    } else {
-      float *T = (float *)dma_smem;
+    }
+  };
+#pragma unroll
+  for (int s0 = 0; s0 < NS - 1; ++s0)
+    if (s0 < n_steps) issue(s0);
+  for (int step = 0; step < n_steps; ++step) {
+    // (a stage is as many loads as there are weight pieces and live row tiles)
+    if (step + NS - 1 > n_steps || NS == 2) wait_vmcnt<0>();
+    else if (live_tiles == 1) wait_vmcnt<(NS - 2) * (LPW - MT + 1)>();
+    else if (live_tiles == 2) wait_vmcnt<(NS - 2) * (LPW - MT + 2)>();
+    else if (live_tiles == 3) wait_vmcnt<(NS - 2) * (LPW - MT + 3)>();
+    else wait_vmcnt<(NS - 2) * LPW>();
+    __syncthreads();
+    if (step + NS - 1 < n_steps) issue((step + NS - 1) % NS);
+    compute(step % NS);
+  }
+  // ---- rows back to their slot and token.  Register i of tile h is row
+  // h * 32 + (i >> 2) * 8 + (lane >> 5) * 4 + (i & 3), column lane & 31.  The tile is staged in LDS
+  // (the operand stages are free now) so that a row leaves as 16-byte pieces: f32 for a plain
+  // product, bf16 act(gate) * up for the fused pair.
+  __syncthreads();  // every wave is done reading the last stage
+  if constexpr (PLANES) {
+    constexpr int P = BN_ + 4;
+    float *T = (float *)dma_smem;
+#pragma unroll
+    for (int p = 0; p < NP; ++p)
 #pragma unroll
       for (int h = 0; h < MT; ++h)
-        if (h < live_tiles)
 #pragma unroll
-          for (int i = 0; i < 16; ++i)
-            T[(h * 32 + (i >> 2) * 8 + (lane >> 5) * 4 + (i & 3)) * TP + wave * 32 + (lane & 31)] = acc[0][h][i];
-    }
+        for (int i = 0; i < 16; ++i)
+          T[(p * BM_ + h * 32 + (i >> 2) * 8 + (lane >> 5) * 4 + (i & 3)) * P + wave * 32 + (lane & 31)] = run[p][h][i];
     __syncthreads();
-    {
-      constexpr int EPV = NP == 2 ? 8 : 4;        // elements per 16-byte piece
-      constexpr int PPR = BN_ / EPV;              // pieces per row
-      const uint32_t rows_here = min((uint32_t)BM_, cnt - m0);
-      for (uint32_t idx = tid; idx < rows_here * PPR; idx += 256) {
-        const uint32_t r = idx / PPR, c = (idx - r * PPR) * EPV;
-        if (n0 + c >= N) continue;  // N % 8 == 0: a piece is inside or outside
-        const uint32_t ent = list[m0 + r], sl = ent >> 16;
-        const uint64_t at = (uint64_t)(ent & 0xFFFFu) * N + n0 + c;
-        if (NP == 2) {
-          uint16_t *out = g.slot[0].h16;
+    const uint32_t pairs_here = min((uint32_t)PAIRS, cnt - m0);
+    for (uint32_t idx = tid; idx < pairs_here * (BN_ / 4); idx += 256) {
+      const uint32_t j = idx / (BN_ / 4), c = (idx - j * (BN_ / 4)) * 4;
+      if (n0 + c >= N) continue;
+      const uint32_t ent = list[m0 + j], sl = ent >> 16;
+      const uint64_t at = (uint64_t)(ent & 0xFFFFu) * N + n0 + c;
+      float4 v[NP];
 #pragma unroll
-          for (int s2 = 1; s2 < 8; ++s2)
-            if (sl == (uint32_t)s2) out = g.slot[s2].h16;
-          *(uint4 *)(out + at) = *(const uint4 *)(dma_smem + r * TP + c);
-        } else {
-          float *out = g.slot[0].c[prob];
+      for (int p = 0; p < NP; ++p) {  // the parts' products, the smallest first
+        const float *t = T + (p * BM_ + j / TPAIRS * 32 + j % TPAIRS) * P + c;
+        const float4 hi = *(const float4 *)t, mid = *(const float4 *)(t + TPAIRS * P), lo = *(const float4 *)(t + 2 * TPAIRS * P);
+        v[p] = make_float4((lo.x + mid.x) + hi.x, (lo.y + mid.y) + hi.y, (lo.z + mid.z) + hi.z, (lo.w + mid.w) + hi.w);
+      }
+      if constexpr (NP == 2) {
+        auto act = [&](float x) { return g.fuse_glu == PRO_GEGLU ? gelu_ref(x) : x * sigmoid_ref(x); };
+        uint16_t *out = g.slot[0].h16;
 #pragma unroll
-          for (int s2 = 1; s2 < 8; ++s2)
-            if (sl == (uint32_t)s2) out = g.slot[s2].c[prob];
-          *(float4 *)(out + at) = *(const float4 *)((const float *)dma_smem + r * TP + c);
-        }
+        for (int s2 = 1; s2 < 8; ++s2)
+          if (sl == (uint32_t)s2) out = g.slot[s2].h16;
+        bf16_planes4(make_float4(act(v[0].x) * v[1].x, act(v[0].y) * v[1].y, act(v[0].z) * v[1].z, act(v[0].w) * v[1].w), out + at,
+                     (uint64_t)g.S * N);
+      } else {
+        float *out = g.slot[0].c[prob];
+#pragma unroll
+        for (int s2 = 1; s2 < 8; ++s2)
+          if (sl == (uint32_t)s2) out = g.slot[s2].c[prob];
+        *(float4 *)(out + at) = v[0];
       }
     }
-    wait_vmcnt<0>();
-    __syncthreads();  // the stages are refilled for the next 128 pairs
+    return;
+  }
+  constexpr int TP = NP == 2 ? BN_ + 8 : BN_ + 4;  // row pitch in elements (keeps 16-byte alignment)
+  if (NP == 2) {
+    uint16_t *T = dma_smem;
+#pragma unroll
+    for (int h = 0; h < MT; ++h)
+      if (h < live_tiles)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          const float gt = acc[0][h][i];
+          const float hv = (g.fuse_glu == PRO_GEGLU ? gelu_fast(gt) : silu_fast(gt)) * acc[NP - 1][h][i];  // (leaves as bf16)
+          T[(h * 32 + (i >> 2) * 8 + (lane >> 5) * 4 + (i & 3)) * TP + wave * 32 + (lane & 31)] = (uint16_t)bf16_bits(hv);
+        }
+  } else {
+    float *T = (float *)dma_smem;
+#pragma unroll
+    for (int h = 0; h < MT; ++h)
+      if (h < live_tiles)
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+          T[(h * 32 + (i >> 2) * 8 + (lane >> 5) * 4 + (i & 3)) * TP + wave * 32 + (lane & 31)] = acc[0][h][i];
+  }
+  __syncthreads();
+  {
+    constexpr int EPV = NP == 2 ? 8 : 4;        // elements per 16-byte piece
+    constexpr int PPR = BN_ / EPV;              // pieces per row
+    const uint32_t rows_here = min((uint32_t)BM_, cnt - m0);
+    for (uint32_t idx = tid; idx < rows_here * PPR; idx += 256) {
+      const uint32_t r = idx / PPR, c = (idx - r * PPR) * EPV;
+      if (n0 + c >= N) continue;  // N % 8 == 0: a piece is inside or outside
+      const uint32_t ent = list[m0 + r], sl = ent >> 16;
+      const uint64_t at = (uint64_t)(ent & 0xFFFFu) * N + n0 + c;
+      if (NP == 2) {
+        uint16_t *out = g.slot[0].h16;
+#pragma unroll
+        for (int s2 = 1; s2 < 8; ++s2)
+          if (sl == (uint32_t)s2) out = g.slot[s2].h16;
+        *(uint4 *)(out + at) = *(const uint4 *)(dma_smem + r * TP + c);
+      } else {
+        float *out = g.slot[0].c[prob];
+#pragma unroll
+        for (int s2 = 1; s2 < 8; ++s2)
+          if (sl == (uint32_t)s2) out = g.slot[s2].c[prob];
+        *(float4 *)(out + at) = *(const float4 *)((const float *)dma_smem + r * TP + c);
+      }
+    }
   }
 }
 
 bool moe_gemm_pipelined_ok(const MoeGemmDesc &g) {
-  if (!g.route_count || !g.route_offset || !g.route_list || g.K % 64 || g.K < 64 || g.pro != PRO_NONE) return false;
+  if (!g.route_count || !g.route_offset || !g.route_list || !g.route_tiles || g.K % 64 || g.K < 64 || g.pro != PRO_NONE) return false;
   for (uint32_t s = 0; s < g.n_slot; ++s)
     if (!g.slot[s].a16 || (uintptr_t)g.slot[s].a16 % 16 || g.slot[s].a_bs % 8) return false;
   for (uint32_t p = 0; p < g.n_prob; ++p)
@@ -2904,18 +2889,18 @@ hipError_t launch_moe_gemm(const LaunchCtx &lc, const MoeGemmDesc &given) {
     if (!moe_gemm_pipelined_ok(g) || (g.fuse_glu ? g.n_prob != 2 || g.prob[0].N != g.prob[1].N : g.n_prob != 1)) return hipErrorInvalidValue;
     for (uint32_t s = 0; s < g.n_slot; ++s)
       if (g.slot[s].a_bs != (int64_t)g.K) return hipErrorInvalidValue;
-    const dim3 grid((max_n + 127) / 128 * (g.route_tiles ? moe_route_max_tiles(g) : g.n_expert), 1, 1);
+    const dim3 grid((max_n + 127) / 128 * moe_route_max_tiles(g), 1, 1);
     return g.fuse_glu ? launch_moe_gemm_dma<2, 3, true>(lc, g, grid) : launch_moe_gemm_dma<1, 3, true>(lc, g, grid);
   }
   if (moe_ring_ok(g)) return launch_moe_ring(lc, g);
   if (g.fuse_glu) {
     if (g.n_prob != 2 || g.prob[0].N != g.prob[1].N || g.pro != PRO_NONE) return hipErrorInvalidValue;
     if (moe_gemm_pipelined_ok(g))
-      return launch_moe_gemm_dma<2, 3>(lc, g, dim3((max_n + 127) / 128 * (g.route_tiles ? moe_route_max_tiles(g) : g.n_expert), 1, 1));
+      return launch_moe_gemm_dma<2, 3>(lc, g, dim3((max_n + 127) / 128 * moe_route_max_tiles(g), 1, 1));
     dim3 grid((max_n + 127) / 128, g.n_expert, 1);
     CG_LAUNCH(lc, moe_gemm_kernel<2>, grid, 256, g);
   } else if (moe_gemm_pipelined_ok(g)) {
-    return launch_moe_gemm_dma<1, 2>(lc, g, dim3((max_n + 127) / 128 * (g.route_tiles ? moe_route_max_tiles(g) : g.n_expert), g.n_prob, 1));
+    return launch_moe_gemm_dma<1, 2>(lc, g, dim3((max_n + 127) / 128 * moe_route_max_tiles(g), g.n_prob, 1));
   } else {
     dim3 grid((max_n + 127) / 128, g.n_expert, g.n_prob);
     CG_LAUNCH(lc, moe_gemm_kernel<1>, grid, 256, g);

@@ -1151,14 +1151,14 @@ static bool moe_slot_pitches(const MoeGemmDesc &g, int64_t *a, int64_t *out) {
   return ab % 2 == 0 && cb % ob == 0;
 }
 
-// (route_tiles, 32-bit byte offsets within a tile's weight rows, three k-steps; otherwise what moe_gemm_pipelined_ok asks)
+// (32-bit byte offsets within a tile's weight rows, three k-steps; otherwise what moe_gemm_pipelined_ok asks)
 bool moe_ring_ok(const MoeGemmDesc &g) {
   // With few pairs to an expert most of a tile's products are padding, and they cost what they cost here, where eight wavefronts
   // wait for weights either way (a whole prefill of 60 experts, 4 to a token: 17 pairs to an expert 7.85 -> 8.55 ms, 34 9.49 ->
   // 9.77, 40 9.73 -> 9.82; 47 10.9 -> 10.3, 73 13.8 -> 12.4).
   if ((uint64_t)g.S * g.n_slot < 44 * (uint64_t)g.n_expert) return false;
   int64_t a, out;
-  if (!moe_gemm_pipelined_ok(g) || !g.route_tiles || g.planes || g.K < 192 || !moe_slot_pitches(g, &a, &out)) return false;
+  if (!moe_gemm_pipelined_ok(g) || g.planes || g.K < 192 || !moe_slot_pitches(g, &a, &out)) return false;
   for (uint32_t p = 0; p < g.n_prob; ++p)
     if (g.prob[p].sbn < 0 || g.prob[p].sbn > (1 << 22)) return false;
   return g.fuse_glu ? g.n_prob == 2 && g.prob[0].N == g.prob[1].N : true;

@@ -559,9 +559,8 @@ struct MoeGemmDesc {
   int32_t planes;
   // optional: the (slot, token) pairs already sorted by expert (launch_moe_route): pairs
   // route_list[route_offset[e] .. + route_count[e]) = slot << 16 | token chose expert e
-  const uint32_t *route_count, *route_offset, *route_list;
-  // optional, with the above: the row tiles of all experts as a work list (launch_moe_route's `tiles`)
-  const uint32_t *route_tiles;
+  // and the row tiles of all experts as a work list (launch_moe_route's `tiles`)
+  const uint32_t *route_count, *route_offset, *route_list, *route_tiles;
   int64_t a_slot, out_slot;  // (set by launch_moe_ring) values between the rows, and between the results, of consecutive slots
   uint32_t k_rotate;  // (set by launch_moe_gemm) as GemmDesc::k_rotate
   // optional (N != 0, moe_dense_ok): one more expert, which every token passes through (a shared expert), in the same launch: its rows a16,
@@ -581,13 +580,13 @@ bool moe_ring_ok(const MoeGemmDesc &g);
 bool moe_dense_ok(const MoeGemmDesc &g);  // ... and g.dense among them
 hipError_t launch_moe_ring(const LaunchCtx &lc, const MoeGemmDesc &g);
 // Sorts the S * n_slot (slot, token) pairs of g by expert into count / offset (n_expert words each) and
-// list (moe_route_list_words; every expert's pairs start at a row tile's); n_expert <= MOE_ROUTE_MAX_EXPERTS.  With these in g.route_*, bf16 input rows
-// (slot[].a16 for every slot) and K % 64 == 0, launch_moe_gemm streams the weights through a
+// list (moe_route_list_words; every expert's pairs start at a row tile's); n_expert <= MOE_ROUTE_MAX_EXPERTS.  With these in
+// g.route_*, bf16 input rows (slot[].a16 for every slot) and K % 64 == 0, launch_moe_gemm streams the weights through a
 // multi-stage direct-to-LDS pipeline.
 enum { MOE_ROUTE_MAX_EXPERTS = 4096 };
 // tiles (1 + moe_route_max_tiles(g) words): the number of row tiles (128 pairs, 20 of planes) over all experts, then
-// for each its expert, the number of that expert's row tiles (1 if they are more than 255) and its own number among them (moe_entry); with it in g.route_tiles a workgroup of launch_moe_gemm owns one row tile
-// of one expert, so the launch stays balanced when most tokens choose the same few experts.
+// for each its expert, the number of that expert's row tiles (1 if they are more than 255) and its own number among them (moe_entry): a
+// workgroup of launch_moe_gemm owns one row tile of one expert, so the launch stays balanced when most tokens choose the same few experts.
 // planes (optional): the S rows of K f32 values at slot[0].a, as the planes that launch_moe_gemm takes
 hipError_t launch_moe_route(const LaunchCtx &lc, const MoeGemmDesc &g, uint32_t *count, uint32_t *offset, uint32_t *list,
                             uint32_t *tiles, uint16_t *planes);
