@@ -2667,15 +2667,20 @@ __global__ void __launch_bounds__(256) moe_gemm_dma_kernel(MoeGemmDesc g) {
   // that tile: an expert of a few pairs moves its weights and 32 rows, not 128), then its share of the weight rows.
   const uint16_t *gp[LPW];  // per-lane source; advances by BK per stage
   auto block_of = [&](int i) { return i < MT ? i * 4 + wave : BM_ / 8 + wave * (LPW - MT) + i - MT; };  // 8-row block of the stacked tile
+  uint32_t ents[MT];  // (one trip to memory; rows past the expert's last pair repeat it: loaded, multiplied, never stored)
+#pragma unroll
+  for (int i = 0; i < MT; ++i) {
+    const int R = block_of(i) * 8 + (lane >> 3);
+    ents[i] = list[min(m0 + (uint32_t)(PLANES ? (R >> 5) * TPAIRS + (R & 31) % TPAIRS : R), cnt - 1)];
+  }
 #pragma unroll
   for (int i = 0; i < LPW; ++i) {
     const int q = block_of(i);
     const int R = q * 8 + (lane >> 3);
     const int c = (lane & 7) ^ ((R >> 1) & 7);
     if (i < MT) {
-      // rows past the expert's last pair repeat it: loaded, multiplied, never stored
-      const int part = PLANES ? min((R & 31) / TPAIRS, 2) : 0, pair = PLANES ? (R >> 5) * TPAIRS + (R & 31) % TPAIRS : R;
-      const uint32_t ent = list[min(m0 + (uint32_t)pair, cnt - 1)], sl = ent >> 16, tok = ent & 0xFFFFu;
+      const int part = PLANES ? min((R & 31) / TPAIRS, 2) : 0;
+      const uint32_t sl = ents[i] >> 16, tok = ents[i] & 0xFFFFu;
       const uint16_t *rows = g.slot[0].a16;
       int64_t bs = g.slot[0].a_bs;
 #pragma unroll
