@@ -594,6 +594,60 @@ def test_decode_from_a_kept_cache_copies_it_in_one_launch(oracle, hip, cg, b, H,
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("b,H,KV,d", [(1, 4, 2, 64), (2, 4, 4, 16)])
+@pytest.mark.parametrize("held", ["k", "v", ""])
+def test_one_cache_is_copied_and_the_other_appended_to(hip, cg, b, H, KV, d, held):
+    """A step behind one that laid both caches out with room, with one of them held by somebody else, or neither; and on past the room there is."""
+    g = np.random.default_rng(d)
+    k0, v0 = (g.standard_normal((b, KV, 4, d)).astype(np.float32) for _ in range(2))
+
+    def step(bd, qv, kc, vc, kx, vx):
+        k, v = lang.concat(bd, 2, kc, kx), lang.concat(bd, 2, vc, vx)
+        kr, vr = helpers.repeat_kv(bd, H // KV, k), helpers.repeat_kv(bd, H // KV, v)
+        attn = lang.matmul(bd, qv, lang.transpose(bd, 2, 3, kr))
+        sh = lang.shape(bd, attn)
+        attn = attn / lang.constant(bd, float(np.sqrt(np.float32(d))), sh)
+        attn = attn + lang.broadcast(bd, helpers.causal_mask(bd, lang.to_nat(bd, 1)), sh)
+        return lang.matmul(bd, nn.softmax(bd, attn), vr), k, v
+
+    it, st = cg.Interpreter(hip, cg.stdlib()), vectors.Fn("step", 5, 3, step).term()
+    kc, vc = hip.realize(hip.tensor(k0)), hip.realize(hip.tensor(v0))
+    prefix = [kc, vc]
+
+    def go(kc, vc, moved):
+        nonlocal k0, v0
+        q, kn, vn = (g.standard_normal((b, h, 1, d)).astype(np.float32) for h in (H, KV, KV))
+        hip.launch_counts(reset=True)
+        out, kc, vc = it.run(st, [hip.tensor(q), kc, vc, hip.tensor(kn), hip.tensor(vn)], moved=moved)
+        hip.realize(out)
+        counts = hip.launch_counts(reset=True)
+        k0, v0 = np.concatenate([k0, kn], 2), np.concatenate([v0, vn], 2)
+        kr, vr = (np.repeat(t, H // KV, 1).astype(np.float64) for t in (k0, v0))
+        s = q.astype(np.float64) @ kr.transpose(0, 1, 3, 2) / np.sqrt(d)
+        p = np.exp(s - s.max(-1, keepdims=True))
+        parity.assert_f32((p / p.sum(-1, keepdims=True)) @ vr, hip.numpy(out))
+        return kc, vc, counts
+
+    kc, vc, counts = go(kc, vc, ())
+    assert counts.get("cache_grow") == 1, counts        # (both)
+    before = [hip.numpy(t) for t in (kc, vc)]
+    keep = {"k": kc, "v": vc, "": None}[held]
+    kc, vc, counts = go(kc, vc, {"k": (2,), "v": (1,), "": (1, 2)}[held])
+    assert counts.get("cache_grow", 0) == (1 if held else 0) and not any(n.startswith(("ew_concat", "kv_append")) for n in counts), counts
+    assert np.array_equal(hip.numpy(kc), k0) and np.array_equal(hip.numpy(vc), v0)
+    if held:
+        assert np.array_equal(hip.numpy(keep), before["kv".index(held)])
+    grown = []
+    while k0.shape[2] < 67:         # (room for 64 rows)
+        kc, vc, counts = go(kc, vc, (1, 2))
+        if counts.get("cache_grow"):
+            grown.append(k0.shape[2])
+    assert grown == [65], grown
+    assert np.array_equal(hip.numpy(kc), k0) and np.array_equal(hip.numpy(vc), v0)
+    assert [np.array_equal(hip.numpy(t), f[:, :, :4]) for t, f in zip(prefix, (k0, v0))] == [True, True]
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("rows", [1, 4, 20, 300])
 def test_products_whose_matrix_or_bias_comes_from_another_of_the_same_rows(oracle, hip, hip_bf16, rows):
     """Products of the same rows that would share a launch, but one's matrix, or its bias, is computed from the other."""

@@ -584,3 +584,21 @@ for s, joined in ((300, True), (3072, True), (3073, False)):
     names = [n for n in fake.fake_hip_launched().decode().split("\\n") if "gem" in n or "moe_ring" in n]
     assert sum("moe_ring" in n for n in names) == 2 and (len(names) == 2) == joined, (s, names)
 """, BF16)
+
+
+def test_a_product_and_a_column_that_start_at_different_k(fake_hip):  # noqa: F811
+    """The sizes of test_large_tiles.py: one launch of 32 x 32 tiles, up to 128 rows of whole multiples of 4 KB with an order of their own."""
+    fake_hip(LAUNCHED + f"""
+for m, n, k, joined in {large.WITH_COLUMN}:
+    both = lambda b, x, w, c: [linear(b, x, w, n, k), linear(b, x, c, 1, k)]
+    term = type("Both", (Term,), {{"sort": lambda self: ([lang.TENSOR] * 3, [lang.TENSOR] * 2), "def_": lambda self, b, a: both(b, a[0] + a[0] - a[0], *a[1:])}})
+    be.sync()
+    fake.fake_hip_products()
+    for t in cg.Interpreter(be, cg.stdlib(), cg.Parameters()).run(term(3, None).term(), [operand(1, m, k), operand(n, k), operand(1, k)]):
+        be.realize(t)
+    be.sync()
+    lines = [line.rsplit(" ", 3) for line in fake.fake_hip_products().decode().splitlines()]
+    assert (len(lines) == 1) == joined, (m, n, k, lines)
+    if joined:
+        assert "gemm_bf16_dma_kernelILi32ELi32E" in lines[0][0] and int(lines[0][3]) == (m <= 128 and k >= 2048 and k % 2048 == 0), (m, n, k, lines)
+""", BF16)

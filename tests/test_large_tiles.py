@@ -416,7 +416,9 @@ def test_routed_experts(oracle, hip_bf16, S, E, F, H, act):
 
 # a product of a few dozen columns and one of a single column of the same rows (a MoE layer's router and its shared expert's gate): one
 # launch, a tile more; partly filled tiles of rows and columns, the fewest k, and more rows than two workgroups to a CU hold
-WITH_COLUMN = [(1024, 60, 2048, True), (17, 60, 1024, True), (33, 34, 448, True), (65, 63, 512, True), (5440, 60, 448, True), (5473, 60, 448, False)]
+# (up to 128 rows of 2048 values and more, whose column tiles start at different k, test_k_order.py; weights of a multiple of 4 KB and others)
+WITH_COLUMN = [(1024, 60, 2048, True), (17, 60, 1024, True), (33, 34, 448, True), (65, 63, 512, True), (5440, 60, 448, True), (5473, 60, 448, False),
+               (20, 60, 2048, True), (128, 63, 2048, True), (90, 33, 2048, True), (128, 60, 2112, True), (129, 60, 2048, True)]
 
 
 @pytest.mark.gpu
