@@ -1097,13 +1097,14 @@ int realize_matmul(cg_backend *be, cg_tensor *n, cg_tensor *addend, bool *added,
       if (group.size() < 2) group.clear();  // pairs (gate / up) keep their own launches and epilogues
     }
     // ... and a product of one column that of a few dozen: the shared expert's gate the router's (gemm_with_column_ok)
-    GemmDesc with = g;
-    with.n_group = 2;
-    with.grp_n[0] = N;
-    with.grp_n[1] = 1;
-    with.grp_b[0] = with.grp_b[1] = g.b;
-    if (group.empty() && n->gemm_candidate && !addend && !ep && !ex.w && batch == 1 && N < 64 && gemm_with_column_ok(be->lc(), with)) {
-      for (cg_tensor *c : std::vector<cg_tensor *>(be->gemm_candidates)) {
+    if (group.empty() && n->gemm_candidate && !addend && !ep && !ex.w && batch == 1 && N < 64) {
+      GemmDesc with = g;
+      with.n_group = 2;
+      with.grp_n[0] = N;
+      with.grp_n[1] = 1;
+      with.grp_b[0] = with.grp_b[1] = g.b;
+      const bool takes = gemm_with_column_ok(be->lc(), with);
+      for (cg_tensor *c : takes ? be->gemm_candidates : std::vector<cg_tensor *>()) {
         if (c == n || c->op != N_MATMUL || c->shape[c->rank - 1] != 1 || c->bias_user || !same_matrix(c->in[0], n->in[0])) continue;
         cg_tensor *w = c->in[1];
         if (w->rank != 3 || w->shape[0] != 1 || w->shape[1] != (int64_t)K || waits_for_product(w)) continue;
