@@ -173,7 +173,7 @@ int try_attn_decode(cg_backend *be, cg_tensor *n, bool *done, AttnMergeLater *la
 int try_gemv_attn_merge(cg_backend *be, cg_tensor *n, cg_tensor *addend, bool *added, bool *done);
 cg_tensor *rows_base(cg_tensor *t);
 bool waits_for_product(const cg_tensor *t);
-bool waits_for_expert(const cg_tensor *t);
+bool waits_for_expert(const cg_tensor *t, const cg_tensor *n);
 int try_gate_up_glu(cg_backend *be, cg_tensor *glu, cg_tensor *g, cg_tensor *u, int gelu, bool *done);
 bool norm_row_readers_ok(cg_backend *be, cg_tensor *base, cg_tensor *view, RmsNormMatch *rm);
 int try_gemv_prologue(cg_backend *be, cg_tensor *n, cg_tensor *addend, bool *added, bool *done);

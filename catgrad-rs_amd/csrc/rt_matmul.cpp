@@ -153,24 +153,29 @@ cg_tensor *rows_base(cg_tensor *t) {
 // Whether a product is among what t still waits for (or all that cannot be looked through quickly).  A product that joins the launch of
 // another has its operands realised while that one is on its way: an operand that waits for a product may wait for the very one, or for a
 // third that would take it along.
-static bool waits_for_product(const cg_tensor *t, bool experts, int *looks) {
-  if (t->op == N_REAL) return false;
+static bool waits_for_product(const cg_tensor *t, const cg_tensor *rows, int *looks) {
+  if (t->op == N_REAL || t == rows) return false;
   ExpertOperand eo;
-  if ((t->op == N_MATMUL && (!experts || (t->rank == 3 && match_expert_operand(t->in[1], t->shape[0], &eo)))) ||
-      (t->op == N_KSUM && !experts) || --*looks < 0)
+  if ((t->op == N_MATMUL && (!rows || (t->rank == 3 && match_expert_operand(t->in[1], t->shape[0], &eo)))) || (t->op == N_KSUM && !rows) ||
+      --*looks < 0)
     return true;
   for (const cg_tensor *in : t->in)
-    if (in && waits_for_product(in, experts, looks)) return true;
+    if (in && waits_for_product(in, rows, looks)) return true;
   return false;
 }
 bool waits_for_product(const cg_tensor *t) {
   int looks = 64;
-  return waits_for_product(t, false, &looks);
+  return waits_for_product(t, nullptr, &looks);
 }
-// ... of routed experts.  (Their indices wait for the router's product, which takes no expert's along.)
-bool waits_for_expert(const cg_tensor *t) {
-  int looks = 256;
-  return waits_for_product(t, true, &looks);
+// ... a product of routed experts, for what n, one of them, or another of the same rows reads besides: indices wait for the router's product,
+// which takes no expert's along, and for the rows, which wait for none of these.
+bool waits_for_expert(const cg_tensor *t, const cg_tensor *n) {
+  if (t->op == N_REAL) return false;
+  cg_tensor *rows = n->in[0], *gate = nullptr, *up = nullptr;
+  int gelu = 0, looks = 256;
+  if (rows->op != N_REAL && match_glu(rows, &gate, &up, &gelu) && gate->op == N_MATMUL) rows = gate->in[0];
+  while ((rows->op == N_RESHAPE || rows->op == N_TRANSPOSE || rows->op == N_BROADCAST) && rows->in[0]) rows = rows->in[0];
+  return waits_for_product(t, rows, &looks);
 }
 
 
@@ -662,8 +667,8 @@ int realize_matmul(cg_backend *be, cg_tensor *n, cg_tensor *addend, bool *added,
     // (a matrix that waits for products first: these may be of the same rows, and would find n on its way)
     ExpertOperand own;
     if (n->rank == 3 && match_expert_operand(n->in[1], n->shape[0], &own)) {
-      if (waits_for_expert(own.idx)) TRY(realize(be, own.idx));
-      if (waits_for_expert(own.w)) TRY(realize(be, own.w));
+      if (waits_for_expert(own.idx, n)) TRY(realize(be, own.idx));
+      if (waits_for_expert(own.w, n)) TRY(realize(be, own.w));
     } else if (n->rank <= 3 && waits_for_product(n->in[1])) {
       TRY(realize(be, n->in[1]));
     }

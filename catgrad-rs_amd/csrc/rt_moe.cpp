@@ -96,7 +96,7 @@ int try_moe_gemm(cg_backend *be, cg_tensor *n, bool *done) {
     if (c->op != N_MATMUL || c->rank != 3 || c->shape[0] != S || c->shape[1] != 1 || c->in[0]->rank != 3 || c->in[0]->shape[2] != K)
       continue;
     ExpertOperand co;
-    if (!match_expert_operand(c->in[1], S, &co) || (c != n && (waits_for_expert(co.w) || waits_for_expert(co.idx)))) continue;
+    if (!match_expert_operand(c->in[1], S, &co) || (c != n && (waits_for_expert(co.w, n) || waits_for_expert(co.idx, n)))) continue;
     if (glu) {
       cg_tensor *g2 = nullptr, *u2 = nullptr;
       int ge2 = 0;
@@ -455,7 +455,7 @@ int try_moe_gemv_slots(cg_backend *be, cg_tensor *n, bool *done) {
     if (c->op != N_MATMUL || c->rank != 3 || c->shape[0] != S || c->shape[1] != 1 || c->in[0]->rank != 3 || c->in[0]->shape[2] != K)
       continue;
     ExpertOperand co;
-    if (!match_expert_operand(c->in[1], S, &co) || (c != n && (waits_for_expert(co.w) || waits_for_expert(co.idx)))) continue;
+    if (!match_expert_operand(c->in[1], S, &co) || (c != n && (waits_for_expert(co.w, n) || waits_for_expert(co.idx, n)))) continue;
     if (!glu) {
       if (c->in[0] != A) continue;
       bool known_w = false, known_i = false;
@@ -699,7 +699,7 @@ int try_moe_gemv(cg_backend *be, cg_tensor *n, bool *done) {
     for (cg_tensor *c : be->gemv_candidates) {
       if (c == n || c->op != N_MATMUL || c->in[0] != A || c->rank != 3 || c->shape[0] != S || members.size() >= 4) continue;
       ExpertOperand co;
-      if (!match_expert_operand(c->in[1], S, &co) || co.idx != eo.idx || waits_for_expert(co.w)) continue;
+      if (!match_expert_operand(c->in[1], S, &co) || co.idx != eo.idx || waits_for_expert(co.w, n)) continue;
       members.push_back(c);
       ops.push_back(co);
     }

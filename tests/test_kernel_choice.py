@@ -602,3 +602,44 @@ for m, n, k, joined in {large.WITH_COLUMN}:
     if joined:
         assert "gemm_bf16_dma_kernelILi32ELi32E" in lines[0][0] and int(lines[0][3]) == (m <= 128 and k >= 2048 and k % 2048 == 0), (m, n, k, lines)
 """, BF16)
+
+
+@pytest.mark.parametrize("flags", [0, BF16])
+@pytest.mark.parametrize("shared", [True, False])
+def test_layers_of_experts_that_wait_for_each_other(fake_hip, flags, shared):  # noqa: F811
+    """Nothing is realised between three layers: with matrices of their own or the same in each (whose experts' products look alike), a few tokens
+    and many.  The experts' launch of a few tokens finds their experts itself, as where the layer in front is there."""
+    fake_hip(LAUNCHED + f"""
+helpers = importlib.import_module("catgrad-rs_amd.llm.helpers")
+k, f, fs, e, top, shared, flags = 512, 256, 1024, 60, 4, {shared}, {flags}
+def chain(rows, layers):
+    re = lambda b, x, *shape: lang.reshape(b, lang.make_shape(b, *shape), x)
+    def layer(b, x, wr, wg, wu, wd, sg, su, sd, gate):
+        h = helpers.rmsnorm_raw(b, 1e-5, x)
+        values, idx = lang.topk(b, top, nn.softmax(b, re(b, linear(b, h, wr, e, k), rows, e)))
+        each, total = re(b, h, rows, 1, k), None
+        for i in range(top):
+            slot = lang.get(b, 1, i, idx)
+            of = lambda w: lang.transpose(b, 1, 2, lang.index(b, 0, slot, w))
+            y = lang.matmul(b, nn.silu(b, lang.matmul(b, each, of(wg))) * lang.matmul(b, each, of(wu)), of(wd))
+            y = y * lang.broadcast(b, re(b, lang.get(b, 1, i, values), rows, 1, 1), lang.shape(b, y))
+            total = y if total is None else total + y
+        y = linear(b, nn.silu(b, linear(b, h, sg, fs, k)) * linear(b, h, su, fs, k), sd, k, fs)
+        y = y * lang.broadcast(b, nn.sigmoid(b, linear(b, h, gate, 1, k)), lang.shape(b, y))
+        return re(b, total, 1, rows, k) + y
+    def all_of_them(b, x, *ws):
+        x = x + x - x
+        for i in range(layers): x = layer(b, x, *(ws if shared else ws[8 * i:8 * i + 8]))
+        return x
+    shapes = ((e, k), (e, f, k), (e, f, k), (e, k, f), (fs, k), (fs, k), (k, fs), (1, k))
+    args = [operand(1, rows, k)] + [operand(*s) for s in shapes * (1 if shared else layers)]
+    be.sync()
+    fake.fake_hip_launched()
+    be.realize(run(all_of_them, *args))
+    be.sync()
+    return [n for n in fake.fake_hip_launched().decode().split("\\n") if n]
+for rows in (1, 4, 9, 20, 300):
+    one, three = chain(rows, 1), chain(rows, 3)
+    if rows < 9:
+        assert not any("softmax_topk" in n for n in three), (rows, three)
+""", flags)
