@@ -206,9 +206,6 @@ struct cg_backend {
   cg_tensor *amax_want = nullptr;
   cgrt::Storage *amax_records = nullptr;
   uint32_t amax_n_records = 0;
-  // set by try_gemv_add around realize_matmul when the addend it passes is a bias vector (one row added
-  // to every row of the product) instead of a tensor shaped like the product
-  bool addend_is_row = false;
   // pinned buffers (PREFETCH_BYTES each) of cg_tensor_prefetch no tensor holds any more; the copy into the
   // last ones given back may still be in flight (its flag says)
   std::deque<void *> pinned_pool;

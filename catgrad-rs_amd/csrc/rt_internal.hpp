@@ -170,18 +170,18 @@ struct AttnMergeLater {
   bool deferred = false;
 };
 int try_attn_decode(cg_backend *be, cg_tensor *n, bool *done, AttnMergeLater *later = nullptr);
-int try_gemv_attn_merge(cg_backend *be, cg_tensor *n, cg_tensor *addend, bool *added, bool *done);
+int try_gemv_attn_merge(cg_backend *be, cg_tensor *n, cg_tensor *addend, bool addend_is_row, bool *added, bool *done);
 cg_tensor *rows_base(cg_tensor *t);
 bool waits_for_product(const cg_tensor *t);
 bool waits_for_expert(const cg_tensor *t, const cg_tensor *n);
 int try_gate_up_glu(cg_backend *be, cg_tensor *glu, cg_tensor *g, cg_tensor *u, int gelu, bool *done);
 bool norm_row_readers_ok(cg_backend *be, cg_tensor *base, cg_tensor *view, RmsNormMatch *rm);
-int try_gemv_prologue(cg_backend *be, cg_tensor *n, cg_tensor *addend, bool *added, bool *done);
+int try_gemv_prologue(cg_backend *be, cg_tensor *n, cg_tensor *addend, bool addend_is_row, bool *added, bool *done);
 bool match_expert_operand(const cg_tensor *t, int64_t S, ExpertOperand *o);
 int try_moe_gemm(cg_backend *be, cg_tensor *n, bool *done);
 int try_moe_gemv_slots(cg_backend *be, cg_tensor *n, bool *done);
 int try_moe_gemv(cg_backend *be, cg_tensor *n, bool *done);
-int realize_matmul(cg_backend *be, cg_tensor *n, cg_tensor *addend, bool *added, MatmulEpilogue *ep);
+int realize_matmul(cg_backend *be, cg_tensor *n, cg_tensor *addend, bool *added, MatmulEpilogue *ep, bool addend_is_row = false);
 int realize_concat(cg_backend *be, cg_tensor *n);
 int realize_index(cg_backend *be, cg_tensor *n);
 int realize_arange(cg_backend *be, cg_tensor *n);

@@ -415,7 +415,7 @@ int try_norm_reader_group(cg_backend *be, cg_tensor *n, bool *done) {
 // q/k/v, gate/up and down_proj of a decode step: one-row products whose input row is an RMSNorm
 // or a SwiGLU/GeGLU of earlier values.  When every consumer of that row is such a product, the
 // row is computed inside the product kernel (launch_gemv_pro) and its node is never realised.
-int try_gemv_prologue(cg_backend *be, cg_tensor *n, cg_tensor *addend, bool *added, bool *done) {
+int try_gemv_prologue(cg_backend *be, cg_tensor *n, cg_tensor *addend, bool addend_is_row, bool *added, bool *done) {
   cg_tensor *A = rows_base(n->in[0]);
   if (A->op == N_REAL || A->dtype != CG_F32 || !n->gemv_candidate || A->rank < 1) return CG_OK;
   const int64_t K = A->shape[A->rank - 1];
@@ -518,7 +518,7 @@ int try_gemv_prologue(cg_backend *be, cg_tensor *n, cg_tensor *addend, bool *add
     pr.b = data_ptr(w);
     pr.c = (float *)dest->st->ptr;
     pr.c_add = (c == n && addend) ? (const float *)data_ptr(addend) : bias_vec[i] ? (const float *)data_ptr(bias_vec[i]) : nullptr;
-    pr.c_add_is_row = (c == n && addend) ? (be->addend_is_row ? 1 : 0) : bias_vec[i] ? 1 : 0;
+    pr.c_add_is_row = (c == n && addend) ? (addend_is_row ? 1 : 0) : bias_vec[i] ? 1 : 0;
     pr.sbn = w->strides[w->rank - 1];
     pr.N = (uint32_t)w->shape[w->rank - 1];
     bytes += (double)pr.N * K * esize(w->stype) + (double)rows * pr.N * 4;
@@ -572,7 +572,7 @@ int try_gemv_prologue(cg_backend *be, cg_tensor *n, cg_tensor *addend, bool *add
 // both are views of the same memory order) and read by nobody else.  The attention is launched here and
 // stops at the partial results of its key ranges; this product's kernel merges them on its way in, so
 // the attention needs no hand-over between its workgroups and its value is never stored.
-int try_gemv_attn_merge(cg_backend *be, cg_tensor *n, cg_tensor *addend, bool *added, bool *done) {
+int try_gemv_attn_merge(cg_backend *be, cg_tensor *n, cg_tensor *addend, bool addend_is_row, bool *added, bool *done) {
   if (!n->gemv_candidate) return CG_OK;
   cg_tensor *att = n->in[0];
   // The merge prologue reads the partials in the attention's own (head, d) order, so every view on the
@@ -597,7 +597,7 @@ int try_gemv_attn_merge(cg_backend *be, cg_tensor *n, cg_tensor *addend, bool *a
     if (w->shape[i] != 1 && w->strides[i] != 0) return CG_OK;
   if (w->stype != ST_F32 && w->stype != ST_BF16) return CG_OK;
   if ((uintptr_t)data_ptr(w) % 16 || w->strides[w->rank - 1] % (16 / esize(w->stype))) return CG_OK;
-  if (addend && (addend->stype != ST_F32 || be->addend_is_row)) return CG_OK;
+  if (addend && (addend->stype != ST_F32 || addend_is_row)) return CG_OK;
   if (att->shape[3] % 4) return CG_OK;  // (the merging prologue reads four values of a head at a time)
   // Once the attention has stopped at its partials its own value is never written, so everything that can
   // fail here comes first: the result's memory now; the launch's own checks are the conditions above plus the
@@ -651,8 +651,9 @@ int try_gemv_attn_merge(cg_backend *be, cg_tensor *n, cg_tensor *addend, bool *a
 
 
 // `addend` (optional; realised, f32, contiguous, shaped like n) is added in the epilogue when a
-// one-row kernel runs the product; *added tells the caller whether that happened.
-int realize_matmul(cg_backend *be, cg_tensor *n, cg_tensor *addend, bool *added, MatmulEpilogue *ep) {
+// one-row kernel runs the product; *added tells the caller whether that happened.  addend_is_row: it is a bias
+// vector instead (one row added to every row of the product), of which one row is there to be read.
+int realize_matmul(cg_backend *be, cg_tensor *n, cg_tensor *addend, bool *added, MatmulEpilogue *ep, bool addend_is_row) {
   if (!addend && n->dtype == CG_F32 && n->rank == 4 && n->shape[2] == 1 && !(be->flags & CG_FLAG_NO_PATTERNS)) {
     bool done = false;
     TRY(try_attn_decode(be, n, &done));
@@ -678,9 +679,9 @@ int realize_matmul(cg_backend *be, cg_tensor *n, cg_tensor *addend, bool *added,
     if (done) return CG_OK;
     if (!addend) TRY(try_norm_reader_group(be, n, &done));
     if (done) return CG_OK;
-    TRY(try_gemv_prologue(be, n, addend, added, &done));
+    TRY(try_gemv_prologue(be, n, addend, addend_is_row, added, &done));
     if (done) return CG_OK;
-    TRY(try_gemv_attn_merge(be, n, addend, added, &done));
+    TRY(try_gemv_attn_merge(be, n, addend, addend_is_row, added, &done));
     if (done) return CG_OK;
   }
   MatOperand A, B;
@@ -906,7 +907,7 @@ int realize_matmul(cg_backend *be, cg_tensor *n, cg_tensor *addend, bool *added,
       g.sb_b1 = g.sb_b1 ? (int64_t)N * K : 0;
       g.sb_b0 = g.sb_b0 ? (int64_t)tb1 * N * K : 0;
     }
-    if (addend && !be->addend_is_row && M <= 8 && g.a_stype == ST_F32 && K > 0 && (g.sbk == 1 || g.sbn == 1 || K == 1 || N == 1)) {
+    if (addend && !addend_is_row && M <= 8 && g.a_stype == ST_F32 && K > 0 && (g.sbk == 1 || g.sbn == 1 || K == 1 || N == 1)) {
       g.c_add = (const float *)data_ptr(addend);
       *added = true;
     }
@@ -1062,7 +1063,7 @@ int realize_matmul(cg_backend *be, cg_tensor *n, cg_tensor *addend, bool *added,
     // q/k/v of a prefill: the other deferred many-row products on the same left operand join this
     // launch as further column ranges (their own weights, their own outputs)
     std::vector<cg_tensor *> group, group_add, group_bias;  // a member, the add that takes its value, its bias vector
-    const bool bias_row = addend && be->addend_is_row;  // `addend` is a vector added to every row
+    const bool bias_row = addend && addend_is_row;  // `addend` is a vector added to every row
     // the same rows: one node, or - each linear folding the batch itself - dense reshapes of one value
     auto dense_view = [](const cg_tensor *t, const Storage **st, int64_t *off) {
       const cg_tensor *base = t->op == N_RESHAPE && t->in[0] ? t->in[0] : t;
@@ -1213,7 +1214,7 @@ int realize_matmul(cg_backend *be, cg_tensor *n, cg_tensor *addend, bool *added,
       g.workspace = (float *)ws->ptr;
       g.splits = splits;
       g.k_per_split = ((g.K + splits - 1) / splits + 63) / 64 * 64;
-      if (addend && !be->addend_is_row && !g.c_add && !g.b_index) {  // the pass that sums the k-slices adds the residual too
+      if (addend && !addend_is_row && !g.c_add && !g.b_index) {  // the pass that sums the k-slices adds the residual too
         g.c_add = (const float *)data_ptr(addend);
         *added = true;
         // ... and the caller may leave that pass to the norm that reads the sum
@@ -1222,7 +1223,7 @@ int realize_matmul(cg_backend *be, cg_tensor *n, cg_tensor *addend, bool *added,
     }
     // A product that is not split along k adds the residual as it stores (2900 rows of 2048: an add of its own reads and
     // writes 72 MB, 11 us at either block end; here it reads 24).
-    if (splits <= 1 && addend && !be->addend_is_row && !*added && !ep && group.empty() && !g.c_add && gemm_add_ok(be->lc(), g)) {
+    if (splits <= 1 && addend && !addend_is_row && !*added && !ep && group.empty() && !g.c_add && gemm_add_ok(be->lc(), g)) {
       g.c_add = (const float *)data_ptr(addend);
       *added = true;
     }

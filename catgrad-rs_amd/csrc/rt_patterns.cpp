@@ -1119,10 +1119,7 @@ int try_gemv_add(cg_backend *be, cg_tensor *root, bool *done) {
       // where q / k / v go out as one launch - otherwise *added stays false and the add runs as an op of its own)
       TRY(realize(be, bv));
       if (mm->op != N_MATMUL || !bias_vector_ready(bv)) return CG_OK;  // (mm: as below)
-      be->addend_is_row = true;
-      int st = realize_matmul(be, mm, bv, &added, nullptr);
-      be->addend_is_row = false;
-      if (st) return st;
+      TRY(realize_matmul(be, mm, bv, &added, nullptr, true));
     } else {
       // A residual that is itself the unsummed k-slices of the previous block's product stays that way for
       // now: the norm under this many-row product sums it (realize_matmul sees to it that it is summed by

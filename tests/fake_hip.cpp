@@ -1,10 +1,10 @@
 // A HIP runtime without a GPU, for tests of what the host does: memory is host memory, a stream is always idle, the two
 // copy kernels are made on the spot and every other launch is none.  fake_hip_refuse(name, n): the n-th launch from now
-// of a kernel whose name holds `name` is refused, as the runtime refuses one that it cannot make
-// ("hipHostMalloc": the n-th such call).  fake_hip_launched(): the
-// names of the kernels launched since the last call; fake_hip_products(): of the matrix products among them a line each, the name and what
-// the kernel is told of its walk along k - slices, values to a slice, whether column tiles start at different ones -; fake_hip_static_lds(n):
-// what every kernel's own __shared__ variables take.
+// of a kernel whose name holds `name` is refused, as the runtime refuses one that it cannot make ("hipHostMalloc": the n-th such call).
+// fake_hip_launched(): the names of the kernels launched since the last call; fake_hip_products(): of the matrix products among them a line
+// each, the name and what the kernel is told of its walk along k - slices, values to a slice, whether column tiles start at different ones -;
+// fake_hip_outside(): those that are told to add values which lie outside of what was allocated; fake_hip_static_lds(n): what every kernel's
+// own __shared__ variables take.
 // Loaded with RTLD_GLOBAL before the library, whose references to the runtime it then answers.
 #include <hip/hip_runtime.h>
 #include <atomic>
@@ -22,7 +22,12 @@ std::map<const void *, std::string> &names() {
   return m;
 }
 std::mutex lock;
-std::string refuse, launched, products;
+std::string refuse, launched, products, outside;
+std::map<const char *, size_t> rooms;  // what hipMalloc has given out
+bool within(const void *p, size_t n) {
+  auto it = rooms.upper_bound((const char *)p);
+  return it != rooms.begin() && (--it, (const char *)p + n <= it->first + it->second);
+}
 std::atomic<int> countdown{0}, waits{0}, static_lds{0};
 thread_local hipError_t last = hipSuccess;
 
@@ -50,11 +55,16 @@ hipError_t launch(const void *f, void **args) {
     if (name.find("NS_8GemmDescE") != std::string::npos) {
       const auto &g = *(const cgk::GemmDesc *)args[0];
       const uint32_t splits = g.splits > 1 ? g.splits : 1;
+      if (g.c_add && splits == 1 && !within(g.c_add, (size_t)g.nb0 * g.nb1 * g.M * g.N * 4)) outside += name + "\n";
       products += name + " " + std::to_string(splits) + " " + std::to_string(splits > 1 ? g.k_per_split : g.K) + " " + std::to_string(g.k_rotate) + "\n";
     }
     if (name.find("NS_11MoeGemmDescE") != std::string::npos) {
       const auto &g = *(const cgk::MoeGemmDesc *)args[0];
       products += name + " 1 " + std::to_string(g.K) + " " + std::to_string(g.k_rotate) + "\n";
+    }
+    if (name.find("splitk_reduce_kernel") != std::string::npos) {  // (slices, sums, values of a slice, slices, what is added)
+      const void *add = *(const void **)args[4];
+      if (add && !within(add, *(uint64_t *)args[2] * 4)) outside += name + "\n";
     }
     if (!refuse.empty() && name.find(refuse) != std::string::npos && countdown.fetch_sub(1) == 1) {
       refuse.clear();
@@ -84,6 +94,7 @@ static const char *taken(std::string &lines) {
 }
 const char *fake_hip_launched() { return taken(launched); }
 const char *fake_hip_products() { return taken(products); }
+const char *fake_hip_outside() { return taken(outside); }
 void fake_hip_static_lds(int n) { static_lds = n; }
 
 void **__hipRegisterFatBinary(const void *) { static void *h[4]; return h; }
@@ -101,7 +112,12 @@ hipError_t hipGetDevicePropertiesR0600(hipDeviceProp_t *p, int) {
 hipError_t hipGetSymbolAddress(void **p, const void *) { static char room[1 << 18]; return *p = room, hipSuccess; }
 hipError_t hipGetLastError() { const hipError_t e = last; return last = hipSuccess, e; }
 const char *hipGetErrorString(hipError_t e) { return e == hipSuccess ? "no error" : "launch refused"; }
-hipError_t hipMalloc(void **p, size_t n) { return memory(p, n); }
+hipError_t hipMalloc(void **p, size_t n) {
+  const hipError_t e = memory(p, n);
+  std::lock_guard<std::mutex> lk(lock);
+  if (e == hipSuccess) rooms[(const char *)*p] = n;
+  return e;
+}
 hipError_t hipHostMalloc(void **p, size_t n, unsigned) {
   std::lock_guard<std::mutex> lk(lock);
   if (refuse == "hipHostMalloc" && countdown.fetch_sub(1) == 1) {
@@ -110,7 +126,11 @@ hipError_t hipHostMalloc(void **p, size_t n, unsigned) {
   }
   return memory(p, n);
 }
-hipError_t hipFree(void *p) { return free(p), hipSuccess; }
+hipError_t hipFree(void *p) {
+  std::lock_guard<std::mutex> lk(lock);
+  rooms.erase((const char *)p);
+  return free(p), hipSuccess;
+}
 hipError_t hipHostFree(void *p) { return free(p), hipSuccess; }
 hipError_t hipMemcpy(void *d, const void *s, size_t n, hipMemcpyKind) { return std::memcpy(d, s, n), hipSuccess; }
 hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind, hipStream_t) { return std::memcpy(d, s, n), hipSuccess; }

@@ -594,6 +594,28 @@ def test_decode_from_a_kept_cache_copies_it_in_one_launch(oracle, hip, cg, b, H,
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("rows", [1, 2, 8, 9, 20, 100, 300])
+@pytest.mark.parametrize("n", [512, 40])
+def test_a_bias_behind_another(oracle, hip, hip_bf16, rows, n):
+    """`linear(x) + bias` of a value that is such a sum itself: what is realised on the way to the second does not change how its bias is read."""
+    k = 512
+    g = np.random.default_rng(rows + n)
+    x = g.standard_normal((1, rows, k)).astype(np.float32)
+    args = [t for m in (k, k, n) for t in (g.standard_normal((m, k)).astype(np.float32) * k ** -0.5, g.standard_normal(m).astype(np.float32))]
+
+    def f(b, x, w1, b1, w2, b2, w3, b3):
+        def biased(x, w, bias, n):
+            y = lang.matmul(b, x, lang.reshape(b, lang.make_shape(b, 1, k, n), lang.transpose(b, 0, 1, w)))
+            return y + lang.broadcast(b, bias, lang.shape(b, y))
+        x = x + x - x
+        y = nn.gelu(b, biased(x, w1, b1, k))
+        return [biased(x + biased(y, w2, b2, k), w3, b3, n)]
+    (ref,) = vectors.run(oracle, f, 1, x, *args)
+    for be, check in ((hip, parity.assert_f32), (hip_bf16, parity.assert_bf16)):
+        check(ref, vectors.run(be, f, 1, x, *args)[0])
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("b,H,KV,d", [(1, 4, 2, 64), (2, 4, 4, 16)])
 @pytest.mark.parametrize("held", ["k", "v", ""])
 def test_one_cache_is_copied_and_the_other_appended_to(hip, cg, b, H, KV, d, held):

@@ -643,3 +643,31 @@ for rows in (1, 4, 9, 20, 300):
     if rows < 9:
         assert not any("softmax_topk" in n for n in three), (rows, three)
 """, flags)
+
+
+@pytest.mark.parametrize("flags", [0, BF16])
+def test_what_a_product_adds_lies_in_memory(fake_hip, flags):  # noqa: F811
+    """`linear(x) + bias` of a value that is such a sum itself, and of residuals: a bias vector is not read as a matrix, whatever was realised
+    on the way to it."""
+    fake_hip(LAUNCHED + f"""
+helpers = importlib.import_module("catgrad-rs_amd.llm.helpers")
+fake.fake_hip_outside.restype = ctypes.c_char_p
+k = 512
+def biased(b, x, w, bias, n):
+    y = linear(b, x, w, n, k)
+    return y + lang.broadcast(b, bias, lang.shape(b, y))
+between = {{"nothing": lambda b, y, x: y, "gelu": lambda b, y, x: nn.gelu(b, y), "silu": lambda b, y, x: nn.silu(b, y), "sigmoid": lambda b, y, x: nn.sigmoid(b, y),
+           "norm": lambda b, y, x: helpers.rmsnorm_raw(b, 1e-5, y), "residual": lambda b, y, x: x + y, "softmax": lambda b, y, x: nn.softmax(b, y)}}
+for rows in (1, 2, 4, 8, 9, 16, 20, 100, 300, 1000):
+    for n in (512, 40):
+        for what, act in between.items():
+            def chain(b, x, w1, b1, w2, b2, w3, b3):
+                x = x + x - x
+                y = act(b, biased(b, x, w1, b1, k), x)
+                return biased(b, act(b, biased(b, y, w2, b2, k), x), w3, b3, n)
+            args = [operand(1, rows, k)]
+            for m in (k, k, n): args += [operand(m, k), be.tensor(np.zeros(m, np.float32))]
+            be.realize(run(chain, *args))
+            be.sync()
+            assert not fake.fake_hip_outside(), (rows, n, what)
+""", flags)
